@@ -51,11 +51,13 @@ class tuning:
     def __enter__(self):
         global _tuning
         self._old, _tuning = _tuning, self._new
+        _tell_native()
         return self._new
 
     def __exit__(self, *exc):
         global _tuning
         _tuning = self._old
+        _tell_native()
         return False
 
 
@@ -182,6 +184,32 @@ def load():
     return lib
 
 
+_native = None
+
+
+def _tell_native():
+    if _native is not None:
+        _native.set_tuning(0 if _tuning is None else ctypes.addressof(_tuning))
+
+
+def native():
+    """The native host path of the layer (_native.so: its forward and autograd node), bound to the library
+    that load() has loaded."""
+    global _native
+    if _native is None:
+        if not os.path.exists(os.path.join(_PKG_DIR, "_native.so")):
+            raise RuntimeError("rzlinear_amd/_native.so is not built; run `python -m rzlinear_amd.build`. "
+                               "rzlinear_amd has no fallback path.")
+        from . import _native as module
+        lib = load()
+        module.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in EXPORTS},
+                    lambda K, N, H, BK, BN, R, levels, index: layer_plan(
+                        K, N, H, BK, BN, (ctypes.c_int32 * 8)(*R), levels, torch.device("cuda", index)), check)
+        _native = module
+        _tell_native()
+    return _native
+
+
 # options of rz_weight_grad_ex
 WG_ACCUMULATE, WG_DHW_F32, WG_DBIAS_F32 = 1, 2, 4
 # tile hashes (rz_hash)
@@ -260,6 +288,8 @@ def clear_layer_plans():
     """Forget every layer plan built so far (they are kept per layer geometry and device until this
     is called; a process that goes through many geometries can release them here)."""
     _layer_plans.clear()
+    if _native is not None:
+        _native.clear_plans()
 
 
 def layer_plan(K, N, H, BK, BN, R, hash_levels, device):

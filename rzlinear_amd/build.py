@@ -1,6 +1,7 @@
-"""Builds librzlinear.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc.
+"""Builds librzlinear.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc, and _native.so (the layer's
+host path over that ABI: torch C++ API, no device code) with the host compiler.
 
-    python -m rzlinear_amd.build          # compile every csrc/*.hip and link
+    python -m rzlinear_amd.build          # compile every csrc/*.hip and link, and csrc/rz_torch.cpp
     python -m rzlinear_amd.build --asm    # also keep the device assembly next to the objects
 
 hipcc cross-compiles for gfx950 without a GPU present, so this runs on a CPU-only host.
@@ -16,6 +17,7 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 OBJ_DIR = os.path.join(PKG_DIR, "build")
 LIB_PATH = os.path.join(PKG_DIR, "librzlinear.so")
+NATIVE_PATH = os.path.join(PKG_DIR, "_native.so")
 
 ARCH = "gfx950"
 # Packed-fp32 VALU forms are switched off for all device code of this library.
@@ -50,6 +52,28 @@ def _compile(src, keep_asm, extra=(), obj_dir=OBJ_DIR):
     return obj
 
 
+def build_native(out=NATIVE_PATH):
+    """Compile csrc/rz_torch.cpp against the installed torch; returns the module's path."""
+    import sysconfig
+
+    import torch
+    base = os.path.join(os.path.dirname(os.path.abspath(torch.__file__)))
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    tmp = out + ".tmp"
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)]
+    for inc in (os.path.join(base, "include"), os.path.join(base, "include", "torch", "csrc", "api", "include"),
+                os.path.join(rocm, "include"), sysconfig.get_paths()["include"]):
+        cmd += ["-isystem", inc]
+    cmd += [os.path.join(CSRC, "rz_torch.cpp"), "-o", tmp, "-L" + os.path.join(base, "lib")]
+    cmd += ["-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("the host compiler failed for rz_torch.cpp:\n%s\n%s" % (r.stdout, r.stderr))
+    os.replace(tmp, out)
+    return out
+
+
 def build(keep_asm=False, jobs=None, verbose=True, extra_flags=(), out=None):
     """Compile every HIP source and link librzlinear.so; returns its path.
 
@@ -60,8 +84,11 @@ def build(keep_asm=False, jobs=None, verbose=True, extra_flags=(), out=None):
     os.makedirs(obj_dir, exist_ok=True)
     srcs = sources()
     jobs = jobs or min(len(srcs), os.cpu_count() or 1, 16)
-    with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=jobs + 1) as ex:
+        native = ex.submit(build_native) if out == LIB_PATH else None
         objs = list(ex.map(lambda s: _compile(s, keep_asm, extra_flags, obj_dir), srcs))
+        if native is not None:
+            native.result()
     tmp = out + ".tmp"
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -77,6 +77,56 @@ static int dtype_bytes(int dtype) {
   }
 }
 
+// The plans of the problems that a thread has met last.  A layer asks for the same plan on every step
+// (workspace size, launch), and working one out — a model evaluated for some sixty cuts — takes the host
+// 2 to 6 us; it is a pure function of `key`.  Direct-mapped, a fixed number of entries per thread.
+template <typename Plan, int WORDS>
+struct PlanMemo {
+  static constexpr unsigned kEntries = 64;
+  struct Entry {
+    int key[WORDS];
+    bool valid;
+    Plan plan;
+  };
+  Entry entries[kEntries];
+  template <typename F>
+  const Plan& get(const int (&key)[WORDS], F&& make) {
+    unsigned h = 2166136261u;
+    for (int v : key) h = (h ^ (unsigned)v) * 16777619u;
+    Entry& e = entries[(h ^ (h >> 15)) % kEntries];
+    bool same = e.valid;
+    for (int i = 0; i < WORDS; i++) same &= e.key[i] == key[i];
+    if (!same) {
+      e.plan = make();
+      for (int i = 0; i < WORDS; i++) e.key[i] = key[i];
+      e.valid = true;
+    }
+    return e.plan;
+  }
+};
+
+#define RZ_TUNING_WORDS(t) (t).tile, (t).stages, (t).lds_image, (t).window, (t).split, (t).clamp, (t).fold, (t).fold_tiles, (t).finish, (t).poll_limit
+
+static SplitPlan split_plan(int I, int J, int R, int elem_bytes, const rz_tuning& t) {
+  static thread_local PlanMemo<SplitPlan, 14> memo;
+  return memo.get({I, J, R, elem_bytes, RZ_TUNING_WORDS(t)}, [&] { return plan_split(I, J, R, elem_bytes, t); });
+}
+
+// How a weight gradient is carried out, for a caller with (`planned`) or without a layer plan.
+struct WeightGradChoice {
+  WeightGradPlan plan;
+  WindowPlan window;
+};
+static WeightGradChoice weight_grad_choice(int M, int K, int N, int H, int BK, int BN, int elem_bytes, int tile_bytes, const rz_tuning& t,
+                                           bool planned) {
+  static thread_local PlanMemo<WeightGradChoice, 19> memo;
+  return memo.get({M, K, N, H, BK, BN, elem_bytes, tile_bytes, planned ? 1 : 0, RZ_TUNING_WORDS(t)}, [&] {
+    WeightGradChoice c = {plan_weight_grad(M, K, N, H, BK, BN, elem_bytes, t, tile_bytes), {}};
+    if (!c.plan.lds_image()) c.window = plan_window(M, K, N, H, BK, BN, elem_bytes, t, c.plan, planned);
+    return c;
+  });
+}
+
 static hipError_t launch_gemm(int dtype, int op, const GemmParams& p, const WeightGradPlan* plan,
                               const SplitPlan* split, const rz_tuning& tuning, hipStream_t s) {
   switch (dtype) {
@@ -303,7 +353,7 @@ static int run_plain_op(int op, int dtype, GemmParams p, const void* bias, void*
   p.stream_c = (size_t)p.I * (size_t)p.J * dtype_bytes(dtype) >= ((size_t)8 << 20) ? 1 : 0;
   if (may_split) {
     // tile and slices are chosen together
-    const SplitPlan sp = plan_split(p.I, p.J, p.R, dtype_bytes(dtype), tuning);
+    const SplitPlan sp = split_plan(p.I, p.J, p.R, dtype_bytes(dtype), tuning);
     if (sp.splits > 1) {
       if (workspace == nullptr || workspace_bytes < sp.workspace_bytes) return RZ_ERR_WORKSPACE;
       p.partial = (float*)workspace;
@@ -445,8 +495,6 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
   const bool accumulate = (flags & RZ_WG_ACCUMULATE) != 0;
   const int dhw_dtype = (flags & RZ_WG_DHW_F32) ? RZ_F32 : dtype;
   const int dbias_dtype = (flags & RZ_WG_DBIAS_F32) ? RZ_F32 : dtype;
-  const WeightGradPlan plan = plan_weight_grad(M, K, N, H, BK, BN, dtype_bytes(dtype), tuning,
-                                               fold_tile_bytes(dtype_bytes(dtype), dhw_dtype == RZ_F32, tuning));
   // a layer plan (device memory, built for exactly this K, N, H, tile and hash) replaces the
   // per-call hashing of the tile offsets and the window kernel's search for its strips
   const bool planned = layer_plan != nullptr;
@@ -455,8 +503,11 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
     lay = layer_plan_layout(K, N, H, BK, BN);
     if (!lay.ok || layer_plan_bytes != lay.words * sizeof(int32_t)) return RZ_ERR_BAD_ARGUMENT;
   }
-  WindowPlan wp = {};
-  if (!plan.lds_image()) wp = plan_window(M, K, N, H, BK, BN, dtype_bytes(dtype), tuning, plan, planned && lay.windows > 0);
+  const WeightGradChoice choice = weight_grad_choice(M, K, N, H, BK, BN, dtype_bytes(dtype),
+                                                     fold_tile_bytes(dtype_bytes(dtype), dhw_dtype == RZ_F32, tuning), tuning,
+                                                     planned && lay.windows > 0);
+  const WeightGradPlan& plan = choice.plan;
+  const WindowPlan& wp = choice.window;
   const WeightGradWorkspace ws = weight_grad_workspace(plan, wp, H, dhw_dtype == RZ_F32, dbias != nullptr, planned);
   if (ws.total_bytes > 0 && (workspace == nullptr || workspace_bytes < ws.total_bytes)) return RZ_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
@@ -754,7 +805,7 @@ RZ_API size_t rz_forward_hashed_workspace_bytes(int M, int K, int N, int H, int 
   const int eb = dtype_bytes(dtype);
   const rz_tuning t = tuning_or_default(tuning);
   if (eb == 0 || M < 1 || K < 1 || N < 1 || !tuning_valid(t)) return 0;
-  return plan_split(M, N, K, eb, t).workspace_bytes;
+  return split_plan(M, N, K, eb, t).workspace_bytes;
 }
 
 RZ_API size_t rz_forward_workspace_bytes(int M, int K, int N, int H, int BK, int BN, int dtype) {
@@ -782,7 +833,7 @@ RZ_API size_t rz_input_grad_hashed_workspace_bytes(int M, int K, int N, int H, i
   const int eb = dtype_bytes(dtype);
   const rz_tuning t = tuning_or_default(tuning);
   if (eb == 0 || M < 1 || K < 1 || N < 1 || !tuning_valid(t)) return 0;
-  return plan_split(M, K, N, eb, t).workspace_bytes;
+  return split_plan(M, K, N, eb, t).workspace_bytes;
 }
 
 RZ_API size_t rz_input_grad_workspace_bytes(int M, int K, int N, int H, int BK, int BN, int dtype) {
@@ -843,10 +894,8 @@ RZ_API size_t rz_weight_grad_hashed_workspace_bytes(int M, int K, int N, int H, 
   if (eb == 0 || M < 1 || K < 1 || N < 1 || H < 1 || !tuning_valid(t)) return 0;
   if (check_tile(BK, BN) != RZ_OK) return 0;
   const bool dhw_f32 = (flags & RZ_WG_DHW_F32) != 0 || dtype == RZ_F32;
-  const WeightGradPlan plan = plan_weight_grad(M, K, N, H, BK, BN, eb, t, fold_tile_bytes(eb, dhw_f32, t));
-  WindowPlan wp = {};
-  if (!plan.lds_image()) wp = plan_window(M, K, N, H, BK, BN, eb, t, plan);
-  return weight_grad_workspace(plan, wp, H, dhw_f32, with_dbias != 0).total_bytes;
+  const WeightGradChoice c = weight_grad_choice(M, K, N, H, BK, BN, eb, fold_tile_bytes(eb, dhw_f32, t), t, false);
+  return weight_grad_workspace(c.plan, c.window, H, dhw_f32, with_dbias != 0).total_bytes;
 }
 
 RZ_API size_t rz_weight_grad_ex_workspace_bytes(int M, int K, int N, int H, int BK, int BN, int dtype,
@@ -992,10 +1041,10 @@ RZ_API int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int
   for (int i = 0; i < 8; i++) out[i] = 0;
   if (op == kWeightGrad) {
     const bool dhw_f32 = (flags & RZ_WG_DHW_F32) != 0 || dtype == RZ_F32;
-    const WeightGradPlan plan = plan_weight_grad(M, K, N, H, BK, BN, eb, t, fold_tile_bytes(eb, dhw_f32, t));
-    WindowPlan wp = {};
-    if (!plan.lds_image())
-      wp = plan_window(M, K, N, H, BK, BN, eb, t, plan, planned && layer_plan_layout(K, N, H, BK, BN).windows > 0);
+    const WeightGradChoice c = weight_grad_choice(M, K, N, H, BK, BN, eb, fold_tile_bytes(eb, dhw_f32, t), t,
+                                                  planned && layer_plan_layout(K, N, H, BK, BN).windows > 0);
+    const WeightGradPlan& plan = c.plan;
+    const WindowPlan& wp = c.window;
     if (wp.use) {
       out[0] = 0; out[1] = 1; out[2] = M; out[3] = 32; out[4] = 4; out[5] = wp.windows; out[7] = wp.windows;
       return RZ_OK;
@@ -1012,7 +1061,7 @@ RZ_API int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int
   }
   if (op != kForward && op != kInputGrad) return RZ_ERR_BAD_ARGUMENT;
   const int I = M, J = op == kForward ? N : K, R = op == kForward ? K : N;
-  const SplitPlan sp = plan_split(I, J, R, eb, t);
+  const SplitPlan sp = split_plan(I, J, R, eb, t);
   const bool cut = sp.splits > 1;
   const int chunk = cut ? sp.r_chunk : R;
   const KernelForm f = kernel_form(op, I, J, R, chunk, sp.tile, tile_count(I, J, sp.tile) * sp.splits, eb, t);
