@@ -61,6 +61,8 @@ static int make_hash(HashParams* h, int K, int N, int H, int BK, int BN, const i
   h->bk_shift = ilog2_exact(BK);
   h->bn_shift = ilog2_exact(BN);
   h->levels = levels;
+  h->R0_inverse = fast_mod_inverse(h->R0);
+  h->range_inverse = fast_mod_inverse(h->range);
   return RZ_OK;
 }
 
@@ -129,10 +131,16 @@ static WeightGradChoice weight_grad_choice(int M, int K, int N, int H, int BK, i
 
 static hipError_t launch_gemm(int dtype, int op, const GemmParams& p, const WeightGradPlan* plan,
                               const SplitPlan* split, const rz_tuning& tuning, hipStream_t s) {
-  switch (dtype) {
-    case RZ_F32: return launch_gemm_f32(op, p, plan, split, tuning, s);
-    case RZ_BF16: return launch_gemm_bf16(op, p, plan, split, tuning, s);
-    case RZ_F16: return launch_gemm_f16(op, p, plan, split, tuning, s);
+  switch (dtype * 3 + op) {
+    case RZ_F32 * 3 + kForward: return launch_forward_f32(p, plan, split, tuning, s);
+    case RZ_F32 * 3 + kInputGrad: return launch_input_grad_f32(p, plan, split, tuning, s);
+    case RZ_F32 * 3 + kWeightGrad: return launch_weight_grad_f32(p, plan, split, tuning, s);
+    case RZ_BF16 * 3 + kForward: return launch_forward_bf16(p, plan, split, tuning, s);
+    case RZ_BF16 * 3 + kInputGrad: return launch_input_grad_bf16(p, plan, split, tuning, s);
+    case RZ_BF16 * 3 + kWeightGrad: return launch_weight_grad_bf16(p, plan, split, tuning, s);
+    case RZ_F16 * 3 + kForward: return launch_forward_f16(p, plan, split, tuning, s);
+    case RZ_F16 * 3 + kInputGrad: return launch_input_grad_f16(p, plan, split, tuning, s);
+    case RZ_F16 * 3 + kWeightGrad: return launch_weight_grad_f16(p, plan, split, tuning, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -178,9 +186,13 @@ __global__ void convert_from_f32_kernel(const float* __restrict__ src, T* __rest
 template <typename T, bool ACC, int GROUPS>
 __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __restrict__ part,
                                                               T* __restrict__ out, int H, int pitch,
-                                                              int nparts) {
+                                                              int nparts, int image_blocks, ColsumTail bias) {
   constexpr int kSlots = 256 / GROUPS;
   __shared__ float4 sums[GROUPS][kSlots];
+  if ((int)blockIdx.x >= image_blocks) {   // (uniform) the bias gradient's workgroups
+    colsum_block<256>(bias, (int)blockIdx.x - image_blocks, threadIdx.x, reinterpret_cast<float*>(sums));
+    return;
+  }
   const int q = threadIdx.x % kSlots, g = threadIdx.x / kSlots;
   const int slot = (blockIdx.x * kSlots + q) * 4;
   float4 s = {0.f, 0.f, 0.f, 0.f};
@@ -205,25 +217,6 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __res
       if (slot + e < H)
         out[slot + e] = ElemTraits<T>::from_float(r[e] + (ACC ? ElemTraits<T>::to_float(out[slot + e]) : 0.f));
   }
-}
-
-// dbias[n] = sum over the rows of part[row][n], converted to the element type.  A workgroup owns
-// 64 columns; four thread groups each add up every fourth row (eight loads in flight), then
-// the groups are combined through LDS in a fixed order.
-template <typename T>
-__global__ __launch_bounds__(256) void reduce_colsum_kernel(const float* __restrict__ part,
-                                                            T* __restrict__ out, int N, int pitch, int rows) {
-  __shared__ float sums[4][64];
-  const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
-  const int n = blockIdx.x * 64 + c;
-  float s = 0.f;
-  if (n < N) {
-#pragma unroll 8
-    for (int r = g; r < rows; r += 4) s += part[(size_t)r * pitch + n];
-  }
-  sums[g][c] = s;
-  __syncthreads();
-  if (g == 0 && n < N) out[n] = ElemTraits<T>::from_float((sums[0][c] + sums[1][c]) + (sums[2][c] + sums[3][c]));
 }
 
 // dbias[n] = sum over the rows m of dY[m][n], for the weight-grad forms that do not stage dY
@@ -386,17 +379,18 @@ static hipError_t zero_words(void* p, size_t bytes, hipStream_t s) {
 // Launchers over the output element type (an rz_dtype code) of the weight-grad tail kernels.
 template <bool ACC>
 static void launch_reduce_partials(int out_dtype, const float* part, void* out, int H, int pitch, int nparts,
-                                   hipStream_t s) {
+                                   const ColsumTail& bias, hipStream_t s) {
   // (16 groups of 16 slots; 32 groups of 8 slots — twice the workgroups, every load of a thread in
   //  flight at once — were no faster: 7.0 against 5.7 us for 256 images of 67 KB)
   constexpr int GROUPS = 16, kSlots = 256 / GROUPS;
-  const dim3 grid((pitch / 4 + kSlots - 1) / kSlots), block(256);
+  const int blocks = (pitch / 4 + kSlots - 1) / kSlots;
+  const dim3 grid(blocks + colsum_blocks(bias, 256)), block(256);
   if (out_dtype == RZ_F32)
-    hipLaunchKernelGGL((reduce_partials_kernel<float, ACC, GROUPS>), grid, block, 0, s, part, (float*)out, H, pitch, nparts);
+    hipLaunchKernelGGL((reduce_partials_kernel<float, ACC, GROUPS>), grid, block, 0, s, part, (float*)out, H, pitch, nparts, blocks, bias);
   else if (out_dtype == RZ_BF16)
-    hipLaunchKernelGGL((reduce_partials_kernel<bf16_t, ACC, GROUPS>), grid, block, 0, s, part, (bf16_t*)out, H, pitch, nparts);
+    hipLaunchKernelGGL((reduce_partials_kernel<bf16_t, ACC, GROUPS>), grid, block, 0, s, part, (bf16_t*)out, H, pitch, nparts, blocks, bias);
   else
-    hipLaunchKernelGGL((reduce_partials_kernel<f16_t, ACC, GROUPS>), grid, block, 0, s, part, (f16_t*)out, H, pitch, nparts);
+    hipLaunchKernelGGL((reduce_partials_kernel<f16_t, ACC, GROUPS>), grid, block, 0, s, part, (f16_t*)out, H, pitch, nparts, blocks, bias);
 }
 
 // (tile_dtype: what the contraction kernel stored the tiles as — floats, or the layer's 16-bit dtype)
@@ -405,7 +399,7 @@ static hipError_t launch_fold_small(const FoldParams& fp, int tile_dtype, hipStr
   if (fp.partial != nullptr || fp.out == nullptr || fp.shares != 1 || tiles > kFoldSmallTiles ||
       fp.window != kFoldSmallThreads || (long long)fp.windows * fp.window < fp.H)
     return hipErrorInvalidValue;
-  const dim3 grid((unsigned)fp.windows), block(kFoldSmallThreads);
+  const dim3 grid((unsigned)(fp.windows + colsum_blocks(fp.bias, kFoldSmallThreads))), block(kFoldSmallThreads);
   if (tile_dtype == RZ_BF16) hipLaunchKernelGGL(fold_small_kernel<bf16_t>, grid, block, 0, s, fp);
   else if (tile_dtype == RZ_F16) hipLaunchKernelGGL(fold_small_kernel<f16_t>, grid, block, 0, s, fp);
   else hipLaunchKernelGGL(fold_small_kernel<float>, grid, block, 0, s, fp);
@@ -424,7 +418,7 @@ static hipError_t launch_fold_as(const FoldParams& fp, hipStream_t s) {
     hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(fold_tiles_kernel<TT>), raised);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(fold_tiles_kernel<TT>, dim3((unsigned)(fp.windows * fp.shares)), dim3(kFoldThreads), lds, s, fp);
+  hipLaunchKernelGGL(fold_tiles_kernel<TT>, dim3((unsigned)(fp.windows * fp.shares + colsum_blocks(fp.bias, kFoldThreads))), dim3(kFoldThreads), lds, s, fp);
   return hipGetLastError();
 }
 
@@ -445,15 +439,10 @@ static void launch_convert(int out_dtype, const float* src, void* dst, int n, hi
     hipLaunchKernelGGL((convert_from_f32_kernel<float, ACC>), grid, block, 0, s, src, (float*)dst, n);
 }
 
-static void launch_reduce_colsum(int out_dtype, const float* part, void* out, int N, int pitch, int rows,
-                                 hipStream_t s) {
-  const dim3 grid((N + 63) / 64), block(256);
-  if (out_dtype == RZ_F32)
-    hipLaunchKernelGGL(reduce_colsum_kernel<float>, grid, block, 0, s, part, (float*)out, N, pitch, rows);
-  else if (out_dtype == RZ_BF16)
-    hipLaunchKernelGGL(reduce_colsum_kernel<bf16_t>, grid, block, 0, s, part, (bf16_t*)out, N, pitch, rows);
-  else
-    hipLaunchKernelGGL(reduce_colsum_kernel<f16_t>, grid, block, 0, s, part, (f16_t*)out, N, pitch, rows);
+// The bias gradient on its own (where no kernel follows the contraction that could carry it).
+__global__ __launch_bounds__(256) void colsum_kernel(ColsumTail bias) {
+  __shared__ float sums[256];
+  colsum_block<256>(bias, blockIdx.x, threadIdx.x, sums);
 }
 
 static inline size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -561,6 +550,7 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
       return RZ_OK;
     }
   }
+  const ColsumTail bias = {p.colsum, dbias, dbias_dtype, N, plan.colsum_pitch, plan.colsum_rows};
   if (plan.fold.use) {
     // no scatter in the contraction: X^T.dY goes to the workspace tile by tile, the fold kernel's
     // workgroups each add up the tiles that land in their window of hashed_weight (per share of
@@ -575,6 +565,7 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
     p.out_tiles_n = (N + BN - 1) / BN;
     if (launch_gemm(dtype, kWeightGrad, p, &plan, nullptr, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
     FoldParams fp;
+    fp.bias = f.shares > 1 ? ColsumTail{} : bias;   // (carried by the last kernel)
     fp.tiles = p.tiles_out;
     fp.plan_header = nullptr;
     fp.plan_start = nullptr;
@@ -614,16 +605,16 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
     fp.shares = f.shares;
     if ((f.small ? launch_fold_small(fp, tile_dtype, s) : launch_fold(fp, tile_dtype, s)) != hipSuccess) return RZ_ERR_LAUNCH;
     if (f.shares > 1) {
-      if (accumulate) launch_reduce_partials<true>(dhw_dtype, fp.partial, dHW, H, fp.pitch, f.shares, s);
-      else launch_reduce_partials<false>(dhw_dtype, fp.partial, dHW, H, fp.pitch, f.shares, s);
+      if (accumulate) launch_reduce_partials<true>(dhw_dtype, fp.partial, dHW, H, fp.pitch, f.shares, bias, s);
+      else launch_reduce_partials<false>(dhw_dtype, fp.partial, dHW, H, fp.pitch, f.shares, bias, s);
     }
   } else if (plan.image_pitch > 0) {
     // every workgroup sums its tiles into an LDS image of dHW and stores it as a partial image;
     // the partial images are then added up (no global atomics, fixed summation order)
     p.scatter = (float*)workspace;
     if (launch_gemm(dtype, kWeightGrad, p, &plan, nullptr, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
-    if (accumulate) launch_reduce_partials<true>(dhw_dtype, p.scatter, dHW, H, plan.image_pitch, (int)plan.workgroups, s);
-    else launch_reduce_partials<false>(dhw_dtype, p.scatter, dHW, H, plan.image_pitch, (int)plan.workgroups, s);
+    if (accumulate) launch_reduce_partials<true>(dhw_dtype, p.scatter, dHW, H, plan.image_pitch, (int)plan.workgroups, bias, s);
+    else launch_reduce_partials<false>(dhw_dtype, p.scatter, dHW, H, plan.image_pitch, (int)plan.workgroups, bias, s);
   } else {
     // hashed_weight too large for an LDS image: tiles go to an fp32 image of dHW by global
     // atomics; an fp32 dHW is its own image (and, accumulating, needs no clearing)
@@ -637,13 +628,9 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
       if (accumulate) launch_convert<true>(dhw_dtype, image, dHW, H, s);
       else launch_convert<false>(dhw_dtype, image, dHW, H, s);
     }
+    if (bias.part != nullptr) hipLaunchKernelGGL(colsum_kernel, dim3(colsum_blocks(bias, 256)), dim3(256), 0, s, bias);
   }
-  if (hipGetLastError() != hipSuccess) return RZ_ERR_LAUNCH;
-  if (dbias != nullptr) {
-    launch_reduce_colsum(dbias_dtype, p.colsum, dbias, N, plan.colsum_pitch, plan.colsum_rows, s);
-    if (hipGetLastError() != hipSuccess) return RZ_ERR_LAUNCH;
-  }
-  return RZ_OK;
+  return hipGetLastError() == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;
 }
 
 }  // namespace rz

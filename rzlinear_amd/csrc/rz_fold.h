@@ -38,7 +38,44 @@
 
 namespace rz {
 
+// The bias gradient's last pass: out[n] = sum over the rows of part[row][n] (the contraction kernel's partial
+// column sums of dY), converted to the output type.  It is work for a few dozen workgroups of less than two
+// microseconds, which as a kernel of its own takes 3 to 5 us (launch and drain); so it rides along: the
+// kernels that finish dHW get `blocks` extra workgroups at the end of their grid that do this instead.
+struct ColsumTail {
+  const float* part;   // null: no bias gradient
+  void* out;
+  int out_dtype;       // an rz_dtype code
+  int N, pitch, rows;
+};
+static constexpr int kColsumCols = 64;   // columns of 256 threads: four groups that each add up every fourth row
+static inline int colsum_blocks(const ColsumTail& c, int threads) {
+  const int cols = kColsumCols * threads / 256;
+  return c.part != nullptr ? (c.N + cols - 1) / cols : 0;
+}
+// `block` of THREADS (a multiple of 256) threads; lds: THREADS floats.  Eight loads in flight per thread; the
+// groups are combined in a fixed order.
+template <int THREADS>
+__device__ __forceinline__ void colsum_block(const ColsumTail& c, int block, int tid, float* lds) {
+  const int col = tid & 63, g = (tid >> 6) & 3, part = tid >> 8;
+  const int n = (block * (THREADS / 256) + part) * kColsumCols + col;
+  float s = 0.f;
+  if (n < c.N) {
+#pragma unroll 8
+    for (int r = g; r < c.rows; r += 4) s += c.part[(size_t)r * c.pitch + n];
+  }
+  lds[tid] = s;
+  __syncthreads();
+  if (g == 0 && n < c.N) {
+    const float v = (lds[tid] + lds[tid + 64]) + (lds[tid + 128] + lds[tid + 192]);
+    if (c.out_dtype == RZ_F32) static_cast<float*>(c.out)[n] = v;
+    else if (c.out_dtype == RZ_BF16) static_cast<bf16_t*>(c.out)[n] = ElemTraits<bf16_t>::from_float(v);
+    else static_cast<f16_t*>(c.out)[n] = ElemTraits<f16_t>::from_float(v);
+  }
+}
+
 struct FoldParams {
+  ColsumTail bias;      // ... and its workgroups, behind the fold's own
   const void* tiles;    // [slices][tiles_k * tiles_n][BK * BN], floats or elements of a 16-bit dtype (the kernels' TT)
   const int32_t* offsets;   // [tiles_k * tiles_n] where every tile starts in hashed_weight (hashed once, by another kernel;
                             // null for the few-tiles kernel: it hashes them itself)
@@ -116,6 +153,10 @@ __global__ __launch_bounds__(kFoldThreads) void fold_tiles_kernel(const FoldPara
   constexpr int kBlockShift = kPer == 4 ? 8 : 9;
   const int lane_e = lane * kPer;
   const unsigned lane16 = lane * 16;
+  if ((int)blockIdx.x >= p.windows * p.shares) {   // (uniform)
+    colsum_block<kFoldThreads>(p.bias, (int)blockIdx.x - p.windows * p.shares, tid, fold_lds);
+    return;
+  }
   const int win = blockIdx.x % p.windows, share = blockIdx.x / p.windows;
   const int w0 = win * p.window;
   const int wlen = (p.H - w0) < p.window ? (p.H - w0) : p.window;
@@ -404,6 +445,10 @@ __global__ __launch_bounds__(kFoldSmallThreads) void fold_small_kernel(const Fol
   __shared__ int list_rel[kFoldSmallTiles];    // ... and where each starts, relative to the first element
   __shared__ int wave_count[kFoldSmallThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if ((int)blockIdx.x >= p.windows) {   // (uniform)
+    colsum_block<kFoldSmallThreads>(p.bias, (int)blockIdx.x - p.windows, tid, reinterpret_cast<float*>(list_id));
+    return;
+  }
   constexpr int kSpan = kFoldSmallThreads * PER;
   const int h0 = blockIdx.x * kSpan;
   const int span = (p.H - h0) < kSpan ? (p.H - h0) : kSpan;

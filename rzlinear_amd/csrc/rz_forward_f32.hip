@@ -1,0 +1,9 @@
+// Instantiation of the forward contraction kernels for element type float.
+#include "rz_gemm_inst.h"
+
+namespace rz {
+hipError_t launch_forward_f32(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning,
+                        hipStream_t stream) {
+  return launch_gemm_t<float, kForward>(p, plan, split, tuning, stream);
+}
+}  // namespace rz

@@ -160,7 +160,7 @@ __device__ __forceinline__ u32x4_t shift_down_16(u32x4_t v, int sh) {
 template <typename T, int OP, int TI, int TJ, int WI, int WJ, int NSTAGE, bool FULL, bool COLSUM = false,
           bool CLAMP = false, int WK = 1>
 struct GemmKernel {
-  static_assert(WK == 1 || (OP != kWeightGrad && NSTAGE == 2), "the R step is shared out only by the pipelined store kernels");
+  static_assert(WK == 1 || NSTAGE >= 2, "the R step is shared out only by the pipelined kernels");
   static_assert(!(FULL && CLAMP), "complete tiles need no clamping");
   static_assert(!COLSUM || OP == kWeightGrad, "column sums belong to the weight-grad contraction");
   typedef ElemTraits<T> Tr;
@@ -170,8 +170,9 @@ struct GemmKernel {
   // R step: 128 bytes of R — except the directly staged 128 tile with eight wavefronts, which
   // is used at about one workgroup per compute unit and has LDS to spare: it takes 256 bytes
   // per step, halving the barriers per flop (8 % faster at 2048^3).
-  static constexpr bool kLongStep = Tr::kBytes == 2 && (FULL || CLAMP) && NSTAGE == 2 && TI == 128 && TJ == 128 &&
-                                    WI * WJ == 8;
+  // ... and the directly staged 64 tile, whose sixteen wavefronts share a step four ways.
+  static constexpr bool kLongStep = Tr::kBytes == 2 && (FULL || CLAMP) && NSTAGE >= 2 &&
+                                    ((TI == 128 && TJ == 128 && WI * WJ == 8) || (TI == 64 && TJ == 64));
   // ... and the fp32 tiles of at most 64 rows in forward / input-grad, whose 128-byte step is over in
   // 0.4 us — less than a load from L2 takes, so that loads issued two steps ahead arrive late, and
   // half as many barriers per flop (1024^3: forward 30.2 -> 28.3 us, input-grad 27.1 -> 25.9 us;
@@ -183,9 +184,13 @@ struct GemmKernel {
   static __device__ __forceinline__ int row_swizzle(int row) { return kPpr == 16 ? (row & 15) : ((row >> 1) & 7); }
   // swizzle of an X-contiguous direct stage: the unit of 32 elements u of row r sits at u ^ unit_swizzle(r)
   // (32-bit: rows r and r + 4, which the two halves of a wavefront read together, land in different banks)
-  static __device__ __forceinline__ int unit_swizzle(int row) { return Tr::kBytes == 2 ? (row & 3) : ((row >> 2) & 1); }
+  // (16-bit rows of 64 elements are two units of 64 bytes: four consecutive rows, which half a wavefront reads
+  //  together, fill two pitches of 128 bytes twice, so every other PAIR of rows is swapped)
+  static __device__ __forceinline__ int unit_swizzle(int row, int pitch) {
+    return Tr::kBytes == 2 ? (pitch == 64 ? ((row >> 1) & 1) : (row & 3)) : ((row >> 2) & 1);
+  }
   static __device__ __forceinline__ int strided_at(int row, int col, int pitch) {
-    return row * pitch + ((((col >> 5) ^ unit_swizzle(row)) << 5) | (col & 31));
+    return row * pitch + ((((col >> 5) ^ unit_swizzle(row, pitch)) << 5) | (col & 31));
   }
   static __device__ __forceinline__ u32x4_t shift_down(u32x4_t v, int sh) {
     return Tr::kBytes == 2 ? shift_down_16(v, sh) : shift_down_32(v, sh);
@@ -197,7 +202,7 @@ struct GemmKernel {
   static_assert(WTI % 32 == 0 && WTJ % 32 == 0, "wavefront tile must be a multiple of 32");
 
   // direct-to-LDS staging (see the head of this file)
-  static constexpr bool kDirect16 = k16 && (FULL || CLAMP) && NSTAGE == 2 && TI >= 128 && TJ >= 128;
+  static constexpr bool kDirect16 = k16 && (FULL || CLAMP) && NSTAGE >= 2 && ((TI >= 128 && TJ >= 128) || (TI == 64 && TJ == 64));
   // fp32, complete tiles: the same staging; a "sub-step" is then eight elements of R (four MFMAs per
   // pair of blocks), and a fragment holds a lane's four values of it
   static constexpr bool kDirect32 = !k16 && RZ_F32_DIRECT && (FULL || CLAMP) && NSTAGE == 2 && TJ >= 64;
@@ -581,7 +586,7 @@ struct GemmKernel {
         row = n * (64 / kSlots) + lane / kSlots;
         const int slot = lane % kSlots;
         constexpr int kPpu = 32 / VEC;                  // 16-byte slots per unit of 32 elements
-        col = (((slot / kPpu) ^ unit_swizzle(row)) << 5) | ((slot % kPpu) * VEC);
+        col = (((slot / kPpu) ^ unit_swizzle(row, LL::kPitch)) << 5) | ((slot % kPpu) * VEC);
       }
     };
     auto direct_load = [&](const T* src, const T* stage, int q, int pieces) {
@@ -860,14 +865,19 @@ struct GemmKernel {
       // when stage s&1 has been read for the last time, the direct-to-LDS loads of step s+2
       // are issued into it; they have a whole step to land and are waited for just before the
       // barrier of step s+1.
+      // With more than two stages (NSTAGE) the same, the loads running NSTAGE steps ahead: before the barrier of
+      // step s those of step s+1 must have landed, the younger ones stay in flight.
       constexpr int NKS = TR / KS / WK;   // sub-steps of this wavefront's part of an R step
+      constexpr int kLoads = LA::kPieces + LB::kPieces;   // direct loads of a wavefront per step
+      static_assert(NSTAGE == 2 || kDirect, "a deeper pipeline is built for direct staging only");
+      auto stage_of = [](int s) -> int { return s % NSTAGE; };
       // fp32: left to itself the compiler moves a sub-step's fragment reads down to just before
       // the MFMAs that use them (read, wait, four MFMAs).  Holding them a sub-step ahead, as
       // written, is faster in the 64 tile (1024^3: 28.7 -> 27.4 us forward, 33.8 -> 31.4 us
       // weight-grad) and in the 256 tile's input-grad (M = 32768, K = N = 2048: 2110 -> 2003 us),
       // slower elsewhere (4096^3 forward 996 -> 1031 us; the 128 tile at 2048^3 154 -> 164 us).
       constexpr bool kPinFrags = !kDirect && sizeof(T) == 4 && (TI == 64 || (TI == 256 && OP == kInputGrad));
-      static_assert(NKS >= 3 && NKS * KS * WK == TR, "pipeline needs at least three sub-steps per R step");
+      static_assert((NKS >= 3 || (kDirect && NKS == 2)) && NKS * KS * WK == TR, "pipeline needs at least three sub-steps per R step (direct staging: two)");
       const int ks0 = wave_k * NKS;
       Frag fa[2][MI], fb[2][MJ];
       auto frags = [&](int st, int ks, int buf) {
@@ -891,7 +901,7 @@ struct GemmKernel {
       auto step = [&](int s, auto late, auto do_commit, auto do_fetch, auto has_next) {
         constexpr int kCommitAt = decltype(late)::value ? NKS - 2 : 0;
         constexpr int kFetchAt = kCommitAt;   // right behind the LDS writes that free the registers
-        const int st = s & 1;
+        const int st = stage_of(s), next = stage_of(s + 1);
         // (its few threads branch, which ends a scheduling region: keep it out of the MFMA stream)
         if constexpr (decltype(do_fetch)::value) hash_ahead(s);
 #pragma unroll
@@ -901,24 +911,27 @@ struct GemmKernel {
             if constexpr (kPinFrags) __builtin_amdgcn_sched_barrier(0);
           } else {
             if constexpr (kDirect) {
-              // the loads of step s+1 (the only ones in flight) must have landed
-              if constexpr (decltype(has_next)::value) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+              // the loads of step s+1 must have landed (near the end: whatever is in flight)
+              if constexpr (decltype(do_fetch)::value) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NSTAGE - 2) * kLoads) : "memory");
+              else if constexpr (decltype(has_next)::value) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             }
             __syncthreads();
             if constexpr (kDirect) {
-              // stage st has been read for the last time: refill it for step s+2
-              if constexpr (decltype(do_fetch)::value) direct_issue(s + 2, st);
-              // (no refill left = the next step is the last one: it may be a partial step)
-              if constexpr (decltype(has_next)::value && !decltype(do_fetch)::value) clear_tail(st ^ 1);
+              // stage st has been read for the last time: refill it for step s+NSTAGE
+              if constexpr (decltype(do_fetch)::value) direct_issue(s + NSTAGE, st);
+              // (the last step may be a partial one)
+              if constexpr (decltype(has_next)::value && !decltype(do_fetch)::value) {
+                if (NSTAGE == 2 || s + 2 == steps) clear_tail(next);
+              }
             }
-            if constexpr (decltype(has_next)::value) frags(st ^ 1, 0, (ks + 1) & 1);
+            if constexpr (decltype(has_next)::value) frags(next, 0, (ks + 1) & 1);
           }
           if constexpr (kDirect && COLSUM) {
-            if (ks == 1) colsum_from_stage(st);   // once per R step, in step order
+            if (ks == (NKS > 2 ? 1 : 0)) colsum_from_stage(st);   // once per R step, in step order, before the stage is refilled
           }
           if constexpr (!kDirect) {
             if (ks == kCommitAt) {
-              if constexpr (decltype(do_commit)::value) commit(st ^ 1);
+              if constexpr (decltype(do_commit)::value) commit(next);
             }
             if (ks == kFetchAt) {
               if constexpr (decltype(do_fetch)::value) fetch(s + 2);
@@ -929,23 +942,25 @@ struct GemmKernel {
       };
       auto loop = [&](auto late) {
         int s = 0;
-        for (; s + 2 < steps; s++) step(s, late, std::true_type{}, std::true_type{}, std::true_type{});
-        if (s + 1 < steps) {
-          step(s, late, std::true_type{}, std::false_type{}, std::true_type{});
-          s++;
+        for (; s + NSTAGE < steps; s++) step(s, late, std::true_type{}, std::true_type{}, std::true_type{});
+        if constexpr (NSTAGE == 2) {
+          if (s + 1 < steps) {
+            step(s, late, std::true_type{}, std::false_type{}, std::true_type{});
+            s++;
+          }
+        } else {
+          for (; s + 1 < steps; s++) step(s, late, std::true_type{}, std::false_type{}, std::true_type{});
         }
         step(s, late, std::false_type{}, std::false_type{}, std::false_type{});
       };
       if (steps > 0) {
         if constexpr (kDirect) {
-          direct_issue(0, 0);
-          if (steps > 1) {
-            direct_issue(1, 1);
-            // loads complete in order: all but the last step's worth have landed
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LA::kPieces + LB::kPieces) : "memory");
-          } else {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          }
+#pragma unroll
+          for (int i = 0; i < NSTAGE; i++)
+            if (i < steps) direct_issue(i, i);
+          // loads complete in order: all but the later steps' have landed
+          if (steps >= NSTAGE) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NSTAGE - 1) * kLoads) : "memory");
+          else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         } else {
           commit(0);
           if (steps > 1) fetch(1);
@@ -960,6 +975,40 @@ struct GemmKernel {
         else loop(std::false_type{});
       }
     }
+
+    // Add up the accumulators of the groups of wavefronts that shared the R steps: every group parks its own in
+    // the dead operand stages and adds up (in group order) a WK-th of each block's rows, which it then stores:
+    // element e of acc is from here on row block_row(e) of the block, e < kElems.
+    constexpr int kElems = 16 / WK;
+    static_assert(WK == 1 || WK == 2 || WK == 4, "a group takes whole quarters of a block's elements");
+    auto block_row = [&](int e) -> int { return ((WK > 1 ? wave_k * (kElems / 4) : 0) + (e >> 2)) * 8 + (lane >> 5) * 4 + (e & 3); };
+    auto merge_groups = [&]() {
+      if constexpr (WK > 1) {
+        float* park = reinterpret_cast<float*>(&sm);
+        static_assert(WK == 1 || sizeof(float) * WK * TI * TJ <= sizeof(T) * NSTAGE * (LA::kElems + LB::kElems), "the accumulators must fit the stages");
+        __syncthreads();   // every wavefront is done reading the stages
+        const int slot = ((wave % (WI * WJ)) * MI * MJ) * 16 * 64 + lane;
+#pragma unroll
+        for (int a = 0; a < MI; a++)
+#pragma unroll
+          for (int b = 0; b < MJ; b++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) park[wave_k * TI * TJ + slot + ((a * MJ + b) * 16 + e) * 64] = acc[a][b][e];
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < MI; a++)
+#pragma unroll
+          for (int b = 0; b < MJ; b++)
+#pragma unroll
+            for (int e = 0; e < kElems; e++) {
+              const int at = slot + ((a * MJ + b) * 16 + wave_k * kElems + e) * 64;
+              float v = park[at];
+#pragma unroll
+              for (int g = 1; g < WK; g++) v += park[g * TI * TJ + at];
+              acc[a][b][e] = v;
+            }
+      }
+    };
 
     // ---- epilogue ---------------------------------------------------------------------------
     // accumulator element e of a 32x32 block: row (e/4)*8 + (lane/32)*4 + e%4, column lane%32
@@ -981,6 +1030,8 @@ struct GemmKernel {
         }
         __syncthreads();
       }
+      merge_groups();
+      if constexpr (WK > 1) __syncthreads();   // (the parked values have been read)
       if (image_mode) {
         const float4 z = {0.f, 0.f, 0.f, 0.f};
         for (int i = tid * 4; i < p.image_pitch; i += kThreads * 4) *reinterpret_cast<float4*>(image + i) = z;
@@ -1011,16 +1062,16 @@ struct GemmKernel {
 #pragma unroll
           for (int b = 0; b < MJ; b++) {
             const int n = j0 + blk_j(b) + (lane & 31);
-            int base[4];
+            int base[kElems / 4];
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-              const int k = i0 + blk_i(a) + g * 8 + (lane >> 5) * 4;
+            for (int g = 0; g < kElems / 4; g++) {
+              const int k = i0 + blk_i(a) + block_row(g * 4);
               const int start = etab[((k >> p.h.bk_shift) - w.tk0) * w.ntn + ((n >> p.h.bn_shift) - w.tn0)];
               base[g] = start < 0 ? -1 : start + (k & (p.h.BK - 1)) * p.h.BN + (n & (p.h.BN - 1));
             }
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-              const int k = i0 + blk_i(a) + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+            for (int e = 0; e < kElems; e++) {
+              const int k = i0 + blk_i(a) + block_row(e);
               const bool inside = FULL || (k < p.I && n < p.J);
               if (FULL || base[e >> 2] >= 0) {
                 const float v = inside ? acc[a][b][e] * p.scale : 0.f;
@@ -1042,18 +1093,18 @@ struct GemmKernel {
 #pragma unroll
           for (int b = 0; b < MJ; b++) {
             const int n = j0 + blk_j(b) + (lane & 31);
-            int base[4];
-            bool ok[4];
+            int base[kElems / 4];
+            bool ok[kElems / 4];
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-              const int k = i0 + blk_i(a) + g * 8 + (lane >> 5) * 4;
+            for (int g = 0; g < kElems / 4; g++) {
+              const int k = i0 + blk_i(a) + block_row(g * 4);
               ok[g] = FULL || (k < p.I && n < p.J);
               base[g] = etab[((k >> p.h.bk_shift) - w.tk0) * w.ntn + ((n >> p.h.bn_shift) - w.tn0)] +
                         (k & (p.h.BK - 1)) * p.h.BN + (n & (p.h.BN - 1));
             }
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-              const int k = i0 + blk_i(a) + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+            for (int e = 0; e < kElems; e++) {
+              const int k = i0 + blk_i(a) + block_row(e);
               if (FULL || (ok[e >> 2] && k < p.I))
                 unsafeAtomicAdd(target + base[e >> 2] + (e & 3) * p.h.BN, acc[a][b][e] * p.scale);
             }
@@ -1079,7 +1130,7 @@ struct GemmKernel {
               const int t = __builtin_amdgcn_readfirstlane(((k0 >> p.h.bk_shift) - w.tk0) * w.ntn +
                                                            ((n0 >> p.h.bn_shift) - w.tn0));
               blk_tile[a][b] = t;
-              blk_base[a][b] = etab[t] + ((k0 & (p.h.BK - 1)) + (lane >> 5) * 4) * p.h.BN +
+              blk_base[a][b] = etab[t] + ((k0 & (p.h.BK - 1)) + block_row(0)) * p.h.BN +
                                ((n0 + (lane & 31)) & (p.h.BN - 1));
             }
           // With many hashed tiles per C tile, tiles whose slices do not meet may share a round:
@@ -1122,14 +1173,14 @@ struct GemmKernel {
 #pragma unroll
                 for (int b = 0; b < MJ; b++) {
                   if (blk_tile[a][b] == t) {
-                    const int k0 = i0 + blk_i(a) + (lane >> 5) * 4;
+                    const int k0 = i0 + blk_i(a) + block_row(0);
                     const bool col_ok = FULL || (j0 + blk_j(b) + (lane & 31) < p.J);
-                    float cur[16];
+                    float cur[kElems];
 #pragma unroll
-                    for (int e = 0; e < 16; e++)
+                    for (int e = 0; e < kElems; e++)
                       cur[e] = image[blk_base[a][b] + ((e >> 2) * 8 + (e & 3)) * p.h.BN];
 #pragma unroll
-                    for (int e = 0; e < 16; e++)
+                    for (int e = 0; e < kElems; e++)
                       if (FULL || (col_ok && k0 + (e >> 2) * 8 + (e & 3) < p.I))
                         image[blk_base[a][b] + ((e >> 2) * 8 + (e & 3)) * p.h.BN] =
                             cur[e] + acc[a][b][e] * p.scale;
@@ -1149,37 +1200,10 @@ struct GemmKernel {
         scatter(p.scatter);
       }
     } else {
-      if constexpr (WK > 1) {
-        // add up the groups' accumulators: groups 1.. park theirs in the dead operand stages,
-        // group 0 adds them (fixed order) and stores the tile
-        float* park = reinterpret_cast<float*>(&sm);
-        static_assert(sizeof(float) * (WK - 1) * TI * TJ <= sizeof(Smem), "the accumulators must fit the stages");
-        __syncthreads();   // every wavefront is done reading the stages
-        const int slot = ((wave % (WI * WJ)) * MI * MJ) * 16 * 64 + lane;
-        if (wave_k > 0) {
-#pragma unroll
-          for (int a = 0; a < MI; a++)
-#pragma unroll
-            for (int b = 0; b < MJ; b++)
-#pragma unroll
-              for (int e = 0; e < 16; e++)
-                park[(wave_k - 1) * TI * TJ + slot + ((a * MJ + b) * 16 + e) * 64] = acc[a][b][e];
-        }
-        __syncthreads();
-        if (wave_k == 0) {
-#pragma unroll
-          for (int g = 1; g < WK; g++)
-#pragma unroll
-            for (int a = 0; a < MI; a++)
-#pragma unroll
-              for (int b = 0; b < MJ; b++)
-#pragma unroll
-                for (int e = 0; e < 16; e++)
-                  acc[a][b][e] += park[(g - 1) * TI * TJ + slot + ((a * MJ + b) * 16 + e) * 64];
-        }
-      }
-      // (of several groups of wavefronts that shared the R steps, the first holds the sums and stores)
-      const bool writer = wave_k == 0;   // (uniform)
+      merge_groups();
+      // (true in every wavefront, which the compiler does not know: the branches keep the passes below apart —
+      //  in one straight line they are scheduled into each other and the 256 tile spills 251 registers)
+      const bool writer = wave_k < WK;   // (uniform)
       float out_scale = p.scale;
       const T* __restrict__ gBias = static_cast<const T*>(p.bias);
       // optional bias of this lane's columns, added in fp32 before the single rounding
@@ -1198,19 +1222,18 @@ struct GemmKernel {
         // so the sum does not depend on who came last; nobody waits for anybody.
         float* __restrict__ gP = p.partial + (size_t)by * (size_t)p.I * (size_t)p.J;
         const bool finishing = p.finish != nullptr;   // (uniform)
-        if (writer) {
+        if (writer)
 #pragma unroll
-          for (int a = 0; a < MI; a++) {
+        for (int a = 0; a < MI; a++) {
 #pragma unroll
-            for (int e = 0; e < 16; e++) {
-              const int row = i0 + blk_i(a) + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+          for (int e = 0; e < kElems; e++) {
+            const int row = i0 + blk_i(a) + block_row(e);
 #pragma unroll
-              for (int b = 0; b < MJ; b++) {
-                const int col = j0 + blk_j(b) + (lane & 31);
-                if (FULL || (row < p.I && col < p.J)) {
-                  if (finishing) store_agent_f32(gP + (size_t)row * p.J + col, acc[a][b][e] * p.scale);
-                  else gP[(size_t)row * p.J + col] = acc[a][b][e] * p.scale;
-                }
+            for (int b = 0; b < MJ; b++) {
+              const int col = j0 + blk_j(b) + (lane & 31);
+              if (FULL || (row < p.I && col < p.J)) {
+                if (finishing) store_agent_f32(gP + (size_t)row * p.J + col, acc[a][b][e] * p.scale);
+                else gP[(size_t)row * p.J + col] = acc[a][b][e] * p.scale;
               }
             }
           }
@@ -1218,7 +1241,7 @@ struct GemmKernel {
         if (!finishing) return;
         const int slices = (int)gridDim.y;
         unsigned* counter = p.finish + (size_t)ti * (size_t)p.tiles_j + tj;
-        int* arrived = reinterpret_cast<int*>(&sm);   // (the stages are dead)
+        int* arrived = sm.off;   // (the offsets are no longer read)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part of the plane is where the others will look
         __syncthreads();
         if (tid == 0) *arrived = (int)__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1234,36 +1257,37 @@ struct GemmKernel {
             const int col = j0 + blk_j(b) + (lane & 31);
             // (half a block at a time: the other slices' values of eight rows are fetched before the first is
             //  used — a whole block's would cost registers that the two-workgroup forms do not have)
+            constexpr int kHalf = kElems < 8 ? kElems : 8;
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-              float v[kFinishSlices][8];
+            for (int h = 0; h < kElems / kHalf; h++) {
+              float v[kFinishSlices][kHalf];
 #pragma unroll
               for (int sl = 0; sl < kFinishSlices; sl++) {
                 if (sl < slices && sl != by) {   // (uniform)
 #pragma unroll
-                  for (int e = 0; e < 8; e++) {
-                    const int row = i0 + blk_i(a) + (h * 2 + (e >> 2)) * 8 + (lane >> 5) * 4 + (e & 3);
+                  for (int e = 0; e < kHalf; e++) {
+                    const int row = i0 + blk_i(a) + block_row(h * kHalf + e);
                     v[sl][e] = (FULL || (row < p.I && col < p.J)) ? load_agent_f32(p.partial + (size_t)sl * plane + (size_t)row * p.J + col) : 0.f;
                   }
                 }
               }
-              float sum[8];
+              float sum[kHalf];
 #pragma unroll
-              for (int e = 0; e < 8; e++) sum[e] = 0.f;
+              for (int e = 0; e < kHalf; e++) sum[e] = 0.f;
 #pragma unroll
               for (int sl = 0; sl < kFinishSlices; sl++) {
                 if (sl == by) {
 #pragma unroll
-                  for (int e = 0; e < 8; e++) sum[e] += __fmul_rn(acc[a][b][h * 8 + e], p.scale);   // (the product as it was stored: not fused into the add)
+                  for (int e = 0; e < kHalf; e++) sum[e] += __fmul_rn(acc[a][b][h * kHalf + e], p.scale);   // (the product as it was stored: not fused into the add)
                 } else if (sl < slices) {
 #pragma unroll
-                  for (int e = 0; e < 8; e++) sum[e] += v[sl][e];
+                  for (int e = 0; e < kHalf; e++) sum[e] += v[sl][e];
                 }
               }
               // (the bias joins the fp32 sum as in the second kernel: an add of its own, rounded to fp32,
               //  not part of a fused multiply-add that rounds straight to the output type)
 #pragma unroll
-              for (int e = 0; e < 8; e++) acc[a][b][h * 8 + e] = __fadd_rn(sum[e], bias[b]);
+              for (int e = 0; e < kHalf; e++) acc[a][b][h * kHalf + e] = __fadd_rn(sum[e], bias[b]);
             }
           }
         }
@@ -1281,8 +1305,8 @@ struct GemmKernel {
 #pragma unroll
         for (int a = 0; a < MI; a++) {
 #pragma unroll
-          for (int e = 0; e < 16; e++) {
-            const int row = i0 + blk_i(a) + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+          for (int e = 0; e < kElems; e++) {
+            const int row = i0 + blk_i(a) + block_row(e);
 #pragma unroll
             for (int b = 0; b < MJ; b++) {
               const int col = j0 + blk_j(b) + (lane & 31);
@@ -1303,8 +1327,12 @@ struct GemmKernel {
   }
 };
 
+// Wavefronts per SIMD that the register allocation has to leave room for: the workgroup's own — and two
+// workgroups' for the sixteen-wavefront form with two stages, which shares its compute unit.
+constexpr int gemm_waves_per_simd(int waves, int stages) { return waves == 16 && stages == 2 ? 8 : (waves + 3) / 4; }
+
 template <typename T, int OP, int TI, int TJ, int WI, int WJ, int NSTAGE, bool FULL, bool COLSUM, bool CLAMP, int WK = 1>
-__global__ __launch_bounds__(64 * WI * WJ * WK) void rz_gemm_kernel(GemmParams p) {
+__global__ __launch_bounds__(64 * WI * WJ * WK, gemm_waves_per_simd(WI * WJ * WK, NSTAGE)) void rz_gemm_kernel(GemmParams p) {
   typedef GemmKernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK> K;
   extern __shared__ __attribute__((aligned(16))) unsigned char rz_smem_raw[];
   K::run(p, *reinterpret_cast<typename K::Smem*>(rz_smem_raw));

@@ -82,38 +82,44 @@ static hipError_t launch_tile(GemmParams p, const WeightGradPlan* plan, const Sp
   // carry full pointers (the step is the same for both fp32 forms).
   const bool far = sizeof(T) == 4 && OP != kWeightGrad &&
                    ((unsigned long long)p.h.range + (unsigned long long)p.h.BK * (unsigned long long)p.h.BN) * sizeof(T) > 0xffffffffull;
-  if (far) {
+  if constexpr (sizeof(T) == 4) if (far) {
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false>::TR) return hipErrorInvalidValue;
     return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, false, WK>(p, plan, split, stream);
   }
-  if (form.full) {
+  // (the 16-bit 64 tile of four wavefronts serves rows shorter than a 16-byte piece only)
+  constexpr bool kCheckedOnly = sizeof(T) == 2 && TILE == 64 && WK == 1;
+  if constexpr (!kCheckedOnly) if (form.full) {
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true>::TR) return hipErrorInvalidValue;
     return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true, COLSUM, false, WK>(p, plan, split, stream);
   }
-  if constexpr (NSTAGE == 2 && (sizeof(T) == 4 || TILE >= 128)) {
+  constexpr bool kSixteen = WI * WJ * WK == 16;
+  if constexpr (NSTAGE >= 2 && !kCheckedOnly) {
     if (form.clamp) {
       if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, false, true, WK>::TR) return hipErrorInvalidValue;
       return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, true, WK>(p, plan, split, stream);
     }
   }
-  if (form.clamp || form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false>::TR) return hipErrorInvalidValue;
-  return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, false, WK>(p, plan, split, stream);
+  if constexpr (kSixteen) {   // (always directly staged)
+    return hipErrorInvalidValue;
+  } else {
+    if (form.full || form.clamp || form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false>::TR) return hipErrorInvalidValue;
+    return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, false, WK>(p, plan, split, stream);
+  }
 }
 
-template <typename T, int TILE, int WI, int WJ, int NSTAGE, int WK = 1>
-static hipError_t launch_op(int op, GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
+template <typename T, int OP, int TILE, int WI, int WJ, int NSTAGE, int WK = 1>
+static hipError_t launch_op(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
                             const KernelForm& form, hipStream_t stream) {
-  switch (op) {
-    case kForward: return launch_tile<T, kForward, TILE, WI, WJ, NSTAGE, false, WK>(p, plan, split, form, stream);
-    case kInputGrad: return launch_tile<T, kInputGrad, TILE, WI, WJ, NSTAGE, false, WK>(p, plan, split, form, stream);
-    case kWeightGrad:
-      if constexpr (WK == 1) {
-        // with a column-sum target the kernel also produces the bias gradient's partial sums
-        if (p.colsum != nullptr) return launch_tile<T, kWeightGrad, TILE, WI, WJ, NSTAGE, true>(p, plan, split, form, stream);
-        return launch_tile<T, kWeightGrad, TILE, WI, WJ, NSTAGE>(p, plan, split, form, stream);
-      }
-      return hipErrorInvalidValue;
-    default: return hipErrorInvalidValue;
+  if constexpr (OP == kWeightGrad) {
+    if constexpr (WK > 1 && sizeof(T) == 4) {
+      return hipErrorInvalidValue;   // (groups of wavefronts share an R step in the fp32 store kernels only)
+    } else {
+      // with a column-sum target the kernel also produces the bias gradient's partial sums
+      if (p.colsum != nullptr) return launch_tile<T, OP, TILE, WI, WJ, NSTAGE, true, WK>(p, plan, split, form, stream);
+      return launch_tile<T, OP, TILE, WI, WJ, NSTAGE, false, WK>(p, plan, split, form, stream);
+    }
+  } else {
+    return launch_tile<T, OP, TILE, WI, WJ, NSTAGE, false, WK>(p, plan, split, form, stream);
   }
 }
 
@@ -123,33 +129,37 @@ static hipError_t launch_op(int op, GemmParams p, const WeightGradPlan* plan, co
 //        eight of 64 x 32 when there is about one workgroup per compute unit; tuning.stages = 1
 //        selects a single-stage form that leans on several workgroups per compute unit
 //        instead of a pipeline (tuning aid)
-//    64:  64 x  64, four wavefronts of 32 x 32, for problems with few tiles; fp32 forward /
-//        input-grad: eight, in two groups that share every R step between them
+//    64:  64 x  64, for problems with few tiles: 16-bit sixteen wavefronts of 32 x 32 in four groups that
+//        share every R step between them; fp32 forward / input-grad eight, in two such groups; fp32
+//        weight-grad, and 16-bit rows shorter than a 16-byte piece, four
 //    32:  32 x  64 (fp32 forward / input-grad whose rows would leave a 64-row tile at most half full): four wavefronts of 32 x 32 in two such groups
-template <typename T>
-static hipError_t launch_gemm_t(int op, GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
+template <typename T, int OP>
+static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
                                 const rz_tuning& tuning, hipStream_t stream) {
-  const bool wg = op == kWeightGrad && plan != nullptr;
+  const bool wg = OP == kWeightGrad && plan != nullptr;
   const bool cut = !wg && split != nullptr && split->splits > 1;
   const int tile = wg ? plan->tile : (split != nullptr ? split->tile : pick_tile(p.I, p.J, (int)sizeof(T), tuning));
   const int chunk = wg ? plan->r_chunk : (cut ? split->r_chunk : p.R);
   const long long workgroups = wg ? plan->workgroups : tile_count(p.I, p.J, tile) * (cut ? split->splits : 1);
-  const KernelForm form = kernel_form(op, p.I, p.J, p.R, chunk, tile, workgroups, (int)sizeof(T), tuning);
-  switch (form.tile * 100 + form.waves * 10 + form.stages) {
-    case 25682: return launch_op<T, 256, 2, 4, 2>(op, p, plan, split, form, stream);
-    case 6442: return launch_op<T, 64, 2, 2, 2>(op, p, plan, split, form, stream);
-    case 6482:   // fp32 forward / input-grad: two groups of four wavefronts share every R step
-      if constexpr (sizeof(T) == 4) return launch_op<T, 64, 2, 2, 2, 2>(op, p, plan, split, form, stream);
+  const KernelForm form = kernel_form(OP, p.I, p.J, p.R, chunk, tile, workgroups, (int)sizeof(T), tuning);
+  switch (form.tile * 1000 + form.waves * 10 + form.stages) {
+    case 256082: return launch_op<T, OP, 256, 2, 4, 2>(p, plan, split, form, stream);
+    case 64042: return launch_op<T, OP, 64, 2, 2, 2>(p, plan, split, form, stream);
+    case 64164:   // 16-bit, at most one workgroup per compute unit: four groups of four wavefronts share every R step
+      if constexpr (sizeof(T) == 2) return launch_op<T, OP, 64, 2, 2, 4, 4>(p, plan, split, form, stream);
       return hipErrorInvalidValue;
-    case 3242:   // fp32 forward / input-grad, rows in 32s: 32 x 64, two groups of two wavefronts
-      if constexpr (sizeof(T) == 4) {
-        if (op == kForward) return launch_tile<T, kForward, 32, 1, 2, 2, false, 2, 64>(p, plan, split, form, stream);
-        if (op == kInputGrad) return launch_tile<T, kInputGrad, 32, 1, 2, 2, false, 2, 64>(p, plan, split, form, stream);
-      }
+    case 64162:   // ... more of them: two LDS stages
+      if constexpr (sizeof(T) == 2) return launch_op<T, OP, 64, 2, 2, 2, 4>(p, plan, split, form, stream);
       return hipErrorInvalidValue;
-    case 12841: return launch_op<T, 128, 2, 2, 1>(op, p, plan, split, form, stream);
-    case 12882: return launch_op<T, 128, 2, 4, 2>(op, p, plan, split, form, stream);
-    case 12842: return launch_op<T, 128, 2, 2, 2>(op, p, plan, split, form, stream);
+    case 64082:   // fp32 forward / input-grad: two groups of four wavefronts share every R step
+      if constexpr (sizeof(T) == 4) return launch_op<T, OP, 64, 2, 2, 2, 2>(p, plan, split, form, stream);
+      return hipErrorInvalidValue;
+    case 32042:   // fp32 forward / input-grad, rows in 32s: 32 x 64, two groups of two wavefronts
+      if constexpr (sizeof(T) == 4 && OP != kWeightGrad) return launch_tile<T, OP, 32, 1, 2, 2, false, 2, 64>(p, plan, split, form, stream);
+      return hipErrorInvalidValue;
+    case 128041: return launch_op<T, OP, 128, 2, 2, 1>(p, plan, split, form, stream);
+    case 128082: return launch_op<T, OP, 128, 2, 4, 2>(p, plan, split, form, stream);
+    case 128042: return launch_op<T, OP, 128, 2, 2, 2>(p, plan, split, form, stream);
     default: return hipErrorInvalidValue;
   }
 }

@@ -1,0 +1,9 @@
+// Instantiation of the input-grad contraction kernels for element type f16_t.
+#include "rz_gemm_inst.h"
+
+namespace rz {
+hipError_t launch_input_grad_f16(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning,
+                        hipStream_t stream) {
+  return launch_gemm_t<f16_t, kInputGrad>(p, plan, split, tuning, stream);
+}
+}  // namespace rz

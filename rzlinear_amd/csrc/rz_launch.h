@@ -40,11 +40,11 @@ static constexpr int kComputeUnits = 256;
 static constexpr int kTargetWorkgroups = 1024;
 
 // Contracted elements per kernel step that every slice of a cut contraction must be a multiple
-// of: 128 bytes, and 256 for the 16-bit 128 tile, whose eight-wavefront form takes 256-byte steps
+// of: 128 bytes, and 256 for the 16-bit 128 and 64 tiles, whose eight- and sixteen-wavefront forms take 256-byte steps
 // (a slice that began in the middle of such a step would start between two hashed tiles).
 static inline int slice_unit(int tile, int elem_bytes, bool weight_grad = false) {
   if (elem_bytes == 4 && tile <= 64 && !weight_grad) return 64;   // (fp32 forward / input-grad, 64 and 32 x 64 tiles: 256-byte steps as well)
-  return ((tile == 128 && elem_bytes == 2) ? 256 : 128) / elem_bytes;
+  return ((tile <= 128 && elem_bytes == 2) ? 256 : 128) / elem_bytes;
 }
 
 // Tile codes: 64, 128, 256 are square C tiles; 32 stands for the 32 x 64 tile of the fp32 forward /
@@ -610,7 +610,9 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
     // (the 32 x 64 tile: fp32 only, and only where 64-row tiles would end in a tile at most half full —
     //  K = N = 10240: M = 96 259 -> 232 us, M = 160 428 -> 353 us, M = 288 668 -> 620 us)
     if (tile == 32 && !forced && (elem_bytes != 4 || (I > 32 && (I - 1) % 64 >= 32))) continue;
-    const int TR = slice_unit(tile, elem_bytes);
+    // (depth 2: an override's number of slices that whole steps of the 16-bit 64 tile cannot make may be cut at
+    //  half of one: the bounds-checked form takes those)
+    const int TR = slice_unit(tile, elem_bytes) / (depth == 2 && tile == 64 && elem_bytes == 2 ? 2 : 1);
     const long long tiles = tile_count(I, J, tile);
     const int r_steps = (R + TR - 1) / TR;
     const double useful = (double)I * (double)J / ((double)tiles * tile * tile_cols(tile));
@@ -662,6 +664,7 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
     const SplitPlan w = plan_split(I, J, R, elem_bytes, whole_only, 1);
     if (w.est_us <= 14.0) return w;
   }
+  if (best.tile == 0 && t.split > 0 && depth < 2) return plan_split(I, J, R, elem_bytes, t, 2);
   if (best.tile == 0 && t.split > 0) {   // (no cut comes out at exactly that many slices: the library's own choice)
     rz_tuning free_cut = t;
     free_cut.split = 0;
@@ -693,33 +696,43 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
   // four-wavefront form does less LDS traffic per flop
   // 64 tile: four wavefronts; fp32 forward / input-grad take eight (two groups that share every R
   // step: a second wavefront per SIMD keeps the MFMA pipe fed while the first waits for LDS)
-  f.waves = tile == 256 ? 8
-            : tile == 32 ? 4
-            : tile == 64 ? ((elem_bytes == 4 && op != kWeightGrad) ? 8 : 4)
-                         : (f.stages == 1 ? 4 : (workgroups <= kComputeUnits * 3 / 2 ? 8 : 4));
-  // (32-bit: every two-stage form stages directly; 16-bit: the tiles of 128 and more)
-  const bool direct_capable = f.stages == 2 && (elem_bytes == 4 || tile >= 128);
+  // (32-bit: every two-stage form stages directly; 16-bit too)
+  const bool direct_capable = f.stages == 2;
+  // 64 tile, 16-bit: sixteen wavefronts in four groups that share every 256-byte step — a problem of few
+  // tiles leaves most compute units idle and the others waiting for memory, and four wavefronts cannot keep
+  // enough loads in flight.  Up to one workgroup per compute unit, four LDS stages (128 KB in flight); beyond
+  // that, two, so that two workgroups share a compute unit.
+  const bool many64 = tile == 64 && elem_bytes == 2;
+  const int waves128 = f.stages == 1 ? 4 : (workgroups <= kComputeUnits * 3 / 2 ? 8 : 4);
   const int step_plain = elem_bytes == 4 ? slice_unit(tile, elem_bytes, op == kWeightGrad) : 128 / elem_bytes;
-  const int step_direct = (direct_capable && elem_bytes == 2 && tile == 128 && f.waves == 8) ? 256 / elem_bytes : step_plain;
+  const int step_direct = (direct_capable && elem_bytes == 2 && ((tile == 128 && waves128 == 8) || many64)) ? 256 / elem_bytes : step_plain;
   f.full = (I % tile == 0) && (J % tile_cols(tile) == 0) && (R % step_direct == 0) && (chunk % step_direct == 0);
   // a plain operand's rows must hold at least one 16-byte piece (a piece that straddles the end of a
   // row is handled in the kernel; a row shorter than a piece is not)
   const int vec = 16 / elem_bytes;
-  const bool pieces_ok = op == kWeightGrad ? (I >= vec && J >= vec) : R >= vec;
+  const bool pieces_ok = (op == kWeightGrad ? (I >= vec && J >= vec) : R >= vec) && (chunk >= R || chunk % step_direct == 0);
   f.clamp = !f.full && direct_capable && pieces_ok && t.clamp != -1;
   f.step = (f.full || f.clamp) ? step_direct : step_plain;
+  f.waves = tile == 256 ? 8
+            : tile == 32 ? 4
+            : tile == 64 ? ((many64 && (f.full || f.clamp)) ? 16 : (elem_bytes == 4 && op != kWeightGrad) ? 8 : 4)
+                         : waves128;
+  if (f.waves == 16) f.stages = workgroups <= kComputeUnits ? 4 : 2;
   return f;
 }
 
-// Fills in the tiling fields of `p` and enqueues the kernel for `op` on `stream`; weight-grad
+// Fill in the tiling fields of `p` and enqueue the kernel of one op and element type on `stream`; weight-grad
 // takes its plan (tile, split of M, scatter mode) from `plan`, the others ignore it.
 // (forward / input-grad take tile and split from `split`, or pick a tile and do not split).
-hipError_t launch_gemm_f32(int op, GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
-                           const rz_tuning& tuning, hipStream_t stream);
-hipError_t launch_gemm_bf16(int op, GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
-                            const rz_tuning& tuning, hipStream_t stream);
-hipError_t launch_gemm_f16(int op, GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
-                           const rz_tuning& tuning, hipStream_t stream);
+hipError_t launch_forward_f32(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning, hipStream_t stream);
+hipError_t launch_input_grad_f32(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning, hipStream_t stream);
+hipError_t launch_weight_grad_f32(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning, hipStream_t stream);
+hipError_t launch_forward_bf16(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning, hipStream_t stream);
+hipError_t launch_input_grad_bf16(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning, hipStream_t stream);
+hipError_t launch_weight_grad_bf16(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning, hipStream_t stream);
+hipError_t launch_forward_f16(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning, hipStream_t stream);
+hipError_t launch_input_grad_f16(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning, hipStream_t stream);
+hipError_t launch_weight_grad_f16(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning, hipStream_t stream);
 
 struct WindowParams;
 // Enqueues the windowed weight-grad kernel; p.window and the tile grid must come from plan_window.

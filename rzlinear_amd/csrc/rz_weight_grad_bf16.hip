@@ -1,0 +1,9 @@
+// Instantiation of the weight-grad contraction kernels for element type bf16_t.
+#include "rz_gemm_inst.h"
+
+namespace rz {
+hipError_t launch_weight_grad_bf16(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning,
+                        hipStream_t stream) {
+  return launch_gemm_t<bf16_t, kWeightGrad>(p, plan, split, tuning, stream);
+}
+}  // namespace rz

@@ -1,0 +1,8 @@
+// Instantiation of the window kernel for element type f16_t.
+#include "rz_gemm_inst.h"
+
+namespace rz {
+hipError_t launch_window_f16(const WindowParams& p, int windows, hipStream_t stream) {
+  return launch_window_t<f16_t>(p, windows, stream);
+}
+}  // namespace rz
