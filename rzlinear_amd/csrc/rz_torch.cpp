@@ -9,8 +9,8 @@
 //
 // `apply` serves the plain case — dense GPU tensors of one device and dtype, a [H] contiguous hashed_weight, the
 // eight constants as an int32 CPU tensor, an ordinary eager call.  For everything else (tensor subclasses,
-// functorch, tracing, an empty batch, arguments that the launchers refuse) it returns None before it has
-// done anything, and the caller goes through the Python Function, whose checks and errors are the
+// functorch, tracing, forward-mode tangents, an empty batch, arguments that the launchers refuse) it returns None before
+// it has done anything, and the caller goes through the Python Function, whose checks and errors are the
 // reference's.
 #include <Python.h>
 
@@ -27,8 +27,8 @@
 #include <torch/csrc/jit/frontend/tracer.h>
 
 #include <array>
-#include <atomic>
 #include <map>
+#include <memory>
 #include <mutex>
 
 #include "../../include/rzlinear.h"
@@ -54,7 +54,10 @@ struct Library {
 Library lib;
 PyObject* plan_provider = nullptr;    // Python: (K, N, H, BK, BN, constants, levels, device index) -> plan tensor
 PyObject* status_check = nullptr;     // Python: raises for a non-zero status
-std::atomic<const rz_tuning*> tuning{nullptr};   // what the Python side's `tuning` context has set (tests, benchmarks)
+// What the Python side's `tuning` context has set (tests, benchmarks): a copy, which a call that is under way
+// in another thread keeps alive.
+std::shared_ptr<const rz_tuning> tuning_in_force;
+std::shared_ptr<const rz_tuning> current_tuning() { return std::atomic_load(&tuning_in_force); }
 
 struct Geometry {
   int K, N, H, BK, BN;
@@ -72,13 +75,17 @@ int dtype_code(at::ScalarType t) {
   }
 }
 
-// a dense GPU tensor that nothing wraps (no subclass, functorch level, lazy conjugate ...)
-bool plain_gpu(const Tensor& t) {
+// a dense tensor that nothing wraps (no subclass, functorch level, lazy conjugate ...)
+bool plain(const Tensor& t) {
   constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot, c10::DispatchKey::Functionalize,
                                          c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
                                          c10::DispatchKey::Conjugate, c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
-  return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(wrapped);
+  return t.defined() && t.layout() == at::kStrided && !t.key_set().has_any(wrapped);
 }
+bool plain_gpu(const Tensor& t) { return plain(t) && t.is_cuda(); }
+
+// a forward-mode tangent rides on it (the Function has no jvp and says so)
+bool has_tangent(const Tensor& t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
 
 // unit column stride (copied only if it has to be) and the row pitch
 Tensor rows(const Tensor& t, int64_t* ld) {
@@ -149,7 +156,8 @@ int forward(const Geometry& g, const Tensor& input, const Tensor& hw, const Tens
   const Tensor x = rows(input, &ldx);
   const int M = (int)x.size(0), code = dtype_code(x.scalar_type());
   *output = empty({M, g.N}, x);
-  const rz_tuning* t = tuning.load(std::memory_order_acquire);
+  const std::shared_ptr<const rz_tuning> keep = current_tuning();
+  const rz_tuning* t = keep.get();
   // (skinny problems cut the contraction and need a scratch buffer for the slices)
   const size_t need = lib.forward_workspace(M, g.K, g.N, g.H, g.BK, g.BN, code, t);
   const at::DataPtr ws = scratch(need);
@@ -160,7 +168,8 @@ int forward(const Geometry& g, const Tensor& input, const Tensor& hw, const Tens
 Tensor input_grad(const Geometry& g, const Tensor& dy, int64_t lddy, const Tensor& hw) {
   const int M = (int)dy.size(0), code = dtype_code(dy.scalar_type());
   Tensor dx = empty({M, g.K}, dy);
-  const rz_tuning* t = tuning.load(std::memory_order_acquire);
+  const std::shared_ptr<const rz_tuning> keep = current_tuning();
+  const rz_tuning* t = keep.get();
   const size_t need = lib.input_grad_workspace(M, g.K, g.N, g.H, g.BK, g.BN, code, t);
   const at::DataPtr ws = scratch(need);
   check(lib.input_grad(dy.data_ptr(), hw.data_ptr(), dx.data_ptr(), ws.get(), need, M, g.K, g.N, g.H, g.BK, g.BN, g.R,
@@ -176,7 +185,8 @@ void weight_grad(const Geometry& g, const Tensor& input, const Tensor& dy, int64
   unsigned flags = accumulate ? RZ_WG_ACCUMULATE : 0u;
   if (out.scalar_type() == at::kFloat) flags |= RZ_WG_DHW_F32;
   const int with_dbias = dbias.defined() ? 1 : 0;
-  const rz_tuning* t = tuning.load(std::memory_order_acquire);
+  const std::shared_ptr<const rz_tuning> keep = current_tuning();
+  const rz_tuning* t = keep.get();
   // (a layer plan: where the library would work by windows of dHW, or fold stored tiles into it)
   Tensor plan;
   if (with_plans) {
@@ -198,7 +208,7 @@ void weight_grad(const Geometry& g, const Tensor& input, const Tensor& dy, int64
 
 // ---- the autograd node --------------------------------------------------------------------------
 struct RzLinearNode : public Node {
-  SavedVariable input, hashed_weight;
+  SavedVariable input, hashed_weight, random_numbers;   // (what the Function saves, whichever gradients are wanted)
   Geometry g;
   c10::SmallVector<int64_t, 2> output_sizes;
   at::TensorOptions output_options;
@@ -207,8 +217,19 @@ struct RzLinearNode : public Node {
   std::string name() const override { return "RzLinearFunctionBackward"; }
 
   void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
     input.reset_data();
     hashed_weight.reset_data();
+    random_numbers.reset_data();
+  }
+
+  // What a saved-tensor hook hands back, and a gradient, may be anything: the pointers below go straight to kernels.
+  void require(const Tensor& t, const char* name, int64_t rows, int64_t cols, const Tensor& grad) const {
+    TORCH_CHECK(plain_gpu(t), "rzlinear_amd: ", name, " of the backward must be a plain dense tensor on a ROCm GPU");
+    TORCH_CHECK(t.device() == grad.device(), "rzlinear_amd: tensors on different devices (", t.device(), ", ", grad.device(), ")");
+    TORCH_CHECK_TYPE(t.scalar_type() == grad.scalar_type(), name, " is ", t.scalar_type(), " but output_grad is ", grad.scalar_type());
+    TORCH_CHECK_VALUE(cols < 0 ? (t.dim() == 1 && t.size(0) == rows) : (t.dim() == 2 && t.size(0) == rows && t.size(1) == cols),
+                      "rzlinear_amd: ", name, " of the backward has shape ", t.sizes());
   }
 
   // The gradient buffer of a parameter whose weight gradient is added in the kernels: its main_grad if it
@@ -243,18 +264,26 @@ struct RzLinearNode : public Node {
     const bool need_input = task_should_compute_output(0), need_weight = task_should_compute_output(1),
                need_bias = task_should_compute_output(2);
     variable_list result(3);
+    Tensor x, hw;
+    {
+      std::lock_guard<std::mutex> lock(mutex_);   // (another thread's backward through this graph may release them)
+      x = input.unpack();
+      hw = hashed_weight.unpack();
+      random_numbers.unpack();   // (freed, or changed in place since the forward: an error, as for the others)
+    }
     Tensor grad = grads[0].defined() ? grads[0] : at::zeros(output_sizes, output_options);
+    require(grad, "output_grad", output_sizes[0], g.N, grad);
+    if (need_input) require(hw, "hashed_weight", g.H, -1, grad);
+    if (need_weight) require(x, "input", output_sizes[0], g.K, grad);
     at::DeviceGuard guard(grad.device());
     int64_t lddy;
     const Tensor dy = rows(grad, &lddy);
-    if (need_input) result[0] = input_grad(g, dy, lddy, hashed_weight.unpack().contiguous());   // (enqueued first, like the reference)
+    if (need_input) result[0] = input_grad(g, dy, lddy, hw.contiguous());   // (enqueued first, like the reference)
     if (need_weight) {   // (with a bias: one pass over dy yields both gradients)
-      const Tensor x = input.unpack();
       if (need_bias) result[2] = empty({g.N}, dy);
       bool accumulate = false;
       Tensor out;
       if (fuse_grad_accumulation) {
-        Tensor hw = hashed_weight.unpack();
         out = fused_target(hw, &accumulate);
       } else {
         out = result[1] = empty({g.H}, dy);
@@ -281,7 +310,8 @@ PyObject* apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor& hw = THPVariable_Unpack(args[1]);
   const Tensor& r = THPVariable_Unpack(args[2]);
   const Tensor bias = has_bias ? THPVariable_Unpack(args[7]) : Tensor();
-  if (!plain_gpu(x) || !plain_gpu(hw) || (has_bias && !plain_gpu(bias)) || lib.forward == nullptr) Py_RETURN_NONE;
+  if (!plain_gpu(x) || !plain_gpu(hw) || (has_bias && !plain_gpu(bias)) || !plain(r) || lib.forward == nullptr) Py_RETURN_NONE;
+  if (has_tangent(x) || has_tangent(hw) || has_tangent(bias)) Py_RETURN_NONE;
   if (c10::impl::dispatch_mode_enabled() || torch::jit::tracer::isTracing()) Py_RETURN_NONE;
   const auto type = x.scalar_type();
   if (dtype_code(type) < 0 || hw.scalar_type() != type || hw.device() != x.device() || x.dim() != 2 || hw.dim() != 1 || !hw.is_contiguous()) Py_RETURN_NONE;
@@ -303,7 +333,7 @@ PyObject* apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
   }
   const int64_t M = x.size(0), K = x.size(1), N = v[0], H = hw.size(0), BK = v[1], BN = v[2];
   if (M < 1 || M > INT32_MAX || K < 1 || K > INT32_MAX || N < 1 || N > INT32_MAX || H > INT32_MAX || BK < 1 || BK > 256 || BN < 1 || BN > 256 || H <= BK * BN) Py_RETURN_NONE;
-  if (has_bias && (bias.scalar_type() != type || bias.device() != x.device() || bias.numel() != N || !bias.is_contiguous())) Py_RETURN_NONE;
+  if (has_bias && (bias.scalar_type() != type || bias.device() != x.device() || bias.dim() != 1 || bias.numel() != N || !bias.is_contiguous())) Py_RETURN_NONE;
   const int fuse = PyObject_IsTrue(args[8]), with_plans = PyObject_IsTrue(args[9]);
   if (fuse < 0 || with_plans < 0) return nullptr;
 
@@ -318,9 +348,9 @@ PyObject* apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
       if (status == RZ_OK && torch::autograd::compute_requires_grad(x, hw, bias)) {
         auto node = std::shared_ptr<RzLinearNode>(new RzLinearNode(), torch::autograd::deleteNode);
         node->set_next_edges(torch::autograd::collect_next_edges(x, hw, bias));
-        const bool want_x = x.requires_grad(), want_hw = hw.requires_grad();
-        if (want_hw) node->input = SavedVariable(x, false);
-        if (want_x || (want_hw && fuse)) node->hashed_weight = SavedVariable(hw, false);
+        node->input = SavedVariable(x, false);
+        node->hashed_weight = SavedVariable(hw, false);
+        node->random_numbers = SavedVariable(r, false);
         node->g = g;
         node->output_sizes = {M, N};
         node->output_options = x.options();
@@ -374,7 +404,8 @@ PyObject* bind(PyObject*, PyObject* args) {
 PyObject* set_tuning(PyObject*, PyObject* arg) {
   void* p = PyLong_AsVoidPtr(arg);
   if (p == nullptr && PyErr_Occurred()) return nullptr;
-  tuning.store(static_cast<const rz_tuning*>(p), std::memory_order_release);
+  std::atomic_store(&tuning_in_force, p == nullptr ? std::shared_ptr<const rz_tuning>()
+                                                   : std::make_shared<const rz_tuning>(*static_cast<const rz_tuning*>(p)));
   Py_RETURN_NONE;
 }
 

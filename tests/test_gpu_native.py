@@ -1,0 +1,152 @@
+"""The native host path of the layer (csrc/rz_torch.cpp) against the Python Function: the same bits for every
+layout it accepts, and the same refusals — what the Function does not support, or would notice, the native
+node must not let through."""
+import numpy as np
+import pytest
+import torch
+from torch.autograd import forward_ad
+
+from helpers import SEED_CONSTANTS
+
+pytestmark = pytest.mark.gpu
+
+K, N, H, TILE = 192, 320, 9000, (32, 64)
+R = torch.tensor(SEED_CONSTANTS[1024], dtype=torch.int32)
+
+
+def _functions():
+    from rzlinear_amd.RzLinearFunction import RzLinearFunction
+
+    class InPython(RzLinearFunction):   # (a subclass never takes the native path)
+        pass
+
+    return RzLinearFunction, InPython
+
+
+def _call(function, x, hw, bias=None, fuse=False):
+    return function.apply(x, hw, R, N, 1, 0.5, *TILE, bias, fuse)
+
+
+def _inputs(dtype=torch.float32, M=37):
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn((M, K), generator=g).to(dtype).cuda()
+    hw = ((torch.rand((H,), generator=g) * 2 - 1) / K ** 0.5).to(dtype).cuda()
+    bias = torch.randn((N,), generator=g).to(dtype).cuda()
+    dy = torch.randn((M, N), generator=g).to(dtype).cuda()
+    return x, hw, bias, dy
+
+
+def _transposed(t):
+    return t.t().contiguous().t()
+
+
+def _pitched(t):
+    wide = torch.zeros((t.shape[0], t.shape[1] + 5), dtype=t.dtype, device=t.device)
+    wide[:, 3:3 + t.shape[1]] = t
+    return wide[:, 3:3 + t.shape[1]]
+
+
+def _every_other_row(t):
+    wide = torch.zeros((2 * t.shape[0], t.shape[1]), dtype=t.dtype, device=t.device)
+    wide[::2] = t
+    return wide[::2]
+
+
+def _one_row_repeated(t):
+    return t[:1].expand(t.shape[0], t.shape[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=str)
+@pytest.mark.parametrize("layout", [lambda t: t, _transposed, _pitched, _every_other_row, _one_row_repeated],
+                         ids=["plain", "transposed", "pitched", "every_other_row", "expanded"])
+def test_same_bits_as_the_python_function(dtype, layout):
+    x, hw, bias, dy = _inputs(dtype)
+    got = []
+    for function in _functions():
+        xs, hs, bs = layout(x).detach().requires_grad_(), hw.clone().requires_grad_(), bias.clone().requires_grad_()
+        y = _call(function, xs, hs, bs)
+        got.append((y,) + torch.autograd.grad(y, (xs, hs, bs), layout(dy)))
+    for a, b in zip(*got):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        np.testing.assert_array_equal(a.detach().float().cpu().numpy(), b.detach().float().cpu().numpy())
+
+
+@pytest.mark.parametrize("wanted", [(1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 0, 1), (0, 1, 1)])
+@pytest.mark.parametrize("changed", ["x", "hw", "R"])
+def test_a_change_in_place_before_the_backward_is_refused(wanted, changed):
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        for t, w in zip((x, hw, bias), wanted):
+            t.requires_grad_(bool(w))
+        r = R.clone()
+        y = function.apply(x, hw, r, N, 1, 0.5, *TILE, bias, False)
+        with torch.no_grad():
+            {"x": x, "hw": hw, "R": r}[changed].add_(1)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            y.backward(dy)
+
+
+@pytest.mark.parametrize("wanted", [(1, 0, 0), (0, 1, 0), (0, 0, 1)])
+def test_a_second_backward_needs_retain_graph(wanted):
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        for t, w in zip((x, hw, bias), wanted):
+            t.requires_grad_(bool(w))
+        y = _call(function, x, hw, bias)
+        y.backward(dy, retain_graph=True)
+        y.backward(dy)
+        with pytest.raises(RuntimeError, match="second time"):
+            y.backward(dy)
+
+
+def test_saved_tensor_hooks_see_what_the_function_saves():
+    seen = []
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        hw.requires_grad_()
+        shapes = []
+
+        def pack(t):
+            shapes.append(tuple(t.shape))
+            return t.cpu()
+
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t if t.dtype == torch.int32 else t.cuda()):
+            y = _call(function, x, hw, bias)
+        grad, = torch.autograd.grad(y, hw, dy)
+        seen.append((shapes, grad.cpu()))
+    assert seen[0][0] == seen[1][0]
+    assert torch.equal(seen[0][1], seen[1][1])
+
+
+@pytest.mark.parametrize("unpack", [lambda t: t.cpu(), lambda t: t.to(torch.int32 if t.dtype == torch.int32 else torch.float64),
+                                    lambda t: t[:5]], ids=["cpu", "dtype", "shape"])
+def test_what_a_hook_hands_back_is_checked_before_a_kernel_sees_it(unpack):
+    function = _functions()[0]
+    x, hw, bias, dy = _inputs()
+    x.requires_grad_()
+    hw.requires_grad_()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        y = _call(function, x, hw, bias)
+    with pytest.raises((RuntimeError, TypeError, ValueError)):
+        y.backward(dy)
+
+
+def test_forward_mode_is_refused():
+    for function in _functions():
+        for which in range(3):
+            args = list(_inputs()[:3])
+            with forward_ad.dual_level():
+                args[which] = forward_ad.make_dual(args[which], torch.ones_like(args[which]))
+                with pytest.raises((RuntimeError, NotImplementedError)):
+                    _call(function, *args)
+
+
+def test_vmap_and_batched_gradients_are_refused():
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(lambda v: _call(function, v, hw, bias))(torch.stack([x, x]))
+        x.requires_grad_()
+        y = _call(function, x, hw, bias)
+        with pytest.raises(RuntimeError):
+            torch.autograd.grad(y, x, torch.stack([dy, dy]), is_grads_batched=True)
