@@ -430,28 +430,36 @@ __global__ __launch_bounds__(kFoldThreads) void fold_tiles_kernel(const FoldPara
 // the machinery above (windows in LDS, shares, run lists walked by wavefronts) costs more than it
 // saves: a 1024 x 1024 layer has 256 tiles and a hashed_weight of 65536 elements, and its whole
 // gradient is a few microseconds of reading.  Here a workgroup of 256 threads owns 256
-// consecutive elements of dHW, one per thread; it lists the tiles whose
-// slice meets its elements (ascending tile index: two barriers per 1024 tiles) and every thread
-// then walks down the list and adds what each tile holds for its element — loads of 64 consecutive
-// floats per wavefront, fixed order of additions (tile by tile, slice by slice),
-// no atomics, every element of dHW written once.
+// consecutive elements of dHW and lists the tiles whose slice meets them, ascending: eight looks per
+// thread, a ballot each, two barriers per 2048 tiles.  Every wavefront then holds all 256 elements, four
+// consecutive ones per lane, and adds up every fourth entry of the list; the four sums of an
+// element are combined through LDS.  Fixed order of additions, no atomics, every element of dHW
+// written once.
+//   What bounds it: instructions, not bytes.  One element per thread and every tile in every wavefront
+// (masks, addresses and a wait for each element of each tile) took 9.5 us at 1024 x 1024 fp32; here a lane's
+// load covers four elements from a scalar base and a wavefront meets a quarter of the tiles.
 static constexpr int kFoldSmallThreads = 256;
 static constexpr int kFoldSmallTiles = 4096;   // tiles at most: the list in LDS can hold every one of them
 
 template <typename TT>
 __global__ __launch_bounds__(kFoldSmallThreads) void fold_small_kernel(const FoldParams p) {
-  constexpr int PER = 1;   // elements of dHW per thread
-  __shared__ int list_id[kFoldSmallTiles];     // tiles that meet this workgroup's elements, ascending
-  __shared__ int list_rel[kFoldSmallTiles];    // ... and where each starts, relative to the first element
-  __shared__ int wave_count[kFoldSmallThreads / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int kWaves = kFoldSmallThreads / 64;
+  constexpr int kPer = kFoldSmallThreads / 64;   // elements of dHW per lane: a wavefront holds the workgroup's whole span
+  constexpr int kLook = 8;                       // tiles a thread looks at per round
+  constexpr int kBatch = 8;                      // entries of the list whose loads a wavefront has in flight together
+  static_assert(kPer == 4 && kWaves == 4, "a load is four elements, a round's counts are int4");
+  static_assert(kFoldSmallThreads * sizeof(float) <= kFoldMarginBytes, "loads reach up to a span beyond the tiles");
+  __shared__ uint16_t list_id[kFoldSmallTiles];   // tiles that meet this workgroup's elements, ascending
+  __shared__ int list_rel[kFoldSmallTiles];       // ... and where each starts, relative to the first element
+  __shared__ int4 counts[kLook];                  // ... of them found by wavefront x, y, z, w
+  __shared__ float4 sums[kWaves][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if ((int)blockIdx.x >= p.windows) {   // (uniform)
-    colsum_block<kFoldSmallThreads>(p.bias, (int)blockIdx.x - p.windows, tid, reinterpret_cast<float*>(list_id));
+    colsum_block<kFoldSmallThreads>(p.bias, (int)blockIdx.x - p.windows, tid, reinterpret_cast<float*>(sums));
     return;
   }
-  constexpr int kSpan = kFoldSmallThreads * PER;
-  const int h0 = blockIdx.x * kSpan;
-  const int span = (p.H - h0) < kSpan ? (p.H - h0) : kSpan;
+  const int h0 = blockIdx.x * kFoldSmallThreads;
+  const int span = (p.H - h0) < kFoldSmallThreads ? (p.H - h0) : kFoldSmallThreads;
   const int E = p.h.BK * p.h.BN, eshift = p.h.bk_shift + p.h.bn_shift;
   const int ntiles = p.tiles_k * p.tiles_n;
   const bool plan_ok = p.plan_header == nullptr || layer_plan_matches(p.plan_header, p.K, p.N, p.H, p.h);   // (uniform)
@@ -460,102 +468,95 @@ __global__ __launch_bounds__(kFoldSmallThreads) void fold_small_kernel(const Fol
   //  match lists nothing)
   const bool even = p.K % p.h.BK == 0 && p.N % p.h.BN == 0;   // (uniform) every tile lies inside K x N
   int listed = 0;
-  for (int first = 0; first < ntiles; first += 4 * kFoldSmallThreads) {
-    // thread t looks at the tiles first + 4 t .. first + 4 t + 3 (ascending over the threads)
-    int rel[4];
-    unsigned hit = 0u;
+  for (int first = 0; first < ntiles; first += kLook * kFoldSmallThreads) {
+    int rel[kLook];
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int id = first + 4 * tid + u;
-      const int idc = id < ntiles ? id : ntiles - 1;
-      // (without a table, the few offsets a thread needs are hashed on the spot)
-      rel[u] = (p.offsets != nullptr ? p.offsets[idc] : (int)tile_offset(p.h, (uint32_t)(idc / p.tiles_n), (uint32_t)(idc % p.tiles_n))) - h0;
-      hit |= (unsigned)((id < ntiles) & (rel[u] > -E) & (rel[u] < span) & plan_ok) << u;
+    for (int u = 0; u < kLook; u++) {
+      const int id0 = first + u * kFoldSmallThreads;
+      rel[u] = p.H;   // (meets nothing)
+      if (id0 < ntiles) {   // (uniform)
+        const int id = id0 + tid < ntiles ? id0 + tid : ntiles - 1;
+        // (without a table, the few offsets a thread needs are hashed on the spot)
+        rel[u] = p.offsets != nullptr ? p.offsets[id] : (int)tile_offset(p.h, (uint32_t)(id / p.tiles_n), (uint32_t)(id % p.tiles_n));
+      }
     }
-    const int mine = __popc(hit);
-    int incl = mine;
+    uint64_t hits[kLook];
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int up = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += up;
+    for (int u = 0; u < kLook; u++) {
+      rel[u] -= h0;
+      hits[u] = __ballot((first + u * kFoldSmallThreads + tid < ntiles) & (rel[u] > -E) & (rel[u] < span) & plan_ok);
     }
     __syncthreads();   // (the counts of the previous round have been read)
-    if (lane == 63) wave_count[wave] = incl;
-    __syncthreads();
-    int at = listed + incl - mine;
-    for (int w = 0; w < kFoldSmallThreads / 64; w++) {
-      const int c = wave_count[w];
-      if (w < wave) at += c;
-      listed += c;
-    }
+    if (lane == 0) {
 #pragma unroll
-    for (int u = 0; u < 4; u++)
-      if ((hit >> u) & 1u) {
-        list_id[at] = first + 4 * tid + u;
+      for (int u = 0; u < kLook; u++) reinterpret_cast<int*>(&counts[u])[wave] = __popcll(hits[u]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kLook; u++) {
+      const int4 c = counts[u];
+      if ((hits[u] >> lane) & 1ull) {
+        const int at = listed + (wave > 0 ? c.x : 0) + (wave > 1 ? c.y : 0) + (wave > 2 ? c.z : 0) +
+                       (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(hits[u] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hits[u], 0u));
+        list_id[at] = (uint16_t)(first + u * kFoldSmallThreads + tid);
         list_rel[at] = rel[u];
-        at++;
       }
+      listed += (c.x + c.y) + (c.z + c.w);
+    }
   }
   __syncthreads();
-  float acc[PER];
-#pragma unroll
-  for (int j = 0; j < PER; j++) acc[j] = plan_ok ? 0.f : __builtin_nanf("");
-  // The list is taken 32 / PER tiles at a time: all loads of a batch are issued before the first value is
-  // used (a load per tile under its own branch would wait out one memory latency after the other: 17
-  // tiles took 10 us that way), and the values are added in list order.  A thread that a tile does not
-  // reach loads the tile buffer's first float instead and adds zero.
-  constexpr int kBatch = 32 / PER;
-  for (int e0 = 0; e0 < listed; e0 += kBatch) {   // (uniform)
-    unsigned off[kBatch][PER];
-    bool ok[kBatch][PER];
+  // Every wavefront takes entries wave, wave + 4, ... of the list, kBatch at a time: all loads of a batch
+  // are issued before the first value is used.  A load's base is uniform (the tile's element that falls on this
+  // workgroup's first one) and may lie up to a span outside the tile: inside the tile buffer and its margins,
+  // whose values the masks replace by zero.
+  float acc[kPer] = {0.f, 0.f, 0.f, 0.f};
+  for (int e0 = wave; e0 < listed; e0 += kWaves * kBatch) {   // (uniform in a wavefront)
+    const int mine = e0 + kWaves * (lane & (kBatch - 1));
+    const int my_id = list_id[mine < listed ? mine : e0];
+    const int my_rel = mine < listed ? list_rel[mine] : kFoldSmallThreads;   // (an empty place: its tile starts behind the span)
+    int id[kBatch], rel[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; u++) {
-      const int e = e0 + u < listed ? e0 + u : listed - 1;
-      const int id = list_id[e], rel = list_rel[e];
-      // rows and columns of the tile inside K x N (what lies beyond was never written)
-      int rows = p.h.BK, cols = p.h.BN;
-      if (!even) {
-        const int tk = id / p.tiles_n, tn = id - tk * p.tiles_n;
-        rows = (p.K - tk * p.h.BK) < p.h.BK ? (p.K - tk * p.h.BK) : p.h.BK;
-        cols = (p.N - tn * p.h.BN) < p.h.BN ? (p.N - tn * p.h.BN) : p.h.BN;
-      }
-      const bool whole = rows == p.h.BK && cols == p.h.BN;
-#pragma unroll
-      for (int j = 0; j < PER; j++) {
-        const int x = tid + j * kFoldSmallThreads - rel;   // element of the tile that lands on this thread's j-th element
-        ok[u][j] = e0 + u < listed && x >= 0 && x < E && tid + j * kFoldSmallThreads < span &&
-                   (whole || ((x >> p.h.bn_shift) < rows && (x & (p.h.BN - 1)) < cols));
-        off[u][j] = ok[u][j] ? ((unsigned)id << eshift) + (unsigned)x : 0u;
-      }
+      id[u] = __builtin_amdgcn_readlane(my_id, u);
+      rel[u] = __builtin_amdgcn_readlane(my_rel, u);
     }
     for (int sl = 0; sl < p.slices; sl++) {
-      const TT* base = reinterpret_cast<const TT*>(p.tiles) + (((size_t)sl * ntiles) << eshift);
-      TT v[kBatch][PER];
+      const TT* base = reinterpret_cast<const TT*>(p.tiles) + (((int64_t)sl * ntiles) << eshift);
+      TT v[kBatch][kPer];
 #pragma unroll
-      for (int u = 0; u < kBatch; u++)
+      for (int u = 0; u < kBatch; u++) __builtin_memcpy(v[u], base + (((int64_t)id[u] << eshift) - rel[u]) + lane * kPer, sizeof(TT) * kPer);
 #pragma unroll
-        for (int j = 0; j < PER; j++) v[u][j] = base[off[u][j]];
+      for (int u = 0; u < kBatch; u++) {
+        const int x = lane * kPer - rel[u];   // element of the tile that lands on this lane's first element
+        if (even) {   // (uniform)
 #pragma unroll
-      for (int u = 0; u < kBatch; u++)
+          for (int j = 0; j < kPer; j++) acc[j] += (unsigned)(x + j) < (unsigned)E ? ElemTraits<TT>::to_float(v[u][j]) : 0.f;
+        } else {
+          // rows and columns of the tile inside K x N (what lies beyond was never written)
+          const int tk = id[u] / p.tiles_n, tn = id[u] - tk * p.tiles_n;
+          const int rows = p.K - tk * p.h.BK, cols = p.N - tn * p.h.BN;
 #pragma unroll
-        for (int j = 0; j < PER; j++) acc[j] += ok[u][j] ? ElemTraits<TT>::to_float(v[u][j]) : 0.f;
+          for (int j = 0; j < kPer; j++)
+            acc[j] += ((unsigned)(x + j) < (unsigned)E && ((x + j) >> p.h.bn_shift) < rows && ((x + j) & (p.h.BN - 1)) < cols) ? ElemTraits<TT>::to_float(v[u][j]) : 0.f;
+        }
+      }
     }
   }
-#pragma unroll
-  for (int j = 0; j < PER; j++) {
-    const int pos = tid + j * kFoldSmallThreads;
-    if (pos >= span) continue;
-    const int q = h0 + pos;
-    if (p.out_dtype == RZ_F32) {
-      float* out = reinterpret_cast<float*>(p.out);
-      out[q] = acc[j] + (p.accumulate ? out[q] : 0.f);
-    } else if (p.out_dtype == RZ_BF16) {
-      bf16_t* out = reinterpret_cast<bf16_t*>(p.out);
-      out[q] = ElemTraits<bf16_t>::from_float(acc[j] + (p.accumulate ? ElemTraits<bf16_t>::to_float(out[q]) : 0.f));
-    } else {
-      f16_t* out = reinterpret_cast<f16_t*>(p.out);
-      out[q] = ElemTraits<f16_t>::from_float(acc[j] + (p.accumulate ? ElemTraits<f16_t>::to_float(out[q]) : 0.f));
-    }
+  sums[wave][lane] = float4{acc[0], acc[1], acc[2], acc[3]};
+  __syncthreads();
+  if (tid >= span) return;
+  const float* part = reinterpret_cast<const float*>(sums) + tid;
+  const float sum = plan_ok ? (part[0] + part[256]) + (part[512] + part[768]) : __builtin_nanf("");
+  const int q = h0 + tid;
+  if (p.out_dtype == RZ_F32) {
+    float* out = reinterpret_cast<float*>(p.out);
+    out[q] = sum + (p.accumulate ? out[q] : 0.f);
+  } else if (p.out_dtype == RZ_BF16) {
+    bf16_t* out = reinterpret_cast<bf16_t*>(p.out);
+    out[q] = ElemTraits<bf16_t>::from_float(sum + (p.accumulate ? ElemTraits<bf16_t>::to_float(out[q]) : 0.f));
+  } else {
+    f16_t* out = reinterpret_cast<f16_t*>(p.out);
+    out[q] = ElemTraits<f16_t>::from_float(sum + (p.accumulate ? ElemTraits<f16_t>::to_float(out[q]) : 0.f));
   }
 }
 
