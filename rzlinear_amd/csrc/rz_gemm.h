@@ -172,7 +172,7 @@ struct GemmKernel {
   // per step, halving the barriers per flop (8 % faster at 2048^3).
   // ... and the directly staged 64 tile, whose sixteen wavefronts share a step four ways.
   static constexpr bool kLongStep = Tr::kBytes == 2 && (FULL || CLAMP) && NSTAGE >= 2 &&
-                                    ((TI == 128 && TJ == 128 && WI * WJ == 8) || (TI == 64 && TJ == 64));
+                                    ((TI == 128 && TJ == 128 && WI * WJ == 8) || (TI == 64 && TJ == 64) || TI == 32);
   // ... and the fp32 tiles of at most 64 rows in forward / input-grad, whose 128-byte step is over in
   // 0.4 us — less than a load from L2 takes, so that loads issued two steps ahead arrive late, and
   // half as many barriers per flop (1024^3: forward 30.2 -> 28.3 us, input-grad 27.1 -> 25.9 us;
@@ -202,7 +202,7 @@ struct GemmKernel {
   static_assert(WTI % 32 == 0 && WTJ % 32 == 0, "wavefront tile must be a multiple of 32");
 
   // direct-to-LDS staging (see the head of this file)
-  static constexpr bool kDirect16 = k16 && (FULL || CLAMP) && NSTAGE >= 2 && ((TI >= 128 && TJ >= 128) || (TI == 64 && TJ == 64));
+  static constexpr bool kDirect16 = k16 && (FULL || CLAMP) && NSTAGE >= 2 && ((TI >= 128 && TJ >= 128) || (TI == 64 && TJ == 64) || (TI == 32 && TJ == 128));
   // fp32, complete tiles: the same staging; a "sub-step" is then eight elements of R (four MFMAs per
   // pair of blocks), and a fragment holds a lane's four values of it
   static constexpr bool kDirect32 = !k16 && RZ_F32_DIRECT && (FULL || CLAMP) && NSTAGE == 2 && TJ >= 64;

@@ -38,7 +38,8 @@ static hipError_t launch_one(GemmParams p, const WeightGradPlan* plan, const Spl
       p.colsum_pitch = plan->colsum_pitch;
     }
   } else if (split != nullptr && split->splits > 1) {
-    if (split->tile != TI || p.partial == nullptr) return hipErrorInvalidValue;
+    constexpr int kPlanTile = TI == 32 && TJ == 128 ? 128 : TI;   // (the C tile of 32 x 128 serves plans of the 128 tile)
+    if (split->tile != kPlanTile || p.partial == nullptr) return hipErrorInvalidValue;
     splits = split->splits;
     p.r_chunk = split->r_chunk;
     // a slice must begin on a step boundary: the offset table of a step assumes that the step
@@ -92,14 +93,14 @@ static hipError_t launch_tile(GemmParams p, const WeightGradPlan* plan, const Sp
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true>::TR) return hipErrorInvalidValue;
     return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true, COLSUM, false, WK>(p, plan, split, stream);
   }
-  constexpr bool kSixteen = WI * WJ * WK == 16;
+  constexpr bool kDirectOnly = WI * WJ * WK == 16 || (sizeof(T) == 2 && NSTAGE == 3);
   if constexpr (NSTAGE >= 2 && !kCheckedOnly) {
     if (form.clamp) {
       if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, false, true, WK>::TR) return hipErrorInvalidValue;
       return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, true, WK>(p, plan, split, stream);
     }
   }
-  if constexpr (kSixteen) {   // (always directly staged)
+  if constexpr (kDirectOnly) {
     return hipErrorInvalidValue;
   } else {
     if (form.full || form.clamp || form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false>::TR) return hipErrorInvalidValue;
@@ -132,6 +133,8 @@ static hipError_t launch_op(GemmParams p, const WeightGradPlan* plan, const Spli
 //    64:  64 x  64, for problems with few tiles: 16-bit sixteen wavefronts of 32 x 32 in four groups that
 //        share every R step between them; fp32 forward / input-grad eight, in two such groups; fp32
 //        weight-grad, and 16-bit rows shorter than a 16-byte piece, four
+//        16-bit forward / input-grad of at most 32 rows: 32 x 128 (eight wavefronts of 32 x 32 in two groups
+//        that share every R step, three LDS stages)
 //    32:  32 x  64 (fp32 forward / input-grad whose rows would leave a 64-row tile at most half full): four wavefronts of 32 x 32 in two such groups
 template <typename T, int OP>
 static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
@@ -142,6 +145,10 @@ static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const 
   const int chunk = wg ? plan->r_chunk : (cut ? split->r_chunk : p.R);
   const long long workgroups = wg ? plan->workgroups : tile_count(p.I, p.J, tile) * (cut ? split->splits : 1);
   const KernelForm form = kernel_form(OP, p.I, p.J, p.R, chunk, tile, workgroups, (int)sizeof(T), tuning);
+  if constexpr (sizeof(T) == 2 && OP != kWeightGrad) {
+    if (form.rows == 32 && form.cols == 128) return launch_tile<T, OP, 32, 1, 4, 3, false, 2, 128>(p, plan, split, form, stream);
+  }
+  if (form.rows != form.tile || form.cols != tile_cols(form.tile)) return hipErrorInvalidValue;
   switch (form.tile * 1000 + form.waves * 10 + form.stages) {
     case 256082: return launch_op<T, OP, 256, 2, 4, 2>(p, plan, split, form, stream);
     case 64042: return launch_op<T, OP, 64, 2, 2, 2>(p, plan, split, form, stream);

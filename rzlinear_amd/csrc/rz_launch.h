@@ -589,7 +589,8 @@ struct SplitPlan {
 // M = 128, 256 tile 104 / 93.  M = 128, K = 2048, N = 8192: 128 tile, three slices 14.7 / 20.8 us.
 // M = 64, K = N = 4096: 64 tile, four slices 12.7 / 13.6; 128 tile 21.3 / 18.4.  Six slices at M = 32: 52 / 40.
 // The 32 x 64 tile has two wavefronts to read with: two slices.
-static inline int finish_slices(int tile, int I, int J) {
+static inline int finish_slices(int tile, int I, int J, int elem_bytes) {
+  if (tile == 128 && elem_bytes == 2 && I <= 32) return kFinishSlices;   // (the 32 x 128 form: no padded rows)
   if (I < (tile == 32 ? 32 : tile)) return 0;
   if (tile == 256 && (double)I * J * 4.0 < 16.0e6) return 0;
   return tile == 32 ? 2 : kFinishSlices;
@@ -644,7 +645,7 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
       //  back by the finishing workgroups, and no second kernel is launched — worth a couple of microseconds
       //  and a plane; fp32, M = 16384, K = 512, N = 1024 input-grad, planes of 33 MB: the 256 tile in two
       //  slices 155 us against the whole 128 tile's 136)
-      if (slices > 1 && slices <= finish_slices(tile, I, J) && t.finish != -1) us += (2.0 * slices - 1.0) * (double)I * J * 4.0 / 4.0e6 + 2.0;
+      if (slices > 1 && slices <= finish_slices(tile, I, J, elem_bytes) && t.finish != -1) us += (2.0 * slices - 1.0) * (double)I * J * 4.0 / 4.0e6 + 2.0;
       else if (slices > 1) us += (2.0 * slices * (double)I * J * 4.0 + (double)I * J * elem_bytes) / 4.0e6 + (direct ? 3.0 : 4.0);
       else whole_us = us;
       // (near ties go to the larger tile and the fewer slices, which come first)
@@ -681,7 +682,7 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
 // elements per step that follow from those.  One function decides for the launch and for
 // rz_plan_query.
 struct KernelForm {
-  int tile, waves, stages;
+  int tile, rows, cols, waves, stages;   // tile: the planner's code; rows x cols: the C tile of the kernel that serves it
   bool full, clamp;
   int step;
 };
@@ -690,6 +691,8 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
                                      int elem_bytes, const rz_tuning& t) {
   KernelForm f;
   f.tile = tile;
+  f.rows = tile;
+  f.cols = tile_cols(tile);
   f.stages = (tile == 128 && t.stages == 1) ? 1 : 2;
   // 128 tile: with about one workgroup per compute unit, eight wavefronts (two per SIMD, 64 x 32
   // each) hide latency better than four of 64 x 64; with more workgroups resident the
@@ -718,6 +721,20 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
             : tile == 64 ? ((many64 && (f.full || f.clamp)) ? 16 : (elem_bytes == 4 && op != kWeightGrad) ? 8 : 4)
                          : waves128;
   if (f.waves == 16) f.stages = workgroups <= kComputeUnits ? 4 : 2;
+  // 16-bit forward / input-grad on the planner's 128 tile, a batch of at most 32 rows (decoding): C tiles of 32 x 128.
+  // The 128 rows of the square tile would stage the batch four times over beside every piece of W; without them three
+  // LDS stages fit, twice as many bytes of W are in flight, and no padded rows are multiplied or stored, so that the
+  // kernel can finish a cut itself (K = N = 10240, H = 6.5 M bf16, three slices: M = 1 28 us, M = 32 44.7 -> 29.2 us, 7.2 TB/s
+  // of W from beyond the L2s).  33 to 64 rows: two such tiles would read W twice; the 64 tile takes those.
+  if (tile == 128 && elem_bytes == 2 && op != kWeightGrad && f.stages == 2 && (f.full || f.clamp) && I <= 32 &&
+      (chunk >= R || chunk % 128 == 0)) {
+    f.rows = 32;
+    f.waves = 8;
+    f.stages = 3;
+    f.step = 128;
+    f.full = I == 32 && J % 128 == 0 && R % 128 == 0 && chunk % 128 == 0;
+    f.clamp = !f.full;
+  }
   return f;
 }
 
