@@ -107,6 +107,8 @@ enum Op { kForward = 0, kInputGrad = 1, kWeightGrad = 2 };
 // Slices of a cut contraction whose values the kernel that finishes its own tiles holds at a time
 // (GemmParams::finish; see finish_slices in rz_launch.h).
 static constexpr int kFinishSlices = 4;
+// ... for a C tile of `rows` rows: those of 32 keep eight (few values per lane, and registers to spare)
+__host__ __device__ constexpr int finish_limit(int rows) { return rows == 32 ? 2 * kFinishSlices : kFinishSlices; }
 
 struct GemmParams {
   const void* A;

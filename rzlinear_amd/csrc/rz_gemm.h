@@ -73,6 +73,13 @@ template <> struct Mfma<f16_t> {
   }
 };
 
+// s + a * b with the product rounded by itself: never a fused multiply-add.
+__device__ __forceinline__ float add_product(float s, float a, float b) {
+#pragma clang fp contract(off)
+  const float product = a * b;
+  return s + product;
+}
+
 // 16 bytes of a plain row-major matrix at (row, col..col+VEC), zero where out of range
 // (FULL: the caller guarantees the piece is in range, no checks).
 template <typename T, bool FULL>
@@ -1258,11 +1265,12 @@ struct GemmKernel {
             // (half a block at a time: the other slices' values of eight rows are fetched before the first is
             //  used — a whole block's would cost registers that the two-workgroup forms do not have)
             constexpr int kHalf = kElems < 8 ? kElems : 8;
+            constexpr int kFinishMax = finish_limit(TI);
 #pragma unroll
             for (int h = 0; h < kElems / kHalf; h++) {
-              float v[kFinishSlices][kHalf];
+              float v[kFinishMax][kHalf];
 #pragma unroll
-              for (int sl = 0; sl < kFinishSlices; sl++) {
+              for (int sl = 0; sl < kFinishMax; sl++) {
                 if (sl < slices && sl != by) {   // (uniform)
 #pragma unroll
                   for (int e = 0; e < kHalf; e++) {
@@ -1275,10 +1283,10 @@ struct GemmKernel {
 #pragma unroll
               for (int e = 0; e < kHalf; e++) sum[e] = 0.f;
 #pragma unroll
-              for (int sl = 0; sl < kFinishSlices; sl++) {
+              for (int sl = 0; sl < kFinishMax; sl++) {
                 if (sl == by) {
 #pragma unroll
-                  for (int e = 0; e < kHalf; e++) sum[e] += __fmul_rn(acc[a][b][h * kHalf + e], p.scale);   // (the product as it was stored: not fused into the add)
+                  for (int e = 0; e < kHalf; e++) sum[e] = add_product(sum[e], acc[a][b][h * kHalf + e], p.scale);   // (the product as it was stored)
                 } else if (sl < slices) {
 #pragma unroll
                   for (int e = 0; e < kHalf; e++) sum[e] += v[sl][e];
@@ -1287,7 +1295,7 @@ struct GemmKernel {
               // (the bias joins the fp32 sum as in the second kernel: an add of its own, rounded to fp32,
               //  not part of a fused multiply-add that rounds straight to the output type)
 #pragma unroll
-              for (int e = 0; e < kHalf; e++) acc[a][b][h * kHalf + e] = __fadd_rn(sum[e], bias[b]);
+              for (int e = 0; e < kHalf; e++) acc[a][b][h * kHalf + e] = sum[e] + bias[b];
             }
           }
         }

@@ -46,7 +46,7 @@ static hipError_t launch_one(GemmParams p, const WeightGradPlan* plan, const Spl
     // lies inside one hashed tile or covers whole ones
     if (p.r_chunk % K::TR != 0) return hipErrorInvalidValue;
     // (the kernel that finishes its own tiles holds the other slices' values in registers)
-    if (p.finish != nullptr && splits > kFinishSlices) return hipErrorInvalidValue;
+    if (p.finish != nullptr && splits > finish_limit(TI)) return hipErrorInvalidValue;
   } else {
     p.r_chunk = r_steps * K::TR;
     p.partial = nullptr;

@@ -580,6 +580,12 @@ struct SplitPlan {
   double est_us;     // what the model expects the launch(es) to take
 };
 
+// 16-bit forward / input-grad of at most 32 rows whose plan is the 128 tile: C tiles of 32 x 128 (see kernel_form).
+// (An override of the tile gets the square one.)
+static inline bool rows32_form(int tile, int I, int elem_bytes, const rz_tuning& t) {
+  return tile == 128 && elem_bytes == 2 && I <= 32 && t.tile == 0;
+}
+
 // Slices up to which a cut contraction is finished by its own kernel (GemmParams::finish; 0: never).  The
 // slice that comes last at a tile reads the others' planes by itself, four bytes per lane and load, after
 // an atomic's round trip: that pays up to four slices, where the rows of a tile are real (a batch of
@@ -589,11 +595,11 @@ struct SplitPlan {
 // M = 128, 256 tile 104 / 93.  M = 128, K = 2048, N = 8192: 128 tile, three slices 14.7 / 20.8 us.
 // M = 64, K = N = 4096: 64 tile, four slices 12.7 / 13.6; 128 tile 21.3 / 18.4.  Six slices at M = 32: 52 / 40.
 // The 32 x 64 tile has two wavefronts to read with: two slices.
-static inline int finish_slices(int tile, int I, int J, int elem_bytes) {
-  if (tile == 128 && elem_bytes == 2 && I <= 32) return kFinishSlices;   // (the 32 x 128 form: no padded rows)
+static inline int finish_slices(int tile, int I, int J, int elem_bytes, const rz_tuning& t) {
+  if (rows32_form(tile, I, elem_bytes, t)) return finish_limit(32);
   if (I < (tile == 32 ? 32 : tile)) return 0;
   if (tile == 256 && (double)I * J * 4.0 < 16.0e6) return 0;
-  return tile == 32 ? 2 : kFinishSlices;
+  return finish_limit(tile);
 }
 
 // Tile and number of slices together: the pair with the least estimated time.  A slice pays the
@@ -645,7 +651,7 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
       //  back by the finishing workgroups, and no second kernel is launched — worth a couple of microseconds
       //  and a plane; fp32, M = 16384, K = 512, N = 1024 input-grad, planes of 33 MB: the 256 tile in two
       //  slices 155 us against the whole 128 tile's 136)
-      if (slices > 1 && slices <= finish_slices(tile, I, J, elem_bytes) && t.finish != -1) us += (2.0 * slices - 1.0) * (double)I * J * 4.0 / 4.0e6 + 2.0;
+      if (slices > 1 && slices <= finish_slices(tile, I, J, elem_bytes, t) && t.finish != -1) us += (2.0 * slices - 1.0) * (double)I * J * 4.0 / 4.0e6 + 2.0;
       else if (slices > 1) us += (2.0 * slices * (double)I * J * 4.0 + (double)I * J * elem_bytes) / 4.0e6 + (direct ? 3.0 : 4.0);
       else whole_us = us;
       // (near ties go to the larger tile and the fewer slices, which come first)
@@ -726,7 +732,7 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
   // LDS stages fit, twice as many bytes of W are in flight, and no padded rows are multiplied or stored, so that the
   // kernel can finish a cut itself (K = N = 10240, H = 6.5 M bf16, three slices: M = 1 28 us, M = 32 44.7 -> 29.2 us, 7.2 TB/s
   // of W from beyond the L2s).  33 to 64 rows: two such tiles would read W twice; the 64 tile takes those.
-  if (tile == 128 && elem_bytes == 2 && op != kWeightGrad && f.stages == 2 && (f.full || f.clamp) && I <= 32 &&
+  if (rows32_form(tile, I, elem_bytes, t) && op != kWeightGrad && f.stages == 2 && (f.full || f.clamp) &&
       (chunk >= R || chunk % 128 == 0)) {
     f.rows = 32;
     f.waves = 8;

@@ -18,33 +18,66 @@ def _say(*a):
     sys.stdout.flush()
 
 
-def _both_ops(oracle, shape, dtype, **tuning):
+def _forward_and_mirrored_input_grad(oracle, shape, dtype, split, tile, slices, finished):
+    """The forward of (M, K, N) and the input-grad of (M, N, K), which the planner prices alike, under the plan that
+    is expected; finished in the kernel or, where the plan stays the same, by a second one: the same bits."""
     from rzlinear_amd import _lib
     from rzlinear_amd.impl.RzLinearBackward import rz_linear_backward_input_grad_tl
     from rzlinear_amd.impl.RzLinearForward import rz_linear_forward_bias_tl
     M, K, N, H, BK, BN = shape
-    _say(shape, dtype, tuning)
-    (x, hw, dy), (x64, hw64, dy64) = make_inputs(M, K, N, H, dtype, seed=M + K)
+    _say(shape, dtype, split)
+    (x, hw, _), (x64, hw64, _) = make_inputs(M, K, N, H, dtype, seed=M + K)
     bias = torch.randn((N,), generator=torch.Generator().manual_seed(4)).to(dtype)
-    with _lib.tuning(**tuning):
-        y = rz_linear_forward_bias_tl(x, hw, bias.cuda(), 0.75, M, K, N, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
-        dx = rz_linear_backward_input_grad_tl(dy, hw, 0.75, M, K, N, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
+    out = []
+    for finish in (0, -1):
+        with _lib.tuning(split=split, finish=finish):
+            for q in (_lib.plan_query(0, M, K, N, H, BK, BN, _lib.dtype_code(x)), _lib.plan_query(1, M, N, K, H, BK, BN, _lib.dtype_code(x))):
+                if finish == 0:
+                    assert (q["tile"], q["slices"], q["shares"]) == (tile, slices, finished)
+                same_plan = (q["tile"], q["slices"]) == (tile, slices)
+            if not same_plan:   # (priced without the finish, another tile may be the better one)
+                continue
+            y = rz_linear_forward_bias_tl(x, hw, bias.cuda(), 0.75, M, K, N, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
+            dx = rz_linear_backward_input_grad_tl(x, hw, 0.75, M, N, K, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
+            out.append((y, dx))
+    y, dx = out[0]
     assert_close(y.float().cpu().numpy(), oracle.forward(x64, hw64, N, BK, BN, R1024, 0.75) + bias.double().numpy(), dtype, "y")
-    assert_close(dx.float().cpu().numpy(), oracle.input_grad(dy64, hw64, K, BK, BN, R1024, 0.75), dtype, "dx")
+    assert_close(dx.float().cpu().numpy(), oracle.input_grad(x64, hw64, N, BK, BN, R1024, 0.75), dtype, "dx")
+    for a, b in zip(out[0], out[-1]):
+        np.testing.assert_array_equal(a.float().cpu().numpy(), b.float().cpu().numpy())
 
 
 @pytest.mark.parametrize("dtype", SIXTEEN, ids=str)
-@pytest.mark.parametrize("split", [-1, 2, 4, 5])   # whole; finished in the kernel; by a second kernel
-@pytest.mark.parametrize("shape", [
-    (32, 640, 1280, 20000, 32, 64),      # complete tiles and steps
-    (1, 640, 1280, 20000, 64, 64),       # one row
-    (31, 700, 1100, 20000, 32, 64),      # last step and last column tile partial, rows of whole pieces (K) and not (N)
-    (17, 641, 1023, 20000, 16, 128),     # nothing a multiple of anything
-    (32, 128, 128, 20000, 64, 32),       # fewer steps than stages
-    (5, 9, 900, 20000, 32, 64),          # a row of little more than one piece
-], ids=lambda s: "x".join(map(str, s)))
-def test_at_most_32_rows(oracle, shape, dtype, split):
-    _both_ops(oracle, shape, dtype, tile=128, split=split)
+@pytest.mark.parametrize("shape,split,slices,finished", [
+    ((32, 2048, 2048, 20000, 32, 64), 0, 8, 1),      # complete tiles and steps, as many slices as the kernel finishes
+    ((32, 2048, 2048, 20000, 64, 64), 3, 3, 1),      # an incomplete last slice
+    ((1, 2048, 2048, 20000, 64, 64), 4, 4, 1),       # one row
+    ((31, 4111, 4099, 20000, 32, 64), 5, 5, 1),      # odd row pitch, last step and last column tile partial
+    ((17, 4100, 4097, 20000, 16, 128), 6, 6, 1),     # ... in other hashed tiles
+    ((7, 2049, 2040, 20000, 128, 32), 0, 6, 1),
+], ids=str)
+def test_16_bit_at_most_32_rows(oracle, shape, split, slices, finished, dtype):
+    _forward_and_mirrored_input_grad(oracle, shape, dtype, split, 128, slices, finished)
+
+
+@pytest.mark.parametrize("dtype", SIXTEEN, ids=str)
+def test_16_bit_at_most_32_rows_uncut(oracle, dtype):
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearForward import rz_linear_forward_tl
+    M, K, N, H, BK, BN = 5, 9, 9000, 20000, 32, 64   # (rows of little more than one 16-byte piece)
+    (x, hw, _), (x64, hw64, _) = make_inputs(M, K, N, H, dtype, seed=1)
+    assert _lib.plan_query(0, M, K, N, H, BK, BN, _lib.dtype_code(x))["tile"] == 128
+    y = rz_linear_forward_tl(x, hw, 0.75, M, K, N, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
+    assert_close(y.float().cpu().numpy(), oracle.forward(x64, hw64, N, BK, BN, R1024, 0.75), dtype, "y")
+
+
+@pytest.mark.parametrize("shape,split,slices,finished", [
+    ((32, 1024, 1024, 20000, 32, 64), 0, 6, 1),
+    ((32, 1024, 1024, 20000, 32, 64), 8, 8, 1),
+    ((32, 2048, 1024, 20000, 64, 64), 16, 16, 0),
+], ids=str)
+def test_fp32_32_rows(oracle, shape, split, slices, finished):
+    _forward_and_mirrored_input_grad(oracle, shape, torch.float32, split, 32, slices, finished)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32] + SIXTEEN, ids=str)
