@@ -357,12 +357,11 @@ struct GemmKernel {
   }
 
   static __device__ __forceinline__ void run(const GemmParams& p, Smem& sm) {
-    run_item(p, sm, threadIdx.x, blockIdx.x, blockIdx.y, gridDim.x);
+    run_item(p, sm, threadIdx.x, blockIdx.x, blockIdx.y, gridDim.x, gridDim.y);
   }
 
-  // One C tile (workgroup id `bx` of `gx`, as the hardware deals them to the XCDs) and slice `by`
-  // of the contracted dimension.
-  static __device__ __forceinline__ void run_item(const GemmParams& p, Smem& sm, const int tid, int bx, int by, int gx) {
+  // One C tile and slice of the contracted dimension, chosen by the workgroup id (bx, by) of a grid of gx x gy.
+  static __device__ __forceinline__ void run_item(const GemmParams& p, Smem& sm, const int tid, int bx, int by, int gx, int gy) {
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // (uniform: lives in a scalar register)
     const int wave_k = wave / (WI * WJ);                 // which part of every R step
@@ -377,10 +376,20 @@ struct GemmKernel {
     // Workgroup ids are dealt round-robin to the 8 XCDs; renumber so that each XCD (one L2)
     // gets a contiguous run of tiles, then walk tiles with J fastest (forward/input-grad
     // share the streamed A panel) or in square-ish groups (weight-grad streams both).
-    int id = bx;
+    // Weight-grad in a multiple of eight slices: slices have no operand in common, so every XCD takes whole
+    // slices, each operand read by one L2 (M = 16384, K = 512, N = 1024 bf16 in eight slices: 29.7 -> 21.5 us).
+    // Not where an XCD would get parts of slices, nor for the cuts of forward and input-grad, whose finishing
+    // slice finds the others' planes in its own L2 (M = 128, K = N = 10240 bf16 in three slices 42 -> 47 us;
+    // M = 3001, K = 2047, N = 1531 fp16 weight-grad in five slices 52 -> 55 us).
+    const bool whole_slices = OP == kWeightGrad && (gy & 7) == 0;
+    int id = whole_slices ? by * gx + bx : bx;
     {
-      const int nwg = gx, per = nwg >> 3, rem = nwg & 7, x = id & 7, q = id >> 3;
+      const int nwg = whole_slices ? gy * gx : gx, per = nwg >> 3, rem = nwg & 7, x = id & 7, q = id >> 3;
       id = x * per + (x < rem ? x : rem) + q;
+    }
+    if (whole_slices) {
+      by = id / gx;
+      id -= by * gx;
     }
     int ti, tj;
     if constexpr (OP == kWeightGrad) {
@@ -1200,7 +1209,7 @@ struct GemmKernel {
           scatter(image);
           __syncthreads();
         }
-        float* dst = p.scatter + ((size_t)by * gx + bx) * (size_t)p.image_pitch;
+        float* dst = p.scatter + ((size_t)by * gx + id) * (size_t)p.image_pitch;
         for (int i = tid * 4; i < p.image_pitch; i += kThreads * 4)
           *reinterpret_cast<float4*>(dst + i) = *reinterpret_cast<const float4*>(image + i);
       } else {
