@@ -256,10 +256,15 @@ struct GemmKernel {
   static constexpr int kOffEntries = (OP == kWeightGrad) ? (TI / 16) * (TJ / 16) : kOffSlots * kOffWindow;
   static constexpr int kTurnEntries = 65;   // weight-grad, behind the offsets: the round of up to 64 hashed tiles, and the number of rounds
 
+  // The 256 tile keeps its column sums (VEC per thread) in LDS: it has no registers left for them, and what it
+  // spills instead comes back through the vector-memory counter, where waiting for it means waiting for the operand
+  // loads just issued as well.
+  static constexpr bool kColsumInLds = COLSUM && TI == 256 && kDirect;
   struct Smem {
     alignas(16) T a[NSTAGE][LA::kElems];
     alignas(16) T b[NSTAGE][LB::kElems];
     int off[kOffEntries];
+    alignas(16) float4 colsum[kColsumInLds ? kThreads * VEC / 4 : 1];   // [VEC / 4][kThreads]
   };
   // after the last R step the operand stages are dead; weight-grad may keep an fp32 image of
   // dHW there
@@ -388,7 +393,7 @@ struct GemmKernel {
       id = x * per + (x < rem ? x : rem) + q;
     }
     if (whole_slices) {
-      by = id / gx;
+      by = __builtin_amdgcn_readfirstlane(id / gx);
       id -= by * gx;
     }
     int ti, tj;
@@ -440,6 +445,26 @@ struct GemmKernel {
     float colsum[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; e++) colsum[e] = 0.f;
+    if constexpr (kColsumInLds) {   // (a thread's own until the epilogue)
+      for (int q = 0; q < VEC / 4; q++) sm.colsum[q * kThreads + tid] = float4{0.f, 0.f, 0.f, 0.f};
+    }
+    // the thread's sums for one turn: from LDS and back, if they are kept there
+    auto colsum_fetch = [&]() {
+      if constexpr (kColsumInLds) {
+#pragma unroll
+        for (int q = 0; q < VEC / 4; q++) {
+          const float4 v = sm.colsum[q * kThreads + tid];
+          colsum[q * 4] = v.x; colsum[q * 4 + 1] = v.y; colsum[q * 4 + 2] = v.z; colsum[q * 4 + 3] = v.w;
+        }
+      }
+    };
+    auto colsum_keep = [&]() {
+      if constexpr (kColsumInLds) {
+#pragma unroll
+        for (int q = 0; q < VEC / 4; q++)
+          sm.colsum[q * kThreads + tid] = float4{colsum[q * 4], colsum[q * 4 + 1], colsum[q * 4 + 2], colsum[q * 4 + 3]};
+      }
+    };
     int colsum_turn = COLSUM ? (r_begin / TR) % p.tiles_i : 0;
 
     auto window = [&](int step) -> OffWindow {
@@ -557,6 +582,7 @@ struct GemmKernel {
       if constexpr (COLSUM) {
         // commits happen once per R step, in step order
         if (colsum_turn == ti) {
+          colsum_fetch();
 #pragma unroll
           for (int q = 0; q < LB::kPieces; q++) {
             T elems[VEC];
@@ -564,6 +590,7 @@ struct GemmKernel {
 #pragma unroll
             for (int e = 0; e < VEC; e++) colsum[e] += Tr::to_float(elems[e]);
           }
+          colsum_keep();
         }
         colsum_turn = (colsum_turn + 1 == p.tiles_i) ? 0 : colsum_turn + 1;
       }
@@ -576,6 +603,7 @@ struct GemmKernel {
       static_assert(!(COLSUM && kDirect) || (TR % kGroups == 0 && (!k16 || kGroups % 4 == 0)), "rows must share a swizzle");
       if (colsum_turn == ti) {
         const int g = tid / LB::kCpr, c = tid % LB::kCpr;
+        colsum_fetch();
 #pragma unroll
         for (int i = 0; i < TR / kGroups; i++) {
           const int row = g + i * kGroups;
@@ -584,6 +612,7 @@ struct GemmKernel {
 #pragma unroll
           for (int e = 0; e < VEC; e++) colsum[e] += Tr::to_float(elems[e]);
         }
+        colsum_keep();
       }
       colsum_turn = (colsum_turn + 1 == p.tiles_i) ? 0 : colsum_turn + 1;
     };
@@ -1036,6 +1065,7 @@ struct GemmKernel {
         // combine the threads that share columns (fixed order), one row of partial sums out
         constexpr int kGroups = kThreads / LB::kCpr;
         static_assert(sizeof(float) * kGroups * TJ <= sizeof(Smem), "column sums must fit the stages");
+        colsum_fetch();
 #pragma unroll
         for (int e = 0; e < VEC; e++) image[(tid / LB::kCpr) * TJ + (tid % LB::kCpr) * VEC + e] = colsum[e];
         __syncthreads();
@@ -1182,6 +1212,24 @@ struct GemmKernel {
 #pragma unroll
               for (int b = 0; b < MJ; b++) blk_tile[a][b] = __builtin_amdgcn_readfirstlane(turn[blk_tile[a][b]]);
           }
+          // What lies outside K x N adds zero, so that the rounds need no bounds checks: left in their loop, the
+          // compiler works all 128 conditions of the 256 tile out ahead and spills them, in the main loop too (M = 32768,
+          // K = 500, N = 1000 bf16 in 32 slices: 85 us, without them and with the column sums in LDS 54; M = 3001, K = 2047,
+          // N = 1531 fp16: 54 -> 47).  (A tile's slice lies inside the image as a whole, and tiles beyond
+          // the grid have their turns like the others.)
+          if constexpr (!FULL) {
+#pragma unroll
+            for (int a = 0; a < MI; a++)
+#pragma unroll
+              for (int b = 0; b < MJ; b++) {
+                const int k0 = i0 + blk_i(a) + block_row(0);
+                const bool col_ok = j0 + blk_j(b) + (lane & 31) < p.J;
+#pragma unroll
+                for (int e = 0; e < kElems; e++)
+                  acc[a][b][e] = (col_ok && k0 + (e >> 2) * 8 + (e & 3) < p.I) ? acc[a][b][e] * p.scale : 0.f;
+              }
+          }
+          const float round_scale = FULL ? p.scale : 1.f;
           for (int t = 0; t < rounds; t++) {
             if (steps > 0) {
 #pragma unroll
@@ -1189,17 +1237,13 @@ struct GemmKernel {
 #pragma unroll
                 for (int b = 0; b < MJ; b++) {
                   if (blk_tile[a][b] == t) {
-                    const int k0 = i0 + blk_i(a) + block_row(0);
-                    const bool col_ok = FULL || (j0 + blk_j(b) + (lane & 31) < p.J);
                     float cur[kElems];
 #pragma unroll
                     for (int e = 0; e < kElems; e++)
                       cur[e] = image[blk_base[a][b] + ((e >> 2) * 8 + (e & 3)) * p.h.BN];
 #pragma unroll
                     for (int e = 0; e < kElems; e++)
-                      if (FULL || (col_ok && k0 + (e >> 2) * 8 + (e & 3) < p.I))
-                        image[blk_base[a][b] + ((e >> 2) * 8 + (e & 3)) * p.h.BN] =
-                            cur[e] + acc[a][b][e] * p.scale;
+                      image[blk_base[a][b] + ((e >> 2) * 8 + (e & 3)) * p.h.BN] = cur[e] + acc[a][b][e] * round_scale;
                   }
                 }
             }
