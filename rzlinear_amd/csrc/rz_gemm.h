@@ -915,7 +915,7 @@ struct GemmKernel {
       constexpr int NKS = TR / KS / WK;   // sub-steps of this wavefront's part of an R step
       constexpr int kLoads = LA::kPieces + LB::kPieces;   // direct loads of a wavefront per step
       static_assert(NSTAGE == 2 || kDirect, "a deeper pipeline is built for direct staging only");
-      auto stage_of = [](int s) -> int { return s % NSTAGE; };
+      auto stage_of = [](int s) -> int { return (int)((unsigned)s % NSTAGE); };
       // fp32: left to itself the compiler moves a sub-step's fragment reads down to just before
       // the MFMAs that use them (read, wait, four MFMAs).  Holding them a sub-step ahead, as
       // written, is faster in the 64 tile (1024^3: 28.7 -> 27.4 us forward, 33.8 -> 31.4 us
