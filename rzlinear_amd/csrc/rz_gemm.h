@@ -620,7 +620,7 @@ struct GemmKernel {
     // instruction with index n = wave * kPieces + q fills LDS bytes [1024 n, 1024 n + 1024) of
     // the stage, lane i the 16 bytes at 16 i; (row, col) is the source piece that the swizzled
     // layout keeps there.
-    auto direct_src = [&](auto L, int layout, int q, int& row, int& col) {
+    auto direct_src = [&](auto L, int layout, int q, int lane, int& row, int& col) {
       typedef decltype(L) LL;
       const int n = wave * LL::kPieces + q;
       if (layout == kRContig) {
@@ -655,10 +655,14 @@ struct GemmKernel {
     // the last, partial step of a ragged contraction, whose pieces beyond R are redirected)
     auto direct_issue_plain_slow = [&](int step, int st) {
       const int r0 = r_begin + step * TR;
+      // (opaque: worked out ahead of the loop, as the compiler would like to, the addresses of this one step take
+      //  registers that every step needs)
+      int l = lane;
+      asm volatile("" : "+v"(l));
 #pragma unroll
       for (int q = 0; q < LA::kPieces; q++) {
         int row, col;
-        direct_src(LA{}, A_LAYOUT, q, row, col);
+        direct_src(LA{}, A_LAYOUT, q, l, row, col);
         // (CLAMP: rows / 16-byte columns beyond I come from the last one inside)
         const int gi = (A_LAYOUT == kRContig) ? i0 + row : i0 + col;
         const int ci = !CLAMP ? gi : (A_LAYOUT == kRContig) ? (gi < p.I ? gi : p.I - 1) : (gi < p.I ? gi : p.I - VEC);
@@ -684,7 +688,7 @@ struct GemmKernel {
 #pragma unroll
         for (int q = 0; q < LB::kPieces; q++) {
           int row, col;
-          direct_src(LB{}, B_LAYOUT, q, row, col);
+          direct_src(LB{}, B_LAYOUT, q, l, row, col);
           const int gj = j0 + col;
           int cj = (!CLAMP || gj < p.J) ? gj : p.J - VEC;
           const int gr = r0 + row;
@@ -709,7 +713,7 @@ struct GemmKernel {
 #pragma unroll
       for (int q = 0; q < LA::kPieces; q++) {
         int row, col;
-        direct_src(LA{}, A_LAYOUT, q, row, col);
+        direct_src(LA{}, A_LAYOUT, q, lane, row, col);
         if constexpr (A_LAYOUT == kRContig) {
           const int gi = i0 + row;
           const int ci = (!CLAMP || gi < p.I) ? row : p.I - 1 - i0;
@@ -725,7 +729,7 @@ struct GemmKernel {
 #pragma unroll
       for (int q = 0; q < LB::kPieces; q++) {
         int row, col;
-        direct_src(LB{}, B_LAYOUT, q, row, col);
+        direct_src(LB{}, B_LAYOUT, q, lane, row, col);
         if constexpr (OP == kWeightGrad) {
           const int gj = j0 + col;
           const int cj = (!CLAMP || gj < p.J) ? col : (p.J - VEC - j0 > 0 ? p.J - VEC - j0 : 0);
@@ -791,17 +795,19 @@ struct GemmKernel {
       if constexpr (CLAMP) {
         if (slow_last) {
           const u32x4_t z = {0u, 0u, 0u, 0u};
+          int t0 = tid;
+          asm volatile("" : "+v"(t0));   // (as in direct_issue_plain_slow)
           // `plain`: the operand's rows lie in memory as they are (not hashed); g, ld: the operand;
           // x0, ext: the tile's first index and the operand's extent along X
           auto clear = [&](auto L, int layout, T* stage, bool plain, const T* g, int64_t ld, int x0, int ext, int rag_x) {
             typedef decltype(L) LL;
             if (layout == kRStrided) {
               const int first = TR - tail;
-              for (int i = tid; i < tail * (LL::kPitch / VEC); i += kThreads)
+              for (int i = t0; i < tail * (LL::kPitch / VEC); i += kThreads)
                 *reinterpret_cast<u32x4_t*>(stage + first * LL::kPitch + i * VEC) = z;
               // the operand's last row (the last one before `first`), the piece that straddles its end
               const int c = ext - rag_x - x0;
-              if (plain && rag_x && r_end == p.R && c >= 0 && c < LL::kPitch && tid == 0) {
+              if (plain && rag_x && r_end == p.R && c >= 0 && c < LL::kPitch && t0 == 0) {
                 const int row = first - 1;
                 u32x4_t v;
                 __builtin_memcpy(&v, g + (int64_t)(p.R - 1) * ld + (ext - VEC), 16);
@@ -809,13 +815,13 @@ struct GemmKernel {
               }
             } else {
               const int pieces = tail / VEC, first = TR / VEC - pieces;
-              for (int i = tid; i < LL::kRows * pieces; i += kThreads) {
+              for (int i = t0; i < LL::kRows * pieces; i += kThreads) {
                 const int row = i / pieces, pz = first + i % pieces;
                 *reinterpret_cast<u32x4_t*>(stage + row * LL::kPitch + (pz ^ row_swizzle(row)) * VEC) = z;
               }
               if (rag_r) {
                 const int pz = first - 1;   // the piece that straddles R
-                for (int row = tid; row < LL::kRows; row += kThreads) {
+                for (int row = t0; row < LL::kRows; row += kThreads) {
                   u32x4_t* at = reinterpret_cast<u32x4_t*>(stage + row * LL::kPitch + (pz ^ row_swizzle(row)) * VEC);
                   u32x4_t v;
                   if (plain && x0 + row >= ext - 1) {   // the operand's last row, and the rows beyond that repeat it
