@@ -466,7 +466,6 @@ __global__ __launch_bounds__(kFoldSmallThreads) void fold_small_kernel(const Fol
   // (the offsets are fetched whether or not the header turns out to match — the caller vouches for the plan's
   //  size, so the reads stay inside it — so that the two fetches travel together; a plan that does not
   //  match lists nothing)
-  const bool even = p.K % p.h.BK == 0 && p.N % p.h.BN == 0;   // (uniform) every tile lies inside K x N
   int listed = 0;
   for (int first = 0; first < ntiles; first += kLook * kFoldSmallThreads) {
     int rel[kLook];
@@ -510,38 +509,46 @@ __global__ __launch_bounds__(kFoldSmallThreads) void fold_small_kernel(const Fol
   // workgroup's first one) and may lie up to a span outside the tile: inside the tile buffer and its margins,
   // whose values the masks replace by zero.
   float acc[kPer] = {0.f, 0.f, 0.f, 0.f};
-  for (int e0 = wave; e0 < listed; e0 += kWaves * kBatch) {   // (uniform in a wavefront)
-    const int mine = e0 + kWaves * (lane & (kBatch - 1));
-    const int my_id = list_id[mine < listed ? mine : e0];
-    const int my_rel = mine < listed ? list_rel[mine] : kFoldSmallThreads;   // (an empty place: its tile starts behind the span)
-    int id[kBatch], rel[kBatch];
-#pragma unroll
-    for (int u = 0; u < kBatch; u++) {
-      id[u] = __builtin_amdgcn_readlane(my_id, u);
-      rel[u] = __builtin_amdgcn_readlane(my_rel, u);
-    }
-    for (int sl = 0; sl < p.slices; sl++) {
-      const TT* base = reinterpret_cast<const TT*>(p.tiles) + (((int64_t)sl * ntiles) << eshift);
-      TT v[kBatch][kPer];
-#pragma unroll
-      for (int u = 0; u < kBatch; u++) __builtin_memcpy(v[u], base + (((int64_t)id[u] << eshift) - rel[u]) + lane * kPer, sizeof(TT) * kPer);
+  auto add_list = [&](auto whole) {   // whole: every tile lies inside K x N
+    for (int e0 = wave; e0 < listed; e0 += kWaves * kBatch) {   // (uniform in a wavefront)
+      const int mine = e0 + kWaves * (lane & (kBatch - 1));
+      const int my_id = list_id[mine < listed ? mine : e0];
+      const int my_rel = mine < listed ? list_rel[mine] : kFoldSmallThreads;   // (an empty place: its tile starts behind the span)
+      int id[kBatch], rel[kBatch];
 #pragma unroll
       for (int u = 0; u < kBatch; u++) {
-        const int x = lane * kPer - rel[u];   // element of the tile that lands on this lane's first element
-        if (even) {   // (uniform)
+        id[u] = __builtin_amdgcn_readlane(my_id, u);
+        rel[u] = __builtin_amdgcn_readlane(my_rel, u);
+      }
+      for (int sl = 0; sl < p.slices; sl++) {
+        const TT* base = reinterpret_cast<const TT*>(p.tiles) + (((int64_t)sl * ntiles) << eshift);
+        TT v[kBatch][kPer];
 #pragma unroll
-          for (int j = 0; j < kPer; j++) acc[j] += (unsigned)(x + j) < (unsigned)E ? ElemTraits<TT>::to_float(v[u][j]) : 0.f;
-        } else {
-          // rows and columns of the tile inside K x N (what lies beyond was never written)
-          const int tk = id[u] / p.tiles_n, tn = id[u] - tk * p.tiles_n;
-          const int rows = p.K - tk * p.h.BK, cols = p.N - tn * p.h.BN;
+        for (int u = 0; u < kBatch; u++) __builtin_memcpy(v[u], base + (((int64_t)id[u] << eshift) - rel[u]) + lane * kPer, sizeof(TT) * kPer);
+        // (opaque: the masks do not depend on the slice, and worked out ahead of this loop the 32 of them are
+        //  spilled scalar registers)
+        int first = lane * kPer;
+        asm volatile("" : "+v"(first));
 #pragma unroll
-          for (int j = 0; j < kPer; j++)
-            acc[j] += ((unsigned)(x + j) < (unsigned)E && ((x + j) >> p.h.bn_shift) < rows && ((x + j) & (p.h.BN - 1)) < cols) ? ElemTraits<TT>::to_float(v[u][j]) : 0.f;
+        for (int u = 0; u < kBatch; u++) {
+          const int x = first - rel[u];   // element of the tile that lands on this lane's first element
+          if constexpr (decltype(whole)::value) {
+#pragma unroll
+            for (int j = 0; j < kPer; j++) acc[j] += (unsigned)(x + j) < (unsigned)E ? ElemTraits<TT>::to_float(v[u][j]) : 0.f;
+          } else {
+            // rows and columns of the tile inside K x N (what lies beyond was never written)
+            const int tk = id[u] / p.tiles_n, tn = id[u] - tk * p.tiles_n;
+            const int rows = p.K - tk * p.h.BK, cols = p.N - tn * p.h.BN;
+#pragma unroll
+            for (int j = 0; j < kPer; j++)
+              acc[j] += ((unsigned)(x + j) < (unsigned)E && ((x + j) >> p.h.bn_shift) < rows && ((x + j) & (p.h.BN - 1)) < cols) ? ElemTraits<TT>::to_float(v[u][j]) : 0.f;
+          }
         }
       }
     }
-  }
+  };
+  if (p.K % p.h.BK == 0 && p.N % p.h.BN == 0) add_list(std::true_type{});   // (uniform)
+  else add_list(std::false_type{});
   sums[wave][lane] = float4{acc[0], acc[1], acc[2], acc[3]};
   __syncthreads();
   if (tid >= span) return;
