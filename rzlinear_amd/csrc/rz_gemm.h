@@ -11,7 +11,7 @@
 // thread (a 32-bit byte offset per piece); the step only moves a uniform base in scalar
 // registers, and a hashed piece adds its tile's table entry.
 //
-// Register staging (the 16-bit 64 tile, rows shorter than 16 bytes, the single-stage form):
+// Register staging (rows shorter than 16 bytes, the single-stage form, ragged shapes with CLAMP switched off):
 // global -> registers (issued one or two steps ahead) -> LDS (one or two stages).  LDS layouts
 // (X = I or J extent of the operand)
 //   16-bit, R contiguous in the source : [X][TR + 8]   fragment = one ds_read_b128 per lane
@@ -22,7 +22,7 @@
 //   fp32                                : [TR][X + pad], one ds_read_b32 per lane; a source
 //       with R contiguous is transposed while it is written (pad 1), else copied (pad 4)
 //
-// Direct staging (16-bit types: the 128 and 256 tiles; fp32: every tile; two stages; complete
+// Direct staging (every tile; two stages, three or four in the forms of few workgroups; complete
 // tiles, or ragged ones with CLAMP below): the tiles go global -> LDS with
 // direct-to-LDS loads, no registers and no LDS write instructions in between.  Such a load
 // puts the 64 lanes' 16-byte pieces at consecutive LDS addresses, so rows cannot be padded;
@@ -31,7 +31,7 @@
 //   R contiguous : [X][TR], row = 8 pieces; piece p of row x sits at slot p ^ ((x >> 1) & 7)
 //                  (16 pieces with the 256-byte R step: slot p ^ (x & 15))
 //   X contiguous : [TR][X], row = X/32 units of 32 elements; unit u of row r sits at u ^ (r & 3)
-//                  (fp32: u ^ ((r >> 2) & 1))
+//                  (two units per row: u ^ ((r >> 1) & 1); fp32: u ^ ((r >> 2) & 1))
 // Both keep the fragment reads free of bank conflicts.  fp32 fragments of a directly staged tile
 // cover eight elements of R at a time, four MFMAs per pair of blocks: MFMA j of the four contracts
 // elements j (lanes 0-31) and 4 + j (lanes 32-63) — any pairing of the two halves is a valid sum as

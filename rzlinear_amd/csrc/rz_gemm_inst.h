@@ -70,7 +70,7 @@ static hipError_t launch_one(GemmParams p, const WeightGradPlan* plan, const Spl
 }
 
 // FULL kernels carry no bounds checks: every tile and every R step must be complete.  Ragged
-// shapes: the directly staged forms (16-bit tiles of 128 and more, all two-stage fp32 forms) still
+// shapes: the directly staged forms (all but the single-stage one) still
 // stage directly, with edge pieces fetched from inside the operands (CLAMP); everything else takes
 // the bounds-checked kernel.
 template <typename T, int OP, int TILE, int WI, int WJ, int NSTAGE, bool COLSUM = false, int WK = 1, int TILE_J = TILE>
