@@ -109,3 +109,53 @@ def test_fold_of_few_tiles(oracle, shape, dtype, accumulate):
                                           with_bias_grad=True, use_layer_plan=plans)
         assert np.abs(out.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()
         assert_close(dbias.float().cpu().numpy(), dy64.sum(0), dtype, "bias gradient")
+
+
+@pytest.mark.parametrize("dtype", SIXTEEN, ids=str)
+@pytest.mark.parametrize("shape", [
+    (64, 1024, 1024, 20000, 32, 64),      # 16 tiles, four stages, complete
+    (70, 650, 1100, 20000, 64, 64),       # partial tiles and last step
+    (65, 129, 131, 20000, 16, 128),       # one step and a bit, odd row pitches
+    (50, 40, 72, 20000, 32, 64),          # less than one step
+    (1030, 300, 1040, 20000, 32, 64),     # more tiles than compute units: two stages
+    (1025, 257, 1099, 20000, 64, 32),     # ... partial, odd row pitches
+], ids=lambda s: "x".join(map(str, s)))
+def test_16_bit_64_tile(oracle, shape, dtype):
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearBackward import input_grad_hashed, weight_grad_hashed
+    from rzlinear_amd.impl.RzLinearForward import forward_hashed
+    M, K, N, H, BK, BN = shape
+    _say(shape, dtype)
+    (x, hw, dy), (x64, hw64, dy64) = make_inputs(M, K, N, H, dtype, seed=M)
+    R = _lib.hash_constants(*rargs(R1024))
+    with _lib.tuning(tile=64, split=-1, window=-1):
+        y = forward_hashed(x, hw, None, 0.75, M, K, N, H, R, BK, BN, 2)
+        dx = input_grad_hashed(dy, hw, 0.75, M, K, N, H, R, BK, BN, 2)
+        dhw, dbias = weight_grad_hashed(x, dy, 0.75, M, K, N, H, R, BK, BN, out=torch.empty(H, device="cuda"), with_bias_grad=True)
+    assert_close(y.float().cpu().numpy(), oracle.forward(x64, hw64, N, BK, BN, R1024, 0.75), dtype, "y")
+    assert_close(dx.float().cpu().numpy(), oracle.input_grad(dy64, hw64, K, BK, BN, R1024, 0.75), dtype, "dx")
+    ref = oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.75)
+    assert np.abs(dhw.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()   # (fp32 sums of exact products)
+    assert_close(dbias.float().cpu().numpy(), dy64.sum(0), dtype, "bias gradient")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32] + SIXTEEN, ids=str)
+@pytest.mark.parametrize("shape", [
+    (4096, 512, 512, 5243, 64, 64),       # sixteen slices of 128 tiles, complete
+    (4090, 500, 1000, 20000, 32, 64),     # eight, partial tiles and a partial last slice
+    (8191, 511, 509, 9000, 64, 64),       # odd row pitches
+], ids=lambda s: "x".join(map(str, s)))
+def test_weight_grad_in_whole_slices_per_xcd(oracle, shape, dtype):
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearBackward import weight_grad_hashed
+    M, K, N, H, BK, BN = shape
+    _say(shape, dtype)
+    (x, _, dy), (x64, _, dy64) = make_inputs(M, K, N, H, dtype, seed=M)
+    q = _lib.plan_query(2, M, K, N, H, BK, BN, _lib.dtype_code(x), _lib.WG_DHW_F32, True)
+    assert q["mode"] == "lds_image" and q["slices"] % 8 == 0, q
+    dhw, dbias = weight_grad_hashed(x, dy, 0.75, M, K, N, H, _lib.hash_constants(*rargs(R1024)), BK, BN,
+                                    out=torch.empty(H, device="cuda"), with_bias_grad=True)
+    ref = oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.75)
+    # (fp32 sums of M products and about a hundred tiles per element)
+    assert np.abs(dhw.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()
+    assert_close(dbias.float().cpu().numpy(), dy64.sum(0), dtype, "bias gradient")
