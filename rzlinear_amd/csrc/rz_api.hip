@@ -219,40 +219,6 @@ __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __res
   }
 }
 
-// dbias[n] = sum over the rows m of dY[m][n], for the weight-grad forms that do not stage dY
-// tile by tile (the window kernel: short M).  A workgroup owns 64 columns; four thread groups
-// each add up every fourth row, then the groups are combined through LDS in a fixed order.
-template <typename T, typename O>
-__global__ __launch_bounds__(256) void colsum_rows_kernel(const T* __restrict__ dY, int64_t ld, O* __restrict__ out,
-                                                          int N, int M) {
-  __shared__ float sums[4][64];
-  const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
-  const int n = blockIdx.x * 64 + c;
-  float s = 0.f;
-  if (n < N) {
-#pragma unroll 8
-    for (int m = g; m < M; m += 4) s += ElemTraits<T>::to_float(dY[(int64_t)m * ld + n]);
-  }
-  sums[g][c] = s;
-  __syncthreads();
-  if (g == 0 && n < N) out[n] = ElemTraits<O>::from_float((sums[0][c] + sums[1][c]) + (sums[2][c] + sums[3][c]));
-}
-
-static void launch_colsum_rows(int dtype, int out_dtype, const void* dY, int64_t ld, void* out, int N, int M,
-                               hipStream_t s) {
-  const dim3 grid((N + 63) / 64), block(256);
-  if (dtype == RZ_F32)
-    hipLaunchKernelGGL((colsum_rows_kernel<float, float>), grid, block, 0, s, (const float*)dY, ld, (float*)out, N, M);
-  else if (dtype == RZ_BF16 && out_dtype == RZ_F32)
-    hipLaunchKernelGGL((colsum_rows_kernel<bf16_t, float>), grid, block, 0, s, (const bf16_t*)dY, ld, (float*)out, N, M);
-  else if (dtype == RZ_BF16)
-    hipLaunchKernelGGL((colsum_rows_kernel<bf16_t, bf16_t>), grid, block, 0, s, (const bf16_t*)dY, ld, (bf16_t*)out, N, M);
-  else if (out_dtype == RZ_F32)
-    hipLaunchKernelGGL((colsum_rows_kernel<f16_t, float>), grid, block, 0, s, (const f16_t*)dY, ld, (float*)out, N, M);
-  else
-    hipLaunchKernelGGL((colsum_rows_kernel<f16_t, f16_t>), grid, block, 0, s, (const f16_t*)dY, ld, (f16_t*)out, N, M);
-}
-
 // C[i][j] = sum over the slices of part[s][i][j] (+ bias[j]), converted to the element type.
 template <typename T>
 __global__ __launch_bounds__(256) void reduce_slices_kernel(const float* __restrict__ part,
@@ -538,16 +504,14 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
       w.tiles_n = (N + BN - 1) / BN;
       w.accumulate = accumulate ? 1 : 0;
       w.out_f32 = dhw_dtype == RZ_F32 ? 1 : 0;
+      w.dbias = dbias;
+      w.dbias_f32 = dbias_dtype == RZ_F32 ? 1 : 0;
+      w.windows = wp.windows;
       w.poll_limit = tuning.poll_limit > 0 ? tuning.poll_limit : kWindowPollLimit;
       hipError_t e = dtype == RZ_F32 ? launch_window_f32(w, wp.windows, s)
                      : dtype == RZ_BF16 ? launch_window_bf16(w, wp.windows, s)
                                         : launch_window_f16(w, wp.windows, s);
-      if (e != hipSuccess) return RZ_ERR_LAUNCH;
-      if (dbias != nullptr) {
-        launch_colsum_rows(dtype, dbias_dtype, dY, lddy, dbias, N, M, s);
-        if (hipGetLastError() != hipSuccess) return RZ_ERR_LAUNCH;
-      }
-      return RZ_OK;
+      return e == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;
     }
   }
   const ColsumTail bias = {p.colsum, dbias, dbias_dtype, N, plan.colsum_pitch, plan.colsum_rows};

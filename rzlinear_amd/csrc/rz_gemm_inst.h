@@ -185,7 +185,9 @@ static hipError_t launch_window_form(const WindowParams& p, int windows, hipStre
     hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds_limit_raised);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(kernel, dim3((unsigned)windows), dim3(K::kThreads), smem, stream, p);
+  if (p.windows != windows) return hipErrorInvalidValue;
+  const int bias_blocks = p.dbias != nullptr ? (p.N + kWindowBiasCols - 1) / kWindowBiasCols : 0;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(windows + bias_blocks)), dim3(K::kThreads), smem, stream, p);
   return hipGetLastError();
 }
 

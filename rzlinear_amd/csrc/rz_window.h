@@ -48,6 +48,9 @@ struct WindowParams {
   int tiles_k, tiles_n;
   int accumulate;    // dHW += gradient instead of dHW = gradient
   int out_f32;       // dHW is fp32 whatever T is
+  void* dbias;       // non-null: the bias gradient (column sums of dY), made by workgroups behind the windows
+  int dbias_f32;     // ... as fp32 whatever T is
+  int windows;       // workgroups that own a window
   int poll_limit;    // looks at the flags of earlier strips before a wavefront gives up (kWindowPollLimit)
 };
 
@@ -650,10 +653,38 @@ struct WindowKernel {
   }
 };
 
+// dbias[n] = sum over the rows m of dY[m][n].  A workgroup of 1024 threads owns 256 columns; four thread groups each add
+// up every fourth row, then the groups are combined through LDS in a fixed order.  (Two microseconds of work for a few
+// dozen workgroups: as a kernel of its own behind this one it took 4.8 us at M = 128, N = 10240.)
+static constexpr int kWindowBiasCols = 256;
+template <typename T>
+__device__ __forceinline__ void window_colsum(const WindowParams& p, int block, int tid, float* sums) {
+  const int c = tid & (kWindowBiasCols - 1), g = tid / kWindowBiasCols;
+  const int n = block * kWindowBiasCols + c;
+  const T* __restrict__ dY = static_cast<const T*>(p.dY);
+  float s = 0.f;
+  if (n < p.N) {
+#pragma unroll 8
+    for (int m = g; m < p.M; m += 4) s += ElemTraits<T>::to_float(dY[(int64_t)m * p.lddy + n]);
+  }
+  sums[tid] = s;
+  __syncthreads();
+  if (g == 0 && n < p.N) {
+    const float v = (sums[c] + sums[kWindowBiasCols + c]) + (sums[2 * kWindowBiasCols + c] + sums[3 * kWindowBiasCols + c]);
+    if (p.dbias_f32) static_cast<float*>(p.dbias)[n] = v;
+    else static_cast<T*>(p.dbias)[n] = ElemTraits<T>::from_float(v);
+  }
+}
+
 template <typename T, int TBN, bool STAGED>
 __global__ __launch_bounds__((WindowKernel<T, TBN, STAGED>::kThreads)) void rz_window_kernel(WindowParams p) {
   typedef WindowKernel<T, TBN, STAGED> K;
   extern __shared__ __attribute__((aligned(16))) unsigned char rz_window_smem[];
+  static_assert(K::kThreads == 4 * kWindowBiasCols && K::kFixedBytes >= sizeof(float) * K::kThreads, "four row groups, whose sums fit the LDS of any window");
+  if ((int)blockIdx.x >= p.windows) {   // (uniform)
+    window_colsum<T>(p, (int)blockIdx.x - p.windows, threadIdx.x, reinterpret_cast<float*>(rz_window_smem));
+    return;
+  }
   K::run(p, *reinterpret_cast<typename K::Smem*>(rz_window_smem));
 }
 

@@ -159,3 +159,24 @@ def test_weight_grad_in_whole_slices_per_xcd(oracle, shape, dtype):
     # (fp32 sums of M products and about a hundred tiles per element)
     assert np.abs(dhw.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()
     assert_close(dbias.float().cpu().numpy(), dy64.sum(0), dtype, "bias gradient")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32] + SIXTEEN, ids=str)
+@pytest.mark.parametrize("shape", [
+    (32, 512, 256, 60000, 32, 64),    # one workgroup of the bias gradient, complete
+    (33, 512, 264, 60000, 32, 64),    # a second one of eight columns
+    (3, 300, 1001, 60000, 32, 32),    # fewer rows than row groups, odd row pitch
+], ids=lambda s: "x".join(map(str, s)))
+def test_bias_gradient_behind_the_windows(oracle, shape, dtype):
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearBackward import weight_grad_hashed
+    M, K, N, H, BK, BN = shape
+    _say(shape, dtype)
+    (x, _, dy), (x64, _, dy64) = make_inputs(M, K, N, H, dtype, seed=M)
+    with _lib.tuning(window=1, fold=-1, lds_image=-1):
+        assert _lib.plan_query(2, M, K, N, H, BK, BN, _lib.dtype_code(x), _lib.WG_DHW_F32, True)["mode"] == "window"
+        dhw, dbias = weight_grad_hashed(x, dy, 0.75, M, K, N, H, _lib.hash_constants(*rargs(R1024)), BK, BN,
+                                        out=torch.empty(H, device="cuda"), with_bias_grad=True)
+    ref = oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.75)
+    assert np.abs(dhw.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()   # (fp32 sums of exact products)
+    assert_close(dbias.float().cpu().numpy(), dy64.sum(0), dtype, "bias gradient")
