@@ -318,7 +318,7 @@ static int run_plain_op(int op, int dtype, GemmParams p, const void* bias, void*
       p.partial = (float*)workspace;
       // the slice that arrives last at a tile finishes it (adds the slices in slice order, then the
       // bias: the bits of the second kernel's sum) — unless told otherwise, or out of counters
-      p.finish = (tuning.finish != -1 && sp.splits <= finish_slices(sp.tile, p.I, p.J, dtype_bytes(dtype), tuning)) ? finish_counters_for(tile_count(p.I, p.J, sp.tile), s) : nullptr;
+      p.finish = (tuning.finish != -1 && sp.splits <= finish_slices(sp.tile, p.I, p.J, p.R, dtype_bytes(dtype), tuning)) ? finish_counters_for(tile_count(p.I, p.J, sp.tile), s) : nullptr;
       p.bias = p.finish != nullptr ? bias : nullptr;
       if (launch_gemm(dtype, op, p, nullptr, &sp, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
       if (p.finish != nullptr) return RZ_OK;
@@ -1018,7 +1018,7 @@ RZ_API int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int
   const KernelForm f = kernel_form(op, I, J, R, chunk, sp.tile, tile_count(I, J, sp.tile) * sp.splits, eb, t);
   out[0] = sp.tile; out[1] = sp.splits; out[2] = chunk; out[3] = f.step; out[4] = cut ? 1 : 0;
   out[5] = (int32_t)(tile_count(I, J, sp.tile) * sp.splits);
-  out[6] = (cut && t.finish != -1 && sp.splits <= finish_slices(sp.tile, I, J, eb, t) && tile_count(I, J, sp.tile) <= (long long)kFinishPerStream) ? 1 : 0;
+  out[6] = (cut && t.finish != -1 && sp.splits <= finish_slices(sp.tile, I, J, R, eb, t) && tile_count(I, J, sp.tile) <= (long long)kFinishPerStream) ? 1 : 0;
   return RZ_OK;
 }
 

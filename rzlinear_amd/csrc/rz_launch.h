@@ -581,9 +581,11 @@ struct SplitPlan {
 };
 
 // 16-bit forward / input-grad of at most 32 rows whose plan is the 128 tile: C tiles of 32 x 128 (see kernel_form).
-// (An override of the tile gets the square one.)
-static inline bool rows32_form(int tile, int I, int elem_bytes, const rz_tuning& t) {
-  return tile == 128 && elem_bytes == 2 && I <= 32 && t.tile == 0;
+// All that decides it is here, because the planner finishes, and prices, a cut by the kernel that will run: an override
+// of the tile, the single-stage form or register staging (clamp = -1, rows shorter than a 16-byte piece) keeps the
+// square tile.  (A cut of the 128 tile is a multiple of the form's step: slice_unit.)
+static inline bool rows32_form(int tile, int I, int R, int elem_bytes, const rz_tuning& t) {
+  return tile == 128 && elem_bytes == 2 && I <= 32 && R * elem_bytes >= 16 && t.tile == 0 && t.stages != 1 && t.clamp != -1;
 }
 
 // Slices up to which a cut contraction is finished by its own kernel (GemmParams::finish; 0: never).  The
@@ -597,8 +599,8 @@ static inline bool rows32_form(int tile, int I, int elem_bytes, const rz_tuning&
 // Tiles of 32 rows have few values per lane and finish up to eight slices: fp32 M = 32, K = N = 1024 in six slices of the
 // 32 x 64 tile 10.5 / 8.0 us through the module (second kernel / finished in the kernel); the 16-bit 32 x 128 tile, M = 32,
 // K = N = 10240 in three, 29.2 us in one kernel where a second one takes 4.8 us more.
-static inline int finish_slices(int tile, int I, int J, int elem_bytes, const rz_tuning& t) {
-  if (rows32_form(tile, I, elem_bytes, t)) return finish_limit(32);
+static inline int finish_slices(int tile, int I, int J, int R, int elem_bytes, const rz_tuning& t) {
+  if (rows32_form(tile, I, R, elem_bytes, t)) return finish_limit(32);
   if (I < (tile == 32 ? 32 : tile)) return 0;
   if (tile == 256 && (double)I * J * 4.0 < 16.0e6) return 0;
   return finish_limit(tile);
@@ -653,7 +655,7 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
       //  back by the finishing workgroups, and no second kernel is launched — worth a couple of microseconds
       //  and a plane; fp32, M = 16384, K = 512, N = 1024 input-grad, planes of 33 MB: the 256 tile in two
       //  slices 155 us against the whole 128 tile's 136)
-      if (slices > 1 && slices <= finish_slices(tile, I, J, elem_bytes, t) && t.finish != -1) us += (2.0 * slices - 1.0) * (double)I * J * 4.0 / 4.0e6 + 2.0;
+      if (slices > 1 && slices <= finish_slices(tile, I, J, R, elem_bytes, t) && t.finish != -1) us += (2.0 * slices - 1.0) * (double)I * J * 4.0 / 4.0e6 + 2.0;
       else if (slices > 1) us += (2.0 * slices * (double)I * J * 4.0 + (double)I * J * elem_bytes) / 4.0e6 + (direct ? 3.0 : 4.0);
       else whole_us = us;
       // (near ties go to the larger tile and the fewer slices, which come first)
@@ -734,8 +736,7 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
   // LDS stages fit, twice as many bytes of W are in flight, and no padded rows are multiplied or stored, so that the
   // kernel can finish a cut itself (K = N = 10240, H = 6.5 M bf16, three slices: M = 1 28 us, M = 32 44.7 -> 29.2 us, 7.2 TB/s
   // of W from beyond the L2s).  33 to 64 rows: two such tiles would read W twice; the 64 tile takes those.
-  if (rows32_form(tile, I, elem_bytes, t) && op != kWeightGrad && f.stages == 2 && (f.full || f.clamp) &&
-      (chunk >= R || chunk % 128 == 0)) {
+  if (op != kWeightGrad && rows32_form(tile, I, R, elem_bytes, t)) {
     f.rows = 32;
     f.waves = 8;
     f.stages = 3;
