@@ -9,14 +9,15 @@
 //
 // `apply` serves the plain case — dense GPU tensors of one device and dtype, a [H] contiguous hashed_weight, the
 // eight constants as an int32 CPU tensor, an ordinary eager call.  For everything else (tensor subclasses,
-// functorch, tracing, forward-mode tangents, an empty batch, arguments that the launchers refuse) it returns None before
-// it has done anything, and the caller goes through the Python Function, whose checks and errors are the
+// any active functorch transform, tracing, forward-mode tangents, an empty batch, arguments that the launchers refuse)
+// it returns None before it has done anything, and the caller goes through the Python Function, whose checks and errors are the
 // reference's.
 #include <Python.h>
 
 #include <ATen/ATen.h>
 #include <ATen/DeviceGuard.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -313,6 +314,9 @@ PyObject* apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!plain_gpu(x) || !plain_gpu(hw) || (has_bias && !plain_gpu(bias)) || !plain(r) || lib.forward == nullptr) Py_RETURN_NONE;
   if (has_tangent(x) || has_tangent(hw) || has_tangent(bias)) Py_RETURN_NONE;
   if (c10::impl::dispatch_mode_enabled() || torch::jit::tracer::isTracing()) Py_RETURN_NONE;
+  // (inside a functorch transform — the key is included as long as there is one — the Function, which has no rule for
+  //  any, refuses every call, also one whose tensors the transform does not wrap)
+  if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) Py_RETURN_NONE;
   const auto type = x.scalar_type();
   if (dtype_code(type) < 0 || hw.scalar_type() != type || hw.device() != x.device() || x.dim() != 2 || hw.dim() != 1 || !hw.is_contiguous()) Py_RETURN_NONE;
   if (!r.device().is_cpu() || r.scalar_type() != at::kInt || r.numel() != 8 || !r.is_contiguous()) Py_RETURN_NONE;

@@ -150,3 +150,24 @@ def test_vmap_and_batched_gradients_are_refused():
         y = _call(function, x, hw, bias)
         with pytest.raises(RuntimeError):
             torch.autograd.grad(y, x, torch.stack([dy, dy]), is_grads_batched=True)
+
+
+_TRANSFORMS = {
+    "vmap": lambda f, v: torch.func.vmap(f)(v),
+    "grad": lambda f, v: torch.func.grad(lambda s: f(s).sum())(v[0]),
+    "jvp": lambda f, v: torch.func.jvp(f, (v[0],), (v[0],)),
+    "functionalize": lambda f, v: torch.func.functionalize(f)(v[0]),
+}
+
+
+@pytest.mark.parametrize("transform", _TRANSFORMS)
+@pytest.mark.parametrize("constant", [True, False], ids=["constant_input", "transformed_input"])
+def test_every_call_inside_a_transform_is_refused(transform, constant):
+    """... whether or not the transform wraps one of its tensors; and taken again once the transform has ended."""
+    for function in _functions():
+        x, hw, bias, _ = _inputs()
+        scale = torch.randn(3, device="cuda")
+        before = _call(function, x, hw, bias)
+        with pytest.raises(RuntimeError):
+            _TRANSFORMS[transform](lambda s: _call(function, x if constant else x * s, hw, bias) * s, scale)
+        assert torch.equal(_call(function, x, hw, bias), before)
