@@ -17,6 +17,7 @@
 #include <ATen/ATen.h>
 #include <ATen/DeviceGuard.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/hip/HIPContextLight.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -100,8 +101,9 @@ Tensor empty(at::IntArrayRef sizes, const Tensor& like) {
   return at::detail::empty_cuda(sizes, like.scalar_type(), like.device(), std::nullopt);
 }
 
-// scratch memory of one call: handed back to torch's caching allocator, in stream order, when the call returns
-at::DataPtr scratch(size_t bytes) { return bytes ? c10::GetAllocator(c10::kCUDA)->allocate(bytes) : at::DataPtr(); }
+// scratch memory of one call, from the allocator that tensors come from (the caching one, unless the program has put
+// another in its place): handed back, in stream order, when the call returns
+at::DataPtr scratch(size_t bytes) { return bytes ? at::cuda::getCUDADeviceAllocator()->allocate(bytes) : at::DataPtr(); }
 
 void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 

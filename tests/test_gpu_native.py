@@ -1,6 +1,10 @@
 """The native host path of the layer (csrc/rz_torch.cpp) against the Python Function: the same bits for every
 layout it accepts, and the same refusals — what the Function does not support, or would notice, the native
 node must not let through."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -171,3 +175,46 @@ def test_every_call_inside_a_transform_is_refused(transform, constant):
         with pytest.raises(RuntimeError):
             _TRANSFORMS[transform](lambda s: _call(function, x if constant else x * s, hw, bias) * s, scale)
         assert torch.equal(_call(function, x, hw, bias), before)
+
+
+_ALLOCATOR = """
+#include <hip/hip_runtime_api.h>
+#include <sys/types.h>
+extern "C" void* plain_alloc(ssize_t size, int, hipStream_t) {
+  void* p = nullptr;
+  return hipMalloc(&p, (size_t)size) == hipSuccess ? p : nullptr;
+}
+extern "C" void plain_free(void* p, ssize_t, int, hipStream_t) { (void)hipFree(p); }
+"""
+
+_UNDER_ANOTHER_ALLOCATOR = """
+import sys
+import torch
+torch.cuda.memory.change_current_allocator(torch.cuda.memory.CUDAPluggableAllocator(sys.argv[1], "plain_alloc", "plain_free"))
+from helpers import SEED_CONSTANTS
+from rzlinear_amd import RzLinear, _lib
+M, K, N = 1, 2048, 512
+layer = RzLinear(K, N, hashed_weight=torch.nn.Parameter(torch.rand(20000).bfloat16()), dtype=torch.bfloat16).cuda()
+x = torch.randn(M, K).bfloat16().cuda().requires_grad_()
+assert _lib.load().rz_forward_hashed_workspace_bytes(M, K, N, 20000, 32, 64, _lib.RZ_BF16, None) > 0
+got = []
+for call in (layer, lambda v: type("InPython", (__import__("rzlinear_amd").RzLinearFunction,), {}).apply(
+        v, layer._hashed_weight, layer._random_numbers, N, 1, 1.0, 32, 64, layer._bias, False)):
+    y = call(x)
+    got.append((y,) + torch.autograd.grad(y, (x, layer._hashed_weight, layer._bias), torch.ones_like(y)))
+assert all(torch.equal(a, b) for a, b in zip(*got))
+print("same", flush=True)
+"""
+
+
+def test_scratch_comes_from_the_allocator_in_force(tmp_path):
+    """A program that has replaced torch's allocator has no caching allocator to take scratch memory from."""
+    source, library = tmp_path / "allocator.cpp", tmp_path / "allocator.so"
+    source.write_text(_ALLOCATOR)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    subprocess.run(["g++", "-D__HIP_PLATFORM_AMD__", "-I%s/include" % rocm, "-shared", "-fPIC", str(source), "-o", str(library),
+                    "-L%s/lib" % rocm, "-lamdhip64"], check=True)
+    tests = os.path.dirname(os.path.abspath(__file__))
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([os.path.dirname(tests), tests, os.environ.get("PYTHONPATH", "")]))
+    child = subprocess.run([sys.executable, "-c", _UNDER_ANOTHER_ALLOCATOR, str(library)], env=env, capture_output=True, text=True, timeout=100)
+    assert child.returncode == 0 and "same" in child.stdout, child.stdout + child.stderr
