@@ -264,8 +264,10 @@ struct RzLinearNode : public Node {
   }
 
   variable_list apply(variable_list&& grads) override {
-    const bool need_input = task_should_compute_output(0), need_weight = task_should_compute_output(1),
-               need_bias = task_should_compute_output(2);
+    // (a fused weight gradient reaches its buffer in every backward through the layer, whichever gradients that backward
+    //  returns: autograd is not handed it and cannot ask for it)
+    const bool need_input = task_should_compute_output(0), need_bias = task_should_compute_output(2),
+               need_weight = fuse_grad_accumulation ? should_compute_output(1) : task_should_compute_output(1);
     variable_list result(3);
     Tensor x, hw;
     {

@@ -103,6 +103,35 @@ def test_a_second_backward_needs_retain_graph(wanted):
             y.backward(dy)
 
 
+@pytest.mark.parametrize("master", [False, True], ids=["grad", "main_grad"])
+@pytest.mark.parametrize("returned", ["x", "bias", "x and bias", "all leaves"])
+def test_a_fused_weight_gradient_is_added_whichever_gradients_the_backward_returns(returned, master):
+    buffers = []
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        for t in (x, hw, bias):
+            t.requires_grad_()
+        if master:
+            hw.main_grad = torch.zeros(H, device="cuda")
+        for _ in range(2):
+            y = _call(function, x, hw, bias, fuse=True)
+            if returned == "all leaves":
+                y.backward(dy)
+            else:
+                torch.autograd.grad(y, [t for n, t in (("x", x), ("bias", bias)) if n in returned.split()], dy)
+        buffers.append(hw.main_grad if master else hw.grad)
+        assert not master or hw.grad is None
+    assert buffers[0].abs().sum() > 0 and torch.equal(*buffers)
+
+
+def test_no_fused_gradient_for_a_weight_that_needs_none():
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        hw.main_grad = torch.zeros(H, device="cuda")
+        _call(function, x.requires_grad_(), hw, bias, fuse=True).backward(dy)
+        assert hw.grad is None and not hw.main_grad.any()
+
+
 def test_saved_tensor_hooks_see_what_the_function_saves():
     seen = []
     for function in _functions():
