@@ -210,6 +210,10 @@ void weight_grad(const Geometry& g, const Tensor& input, const Tensor& dy, int64
 }
 
 // ---- the autograd node --------------------------------------------------------------------------
+// An edge and a gradient for every tensor that the Function is given, the hash constants among them, which never need
+// one: these are the positions that a hook on the node sees.
+enum { kInput = 0, kWeight = 1, kBias = 3 };   // (2: the hash constants)
+
 struct RzLinearNode : public Node {
   SavedVariable input, hashed_weight, random_numbers;   // (what the Function saves, whichever gradients are wanted)
   Geometry g;
@@ -266,9 +270,10 @@ struct RzLinearNode : public Node {
   variable_list apply(variable_list&& grads) override {
     // (a fused weight gradient reaches its buffer in every backward through the layer, whichever gradients that backward
     //  returns: autograd is not handed it and cannot ask for it)
-    const bool need_input = task_should_compute_output(0), need_bias = task_should_compute_output(2),
-               need_weight = fuse_grad_accumulation ? should_compute_output(1) : task_should_compute_output(1);
-    variable_list result(3);
+    const bool need_input = task_should_compute_output(kInput), need_bias = num_outputs() > kBias && task_should_compute_output(kBias),
+               need_weight = fuse_grad_accumulation ? should_compute_output(kWeight) : task_should_compute_output(kWeight);
+    variable_list result(num_outputs());
+    Tensor bias_grad;
     Tensor x, hw;
     {
       std::lock_guard<std::mutex> lock(mutex_);   // (another thread's backward through this graph may release them)
@@ -283,20 +288,21 @@ struct RzLinearNode : public Node {
     at::DeviceGuard guard(grad.device());
     int64_t lddy;
     const Tensor dy = rows(grad, &lddy);
-    if (need_input) result[0] = input_grad(g, dy, lddy, hw.contiguous());   // (enqueued first, like the reference)
+    if (need_input) result[kInput] = input_grad(g, dy, lddy, hw.contiguous());   // (enqueued first, like the reference)
     if (need_weight) {   // (with a bias: one pass over dy yields both gradients)
-      if (need_bias) result[2] = empty({g.N}, dy);
+      if (need_bias) bias_grad = empty({g.N}, dy);
       bool accumulate = false;
       Tensor out;
       if (fuse_grad_accumulation) {
         out = fused_target(hw, &accumulate);
       } else {
-        out = result[1] = empty({g.H}, dy);
+        out = result[kWeight] = empty({g.H}, dy);
       }
-      weight_grad(g, x, dy, lddy, out, accumulate, result[2], with_plans);
+      weight_grad(g, x, dy, lddy, out, accumulate, bias_grad, with_plans);
     } else if (need_bias) {
-      result[2] = grad.sum(0);
+      bias_grad = grad.sum(0);
     }
+    if (need_bias) result[kBias] = std::move(bias_grad);
     return result;
   }
 };
@@ -355,7 +361,7 @@ PyObject* apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
       status = forward(g, x, hw, bias, &output);
       if (status == RZ_OK && torch::autograd::compute_requires_grad(x, hw, bias)) {
         auto node = std::shared_ptr<RzLinearNode>(new RzLinearNode(), torch::autograd::deleteNode);
-        node->set_next_edges(torch::autograd::collect_next_edges(x, hw, bias));
+        node->set_next_edges(has_bias ? torch::autograd::collect_next_edges(x, hw, r, bias) : torch::autograd::collect_next_edges(x, hw, r));
         node->input = SavedVariable(x, false);
         node->hashed_weight = SavedVariable(hw, false);
         node->random_numbers = SavedVariable(r, false);

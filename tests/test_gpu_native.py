@@ -132,6 +132,23 @@ def test_no_fused_gradient_for_a_weight_that_needs_none():
         assert hw.grad is None and not hw.main_grad.any()
 
 
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_the_node_has_an_edge_and_a_gradient_for_every_tensor(with_bias):
+    seen = []
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        for t in (x, hw, bias):
+            t.requires_grad_()
+        y = _call(function, x, hw, bias if with_bias else None)
+        targets = [getattr(n, "variable", None) for n, _ in y.grad_fn.next_functions]
+        assert [t is e for t, e in zip(targets, (x, hw, None, bias))] == [True] * (3 + with_bias)
+        shapes = []
+        y.grad_fn.register_hook(lambda ins, outs: shapes.append([None if g is None else tuple(g.shape) for g in ins + outs]))
+        y.backward(dy)
+        seen.append(shapes)
+    assert seen[0] == seen[1] and len(seen[0]) == 1
+
+
 def test_saved_tensor_hooks_see_what_the_function_saves():
     seen = []
     for function in _functions():
