@@ -329,7 +329,7 @@ PyObject* apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) Py_RETURN_NONE;
   const auto type = x.scalar_type();
   if (dtype_code(type) < 0 || hw.scalar_type() != type || hw.device() != x.device() || x.dim() != 2 || hw.dim() != 1 || !hw.is_contiguous()) Py_RETURN_NONE;
-  if (!r.device().is_cpu() || r.scalar_type() != at::kInt || r.numel() != 8 || !r.is_contiguous()) Py_RETURN_NONE;
+  if (!r.device().is_cpu() || r.scalar_type() != at::kInt || r.dim() != 1 || r.numel() != 8 || !r.is_contiguous()) Py_RETURN_NONE;
   long v[3];   // output_dim, BK, BN
   for (int i = 0; i < 3; i++) {
     PyObject* o = args[i == 0 ? 3 : i + 4];

@@ -181,6 +181,41 @@ def test_what_a_hook_hands_back_is_checked_before_a_kernel_sees_it(unpack):
         y.backward(dy)
 
 
+_REFUSED = {   # name: (index of the argument of apply, what takes its place)
+    "constants in two rows": (2, lambda t: t.view(2, 4)),
+    "seven constants": (2, lambda t: t[:7]),
+    "a negative constant": (2, lambda t: -t),
+    "constants in a list": (2, lambda t: t.tolist()),
+    "a batch of matrices": (0, lambda t: t[None]),
+    "a vector": (0, lambda t: t[0]),
+    "another input dtype": (0, lambda t: t.half()),
+    "input on the host": (0, lambda t: t.cpu()),
+    "a two-dimensional weight": (1, lambda t: t.view(9, -1)),
+    "a weight of one tile": (1, lambda t: t[:TILE[0] * TILE[1]]),
+    "weight on the host": (1, lambda t: t.cpu()),
+    "a short bias": (8, lambda t: t[:-1]),
+    "another bias dtype": (8, lambda t: t.half()),
+    "no output columns": (3, lambda n: 0),
+    "a fraction of columns": (3, lambda n: float(n)),
+    "a tile of 24 rows": (6, lambda n: 24),
+    "no scale": (5, lambda f: None),
+}
+
+
+@pytest.mark.parametrize("name", _REFUSED)
+def test_what_the_function_refuses_is_refused_alike(name):
+    at, change = _REFUSED[name]
+    kinds = []
+    for function in _functions():
+        x, hw, bias, _ = _inputs()
+        args = [x, hw, R, N, 1, 0.5, *TILE, bias, False]
+        args[at] = change(args[at])
+        with pytest.raises(Exception) as refused:
+            function.apply(*args)
+        kinds.append(refused.type)
+    assert kinds[0] is kinds[1]
+
+
 def test_forward_mode_is_refused():
     for function in _functions():
         for which in range(3):
