@@ -16,8 +16,10 @@
 
 #include <ATen/ATen.h>
 #include <ATen/DeviceGuard.h>
+#include <ATen/SequenceNumber.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/HIPContextLight.h>
+#include <ATen/record_function.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
@@ -355,6 +357,13 @@ PyObject* apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
   std::copy(r.data_ptr<int32_t>(), r.data_ptr<int32_t>() + 8, g.R);
   Tensor output;
   int status;
+  // what a profiler sees: the Function's name and arguments (the backward is named by the node)
+  at::RecordFunction event(at::RecordScope::FUNCTION);
+  if (event.isActive()) {
+    const c10::IValue none;
+    const std::array<c10::IValue, 10> inputs = {x, hw, r, none, none, none, none, none, has_bias ? c10::IValue(bias) : none, none};
+    at::detail::record_function_with_scope(event, "RzLinearFunction", inputs, (int64_t)at::sequence_number::peek());
+  }
   {
     PyThreadState* saved = PyEval_SaveThread();   // (a full launch queue makes the runtime wait)
     try {

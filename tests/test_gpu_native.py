@@ -258,6 +258,23 @@ def test_every_call_inside_a_transform_is_refused(transform, constant):
         assert torch.equal(_call(function, x, hw, bias), before)
 
 
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_a_profiler_names_forward_and_backward(with_bias):
+    seen = []
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        x.requires_grad_()
+        for _ in range(2):   # (not the first call: that one also builds what it keeps)
+            with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], record_shapes=True) as profile:
+                y = _call(function, x, hw, bias if with_bias else None)
+                y.backward(dy)
+        events = {e.name: e for e in profile.events()}
+        forward, backward = events[function.__name__], events[function.__name__ + "Backward"]
+        assert forward.sequence_nr == backward.sequence_nr >= 0
+        seen.append((forward.input_shapes, backward.input_shapes))
+    assert seen[0] == seen[1]
+
+
 _ALLOCATOR = """
 #include <hip/hip_runtime_api.h>
 #include <sys/types.h>
