@@ -201,10 +201,11 @@ def native():
             raise RuntimeError("rzlinear_amd/_native.so is not built; run `python -m rzlinear_amd.build`. "
                                "rzlinear_amd has no fallback path.")
         from . import _native as module
+        from .RzLinearFunction import _function_output
         lib = load()
         module.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in EXPORTS},
                     lambda K, N, H, BK, BN, R, levels, index: layer_plan(
-                        K, N, H, BK, BN, (ctypes.c_int32 * 8)(*R), levels, torch.device("cuda", index)), check)
+                        K, N, H, BK, BN, (ctypes.c_int32 * 8)(*R), levels, torch.device("cuda", index)), check, _function_output)
         _native = module
         _tell_native()
     return _native

@@ -58,6 +58,7 @@ struct Library {
 Library lib;
 PyObject* plan_provider = nullptr;    // Python: (K, N, H, BK, BN, constants, levels, device index) -> plan tensor
 PyObject* status_check = nullptr;     // Python: raises for a non-zero status
+PyObject* function_node = nullptr;    // Python: the Function's own node for given saved tensors and arguments
 // What the Python side's `tuning` context has set (tests, benchmarks): a copy, which a call that is under way
 // in another thread keeps alive.
 std::shared_ptr<const rz_tuning> tuning_in_force;
@@ -222,14 +223,52 @@ struct RzLinearNode : public Node {
   c10::SmallVector<int64_t, 2> output_sizes;
   at::TensorOptions output_options;
   bool fuse_grad_accumulation = false, with_plans = true;
+  // (compiled autograd only) the node that the Function would have left here
+  std::shared_ptr<Node> of_function;
 
   std::string name() const override { return "RzLinearFunctionBackward"; }
 
   void release_variables() override {
-    std::lock_guard<std::mutex> lock(mutex_);
-    input.reset_data();
-    hashed_weight.reset_data();
-    random_numbers.reset_data();
+    std::shared_ptr<Node> other;
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      input.reset_data();
+      hashed_weight.reset_data();
+      random_numbers.reset_data();
+      other.swap(of_function);
+    }
+    if (other) other->release_variables();
+  }
+
+  // Compiled autograd does not run a node: it collects what the node has saved and records a call of its backward.
+  // The Function's node can be taken apart like that, so one is made, with the same edges, and stands in for this one.
+  void compiled_args(torch::dynamo::autograd::CompiledNodeArgs& args) const override { const_cast<RzLinearNode*>(this)->function_twin().compiled_args(args); }
+  variable_list apply_with_saved(const variable_list& inputs, torch::dynamo::autograd::SwapSavedVariables& saved) override {
+    return function_twin().apply_with_saved(inputs, saved);
+  }
+  Node& function_twin() {
+    if (of_function) return *of_function;
+    const variable_list kept = saved();
+    const bool has_bias = num_outputs() > kBias;
+    PyGILState_STATE gil = PyGILState_Ensure();
+    PyObject* r = PyObject_CallFunction(function_node, "NNNifiiOOO", THPVariable_Wrap(kept[0]), THPVariable_Wrap(kept[1]), THPVariable_Wrap(kept[2]),
+                                        g.N, g.scale, g.BK, g.BN, has_bias ? Py_True : Py_False,
+                                        has_bias && should_compute_output(kBias) ? Py_True : Py_False, fuse_grad_accumulation ? Py_True : Py_False);
+    python_error err;
+    if (r == nullptr) err.persist();
+    else if (THPVariable_Check(r)) of_function = THPVariable_Unpack(r).grad_fn();
+    Py_XDECREF(r);
+    PyGILState_Release(gil);
+    if (r == nullptr) throw err;
+    TORCH_CHECK(of_function, "the Function left no node");
+    of_function->set_next_edges(torch::autograd::edge_list(next_edges()));
+    return *of_function;
+  }
+
+  // input, hashed_weight and the hash constants (an error if they have been freed, or changed in place since the forward)
+  variable_list saved() {
+    std::lock_guard<std::mutex> lock(mutex_);   // (another thread's backward through this graph may release them)
+    return {input.unpack(), hashed_weight.unpack(), random_numbers.unpack()};
   }
 
   // What a saved-tensor hook hands back, and a gradient, may be anything: the pointers below go straight to kernels.
@@ -276,13 +315,9 @@ struct RzLinearNode : public Node {
                need_weight = fuse_grad_accumulation ? should_compute_output(kWeight) : task_should_compute_output(kWeight);
     variable_list result(num_outputs());
     Tensor bias_grad;
-    Tensor x, hw;
-    {
-      std::lock_guard<std::mutex> lock(mutex_);   // (another thread's backward through this graph may release them)
-      x = input.unpack();
-      hw = hashed_weight.unpack();
-      random_numbers.unpack();   // (freed, or changed in place since the forward: an error, as for the others)
-    }
+    const variable_list kept = saved();
+    const Tensor& x = kept[0];
+    Tensor hw = kept[1];
     Tensor grad = grads[0].defined() ? grads[0] : at::zeros(output_sizes, output_options);
     require(grad, "output_grad", output_sizes[0], g.N, grad);
     if (need_input) require(hw, "hashed_weight", g.H, -1, grad);
@@ -392,10 +427,10 @@ PyObject* apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind({entry point: address}, plan_provider, status_check)
+// bind({entry point: address}, plan_provider, status_check, function_node)
 PyObject* bind(PyObject*, PyObject* args) {
-  PyObject *table, *provider, *checker;
-  if (!PyArg_ParseTuple(args, "O!OO", &PyDict_Type, &table, &provider, &checker)) return nullptr;
+  PyObject *table, *provider, *checker, *maker;
+  if (!PyArg_ParseTuple(args, "O!OOO", &PyDict_Type, &table, &provider, &checker, &maker)) return nullptr;
   auto address = [&](const char* name) -> void* {
     PyObject* o = PyDict_GetItemString(table, name);
     if (o == nullptr) PyErr_Format(PyExc_KeyError, "no address for %s", name);
@@ -415,10 +450,13 @@ PyObject* bind(PyObject*, PyObject* args) {
 #undef RZ_BIND
   Py_INCREF(provider);
   Py_INCREF(checker);
+  Py_INCREF(maker);
   Py_XDECREF(plan_provider);
   Py_XDECREF(status_check);
+  Py_XDECREF(function_node);
   plan_provider = provider;
   status_check = checker;
+  function_node = maker;
   lib = l;
   Py_RETURN_NONE;
 }

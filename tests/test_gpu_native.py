@@ -258,6 +258,38 @@ def test_every_call_inside_a_transform_is_refused(transform, constant):
         assert torch.equal(_call(function, x, hw, bias), before)
 
 
+@pytest.mark.parametrize("fuse", [False, True])
+@pytest.mark.parametrize("wanted", [(1, 1, 1), (1, 0, 0), (0, 1, 0), (0, 0, 1), (0, 1, None), (1, 1, None)])
+def test_compiled_autograd_takes_the_node_apart(wanted, fuse):
+    from torch._dynamo import compiled_autograd
+    got = []
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        leaves = (x, hw) if wanted[2] is None else (x, hw, bias)
+        for t, w in zip(leaves, wanted):
+            t.requires_grad_(bool(w))
+        # (behind an operation and in front of one, so that edges of both kinds are met)
+        y = _call(function, x * 2, hw, bias if wanted[2] is not None else None, fuse=fuse) * 3
+        with compiled_autograd._enable(torch.compile(backend="eager")):
+            y.backward(dy, retain_graph=True)
+            y.backward(dy)
+            with pytest.raises(RuntimeError, match="second time"):
+                y.backward(dy)
+        assert [t.grad is not None for t in leaves] == [bool(w) for w in wanted[:len(leaves)]]
+        got.append([t.grad for t in leaves if t.grad is not None])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+def test_compiled_autograd_notices_a_change_in_place():
+    from torch._dynamo import compiled_autograd
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        y = _call(function, x, hw.requires_grad_(), bias)
+        x.add_(1)
+        with compiled_autograd._enable(torch.compile(backend="eager")), pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            y.backward(dy)
+
+
 @pytest.mark.parametrize("with_bias", [False, True])
 def test_a_profiler_names_forward_and_backward(with_bias):
     seen = []
