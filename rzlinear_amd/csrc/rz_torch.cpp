@@ -26,6 +26,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -122,6 +123,14 @@ void check(int status) {
   if (r == nullptr) throw err;
   TORCH_CHECK(false, "librzlinear: status ", status);
 }
+
+// Lets go of the interpreter lock for its lifetime, if this thread holds it.
+struct WithoutGil {
+  PyThreadState* held = PyGILState_Check() ? PyEval_SaveThread() : nullptr;
+  ~WithoutGil() {
+    if (held != nullptr) PyEval_RestoreThread(held);
+  }
+};
 
 // ---- layer plans --------------------------------------------------------------------------------
 // Built and owned by the Python side (_lib.layer_plan); kept here too, so that a step need not ask for them
@@ -267,6 +276,7 @@ struct RzLinearNode : public Node {
 
   // input, hashed_weight and the hash constants (an error if they have been freed, or changed in place since the forward)
   variable_list saved() {
+    const WithoutGil released;   // (a saved-tensor hook of the thread that holds the mutex may be waiting for it)
     std::lock_guard<std::mutex> lock(mutex_);   // (another thread's backward through this graph may release them)
     return {input.unpack(), hashed_weight.unpack(), random_numbers.unpack()};
   }
@@ -343,6 +353,26 @@ struct RzLinearNode : public Node {
     return result;
   }
 };
+
+// ---- the node as Python sees it: grad_fn of the layer's output ----------------------------------
+PyObject* saved_tensors(PyObject* self, void*) {
+  HANDLE_TH_ERRORS
+  auto* node = static_cast<RzLinearNode*>(reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata.get());
+  const variable_list kept = node->saved();
+  return Py_BuildValue("NNN", THPVariable_Wrap(kept[0]), THPVariable_Wrap(kept[1]), THPVariable_Wrap(kept[2]));
+  END_HANDLE_TH_ERRORS
+}
+
+bool register_node_type() {
+  using namespace torch::autograd;
+  static PyTypeObject type;
+  static PyGetSetDef properties[] = {THP_FUNCTION_DEFAULT_PROPERTIES,
+                                     {"saved_tensors", saved_tensors, nullptr, "what the forward kept for the backward", nullptr},
+                                     {nullptr, nullptr, nullptr, nullptr, nullptr}};
+  if (_initFunctionPyTypeObject(type, "RzLinearFunctionBackward", properties, nullptr) == nullptr) return false;
+  registerCppFunction(typeid(RzLinearNode), &type);
+  return true;
+}
 
 // ---- apply(input, hashed_weight, random_numbers, output_dim, init_factor, BK, BN, bias, fuse, with_plans) ----
 PyObject* apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -491,4 +521,4 @@ PyModuleDef definition = {PyModuleDef_HEAD_INIT, "_native", "native host path of
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&definition); }
+PyMODINIT_FUNC PyInit__native() { return register_node_type() ? PyModule_Create(&definition) : nullptr; }

@@ -149,6 +149,18 @@ def test_the_node_has_an_edge_and_a_gradient_for_every_tensor(with_bias):
     assert seen[0] == seen[1] and len(seen[0]) == 1
 
 
+def test_the_node_shows_what_it_has_saved():
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        y = _call(function, x, hw.requires_grad_(), bias)
+        assert type(y.grad_fn).__name__ == y.grad_fn.name() == function.__name__ + "Backward"
+        saved = y.grad_fn.saved_tensors
+        assert type(saved) is tuple and [a is b for a, b in zip(saved, (x, hw, R))] == [True, True, True]
+        y.backward(dy)
+        with pytest.raises(RuntimeError, match="second time"):
+            y.grad_fn.saved_tensors
+
+
 def test_saved_tensor_hooks_see_what_the_function_saves():
     seen = []
     for function in _functions():
