@@ -60,6 +60,41 @@ def test_16_bit_at_most_32_rows(oracle, shape, split, slices, finished, dtype):
     _forward_and_mirrored_input_grad(oracle, shape, dtype, split, 128, slices, finished)
 
 
+@pytest.mark.parametrize("dtype,shape,slices", [
+    (torch.bfloat16, (32, 2048, 2048, 20000, 32, 64), 8),
+    (torch.float16, (1, 2048, 512, 20000, 32, 64), 8),
+    (torch.bfloat16, (7, 2049, 2040, 20000, 128, 32), 6),
+    (torch.float32, (32, 1024, 1024, 20000, 32, 64), 6),
+], ids=str)
+def test_a_captured_cut_takes_the_second_kernel_with_the_same_bits(dtype, shape, slices):
+    """A stream under capture gets no counters: the same plan, its planes added by the second kernel.  (The `finish`
+    override, which does that too, may change the plan.)"""
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearForward import forward_hashed
+    M, K, N, H, BK, BN = shape
+    _say("captured", shape, dtype)
+    (x, hw, _), _ = make_inputs(M, K, N, H, dtype, seed=M + K)
+    bias = torch.randn((N,), generator=torch.Generator().manual_seed(4)).to(dtype).cuda()
+    q = _lib.plan_query(0, M, K, N, H, BK, BN, _lib.dtype_code(x))
+    assert (q["slices"], q["shares"]) == (slices, 1)
+
+    def forward():
+        return forward_hashed(x, hw, bias, 0.75, M, K, N, H, _lib.hash_constants(*rargs(R1024)), BK, BN, 2)
+
+    forward()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = forward()
+    for replay in range(3):
+        x.copy_(torch.randn((M, K), generator=torch.Generator().manual_seed(replay)).to(dtype))
+        finished = forward()
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, finished), replay
+
+
 @pytest.mark.parametrize("dtype", SIXTEEN, ids=str)
 def test_16_bit_at_most_32_rows_uncut(oracle, dtype):
     from rzlinear_amd import _lib
