@@ -74,38 +74,38 @@ TRAFFIC = {
     #  FETCH_SIZE = 131085, WRITE_SIZE = 262144)
     ("square4096", "bf16"): {
         "profile": "profiles/rz_gemm_bf16_square4096.txt",
-        "bytes": {"forward": int((16679.6 * 2.0 + 32768.0) * 1024),       # algorithmic: 64.03 MiB
-                  "input_grad": int((16676.4 * 2.0 + 32768.0) * 1024),
-                  "weight_grad": int((98478.0 * 2.0 + 16784.6) * 1024)},  # X, dY re-read by the XCDs' tile groups; + partial images
+        "bytes": {"forward": int((16691.8 * 2.0 + 32768.0) * 1024),       # algorithmic: 64.03 MiB
+                  "input_grad": int((16677.6 * 2.0 + 32768.0) * 1024),
+                  "weight_grad": int((98477.3 * 2.0 + 16780.4) * 1024)},  # X, dY re-read by the XCDs' tile groups; + partial images
     },
     ("square2048", "bf16"): {
         "profile": "profiles/rz_gemm_bf16_square2048.txt",
-        "bytes": {"forward": int((4349.3 * 2.0 + 8192.0) * 1024), "input_grad": int((4342.2 * 2.0 + 8192.0) * 1024),
-                  "weight_grad": int((24699.1 * 2.0 + 16384.0) * 1024)},
+        "bytes": {"forward": int((4349.6 * 2.0 + 8192.0) * 1024), "input_grad": int((4331.5 * 2.0 + 8192.0) * 1024),
+                  "weight_grad": int((24695.7 * 2.0 + 16384.0) * 1024)},
     },
     ("square4096", "fp32"): {
         "profile": "profiles/rz_gemm_fp32_square4096.txt",
-        "bytes": {"forward": int((33229.8 * 2.0 + 65536.0) * 1024),       # algorithmic: 128.06 MiB
-                  "input_grad": int((33225.7 * 2.0 + 65536.0) * 1024),
-                  "weight_grad": int((196812.8 * 2.0 + 16784.7) * 1024)},
+        "bytes": {"forward": int((33235.6 * 2.0 + 65536.0) * 1024),       # algorithmic: 128.06 MiB
+                  "input_grad": int((33227.7 * 2.0 + 65536.0) * 1024),
+                  "weight_grad": int((196813.9 * 2.0 + 16780.6) * 1024)},
     },
     ("cpu_ref_1024", "fp32"): {
         "profile": "profiles/rz_gemm_fp32_cpu_ref_1024.txt",
-        "bytes": {"forward": int((3160.8 * 2.0 + 4096.0) * 1024), "input_grad": int((3159.0 * 2.0 + 4096.0) * 1024),
-                  "weight_grad": int((12338.6 * 2.0 + 4096.0) * 1024)},   # X^T.dY written tile by tile: 4 MiB
+        "bytes": {"forward": int((3162.0 * 2.0 + 4096.0) * 1024), "input_grad": int((3157.0 * 2.0 + 4096.0) * 1024),
+                  "weight_grad": int((12338.5 * 2.0 + 4096.0) * 1024)},   # X^T.dY written tile by tile: 4 MiB
     },
     ("ffn", "bf16"): {
         "profile": "profiles/rz_gemm_fold_bf16_ffn.txt",
-        "bytes": {"forward": int((70690.9 * 2.0 + 262144.0) * 1024),      # algorithmic: 320.1 MiB
-                  "input_grad": int((132331.1 * 2.0 + 65536.0) * 1024),
+        "bytes": {"forward": int((70672.0 * 2.0 + 262144.0) * 1024),      # algorithmic: 320.1 MiB
+                  "input_grad": int((132301.2 * 2.0 + 65536.0) * 1024),
                   # contraction (X, dY re-read by the XCDs' tile groups; X^T.dY written tile by tile in bf16: 128 MiB)
-                  "weight_grad": int((786599.9 * 2.0 + 131072.0) * 1024)},
+                  "weight_grad": int((786602.3 * 2.0 + 131072.0) * 1024)},
     },
     ("grid_1024_10240", "bf16"): {
         "profile": "profiles/rz_gemm_fold_bf16_grid_1024_10240.txt",
-        "bytes": {"forward": int((396677.9 * 2.0 + 143380.0) * 1024),     # (three slices: fp32 partial planes written, read back by the slice that finishes)
-                  "input_grad": int((382509.1 * 2.0 + 143380.1) * 1024),
-                  "weight_grad": int((172198.8 * 2.0 + 204800.0) * 1024)},      # (X^T.dY tile by tile in bf16: 200 MiB)
+        "bytes": {"forward": int((396950.8 * 2.0 + 143380.0) * 1024),     # (three slices: fp32 partial planes written, read back by the slice that finishes)
+                  "input_grad": int((382347.7 * 2.0 + 143380.0) * 1024),
+                  "weight_grad": int((172202.6 * 2.0 + 204800.0) * 1024)},      # (X^T.dY tile by tile in bf16: 200 MiB)
     },
 }
 
