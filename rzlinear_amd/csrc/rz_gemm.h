@@ -382,7 +382,8 @@ struct GemmKernel {
     // gets a contiguous run of tiles, then walk tiles with J fastest (forward/input-grad
     // share the streamed A panel) or in square-ish groups (weight-grad streams both).
     // Weight-grad in a multiple of eight slices: slices have no operand in common, so every XCD takes whole
-    // slices, each operand read by one L2 (M = 16384, K = 512, N = 1024 bf16 in eight slices: 29.7 -> 21.5 us).
+    // slices, each operand read by one L2 (bf16, weight-grad with what adds up the images: M = 16384, K = 512, N = 1024 in
+    // eight slices 32.5 -> 25.6 us, of which this kernel 29.7 -> 23.6; M = 32768, K = N = 512 in sixteen 36.4 -> 25.6 us).
     // Not where an XCD would get parts of slices, nor for the cuts of forward and input-grad, whose finishing
     // slice finds the others' planes in its own L2 (M = 128, K = N = 10240 bf16 in three slices 42 -> 47 us;
     // M = 3001, K = 2047, N = 1531 fp16 weight-grad in five slices 52 -> 55 us).

@@ -598,7 +598,7 @@ static inline bool rows32_form(int tile, int I, int R, int elem_bytes, const rz_
 // M = 64, K = N = 4096: 64 tile, four slices 12.7 / 13.6; 128 tile 21.3 / 18.4.  Six slices at M = 32: 52 / 40.
 // Tiles of 32 rows have few values per lane and finish up to eight slices: fp32 M = 32, K = N = 1024 in six slices of the
 // 32 x 64 tile 10.5 / 8.0 us through the module (second kernel / finished in the kernel); the 16-bit 32 x 128 tile, M = 32,
-// K = N = 10240 in three, 29.2 us in one kernel where a second one takes 4.8 us more.
+// K = N = 10240 in three, 29.4 us in one kernel where a second one takes 4.8 us more.
 static inline int finish_slices(int tile, int I, int J, int R, int elem_bytes, const rz_tuning& t) {
   if (rows32_form(tile, I, R, elem_bytes, t)) return finish_limit(32);
   if (I < (tile == 32 ? 32 : tile)) return 0;
@@ -734,8 +734,8 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
   // 16-bit forward / input-grad on the planner's 128 tile, a batch of at most 32 rows (decoding): C tiles of 32 x 128.
   // The 128 rows of the square tile would stage the batch four times over beside every piece of W; without them three
   // LDS stages fit, twice as many bytes of W are in flight, and no padded rows are multiplied or stored, so that the
-  // kernel can finish a cut itself (K = N = 10240, H = 6.5 M bf16, three slices: M = 1 28 us, M = 32 44.7 -> 29.2 us, 7.2 TB/s
-  // of W from beyond the L2s).  33 to 64 rows: two such tiles would read W twice; the 64 tile takes those.
+  // kernel can finish a cut itself (K = N = 10240, H = 6.5 M bf16, three slices: M = 1 43.5 -> 28.3 us, M = 32 42.0 -> 29.4 us,
+  // 7.1 TB/s of W from beyond the L2s).  33 to 64 rows: two such tiles would read W twice; the 64 tile takes those.
   if (op != kWeightGrad && rows32_form(tile, I, R, elem_bytes, t)) {
     f.rows = 32;
     f.waves = 8;
