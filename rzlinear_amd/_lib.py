@@ -206,6 +206,7 @@ def native():
         module.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in EXPORTS},
                     lambda K, N, H, BK, BN, R, levels, index: layer_plan(
                         K, N, H, BK, BN, (ctypes.c_int32 * 8)(*R), levels, torch.device("cuda", index)), check, _function_output)
+        torch.autograd.graph.Node.register(module.RzLinearFunctionBackward)   # (isinstance, as for any other node)
         _native = module
         _tell_native()
     return _native

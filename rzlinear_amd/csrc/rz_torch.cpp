@@ -363,15 +363,16 @@ PyObject* saved_tensors(PyObject* self, void*) {
   END_HANDLE_TH_ERRORS
 }
 
-bool register_node_type() {
+PyTypeObject node_type;
+
+bool register_node_type(PyObject* module) {
   using namespace torch::autograd;
-  static PyTypeObject type;
   static PyGetSetDef properties[] = {THP_FUNCTION_DEFAULT_PROPERTIES,
                                      {"saved_tensors", saved_tensors, nullptr, "what the forward kept for the backward", nullptr},
                                      {nullptr, nullptr, nullptr, nullptr, nullptr}};
-  if (_initFunctionPyTypeObject(type, "RzLinearFunctionBackward", properties, nullptr) == nullptr) return false;
-  registerCppFunction(typeid(RzLinearNode), &type);
-  return true;
+  if (_initFunctionPyTypeObject(node_type, "RzLinearFunctionBackward", properties, nullptr) == nullptr) return false;
+  registerCppFunction(typeid(RzLinearNode), &node_type);
+  return PyModule_AddObjectRef(module, "RzLinearFunctionBackward", reinterpret_cast<PyObject*>(&node_type)) == 0;
 }
 
 // ---- apply(input, hashed_weight, random_numbers, output_dim, init_factor, BK, BN, bias, fuse, with_plans) ----
@@ -521,4 +522,8 @@ PyModuleDef definition = {PyModuleDef_HEAD_INIT, "_native", "native host path of
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native() { return register_node_type() ? PyModule_Create(&definition) : nullptr; }
+PyMODINIT_FUNC PyInit__native() {
+  PyObject* module = PyModule_Create(&definition);
+  if (module != nullptr && !register_node_type(module)) Py_CLEAR(module);
+  return module;
+}

@@ -154,6 +154,7 @@ def test_the_node_shows_what_it_has_saved():
         x, hw, bias, dy = _inputs()
         y = _call(function, x, hw.requires_grad_(), bias)
         assert type(y.grad_fn).__name__ == y.grad_fn.name() == function.__name__ + "Backward"
+        assert isinstance(y.grad_fn, torch.autograd.graph.Node)
         saved = y.grad_fn.saved_tensors
         assert type(saved) is tuple and [a is b for a, b in zip(saved, (x, hw, R))] == [True, True, True]
         y.backward(dy)
