@@ -174,12 +174,10 @@ struct GemmKernel {
   static constexpr int kThreads = 64 * WI * WJ * WK;
   static constexpr int VEC = Tr::kVec;
   static constexpr bool k16 = (Tr::kBytes == 2);
-  // R step: 128 bytes of R — except the directly staged 128 tile with eight wavefronts, which
-  // is used at about one workgroup per compute unit and has LDS to spare: it takes 256 bytes
-  // per step, halving the barriers per flop (8 % faster at 2048^3).
-  // ... and the directly staged 64 tile, whose sixteen wavefronts share a step four ways.
+  // R step: 128 bytes of R — except the directly staged 16-bit 64 and 32 x 128 tiles, whose groups of wavefronts
+  // share a step of 256 bytes.
   static constexpr bool kLongStep = Tr::kBytes == 2 && (FULL || CLAMP) && NSTAGE >= 2 &&
-                                    ((TI == 128 && TJ == 128 && WI * WJ == 8) || (TI == 64 && TJ == 64) || TI == 32);
+                                    ((TI == 64 && TJ == 64) || TI == 32);
   // ... and the fp32 tiles of at most 64 rows in forward / input-grad, whose 128-byte step is over in
   // 0.4 us — less than a load from L2 takes, so that loads issued two steps ahead arrive late, and
   // half as many barriers per flop (1024^3: forward 30.2 -> 28.3 us, input-grad 27.1 -> 25.9 us;

@@ -87,13 +87,13 @@ static hipError_t launch_tile(GemmParams p, const WeightGradPlan* plan, const Sp
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false>::TR) return hipErrorInvalidValue;
     return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, false, WK>(p, plan, split, stream);
   }
-  // (the 16-bit 64 tile of four wavefronts serves rows shorter than a 16-byte piece only)
-  constexpr bool kCheckedOnly = sizeof(T) == 2 && TILE == 64 && WK == 1;
+  // (the 16-bit 64 tile of four wavefronts, and the 128 tile of eight with two stages, serve rows shorter than a 16-byte piece only)
+  constexpr bool kCheckedOnly = sizeof(T) == 2 && WK == 1 && (TILE == 64 || (TILE == 128 && WI * WJ == 8 && NSTAGE == 2));
   if constexpr (!kCheckedOnly) if (form.full) {
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true>::TR) return hipErrorInvalidValue;
     return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true, COLSUM, false, WK>(p, plan, split, stream);
   }
-  constexpr bool kDirectOnly = WI * WJ * WK == 16 || (sizeof(T) == 2 && NSTAGE == 3);
+  constexpr bool kDirectOnly = WI * WJ * WK == 16 || (sizeof(T) == 2 && NSTAGE >= 3);
   if constexpr (NSTAGE >= 2 && !kCheckedOnly) {
     if (form.clamp) {
       if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, false, true, WK>::TR) return hipErrorInvalidValue;
@@ -127,7 +127,7 @@ static hipError_t launch_op(GemmParams p, const WeightGradPlan* plan, const Spli
 // Tile shapes (all two LDS stages, software pipelined unless noted):
 //   256: 256 x 256, eight wavefronts of 128 x 64, one workgroup per compute unit
 //   128: 128 x 128, four wavefronts of 64 x 64 (up to two workgroups per compute unit) or
-//        eight of 64 x 32 when there is about one workgroup per compute unit; tuning.stages = 1
+//        eight of 64 x 32 when there is about one workgroup per compute unit (16-bit: four LDS stages); tuning.stages = 1
 //        selects a single-stage form that leans on several workgroups per compute unit
 //        instead of a pipeline (tuning aid)
 //    64:  64 x  64, for problems with few tiles: 16-bit sixteen wavefronts of 32 x 32 in four groups that
@@ -166,6 +166,9 @@ static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const 
       return hipErrorInvalidValue;
     case 128041: return launch_op<T, OP, 128, 2, 2, 1>(p, plan, split, form, stream);
     case 128082: return launch_op<T, OP, 128, 2, 4, 2>(p, plan, split, form, stream);
+    case 128084:
+      if constexpr (sizeof(T) == 2) return launch_op<T, OP, 128, 2, 4, 4>(p, plan, split, form, stream);
+      return hipErrorInvalidValue;
     case 128042: return launch_op<T, OP, 128, 2, 2, 2>(p, plan, split, form, stream);
     default: return hipErrorInvalidValue;
   }

@@ -40,8 +40,9 @@ static constexpr int kComputeUnits = 256;
 static constexpr int kTargetWorkgroups = 1024;
 
 // Contracted elements per kernel step that every slice of a cut contraction must be a multiple
-// of: 128 bytes, and 256 for the 16-bit 128 and 64 tiles, whose eight- and sixteen-wavefront forms take 256-byte steps
-// (a slice that began in the middle of such a step would start between two hashed tiles).
+// of: 128 bytes, and 256 for the 16-bit 64 tile, whose sixteen wavefronts take 256-byte steps (a slice that began
+// in the middle of such a step would start between two hashed tiles), and for the 16-bit 128 tile, whose plans the 32 x 128
+// tile with its 256-byte steps may carry out.
 static inline int slice_unit(int tile, int elem_bytes, bool weight_grad = false) {
   if (elem_bytes == 4 && tile <= 64 && !weight_grad) return 64;   // (fp32 forward / input-grad, 64 and 32 x 64 tiles: 256-byte steps as well)
   return ((tile <= 128 && elem_bytes == 2) ? 256 : 128) / elem_bytes;
@@ -707,6 +708,10 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
   // 128 tile: with about one workgroup per compute unit, eight wavefronts (two per SIMD, 64 x 32
   // each) hide latency better than four of 64 x 64; with more workgroups resident the
   // four-wavefront form does less LDS traffic per flop
+  // 16-bit, eight wavefronts, directly staged: four stages of 128 bytes of R (128 KB).  With two of 256 bytes, in as
+  // much LDS, the loads of a step were issued when the last ones had landed, so that between two barriers nothing was in
+  // flight for a while; now three steps are at any time (M = 128, K = N = 10240 in three slices, forward and input-grad:
+  // 44.7 -> 42.3 and 45.2 -> 41.0 us; M = 3001, K = 2047, N = 1531 input-grad 42.0 -> 40.4 us; 2048^3 as before, 22.5)
   // 64 tile: four wavefronts; fp32 forward / input-grad take eight (two groups that share every R
   // step: a second wavefront per SIMD keeps the MFMA pipe fed while the first waits for LDS)
   // (32-bit: every two-stage form stages directly; 16-bit too)
@@ -718,7 +723,7 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
   const bool many64 = tile == 64 && elem_bytes == 2;
   const int waves128 = f.stages == 1 ? 4 : (workgroups <= kComputeUnits * 3 / 2 ? 8 : 4);
   const int step_plain = elem_bytes == 4 ? slice_unit(tile, elem_bytes, op == kWeightGrad) : 128 / elem_bytes;
-  const int step_direct = (direct_capable && elem_bytes == 2 && ((tile == 128 && waves128 == 8) || many64)) ? 256 / elem_bytes : step_plain;
+  const int step_direct = (direct_capable && elem_bytes == 2 && many64) ? 256 / elem_bytes : step_plain;
   f.full = (I % tile == 0) && (J % tile_cols(tile) == 0) && (R % step_direct == 0) && (chunk % step_direct == 0);
   // a plain operand's rows must hold at least one 16-byte piece (a piece that straddles the end of a
   // row is handled in the kernel; a row shorter than a piece is not)
@@ -730,6 +735,7 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
             : tile == 32 ? 4
             : tile == 64 ? ((many64 && (f.full || f.clamp)) ? 16 : (elem_bytes == 4 && op != kWeightGrad) ? 8 : 4)
                          : waves128;
+  if (tile == 128 && f.waves == 8 && elem_bytes == 2 && (f.full || f.clamp)) f.stages = 4;
   if (f.waves == 16) f.stages = workgroups <= kComputeUnits ? 4 : 2;
   // 16-bit forward / input-grad on the planner's 128 tile, a batch of at most 32 rows (decoding): C tiles of 32 x 128.
   // The 128 rows of the square tile would stage the batch four times over beside every piece of W; without them three

@@ -215,3 +215,37 @@ def test_bias_gradient_behind_the_windows(oracle, shape, dtype):
     ref = oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.75)
     assert np.abs(dhw.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()   # (fp32 sums of exact products)
     assert_close(dbias.float().cpu().numpy(), dy64.sum(0), dtype, "bias gradient")
+
+
+@pytest.mark.parametrize("dtype", SIXTEEN, ids=str)
+@pytest.mark.parametrize("extents", [(256, 384), (250, 391)], ids=str)
+@pytest.mark.parametrize("steps,rest", [(1, 0), (2, 0), (3, 0), (4, 0), (5, 0), (6, 0), (9, 0), (36, 0),
+                                        (0, 17), (1, 1), (2, 31), (3, 32), (4, 63), (5, 33), (17, 8)], ids=str)
+@pytest.mark.parametrize("tile", [128])
+def test_16_bit_pipelined_tiles_at_few_steps(oracle, tile, steps, rest, extents, dtype):
+    """The loops that load several R steps of 64 elements ahead: fewer steps than are in flight, every remainder of the
+    stages, a partial last step, past the first bank of the offset table; complete and ragged tiles; all three operations,
+    dHW through LDS images and through stored tiles, bias gradient included."""
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearBackward import rz_linear_backward_input_grad_tl, weight_grad_hashed
+    from rzlinear_amd.impl.RzLinearForward import rz_linear_forward_bias_tl
+    r, (a, b), H, BK, BN = 64 * steps + rest, extents, 20000, 32, 64
+    _say(tile, r, extents, dtype)
+    R = _lib.hash_constants(*rargs(R1024))
+    bias = torch.randn((b,), generator=torch.Generator().manual_seed(4)).to(dtype)
+    with _lib.tuning(tile=tile, split=-1):
+        (x, hw, _), (x64, hw64, _) = make_inputs(a, r, b, H, dtype, seed=r)
+        y = rz_linear_forward_bias_tl(x, hw, bias.cuda(), 0.75, a, r, b, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
+        assert_close(y.float().cpu().numpy(), oracle.forward(x64, hw64, b, BK, BN, R1024, 0.75) + bias.double().numpy(), dtype, "y")
+        (_, hw, dy), (_, hw64, dy64) = make_inputs(a, b, r, H, dtype, seed=r)
+        dx = rz_linear_backward_input_grad_tl(dy, hw, 0.75, a, b, r, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
+        assert_close(dx.float().cpu().numpy(), oracle.input_grad(dy64, hw64, b, BK, BN, R1024, 0.75), dtype, "dx")
+    (x, _, dy), (x64, _, dy64) = make_inputs(r, a, b, H, dtype, seed=r)
+    ref = oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.5)
+    for how in ({"window": -1}, {"lds_image": -1, "window": -1, "fold": 2}):
+        out = torch.empty((H,), dtype=torch.float32, device="cuda")
+        with _lib.tuning(tile=tile, **how):
+            _, dbias = weight_grad_hashed(x, dy, 0.5, r, a, b, H, R, BK, BN, out=out, with_bias_grad=True)
+        # (fp32 sums of exact products: at most r of them per stored value and a few dozen values per slot)
+        assert np.abs(out.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()
+        assert_close(dbias.float().cpu().numpy(), dy64.sum(0), dtype, "bias gradient")
