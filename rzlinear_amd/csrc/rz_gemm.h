@@ -32,6 +32,8 @@
 //                  (16 pieces with the 256-byte R step: slot p ^ (x & 15))
 //   X contiguous : [TR][X], row = X/32 units of 32 elements; unit u of row r sits at u ^ (r & 3)
 //                  (two units per row: u ^ ((r >> 1) & 1); fp32: u ^ ((r >> 2) & 1))
+//                  (16-bit 256 tile: two halves [TR][128] side by side, chunks of 16 elements: chunk c of row r at
+//                  c ^ ((r & 3) << 1 | (r >> 3 & 1)), for fragments of 16 columns by 32 rows)
 // Both keep the fragment reads free of bank conflicts.  fp32 fragments of a directly staged tile
 // cover eight elements of R at a time, four MFMAs per pair of blocks: MFMA j of the four contracts
 // elements j (lanes 0-31) and 4 + j (lanes 32-63) — any pairing of the two halves is a valid sum as
@@ -60,6 +62,9 @@ template <> struct Mfma<float> {
 };
 template <> struct Mfma<bf16_t> {
   typedef u32x4_t Frag;
+  static __device__ __forceinline__ f32x4_t run16(Frag a, Frag b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  }
   static __device__ __forceinline__ f32x16_t run(Frag a, Frag b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a),
                                                    __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
@@ -67,6 +72,9 @@ template <> struct Mfma<bf16_t> {
 };
 template <> struct Mfma<f16_t> {
   typedef u32x4_t Frag;
+  static __device__ __forceinline__ f32x4_t run16(Frag a, Frag b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  }
   static __device__ __forceinline__ f32x16_t run(Frag a, Frag b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a),
                                                   __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
@@ -194,7 +202,11 @@ struct GemmKernel {
   static __device__ __forceinline__ int unit_swizzle(int row, int pitch) {
     return Tr::kBytes == 2 ? (pitch == 64 ? ((row >> 1) & 1) : (row & 3)) : ((row >> 2) & 1);
   }
+  // (kBlk16: chunks of 16 elements; the rows that half a wavefront reads together, r .. r + 3 and r + 8 .. r + 11 for one
+  //  chunk, come from eight different chunks' places, that is from all banks)
+  static __device__ __forceinline__ int chunk_swizzle(int row) { return (row & 3) << 1 | ((row >> 3) & 1); }
   static __device__ __forceinline__ int strided_at(int row, int col, int pitch) {
+    if constexpr (kBlk16) return (col >> 7) * (TR * 128) + row * 128 + (((((col & 127) >> 4) ^ chunk_swizzle(row)) << 4) | (col & 15));
     return row * pitch + ((((col >> 5) ^ unit_swizzle(row, pitch)) << 5) | (col & 31));
   }
   static __device__ __forceinline__ u32x4_t shift_down(u32x4_t v, int sh) {
@@ -212,7 +224,11 @@ struct GemmKernel {
   // pair of blocks), and a fragment holds a lane's four values of it
   static constexpr bool kDirect32 = !k16 && RZ_F32_DIRECT && (FULL || CLAMP) && NSTAGE == 2 && TJ >= 64;
   static constexpr bool kDirect = kDirect16 || kDirect32;
-  static constexpr int KS = kDirect32 ? 8 : Tr::kMfmaK;
+  // The 16-bit 256 tile multiplies blocks of 16 x 16 by 32 elements of R (v_mfma_f32_16x16x32) in a loop written for it
+  // (see `step` under kBlk16); the other kernels blocks of 32 x 32.  Under a long matrix load the board lowers its clock
+  // to keep to its power: a stream of 16x16x32 alone ran at 2063 TFLOP/s here, one of 32x32x16 at 1840.
+  static constexpr bool kBlk16 = kDirect16 && TI == 256 && TJ == 256 && WI == 2 && WJ == 4 && NSTAGE == 2;
+  static constexpr int KS = kDirect32 ? 8 : kBlk16 ? 32 : Tr::kMfmaK;
   typedef typename std::conditional<kDirect32, f32x4_t, typename Mfma<T>::Frag>::type Frag;
   static __device__ __forceinline__ f32x16_t mma(Frag a, Frag b, f32x16_t c) {
     if constexpr (kDirect32) {
@@ -225,11 +241,12 @@ struct GemmKernel {
   }
 
   template <int LAYOUT, int TX> struct Lds {
-    static constexpr int kPitch = kDirect ? (LAYOUT == kRContig ? TR : TX)
+    static constexpr int kPitch = kDirect ? (LAYOUT == kRContig ? TR : kBlk16 ? 128 : TX)
                                   : k16   ? (LAYOUT == kRContig ? TR + 8 : TX + 32)
                                           : (LAYOUT == kRContig ? TX + 1 : TX + 4);
     static constexpr int kRows = ((k16 || kDirect) && LAYOUT == kRContig) ? TX : TR;
-    static constexpr int kElems = ((kPitch * kRows + 7) / 8) * 8;
+    static constexpr int kHalves = (kBlk16 && LAYOUT == kRStrided) ? TX / 128 : 1;   // side by side: [kHalves][TR][128]
+    static constexpr int kElems = ((kPitch * kRows * kHalves + 7) / 8) * 8;
     static_assert(!kDirect32 || LAYOUT == kRContig || (TX >= 64 && TX <= 256), "a direct load instruction fills whole rows of two or more 128-byte units");
     // source tile as seen by the global loads
     static constexpr int kSrcRows = (LAYOUT == kRContig) ? TX : TR;
@@ -423,6 +440,15 @@ struct GemmKernel {
       for (int b = 0; b < MJ; b++)
 #pragma unroll
         for (int e = 0; e < 16; e++) acc[a][b][e] = 0.f;
+
+    // (kBlk16) the accumulators of the 16 x 16 blocks
+    f32x4_t blk[kBlk16 ? MI * 2 : 1][kBlk16 ? MJ * 2 : 1];
+    if constexpr (kBlk16) {
+#pragma unroll
+      for (int a = 0; a < MI * 2; a++)
+#pragma unroll
+        for (int b = 0; b < MJ * 2; b++) blk[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
 
     u32x4_t ra[LA::kPieces], rb[LB::kPieces];
     // elements of the last R step that lie beyond R (ragged contraction, direct staging)
@@ -619,40 +645,61 @@ struct GemmKernel {
     // instruction with index n = wave * kPieces + q fills LDS bytes [1024 n, 1024 n + 1024) of
     // the stage, lane i the 16 bytes at 16 i; (row, col) is the source piece that the swizzled
     // layout keeps there.
-    auto direct_src = [&](auto L, int layout, int q, int lane, int& row, int& col) {
+    // the 1024 bytes of the stage that a wavefront's q-th load fills.  (kBlk16: the first half of its pieces of A lies in
+    //  the first half of what the wavefronts multiply — rows, or columns of X — the others in the second: they
+    //  are refilled at different times)
+    auto piece_b = [&](int q) -> int { return wave * LB::kPieces + q; };
+    auto piece_a = [&](int q) -> int {
+      if constexpr (kBlk16) {
+        const int h = q / (LA::kPieces / 2), m = wave * (LA::kPieces / 2) + q % (LA::kPieces / 2);
+        return A_LAYOUT == kRContig ? (m >> 3) * 16 + h * 8 + (m & 7) : h * 16 + m;
+      }
+      return wave * LA::kPieces + q;
+    };
+    auto direct_src = [&](auto L, bool is_a, int layout, int q, int lane, int& row, int& col) {
       typedef decltype(L) LL;
-      const int n = wave * LL::kPieces + q;
+      const int n = is_a ? piece_a(q) : piece_b(q);
       if (layout == kRContig) {
         row = n * (64 / kPpr) + lane / kPpr;
         col = ((lane % kPpr) ^ row_swizzle(row)) * VEC;
       } else {
         constexpr int kSlots = LL::kPitch / VEC;        // 16-byte slots per row
-        row = n * (64 / kSlots) + lane / kSlots;
+        constexpr int kPer = kBlk16 ? TR / (64 / (kBlk16 ? kSlots : 1)) : 1;          // instructions per half (kBlk16)
+        row = (kBlk16 ? n % kPer : n) * (64 / kSlots) + lane / kSlots;
         const int slot = lane % kSlots;
         constexpr int kPpu = 32 / VEC;                  // 16-byte slots per unit of 32 elements
-        col = (((slot / kPpu) ^ unit_swizzle(row, LL::kPitch)) << 5) | ((slot % kPpu) * VEC);
+        if constexpr (kBlk16) col = (n / kPer) * 128 + ((((slot >> 1) ^ chunk_swizzle(row)) << 4) | ((slot & 1) * VEC));
+        else col = (((slot / kPpu) ^ unit_swizzle(row, LL::kPitch)) << 5) | ((slot % kPpu) * VEC);
       }
     };
-    auto direct_load = [&](const T* src, const T* stage, int q, int pieces) {
+    // LDS addresses as 32-bit numbers, worked out once and kept in scalar registers (opaque: otherwise the compiler
+    // converts the generic pointers again for every load, a dozen scalar instructions each)
+    typedef const T __attribute__((address_space(3)))* lds_ptr;
+    uint32_t lds_a = 0, lds_b = 0;
+    if constexpr (kDirect) {
+      lds_a = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)sm.a[0]);
+      lds_b = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)sm.b[0]);
+      asm volatile("" : "+s"(lds_a), "+s"(lds_b));
+    }
+    auto stage_a = [&](int st) -> uint32_t { return lds_a + (uint32_t)st * (uint32_t)(LA::kElems * sizeof(T)); };
+    auto stage_b = [&](int st) -> uint32_t { return lds_b + (uint32_t)st * (uint32_t)(LB::kElems * sizeof(T)); };
+    auto direct_load = [&](const T* src, uint32_t stage, int n) {
       // the LDS address goes through M0 and must be the same for the whole wavefront
-      typedef const T __attribute__((address_space(3)))* lds_ptr;
-      const uint32_t dst = __builtin_amdgcn_readfirstlane(
-          (uint32_t)(uintptr_t)(lds_ptr)(stage) + (uint32_t)((wave * pieces + q) * 1024));
+      const uint32_t dst = __builtin_amdgcn_readfirstlane(stage + (uint32_t)(n * 1024));
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst), "v"(src)
                    : "memory", "m0");
     };
     // the same load with the address split into a uniform 64-bit base (scalar registers) and a
     // per-lane 32-bit byte offset: the offsets are computed once, the base moves with the step
-    auto direct_load_so = [&](const void* base, uint32_t voff, const T* stage, int q, int pieces) {
-      typedef const T __attribute__((address_space(3)))* lds_ptr;
-      const uint32_t dst = __builtin_amdgcn_readfirstlane(
-          (uint32_t)(uintptr_t)(lds_ptr)(stage) + (uint32_t)((wave * pieces + q) * 1024));
+    auto direct_load_so = [&](const void* base, uint32_t voff, uint32_t stage, int n) {
+      const uint32_t dst = __builtin_amdgcn_readfirstlane(stage + (uint32_t)(n * 1024));
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dst), "v"(voff), "s"(base)
                    : "memory", "m0");
     };
     // the plain tiles of R step `step` -> LDS stage `st`, addresses computed in full (used for
     // the last, partial step of a ragged contraction, whose pieces beyond R are redirected)
-    auto direct_issue_plain_slow = [&](int step, int st) {
+    // (`part`: 0 the first half of A with a plain B, 1 the second half of A, see piece_a; 2 everything)
+    auto direct_issue_plain_slow = [&](int step, int st, int part) {
       const int r0 = r_begin + step * TR;
       // (opaque: worked out ahead of the loop, as the compiler would like to, the addresses of this one step take
       //  registers that every step needs)
@@ -660,8 +707,9 @@ struct GemmKernel {
       asm volatile("" : "+v"(l));
 #pragma unroll
       for (int q = 0; q < LA::kPieces; q++) {
+        if (part < 2 && q / (LA::kPieces / 2) != part) continue;
         int row, col;
-        direct_src(LA{}, A_LAYOUT, q, l, row, col);
+        direct_src(LA{}, true, A_LAYOUT, q, l, row, col);
         // (CLAMP: rows / 16-byte columns beyond I come from the last one inside)
         const int gi = (A_LAYOUT == kRContig) ? i0 + row : i0 + col;
         const int ci = !CLAMP ? gi : (A_LAYOUT == kRContig) ? (gi < p.I ? gi : p.I - 1) : (gi < p.I ? gi : p.I - VEC);
@@ -681,19 +729,20 @@ struct GemmKernel {
         }
         const T* src = (A_LAYOUT == kRContig) ? gA + (int64_t)ci * p.lda + cc
                                               : gA + (int64_t)cr * p.lda + ca;
-        direct_load(src, sm.a[st], q, LA::kPieces);
+        direct_load(src, stage_a(st), piece_a(q));
       }
       if constexpr (OP == kWeightGrad) {
 #pragma unroll
         for (int q = 0; q < LB::kPieces; q++) {
+          if (part == 1) continue;
           int row, col;
-          direct_src(LB{}, B_LAYOUT, q, l, row, col);
+          direct_src(LB{}, false, B_LAYOUT, q, l, row, col);
           const int gj = j0 + col;
           int cj = (!CLAMP || gj < p.J) ? gj : p.J - VEC;
           const int gr = r0 + row;
           const int cr = (CLAMP && gr >= p.R) ? p.R - 1 : gr;
           if (CLAMP && rag_j && cr == p.R - 1 && gj < p.J && gj + VEC > p.J) cj = p.J - VEC;
-          direct_load(gB + (int64_t)cr * p.ldb + cj, sm.b[st], q, LB::kPieces);
+          direct_load(gB + (int64_t)cr * p.ldb + cj, stage_b(st), piece_b(q));
         }
       }
     };
@@ -712,7 +761,7 @@ struct GemmKernel {
 #pragma unroll
       for (int q = 0; q < LA::kPieces; q++) {
         int row, col;
-        direct_src(LA{}, A_LAYOUT, q, lane, row, col);
+        direct_src(LA{}, true, A_LAYOUT, q, lane, row, col);
         if constexpr (A_LAYOUT == kRContig) {
           const int gi = i0 + row;
           const int ci = (!CLAMP || gi < p.I) ? row : p.I - 1 - i0;
@@ -728,7 +777,7 @@ struct GemmKernel {
 #pragma unroll
       for (int q = 0; q < LB::kPieces; q++) {
         int row, col;
-        direct_src(LB{}, B_LAYOUT, q, lane, row, col);
+        direct_src(LB{}, false, B_LAYOUT, q, lane, row, col);
         if constexpr (OP == kWeightGrad) {
           const int gj = j0 + col;
           const int cj = (!CLAMP || gj < p.J) ? col : (p.J - VEC - j0 > 0 ? p.J - VEC - j0 : 0);
@@ -757,30 +806,38 @@ struct GemmKernel {
       return (const T*)(uintptr_t)(((uint64_t)hi << 32) | lo);
     };
     // all tiles of R step `step` -> LDS stage `st`
+    // the offset-table entries of a step's hashed pieces; 16-bit: read a sub-step before the loads that need them (fp32, whose
+    // sub-steps are long, reads them with the loads: M = 8192, K = N = 2048 forward 476 us, early 482)
+    constexpr bool kEarlyLookup = k16;
+    uint32_t looked[kDirect && OP != kWeightGrad ? LB::kPieces : 1];
+    auto direct_lookup = [&](int step) {
+      if constexpr (kDirect && OP != kWeightGrad) {
+        const int* tab = sm.off + (step & (kOffSlots - 1)) * kOffWindow;
+#pragma unroll
+        for (int q = 0; q < LB::kPieces; q++) looked[q] = (uint32_t)tab[b_tab[q]];
+      }
+    };
     auto direct_issue = [&](int step, int st) {
       const int r0 = r_begin + step * TR;
       if (CLAMP && slow_last && step == steps - 1) {   // (uniform) the partial last step, or the one with the operands' last row
-        direct_issue_plain_slow(step, st);
+        direct_issue_plain_slow(step, st, 2);
       } else {
         // first element of the A tile of this step (uniform)
         const T* a_base = uniform_ptr((A_LAYOUT == kRContig) ? gA + (int64_t)i0 * p.lda + r0 : gA + (int64_t)r0 * p.lda + i0);
 #pragma unroll
-        for (int q = 0; q < LA::kPieces; q++) direct_load_so(a_base, a_voff[q], sm.a[st], q, LA::kPieces);
+        for (int q = 0; q < LA::kPieces; q++) direct_load_so(a_base, a_voff[q], stage_a(st), piece_a(q));
         if constexpr (OP == kWeightGrad) {
           const T* b_base = uniform_ptr(gB + (int64_t)r0 * p.ldb + j0);
 #pragma unroll
-          for (int q = 0; q < LB::kPieces; q++) direct_load_so(b_base, b_voff[q], sm.b[st], q, LB::kPieces);
+          for (int q = 0; q < LB::kPieces; q++) direct_load_so(b_base, b_voff[q], stage_b(st), piece_b(q));
         }
       }
       if constexpr (OP != kWeightGrad) {
-        const int* tab = sm.off + (step & (kOffSlots - 1)) * kOffWindow;
         const T* hw_base = uniform_ptr(gHW);
-        uint32_t off[LB::kPieces];
-#pragma unroll
-        for (int q = 0; q < LB::kPieces; q++) off[q] = (uint32_t)tab[b_tab[q]];   // all lookups first, then the loads
+        if constexpr (!kEarlyLookup) direct_lookup(step);
 #pragma unroll
         for (int q = 0; q < LB::kPieces; q++)
-          direct_load_so(hw_base, off[q] * (uint32_t)sizeof(T) + b_voff[q], sm.b[st], q, LB::kPieces);
+          direct_load_so(hw_base, looked[q] * (uint32_t)sizeof(T) + b_voff[q], stage_b(st), piece_b(q));
       }
     };
     // CLAMP, last R step: once every wavefront's loads of that step have landed (the caller has just
@@ -802,11 +859,12 @@ struct GemmKernel {
             typedef decltype(L) LL;
             if (layout == kRStrided) {
               const int first = TR - tail;
-              for (int i = t0; i < tail * (LL::kPitch / VEC); i += kThreads)
-                *reinterpret_cast<u32x4_t*>(stage + first * LL::kPitch + i * VEC) = z;
+              for (int h = 0; h < LL::kHalves; h++)
+                for (int i = t0; i < tail * (LL::kPitch / VEC); i += kThreads)
+                  *reinterpret_cast<u32x4_t*>(stage + (h * TR + first) * LL::kPitch + i * VEC) = z;
               // the operand's last row (the last one before `first`), the piece that straddles its end
               const int c = ext - rag_x - x0;
-              if (plain && rag_x && r_end == p.R && c >= 0 && c < LL::kPitch && t0 == 0) {
+              if (plain && rag_x && r_end == p.R && c >= 0 && c < LL::kPitch * LL::kHalves && t0 == 0) {
                 const int row = first - 1;
                 u32x4_t v;
                 __builtin_memcpy(&v, g + (int64_t)(p.R - 1) * ld + (ext - VEC), 16);
@@ -890,7 +948,205 @@ struct GemmKernel {
       if constexpr (OP != kWeightGrad) __syncthreads();
       if constexpr (!kDirect) fetch(0);
     }
-    if constexpr (NSTAGE == 1) {
+    if constexpr (kBlk16) {
+      // The 16-bit 256 tile: 256 x 256 by steps of 64 in two stages of 64 KB, eight wavefronts of 128 x 64.  What bounds this
+      // loop is what is issued beside the matrix instructions (two wavefronts of a SIMD have 64 of them each per step, 16
+      // clocks apiece, and the barriers and waits cost next to nothing), and the power that all of it draws.  So:
+      //  - a step is eight phases of eight MFMAs: (two blocks of A's rows) x (all of B's) x (one sub-step of 32).  Phase
+      //    2 i + k multiplies A's pair i by sub-step k; B's fragments stay in registers for the whole step, and every phase
+      //    reads only the next one's two fragments of A, so that nothing is spilled (a whole sub-step read ahead is);
+      //  - the order is held by sched_barrier: left alone the compiler moves the reads down to where they are used;
+      //  - addresses are 32-bit LDS addresses and running pointers, no arithmetic is left to do per load or fragment;
+      //  - one load per phase, not eight behind a barrier (that kept all wavefronts from multiplying while they waited
+      //    to issue them): A's first half of rows and B are free for the step after next from phase 3 on, A's second half
+      //    from phase 7 on, and each part is waited for only where it is first read.
+      // 4096^3 bf16, forward / input-grad / weight-grad: 112.8 / 112.5 / 123.1 -> 100.4 / 98.7 / 111.5 us; M = 8192, K = 4096, N = 16384:
+      // 877 / 877 / 904 -> 774 / 743 / 811 us (1.42 / 1.48 / 1.36 PFLOP/s).  Same bits as the loop with blocks of 32 x 32.
+      // Not faster: four wavefronts of 128 x 128 (126 us weight-grad), wave priorities, a deeper pipeline alone.
+      constexpr int FI = MI * 2, FJ = MJ * 2, NS = TR / 32;   // blocks of the wavefront, sub-steps
+      static_assert(FI == 8 && FJ == 4 && NS == 2 && LA::kPieces == 4, "the phases below are written for this shape");
+      constexpr int kFirst = LA::kPieces / 2 + LB::kPieces, kSecond = LA::kPieces / 2;   // loads of the two parts of a step
+      // LDS addresses are 32-bit numbers, worked out once: one register per distinct swizzle of a fragment, one scalar
+      // register per operand for the loads.  Everything known when the kernel is compiled is in an instruction's offset.
+      // (opaque, or the compiler works them out again at every use)
+      auto rel = [&](bool is_a, int f) -> int {   // first row / column of block f, from the wavefront's first
+        if constexpr (OP == kWeightGrad) return (f >> 1) * (is_a ? WI : WJ) * 32 + (f & 1) * 16;
+        else return f * 16;
+      };
+      constexpr int kNA = A_LAYOUT == kRContig ? NS : FI / 2, kNB = B_LAYOUT == kRContig ? NS : (OP == kWeightGrad ? FJ / 2 : FJ);
+      uint32_t base_a[kNA], base_b[kNB];
+      auto bases = [&](int layout, uint32_t* base, int n, bool is_a, int x0, uint32_t at) {
+#pragma unroll
+        for (int i = 0; i < n; i++) {
+          if (layout == kRContig) {
+            const int row = x0 + (lane & 15), piece = i * 4 + (lane >> 4);
+            base[i] = at + (uint32_t)(row * TR + ((piece ^ row_swizzle(row)) << 3)) * 2u;
+          } else {
+            const int g = lane >> 4, jl = lane & 15, row = 8 * g + (jl >> 2);
+            base[i] = at + (uint32_t)strided_at(row, (x0 ^ rel(is_a, i)) + 4 * (jl & 3), 128) * 2u;
+          }
+          asm volatile("" : "+v"(base[i]));
+        }
+      };
+      bases(A_LAYOUT, base_a, kNA, true, OP == kWeightGrad ? wave_i * 32 : wave_i * WTI, lds_a);
+      bases(B_LAYOUT, base_b, kNB, false, OP == kWeightGrad ? wave_j * 32 : wave_j * WTJ, lds_b);
+      auto read_frag = [&](bool is_a, int st, int ks, int f) -> u32x4_t {
+        const int layout = is_a ? A_LAYOUT : B_LAYOUT, n = is_a ? kNA : kNB;
+        const int which = layout == kRContig ? ks : f % n;
+        const uint32_t base = is_a ? base_a[which] : base_b[which];
+        const int at = (st * (is_a ? LA::kElems : LB::kElems) + (layout == kRContig ? f * 16 * TR : ks * 32 * 128 + (rel(is_a, f) >> 7) * TR * 128)) * 2;
+        if (layout == kRContig) {
+          typedef const u32x4_t __attribute__((address_space(3)))* ptr;
+          return *(ptr)(uintptr_t)(base + (uint32_t)at);
+        }
+        typedef s16x4_t __attribute__((address_space(3)))* ptr;
+        const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(uintptr_t)(base + (uint32_t)at));
+        const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(uintptr_t)(base + (uint32_t)(at + 4 * 128 * 2)));
+        const u32x2_t l2 = __builtin_bit_cast(u32x2_t, lo), h2 = __builtin_bit_cast(u32x2_t, hi);
+        return u32x4_t{l2[0], l2[1], h2[0], h2[1]};
+      };
+      uint32_t dma_a = __builtin_amdgcn_readfirstlane(lds_a + (uint32_t)piece_a(0) * 1024u);
+      uint32_t dma_b = __builtin_amdgcn_readfirstlane(lds_b + (uint32_t)piece_b(0) * 1024u);
+      asm volatile("" : "+s"(dma_a), "+s"(dma_b));
+      // first element of A's (and a plain B's) tile of the R step whose loads are being issued
+      const T* a_ptr = uniform_ptr(A_LAYOUT == kRContig ? gA + (int64_t)i0 * p.lda + r_begin : gA + (int64_t)r_begin * p.lda + i0);
+      const T* b_ptr = uniform_ptr(OP == kWeightGrad ? gB + (int64_t)r_begin * p.ldb + j0 : gHW);
+      const int64_t a_step = A_LAYOUT == kRContig ? TR : TR * p.lda, b_step = OP == kWeightGrad ? TR * p.ldb : 0;
+      auto load_lds = [&](const T* base, uint32_t voff, uint32_t dma, int at) {
+        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dma), "v"(voff), "s"(base), "n"(at) : "memory", "scc");
+      };
+      // the tile offsets of step `step`'s pieces of W, added to what is fixed of their addresses
+      uint32_t tab_at[OP != kWeightGrad ? LB::kPieces : 1], hw_off[OP != kWeightGrad ? LB::kPieces : 1];
+      if constexpr (OP != kWeightGrad) {
+        typedef const int __attribute__((address_space(3)))* off_ptr;
+#pragma unroll
+        for (int q = 0; q < LB::kPieces; q++) {
+          tab_at[q] = (uint32_t)(uintptr_t)(off_ptr)sm.off + (uint32_t)b_tab[q] * 4u;
+          asm volatile("" : "+v"(tab_at[q]));
+        }
+      }
+      auto lookup = [&](int step) {
+        if constexpr (OP != kWeightGrad) {
+          typedef const uint32_t __attribute__((address_space(3)))* off_ptr;
+          const uint32_t slot = (uint32_t)((step & (kOffSlots - 1)) * kOffWindow * 4);
+#pragma unroll
+          for (int q = 0; q < LB::kPieces; q++) hw_off[q] = *(off_ptr)(uintptr_t)(tab_at[q] + slot);
+        }
+      };
+      // The j-th of a wavefront's eight loads for R step `step`: 0, 1 the first half of A, 2 .. 5 B, 6, 7 the second half of A.
+      auto issue = [&](int step, int st, int j, auto last) {
+        const int sa = st * (int)(LA::kElems * sizeof(T)), sb = st * (int)(LB::kElems * sizeof(T));
+        constexpr int kHalfA = (A_LAYOUT == kRContig ? 8 : 16) * 1024;   // from one half of A to the other
+        if (decltype(last)::value && CLAMP && slow_last && step == steps - 1) {   // (uniform)
+          if (j == 0) direct_issue_plain_slow(step, st, 0);
+          if (j == 6) direct_issue_plain_slow(step, st, 1);
+          if (OP == kWeightGrad) return;
+        } else if (j < 2 || j >= 6) {
+          load_lds(a_ptr, a_voff[j < 2 ? j : j - 4], dma_a, sa + (j & 1) * 1024 + (j >= 6 ? kHalfA : 0));
+        } else if constexpr (OP == kWeightGrad) {
+          load_lds(b_ptr, b_voff[j - 2], dma_b, sb + (j - 2) * 1024);
+        }
+        if constexpr (OP != kWeightGrad) {
+          if (j >= 2 && j < 6) load_lds(b_ptr, hw_off[j - 2] * (uint32_t)sizeof(T) + b_voff[j - 2], dma_b, sb + (j - 2) * 1024);
+        }
+      };
+      u32x4_t fa[2][2], fb[2][FJ];   // A: two blocks of a phase, two phases; B: the sub-steps of the R step
+      auto step = [&](int s, auto stage, auto inner) {
+        // (inner: a step whose loads, and its successor's, are issued as a whole: no conditions)
+        constexpr bool kInner = decltype(inner)::value;
+        constexpr int st = decltype(stage)::value, next = st ^ 1;
+        const bool has_next = kInner || s + 1 < steps, fetching = kInner || s + 2 < steps;   // (uniform)
+        const std::integral_constant<bool, !kInner> last{};
+#pragma unroll
+        for (int ph = 0; ph < 8; ph++) {
+          const int ap = ph >> 1, ks = ph & 1;
+          if (ph == 3) {
+            // A's second half of this step has landed; its first half and B have been read by every wavefront
+            if (fetching) {
+#pragma unroll
+              for (int q = 0; q < (OP != kWeightGrad ? LB::kPieces : 0); q++) asm volatile("" : "+v"(hw_off[q]));
+            }
+            if (has_next) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFirst + kSecond) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            a_ptr += a_step;
+            b_ptr += b_step;
+          } else if (ph == 7) {
+            if (has_next) {
+              if (fetching) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFirst + kSecond - 1) : "memory");
+              else if (CLAMP && slow_last) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+              else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kSecond) : "memory");
+              if (!fetching) clear_tail(next);
+            }
+          }
+          if (ph == 0) {
+#pragma unroll
+            for (int f = 0; f < FJ; f++) fb[1][f] = read_frag(false, st, 1, f);
+          }
+          if (ph < 7) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) fa[(ph + 1) & 1][i] = read_frag(true, st, (ph + 1) & 1, ((ph + 1) >> 1) * 2 + i);
+            if (ph == 1 && fetching) lookup(s + 2);
+          } else if (has_next) {
+#pragma unroll
+            for (int f = 0; f < FJ; f++) fb[0][f] = read_frag(false, next, 0, f);
+#pragma unroll
+            for (int i = 0; i < 2; i++) fa[0][i] = read_frag(true, next, 0, i);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < 2; i++) {
+#pragma unroll
+            for (int b = 0; b < FJ; b++) blk[ap * 2 + i][b] = Mfma<T>::run16(fa[ph & 1][i], fb[ks][b], blk[ap * 2 + i][b]);
+            if (i == 0) {
+              __builtin_amdgcn_sched_barrier(0);
+              if (ph < 2 && has_next) issue(s + 1, next, 6 + ph, last);
+              if (ph == 3 && fetching) issue(s + 2, st, 0, last);
+              if (ph >= 3 && fetching) issue(s + 2, st, ph - 2, last);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (COLSUM) {
+            if (ph == 0) colsum_from_stage(st);
+          }
+        }
+      };
+      if (steps > 0) {
+        const std::integral_constant<bool, true> last{};
+        lookup(0);
+#pragma unroll
+        for (int j = 0; j < 8; j++) issue(0, 0, j, last);
+        if (steps > 1) {
+          a_ptr += a_step;
+          b_ptr += b_step;
+          lookup(1);
+#pragma unroll
+          for (int j = 0; j < 6; j++) issue(1, 1, j, last);
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kFirst + kSecond) : "memory");
+        } else {
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        __syncthreads();
+        if (steps == 1) clear_tail(0);
+#pragma unroll
+        for (int f = 0; f < FJ; f++) fb[0][f] = read_frag(false, 0, 0, f);
+#pragma unroll
+        for (int i = 0; i < 2; i++) fa[0][i] = read_frag(true, 0, 0, i);
+        // (the offset tables are refilled for the steps from s + kOffBank on, every kOffBank steps)
+        int s = 0;
+        const int whole = steps - ((CLAMP && slow_last) ? 1 : 0);   // (the last step's loads may need care)
+        for (; s + 3 < whole; s += 2) {
+          hash_ahead(s);
+          step(s, std::integral_constant<int, 0>{}, std::integral_constant<bool, true>{});
+          step(s + 1, std::integral_constant<int, 1>{}, std::integral_constant<bool, true>{});
+        }
+        for (; s < steps; s += 2) {
+          hash_ahead(s);
+          step(s, std::integral_constant<int, 0>{}, std::integral_constant<bool, false>{});
+          if (s + 1 < steps) step(s + 1, std::integral_constant<int, 1>{}, std::integral_constant<bool, false>{});
+        }
+      }
+    } else if constexpr (NSTAGE == 1) {
       // one LDS stage: write it, read it, two barriers per step; relies on several
       // workgroups per compute unit to overlap the phases
       for (int s = 0; s < steps; s++) {
@@ -958,6 +1214,9 @@ struct GemmKernel {
         for (int ks = 0; ks < NKS; ks++) {
           if (ks + 1 < NKS) {
             frags(st, ks + 1, (ks + 1) & 1);
+            if constexpr (decltype(do_fetch)::value && kDirect && kEarlyLookup) {
+              if (ks + 2 == NKS) direct_lookup(s + NSTAGE);
+            }
             if constexpr (kPinFrags) __builtin_amdgcn_sched_barrier(0);
           } else {
             if constexpr (kDirect) {
@@ -1007,7 +1266,10 @@ struct GemmKernel {
         if constexpr (kDirect) {
 #pragma unroll
           for (int i = 0; i < NSTAGE; i++)
-            if (i < steps) direct_issue(i, i);
+            if (i < steps) {
+              if constexpr (kEarlyLookup) direct_lookup(i);
+              direct_issue(i, i);
+            }
           // loads complete in order: all but the later steps' have landed
           if (steps >= NSTAGE) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NSTAGE - 1) * kLoads) : "memory");
           else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1024,6 +1286,26 @@ struct GemmKernel {
         if (kThreads == 512 && wave >= 4) loop(std::true_type{});
         else loop(std::false_type{});
       }
+    }
+
+    // (kBlk16) to the layout of 32 x 32 blocks that the epilogue knows: element e of a 16 x 16 block is row 4 (lane / 16) + e,
+    // column lane % 16; of two blocks side by side, the rows of 16 lanes change places so that 32 lanes hold one row
+    if constexpr (kBlk16) {
+#pragma unroll
+      for (int a = 0; a < MI * 2; a++)
+#pragma unroll
+        for (int b = 0; b < MJ; b++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            // (by value: a bit cast of a vector's element itself reads element 0)
+            const float lo = blk[a][2 * b][e], hi = blk[a][2 * b + 1][e];
+            const u32x2_t x = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi), false, false);
+            const uint32_t x0 = x[0], x1 = x[1];
+            const u32x2_t y = __builtin_amdgcn_permlane32_swap(x0, x1, false, false);
+            const uint32_t y0 = y[0], y1 = y[1];
+            acc[a >> 1][b][(a & 1) * 8 + e] = __builtin_bit_cast(float, y0);
+            acc[a >> 1][b][(a & 1) * 8 + 4 + e] = __builtin_bit_cast(float, y1);
+          }
     }
 
     // Add up the accumulators of the groups of wavefronts that shared the R steps: every group parks its own in
