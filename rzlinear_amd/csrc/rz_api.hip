@@ -1017,7 +1017,8 @@ RZ_API int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int
   const int chunk = cut ? sp.r_chunk : R;
   const KernelForm f = kernel_form(op, I, J, R, chunk, sp.tile, tile_count(I, J, sp.tile) * sp.splits, eb, t);
   out[0] = sp.tile; out[1] = sp.splits; out[2] = chunk; out[3] = f.step; out[4] = cut ? 1 : 0;
-  out[5] = (int32_t)(tile_count(I, J, sp.tile) * sp.splits);
+  const long long tiles = f.rows == sp.tile ? tile_count(I, J, sp.tile) : (long long)((I + f.rows - 1) / f.rows) * ((J + f.cols - 1) / f.cols);
+  out[5] = (int32_t)(tiles * sp.splits);
   out[6] = (cut && t.finish != -1 && sp.splits <= finish_slices(sp.tile, I, J, R, eb, t) && tile_count(I, J, sp.tile) <= (long long)kFinishPerStream) ? 1 : 0;
   return RZ_OK;
 }

@@ -224,10 +224,11 @@ struct GemmKernel {
   // pair of blocks), and a fragment holds a lane's four values of it
   static constexpr bool kDirect32 = !k16 && RZ_F32_DIRECT && (FULL || CLAMP) && NSTAGE == 2 && TJ >= 64;
   static constexpr bool kDirect = kDirect16 || kDirect32;
-  // The 16-bit 256 tile multiplies blocks of 16 x 16 by 32 elements of R (v_mfma_f32_16x16x32) in a loop written for it
+  // The 16-bit 256 and 256 x 128 tiles multiply blocks of 16 x 16 by 32 elements of R (v_mfma_f32_16x16x32) in a loop written for it
   // (see `step` under kBlk16); the other kernels blocks of 32 x 32.  Under a long matrix load the board lowers its clock
   // to keep to its power: a stream of 16x16x32 alone ran at 2063 TFLOP/s here, one of 32x32x16 at 1840.
-  static constexpr bool kBlk16 = kDirect16 && TI == 256 && TJ == 256 && WI == 2 && WJ == 4 && NSTAGE == 2;
+  static constexpr bool kPair = k16 && NSTAGE == 3 && TI == 256 && TJ == 128 && WI == 4 && WJ == 2;   // two 128 tiles
+  static constexpr bool kBlk16 = kDirect16 && (kPair || (TI == 256 && TJ == 256 && WI == 2 && WJ == 4 && NSTAGE == 2));
   static constexpr int KS = kDirect32 ? 8 : kBlk16 ? 32 : Tr::kMfmaK;
   typedef typename std::conditional<kDirect32, f32x4_t, typename Mfma<T>::Frag>::type Frag;
   static __device__ __forceinline__ f32x16_t mma(Frag a, Frag b, f32x16_t c) {
@@ -650,7 +651,7 @@ struct GemmKernel {
     //  are refilled at different times)
     auto piece_b = [&](int q) -> int { return wave * LB::kPieces + q; };
     auto piece_a = [&](int q) -> int {
-      if constexpr (kBlk16) {
+      if constexpr (kBlk16 && !kPair) {
         const int h = q / (LA::kPieces / 2), m = wave * (LA::kPieces / 2) + q % (LA::kPieces / 2);
         return A_LAYOUT == kRContig ? (m >> 3) * 16 + h * 8 + (m & 7) : h * 16 + m;
       }
@@ -964,8 +965,9 @@ struct GemmKernel {
       // 877 / 877 / 904 -> 774 / 743 / 811 us (1.42 / 1.48 / 1.36 PFLOP/s).  Same bits as the loop with blocks of 32 x 32.
       // Not faster: four wavefronts of 128 x 128 (126 us weight-grad), wave priorities, a deeper pipeline alone.
       constexpr int FI = MI * 2, FJ = MJ * 2, NS = TR / 32;   // blocks of the wavefront, sub-steps
-      static_assert(FI == 8 && FJ == 4 && NS == 2 && LA::kPieces == 4, "the phases below are written for this shape");
-      constexpr int kFirst = LA::kPieces / 2 + LB::kPieces, kSecond = LA::kPieces / 2;   // loads of the two parts of a step
+      constexpr int PH = FI;   // phases of a step
+      static_assert(FI == (kPair ? 4 : 8) && FJ == 4 && NS == 2, "the phases below are written for these shapes");
+      constexpr int kLoads = LA::kPieces + LB::kPieces;   // of a wavefront per step
       // LDS addresses are 32-bit numbers, worked out once: one register per distinct swizzle of a fragment, one scalar
       // register per operand for the loads.  Everything known when the kernel is compiled is in an instruction's offset.
       // (opaque, or the compiler works them out again at every use)
@@ -1033,96 +1035,142 @@ struct GemmKernel {
           for (int q = 0; q < LB::kPieces; q++) hw_off[q] = *(off_ptr)(uintptr_t)(tab_at[q] + slot);
         }
       };
-      // The j-th of a wavefront's eight loads for R step `step`: 0, 1 the first half of A, 2 .. 5 B, 6, 7 the second half of A.
+      // The j-th of a wavefront's loads for R step `step`.  Two stages: 0, 1 the first half of A, 2 .. 5 B, 6, 7 the second
+      // half of A; three: B, then A.
       auto issue = [&](int step, int st, int j, auto last) {
         const int sa = st * (int)(LA::kElems * sizeof(T)), sb = st * (int)(LB::kElems * sizeof(T));
         constexpr int kHalfA = (A_LAYOUT == kRContig ? 8 : 16) * 1024;   // from one half of A to the other
-        if (decltype(last)::value && CLAMP && slow_last && step == steps - 1) {   // (uniform)
-          if (j == 0) direct_issue_plain_slow(step, st, 0);
-          if (j == 6) direct_issue_plain_slow(step, st, 1);
-          if (OP == kWeightGrad) return;
-        } else if (j < 2 || j >= 6) {
-          load_lds(a_ptr, a_voff[j < 2 ? j : j - 4], dma_a, sa + (j & 1) * 1024 + (j >= 6 ? kHalfA : 0));
-        } else if constexpr (OP == kWeightGrad) {
-          load_lds(b_ptr, b_voff[j - 2], dma_b, sb + (j - 2) * 1024);
-        }
-        if constexpr (OP != kWeightGrad) {
-          if (j >= 2 && j < 6) load_lds(b_ptr, hw_off[j - 2] * (uint32_t)sizeof(T) + b_voff[j - 2], dma_b, sb + (j - 2) * 1024);
+        constexpr int kFirstB = kPair ? 0 : 2;
+        const bool is_b = j >= kFirstB && j < kFirstB + LB::kPieces;
+        const int q = is_b ? j - kFirstB : kPair ? j - LB::kPieces : j < 2 ? j : j - 4;
+        if (is_b && OP != kWeightGrad) {
+          load_lds(b_ptr, hw_off[q] * (uint32_t)sizeof(T) + b_voff[q], dma_b, sb + q * 1024);
+        } else if (decltype(last)::value && CLAMP && slow_last && step == steps - 1) {   // (uniform)
+          if (kPair ? !is_b && q == 0 : j == 0) direct_issue_plain_slow(step, st, kPair ? 2 : 0);
+          if (!kPair && j == 6) direct_issue_plain_slow(step, st, 1);
+        } else if (is_b) {
+          load_lds(b_ptr, b_voff[q], dma_b, sb + q * 1024);
+        } else {
+          load_lds(a_ptr, a_voff[q], dma_a, sa + (kPair ? q * 1024 : (j & 1) * 1024 + (j >= 6 ? kHalfA : 0)));
         }
       };
       u32x4_t fa[2][2], fb[2][FJ];   // A: two blocks of a phase, two phases; B: the sub-steps of the R step
+      // the fragments that phase ph reads ahead for the next one (and the rest of B's in phase 0)
+      auto read_ahead = [&](int st, int next, int ph, bool has_next) {
+        if (ph == 0) {
+#pragma unroll
+          for (int f = 0; f < FJ; f++) fb[1][f] = read_frag(false, st, 1, f);
+        }
+        if (ph + 1 < PH) {
+#pragma unroll
+          for (int i = 0; i < 2; i++) fa[(ph + 1) & 1][i] = read_frag(true, st, (ph + 1) & 1, ((ph + 1) >> 1) * 2 + i);
+        } else if (has_next) {
+#pragma unroll
+          for (int f = 0; f < FJ; f++) fb[0][f] = read_frag(false, next, 0, f);
+#pragma unroll
+          for (int i = 0; i < 2; i++) fa[0][i] = read_frag(true, next, 0, i);
+        }
+      };
+      // phase ph's matrix instructions, `between` in their middle
+      auto multiply = [&](int ph, auto&& between) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+#pragma unroll
+          for (int b = 0; b < FJ; b++) blk[(ph >> 1) * 2 + i][b] = Mfma<T>::run16(fa[ph & 1][i], fb[ph & 1][b], blk[(ph >> 1) * 2 + i][b]);
+          if (i == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            between();
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto keep_lookups = [&]() {
+#pragma unroll
+        for (int q = 0; q < (OP != kWeightGrad ? LB::kPieces : 0); q++) asm volatile("" : "+v"(hw_off[q]));
+      };
+      auto advance = [&]() {
+        a_ptr += a_step;
+        b_ptr += b_step;
+      };
       auto step = [&](int s, auto stage, auto inner) {
         // (inner: a step whose loads, and its successor's, are issued as a whole: no conditions)
         constexpr bool kInner = decltype(inner)::value;
-        constexpr int st = decltype(stage)::value, next = st ^ 1;
+        constexpr int st = decltype(stage)::value, next = (st + 1) % NSTAGE;
         const bool has_next = kInner || s + 1 < steps, fetching = kInner || s + 2 < steps;   // (uniform)
         const std::integral_constant<bool, !kInner> last{};
+        if constexpr (kPair) {
+          // three stages: the loads of step s + 2 go to the stage of step s - 1
+          constexpr int kInPhase[5] = {0, 2, 4, 5, 6}, kBehind = kInPhase[3];   // loads issued before phase ph; before the wait
+          static_assert(kLoads == 6, "loads per phase");
 #pragma unroll
-        for (int ph = 0; ph < 8; ph++) {
-          const int ap = ph >> 1, ks = ph & 1;
-          if (ph == 3) {
-            // A's second half of this step has landed; its first half and B have been read by every wavefront
-            if (fetching) {
-#pragma unroll
-              for (int q = 0; q < (OP != kWeightGrad ? LB::kPieces : 0); q++) asm volatile("" : "+v"(hw_off[q]));
+          for (int ph = 0; ph < PH; ph++) {
+            if (ph == PH - 1 && has_next) {
+              if (fetching) {
+                keep_lookups();
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kBehind) : "memory");
+              } else {
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                clear_tail(next);
+              }
             }
-            if (has_next) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFirst + kSecond) : "memory");
-            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            a_ptr += a_step;
-            b_ptr += b_step;
-          } else if (ph == 7) {
-            if (has_next) {
+            read_ahead(st, next, ph, has_next);
+            if (ph == 2 && (kInner || s + 3 < steps)) lookup(s + 3);
+            multiply(ph, [&]() {
+              if (fetching) {
+#pragma unroll
+                for (int j = kInPhase[ph]; j < kInPhase[ph + 1]; j++) issue(s + 2, (st + 2) % NSTAGE, j, last);
+              }
+              if (ph == PH - 1) advance();
+            });
+          }
+        } else {
+          constexpr int kFirst = LA::kPieces / 2 + LB::kPieces, kSecond = LA::kPieces / 2;   // loads of the two parts of a step
+#pragma unroll
+          for (int ph = 0; ph < PH; ph++) {
+            if (ph == 3) {
+              // A's second half of this step has landed; its first half and B have been read by every wavefront
+              if (fetching) keep_lookups();
+              if (has_next) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFirst + kSecond) : "memory");
+              else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+              advance();
+            } else if (ph == 7 && has_next) {
               if (fetching) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kFirst + kSecond - 1) : "memory");
               else if (CLAMP && slow_last) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
               else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kSecond) : "memory");
               if (!fetching) clear_tail(next);
             }
-          }
-          if (ph == 0) {
-#pragma unroll
-            for (int f = 0; f < FJ; f++) fb[1][f] = read_frag(false, st, 1, f);
-          }
-          if (ph < 7) {
-#pragma unroll
-            for (int i = 0; i < 2; i++) fa[(ph + 1) & 1][i] = read_frag(true, st, (ph + 1) & 1, ((ph + 1) >> 1) * 2 + i);
+            read_ahead(st, next, ph, has_next);
             if (ph == 1 && fetching) lookup(s + 2);
-          } else if (has_next) {
-#pragma unroll
-            for (int f = 0; f < FJ; f++) fb[0][f] = read_frag(false, next, 0, f);
-#pragma unroll
-            for (int i = 0; i < 2; i++) fa[0][i] = read_frag(true, next, 0, i);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int i = 0; i < 2; i++) {
-#pragma unroll
-            for (int b = 0; b < FJ; b++) blk[ap * 2 + i][b] = Mfma<T>::run16(fa[ph & 1][i], fb[ks][b], blk[ap * 2 + i][b]);
-            if (i == 0) {
-              __builtin_amdgcn_sched_barrier(0);
+            multiply(ph, [&]() {
               if (ph < 2 && has_next) issue(s + 1, next, 6 + ph, last);
               if (ph == 3 && fetching) issue(s + 2, st, 0, last);
               if (ph >= 3 && fetching) issue(s + 2, st, ph - 2, last);
-              __builtin_amdgcn_sched_barrier(0);
+            });
+            if constexpr (COLSUM) {
+              if (ph == 0) colsum_from_stage(st);
             }
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          if constexpr (COLSUM) {
-            if (ph == 0) colsum_from_stage(st);
           }
         }
       };
       if (steps > 0) {
         const std::integral_constant<bool, true> last{};
+        constexpr int kAhead = kPair ? kLoads : kLoads - LA::kPieces / 2;   // of the second step's loads, those issued here
         lookup(0);
 #pragma unroll
-        for (int j = 0; j < 8; j++) issue(0, 0, j, last);
+        for (int j = 0; j < kLoads; j++) issue(0, 0, j, last);
+        advance();
         if (steps > 1) {
-          a_ptr += a_step;
-          b_ptr += b_step;
           lookup(1);
 #pragma unroll
-          for (int j = 0; j < 6; j++) issue(1, 1, j, last);
-          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kFirst + kSecond) : "memory");
+          for (int j = 0; j < kAhead; j++) issue(1, 1, j, last);
+          // (kPair: all of step 0 has landed; two stages: all but the second half of A, waited for in phase 3)
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPair ? kLoads : kAhead + LA::kPieces / 2) : "memory");
+          if constexpr (kPair) {
+            advance();
+            if (steps > 2) lookup(2);
+          }
         } else {
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
@@ -1132,18 +1180,30 @@ struct GemmKernel {
         for (int f = 0; f < FJ; f++) fb[0][f] = read_frag(false, 0, 0, f);
 #pragma unroll
         for (int i = 0; i < 2; i++) fa[0][i] = read_frag(true, 0, 0, i);
-        // (the offset tables are refilled for the steps from s + kOffBank on, every kOffBank steps)
+        const std::integral_constant<bool, true> inner{};
+        const std::integral_constant<bool, false> outer{};
         int s = 0;
         const int whole = steps - ((CLAMP && slow_last) ? 1 : 0);   // (the last step's loads may need care)
-        for (; s + 3 < whole; s += 2) {
+        // (the steps of a turn of the stages, as long as all they load, and look up, exists)
+        for (; s + NSTAGE + (kPair ? 2 : 1) < whole; s += NSTAGE) {
           hash_ahead(s);
-          step(s, std::integral_constant<int, 0>{}, std::integral_constant<bool, true>{});
-          step(s + 1, std::integral_constant<int, 1>{}, std::integral_constant<bool, true>{});
+          step(s, std::integral_constant<int, 0>{}, inner);
+          if constexpr (kPair) hash_ahead(s + 1);
+          step(s + 1, std::integral_constant<int, 1>{}, inner);
+          if constexpr (kPair) {
+            hash_ahead(s + 2);
+            step(s + 2, std::integral_constant<int, 2 % NSTAGE>{}, inner);
+          }
         }
-        for (; s < steps; s += 2) {
+        for (; s < steps; s += NSTAGE) {
           hash_ahead(s);
-          step(s, std::integral_constant<int, 0>{}, std::integral_constant<bool, false>{});
-          if (s + 1 < steps) step(s + 1, std::integral_constant<int, 1>{}, std::integral_constant<bool, false>{});
+          step(s, std::integral_constant<int, 0>{}, outer);
+          if (kPair) hash_ahead(s + 1);
+          if (s + 1 < steps) step(s + 1, std::integral_constant<int, 1>{}, outer);
+          if constexpr (kPair) {
+            hash_ahead(s + 2);
+            if (s + 2 < steps) step(s + 2, std::integral_constant<int, 2 % NSTAGE>{}, outer);
+          }
         }
       }
     } else if constexpr (NSTAGE == 1) {

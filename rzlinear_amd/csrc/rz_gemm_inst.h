@@ -38,7 +38,7 @@ static hipError_t launch_one(GemmParams p, const WeightGradPlan* plan, const Spl
       p.colsum_pitch = plan->colsum_pitch;
     }
   } else if (split != nullptr && split->splits > 1) {
-    constexpr int kPlanTile = TI == 32 && TJ == 128 ? 128 : TI;   // (the C tile of 32 x 128 serves plans of the 128 tile)
+    constexpr int kPlanTile = TI != TJ && TJ == 128 ? 128 : TI;   // (the C tiles of 32 x 128 and 256 x 128 serve plans of the 128 tile)
     if (split->tile != kPlanTile || p.partial == nullptr) return hipErrorInvalidValue;
     splits = split->splits;
     p.r_chunk = split->r_chunk;
@@ -130,6 +130,7 @@ static hipError_t launch_op(GemmParams p, const WeightGradPlan* plan, const Spli
 //        eight of 64 x 32 when there is about one workgroup per compute unit (16-bit: four LDS stages); tuning.stages = 1
 //        selects a single-stage form that leans on several workgroups per compute unit
 //        instead of a pipeline (tuning aid)
+//        16-bit forward / input-grad: 256 x 128, eight wavefronts of 64 x 64, three LDS stages, where pairs are faster
 //    64:  64 x  64, for problems with few tiles: 16-bit sixteen wavefronts of 32 x 32 in four groups that
 //        share every R step between them; fp32 forward / input-grad eight, in two such groups; fp32
 //        weight-grad, and 16-bit rows shorter than a 16-byte piece, four
@@ -147,6 +148,9 @@ static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const 
   const KernelForm form = kernel_form(OP, p.I, p.J, p.R, chunk, tile, workgroups, (int)sizeof(T), tuning);
   if constexpr (sizeof(T) == 2 && OP != kWeightGrad) {
     if (form.rows == 32 && form.cols == 128) return launch_tile<T, OP, 32, 1, 4, 3, false, 2, 128>(p, plan, split, form, stream);
+  }
+  if constexpr (sizeof(T) == 2 && OP != kWeightGrad) {
+    if (form.rows == 256 && form.cols == 128) return launch_tile<T, OP, 256, 4, 2, 3, false, 1, 128>(p, plan, split, form, stream);
   }
   if (form.rows != form.tile || form.cols != tile_cols(form.tile)) return hipErrorInvalidValue;
   switch (form.tile * 1000 + form.waves * 10 + form.stages) {

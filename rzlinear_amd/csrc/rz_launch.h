@@ -589,6 +589,38 @@ static inline bool rows32_form(int tile, int I, int R, int elem_bytes, const rz_
   return tile == 128 && elem_bytes == 2 && I <= 32 && R * elem_bytes >= 16 && t.tile == 0 && t.stages != 1 && t.clamp != -1;
 }
 
+// 16-bit forward / input-grad of more than 64 rows: roughly how long the contraction kernel takes, in microseconds, with C tiles
+// of rows x cols over `slices` slices of `steps` steps of 64.  A round of workgroups takes its steps and a fixed part (fill,
+// store of C); the 256-row tiles' steps take longer the fuller the chip is, because the board lowers its clock.  Fitted to
+// 2790 measurements (forward and input-grad of 84 shapes of 40 to 16384 rows and 256 to 12000 columns, aligned and odd, every
+// tile and one to eight slices): the plan taken with it is 1.5 % from the best form measured on average, that of the
+// rate model before it, which knew neither the 256 x 128 tile nor the present 256 tile, 6.9 %.
+static inline double store16_us(int rows, int cols, int I, int J, int slices, double steps) {
+  const double wgs = (double)(((I + rows - 1) / rows) * (long long)((J + cols - 1) / cols)) * slices;
+  auto rounds_of = [&](double per) { return (double)((long long)((wgs + per - 1) / per)); };
+  const double rounds = rounds_of(kComputeUnits), fill = wgs / (rounds * kComputeUnits);
+  const double launch = 2.8;
+  if (rows == 256 && cols == 256) return launch + rounds * (steps * 0.973 * (1.0 + 0.394 * fill) + 11.4);
+  if (rows == 256) return launch + rounds * (steps * 0.55 * (1.0 + 0.41 * fill) + 6.5);
+  if (rows == 128) {
+    const double one = steps * 0.474 + 4.5, two = steps * 1.079 + 3.8;   // a compute unit's one workgroup of eight wavefronts; two of four
+    if (wgs <= kComputeUnits * 3 / 2) return launch + rounds * one;
+    const double full = (double)((long long)(wgs / (2 * kComputeUnits))), rest = wgs - full * 2 * kComputeUnits;
+    return launch + full * two + (rest <= 0.0 ? 0.0 : rest > kComputeUnits ? two : one * 1.217);
+  }
+  return launch + (wgs <= kComputeUnits ? steps * 0.214 + 2.3 : rounds_of(2 * kComputeUnits) * (steps * 0.441 + 2.3));
+}
+
+// ... whose plan is the 128 tile: whether pairs of tiles, 256 x 128, are faster (the square tile reads a half more from LDS per
+// multiplication, which is what bounds it; a pair leaves half the compute units idle where there are few tiles).  bf16: 2048 x 4096
+// over 1024 23.2 -> 20.1 us; 3001 x 1531 over 2047 49.7 -> 35.9; but 2048^3 22.8 -> 29.4 if it were taken there.
+static inline bool pair_form(int tile, int I, int J, int R, int chunk, int elem_bytes, const rz_tuning& t) {
+  if (tile != 128 || elem_bytes != 2 || I <= 128 || R < 8 || t.tile != 0 || t.stages == 1 || t.clamp == -1) return false;
+  const int slices = chunk < R ? (R + chunk - 1) / chunk : 1;
+  const double steps = (double)(((chunk < R ? chunk : R) + 63) / 64);
+  return store16_us(256, 128, I, J, slices, steps) < store16_us(128, 128, I, J, slices, steps) * 0.97;
+}
+
 // Slices up to which a cut contraction is finished by its own kernel (GemmParams::finish; 0: never).  The
 // slice that comes last at a tile reads the others' planes by itself, four bytes per lane and load, after
 // an atomic's round trip: that pays up to four slices, where the rows of a tile are real (a batch of
@@ -652,11 +684,19 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
       const double steps = (double)steps_per * (TR * elem_bytes / 128);
       const double rate = peak * tile_rate((double)tiles * slices, tile, elem_bytes, lo64, direct || elem_bytes == 2) * useful * steps / (steps + fill);
       double us = 2.0 * (double)I * (double)J * (double)R / rate + 4.0;
+      // (16-bit, more than 64 rows: by the fitted times of the kernels; a slice's planes as fitted with them)
+      const bool fitted = elem_bytes == 2 && I > 64;
+      if (fitted) {
+        const bool pair = pair_form(tile, I, J, R, slices > 1 ? steps_per * TR : R, elem_bytes, t);
+        us = store16_us(pair ? 256 : tile, tile, I, J, slices, (double)steps_per * (TR / 64.0));
+      }
       // (up to finish_slices the kernel finishes its own tiles: every plane is written, all but one are read
       //  back by the finishing workgroups, and no second kernel is launched — worth a couple of microseconds
       //  and a plane; fp32, M = 16384, K = 512, N = 1024 input-grad, planes of 33 MB: the 256 tile in two
       //  slices 155 us against the whole 128 tile's 136)
-      if (slices > 1 && slices <= finish_slices(tile, I, J, R, elem_bytes, t) && t.finish != -1) us += (2.0 * slices - 1.0) * (double)I * J * 4.0 / 4.0e6 + 2.0;
+      const bool finished = slices > 1 && slices <= finish_slices(tile, I, J, R, elem_bytes, t) && t.finish != -1;
+      if (slices > 1 && fitted) us += finished ? (2.0 * slices - 1.0) * (double)I * J * 4.0 / 8.0e6 + 3.5 : (2.0 * slices * (double)I * J * 4.0 + (double)I * J * elem_bytes) / 7.0e6 + 0.5;
+      else if (finished) us += (2.0 * slices - 1.0) * (double)I * J * 4.0 / 4.0e6 + 2.0;
       else if (slices > 1) us += (2.0 * slices * (double)I * J * 4.0 + (double)I * J * elem_bytes) / 4.0e6 + (direct ? 3.0 : 4.0);
       else whole_us = us;
       // (near ties go to the larger tile and the fewer slices, which come first)
@@ -748,6 +788,14 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
     f.stages = 3;
     f.step = 128;
     f.full = I == 32 && J % 128 == 0 && R % 128 == 0 && chunk % 128 == 0;
+    f.clamp = !f.full;
+  }
+  // 16-bit forward / input-grad on the planner's 128 tile: two tiles of one column by one workgroup, where that is the faster
+  if (op != kWeightGrad && f.rows == 128 && pair_form(tile, I, J, R, chunk, elem_bytes, t)) {
+    f.rows = 256;
+    f.waves = 8;
+    f.stages = 3;
+    f.full = I % 256 == 0 && J % 128 == 0 && R % 64 == 0 && chunk % 64 == 0;
     f.clamp = !f.full;
   }
   return f;

@@ -249,3 +249,45 @@ def test_16_bit_pipelined_tiles_at_few_steps(oracle, tile, steps, rest, extents,
         # (fp32 sums of exact products: at most r of them per stored value and a few dozen values per slot)
         assert np.abs(out.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()
         assert_close(dbias.float().cpu().numpy(), dy64.sum(0), dtype, "bias gradient")
+
+
+@pytest.mark.parametrize("dtype", SIXTEEN, ids=str)
+@pytest.mark.parametrize("extents", [(2048, 2304), (2030, 2299)], ids=str)
+@pytest.mark.parametrize("r", [8, 64, 65, 128, 191, 192, 256, 300, 320, 384, 1000, 1088, 2300], ids=str)
+def test_16_bit_pairs_of_tiles(oracle, extents, r, dtype):
+    """288 tiles of 128 are more than compute units: pairs, 144 workgroups of 256 x 128 — fewer steps than its three stages
+    hold, every remainder of them, a partial last step, past the first bank of the offset table; complete and ragged."""
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearBackward import rz_linear_backward_input_grad_tl
+    from rzlinear_amd.impl.RzLinearForward import rz_linear_forward_bias_tl
+    (a, b), H, BK, BN = extents, 20000, 32, 64
+    _say(r, extents, dtype)
+    bias = torch.randn((b,), generator=torch.Generator().manual_seed(4)).to(dtype)
+    (x, hw, _), (x64, hw64, _) = make_inputs(a, r, b, H, dtype, seed=r)
+    with _lib.tuning(split=-1):
+        for op, K, N in ((0, r, b), (1, b, r)):
+            q = _lib.plan_query(op, a, K, N, H, BK, BN, _lib.dtype_code(x))
+            assert (q["tile"], q["slices"], q["workgroups"], q["step"]) == (128, 1, 144, 64)
+        y = rz_linear_forward_bias_tl(x, hw, bias.cuda(), 0.75, a, r, b, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
+        dx = rz_linear_backward_input_grad_tl(x, hw, 0.75, a, b, r, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
+    assert_close(y.float().cpu().numpy(), oracle.forward(x64, hw64, b, BK, BN, R1024, 0.75) + bias.double().numpy(), dtype, "y")
+    assert_close(dx.float().cpu().numpy(), oracle.input_grad(x64, hw64, b, BK, BN, R1024, 0.75), dtype, "dx")
+
+
+@pytest.mark.parametrize("shape,slices", [((200, 6000, 6000, 20000, 32, 64), 5), ((896, 3968, 2368, 20000, 64, 64), 3), ((900, 4001, 2371, 20000, 32, 64), 3)], ids=str)
+def test_16_bit_cut_pairs_of_tiles(oracle, shape, slices):
+    """Pairs over slices of the contraction, their planes added by the second kernel or in the kernel: the same bits."""
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearForward import rz_linear_forward_bias_tl
+    M, K, N, H, BK, BN = shape
+    _say(shape)
+    (x, hw, _), (x64, hw64, _) = make_inputs(M, K, N, H, torch.bfloat16, seed=3)
+    bias = torch.randn((N,), generator=torch.Generator().manual_seed(4)).bfloat16()
+    out = []
+    for finish in (0, -1):
+        with _lib.tuning(split=slices, finish=finish):
+            q = _lib.plan_query(0, M, K, N, H, BK, BN, _lib.RZ_BF16)
+            assert (q["tile"], q["slices"], q["workgroups"]) == (128, slices, -(-M // 256) * -(-N // 128) * slices)
+            out.append(rz_linear_forward_bias_tl(x, hw, bias.cuda(), 0.75, M, K, N, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN))
+    assert torch.equal(out[0], out[1])
+    assert_close(out[0].float().cpu().numpy(), oracle.forward(x64, hw64, N, BK, BN, R1024, 0.75) + bias.double().numpy(), torch.bfloat16, "y")
