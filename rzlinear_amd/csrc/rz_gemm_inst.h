@@ -202,8 +202,8 @@ static hipError_t launch_window_form(const WindowParams& p, int windows, hipStre
 template <typename T, int TBN>
 static hipError_t launch_window_one(const WindowParams& p, int windows, hipStream_t stream) {
   constexpr int kVec = 16 / (int)sizeof(T);
-  // (the staged form keeps a lane's piece offsets, up to sixteen rows, in 32-bit registers)
-  if (p.K % kVec == 0 && p.N % kVec == 0 && p.ldx < (1 << 26) && p.lddy < (1 << 26))
+  // (the staged form keeps the byte offsets of a lane's pieces, up to sixteen rows, in 32-bit registers)
+  if (p.K % kVec == 0 && p.N % kVec == 0 && p.ldx < (1 << 25) && p.lddy < (1 << 25))
     return launch_window_form<T, TBN, true>(p, windows, stream);
   return launch_window_form<T, TBN, false>(p, windows, stream);
 }

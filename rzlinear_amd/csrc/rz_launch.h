@@ -478,8 +478,8 @@ static inline WindowPlan plan_window(int M, int K, int N, int H, int BK, int BN,
   const long long w = pl.window;
   // Rough times in microseconds, fitted to measurements at K = N = 10240, H = 6.5 M on MI355X.
   // Scatter kernel: K*N atomics at about 184 G/s plus the product.  Window kernel: every
-  // workgroup works through tiles * (window + tile) / H tiles; a tile costs about 0.31 us plus
-  // 0.18 us (16-bit), or 0.43 us plus 0.63 us (fp32: the fp32 MFMA rate), per 32 rows of M (the
+  // workgroup works through tiles * (window + tile) / H tiles; a tile costs about 0.25 us plus
+  // 0.16 us (16-bit; M = 32 56 us, 128 91, 192 135, 256 188), or 0.43 us plus 0.63 us (fp32: the fp32 MFMA rate), per 32 rows of M (the
   // operands of every tile come out of L2 again: tiles that share a window share no rows or
   // columns of W; a wavefront has three groups of rows in flight, which is what its registers hold).
   const double chunks = (double)((M + 31) / 32);
@@ -491,7 +491,7 @@ static inline WindowPlan plan_window(int M, int K, int N, int H, int BK, int BN,
   //  time per tile — M = 256, K = 10239, N = 10240, bf16: 411 us against 190 us with K = 10240)
   const int vec = 16 / elem_bytes;
   const double by_elements = (K % vec == 0 && N % vec == 0) ? 1.0 : 2.2;
-  double t_window = wg_rounds * per_wg * by_elements * ((elem_bytes == 4 ? 0.43 + 0.63 * chunks : 0.31 + 0.18 * chunks)) + (planned ? 5.0 : 28.0);
+  double t_window = wg_rounds * per_wg * by_elements * ((elem_bytes == 4 ? 0.43 + 0.63 * chunks : 0.25 + 0.16 * chunks)) + (planned ? 5.0 : 28.0);
   // Every element of dHW receives K*N / H tiles, and the adds into one place of a window go in a
   // fixed order, one after the other: with many tiles per element that chain is what takes the
   // time, about 1.7 us a link (K = 2048, N = 8192, H = 200000: 84 links, 158 us at M = 32 — folded

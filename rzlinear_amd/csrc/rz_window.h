@@ -15,7 +15,7 @@
 // so no wavefront waits for another — and adds the part inside the window with plain LDS
 // read-add-write.  Slices of different
 // tiles may overlap: a tile is added only after every earlier tile of the list whose slice
-// meets its own has been added (a flag per list entry, polled in LDS), so the summation order
+// meets its own has been added (the wavefronts' progress, polled in LDS), so the summation order
 // of every element is the list order whatever the timing.  Finally the window is stored: every
 // element of dHW is written exactly once, with no atomics and no clearing pass.  A tile that
 // straddles a window boundary is computed by both neighbours.
@@ -101,7 +101,7 @@ struct WindowKernel {
   struct Smem {
     int list[kList];              // units found in this pass (tile id * units per tile + unit), ascending
     int offs[kList];              // ... their offsets in hashed_weight
-    int done[kList];              // ... and whether they have been added to the window
+    int progress[kWaves];         // how many of its units every wavefront has added to the window
     int count[2][kWaves];
     int spoilt;                   // a wavefront gave up waiting for an earlier strip: the window is stored as NaN
     alignas(16) T stage[kWaves][kStageElems];
@@ -242,7 +242,6 @@ struct WindowKernel {
         for (int i = tid; i < found; i += kThreads) {
           sm.list[i] = min(max(p.plan_list[plan_lo + lo + i], 0), (total << ushift) - 1);
           sm.offs[i] = min(max(p.plan_offs[plan_lo + lo + i], 0), p.H - 1);
-          sm.done[i] = 0;
         }
         hi = lo + found;
       } else {
@@ -304,7 +303,6 @@ struct WindowKernel {
                 hits &= hits - 1u;
                 sm.list[mine] = (id << ushift) + un;
                 sm.offs[mine] = (int)unit_start(offv[u], un);
-                sm.done[mine] = 0;
                 mine++;
               }
               at += __shfl(incl, 63, 64);
@@ -313,7 +311,8 @@ struct WindowKernel {
         }
       }
       lo = hi;
-      __syncthreads();   // list complete, flags cleared
+      if (tid < kWaves) sm.progress[tid] = 0;
+      __syncthreads();   // list complete, progress cleared
 
       // ---- every wavefront works through list entries wave, wave + kWaves, ... on its own ----
       // An item is one group of rows of M of one tile.  No barrier in here: a wavefront that
@@ -326,15 +325,27 @@ struct WindowKernel {
       // for ALL loads at the first use behind the join — the item just requested included.
       // Beyond the wavefront's last item the last strip is fetched again (valid addresses, in
       // cache; what arrives is multiplied into accumulators that nobody reads any more).
-      // Staged form: what a fetch needs of its strip is worked out once per strip and kept in
-      // scalar registers (the strip's first column in X and in dY, whether all its columns
-      // exist), and what it needs of the lane once per kernel (lane_x / lane_y: element
-      // offset of the lane's piece from the group's first row); an item then costs two scalar
-      // multiply-adds and three loads with a uniform base.  Only groups with rows beyond M and
-      // strips at the edge of the matrix take the path with per-lane checks.
-      // (offsets, not pointers: a pointer carried round the loop would lose its address space
-      //  and turn the loads into flat ones, which also count as LDS traffic)
-      int strip_x = 0, strip_k0 = 0, strip_n0 = 0;
+      // Staged form: what a fetch needs of its strip is worked out once per strip: whether all its columns exist, and
+      // the byte offset of every piece of the lane from the group's first row (32 bits).  The group's rows are a
+      // uniform pointer that moves on with the groups, so that an item costs two scalar additions and three loads
+      // with a scalar base.  Only groups with rows beyond M and strips at the edge of the matrix take the path with
+      // per-lane checks, which changes offsets, not pointers: a choice between two pointers loses their address space, and
+      // flat loads count as LDS traffic too, so that every wait for LDS waited for the loads just issued (K = N = 10240, bf16:
+      // M = 32 68.0 -> 62.1 us, M = 128 110.5 -> 95.6 us).
+      typedef uint32_t u32x4_any_t __attribute__((ext_vector_type(4), aligned(2)));   // (a piece starts at any element)
+      typedef const char __attribute__((address_space(1)))* global_ptr;
+      auto load_piece = [&](const T* rows, uint32_t at) -> u32x4_t {
+        return *reinterpret_cast<const u32x4_any_t __attribute__((address_space(1)))*>((global_ptr)rows + at);
+      };
+      const T* rows_x = gX;
+      const T* rows_y = gdY;
+      const int64_t next_x = kGroupRows * p.ldx, next_y = kGroupRows * p.lddy;
+      uint32_t at_x = 0, at_y[BJ];
+#pragma unroll
+      for (int q = 0; q < BJ; q++) at_y[q] = 0;
+      // every unit lies inside the matrices as a whole
+      const bool all_whole = (p.K & (p.h.BK - 1)) == 0 && (p.N & (TBN - 1)) == 0;
+      int strip_k0 = 0, strip_n0 = 0;
       bool strip_whole = false;
       // which of a lane's pieces of the group at row m0 of the unit at (k0, n0) lie inside the matrices
       auto pieces_inside = [&](int m0, int k0, int n0, bool& okx, bool (&oky)[BJ]) {
@@ -346,7 +357,7 @@ struct WindowKernel {
       };
       // ... and the same for the strip being multiplied
       int mult_k0 = 0, mult_n0 = 0;
-      bool mult_whole = false;
+      bool mult_whole = all_whole;
       auto fetch_next = [&](auto set) {
         constexpr int S = decltype(set)::value;
         if constexpr (STAGED) {
@@ -359,17 +370,18 @@ struct WindowKernel {
             strip_n0 = tn * TBN + (un % kParts) * UC;      // ... and first column
             strip_whole = strip_k0 + 32 <= p.K && strip_n0 + UC <= p.N;
             // (a strip that begins beyond K contributes nothing; its base is kept inside the matrix)
-            strip_x = strip_k0 < p.K ? strip_k0 : p.K - 1;
+            at_x = (uint32_t)(lane_x + (strip_k0 < p.K ? strip_k0 : p.K - 1)) * (uint32_t)sizeof(T);
+#pragma unroll
+            for (int q = 0; q < BJ; q++) at_y[q] = (uint32_t)(lane_y[q] + strip_n0) * (uint32_t)sizeof(T);
+            rows_x = gX;
+            rows_y = gdY;
           }
           const int m0 = fg * kGroupRows;
-          const T* rows_x = gX + ((int64_t)m0 * p.ldx + strip_x);
-          const T* rows_y = gdY + ((int64_t)m0 * p.lddy + strip_n0);
-          const T* src_x = rows_x + lane_x;
-          const T* src_y[BJ];
+          uint32_t fetch_x = at_x, fetch_y[BJ];
 #pragma unroll
-          for (int q = 0; q < BJ; q++) src_y[q] = rows_y + lane_y[q];
+          for (int q = 0; q < BJ; q++) fetch_y[q] = at_y[q];
           if (!(strip_whole && m0 + kGroupRows <= p.M)) {   // (uniform, rare)
-            // a piece outside the matrix is fetched from inside it (and replaced by zero when the
+            // a piece outside the matrix is fetched from the group's first row (and replaced by zero when the
             // item is multiplied, where the same checks are made again: nothing about a set is
             // carried round the ring but its data)
             // (the empty statement keeps this block out of the usual path: its arithmetic would
@@ -377,13 +389,15 @@ struct WindowKernel {
             asm volatile("" ::: "memory");
             bool okx, oky[BJ];
             pieces_inside(m0, strip_k0, strip_n0, okx, oky);
-            src_x = okx ? src_x : gX + (int64_t)m0 * p.ldx;
+            fetch_x = okx ? at_x : 0u;
 #pragma unroll
-            for (int q = 0; q < BJ; q++) src_y[q] = oky[q] ? src_y[q] : gdY + (int64_t)m0 * p.lddy;
+            for (int q = 0; q < BJ; q++) fetch_y[q] = oky[q] ? at_y[q] : 0u;
           }
-          __builtin_memcpy(&px[S], src_x, 16);
+          px[S] = load_piece(rows_x, fetch_x);
 #pragma unroll
-          for (int q = 0; q < BJ; q++) __builtin_memcpy(&py[S][q], src_y[q], 16);
+          for (int q = 0; q < BJ; q++) py[S][q] = load_piece(rows_y, fetch_y[q]);
+          rows_x += next_x;
+          rows_y += next_y;
           if (++fg == ngroups) {
             fg = 0;
             ft++;
@@ -424,23 +438,42 @@ struct WindowKernel {
           }
         }
       };
+      // The earlier entries whose spans meet that of entry e must be added before it.  Lane l looks at the entries l,
+      // l + 64, ..., all of wavefront l % kWaves, which adds its entries in order: what counts is the last of them that
+      // meets.  Worked out when a unit begins, while its loads are on their way; what is left for the end, where other
+      // wavefronts wait in turn, is one look at the wavefronts' progress.  (Looking at every earlier entry's offset and flag
+      // there: K = N = 10240 bf16 with M = 32 / 128 62.1 / 95.6 us; so 56.4 / 91.3.)
+      int need_added = 0;
+      auto must_be_added = [&](int e) -> int {
+        const int off = __builtin_amdgcn_readfirstlane(sm.offs[e]);
+        int need = 0;
+        for (int f0 = 0; f0 < e; f0 += 4 * 64) {   // (uniform; four reads at a time)
+          int d[4];
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const int f = f0 + q * 64 + lane;
+            d[q] = sm.offs[f < e ? f : e] - off;
+          }
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const int f = f0 + q * 64 + lane;
+            if (f < e && d[q] < kUnitSpan && d[q] > -kUnitSpan) need = f / kWaves + 1;
+          }
+        }
+        return need;
+      };
       // add the finished strip of list entry `e` into the window, after the earlier strips whose
-      // slices meet its own, and raise its flag
+      // slices meet its own, and count it
       auto add_tile = [&](int e) {
         const int tile_off = __builtin_amdgcn_readfirstlane(sm.offs[e]);
-        // lane l looks at the earlier entries l, l + 64, ...: straight-line LDS reads, no branches.
+        // (need_added: how many units lane l's wavefront, l % kWaves, must have added, see must_be_added: one LDS read per look)
         // The wait is bounded: an entry only waits for earlier ones, whose owners wait for still
-        // earlier ones, so it ends by itself; should a flag never come all the same (a list that
-        // is not what this kernel expects), the wavefront gives up after kPollLimit looks, marks
+        // earlier ones, so it ends by itself; should one never be added all the same (a list that
+        // is not what this kernel expects), the wavefront gives up after poll_limit looks, marks
         // the window as spoilt and goes on, so that every wavefront reaches the end of the kernel.
         for (int polls = 0;; polls++) {
-          bool pending = false;
-          for (int f = lane; f < e; f += 64) {
-            const int d = sm.offs[f] - tile_off;
-            const int dn = __hip_atomic_load(&sm.done[f], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            pending |= (d < kUnitSpan) & (d > -kUnitSpan) & (dn == 0);
-          }
-          if (!__any(pending)) break;
+          const int added = __hip_atomic_load(&sm.progress[lane % kWaves], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          if (!__any(added < need_added)) break;
           if (polls >= p.poll_limit) {   // (uniform)
             if (lane == 0) __hip_atomic_store(&sm.spoilt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             break;
@@ -500,13 +533,14 @@ struct WindowKernel {
             }
           }
         }
-        if (lane == 0) __hip_atomic_store(&sm.done[e], 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (lane == 0) __hip_atomic_store(&sm.progress[wave], e / kWaves + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
       };
       int pt = 0, pg = 0;      // tile ordinal and group of the item being multiplied
       auto item = [&](auto set) {
         constexpr int S = decltype(set)::value;
         // the set freed by the previous item takes the loads of the item kDepth - 1 ahead
         fetch_next(std::integral_constant<int, (S + kDepth - 1) % kDepth>{});
+        if (pg == 0 && pt < my_tiles) need_added = must_be_added(wave + pt * kWaves);   // (uniform)
         if constexpr (STAGED) {
           {
             // pieces -> this wavefront's staging area (LDS operations of one wavefront are carried
@@ -518,7 +552,7 @@ struct WindowKernel {
             u32x4_t wx = px[S], wy[BJ];
 #pragma unroll
             for (int q = 0; q < BJ; q++) wy[q] = py[S][q];
-            if (pg == 0) {   // (uniform) a new unit
+            if (pg == 0 && !all_whole) {   // (uniform) a new unit
               const int ptc = pt < my_tiles ? pt : my_tiles - 1;
               const int v = __builtin_amdgcn_readfirstlane(sm.list[wave + ptc * kWaves]);
               const int id = v >> ushift, un = v & (units - 1), tk = id / p.tiles_n;
@@ -528,6 +562,7 @@ struct WindowKernel {
             }
             if (!(mult_whole && (pg + 1) * kGroupRows <= p.M)) {
               asm volatile("" ::: "memory");
+              // (with all_whole the coordinates are zero: only the rows can lie outside)
               bool okx, oky[BJ];
               pieces_inside(pg * kGroupRows, mult_k0, mult_n0, okx, oky);
               wx = okx ? wx : z;
