@@ -1348,8 +1348,10 @@ struct GemmKernel {
       }
     }
 
-    // (kBlk16) to the layout of 32 x 32 blocks that the epilogue knows: element e of a 16 x 16 block is row 4 (lane / 16) + e,
-    // column lane % 16; of two blocks side by side, the rows of 16 lanes change places so that 32 lanes hold one row
+    // (kBlk16) to 32 x 32 blocks with a row's 32 columns in 32 lanes: element e of a 16 x 16 block is row 4 (lane / 16) + e, column
+    // lane % 16; of two blocks side by side, odd and even groups of 16 lanes change places.  (Rows as block_row says.  A
+    // second exchange, of halves, would give the rows of a 32x32 MFMA's result, but costs as much again: K = N = 10240 bf16 weight-grad
+    // of M = 64, where 1600 tiles have one step each, 126 -> 123 us.)
     if constexpr (kBlk16) {
 #pragma unroll
       for (int a = 0; a < MI * 2; a++)
@@ -1361,10 +1363,8 @@ struct GemmKernel {
             const float lo = blk[a][2 * b][e], hi = blk[a][2 * b + 1][e];
             const u32x2_t x = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi), false, false);
             const uint32_t x0 = x[0], x1 = x[1];
-            const u32x2_t y = __builtin_amdgcn_permlane32_swap(x0, x1, false, false);
-            const uint32_t y0 = y[0], y1 = y[1];
-            acc[a >> 1][b][(a & 1) * 8 + e] = __builtin_bit_cast(float, y0);
-            acc[a >> 1][b][(a & 1) * 8 + 4 + e] = __builtin_bit_cast(float, y1);
+            acc[a >> 1][b][(a & 1) * 8 + e] = __builtin_bit_cast(float, x0);
+            acc[a >> 1][b][(a & 1) * 8 + 4 + e] = __builtin_bit_cast(float, x1);
           }
     }
 
@@ -1373,7 +1373,9 @@ struct GemmKernel {
     // element e of acc is from here on row block_row(e) of the block, e < kElems.
     constexpr int kElems = 16 / WK;
     static_assert(WK == 1 || WK == 2 || WK == 4, "a group takes whole quarters of a block's elements");
-    auto block_row = [&](int e) -> int { return ((WK > 1 ? wave_k * (kElems / 4) : 0) + (e >> 2)) * 8 + (lane >> 5) * 4 + (e & 3); };
+    auto row_step = [](int e) -> int { return kBlk16 ? (e >> 3) * 16 + ((e >> 2) & 1) * 4 + (e & 3) : (e >> 2) * 8 + (e & 3); };
+    const int row_base = (WK > 1 ? wave_k * (kElems / 4) : 0) * 8 + (lane >> 5) * (kBlk16 ? 8 : 4);
+    auto block_row = [&](int e) -> int { return row_base + row_step(e); };
     auto merge_groups = [&]() {
       if constexpr (WK > 1) {
         float* park = reinterpret_cast<float*>(&sm);
@@ -1403,7 +1405,7 @@ struct GemmKernel {
     };
 
     // ---- epilogue ---------------------------------------------------------------------------
-    // accumulator element e of a 32x32 block: row (e/4)*8 + (lane/32)*4 + e%4, column lane%32
+    // accumulator element e of a 32x32 block: row block_row(e), column lane % 32
     if constexpr (OP == kWeightGrad) {
       const bool image_mode = p.image_pitch > 0;
       float* image = reinterpret_cast<float*>(&sm);   // aliases the operand stages
@@ -1434,8 +1436,9 @@ struct GemmKernel {
       int* etab = image_mode ? reinterpret_cast<int*>(image + p.image_pitch) : sm.off;
       const OffWindow w = off_window(p.h, i0, TI, j0, TJ);
       const bool tiled = p.tiles_out != nullptr;
+      const int ntn_shift = __builtin_ctz(w.ntn);   // (a power of two)
       for (int t = tid; t < w.count; t += kThreads) {
-        const int tk = w.tk0 + t / w.ntn, tn = w.tn0 + t % w.ntn;
+        const int tk = w.tk0 + (t >> ntn_shift), tn = w.tn0 + (t & (w.ntn - 1));
         if (tiled)   // where the tile starts in the tile-by-tile output (-1: the C tile reaches beyond the grid)
           etab[t] = (tk < p.out_tiles_k && tn < p.out_tiles_n)
                         ? ((by * p.out_tiles_k + tk) * p.out_tiles_n + tn) << (p.h.bk_shift + p.h.bn_shift)
@@ -1450,6 +1453,35 @@ struct GemmKernel {
         // (narrow: the tiles are kept in the layer's 16-bit dtype — each value rounded once here, added up in fp32 by the fold)
         constexpr bool kNarrow = decltype(narrow)::value;
         T* const out16 = reinterpret_cast<T*>(p.tiles_out);
+        if (p.h.bk_shift >= 5 && p.h.bn_shift >= 5) {
+          // a 32 x 32 block lies in one hashed tile: its first element is worked out in scalar registers and moved on by rows
+          // there, and a lane's part is the same for every block, so that a value costs its scaling, its rounding and its store
+          // (K = N = 10240, M = 1024 bf16: the epilogue took 36 of 211 us, 21 of them for everything but the stores; 199 us so, and
+          // M = 64, K = 12000, N = 9000, ragged tiles, 86 -> 63 us)
+          const uint32_t lane_at = (uint32_t)(row_base * p.h.BN + (lane & 31));
+#pragma unroll
+          for (int a = 0; a < MI; a++)
+#pragma unroll
+            for (int b = 0; b < MJ; b++) {
+              const int k0 = i0 + blk_i(a), n0 = j0 + blk_j(b);   // (uniform)
+              const int start = __builtin_amdgcn_readfirstlane(etab[(((k0 >> p.h.bk_shift) - w.tk0) << ntn_shift) + ((n0 >> p.h.bn_shift) - w.tn0)]);
+              if (start < 0) continue;   // (beyond the grid)
+              const uint32_t first = (uint32_t)(start + (k0 & (p.h.BK - 1)) * p.h.BN + (n0 & (p.h.BN - 1)));
+              auto store_block = [&](auto whole) {
+                const bool col_ok = n0 + (lane & 31) < p.J;
+#pragma unroll
+                for (int e = 0; e < kElems; e++) {
+                  const uint32_t row = first + (uint32_t)(row_step(e) * p.h.BN);   // (uniform)
+                  const float v = (decltype(whole)::value || (col_ok && k0 + block_row(e) < p.I)) ? acc[a][b][e] * p.scale : 0.f;
+                  if constexpr (kNarrow) (out16 + row)[lane_at] = Tr::from_float(v);
+                  else (p.tiles_out + row)[lane_at] = v;
+                }
+              };
+              if (FULL || (k0 + 32 <= p.I && n0 + 32 <= p.J)) store_block(std::true_type{});   // (uniform)
+              else store_block(std::false_type{});
+            }
+          return;
+        }
 #pragma unroll
         for (int a = 0; a < MI; a++)
 #pragma unroll
@@ -1573,7 +1605,7 @@ struct GemmKernel {
                 const bool col_ok = j0 + blk_j(b) + (lane & 31) < p.J;
 #pragma unroll
                 for (int e = 0; e < kElems; e++)
-                  acc[a][b][e] = (col_ok && k0 + (e >> 2) * 8 + (e & 3) < p.I) ? acc[a][b][e] * p.scale : 0.f;
+                  acc[a][b][e] = (col_ok && k0 + row_step(e) < p.I) ? acc[a][b][e] * p.scale : 0.f;
               }
           }
           const float round_scale = FULL ? p.scale : 1.f;
@@ -1587,10 +1619,10 @@ struct GemmKernel {
                     float cur[kElems];
 #pragma unroll
                     for (int e = 0; e < kElems; e++)
-                      cur[e] = image[blk_base[a][b] + ((e >> 2) * 8 + (e & 3)) * p.h.BN];
+                      cur[e] = image[blk_base[a][b] + row_step(e) * p.h.BN];
 #pragma unroll
                     for (int e = 0; e < kElems; e++)
-                      image[blk_base[a][b] + ((e >> 2) * 8 + (e & 3)) * p.h.BN] = cur[e] + acc[a][b][e] * round_scale;
+                      image[blk_base[a][b] + row_step(e) * p.h.BN] = cur[e] + acc[a][b][e] * round_scale;
                   }
                 }
             }

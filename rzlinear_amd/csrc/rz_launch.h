@@ -335,6 +335,13 @@ static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK
     // M = 1024 1938 -> 1797 us, M = 4096 7002 -> 6449 us; K = N = 4096, one round exactly, stays
     // with the 256 tile: 1043 against 1085 us); with fewer, a short M takes the 128 tile, whose
     // paired workgroups hide each other's stores
+    // 16-bit with a short M: a workgroup of the 256 tile is then mostly fill and store, which two workgroups of the 128 tile
+    // on a compute unit hide behind each other — from two rounds of 256 tiles on (M = 64: K = N = 6000 78 -> 73 us, K = 12000,
+    // N = 9000 140 -> 135; K = 8192, N = 4096, two rounds exactly, 65 either way; M = 512: 104 / 100 and 205 / 214 us)
+    if (pl.tile == 256 && elem_bytes == 2 && t.fold != -1 && M <= 256 && tile_count(K, N, 256) > 2 * kComputeUnits) {
+      const FoldPlan f = plan_fold(K, N, H, BK, BN, 1);
+      if (f.use && !f.small) pl.tile = 128;
+    }
     if (pl.tile == 256 && elem_bytes == 4 && t.fold != -1 && plan_fold(K, N, H, BK, BN, 1).use) {
       const long long t256 = tile_count(K, N, 256), t128 = tile_count(K, N, 128);
       if (t256 >= kComputeUnits ? kPairRate128F32 * filled_128(t128) > filled_256(t256) * 1.01 : M <= 2048) pl.tile = 128;
