@@ -120,10 +120,11 @@ struct WeightGradChoice {
   WindowPlan window;
 };
 static WeightGradChoice weight_grad_choice(int M, int K, int N, int H, int BK, int BN, int elem_bytes, int tile_bytes, const rz_tuning& t,
-                                           bool planned) {
-  static thread_local PlanMemo<WeightGradChoice, 19> memo;
-  return memo.get({M, K, N, H, BK, BN, elem_bytes, tile_bytes, planned ? 1 : 0, RZ_TUNING_WORDS(t)}, [&] {
-    WeightGradChoice c = {plan_weight_grad(M, K, N, H, BK, BN, elem_bytes, t, tile_bytes), {}};
+                                           bool planned, size_t limit = (size_t)-1) {
+  static thread_local PlanMemo<WeightGradChoice, 20> memo;
+  const int limit_mb = limit == (size_t)-1 ? -1 : (int)(limit >> 20);
+  return memo.get({M, K, N, H, BK, BN, elem_bytes, tile_bytes, planned ? 1 : 0, limit_mb, RZ_TUNING_WORDS(t)}, [&] {
+    WeightGradChoice c = {plan_weight_grad(M, K, N, H, BK, BN, elem_bytes, t, tile_bytes, limit), {}};
     if (!c.plan.lds_image()) c.window = plan_window(M, K, N, H, BK, BN, elem_bytes, t, c.plan, planned);
     return c;
   });
@@ -436,7 +437,7 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
                             const int32_t R[8], float init_factor, int64_t ldx, int64_t lddy, int dtype,
                             unsigned flags, void* stream, int hash_levels = RZ_HASH_TWO_LEVEL,
                             const rz_tuning* tuning_arg = nullptr, const int32_t* layer_plan = nullptr,
-                            size_t layer_plan_bytes = 0) {
+                            size_t layer_plan_bytes = 0, size_t limit = (size_t)-1) {
   if (X == nullptr || dY == nullptr || dHW == nullptr) return RZ_ERR_NULL_POINTER;
   if (dtype_bytes(dtype) == 0) return RZ_ERR_BAD_DTYPE;
   if (M < 1 || ldx < K || lddy < N) return RZ_ERR_BAD_SHAPE;
@@ -460,7 +461,7 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
   }
   const WeightGradChoice choice = weight_grad_choice(M, K, N, H, BK, BN, dtype_bytes(dtype),
                                                      fold_tile_bytes(dtype_bytes(dtype), dhw_dtype == RZ_F32, tuning), tuning,
-                                                     planned && lay.windows > 0);
+                                                     planned && lay.windows > 0, limit);
   const WeightGradPlan& plan = choice.plan;
   const WindowPlan& wp = choice.window;
   const WeightGradWorkspace ws = weight_grad_workspace(plan, wp, H, dhw_dtype == RZ_F32, dbias != nullptr, planned);
@@ -595,6 +596,17 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
     if (bias.part != nullptr) hipLaunchKernelGGL(colsum_kernel, dim3(colsum_blocks(bias, 256)), dim3(256), 0, s, bias);
   }
   return hipGetLastError() == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;
+}
+
+// Workspace of a weight-grad call without a layer plan (0: bad arguments).
+static size_t weight_grad_bytes(int M, int K, int N, int H, int BK, int BN, int dtype, unsigned flags, int with_dbias, const rz_tuning& t,
+                                size_t limit) {
+  const int eb = dtype_bytes(dtype);
+  if (eb == 0 || M < 1 || K < 1 || N < 1 || H < 1 || !tuning_valid(t)) return 0;
+  if (check_tile(BK, BN) != RZ_OK) return 0;
+  const bool dhw_f32 = (flags & RZ_WG_DHW_F32) != 0 || dtype == RZ_F32;
+  const WeightGradChoice c = weight_grad_choice(M, K, N, H, BK, BN, eb, fold_tile_bytes(eb, dhw_f32, t), t, false, limit);
+  return weight_grad_workspace(c.plan, c.window, H, dhw_f32, with_dbias != 0).total_bytes;
 }
 
 }  // namespace rz
@@ -815,13 +827,13 @@ RZ_API int rz_weight_grad_static(const void* X, const void* dY, void* dHW, int M
                                  int BN, const int32_t R[8], float init_factor, int64_t ldx, int64_t lddy,
                                  int dtype, void* stream) {
   // the same kernels and checks as rz_weight_grad; only the workspace differs.  The plan is the
-  // same too, except that the fold (whose tile-by-tile buffer takes 4*K*N bytes and more) gives
-  // way to the scatter kernel when it does not fit the scratch array.
+  // same too, except that the contraction is cut for the fold no further than its tile-by-tile buffer fits the
+  // scratch array, and that the fold gives way to the scatter kernel when it does not fit at all.
   rz_tuning tuning = {};
   if (dtype_bytes(dtype) != 0 && M >= 1 && K >= 1 && N >= 1 && H >= 1) {
-    if (rz_weight_grad_hashed_workspace_bytes(M, K, N, H, BK, BN, dtype, 0u, 0, &tuning) > kScratchBytes) {
+    if (weight_grad_bytes(M, K, N, H, BK, BN, dtype, 0u, 0, tuning, kScratchBytes) > kScratchBytes) {
       tuning.fold = -1;
-      if (rz_weight_grad_hashed_workspace_bytes(M, K, N, H, BK, BN, dtype, 0u, 0, &tuning) > kScratchBytes)
+      if (weight_grad_bytes(M, K, N, H, BK, BN, dtype, 0u, 0, tuning, kScratchBytes) > kScratchBytes)
         return RZ_ERR_SCRATCH_LIMIT;
     }
   }
@@ -835,18 +847,12 @@ RZ_API int rz_weight_grad_static(const void* X, const void* dY, void* dHW, int M
   void* ws = scratch_of_current_device(dHW, &st);
   if (ws == nullptr) return st;
   return weight_grad_impl(X, dY, dHW, nullptr, ws, kScratchBytes, M, K, N, H, BK, BN, R, init_factor, ldx, lddy,
-                          dtype, 0u, stream, RZ_HASH_TWO_LEVEL, &tuning);
+                          dtype, 0u, stream, RZ_HASH_TWO_LEVEL, &tuning, nullptr, 0, kScratchBytes);
 }
 
 RZ_API size_t rz_weight_grad_hashed_workspace_bytes(int M, int K, int N, int H, int BK, int BN, int dtype,
                                                     unsigned flags, int with_dbias, const rz_tuning* tuning) {
-  const int eb = dtype_bytes(dtype);
-  const rz_tuning t = tuning_or_default(tuning);
-  if (eb == 0 || M < 1 || K < 1 || N < 1 || H < 1 || !tuning_valid(t)) return 0;
-  if (check_tile(BK, BN) != RZ_OK) return 0;
-  const bool dhw_f32 = (flags & RZ_WG_DHW_F32) != 0 || dtype == RZ_F32;
-  const WeightGradChoice c = weight_grad_choice(M, K, N, H, BK, BN, eb, fold_tile_bytes(eb, dhw_f32, t), t, false);
-  return weight_grad_workspace(c.plan, c.window, H, dhw_f32, with_dbias != 0).total_bytes;
+  return weight_grad_bytes(M, K, N, H, BK, BN, dtype, flags, with_dbias, tuning_or_default(tuning), (size_t)-1);
 }
 
 RZ_API size_t rz_weight_grad_ex_workspace_bytes(int M, int K, int N, int H, int BK, int BN, int dtype,

@@ -272,12 +272,56 @@ static inline double filled_128(long long tiles) {
 // 1600 tiles in seven half-rounds against 400 in two rounds)
 static constexpr double kPairRate128F32 = 0.955;
 
-static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK, int BN, int elem_bytes,
-                                              const rz_tuning& t, int tile_bytes = 4) {
+// 16-bit forward / input-grad of more than 64 rows: roughly how long the contraction kernel takes, in microseconds, with C tiles
+// of rows x cols over `slices` slices of `steps` steps of 64.  A round of workgroups takes its steps and a fixed part (fill,
+// store of C); the 256-row tiles' steps take longer the fuller the chip is, because the board lowers its clock.  Fitted to
+// 2790 measurements (forward and input-grad of 84 shapes of 40 to 16384 rows and 256 to 12000 columns, aligned and odd, every
+// tile and one to eight slices): the plan taken with it is 1.5 % from the best form measured on average, that of the
+// rate model before it, which knew neither the 256 x 128 tile nor the present 256 tile, 6.9 %.
+static inline double store16_us(int rows, int cols, int I, int J, int slices, double steps) {
+  const double wgs = (double)(((I + rows - 1) / rows) * (long long)((J + cols - 1) / cols)) * slices;
+  auto rounds_of = [&](double per) { return (double)((long long)((wgs + per - 1) / per)); };
+  const double rounds = rounds_of(kComputeUnits), fill = wgs / (rounds * kComputeUnits);
+  const double launch = 2.8;
+  if (rows == 256 && cols == 256) return launch + rounds * (steps * 0.973 * (1.0 + 0.394 * fill) + 11.4);
+  if (rows == 256) return launch + rounds * (steps * 0.55 * (1.0 + 0.41 * fill) + 6.5);
+  if (rows == 128) {
+    const double one = steps * 0.474 + 4.5, two = steps * 1.079 + 3.8;   // a compute unit's one workgroup of eight wavefronts; two of four
+    if (wgs <= kComputeUnits * 3 / 2) return launch + rounds * one;
+    const double full = (double)((long long)(wgs / (2 * kComputeUnits))), rest = wgs - full * 2 * kComputeUnits;
+    return launch + full * two + (rest <= 0.0 ? 0.0 : rest > kComputeUnits ? two : one * 1.217);
+  }
+  return launch + (wgs <= kComputeUnits ? steps * 0.214 + 2.3 : rounds_of(2 * kComputeUnits) * (steps * 0.441 + 2.3));
+}
+
+// The contraction kernel of a 16-bit weight-grad, in microseconds.  The 128 tile's loop loads both operands across the rows
+// of its tile: 1.15 times its forward's with one workgroup on a compute unit, 0.88 with two and whole 16-byte pieces.
+static inline double weight_grad16_us(int tile, int M, int K, int N, int slices) {
+  const double steps = (double)((M + 63) / 64 + slices - 1) / slices;
+  if (tile != 128) return store16_us(tile, tile, K, N, slices, steps);
+  const bool one = tile_count(K, N, 128) * slices <= kComputeUnits * 3 / 2, whole = K % 8 == 0 && N % 8 == 0;
+  return store16_us(128, 128, K, N, slices, steps * (one ? 1.15 : whole ? 0.88 : 1.0));
+}
+
+// ... and what its tiles cost beyond it, stored for the fold kernel and read back.
+static inline double stored_tiles_us(int tile, int M, int K, int N, int slices, int tile_bytes) {
+  return weight_grad16_us(tile, M, K, N, slices) + (double)slices * K * N * tile_bytes * (1.0 / 4.7e6 + 0.3 / 5.0e6);
+}
+
+// A plan for the fold that was chosen as a whole (see plan_weight_grad).
+struct FoldChoice {
+  int tile, slices, tile_bytes;
+};
+
+static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H, int BK, int BN, int elem_bytes,
+                                                      const rz_tuning& t, int tile_bytes, const FoldChoice* chosen = nullptr) {
   WeightGradPlan pl;
   const int pitch = (H + 3) & ~3;
   const bool image = t.lds_image != -1 && (size_t)pitch * sizeof(float) <= kMaxImageBytes;
-  if (t.tile) {
+  if (chosen != nullptr) {
+    pl.tile = chosen->tile;
+    tile_bytes = chosen->tile_bytes;
+  } else if (t.tile) {
     pl.tile = t.tile == 32 ? 64 : t.tile;   // (the 32 x 64 tile serves forward / input-grad only)
   } else if (image) {
     // with the LDS image the M loop can be cut freely (a slice costs one partial image), so
@@ -358,7 +402,9 @@ static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK
   if (want > r_steps) want = r_steps;
   if (want < 1) want = 1;
   if (image && pl.tile >= 128) want = image_slices(tiles, r_steps);
-  if (!image) {
+  if (chosen != nullptr) {
+    want = chosen->slices;
+  } else if (!image) {
     // every slice repeats the K*N adds of the scatter (global atomics, about 5.4 ps each, some 70 %
     // of which the contraction does not hide): the number of slices with the least estimated time
     if (want > 8) want = 8;
@@ -432,6 +478,45 @@ static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK
   pl.colsum_rows = pl.splits * ((K + pl.tile - 1) / pl.tile);
   pl.colsum_pitch = ((N + pl.tile - 1) / pl.tile) * pl.tile;
   pl.colsum_bytes = (size_t)pl.colsum_rows * pl.colsum_pitch * sizeof(float);
+  return pl;
+}
+
+// 16-bit with the tiles stored for the fold kernel: tile and slices together, by the fitted times (the rates above cut M no
+// further than the atomics' K*N adds per slice allow, and know neither what a workgroup's fill and store cost nor the present
+// tiles).  A slice's stored tiles are partial sums: where there are more of them than in the plan by rate they are stored in
+// fp32, whatever the layer's dtype, and so are they where that plan adds into an fp32 image.  (bf16, the module's
+// call: M = 20442, K = 6647, N = 591 477 -> 221 us; 14592, 8448, 448 232 -> 128; from the atomics 11552, 5632, 768 195 -> 121;
+// 200 drawn shapes whose plan changed 1.31 times as fast in the mean, the least 0.97.)
+// limit: bytes of scratch memory that the fold may take.
+static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK, int BN, int elem_bytes,
+                                              const rz_tuning& t, int tile_bytes = 4, size_t limit = (size_t)-1) {
+  const WeightGradPlan by_rate = plan_weight_grad_by_rate(M, K, N, H, BK, BN, elem_bytes, t, tile_bytes);
+  if (elem_bytes != 2 || by_rate.image_pitch > 0 || t.tile != 0 || t.fold == -1) return by_rate;
+  FoldChoice best = {0, 0, 0};
+  // (the plan by rate is left only for one that is faster by more than the fit's error; the 64 tile's times are not fitted for
+  //  this; the atomics: the part of K*N per slice that the contraction does not hide)
+  double best_us = -1.0 + 0.90 * (by_rate.fold.use ? stored_tiles_us(by_rate.tile, M, K, N, by_rate.splits, tile_bytes)
+                                                   : weight_grad16_us(by_rate.tile, M, K, N, by_rate.splits) + (double)by_rate.splits * K * N * 2.8e-6);
+  const int tiles_of[2] = {256, 128};
+  for (int tile : tiles_of) {
+    const int unit = slice_unit(tile, elem_bytes, true), steps = (M + unit - 1) / unit;
+    for (int w = 1; w <= 8 && w <= steps; w++) {
+      const int per = (steps + w - 1) / w;
+      const int bytes = by_rate.fold.use && w <= by_rate.splits ? tile_bytes : 4;
+      const FoldPlan f = plan_fold(K, N, H, BK, BN, w, t.fold == 2, bytes);
+      if ((steps + per - 1) / per != w || !f.use || f.tiles_bytes + f.partial_bytes + f.offsets_bytes > limit) continue;
+      const double us = stored_tiles_us(tile, M, K, N, w, bytes);
+      if (us < best_us * (best.tile == 0 ? 1.0 : 0.97)) {
+        best_us = us;
+        best = {tile, w, bytes};
+      }
+    }
+  }
+  if (best.tile == 0 || (best.tile == by_rate.tile && best.slices == by_rate.splits)) return by_rate;
+  WeightGradPlan pl = plan_weight_grad_by_rate(M, K, N, H, BK, BN, elem_bytes, t, tile_bytes, &best);
+  if (!pl.fold.use) return by_rate;
+  // (the window kernel adds in fp32: 16-bit tiles take no call from it that the plan by rate leaves to it)
+  if (by_rate.fold.use && best.tile_bytes == 2) pl.fold_us = by_rate.fold_us;
   return pl;
 }
 
@@ -596,29 +681,7 @@ static inline bool rows32_form(int tile, int I, int R, int elem_bytes, const rz_
   return tile == 128 && elem_bytes == 2 && I <= 32 && R * elem_bytes >= 16 && t.tile == 0 && t.stages != 1 && t.clamp != -1;
 }
 
-// 16-bit forward / input-grad of more than 64 rows: roughly how long the contraction kernel takes, in microseconds, with C tiles
-// of rows x cols over `slices` slices of `steps` steps of 64.  A round of workgroups takes its steps and a fixed part (fill,
-// store of C); the 256-row tiles' steps take longer the fuller the chip is, because the board lowers its clock.  Fitted to
-// 2790 measurements (forward and input-grad of 84 shapes of 40 to 16384 rows and 256 to 12000 columns, aligned and odd, every
-// tile and one to eight slices): the plan taken with it is 1.5 % from the best form measured on average, that of the
-// rate model before it, which knew neither the 256 x 128 tile nor the present 256 tile, 6.9 %.
-static inline double store16_us(int rows, int cols, int I, int J, int slices, double steps) {
-  const double wgs = (double)(((I + rows - 1) / rows) * (long long)((J + cols - 1) / cols)) * slices;
-  auto rounds_of = [&](double per) { return (double)((long long)((wgs + per - 1) / per)); };
-  const double rounds = rounds_of(kComputeUnits), fill = wgs / (rounds * kComputeUnits);
-  const double launch = 2.8;
-  if (rows == 256 && cols == 256) return launch + rounds * (steps * 0.973 * (1.0 + 0.394 * fill) + 11.4);
-  if (rows == 256) return launch + rounds * (steps * 0.55 * (1.0 + 0.41 * fill) + 6.5);
-  if (rows == 128) {
-    const double one = steps * 0.474 + 4.5, two = steps * 1.079 + 3.8;   // a compute unit's one workgroup of eight wavefronts; two of four
-    if (wgs <= kComputeUnits * 3 / 2) return launch + rounds * one;
-    const double full = (double)((long long)(wgs / (2 * kComputeUnits))), rest = wgs - full * 2 * kComputeUnits;
-    return launch + full * two + (rest <= 0.0 ? 0.0 : rest > kComputeUnits ? two : one * 1.217);
-  }
-  return launch + (wgs <= kComputeUnits ? steps * 0.214 + 2.3 : rounds_of(2 * kComputeUnits) * (steps * 0.441 + 2.3));
-}
-
-// ... whose plan is the 128 tile: whether pairs of tiles, 256 x 128, are faster (the square tile reads a half more from LDS per
+// A 16-bit forward / input-grad whose plan is the 128 tile: whether pairs of tiles, 256 x 128, are faster (the square tile reads a half more from LDS per
 // multiplication, which is what bounds it; a pair leaves half the compute units idle where there are few tiles).  bf16: 2048 x 4096
 // over 1024 23.2 -> 20.1 us; 3001 x 1531 over 2047 49.7 -> 35.9; but 2048^3 22.8 -> 29.4 if it were taken there.
 static inline bool pair_form(int tile, int I, int J, int R, int chunk, int elem_bytes, const rz_tuning& t) {

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import SEED_CONSTANTS, assert_close, make_inputs, rargs
+from helpers import SEED_CONSTANTS, assert_close, make_inputs, rargs, stored_tiles_slack
 
 pytestmark = pytest.mark.gpu
 
@@ -291,3 +291,48 @@ def test_16_bit_cut_pairs_of_tiles(oracle, shape, slices):
             out.append(rz_linear_forward_bias_tl(x, hw, bias.cuda(), 0.75, M, K, N, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN))
     assert torch.equal(out[0], out[1])
     assert_close(out[0].float().cpu().numpy(), oracle.forward(x64, hw64, N, BK, BN, R1024, 0.75) + bias.double().numpy(), torch.bfloat16, "y")
+
+
+@pytest.mark.parametrize("shape,tile,slices", [
+    ((1056, 1280, 4144, 265216, 64, 64), 256, 2),     # added by atomics when cut no further than those allow
+    ((1948, 2184, 1810, 197652, 64, 64), 256, 2),     # odd row pitches, partial tiles and a partial last step
+    ((4846, 519, 1167, 41000, 64, 64), 128, 5),       # the fewest tiles
+    ((2322, 536, 3404, 91227, 64, 64), 128, 3),
+], ids=str)
+def test_16_bit_weight_grad_in_stored_slices(oracle, shape, tile, slices):
+    """Slices of M stored tile by tile are partial sums and kept in fp32: only dHW itself is rounded."""
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearBackward import weight_grad_hashed
+    M, K, N, H, BK, BN = shape
+    _say(shape)
+    (x, _, dy), (x64, _, dy64) = make_inputs(M, K, N, H, torch.bfloat16, seed=M)
+    R = _lib.hash_constants(*rargs(R1024))
+    ref = oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.5)
+    q = _lib.plan_query(2, M, K, N, H, BK, BN, _lib.RZ_BF16)
+    assert (q["mode"], q["tile"], q["slices"]) == ("fold", tile, slices)
+    for plans in (False, True):
+        dhw, dbias = weight_grad_hashed(x, dy, 0.5, M, K, N, H, R, BK, BN, with_bias_grad=True, use_layer_plan=plans)
+        assert_close(dhw.float().cpu().numpy(), ref, torch.bfloat16, "dHW")
+        assert_close(dbias.float().cpu().numpy(), dy64.sum(0), torch.bfloat16, "bias gradient")
+
+
+def test_static_scratch_takes_the_cut_that_fits(oracle):
+    """rz_weight_grad stores two or more slices for this problem, more than the static scratch holds; the static entry point
+    keeps the plan that it would hold, folded in a fixed order."""
+    import ctypes
+    from rzlinear_amd import _lib
+    lib = _lib.load()
+    M, K, N, H, BK, BN = 1878, 781, 4746, 185331, 64, 64
+    assert _lib.plan_query(2, M, K, N, H, BK, BN, _lib.RZ_BF16)["slices"] > 1
+    assert lib.rz_weight_grad_workspace_bytes(M, K, N, H, BK, BN, _lib.RZ_BF16) > 32 << 20
+    _say("static scratch, fewer slices", (M, K, N, H))
+    (x, _, dy), (x64, _, dy64) = make_inputs(M, K, N, H, torch.bfloat16, seed=72)
+    slack = stored_tiles_slack(oracle, x64, dy64, (M, K, N, H, BK, BN), R1024, 0.5, torch.bfloat16)
+    R = (ctypes.c_int32 * 8)(*R1024)
+    out = [torch.full((H,), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(3)]
+    for o in out:
+        _lib.check(lib.rz_weight_grad_static(x.data_ptr(), dy.data_ptr(), o.data_ptr(), M, K, N, H, BK, BN, R, 0.5, K, N,
+                                             _lib.RZ_BF16, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    assert_close(out[0].float().cpu().numpy(), oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.5), torch.bfloat16, "dHW", slack=slack)
