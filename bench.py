@@ -74,14 +74,14 @@ TRAFFIC = {
     #  FETCH_SIZE = 131085, WRITE_SIZE = 262144)
     ("square4096", "bf16"): {
         "profile": "profiles/rz_gemm_bf16_square4096.txt",
-        "bytes": {"forward": int((16691.8 * 2.0 + 32768.0) * 1024),       # algorithmic: 64.03 MiB
-                  "input_grad": int((16677.6 * 2.0 + 32768.0) * 1024),
-                  "weight_grad": int((98477.3 * 2.0 + 16780.4) * 1024)},  # X, dY re-read by the XCDs' tile groups; + partial images
+        "bytes": {"forward": int((16688.9 * 2.0 + 32768.0) * 1024),       # algorithmic: 64.03 MiB
+                  "input_grad": int((16683.4 * 2.0 + 32768.0) * 1024),
+                  "weight_grad": int((98466.4 * 2.0 + 16780.4) * 1024)},  # X, dY re-read by the XCDs' tile groups; + partial images
     },
     ("square2048", "bf16"): {
         "profile": "profiles/rz_gemm_bf16_square2048.txt",
-        "bytes": {"forward": int((4349.6 * 2.0 + 8192.0) * 1024), "input_grad": int((4331.5 * 2.0 + 8192.0) * 1024),
-                  "weight_grad": int((24695.7 * 2.0 + 16384.0) * 1024)},
+        "bytes": {"forward": int((4331.0 * 2.0 + 8192.0) * 1024), "input_grad": int((4328.4 * 2.0 + 8192.0) * 1024),
+                  "weight_grad": int((24672.7 * 2.0 + 16384.0) * 1024)},
     },
     ("square4096", "fp32"): {
         "profile": "profiles/rz_gemm_fp32_square4096.txt",
@@ -96,16 +96,16 @@ TRAFFIC = {
     },
     ("ffn", "bf16"): {
         "profile": "profiles/rz_gemm_fold_bf16_ffn.txt",
-        "bytes": {"forward": int((70672.0 * 2.0 + 262144.0) * 1024),      # algorithmic: 320.1 MiB
-                  "input_grad": int((132301.2 * 2.0 + 65536.0) * 1024),
+        "bytes": {"forward": int((69914.0 * 2.0 + 262144.0) * 1024),      # algorithmic: 320.1 MiB
+                  "input_grad": int((132289.8 * 2.0 + 65536.0) * 1024),
                   # contraction (X, dY re-read by the XCDs' tile groups; X^T.dY written tile by tile in bf16: 128 MiB)
-                  "weight_grad": int((786602.3 * 2.0 + 131072.0) * 1024)},
+                  "weight_grad": int((786585.8 * 2.0 + 131072.0) * 1024)},
     },
     ("grid_1024_10240", "bf16"): {
         "profile": "profiles/rz_gemm_fold_bf16_grid_1024_10240.txt",
-        "bytes": {"forward": int((396950.8 * 2.0 + 143380.0) * 1024),     # (three slices: fp32 partial planes written, read back by the slice that finishes)
-                  "input_grad": int((382347.7 * 2.0 + 143380.0) * 1024),
-                  "weight_grad": int((172202.6 * 2.0 + 204800.0) * 1024)},      # (X^T.dY tile by tile in bf16: 200 MiB)
+        "bytes": {"forward": int((398007.3 * 2.0 + 143380.0) * 1024),     # (three slices: fp32 partial planes written, read back by the slice that finishes)
+                  "input_grad": int((377290.8 * 2.0 + 143380.0) * 1024),
+                  "weight_grad": int((172182.1 * 2.0 + 204800.0) * 1024)},      # (X^T.dY tile by tile in bf16: 200 MiB)
     },
 }
 

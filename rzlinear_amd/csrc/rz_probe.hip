@@ -2,10 +2,11 @@
 // when nothing else is in the way.  The dense peak of the data sheet is clock x MFMA width at the
 // boost clock; under matrix load with real (non-constant) operands the clock is lower, and by how
 // much is a property of the board that only a measurement gives.  The kernel below has the shape of
-// the contraction kernels' inner loop — eight wavefronts per compute unit, 32 MFMA 32x32x16 per
+// the contraction kernels' inner loop (of the 32x32 blocks) — eight wavefronts per compute unit, 32 MFMA 32x32x16 per
 // wavefront and step on eight accumulator blocks — and nothing else: its operands come out of
 // registers (mode 0) or, like the real fragments, out of LDS with one barrier per step (mode 1).
 // It reads no global memory inside the loop and writes one float per thread at the end.
+// (The 16-bit 256-row tiles multiply the same products in blocks of 16x16x32, of which the board sustains about a tenth more.)
 #include "../../include/rzlinear.h"
 
 #include <hip/hip_runtime.h>
