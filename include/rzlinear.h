@@ -214,8 +214,8 @@ int rz_weight_grad(const void* X, const void* dY, void* dHW, void* workspace,
  * own copy until the process ends).  No counterpart in the reference; it is for callers that
  * cannot allocate: code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc.  Same arguments, results and status codes as rz_weight_grad otherwise.  A problem
- * for which rz_weight_grad would store X^T.dY tile by tile in more than 32 MiB takes the scatter
- * kernel with global atomics instead; a problem that needs more than 32 MiB even so is refused
+ * for which rz_weight_grad would store X^T.dY tile by tile in more than 32 MiB is cut into fewer slices of M where
+ * that fits, else takes the scatter kernel with global atomics; a problem that needs more than 32 MiB even so is refused
  * with RZ_ERR_SCRATCH_LIMIT (at M = N = K = 4096, H = 16778 the need is 17 MB).  The first call on a device looks the array's
  * address up (make that call outside a graph capture).  The array used is that of the CURRENT device, which must be
  * the device that holds dHW (and the other operands, and the stream): a call whose dHW lives on another device, or is
