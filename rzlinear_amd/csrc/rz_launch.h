@@ -308,13 +308,34 @@ static inline double stored_tiles_us(int tile, int M, int K, int N, int slices, 
   return weight_grad16_us(tile, M, K, N, slices) + (double)slices * K * N * tile_bytes * (1.0 / 4.7e6 + 0.3 / 5.0e6);
 }
 
+// A 16-bit weight-grad through LDS images, in microseconds, its reduction included: `wgs` workgroups of `steps` steps of 64.  A round
+// takes its steps (odd rows longer) and a fixed part of fill, image rounds (by hashed tiles of the C tile) and store; every workgroup
+// writes an image that is read once.  Two workgroups of the 128 tile share a compute unit where two images fit its LDS.  Fitted to
+// 752 shapes with either tile (M of 64 to 20000, K, N of 200 to 9000, H of 4200 to 36000, aligned and odd): 6 % rms.
+static inline double image16_us(int tile, long long wgs, long long steps, int pitch, int K, int N, int BK, int BN) {
+  const double bytes = (double)pitch * 4.0, hashed = (double)((tile + BK - 1) / BK) * ((tile + BN - 1) / BN);
+  const double rounds = (double)((wgs + kComputeUnits - 1) / kComputeUnits);
+  const bool odd = K % 8 != 0 || N % 8 != 0;
+  const double both = 8.58 + 0.78 * (double)wgs * bytes * 2.0 / 5e6;
+  if (tile == 256) {
+    const double fill = (double)wgs / (rounds * kComputeUnits);
+    return both + rounds * ((double)steps * 0.764 * (1.0 + 0.824 * fill) * (odd ? 1.036 : 1.0) + 7.17 + 0.236 * hashed);
+  }
+  const double n = (double)steps * (odd ? 1.197 : 1.0);
+  const double one = n * 0.461 + 2.77 + 0.252 * hashed, two = n * 0.896 + 3.17 + 0.087 * hashed;
+  if (wgs <= kComputeUnits * 3 / 2) return both + rounds * one;
+  if (bytes > 78 * 1024) return both + rounds * (n * 0.627 + 2.77 + 0.132 * hashed);
+  const long long full = wgs / (2 * kComputeUnits), rest = wgs - full * 2 * kComputeUnits;
+  return both + (double)full * two + (rest == 0 ? 0.0 : rest > kComputeUnits ? two : one * 1.08);
+}
+
 // A plan for the fold that was chosen as a whole (see plan_weight_grad).
 struct FoldChoice {
   int tile, slices, tile_bytes;
 };
 
 static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H, int BK, int BN, int elem_bytes,
-                                                      const rz_tuning& t, int tile_bytes, const FoldChoice* chosen = nullptr) {
+                                                      const rz_tuning& t, int tile_bytes, size_t limit, const FoldChoice* chosen = nullptr) {
   WeightGradPlan pl;
   const int pitch = (H + 3) & ~3;
   const bool image = t.lds_image != -1 && (size_t)pitch * sizeof(float) <= kMaxImageBytes;
@@ -371,6 +392,15 @@ static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H
         const double t128 = work_us * (st128 + 4.0) / st128 / (0.82 * filled(w128, kComputeUnits)) + (double)w128 * image_us;
         if (t128 < t256 * 0.97) pl.tile = 128;
       }
+      // ... and the other one where the fitted times, which know two 128 workgroups on a compute unit and what a hashed tile costs in the
+      // image rounds, promise more than the fit's error.  (bf16: M = 3200, K = 1536, N = 1152 35.4 -> 24.8 us with the 128
+      // tile, 96 x 9344 x 3712 77.6 -> 52.0; 110 drawn shapes whose
+      // tile changed 1.18 times as fast in the mean, the least 0.93)
+      const double us256 = image16_us(256, w256, ((M + 63) / 64 + s256 - 1) / s256, pitch, K, N, BK, BN);
+      const double us128 = image16_us(128, w128, 2 * (((M + 127) / 128 + s128 - 1) / s128), pitch, K, N, BK, BN);
+      const int by_rate = pl.tile, other = 384 - by_rate;
+      const size_t other_bytes = (size_t)(other == 128 ? w128 : w256) * pitch * sizeof(float);
+      if ((other == 128 ? us128 : us256) < 0.92 * (other == 128 ? us256 : us128) && other_bytes <= limit) pl.tile = other;
     }
   } else {
     pl.tile = pick_tile(K, N, elem_bytes, t);
@@ -487,10 +517,10 @@ static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H
 // fp32, whatever the layer's dtype, and so are they where that plan adds into an fp32 image.  (bf16, the module's
 // call: M = 20442, K = 6647, N = 591 477 -> 221 us; 14592, 8448, 448 232 -> 128; from the atomics 11552, 5632, 768 195 -> 121;
 // 200 drawn shapes whose plan changed 1.31 times as fast in the mean, the least 0.97.)
-// limit: bytes of scratch memory that the fold may take.
+// limit: bytes of scratch memory that images or the fold may take.
 static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK, int BN, int elem_bytes,
                                               const rz_tuning& t, int tile_bytes = 4, size_t limit = (size_t)-1) {
-  const WeightGradPlan by_rate = plan_weight_grad_by_rate(M, K, N, H, BK, BN, elem_bytes, t, tile_bytes);
+  const WeightGradPlan by_rate = plan_weight_grad_by_rate(M, K, N, H, BK, BN, elem_bytes, t, tile_bytes, limit);
   if (elem_bytes != 2 || by_rate.image_pitch > 0 || t.tile != 0 || t.fold == -1) return by_rate;
   FoldChoice best = {0, 0, 0};
   // (the plan by rate is left only for one that is faster by more than the fit's error; the 64 tile's times are not fitted for
@@ -513,7 +543,7 @@ static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK
     }
   }
   if (best.tile == 0 || (best.tile == by_rate.tile && best.slices == by_rate.splits)) return by_rate;
-  WeightGradPlan pl = plan_weight_grad_by_rate(M, K, N, H, BK, BN, elem_bytes, t, tile_bytes, &best);
+  WeightGradPlan pl = plan_weight_grad_by_rate(M, K, N, H, BK, BN, elem_bytes, t, tile_bytes, limit, &best);
   if (!pl.fold.use) return by_rate;
   // (the window kernel adds in fp32: 16-bit tiles take no call from it that the plan by rate leaves to it)
   if (by_rate.fold.use && best.tile_bytes == 2) pl.fold_us = by_rate.fold_us;

@@ -336,3 +336,22 @@ def test_static_scratch_takes_the_cut_that_fits(oracle):
     torch.cuda.synchronize()
     assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
     assert_close(out[0].float().cpu().numpy(), oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.5), torch.bfloat16, "dHW", slack=slack)
+
+
+@pytest.mark.parametrize("shape,slices", [
+    ((96, 449, 6200, 27389, 64, 64), 1),       # 196 workgroups, odd rows, partial tiles
+    ((933, 849, 463, 24001, 32, 64), 8),
+    ((96, 8768, 2496, 8233, 32, 64), 1),       # 1380 workgroups, two on a compute unit
+], ids=str)
+def test_16_bit_image_in_128_tiles(oracle, shape, slices):
+    """Images of the 128 tile where the fitted times prefer it to the 256 tile."""
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearBackward import weight_grad_hashed
+    M, K, N, H, BK, BN = shape
+    _say(shape)
+    (x, _, dy), (x64, _, dy64) = make_inputs(M, K, N, H, torch.bfloat16, seed=M)
+    q = _lib.plan_query(2, M, K, N, H, BK, BN, _lib.RZ_BF16)
+    assert (q["mode"], q["tile"], q["slices"]) == ("lds_image", 128, slices)
+    dhw, dbias = weight_grad_hashed(x, dy, 0.5, M, K, N, H, _lib.hash_constants(*rargs(R1024)), BK, BN, with_bias_grad=True)
+    assert_close(dhw.float().cpu().numpy(), oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.5), torch.bfloat16, "dHW")
+    assert_close(dbias.float().cpu().numpy(), dy64.sum(0), torch.bfloat16, "bias gradient")
