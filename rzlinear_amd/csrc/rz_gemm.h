@@ -1745,7 +1745,8 @@ struct GemmKernel {
       // reach L2 together.  A large C is stored with streaming stores: nothing here reads it
       // again, and kept in L2 it would push out the operand panels that the workgroups of the
       // next round still share (ffn input-grad, 64 MB of dX: 883 -> 861 us).
-      auto store_c = [&](auto streaming) {
+      // (whole: every block of the wavefront lies inside C)
+      auto store_c = [&](auto streaming, auto whole) {
 #pragma unroll
         for (int a = 0; a < MI; a++) {
 #pragma unroll
@@ -1754,7 +1755,7 @@ struct GemmKernel {
 #pragma unroll
             for (int b = 0; b < MJ; b++) {
               const int col = j0 + blk_j(b) + (lane & 31);
-              if (FULL || (row < p.I && col < p.J)) {
+              if (decltype(whole)::value || (row < p.I && col < p.J)) {
                 const T value = Tr::from_float(acc[a][b][e] * out_scale + bias[b]);
                 T* dst = gC + (int64_t)row * p.ldc + col;
                 if constexpr (!decltype(streaming)::value) *dst = value;
@@ -1765,8 +1766,23 @@ struct GemmKernel {
           }
         }
       };
-      if (p.stream_c) store_c(std::true_type{});
-      else store_c(std::false_type{});
+      // (the 16-bit 256-row tiles: a ragged C has few wavefronts at its edges, and a check per value costs all of them about 2 us a
+      //  tile: bf16 forward M = 16384, K = 264, N = 4096 81 -> 64 us, 8696 x 512 x 13568 179 -> 152)
+      bool inside = FULL;
+      if constexpr (!FULL && kBlk16) {
+        inside = true;
+#pragma unroll
+        for (int a = 0; a < MI; a++) inside = inside && i0 + blk_i(a) + 32 <= p.I;
+#pragma unroll
+        for (int b = 0; b < MJ; b++) inside = inside && j0 + blk_j(b) + 32 <= p.J;
+      }
+      if (FULL || (kBlk16 && inside)) {   // (uniform)
+        if (p.stream_c) store_c(std::true_type{}, std::true_type{});
+        else store_c(std::false_type{}, std::true_type{});
+      } else if constexpr (!FULL) {
+        if (p.stream_c) store_c(std::true_type{}, std::false_type{});
+        else store_c(std::false_type{}, std::false_type{});
+      }
     }
   }
 };
