@@ -339,6 +339,9 @@ static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H
   WeightGradPlan pl;
   const int pitch = (H + 3) & ~3;
   const bool image = t.lds_image != -1 && (size_t)pitch * sizeof(float) <= kMaxImageBytes;
+  // The tile that the comparison with the window kernel prices, where it is not the one that runs: the window kernel adds in
+  // fp32, so tiles that are stored in 16 bits are not to take a call from it because they have become cheaper.
+  int priced_tile = 0;
   if (chosen != nullptr) {
     pl.tile = chosen->tile;
     tile_bytes = chosen->tile_bytes;
@@ -414,7 +417,10 @@ static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H
     // N = 9000 140 -> 135; K = 8192, N = 4096, two rounds exactly, 65 either way; M = 512: 104 / 100 and 205 / 214 us)
     if (pl.tile == 256 && elem_bytes == 2 && t.fold != -1 && M <= 256 && tile_count(K, N, 256) > 2 * kComputeUnits) {
       const FoldPlan f = plan_fold(K, N, H, BK, BN, 1);
-      if (f.use && !f.small) pl.tile = 128;
+      if (f.use && !f.small) {
+        pl.tile = 128;
+        if (tile_bytes == 2) priced_tile = 256;
+      }
     }
     if (pl.tile == 256 && elem_bytes == 4 && t.fold != -1 && plan_fold(K, N, H, BK, BN, 1).use) {
       const long long t256 = tile_count(K, N, 256), t128 = tile_count(K, N, 128);
@@ -492,10 +498,12 @@ static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H
         // (for the comparison with the window kernel: every round of workgroups of the contraction
         //  kernel also pays its fill, drain and store — about 5 us for a round of 256 tiles, 10 us
         //  in fp32, in proportion to the tile's area — which matters when M is small)
-        const double round_us = (elem_bytes == 4 ? 10.0 : 5.0) * (double)pl.tile * pl.tile / 65536.0;
+        const int priced = priced_tile ? priced_tile : pl.tile;
+        const long long priced_wgs = priced_tile ? tile_count(K, N, priced_tile) * pl.splits : pl.workgroups;
+        const double round_us = (elem_bytes == 4 ? 10.0 : 5.0) * (double)priced * priced / 65536.0;
         // (a contraction shorter than the stores of its tiles takes the time of the stores — fp32, K = N = 10240,
         //  H = 2^20, M = 32: 220 us in all)
-        const double contraction_us = product_us + round_us * (double)((pl.workgroups + kComputeUnits - 1) / kComputeUnits);
+        const double contraction_us = product_us + round_us * (double)((priced_wgs + kComputeUnits - 1) / kComputeUnits);
         pl.fold_us = (contraction_us > store_us ? contraction_us : store_us) + fold_us - (store_us > product_us ? store_us - product_us : 0.0);
       }
     }

@@ -54,3 +54,15 @@ def test_no_baseline_configuration_takes_the_atomic_scatter():
     elements) and for many small tiles under a batch of a few rows, where they are faster."""
     assert all(mode != "atomics" for _, plan in PLANS.values() for _, _, mode in plan)
     assert _lib.plan_query(2, 128, 2048, 1024, 1 << 20, 256, 128, BF16)["mode"] == "atomics"
+
+
+@pytest.mark.parametrize("shape", [
+    (96, 11712, 13760, 1611571, 32, 64), (93, 4672, 9344, 1309655, 32, 64), (127, 10560, 3904, 1236787, 32, 64),
+    (158, 3520, 10368, 1094860, 32, 64), (61, 8192, 4608, 1282982, 32, 64), (91, 9088, 3648, 1170819, 64, 64),
+    (72, 3648, 10048, 1249083, 64, 64),
+], ids=str)
+@pytest.mark.parametrize("code", [BF16, F16])
+def test_a_short_batch_keeps_the_window_kernels_fp32_sums(shape, code):
+    """The 128 tile that a short batch takes makes its fold cheaper; tiles stored in 16 bits must not win a call from the window
+    kernel, which adds in fp32, by that.  (Each of these lies where the two tiles' prices fall on either side of the window kernel's.)"""
+    assert _lib.plan_query(2, *shape, code, planned=True)["mode"] == "window"
