@@ -1015,7 +1015,7 @@ struct GemmKernel {
       const T* b_ptr = uniform_ptr(OP == kWeightGrad ? gB + (int64_t)r_begin * p.ldb + j0 : gHW);
       const int64_t a_step = A_LAYOUT == kRContig ? TR : TR * p.lda, b_step = OP == kWeightGrad ? TR * p.ldb : 0;
       auto load_lds = [&](const T* base, uint32_t voff, uint32_t dma, int at) {
-        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dma), "v"(voff), "s"(base), "n"(at) : "memory", "scc");
+        asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(dma), "v"(voff), "s"(base), "n"(at) : "memory", "m0", "scc");
       };
       // the tile offsets of step `step`'s pieces of W, added to what is fixed of their addresses
       uint32_t tab_at[OP != kWeightGrad ? LB::kPieces : 1], hw_off[OP != kWeightGrad ? LB::kPieces : 1];
