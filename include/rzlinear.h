@@ -324,10 +324,12 @@ int rz_weight_grad_planned(const void* X, const void* dY, void* dHW, void* dbias
  * (modes 4 and 5, else 0) } with mode 0 = plain store, 1 = split contraction with
  * fp32 partial planes, 2 = weight-grad through LDS images of dHW, 3 = weight-grad by global
  * atomics, 4 = weight-grad by windows of dHW, 5 = weight-grad stored tile by tile and folded
- * into dHW by a second kernel.  For tests of the planning logic and for tuning; no counterpart in the
- * reference.
+ * into dHW by a second kernel.  RZ_PLAN_TILE_BYTES in flags: out[6] of a mode 5 answer is instead how many
+ * bytes a stored element of X^T.dY takes: 4 (fp32), or 2 (the layer's dtype: one more rounding).  For tests of
+ * the planning logic and for tuning; no counterpart in the reference.
  */
 #define RZ_PLAN_WITH_LAYER_PLAN 0x100u
+#define RZ_PLAN_TILE_BYTES 0x200u
 int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int dtype, unsigned flags,
                   int with_dbias, const rz_tuning* tuning, int32_t out[8]);
 

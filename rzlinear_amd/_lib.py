@@ -320,14 +320,15 @@ def layer_plan(K, N, H, BK, BN, R, hash_levels, device):
 PLAN_MODES = {0: "store", 1: "split", 2: "lds_image", 3: "atomics", 4: "window", 5: "fold"}
 
 
-PLAN_WITH_LAYER_PLAN = 0x100
+PLAN_WITH_LAYER_PLAN, PLAN_TILE_BYTES = 0x100, 0x200
 
 
 def plan_query(op, M, K, N, H, BK, BN, dtype_code_, flags=0, with_dbias=False, planned=False):
     """How the library would carry out a call (rz_plan_query), under the current tuning:
     dict(tile, slices, slice_len, step, mode, workgroups, shares, windows).  op: 0 forward, 1 input-grad,
     2 weight-grad; planned: the call will carry a layer plan (rz_weight_grad_planned).  For mode "split",
-    shares = 1 says that the kernel finishes its own tiles (no second kernel)."""
+    shares = 1 says that the kernel finishes its own tiles (no second kernel).  flags=PLAN_TILE_BYTES: for mode
+    "fold", shares is how many bytes a stored element of X^T.dY takes."""
     t = _tuning
     if planned:
         flags |= PLAN_WITH_LAYER_PLAN

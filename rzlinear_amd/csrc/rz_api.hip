@@ -1011,7 +1011,7 @@ RZ_API int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int
     out[4] = plan.fold.use ? 5 : plan.image_pitch > 0 ? 2 : 3;
     out[5] = (int32_t)plan.workgroups;
     if (plan.fold.use) {
-      out[6] = plan.fold.shares;
+      out[6] = (flags & RZ_PLAN_TILE_BYTES) != 0 ? plan.fold.tile_bytes : plan.fold.shares;
       out[7] = plan.fold.windows;
     }
     return RZ_OK;

@@ -49,30 +49,41 @@ def elementwise_excess(out, ref, dtype, floor=1e-5, slack=None):
     return float((np.abs(out - ref) / bound).max()) if out.size else 0.0
 
 
+def stored_tile_bytes(shape, code, planned, flags=0):
+    """Bytes of a stored element of X^T.dY where the weight gradient of this problem is folded, else None."""
+    from rzlinear_amd import _lib
+    q = _lib.plan_query(2, *shape, code, flags=flags | _lib.PLAN_TILE_BYTES, planned=planned)
+    return q["shares"] if q["mode"] == "fold" else None
+
+
 def stored_tiles_slack(oracle, x64, dy64, shape, R, scale, dtype, hash_levels=None):
     """What the element-wise bound of a 16-bit dHW gains when the weight gradient goes through the fold with
     the tiles of X^T.dY stored in the layer's dtype (rz_tuning.fold_tiles = 0): every stored value — one per
     element of X^T.dY and slice of M, complete fp32 sums — is rounded once (ROUNDING[dtype] of its magnitude
     at most) before the fold adds the values of a slot up in fp32.  Returns the allowance per element of dHW, or None
-    where no plan of this problem takes that path (fp32 layers; LDS image, window kernel, atomics)."""
+    where no plan of this problem takes that path (fp32 layers; LDS image, window kernel, atomics; tiles that are
+    stored in fp32 for a 16-bit layer too)."""
     from rzlinear_amd import _lib
     if dtype == torch.float32:
         return None
     M, K, N, H, BK, BN = shape
     code = _lib.RZ_BF16 if dtype == torch.bfloat16 else _lib.RZ_F16
     plans = [_lib.plan_query(2, M, K, N, H, BK, BN, code, planned=p) for p in (False, True)]
-    folds = [p for p in plans if p["mode"] == "fold"]
+    folds = [p for p, planned in zip(plans, (False, True)) if stored_tile_bytes(shape, code, planned) == 2]
     if not folds:
         return None
+    return np.maximum.reduce([rounded_tiles_slack(oracle, x64, dy64, shape, R, scale, dtype, p["slice_len"] if p["slices"] > 1 else M, hash_levels)
+                              for p in folds])
+
+
+def rounded_tiles_slack(oracle, x64, dy64, shape, R, scale, dtype, step, hash_levels=None):
+    """That allowance for a call that is known to store its tiles in the layer's dtype, one for every slice of `step` rows of M."""
+    M, K, N, H, BK, BN = shape
     idx = oracle.index_map(K, N, H, BK, BN, R) if hash_levels is None else oracle.index_map(K, N, H, BK, BN, R, hash_levels)
-    slack = np.zeros((H,), dtype=np.float64)
-    for p in folds:
-        step = p["slice_len"] if p["slices"] > 1 else M
-        stored = sum(np.abs(x64[m:m + step].T @ dy64[m:m + step]) for m in range(0, M, step)) * abs(scale)
-        s = np.zeros((H,), dtype=np.float64)
-        np.add.at(s, idx.reshape(-1), stored.reshape(-1))
-        slack = np.maximum(slack, s)
-    return ROUNDING[dtype] * slack
+    stored = sum(np.abs(x64[m:m + step].T @ dy64[m:m + step]) for m in range(0, M, step)) * abs(scale)
+    s = np.zeros((H,), dtype=np.float64)
+    np.add.at(s, idx.reshape(-1), stored.reshape(-1))
+    return ROUNDING[dtype] * s
 
 
 def assert_close(out, ref, dtype, what="", slack=None):

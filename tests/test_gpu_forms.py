@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import SEED_CONSTANTS, assert_close, make_inputs, rargs, stored_tiles_slack
+from helpers import SEED_CONSTANTS, assert_close, make_inputs, rargs, rounded_tiles_slack, stored_tile_bytes
 
 pytestmark = pytest.mark.gpu
 
@@ -310,6 +310,7 @@ def test_16_bit_weight_grad_in_stored_slices(oracle, shape, tile, slices):
     ref = oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.5)
     q = _lib.plan_query(2, M, K, N, H, BK, BN, _lib.RZ_BF16)
     assert (q["mode"], q["tile"], q["slices"]) == ("fold", tile, slices)
+    assert all(stored_tile_bytes(shape, _lib.RZ_BF16, planned) == 4 for planned in (False, True))
     for plans in (False, True):
         dhw, dbias = weight_grad_hashed(x, dy, 0.5, M, K, N, H, R, BK, BN, with_bias_grad=True, use_layer_plan=plans)
         assert_close(dhw.float().cpu().numpy(), ref, torch.bfloat16, "dHW")
@@ -327,7 +328,8 @@ def test_static_scratch_takes_the_cut_that_fits(oracle):
     assert lib.rz_weight_grad_workspace_bytes(M, K, N, H, BK, BN, _lib.RZ_BF16) > 32 << 20
     _say("static scratch, fewer slices", (M, K, N, H))
     (x, _, dy), (x64, _, dy64) = make_inputs(M, K, N, H, torch.bfloat16, seed=72)
-    slack = stored_tiles_slack(oracle, x64, dy64, (M, K, N, H, BK, BN), R1024, 0.5, torch.bfloat16)
+    # (its tiles are whole sums over M, rounded once to bf16; the slices of the other entry points are kept in fp32)
+    slack = rounded_tiles_slack(oracle, x64, dy64, (M, K, N, H, BK, BN), R1024, 0.5, torch.bfloat16, M)
     R = (ctypes.c_int32 * 8)(*R1024)
     out = [torch.full((H,), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(3)]
     for o in out:

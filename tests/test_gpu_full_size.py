@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import SEED_CONSTANTS, TOL, ULP, rargs, ROUNDING
+from helpers import SEED_CONSTANTS, TOL, ULP, rargs, ROUNDING, stored_tile_bytes
 
 pytestmark = pytest.mark.gpu
 
@@ -104,7 +104,8 @@ def test_baseline_configuration_at_full_size(oracle, name):
     if dtype != torch.float32:
         from rzlinear_amd import _lib
         code = _lib.RZ_BF16 if dtype == torch.bfloat16 else _lib.RZ_F16
-        folds = [q for q in (_lib.plan_query(2, M, K, N, H, BK, BN, code, planned=p) for p in (False, True)) if q["mode"] == "fold"]
+        folds = [_lib.plan_query(2, M, K, N, H, BK, BN, code, planned=p) for p in (False, True)
+                 if stored_tile_bytes((M, K, N, H, BK, BN), code, p) == 2]
         for q in folds:
             step = q["slice_len"] if q["slices"] > 1 else M
             stored = sum((x[m:m + step].double().t() @ dy[m:m + step].double()).abs() for m in range(0, M, step))

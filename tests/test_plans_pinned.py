@@ -7,6 +7,8 @@ import pytest
 
 from rzlinear_amd import _lib
 
+from helpers import stored_tile_bytes
+
 F32, BF16, F16 = _lib.RZ_F32, _lib.RZ_BF16, _lib.RZ_F16
 
 # name: ((M, K, N, H, BLOCK_K, BLOCK_N, dtype), [(tile, slices, mode) for forward, input-grad, weight-grad])
@@ -54,6 +56,24 @@ def test_no_baseline_configuration_takes_the_atomic_scatter():
     elements) and for many small tiles under a batch of a few rows, where they are faster."""
     assert all(mode != "atomics" for _, plan in PLANS.values() for _, _, mode in plan)
     assert _lib.plan_query(2, 128, 2048, 1024, 1 << 20, 256, 128, BF16)["mode"] == "atomics"
+
+
+@pytest.mark.parametrize("shape,code,bytes_of_each", [
+    ((8192, 4096, 16384, 67109, 64, 64), BF16, 2), ((1024, 10240, 10240, 6553600, 32, 64), F16, 2),
+    ((1024, 10240, 10240, 6553600, 32, 64), F32, 4), ((1024, 1024, 1024, 65536, 64, 64), F32, 4),
+    ((96, 10240, 10240, 67109, 64, 64), BF16, 2),        # the 128 tile of a short batch, one slice
+    ((20442, 6647, 591, 245486, 64, 64), BF16, 4),       # cut further than the plan by rate
+    ((14592, 8448, 448, 236544, 64, 64), F16, 4),
+    ((11552, 5632, 768, 270336, 64, 64), BF16, 4),       # added into an fp32 image by that plan
+    ((4846, 519, 1167, 41000, 64, 64), BF16, 4), ((2322, 536, 3404, 91227, 64, 64), BF16, 4),
+    ((1056, 1280, 4144, 265216, 64, 64), BF16, 4), ((1948, 2184, 1810, 197652, 64, 64), F16, 4),
+], ids=str)
+def test_width_of_the_stored_tiles(shape, code, bytes_of_each):
+    """Tiles of a 16-bit layer are stored in its dtype where a stored value is a sum over M cut no further than by the plan by
+    rate, and in fp32 where it is a partial sum of a further cut or would otherwise be added in fp32."""
+    for planned in (False, True):
+        assert stored_tile_bytes(shape, code, planned) == bytes_of_each
+        assert stored_tile_bytes(shape, code, planned, _lib.WG_DHW_F32) == 4   # (an fp32 dHW never has them rounded)
 
 
 @pytest.mark.parametrize("shape", [
