@@ -674,16 +674,23 @@ struct GemmKernel {
       }
     };
     // LDS addresses as 32-bit numbers, worked out once and kept in scalar registers (opaque: otherwise the compiler
-    // converts the generic pointers again for every load, a dozen scalar instructions each)
+    // converts the generic pointers again for every load, a dozen scalar instructions each).  Not in the fp32 256 tile's forward,
+    // whose long MFMAs hide those instructions and whose loop comes out in a worse order without them (4096^3 937 against
+    // 944 us, 32768 x 2048 x 2048 1890 against 1902; its input-grad and weight-grad are the same either way).
+    constexpr bool kLdsWords = kDirect && !(kDirect32 && TI == 256 && OP == kForward);
     typedef const T __attribute__((address_space(3)))* lds_ptr;
     uint32_t lds_a = 0, lds_b = 0;
-    if constexpr (kDirect) {
+    if constexpr (kLdsWords) {
       lds_a = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)sm.a[0]);
       lds_b = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lds_ptr)sm.b[0]);
       asm volatile("" : "+s"(lds_a), "+s"(lds_b));
     }
-    auto stage_a = [&](int st) -> uint32_t { return lds_a + (uint32_t)st * (uint32_t)(LA::kElems * sizeof(T)); };
-    auto stage_b = [&](int st) -> uint32_t { return lds_b + (uint32_t)st * (uint32_t)(LB::kElems * sizeof(T)); };
+    auto stage_a = [&](int st) -> uint32_t {
+      return kLdsWords ? lds_a + (uint32_t)st * (uint32_t)(LA::kElems * sizeof(T)) : (uint32_t)(uintptr_t)(lds_ptr)sm.a[st];
+    };
+    auto stage_b = [&](int st) -> uint32_t {
+      return kLdsWords ? lds_b + (uint32_t)st * (uint32_t)(LB::kElems * sizeof(T)) : (uint32_t)(uintptr_t)(lds_ptr)sm.b[st];
+    };
     auto direct_load = [&](const T* src, uint32_t stage, int n) {
       // the LDS address goes through M0 and must be the same for the whole wavefront
       const uint32_t dst = __builtin_amdgcn_readfirstlane(stage + (uint32_t)(n * 1024));
