@@ -218,7 +218,7 @@ def test_bias_gradient_behind_the_windows(oracle, shape, dtype):
 
 
 @pytest.mark.parametrize("dtype", SIXTEEN, ids=str)
-@pytest.mark.parametrize("extents", [(256, 384), (250, 391)], ids=str)
+@pytest.mark.parametrize("extents", [(256, 512), (256, 384), (250, 391)], ids=str)   # (both tiles complete; the 128 tile; neither)
 @pytest.mark.parametrize("steps,rest", [(1, 0), (2, 0), (3, 0), (4, 0), (5, 0), (6, 0), (9, 0), (36, 0),
                                         (0, 17), (1, 1), (2, 31), (3, 32), (4, 63), (5, 33), (17, 8)], ids=str)
 @pytest.mark.parametrize("tile", [128, 256])
@@ -272,6 +272,91 @@ def test_16_bit_pairs_of_tiles(oracle, extents, r, dtype):
         dx = rz_linear_backward_input_grad_tl(x, hw, 0.75, a, b, r, H, *rargs(R1024), BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
     assert_close(y.float().cpu().numpy(), oracle.forward(x64, hw64, b, BK, BN, R1024, 0.75) + bias.double().numpy(), dtype, "y")
     assert_close(dx.float().cpu().numpy(), oracle.input_grad(x64, hw64, b, BK, BN, R1024, 0.75), dtype, "dx")
+
+
+def _odd_pitch(t, before):
+    """A view with the values of t inside rows of odd pitch, at an odd start, with infinities and NaN all around it."""
+    cols = t.shape[1]
+    big = torch.full((t.shape[0], before + cols + 2 + (before + cols + 1) % 2), float("inf"), dtype=t.dtype, device=t.device)
+    big[:, ::2] = float("nan")
+    view = big[:, before:before + cols]
+    view.copy_(t)
+    assert view.stride(0) % 2 == 1 and view.data_ptr() % 16 != 0
+    return view
+
+
+@pytest.mark.parametrize("dtype", SIXTEEN, ids=str)
+@pytest.mark.parametrize("extents", [(256, 512), (250, 391)], ids=str)
+@pytest.mark.parametrize("r", [17, 64, 191, 256, 300, 1088], ids=str)
+@pytest.mark.parametrize("tile", [128, 256])
+def test_16_bit_pipelined_tiles_in_odd_pitches(oracle, tile, r, extents, dtype):
+    """Operands that are part of wider rows: what lies behind a row's last element (infinities and NaN) is fetched with it and
+    must be cleared in LDS, in both halves of the 256 tile's rows; all three operations, dHW through images and stored tiles."""
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearBackward import rz_linear_backward_input_grad_tl, weight_grad_hashed
+    from rzlinear_amd.impl.RzLinearForward import rz_linear_forward_tl
+    (a, b), H, BK, BN = extents, 20000, 32, 64
+    _say(tile, r, extents, dtype)
+    R = _lib.hash_constants(*rargs(R1024))
+    kw = dict(BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
+    with _lib.tuning(tile=tile, split=-1):
+        (x, hw, _), (x64, hw64, _) = make_inputs(a, r, b, H, dtype, seed=r)
+        y = rz_linear_forward_tl(_odd_pitch(x, 1), hw, 0.75, a, r, b, H, *rargs(R1024), **kw)
+        assert_close(y.float().cpu().numpy(), oracle.forward(x64, hw64, b, BK, BN, R1024, 0.75), dtype, "y")
+        (_, hw, dy), (_, hw64, dy64) = make_inputs(a, b, r, H, dtype, seed=r)
+        dx = rz_linear_backward_input_grad_tl(_odd_pitch(dy, 3), hw, 0.75, a, b, r, H, *rargs(R1024), **kw)
+        assert_close(dx.float().cpu().numpy(), oracle.input_grad(dy64, hw64, b, BK, BN, R1024, 0.75), dtype, "dx")
+    (x, _, dy), (x64, _, dy64) = make_inputs(r, a, b, H, dtype, seed=r)
+    ref = oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.5)
+    for how in ({"window": -1}, {"lds_image": -1, "window": -1, "fold": 2}):
+        out = torch.empty((H,), dtype=torch.float32, device="cuda")
+        with _lib.tuning(tile=tile, **how):
+            _, dbias = weight_grad_hashed(_odd_pitch(x, 3), _odd_pitch(dy, 1), 0.5, r, a, b, H, R, BK, BN, out=out, with_bias_grad=True)
+        # (fp32 sums of exact products: at most r of them per stored value and a few dozen values per slot)
+        assert np.abs(out.cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()
+        assert_close(dbias.float().cpu().numpy(), dy64.sum(0), dtype, "bias gradient")
+
+
+@pytest.mark.parametrize("dtype", SIXTEEN, ids=str)
+@pytest.mark.parametrize("extents", [(2048, 2304), (2030, 2299)], ids=str)
+@pytest.mark.parametrize("r", [65, 192, 300], ids=str)
+def test_16_bit_pairs_of_tiles_in_odd_pitches(oracle, extents, r, dtype):
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearBackward import rz_linear_backward_input_grad_tl
+    from rzlinear_amd.impl.RzLinearForward import rz_linear_forward_tl
+    (a, b), H, BK, BN = extents, 20000, 32, 64
+    _say(r, extents, dtype)
+    (x, hw, _), (x64, hw64, _) = make_inputs(a, r, b, H, dtype, seed=r)
+    wide, kw = _odd_pitch(x, 1), dict(BLOCK_SIZE_K=BK, BLOCK_SIZE_N=BN)
+    with _lib.tuning(split=-1):
+        for op, K, N in ((0, r, b), (1, b, r)):
+            q = _lib.plan_query(op, a, K, N, H, BK, BN, _lib.dtype_code(x))
+            assert (q["tile"], q["slices"], q["workgroups"], q["step"]) == (128, 1, 144, 64)
+        y = rz_linear_forward_tl(wide, hw, 0.75, a, r, b, H, *rargs(R1024), **kw)
+        dx = rz_linear_backward_input_grad_tl(wide, hw, 0.75, a, b, r, H, *rargs(R1024), **kw)
+    assert_close(y.float().cpu().numpy(), oracle.forward(x64, hw64, b, BK, BN, R1024, 0.75), dtype, "y")
+    assert_close(dx.float().cpu().numpy(), oracle.input_grad(x64, hw64, b, BK, BN, R1024, 0.75), dtype, "dx")
+
+
+@pytest.mark.parametrize("shape,mode,tile", [
+    ((96, 449, 6200, 27389, 64, 64), "lds_image", 128),        # images of the 128 tile, K odd
+    ((2000, 2043, 2051, 20000, 32, 64), "lds_image", 256),     # slices, a partial last one
+    ((1948, 2184, 1810, 197652, 64, 64), "fold", 256),         # stored slices in fp32
+    ((2322, 536, 3404, 91227, 64, 64), "fold", 128),
+], ids=str)
+def test_16_bit_weight_grad_plans_in_odd_pitches(oracle, shape, mode, tile):
+    """The plans that sizes pick by themselves, on operands inside wider rows."""
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearBackward import weight_grad_hashed
+    M, K, N, H, BK, BN = shape
+    _say(shape)
+    q = _lib.plan_query(2, M, K, N, H, BK, BN, _lib.RZ_BF16)
+    assert (q["mode"], q["tile"]) == (mode, tile), q
+    (x, _, dy), (x64, _, dy64) = make_inputs(M, K, N, H, torch.bfloat16, seed=M)
+    dhw, dbias = weight_grad_hashed(_odd_pitch(x, 1), _odd_pitch(dy, 3), 0.5, M, K, N, H, _lib.hash_constants(*rargs(R1024)), BK, BN,
+                                    with_bias_grad=True)
+    assert_close(dhw.float().cpu().numpy(), oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.5), torch.bfloat16, "dHW")
+    assert_close(dbias.float().cpu().numpy(), dy64.sum(0), torch.bfloat16, "bias gradient")
 
 
 @pytest.mark.parametrize("shape,slices", [((200, 6000, 6000, 20000, 32, 64), 5), ((896, 3968, 2368, 20000, 64, 64), 3), ((900, 4001, 2371, 20000, 32, 64), 3)], ids=str)
