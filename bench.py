@@ -309,10 +309,10 @@ def api_level(torch, wl, warmup, steps):
 
 def mfma_ceiling(torch, _lib, wl, launches=100):
     """The MFMA rate this GPU sustains on the matrix work alone of one contraction of the headline
-    shape, with operands distributed like the workload's: rz_mfma_probe runs the inner loop's
-    MFMA stream (256 workgroups of eight wavefronts, 32 MFMA 32x32x16 per wavefront and step, as
-    many steps as make 2*M*N*K flop) without global loads, hashing or stores — mode 0 out of
-    registers, mode 1 with the fragment reads from LDS and the barrier per step.  The gap between
+    shape, with operands distributed like the workload's: rz_mfma_probe runs streams of MFMA (256 workgroups
+    of eight wavefronts, as many steps as make 2*M*N*K flop) without global loads, hashing or stores — of 16x16x32
+    out of registers, the instruction of the 16-bit 256-row tiles and so what their rate is compared with, and of 32x32x16,
+    which the smaller tiles use, out of registers and with fragment reads from LDS and a barrier per step.  The gap between
     these figures and the data sheet's peak is the clock under matrix load (reported), not the
     kernels'.  16-bit types only."""
     if wl["dname"] == "fp32":
@@ -325,9 +325,9 @@ def mfma_ceiling(torch, _lib, wl, launches=100):
     steps = max(1, int(round(wl["flop_gemm"] / (wgs * 8 * 32 * 32768.0))))
     out = torch.empty((wgs * 512,), dtype=torch.float32, device=dev)
     ticks = torch.zeros((2 * wgs,), dtype=torch.int64, device=dev)
-    res = {"what": "rz_mfma_probe: %d workgroups x 8 wavefronts x %d steps x 32 MFMA 32x32x16 (%.1f GFLOP per launch), operands = "
+    res = {"what": "rz_mfma_probe: %d workgroups x 8 wavefronts x %d steps x 64 MFMA 16x16x32 or 32 of 32x32x16 (%.1f GFLOP per launch), operands = "
                    "the workload's X; %d launches after as many untimed" % (wgs, steps, wgs * 8 * steps * 32 * 32768 / 1e9, launches)}
-    for mode, key in ((0, "registers_only"), (1, "with_lds_fragments_and_barrier")):
+    for mode, key in ((2, "blocks_16x16x32"), (0, "registers_only"), (1, "with_lds_fragments_and_barrier")):
         def launch():
             _lib.check(lib.rz_mfma_probe(operands.data_ptr(), out.data_ptr(), ticks.data_ptr(), wgs, steps, mode, wl["code"], stream))
         for _ in range(launches):
@@ -497,7 +497,7 @@ def main():
     ceiling = None if args.no_ceiling else mfma_ceiling(torch, _lib, wl)
     if ceiling is not None:
         roofline["practical_ceiling"] = ceiling
-        roofline["frac_of_practical_ceiling"] = round(leg_tflops[slowest] / ceiling["registers_only"]["tflops"], 4)
+        roofline["frac_of_practical_ceiling"] = round(leg_tflops[slowest] / ceiling["blocks_16x16x32"]["tflops"], 4)
 
     cpu_baseline = None
     if not args.no_cpu_baseline:

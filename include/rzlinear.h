@@ -372,10 +372,11 @@ int rz_adam_step(void* param, const void* grad, float* exp_avg, float* exp_avg_s
 /*
  * Measurement aid, no counterpart in the reference: the MFMA rate this GPU sustains on the
  * matrix work of the contraction kernels' inner loop when nothing else is in the way.  Launches
- * `workgroups` workgroups of eight wavefronts (one per compute unit fits); every wavefront issues
- * steps * 32 MFMA 32x32x16 on eight accumulator blocks, i.e. a launch is
- * workgroups * 8 * steps * 32 * 32768 flop.  mode 0: operands stay in registers; mode 1: fragments
- * come out of LDS (six 1 KB reads per eight MFMA, one barrier per step), as in the real loop.
+ * `workgroups` workgroups of eight wavefronts (one per compute unit fits); a launch is
+ * workgroups * 8 * steps * 32 * 32768 flop.  Modes 0 and 1: every wavefront issues steps * 32 MFMA 32x32x16
+ * on eight accumulator blocks, with operands that stay in registers (0) or fragments that
+ * come out of LDS (1: six 1 KB reads per eight MFMA, one barrier per step).  Mode 2: steps * 64 MFMA 16x16x32 on
+ * 32 accumulator blocks, the instruction of the 16-bit 256-row tiles, operands in registers.
  * operands: 64 KB of 16-bit values of `dtype` (RZ_BF16 or RZ_F16) in device memory — the clock
  * under matrix load depends on how much the operand bits toggle, so pass values like the real
  * data's.  out: workgroups * 512 floats (written, meaningless).  ticks: 2 * workgroups uint64:

@@ -1,12 +1,13 @@
 // Measurement aid: what this GPU sustains on the MFMA work of one 256 x 256 C tile per compute unit
 // when nothing else is in the way.  The dense peak of the data sheet is clock x MFMA width at the
 // boost clock; under matrix load with real (non-constant) operands the clock is lower, and by how
-// much is a property of the board that only a measurement gives.  The kernel below has the shape of
-// the contraction kernels' inner loop (of the 32x32 blocks) — eight wavefronts per compute unit, 32 MFMA 32x32x16 per
-// wavefront and step on eight accumulator blocks — and nothing else: its operands come out of
-// registers (mode 0) or, like the real fragments, out of LDS with one barrier per step (mode 1).
-// It reads no global memory inside the loop and writes one float per thread at the end.
-// (The 16-bit 256-row tiles multiply the same products in blocks of 16x16x32, of which the board sustains about a tenth more.)
+// much is a property of the board that only a measurement gives.  The kernels below have the shape of
+// the contraction kernels' inner loops — eight wavefronts per compute unit, each of which multiplies 128 x 64 by 64
+// elements per step — and nothing else.  Blocks of 32 x 32, 32 MFMA 32x32x16 per step: operands out of
+// registers (mode 0) or, like the real fragments, out of LDS with one barrier per step (mode 1).  Blocks of 16 x 16, 64
+// MFMA 16x16x32 per step, as the 16-bit 256-row tiles multiply: operands out of registers (mode 2); the board
+// sustains about a tenth more of them.
+// They read no global memory inside the loop and write one float per thread at the end.
 #include "../../include/rzlinear.h"
 
 #include <hip/hip_runtime.h>
@@ -17,11 +18,17 @@ namespace rz {
 
 template <typename T> struct ProbeMfma;
 template <> struct ProbeMfma<bf16_t> {
+  static __device__ __forceinline__ f32x4_t run16(u32x4_t a, u32x4_t b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  }
   static __device__ __forceinline__ f32x16_t run(u32x4_t a, u32x4_t b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
   }
 };
 template <> struct ProbeMfma<f16_t> {
+  static __device__ __forceinline__ f32x4_t run16(u32x4_t a, u32x4_t b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+  }
   static __device__ __forceinline__ f32x16_t run(u32x4_t a, u32x4_t b, f32x16_t c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
   }
@@ -84,13 +91,52 @@ __global__ __launch_bounds__(kProbeThreads) void mfma_probe_kernel(const uint32_
   }
 }
 
+// ... and blocks of 16 x 16: a step is two sub-steps of 8 x 4 MFMA, whose twelve fragments stay in registers
+template <typename T>
+__global__ __launch_bounds__(kProbeThreads) void mfma16_probe_kernel(const uint32_t* __restrict__ operands, float* __restrict__ out,
+                                                                   unsigned long long* __restrict__ ticks, int steps) {
+  const int lane = threadIdx.x & 63;
+  f32x4_t acc[8][4];
+#pragma unroll
+  for (int a = 0; a < 8; a++)
+#pragma unroll
+    for (int b = 0; b < 4; b++) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  u32x4_t fa[8], fb[4];
+#pragma unroll
+  for (int i = 0; i < 8; i++) fa[i] = *reinterpret_cast<const u32x4_t*>(operands + (i * 64 + lane) * 4);
+#pragma unroll
+  for (int i = 0; i < 4; i++) fb[i] = *reinterpret_cast<const u32x4_t*>(operands + ((8 + i) * 64 + lane) * 4);
+  const unsigned long long c0 = __builtin_readcyclecounter(), r0 = __builtin_amdgcn_s_memrealtime();
+  for (int s = 0; s < steps; s++) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+      for (int a = 0; a < 8; a++)
+#pragma unroll
+        for (int b = 0; b < 4; b++) acc[a][b] = ProbeMfma<T>::run16(fa[a], fb[b], acc[a][b]);
+  }
+  const unsigned long long c1 = __builtin_readcyclecounter(), r1 = __builtin_amdgcn_s_memrealtime();
+  float sum = 0.f;
+#pragma unroll
+  for (int a = 0; a < 8; a++)
+#pragma unroll
+    for (int b = 0; b < 4; b++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) sum += acc[a][b][e];
+  out[blockIdx.x * kProbeThreads + threadIdx.x] = sum;
+  if (threadIdx.x == 0) {
+    ticks[2 * blockIdx.x] = c1 - c0;
+    ticks[2 * blockIdx.x + 1] = r1 - r0;
+  }
+}
+
 }  // namespace rz
 
 extern "C" __attribute__((visibility("default"))) int rz_mfma_probe(const void* operands, void* out, void* ticks, int workgroups,
                                                                     int steps, int mode, int dtype, void* stream) {
   using namespace rz;
   if (operands == nullptr || out == nullptr || ticks == nullptr) return RZ_ERR_NULL_POINTER;
-  if (workgroups < 1 || workgroups > 65536 || steps < 1 || (mode != 0 && mode != 1)) return RZ_ERR_BAD_ARGUMENT;
+  if (workgroups < 1 || workgroups > 65536 || steps < 1 || mode < 0 || mode > 2) return RZ_ERR_BAD_ARGUMENT;
   if (dtype != RZ_BF16 && dtype != RZ_F16) return RZ_ERR_BAD_DTYPE;
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid((unsigned)workgroups), block(kProbeThreads);
@@ -98,7 +144,9 @@ extern "C" __attribute__((visibility("default"))) int rz_mfma_probe(const void* 
   float* o = static_cast<float*>(out);
   unsigned long long* t = static_cast<unsigned long long*>(ticks);
   const size_t lds = mode == 1 ? kProbeLdsBytes : 0;
-  if (dtype == RZ_BF16 && mode == 0) hipLaunchKernelGGL((mfma_probe_kernel<bf16_t, 0>), grid, block, lds, s, src, o, t, steps);
+  if (dtype == RZ_BF16 && mode == 2) hipLaunchKernelGGL((mfma16_probe_kernel<bf16_t>), grid, block, 0, s, src, o, t, steps);
+  else if (mode == 2) hipLaunchKernelGGL((mfma16_probe_kernel<f16_t>), grid, block, 0, s, src, o, t, steps);
+  else if (dtype == RZ_BF16 && mode == 0) hipLaunchKernelGGL((mfma_probe_kernel<bf16_t, 0>), grid, block, lds, s, src, o, t, steps);
   else if (dtype == RZ_BF16) hipLaunchKernelGGL((mfma_probe_kernel<bf16_t, 1>), grid, block, lds, s, src, o, t, steps);
   else if (mode == 0) hipLaunchKernelGGL((mfma_probe_kernel<f16_t, 0>), grid, block, lds, s, src, o, t, steps);
   else hipLaunchKernelGGL((mfma_probe_kernel<f16_t, 1>), grid, block, lds, s, src, o, t, steps);

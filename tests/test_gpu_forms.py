@@ -442,3 +442,18 @@ def test_16_bit_image_in_128_tiles(oracle, shape, slices):
     dhw, dbias = weight_grad_hashed(x, dy, 0.5, M, K, N, H, _lib.hash_constants(*rargs(R1024)), BK, BN, with_bias_grad=True)
     assert_close(dhw.float().cpu().numpy(), oracle.weight_grad(x64, dy64, H, BK, BN, R1024, 0.5), torch.bfloat16, "dHW")
     assert_close(dbias.float().cpu().numpy(), dy64.sum(0), torch.bfloat16, "bias gradient")
+
+
+@pytest.mark.parametrize("dtype", SIXTEEN, ids=str)
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_mfma_probe_multiplies_what_it_says(mode, dtype):
+    """Every mode does the same work: with operands of one, a thread adds up 128 accumulators of 64 products per step."""
+    from rzlinear_amd import _lib
+    wgs, steps = 3, 5
+    operands = torch.ones((32768,), dtype=dtype, device="cuda")
+    out = torch.zeros((wgs * 512,), dtype=torch.float32, device="cuda")
+    ticks = torch.zeros((2 * wgs,), dtype=torch.int64, device="cuda")
+    _lib.check(_lib.load().rz_mfma_probe(operands.data_ptr(), out.data_ptr(), ticks.data_ptr(), wgs, steps, mode,
+                                         _lib.dtype_code(operands), torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(out.cpu(), torch.full((wgs * 512,), 128.0 * 64 * steps))   # (whole numbers: exact in fp32)
+    assert bool((ticks[::2] > 0).all())
