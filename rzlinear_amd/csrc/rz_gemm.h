@@ -965,7 +965,8 @@ struct GemmKernel {
       //    reads only the next one's two fragments of A, so that nothing is spilled (a whole sub-step read ahead is);
       //  - the order is held by sched_barrier: left alone the compiler moves the reads down to where they are used;
       //  - addresses are 32-bit LDS addresses and running pointers, no arithmetic is left to do per load or fragment;
-      //  - one load per phase, not eight behind a barrier (that kept all wavefronts from multiplying while they waited
+      //  - one load per phase (the first phase in which there is room for any, and two of the four of the 256 x 128 tile, issue
+      //    two), not eight behind a barrier (that kept all wavefronts from multiplying while they waited
       //    to issue them): A's first half of rows and B are free for the step after next from phase 3 on, A's second half
       //    from phase 7 on, and each part is waited for only where it is first read.
       // 4096^3 bf16, forward / input-grad / weight-grad: 112.8 / 112.5 / 123.1 -> 100.4 / 98.7 / 111.5 us; M = 8192, K = 4096, N = 16384:

@@ -380,8 +380,9 @@ static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H
       // 16-bit: the two tiles by estimated time.  Fitted on MI355X (weight-grad, 256 workgroups):
       // a 256 workgroup pays about 5.5 steps of 64 rows for its fill, its image rounds and the
       // store of its image, whatever the length of its loop; the 128 tile in its eight-wavefront
-      // form (steps of 128 rows, up to 384 workgroups) runs at 0.82 of the 256 tile's rate and
-      // pays about 4 of its steps.  Both write one image per workgroup.  (2048^3: 32.4 -> 30.5 us;
+      // form (up to 384 workgroups) runs at 0.82 of the 256 tile's rate and pays about 4 times 128
+      // rows.  Both write one image per workgroup.  These are the rates of earlier loops of both tiles: the rule
+      // decides where the fitted times below see no clear difference.  (2048^3: 32.4 -> 30.5 us;
       // M = 8192, K = N = 2048 stays with the 256 tile: 72.8 against 82.1 us.)
       const long long tiles128 = tile_count(K, N, 128);
       const long long s256 = image_slices(tiles256, (M + 63) / 64), s128 = image_slices(tiles128, (M + 127) / 128);
@@ -407,11 +408,6 @@ static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H
     }
   } else {
     pl.tile = pick_tile(K, N, elem_bytes, t);
-    // fp32 with the tiles stored for the fold kernel: by how the two tiles fill their rounds when
-    // there are at least as many 256 tiles as compute units (K = N = 10240: M = 128 455 -> 401 us,
-    // M = 1024 1938 -> 1797 us, M = 4096 7002 -> 6449 us; K = N = 4096, one round exactly, stays
-    // with the 256 tile: 1043 against 1085 us); with fewer, a short M takes the 128 tile, whose
-    // paired workgroups hide each other's stores
     // 16-bit with a short M: a workgroup of the 256 tile is then mostly fill and store, which two workgroups of the 128 tile
     // on a compute unit hide behind each other — from two rounds of 256 tiles on (M = 64: K = N = 6000 78 -> 73 us, K = 12000,
     // N = 9000 140 -> 135; K = 8192, N = 4096, two rounds exactly, 65 either way; M = 512: 104 / 100 and 205 / 214 us)
@@ -422,6 +418,11 @@ static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H
         if (tile_bytes == 2) priced_tile = 256;
       }
     }
+    // fp32 with the tiles stored for the fold kernel: by how the two tiles fill their rounds when
+    // there are at least as many 256 tiles as compute units (K = N = 10240: M = 128 455 -> 401 us,
+    // M = 1024 1938 -> 1797 us, M = 4096 7002 -> 6449 us; K = N = 4096, one round exactly, stays
+    // with the 256 tile: 1043 against 1085 us); with fewer, a short M takes the 128 tile, whose
+    // paired workgroups hide each other's stores
     if (pl.tile == 256 && elem_bytes == 4 && t.fold != -1 && plan_fold(K, N, H, BK, BN, 1).use) {
       const long long t256 = tile_count(K, N, 256), t128 = tile_count(K, N, 128);
       if (t256 >= kComputeUnits ? kPairRate128F32 * filled_128(t128) > filled_256(t256) * 1.01 : M <= 2048) pl.tile = 128;
