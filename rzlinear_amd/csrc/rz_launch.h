@@ -525,7 +525,7 @@ static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H
 // tiles).  A slice's stored tiles are partial sums: where there are more of them than in the plan by rate they are stored in
 // fp32, whatever the layer's dtype, and so are they where that plan adds into an fp32 image.  (bf16, the module's
 // call: M = 20442, K = 6647, N = 591 477 -> 221 us; 14592, 8448, 448 232 -> 128; from the atomics 11552, 5632, 768 195 -> 121;
-// 200 drawn shapes whose plan changed 1.31 times as fast in the mean, the least 0.97.)
+// 368 drawn shapes whose plan changed 1.23 times as fast in the mean, the least 0.985.)
 // limit: bytes of scratch memory that images or the fold may take.
 static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK, int BN, int elem_bytes,
                                               const rz_tuning& t, int tile_bytes = 4, size_t limit = (size_t)-1) {
@@ -534,6 +534,11 @@ static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK
   FoldChoice best = {0, 0, 0};
   // (the plan by rate is left only for one that is faster by more than the fit's error; the 64 tile's times are not fitted for
   //  this; the atomics: the part of K*N per slice that the contraction does not hide)
+  // (in place of atomics the fold is a kernel more, 8 us of launch and of looking for tiles that the fitted times leave out, as
+  //  they are the same for every fold.  438 drawn calls of 4 to 32768 rows whose plan by rate adds by atomics: 256 of them leave it, 1.22 times as
+  //  fast in the mean, the least 0.985; without the 8 us 343 left it, 40 of them slower, down to 0.88 — M = 1085, K = 4416,
+  //  N = 1024, H = 282624 46 -> 50 us)
+  const double fold_kernel_us = by_rate.fold.use ? 0.0 : 8.0;
   double best_us = -1.0 + 0.90 * (by_rate.fold.use ? stored_tiles_us(by_rate.tile, M, K, N, by_rate.splits, tile_bytes)
                                                    : weight_grad16_us(by_rate.tile, M, K, N, by_rate.splits) + (double)by_rate.splits * K * N * 2.8e-6);
   const int tiles_of[2] = {256, 128};
@@ -544,7 +549,7 @@ static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK
       const int bytes = by_rate.fold.use && w <= by_rate.splits ? tile_bytes : 4;
       const FoldPlan f = plan_fold(K, N, H, BK, BN, w, t.fold == 2, bytes);
       if ((steps + per - 1) / per != w || !f.use || f.tiles_bytes + f.partial_bytes + f.offsets_bytes > limit) continue;
-      const double us = stored_tiles_us(tile, M, K, N, w, bytes);
+      const double us = stored_tiles_us(tile, M, K, N, w, bytes) + fold_kernel_us;
       if (us < best_us * (best.tile == 0 ? 1.0 : 0.97)) {
         best_us = us;
         best = {tile, w, bytes};

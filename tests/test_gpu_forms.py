@@ -379,7 +379,7 @@ def test_16_bit_cut_pairs_of_tiles(oracle, shape, slices):
 
 
 @pytest.mark.parametrize("shape,tile,slices", [
-    ((1056, 1280, 4144, 265216, 64, 64), 256, 2),     # added by atomics when cut no further than those allow
+    ((1963, 1344, 3328, 279552, 64, 64), 256, 2),     # added by atomics when cut no further than those allow
     ((1948, 2184, 1810, 197652, 64, 64), 256, 2),     # odd row pitches, partial tiles and a partial last step
     ((4846, 519, 1167, 41000, 64, 64), 128, 5),       # the fewest tiles
     ((2322, 536, 3404, 91227, 64, 64), 128, 3),
