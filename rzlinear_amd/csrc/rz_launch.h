@@ -534,13 +534,14 @@ static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK
   FoldChoice best = {0, 0, 0};
   // (the plan by rate is left only for one that is faster by more than the fit's error; the 64 tile's times are not fitted for
   //  this; the atomics: the part of K*N per slice that the contraction does not hide)
-  // (in place of atomics the fold is a kernel more, 8 us of launch and of looking for tiles that the fitted times leave out, as
-  //  they are the same for every fold.  438 drawn calls of 4 to 32768 rows whose plan by rate adds by atomics: 256 of them leave it, 1.22 times as
-  //  fast in the mean, the least 0.985; without the 8 us 343 left it, 40 of them slower, down to 0.88 — M = 1085, K = 4416,
-  //  N = 1024, H = 282624 46 -> 50 us)
-  const double fold_kernel_us = by_rate.fold.use ? 0.0 : 8.0;
-  double best_us = -1.0 + 0.90 * (by_rate.fold.use ? stored_tiles_us(by_rate.tile, M, K, N, by_rate.splits, tile_bytes)
-                                                   : weight_grad16_us(by_rate.tile, M, K, N, by_rate.splits) + (double)by_rate.splits * K * N * 2.8e-6);
+  // (in place of atomics the fold is a kernel more, 12 us of launch and of looking for tiles that the fitted times leave out, as
+  //  they are the same for every fold; with them both prices are within a few per cent of what is measured.  Of 438 drawn
+  //  calls of 4 to 32768 rows whose plan by rate adds by atomics 288 leave it, 1.20 times as fast in the mean, the least 0.96; without
+  //  the 12 us 343 left it, 40 of them slower, down to 0.88 — M = 1085, K = 4416, N = 1024, H = 282624 46 -> 50 us)
+  const double by_rate_us = by_rate.fold.use ? stored_tiles_us(by_rate.tile, M, K, N, by_rate.splits, tile_bytes)
+                                             : weight_grad16_us(by_rate.tile, M, K, N, by_rate.splits) + (double)by_rate.splits * K * N * 2.8e-6;
+  double best_us = 0.90 * by_rate_us - 1.0;
+  if (!by_rate.fold.use && by_rate_us - 12.0 < best_us) best_us = by_rate_us - 12.0;
   const int tiles_of[2] = {256, 128};
   for (int tile : tiles_of) {
     const int unit = slice_unit(tile, elem_bytes, true), steps = (M + unit - 1) / unit;
@@ -549,7 +550,7 @@ static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK
       const int bytes = by_rate.fold.use && w <= by_rate.splits ? tile_bytes : 4;
       const FoldPlan f = plan_fold(K, N, H, BK, BN, w, t.fold == 2, bytes);
       if ((steps + per - 1) / per != w || !f.use || f.tiles_bytes + f.partial_bytes + f.offsets_bytes > limit) continue;
-      const double us = stored_tiles_us(tile, M, K, N, w, bytes) + fold_kernel_us;
+      const double us = stored_tiles_us(tile, M, K, N, w, bytes);
       if (us < best_us * (best.tile == 0 ? 1.0 : 0.97)) {
         best_us = us;
         best = {tile, w, bytes};
