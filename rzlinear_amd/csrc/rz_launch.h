@@ -397,11 +397,15 @@ static inline WeightGradPlan plan_weight_grad_by_rate(int M, int K, int N, int H
         if (t128 < t256 * 0.97) pl.tile = 128;
       }
       // ... and the other one where the fitted times, which know two 128 workgroups on a compute unit and what a hashed tile costs in the
-      // image rounds, promise more than the fit's error.  (bf16: M = 3200, K = 1536, N = 1152 35.4 -> 24.8 us with the 128
-      // tile, 96 x 9344 x 3712 77.6 -> 52.0; 110 drawn shapes whose
-      // tile changed 1.18 times as fast in the mean, the least 0.93)
+      // image rounds, promise more than the fit's usual error.  (bf16: M = 3200, K = 1536, N = 1152 35.4 -> 24.8 us with the 128
+      // tile, 96 x 9344 x 3712 77.6 -> 52.0)  They were fitted from 64 rows on: with fewer a call is little but its images, and
+      // what those of the 128 tile have more costs 0.22 us a MB from 8 MB on (M = 36, K = 1863, N = 1524, H = 33541: 24 MB of images
+      // instead of 6 25.5 against 24.2 us).  Of 4000 drawn shapes of 4 to 32768 rows with a tile of either size 666 change theirs, 1.29 times as
+      // fast in the mean; six are more than 2 % slower, the least 0.89 (M = 21162, K = 1152, N = 448).
       const double us256 = image16_us(256, w256, ((M + 63) / 64 + s256 - 1) / s256, pitch, K, N, BK, BN);
-      const double us128 = image16_us(128, w128, 2 * (((M + 127) / 128 + s128 - 1) / s128), pitch, K, N, BK, BN);
+      double us128 = image16_us(128, w128, 2 * (((M + 127) / 128 + s128 - 1) / s128), pitch, K, N, BK, BN);
+      const double more_mb = (double)(w128 - w256) * pitch * sizeof(float) * 1e-6;
+      if (M <= 64 && w128 <= 2 * kComputeUnits && more_mb > 8.0) us128 += 0.22 * (more_mb - 8.0);
       const int by_rate = pl.tile, other = 384 - by_rate;
       const size_t other_bytes = (size_t)(other == 128 ? w128 : w256) * pitch * sizeof(float);
       if ((other == 128 ? us128 : us256) < 0.92 * (other == 128 ? us256 : us128) && other_bytes <= limit) pl.tile = other;

@@ -96,3 +96,15 @@ def test_a_short_batch_keeps_the_window_kernels_fp32_sums(shape, code):
 def test_slices_are_stored_in_place_of_atomics_only_where_that_pays_for_the_fold_kernel(shape, mode):
     """Measured (bf16): the first five are 3 to 12 % slower with stored slices, the others 3 to 60 % faster."""
     assert _lib.plan_query(2, *shape, BF16, planned=True)["mode"] == mode
+
+
+@pytest.mark.parametrize("shape,tile", [
+    ((36, 1863, 1524, 33541, 32, 64), 256), ((50, 704, 8704, 17299, 32, 64), 256), ((14, 2816, 1216, 33208, 32, 64), 256),
+    ((23, 497, 8162, 29777, 32, 64), 256), ((11, 5952, 512, 29736, 64, 64), 256),
+    ((19, 5120, 704, 8192, 32, 64), 128), ((18, 1368, 1112, 33794, 64, 64), 128), ((41, 8960, 704, 8192, 32, 64), 128),
+    ((96, 8768, 2496, 8233, 32, 64), 128),
+], ids=str)
+def test_a_batch_below_the_fit_pays_for_the_images_of_the_128_tile(shape, tile):
+    """Measured (bf16): the first five are 5 to 9 % slower with the 128 tile, the next three 12 to 60 % faster."""
+    q = _lib.plan_query(2, *shape, BF16, planned=True)
+    assert (q["mode"], q["tile"]) == ("lds_image", tile)
