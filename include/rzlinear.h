@@ -176,9 +176,10 @@ int rz_input_grad_ws(const void* dY, const void* HW, void* dX, void* workspace,
  * When hashed_weight is small enough for an fp32 image of dHW to fit the LDS of a compute
  * unit, every workgroup stores one partial image ([workgroups][H rounded up to 4] floats) that
  * a second kernel adds up.  Otherwise one of three: with many W tiles per element of dHW the
- * contraction stores X^T.dY tile by tile (4 * ceil(K/BK)*BK * ceil(N/BN)*BN bytes per slice of M)
+ * contraction stores X^T.dY tile by tile (4 * ceil(K/BK)*BK * ceil(N/BN)*BN bytes per slice of M, up to eight slices)
  * and a second kernel folds the tiles into dHW (plus a few images of dHW and one int32 offset
- * per W tile); with M small against K*N, dHW is computed in windows and the workspace holds
+ * per W tile) — 16-bit: wherever that is the faster, though it can take several times the bytes of X and
+ * dY where atomic adds would need 4 * H (rz_tuning.fold = -1 forgoes it); with M small against K*N, dHW is computed in windows and the workspace holds
  * only the offsets; with few tiles the 16-bit types need an fp32 image of dHW (H floats) for
  * atomic adds and fp32 needs nothing.  The size depends on M: ask again when the batch size
  * changes.

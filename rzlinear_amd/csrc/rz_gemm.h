@@ -969,7 +969,7 @@ struct GemmKernel {
       //    two), not eight behind a barrier (that kept all wavefronts from multiplying while they waited
       //    to issue them): A's first half of rows and B are free for the step after next from phase 3 on, A's second half
       //    from phase 7 on, and each part is waited for only where it is first read.
-      // 4096^3 bf16, forward / input-grad / weight-grad: 112.8 / 112.5 / 123.1 -> 100.4 / 98.7 / 111.5 us; M = 8192, K = 4096, N = 16384:
+      // 4096^3 bf16, forward / input-grad / weight-grad, one operation at a time, with the reduction: 112.8 / 112.5 / 123.1 -> 100.4 / 98.7 / 111.5 us; M = 8192, K = 4096, N = 16384:
       // 877 / 877 / 904 -> 774 / 743 / 811 us (1.42 / 1.48 / 1.36 PFLOP/s).  Same bits as the loop with blocks of 32 x 32.
       // Not faster: four wavefronts of 128 x 128 (126 us weight-grad), wave priorities, a deeper pipeline alone.
       constexpr int FI = MI * 2, FJ = MJ * 2, NS = TR / 32;   // blocks of the wavefront, sub-steps

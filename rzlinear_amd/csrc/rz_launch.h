@@ -540,7 +540,7 @@ static inline WeightGradPlan plan_weight_grad(int M, int K, int N, int H, int BK
   //  this; the atomics: the part of K*N per slice that the contraction does not hide)
   // (in place of atomics the fold is a kernel more, 12 us of launch and of looking for tiles that the fitted times leave out, as
   //  they are the same for every fold; with them both prices are within a few per cent of what is measured.  Of 438 drawn
-  //  calls of 4 to 32768 rows whose plan by rate adds by atomics 288 leave it, 1.20 times as fast in the mean, the least 0.96; without
+  //  calls of 4 to 32768 rows whose plan by rate adds by atomics 289 leave it, 1.20 times as fast in the mean, the least 0.96; without
   //  the 12 us 343 left it, 40 of them slower, down to 0.88 — M = 1085, K = 4416, N = 1024, H = 282624 46 -> 50 us)
   const double by_rate_us = by_rate.fold.use ? stored_tiles_us(by_rate.tile, M, K, N, by_rate.splits, tile_bytes)
                                              : weight_grad16_us(by_rate.tile, M, K, N, by_rate.splits) + (double)by_rate.splits * K * N * 2.8e-6;
