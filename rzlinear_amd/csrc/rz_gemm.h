@@ -172,8 +172,10 @@ __device__ __forceinline__ u32x4_t shift_down_16(u32x4_t v, int sh) {
 // the g-th part of every R step and the groups' accumulators are added through LDS at the end.
 // For a tile with one wavefront per SIMD (fp32, 64 x 64) this puts a second wavefront on every
 // SIMD, which fills the MFMA pipe while the first waits for its fragments.
+// SHORT (16-bit 256 tile): the loop of the other tiles, with blocks of 32 x 32, for a few R steps: the phase loop is the faster
+// per step but costs about 1 us more before and after it, ragged 2 to 3 us (see short_loop).  Same bits.
 template <typename T, int OP, int TI, int TJ, int WI, int WJ, int NSTAGE, bool FULL, bool COLSUM = false,
-          bool CLAMP = false, int WK = 1>
+          bool CLAMP = false, int WK = 1, bool SHORT = false>
 struct GemmKernel {
   static_assert(WK == 1 || NSTAGE >= 2, "the R step is shared out only by the pipelined kernels");
   static_assert(!(FULL && CLAMP), "complete tiles need no clamping");
@@ -228,7 +230,7 @@ struct GemmKernel {
   // (see `step` under kBlk16); the other kernels blocks of 32 x 32.  Under a long matrix load the board lowers its clock
   // to keep to its power: a stream of 16x16x32 alone ran at 2063 TFLOP/s here, one of 32x32x16 at 1840.
   static constexpr bool kPair = k16 && NSTAGE == 3 && TI == 256 && TJ == 128 && WI == 4 && WJ == 2;   // two 128 tiles
-  static constexpr bool kBlk16 = kDirect16 && (kPair || (TI == 256 && TJ == 256 && WI == 2 && WJ == 4 && NSTAGE == 2));
+  static constexpr bool kBlk16 = kDirect16 && !SHORT && (kPair || (TI == 256 && TJ == 256 && WI == 2 && WJ == 4 && NSTAGE == 2));
   static constexpr int KS = kDirect32 ? 8 : kBlk16 ? 32 : Tr::kMfmaK;
   typedef typename std::conditional<kDirect32, f32x4_t, typename Mfma<T>::Frag>::type Frag;
   static __device__ __forceinline__ f32x16_t mma(Frag a, Frag b, f32x16_t c) {
@@ -1777,14 +1779,15 @@ struct GemmKernel {
       // (the 16-bit 256-row tiles: a ragged C has few wavefronts at its edges, and a check per value costs all of them about 2 us a
       //  tile: bf16 forward M = 16384, K = 264, N = 4096 81 -> 64 us, 8696 x 512 x 13568 179 -> 152)
       bool inside = FULL;
-      if constexpr (!FULL && kBlk16) {
+      constexpr bool kEdges = !FULL && CLAMP && k16 && TI == 256;
+      if constexpr (kEdges) {
         inside = true;
 #pragma unroll
         for (int a = 0; a < MI; a++) inside = inside && i0 + blk_i(a) + 32 <= p.I;
 #pragma unroll
         for (int b = 0; b < MJ; b++) inside = inside && j0 + blk_j(b) + 32 <= p.J;
       }
-      if (FULL || (kBlk16 && inside)) {   // (uniform)
+      if (FULL || (kEdges && inside)) {   // (uniform)
         if (p.stream_c) store_c(std::true_type{}, std::true_type{});
         else store_c(std::false_type{}, std::true_type{});
       } else if constexpr (!FULL) {
@@ -1799,9 +1802,9 @@ struct GemmKernel {
 // workgroups' for the sixteen-wavefront form with two stages, which shares its compute unit.
 constexpr int gemm_waves_per_simd(int waves, int stages) { return waves == 16 && stages == 2 ? 8 : (waves + 3) / 4; }
 
-template <typename T, int OP, int TI, int TJ, int WI, int WJ, int NSTAGE, bool FULL, bool COLSUM, bool CLAMP, int WK = 1>
+template <typename T, int OP, int TI, int TJ, int WI, int WJ, int NSTAGE, bool FULL, bool COLSUM, bool CLAMP, int WK = 1, bool SHORT = false>
 __global__ __launch_bounds__(64 * WI * WJ * WK, gemm_waves_per_simd(WI * WJ * WK, NSTAGE)) void rz_gemm_kernel(GemmParams p) {
-  typedef GemmKernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK> K;
+  typedef GemmKernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK, SHORT> K;
   extern __shared__ __attribute__((aligned(16))) unsigned char rz_smem_raw[];
   K::run(p, *reinterpret_cast<typename K::Smem*>(rz_smem_raw));
 }

@@ -10,11 +10,11 @@
 namespace rz {
 
 template <typename T, int OP, int TI, int TJ, int WI, int WJ, int NSTAGE, bool FULL, bool COLSUM, bool CLAMP = false,
-          int WK = 1>
+          int WK = 1, bool SHORT = false>
 static hipError_t launch_one(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
                              hipStream_t stream) {
   static std::atomic<uint64_t> lds_limit_raised{0};
-  typedef GemmKernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK> K;
+  typedef GemmKernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK, SHORT> K;
   p.tiles_i = (p.I + TI - 1) / TI;
   p.tiles_j = (p.J + TJ - 1) / TJ;
   const long long tiles = (long long)p.tiles_i * p.tiles_j;
@@ -52,7 +52,7 @@ static hipError_t launch_one(GemmParams p, const WeightGradPlan* plan, const Spl
     p.partial = nullptr;
     p.finish = nullptr;
   }
-  auto kernel = rz_gemm_kernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK>;
+  auto kernel = rz_gemm_kernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK, SHORT>;
   size_t smem = sizeof(typename K::Smem);
   static_assert(sizeof(typename K::Smem) <= 160 * 1024, "tile does not fit the 160 KB LDS of a compute unit");
   if (OP == kWeightGrad && p.image_pitch > 0) {
@@ -88,6 +88,13 @@ static hipError_t launch_tile(GemmParams p, const WeightGradPlan* plan, const Sp
     return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, false, WK>(p, plan, split, stream);
   }
   // (the 16-bit 64 tile of four wavefronts, and the 128 tile of eight with two stages, serve rows shorter than a 16-byte piece only)
+  // (16-bit 256 tile, a few R steps)
+  if constexpr (sizeof(T) == 2 && TILE == 256 && TILE_J == 256) if (form.short_loop) {
+    if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true, false, false, WK, true>::TR) return hipErrorInvalidValue;
+    if (form.full) return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true, COLSUM, false, WK, true>(p, plan, split, stream);
+    if (form.clamp) return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, true, WK, true>(p, plan, split, stream);
+    return hipErrorInvalidValue;
+  }
   constexpr bool kCheckedOnly = sizeof(T) == 2 && WK == 1 && (TILE == 64 || (TILE == 128 && WI * WJ == 8 && NSTAGE == 2));
   if constexpr (!kCheckedOnly) if (form.full) {
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true>::TR) return hipErrorInvalidValue;
@@ -125,7 +132,7 @@ static hipError_t launch_op(GemmParams p, const WeightGradPlan* plan, const Spli
 }
 
 // Tile shapes (all two LDS stages, software pipelined unless noted):
-//   256: 256 x 256, eight wavefronts of 128 x 64, one workgroup per compute unit
+//   256: 256 x 256, eight wavefronts of 128 x 64, one workgroup per compute unit (16-bit: a loop of its own, except for a few R steps)
 //   128: 128 x 128, four wavefronts of 64 x 64 (up to two workgroups per compute unit) or
 //        eight of 64 x 32 when there is about one workgroup per compute unit (16-bit: four LDS stages); tuning.stages = 1
 //        selects a single-stage form that leans on several workgroups per compute unit

@@ -854,8 +854,18 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
 struct KernelForm {
   int tile, rows, cols, waves, stages;   // tile: the planner's code; rows x cols: the C tile of the kernel that serves it
   bool full, clamp;
+  bool short_loop;   // 16-bit 256 tile: the loop for a few R steps
   int step;
 };
+
+// 16-bit 256 tile: whether `steps` R steps of 64 are too few for the phase loop.  It gains 3 to 5 % per step but takes 1.1 us more around
+// its steps (of which the exchange of accumulators is 0.3), with ragged tiles 2 to 3, than the loop of the other tiles.  bf16, us (other
+// loop / phase loop), K = N or M = N = 4096 if not said: forward of 1 / 5 / 6 / 8 steps 11.3 / 12.5, 16.2 / 16.5, 17.8 / 17.8, 20.5 / 20.2; ragged,
+// 4090 x 4000, 1 / 6 / 12 / 16 steps 14.4 / 17.2, 21.6 / 23.0, 32.0 / 31.9, 39.3 / 38.4, 2030 x 4090 (half the chip) 14.0 / 17.4, 21.4 / 23.9, 29.6 / 30.8,
+// 35.1 / 35.6; weight-grad 1 / 3 / 4 steps 23.4 / 23.7, 26.2 / 26.4, 27.5 / 27.4; ragged 1 / 8 / 10 steps 25.2 / 26.7, 32.8 / 33.3, 35.0 / 35.2.
+static inline bool short_loop(int op, bool full, int steps) {
+  return steps <= (op == kWeightGrad ? (full ? 3 : 8) : (full ? 5 : 10));
+}
 
 static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int tile, long long workgroups,
                                      int elem_bytes, const rz_tuning& t) {
@@ -917,6 +927,7 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
     f.full = I % 256 == 0 && J % 128 == 0 && R % 64 == 0 && chunk % 64 == 0;
     f.clamp = !f.full;
   }
+  f.short_loop = elem_bytes == 2 && tile == 256 && (f.full || f.clamp) && short_loop(op, f.full, ((chunk < R ? chunk : R) + 63) / 64);
   return f;
 }
 

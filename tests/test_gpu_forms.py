@@ -219,13 +219,14 @@ def test_bias_gradient_behind_the_windows(oracle, shape, dtype):
 
 @pytest.mark.parametrize("dtype", SIXTEEN, ids=str)
 @pytest.mark.parametrize("extents", [(256, 512), (256, 384), (250, 391)], ids=str)   # (both tiles complete; the 128 tile; neither)
-@pytest.mark.parametrize("steps,rest", [(1, 0), (2, 0), (3, 0), (4, 0), (5, 0), (6, 0), (9, 0), (36, 0),
-                                        (0, 17), (1, 1), (2, 31), (3, 32), (4, 63), (5, 33), (17, 8)], ids=str)
+@pytest.mark.parametrize("steps,rest", [(1, 0), (2, 0), (3, 0), (4, 0), (5, 0), (6, 0), (7, 0), (9, 0), (36, 0),
+                                        (0, 17), (1, 1), (2, 31), (3, 32), (4, 63), (5, 33), (7, 33), (8, 33), (9, 63),
+                                        (10, 1), (11, 40), (12, 17), (17, 8)], ids=str)
 @pytest.mark.parametrize("tile", [128, 256])
 def test_16_bit_pipelined_tiles_at_few_steps(oracle, tile, steps, rest, extents, dtype):
     """The loops that load several R steps of 64 elements ahead: fewer steps than are in flight, every remainder of the
-    stages, a partial last step, past the first bank of the offset table; complete and ragged tiles; all three operations,
-    dHW through LDS images and through stored tiles, bias gradient included."""
+    stages, a partial last step, past the first bank of the offset table; the 256 tile's two loops on either side of the rule that chooses; complete and ragged tiles; all
+    three operations, dHW through LDS images and through stored tiles, bias gradient included."""
     from rzlinear_amd import _lib
     from rzlinear_amd.impl.RzLinearBackward import rz_linear_backward_input_grad_tl, weight_grad_hashed
     from rzlinear_amd.impl.RzLinearForward import rz_linear_forward_bias_tl
