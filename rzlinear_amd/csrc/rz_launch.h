@@ -276,8 +276,8 @@ static constexpr double kPairRate128F32 = 0.955;
 // of rows x cols over `slices` slices of `steps` steps of 64.  A round of workgroups takes its steps and a fixed part (fill,
 // store of C); the 256-row tiles' steps take longer the fuller the chip is, because the board lowers its clock.  Fitted to
 // 2790 measurements (forward and input-grad of 84 shapes of 40 to 16384 rows and 256 to 12000 columns, aligned and odd, every
-// tile and one to eight slices): the plan taken with it is 1.5 % from the best form measured on average, that of the
-// rate model before it, which knew neither the 256 x 128 tile nor the present 256 tile, 6.9 %.
+// tile and one to eight slices): on those the plan taken with it was 1.5 % from the best form on average, that of the
+// rate model before it, which knew neither the 256 x 128 tile nor the present 256 tile, 6.9 %; small calls: see plan_split.
 static inline double store16_us(int rows, int cols, int I, int J, int slices, double steps) {
   const double wgs = (double)(((I + rows - 1) / rows) * (long long)((J + cols - 1) / cols)) * slices;
   auto rounds_of = [&](double per) { return (double)((long long)((wgs + per - 1) / per)); };
@@ -758,10 +758,59 @@ static inline int finish_slices(int tile, int I, int J, int R, int elem_bytes, c
   return finish_limit(tile);
 }
 
+// 16-bit 256 tile: whether `steps` R steps of 64 are too few for the phase loop.  It gains 3 to 5 % per step but takes 1.1 us more around
+// its steps (of which the exchange of accumulators is 0.3), with ragged tiles 2 to 3, than the loop of the other tiles.  bf16, us (other
+// loop / phase loop), K = N or M = N = 4096 if not said: forward of 1 / 5 / 6 / 8 steps 11.3 / 12.5, 16.2 / 16.5, 17.8 / 17.8, 20.5 / 20.2; ragged,
+// 4090 x 4000, 1 / 6 / 12 / 16 steps 14.4 / 17.2, 21.6 / 23.0, 32.0 / 31.9, 39.3 / 38.4, 2030 x 4090 (half the chip) 14.0 / 17.4, 21.4 / 23.9, 29.6 / 30.8,
+// 35.1 / 35.6; weight-grad 1 / 3 / 4 steps 23.4 / 23.7, 26.2 / 26.4, 27.5 / 27.4; ragged 1 / 8 / 10 steps 25.2 / 26.7, 32.8 / 33.3, 35.0 / 35.2.
+static inline bool short_loop(int op, bool full, int steps) {
+  return steps <= (op == kWeightGrad ? (full ? 3 : 8) : (full ? 5 : 10));
+}
+
+// 16-bit forward / input-grad of more than 64 rows: roughly how long the call takes, in microseconds, as a sum over what its kernels do:
+// rounds of workgroups take their steps and a fixed part, both longer the fuller the chip, with ragged tiles, and with rows that are not whole
+// 16-byte pieces; a cut takes a fixed part and its planes, whether its own kernel finishes it or a second one.  Fitted to 54 000
+// GPU-bound measurements (forward and input-grad of 2360 shapes of 65 to 32768 rows and 64 to 16384 columns, aligned and odd, every tile,
+// one to twelve slices).
+struct Forward16Times {
+  double launch, step, step_fill, step_ragged, step_odd, round, round_ragged, round_odd, round_fill;
+  double finish, finish_mb, second, second_mb, second_slice;   // us, us per MB of planes written and read, us per slice beyond eight
+};
+static inline double forward16_us(int rows, int cols, int I, int J, int R, int slices, int steps, bool finished) {
+  static constexpr Forward16Times kTimes[7] = {
+    {1.978, 0.198, 0.025, 0.004, 0.051, 1.999, 1.049, 0.100, 0.240, 2.615, 0.098, 3.034, 0.209, 0.433},   // 64 tile, at most one workgroup per compute unit
+    {4.458, 0.263, 0.194, 0.015, 0.068, -1.211, 0.953, 0.178, 3.756, 3.314, 0.008, 3.387, 0.080, 0.198},   // 64 tile, two per compute unit
+    {2.197, 0.420, 0.088, 0.012, 0.099, 1.594, 1.426, 0.193, 1.129, 5.960, 0.102, 2.961, 0.201, 0.001},   // 128 tile of eight wavefronts
+    {3.117, 0.487, 0.487, 0.009, 0.179, 1.435, 1.654, 0.849, 1.360, 10.317, 0.114, 7.999, 0.076, 0.001},   // 128 tile of four, pairs on a compute unit
+    {2.550, 0.592, 0.134, 0.013, 0.164, 2.418, 1.313, 0.965, 1.519, 11.180, 0.107, 3.789, 0.197, 0.001},   // 256 x 128
+    {5.198, 1.201, 0.123, 0.000, 0.144, 0.566, 1.771, 1.471, 4.903, 12.357, 0.159, 6.117, 0.143, 0.001},   // 256 tile, few steps
+    {2.453, 0.966, 0.351, 0.021, 0.092, 6.473, 1.870, 1.543, 0.819, 8.326, 0.187, 4.928, 0.118, 0.001},   // 256 tile
+  };
+  const long long wgs = (long long)((I + rows - 1) / rows) * ((J + cols - 1) / cols) * slices;
+  const bool full = I % rows == 0 && J % cols == 0 && R % (rows == 64 ? 128 : 64) == 0;
+  const double n = steps, ragged = full ? 0.0 : 1.0, odd = (R % 8 != 0 || J % 8 != 0) ? 1.0 : 0.0;
+  const long long per = rows == 64 && wgs > kComputeUnits ? 2 * kComputeUnits : kComputeUnits;
+  double rounds = (double)((wgs + per - 1) / per), fill = (double)wgs / (rounds * per);
+  int which = cols == 256 ? (short_loop(kForward, full, steps) ? 5 : 6) : rows == 256 ? 4 : rows == 64 ? (wgs <= kComputeUnits ? 0 : 1) : 2;
+  if (which == 2 && wgs > kComputeUnits * 3 / 2) {   // (a compute unit's last workgroup without a partner takes 0.62 of a pair's time)
+    which = 3;
+    const long long pairs = wgs / (2 * kComputeUnits), rest = wgs - pairs * 2 * kComputeUnits;
+    rounds = (double)pairs + (rest == 0 ? 0.0 : rest > kComputeUnits ? 1.0 : 0.62);
+    fill = 1.0;
+  }
+  const Forward16Times& c = kTimes[which];
+  const double us = c.launch + rounds * (n * (c.step + c.step_fill * fill + c.step_ragged * ragged + c.step_odd * odd) +
+                                         c.round + c.round_ragged * ragged + c.round_odd * odd + c.round_fill * fill);
+  if (slices == 1) return us;
+  const double mb = (double)I * J * 4.0e-6;
+  return us + (finished ? c.finish + c.finish_mb * (2.0 * slices - 1.0) * mb
+                        : c.second + c.second_mb * (2.0 * slices + 0.5) * mb + (slices > 8 ? c.second_slice * (slices - 8) : 0.0));
+}
+
 // Tile and number of slices together: the pair with the least estimated time.  A slice pays the
 // fill and drain of its pipeline (about three steps), the cut pays the fp32 partial planes
 // (written, read back) and the launch of the kernel that adds them.
-static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz_tuning& t, int depth = 0) {
+static inline SplitPlan plan_split_by_rate(int I, int J, int R, int elem_bytes, const rz_tuning& t, int depth = 0) {
   SplitPlan best = {};
   double best_us = 0.0;
   const double peak = elem_bytes == 4 ? 149e6 : 1150e6;   // flop per microsecond of the 256 tile on a full chip
@@ -832,15 +881,55 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
   if (elem_bytes == 2 && t.split == 0 && best.splits > 1 && depth == 0) {
     rz_tuning whole_only = t;
     whole_only.split = -1;
-    const SplitPlan w = plan_split(I, J, R, elem_bytes, whole_only, 1);
+    const SplitPlan w = plan_split_by_rate(I, J, R, elem_bytes, whole_only, 1);
     if (w.est_us <= 14.0) return w;
   }
-  if (best.tile == 0 && t.split > 0 && depth < 2) return plan_split(I, J, R, elem_bytes, t, 2);
+  if (best.tile == 0 && t.split > 0 && depth < 2) return plan_split_by_rate(I, J, R, elem_bytes, t, 2);
   if (best.tile == 0 && t.split > 0) {   // (no cut comes out at exactly that many slices: the library's own choice)
     rz_tuning free_cut = t;
     free_cut.split = 0;
-    return plan_split(I, J, R, elem_bytes, free_cut);
+    return plan_split_by_rate(I, J, R, elem_bytes, free_cut);
   }
+  best.workspace_bytes = best.splits > 1 ? (size_t)best.splits * (size_t)I * (size_t)J * sizeof(float) : 0;
+  best.est_us = best_us;
+  return best;
+}
+
+// ... and for a 16-bit batch of more than 64 rows the plan with the least time by forward16_us, where that promises 7 % more than
+// the fit's error in telling two plans apart.  (The times of the plan by rate know no ragged tiles and take a second kernel for half a
+// microsecond.  Measured, 2992 calls: the plan by rate is 3.9 % from the best form on average and more than 10 % in 1 call of 6; so
+// 1.2 %, 1 in 22, and 18 calls are more than 3 % slower than by rate, 431 faster — M = 192, K = 3712, N = 1152 forward 15.1 -> 10.3 us, four slices
+// for eight; M = 101, K = 2233, N = 1012 15.2 -> 10.8, four for one.  Without the 7 %: 0.7 %, but 102 are slower; in a long training pass
+// near ties fall as the plan by rate has them: M = 1024, K = N = 10240 in three slices 658 us, whole 671.)
+static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz_tuning& t) {
+  const SplitPlan by_rate = plan_split_by_rate(I, J, R, elem_bytes, t);
+  if (elem_bytes != 2 || I <= 64 || R < 8 || t.tile != 0 || t.split != 0 || t.stages == 1 || t.clamp == -1) return by_rate;
+  auto time_of = [&](int tile, int slices, int chunk) {
+    const bool pair = pair_form(tile, I, J, R, slices > 1 ? chunk : R, elem_bytes, t);
+    const bool finished = slices > 1 && slices <= finish_slices(tile, I, J, R, elem_bytes, t) && t.finish != -1;
+    return forward16_us(pair ? 256 : tile, tile, I, J, R, slices, chunk / 64, finished);
+  };
+  SplitPlan best = by_rate;
+  double best_us = 0.0;
+  const int tiles_of[3] = {256, 128, 64};
+  for (int tile : tiles_of) {
+    const int TR = slice_unit(tile, elem_bytes), r_steps = (R + TR - 1) / TR;
+    for (int slices = 1; slices <= 16; slices++) {
+      const int chunk = (r_steps + slices - 1) / slices * TR;
+      if (((r_steps * TR + chunk - 1) / chunk) != slices) continue;   // (the same cut as fewer slices)
+      if (slices > 1 && chunk < 4 * 64) break;   // slices of a few steps are all fill and drain
+      const double us = time_of(tile, slices, chunk);
+      if (best_us == 0.0 || us < best_us * 0.97) {   // (near ties go to the larger tile and the fewer slices)
+        best.tile = tile;
+        best.splits = slices;
+        best.r_chunk = chunk;
+        best_us = us;
+      }
+    }
+  }
+  const int unit = slice_unit(by_rate.tile, elem_bytes);
+  const double by_rate_us = time_of(by_rate.tile, by_rate.splits, by_rate.splits > 1 ? by_rate.r_chunk : (R + unit - 1) / unit * unit);
+  if (best_us >= 0.93 * by_rate_us) return by_rate;
   best.workspace_bytes = best.splits > 1 ? (size_t)best.splits * (size_t)I * (size_t)J * sizeof(float) : 0;
   best.est_us = best_us;
   return best;
@@ -857,15 +946,6 @@ struct KernelForm {
   bool short_loop;   // 16-bit 256 tile: the loop for a few R steps
   int step;
 };
-
-// 16-bit 256 tile: whether `steps` R steps of 64 are too few for the phase loop.  It gains 3 to 5 % per step but takes 1.1 us more around
-// its steps (of which the exchange of accumulators is 0.3), with ragged tiles 2 to 3, than the loop of the other tiles.  bf16, us (other
-// loop / phase loop), K = N or M = N = 4096 if not said: forward of 1 / 5 / 6 / 8 steps 11.3 / 12.5, 16.2 / 16.5, 17.8 / 17.8, 20.5 / 20.2; ragged,
-// 4090 x 4000, 1 / 6 / 12 / 16 steps 14.4 / 17.2, 21.6 / 23.0, 32.0 / 31.9, 39.3 / 38.4, 2030 x 4090 (half the chip) 14.0 / 17.4, 21.4 / 23.9, 29.6 / 30.8,
-// 35.1 / 35.6; weight-grad 1 / 3 / 4 steps 23.4 / 23.7, 26.2 / 26.4, 27.5 / 27.4; ragged 1 / 8 / 10 steps 25.2 / 26.7, 32.8 / 33.3, 35.0 / 35.2.
-static inline bool short_loop(int op, bool full, int steps) {
-  return steps <= (op == kWeightGrad ? (full ? 3 : 8) : (full ? 5 : 10));
-}
 
 static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int tile, long long workgroups,
                                      int elem_bytes, const rz_tuning& t) {

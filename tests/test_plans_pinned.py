@@ -108,3 +108,15 @@ def test_a_batch_below_the_fit_pays_for_the_images_of_the_128_tile(shape, tile):
     """Measured (bf16): the first five are 5 to 9 % slower with the 128 tile, the next three 12 to 60 % faster."""
     q = _lib.plan_query(2, *shape, BF16, planned=True)
     assert (q["mode"], q["tile"]) == ("lds_image", tile)
+
+
+@pytest.mark.parametrize("op,shape,plan", [
+    (0, (192, 3712, 1152, 267264, 32, 64), (64, 4)), (0, (640, 3072, 384, 16384, 64, 64), (64, 4)), (0, (101, 2233, 1012, 16384, 64, 64), (64, 4)),
+    (1, (352, 896, 3328, 186368, 32, 64), (64, 3)), (1, (96, 1792, 2880, 322560, 64, 64), (64, 4)), (1, (274, 649, 3240, 131422, 64, 64), (64, 4)),
+    (1, (224, 1024, 7296, 466944, 64, 64), (64, 4)), (0, (2368, 256, 13056, 33423, 32, 64), (256, 1)), (0, (12320, 256, 6080, 97280, 32, 64), (256, 1)),
+], ids=str)
+@pytest.mark.parametrize("code", [BF16, F16])
+def test_16_bit_plans_that_a_second_kernel_or_ragged_tiles_make_slower(op, shape, plan, code):
+    """Measured (bf16): other cuts, with a second kernel, or none, or the 128 tile for a few steps are 10 to 45 % slower here."""
+    q = _lib.plan_query(op, *shape, code)
+    assert (q["tile"], q["slices"]) == plan
