@@ -503,7 +503,7 @@ def main():
     if not args.no_cpu_baseline:
         from oracle import cpu_path   # checker/baseline only: never on the measured GPU path
         # every host core this job may use: the machine's, unless the job was given a smaller
-        # share through OMP_NUM_THREADS (GPU boxes hand one GPU's job a share of the host)
+        # share through OMP_NUM_THREADS
         share = os.environ.get("OMP_NUM_THREADS")
         cores = os.cpu_count() or 1
         if share and share.isdigit() and int(share) > 0:
