@@ -180,7 +180,8 @@ int rz_input_grad_ws(const void* dY, const void* HW, void* dX, void* workspace,
  * and a second kernel folds the tiles into dHW (plus a few images of dHW and one int32 offset
  * per W tile) — 16-bit: wherever that is the faster, though it can take several times the bytes of X and
  * dY where atomic adds would need 4 * H (rz_tuning.fold = -1 forgoes it); with M small against K*N, dHW is computed in windows and the workspace holds
- * only the offsets; with few tiles the 16-bit types need an fp32 image of dHW (H floats) for
+ * the offsets and X and dY once more, as the fragments that the kernel multiplies (a workspace with room for the offsets
+ * alone, or none where a layer plan has them, is enough: the call is then slower); with few tiles the 16-bit types need an fp32 image of dHW (H floats) for
  * atomic adds and fp32 needs nothing.  The size depends on M: ask again when the batch size
  * changes.
  */

@@ -125,7 +125,7 @@ static WeightGradChoice weight_grad_choice(int M, int K, int N, int H, int BK, i
   const int limit_mb = limit == (size_t)-1 ? -1 : (int)(limit >> 20);
   return memo.get({M, K, N, H, BK, BN, elem_bytes, tile_bytes, planned ? 1 : 0, limit_mb, RZ_TUNING_WORDS(t)}, [&] {
     WeightGradChoice c = {plan_weight_grad(M, K, N, H, BK, BN, elem_bytes, t, tile_bytes, limit), {}};
-    if (!c.plan.lds_image()) c.window = plan_window(M, K, N, H, BK, BN, elem_bytes, t, c.plan, planned);
+    if (!c.plan.lds_image()) c.window = plan_window(M, K, N, H, BK, BN, elem_bytes, t, c.plan, planned, limit);
     return c;
   });
 }
@@ -416,7 +416,7 @@ static inline size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Workspace layout of a weight-grad call: [main][column sums].  main = the partial images (LDS
 // image mode), the tile-by-tile X^T.dY followed by the fold kernel's images, the table of tile
-// offsets (window kernel) or, for the atomic scatter into a 16-bit dHW, its fp32 image.
+// offsets (window kernel; where there is room behind it, see window_pack_kernel, X and dY as fragments) or, for the atomic scatter into a 16-bit dHW, its fp32 image.
 struct WeightGradWorkspace {
   size_t main_bytes, total_bytes;
 };
@@ -508,6 +508,14 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
       w.dbias = dbias;
       w.dbias_f32 = dbias_dtype == RZ_F32 ? 1 : 0;
       w.windows = wp.windows;
+      // where the workspace has room behind the offsets: X and dY as fragments (the same bits, faster)
+      const uintptr_t pack_at = ((uintptr_t)workspace + ws.main_bytes + 15) & ~(uintptr_t)15;
+      if (wp.pack_bytes > 0 && workspace != nullptr && pack_at - (uintptr_t)workspace <= workspace_bytes &&
+          workspace_bytes - (pack_at - (uintptr_t)workspace) >= wp.pack_bytes) {
+        const size_t group = dtype == RZ_F32 ? 8 : 16, rows = ((size_t)M + group - 1) / group * group;
+        w.packed_x = (void*)pack_at;
+        w.packed_y = (void*)(pack_at + rows * dtype_bytes(dtype) * (size_t)w.tiles_k * BK);
+      }
       w.poll_limit = tuning.poll_limit > 0 ? tuning.poll_limit : kWindowPollLimit;
       hipError_t e = dtype == RZ_F32 ? launch_window_f32(w, wp.windows, s)
                      : dtype == RZ_BF16 ? launch_window_bf16(w, wp.windows, s)
@@ -606,7 +614,13 @@ static size_t weight_grad_bytes(int M, int K, int N, int H, int BK, int BN, int 
   if (check_tile(BK, BN) != RZ_OK) return 0;
   const bool dhw_f32 = (flags & RZ_WG_DHW_F32) != 0 || dtype == RZ_F32;
   const WeightGradChoice c = weight_grad_choice(M, K, N, H, BK, BN, eb, fold_tile_bytes(eb, dhw_f32, t), t, false, limit);
-  return weight_grad_workspace(c.plan, c.window, H, dhw_f32, with_dbias != 0).total_bytes;
+  size_t bytes = weight_grad_workspace(c.plan, c.window, H, dhw_f32, with_dbias != 0).total_bytes;
+  if (limit != (size_t)-1) return bytes;   // (what the call cannot do without)
+  // room for the fragments of the window kernel, also where only a caller with a layer plan is to get there
+  if (c.window.use) return bytes + 16 + c.window.pack_bytes;
+  const WeightGradChoice planned = weight_grad_choice(M, K, N, H, BK, BN, eb, fold_tile_bytes(eb, dhw_f32, t), t, true);
+  if (planned.window.use && bytes < 16 + planned.window.pack_bytes) bytes = 16 + planned.window.pack_bytes;
+  return bytes;
 }
 
 }  // namespace rz

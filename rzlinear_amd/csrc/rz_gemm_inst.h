@@ -185,15 +185,16 @@ static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const 
   }
 }
 
-template <typename T, int TBN, bool STAGED>
-static hipError_t launch_window_form(const WindowParams& p, int windows, hipStream_t stream) {
-  typedef WindowKernel<T, TBN, STAGED> K;
-  static_assert(K::kFixedBytes + sizeof(float) * kWindowFloats <= 160 * 1024, "window does not fit the LDS");
+template <typename T, int TBN, int OPERANDS>
+static hipError_t launch_window_form(WindowParams p, int windows, hipStream_t stream) {
+  typedef WindowKernel<T, TBN, OPERANDS> K;
+  static_assert(K::kImageFloats >= kWindowFloats, "window does not fit the LDS");
   if (p.window < 4 || p.window > kWindowFloats || (p.window & 3) || windows < 1) return hipErrorInvalidValue;
   if ((long long)windows * p.window < p.H) return hipErrorInvalidValue;
   if (p.h.BN != TBN || !window_tile_supported(p.h.BK, p.h.BN)) return hipErrorInvalidValue;
-  auto kernel = rz_window_kernel<T, TBN, STAGED>;
-  const size_t smem = K::kFixedBytes + sizeof(float) * (size_t)p.window;
+  auto kernel = rz_window_kernel<T, TBN, OPERANDS>;
+  p.images = window_images(p.window, OPERANDS == kPacked);
+  const size_t smem = K::kFixedBytes + sizeof(float) * (size_t)p.window * p.images;
   static std::atomic<uint64_t> lds_limit_raised{0};
   if (smem > 64 * 1024) {
     hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds_limit_raised);
@@ -205,14 +206,25 @@ static hipError_t launch_window_form(const WindowParams& p, int windows, hipStre
   return hipGetLastError();
 }
 
-// Operands whose rows hold whole 16-byte pieces go through the staged form.
+// With room for them the operands are laid out as fragments first; else, where their rows hold whole 16-byte pieces, they go
+// through the staged form.
 template <typename T, int TBN>
 static hipError_t launch_window_one(const WindowParams& p, int windows, hipStream_t stream) {
   constexpr int kVec = 16 / (int)sizeof(T);
+  if (p.packed_x != nullptr && p.packed_y != nullptr) {
+    // (blocks of 32 columns up to whole hashed tiles: every unit of every tile has its fragments, see window_pack_bytes)
+    const long long blocks_x = (long long)p.tiles_k * (p.h.BK / 32), blocks_y = (long long)p.tiles_n * (TBN / 32);
+    constexpr int kRows = WindowKernel<T, TBN, kPacked>::kGroupRows;
+    const long long ngroups = (p.M + kRows - 1) / kRows, wgs = ((blocks_x + blocks_y) * ngroups + 3) / 4;
+    if (wgs > 0x1fffffffLL) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(window_pack_kernel<T>, dim3((unsigned)wgs), dim3(256), 0, stream, p, (int)blocks_x, (int)blocks_y, (int)ngroups);
+    hipError_t e = hipGetLastError();
+    return e != hipSuccess ? e : launch_window_form<T, TBN, kPacked>(p, windows, stream);
+  }
   // (the staged form keeps the byte offsets of a lane's pieces, up to sixteen rows, in 32-bit registers)
   if (p.K % kVec == 0 && p.N % kVec == 0 && p.ldx < (1 << 25) && p.lddy < (1 << 25))
-    return launch_window_form<T, TBN, true>(p, windows, stream);
-  return launch_window_form<T, TBN, false>(p, windows, stream);
+    return launch_window_form<T, TBN, kStaged>(p, windows, stream);
+  return launch_window_form<T, TBN, kByElement>(p, windows, stream);
 }
 
 template <typename T>

@@ -577,6 +577,7 @@ struct WindowPlan {
   int window;    // elements of dHW per workgroup
   int windows;   // workgroups
   long long tiles;   // W tiles (entries of the offset table the kernel scans)
+  size_t pack_bytes; // X and dY as fragments (workspace that the call can do without)
 };
 static constexpr int kWindowFloats = 25600;   // LDS floats a workgroup can hold next to its staging
 
@@ -606,43 +607,70 @@ static inline void window_geometry(int H, int* window, int* windows) {
   *windows = (int)(((long long)H + w - 1) / w);
 }
 
-// planned: the caller holds a layer plan, so the kernel neither hashes the tile offsets nor scans
+// Images of a window that a workgroup keeps in LDS, a power of two up to its sixteen wavefronts.  With a small window nearly every
+// unit meets the one before it in the list, and the chain of adds takes most of the time; with images a unit waits for those of
+// its own image only (bf16, windows of 4096: M = 16, K = 2048, N = 8192 35.6 -> 20 us, M = 64, K = N = 4096 39.4 -> 24.7;
+// windows of 1024: M = 32, K = N = 2048 37 -> 15.5).  The packed form has no staging area, so that half as much again fits.
+constexpr int window_image_floats(bool packed) { return packed ? kWindowFloats * 3 / 2 : kWindowFloats; }
+static inline int window_images(int window, bool packed) {
+  int n = 1;
+  while (n < 16 && 2 * n * window <= window_image_floats(packed)) n *= 2;
+  return n;
+}
+
+// Bytes of X and dY as fragments (window_pack_kernel): the rows up to whole groups, the columns up to whole hashed tiles.
+static inline size_t window_pack_bytes(int M, int K, int N, int BK, int BN, int elem_bytes) {
+  const size_t group = elem_bytes == 4 ? 8 : 16, rows = ((size_t)M + group - 1) / group * group;
+  return rows * (size_t)elem_bytes * ((size_t)((K + BK - 1) / BK) * BK + (size_t)((N + BN - 1) / BN) * BN);
+}
+
+// What the window kernel takes with its operands as fragments (with the kernel that makes them), staged, or element by element:
+// microseconds on MI355X, fitted to 770 calls of drawn shapes (1 to 700 rows, 128 to 14000 columns, tiles of 32 x 64 and 64 x 64,
+// K * N / H of 16 and 100) in captured graphs; the fits' error is 8 % (element by element in fp32 15 %).  A workgroup works through
+// the units that meet its window, each at a fixed price and one per 32 rows of M; in 16 bits the latter grows where X and dY outgrow
+// an L2 (4 MB), from which every unit reads its own rows and columns.  The adds into one place of an image go one after the
+// other: K * N / H links, of the images' share each.  The greater of the two sets the time; of the smaller one a part still shows.
+static inline double window_us(int M, int K, int N, int H, int BK, int BN, int elem_bytes, int window, int windows, bool packed) {
+  struct Fit { double fixed, per_mb, unit, rows, misses, link, rest; };
+  static const Fit fits[2][3] = {{{10.4, 2.0, 0.160, 0.040, 0.040, 2.3, 0.17}, {10.1, 0.9, 0.171, 0.063, 0.039, 1.8, 0.41}, {12.6, 3.0, 0.219, 0.178, 0.066, 3.1, 0.05}},
+                                 {{11.7, 4.7, 0.050, 0.320, 0.0, 3.3, 0.40}, {12.6, 3.4, 0.083, 0.290, 0.0, 1.66, 1.0}, {13.6, 8.2, 0.0, 0.524, 0.0, 1.14, 1.0}}};
+  const bool whole = K % (16 / elem_bytes) == 0 && N % (16 / elem_bytes) == 0;
+  const Fit& f = fits[elem_bytes == 4][packed ? 0 : whole ? 1 : 2];
+  const double tiles = (double)((K + BK - 1) / BK) * (double)((N + BN - 1) / BN);
+  const double units = tiles * window_units(BK, BN) * ((double)window + window_unit_span(BN)) / (double)H;
+  const double rounds = (double)((windows + kComputeUnits - 1) / kComputeUnits);
+  const double chunks = M > 16 ? M / 32.0 : 0.5, mb = (double)M * ((double)K + N) * elem_bytes * 1e-6;
+  const double work_us = rounds * units * (f.unit + chunks * (f.rows + (mb > 4.3 ? f.misses * (1.0 - 4.3 / mb) : 0.0)));
+  const double chain_us = f.link * (double)K * N / (double)H / window_images(window, packed);
+  return f.fixed + f.per_mb * mb + (work_us > chain_us ? work_us + f.rest * chain_us : chain_us + f.rest * work_us);
+}
+
+// limit: bytes of workspace that the call may have.  planned: the caller holds a layer plan, so the kernel neither hashes the tile offsets nor scans
 // them for its strips (some 25 us less, measured at K = N = 10240).
 static inline WindowPlan plan_window(int M, int K, int N, int H, int BK, int BN, int elem_bytes, const rz_tuning& t,
-                                     const WeightGradPlan& other, bool planned = false) {
-  WindowPlan pl = {false, 0, 0, 0};
+                                     const WeightGradPlan& other, bool planned = false, size_t limit = (size_t)-1) {
+  WindowPlan pl = {false, 0, 0, 0, 0};
   if (t.window == -1 || !window_tile_supported(BK, BN)) return pl;
   const long long tiles = (long long)((K + BK - 1) / BK) * ((N + BN - 1) / BN);
   if (tiles > (1 << 20)) return pl;              // every workgroup scans every tile's offset
   pl.tiles = tiles;
   window_geometry(H, &pl.window, &pl.windows);
-  const long long w = pl.window;
-  // Rough times in microseconds, fitted to measurements at K = N = 10240, H = 6.5 M on MI355X.
-  // Scatter kernel: K*N atomics at about 184 G/s plus the product.  Window kernel: every
-  // workgroup works through tiles * (window + tile) / H tiles; a tile costs about 0.25 us plus
-  // 0.16 us (16-bit; M = 32 56 us, 128 91, 192 135, 256 188), or 0.43 us plus 0.63 us (fp32: the fp32 MFMA rate), per 32 rows of M (the
-  // operands of every tile come out of L2 again: tiles that share a window share no rows or
-  // columns of W; a wavefront has three groups of rows in flight, which is what its registers hold).
-  const double chunks = (double)((M + 31) / 32);
-  // (in units of 64 x 64 tiles, i.e. of two strips of 64 columns: the figures below were fitted on those;
-  //  32-column tiles take the time of 64-column ones — their units are half empty)
-  const double per_wg = (double)tiles * ((double)w + (double)BK * BN) / (double)H * ((double)BK / 64.0) * (BN > 64 ? BN / 64.0 : 1.0);
-  const double wg_rounds = (double)((pl.windows + kComputeUnits - 1) / kComputeUnits);
-  // (rows of X or dY that are not whole 16-byte pieces are fetched element by element: about 2.2 times the
-  //  time per tile — M = 256, K = 10239, N = 10240, bf16: 411 us against 190 us with K = 10240)
-  const int vec = 16 / elem_bytes;
-  const double by_elements = (K % vec == 0 && N % vec == 0) ? 1.0 : 2.2;
-  double t_window = wg_rounds * per_wg * by_elements * ((elem_bytes == 4 ? 0.43 + 0.63 * chunks : 0.25 + 0.16 * chunks)) + (planned ? 5.0 : 28.0);
-  // Every element of dHW receives K*N / H tiles, and the adds into one place of a window go in a
-  // fixed order, one after the other: with many tiles per element that chain is what takes the
-  // time, about 1.7 us a link (K = 2048, N = 8192, H = 200000: 84 links, 158 us at M = 32 — folded
-  // 57 us; K = N = 10240, H = 200000: 524 links, 1048 us).
-  // (fp32, K = N = 10240, H = 2^20, M = 32: 100 links, 260 us — folded 220 us)
-  const double chain_us = (elem_bytes == 4 ? 2.4 : 1.7) * (double)K * (double)N / (double)H + 10.0;
-  if (t_window < chain_us) t_window = chain_us;
-  // ... against what the contraction kernel's plan would take: the fold, or the atomic scatter
+  // The operands as fragments where that is faster, by more than the launch that it adds costs a host that is the bound (K = N =
+  // 10240, H = 6.5 M, bf16: M = 8 55 -> 51 us, 32 59 -> 53, 128 99 -> 77, 256 180 -> 144; fp32: 32 113 -> 105, but 64 169 -> 174 and
+  // 128 287 -> 318, where the matrix pipe is the bound and the staged form keeps it busier).
+  double t_window = window_us(M, K, N, H, BK, BN, elem_bytes, pl.window, pl.windows, false);
+  const size_t pack_bytes = window_pack_bytes(M, K, N, BK, BN, elem_bytes);
+  const double packed_us = window_us(M, K, N, H, BK, BN, elem_bytes, pl.window, pl.windows, true);
+  if (packed_us + 3.0 < t_window && pack_bytes <= limit && (size_t)tiles * sizeof(int32_t) + 512 <= limit - pack_bytes) {
+    t_window = packed_us;
+    pl.pack_bytes = pack_bytes;
+  }
+  if (!planned) t_window += 23.0;   // (the offsets hashed, every workgroup's search among them)
+  // ... against what the contraction kernel's plan would take: the fold, or the atomic scatter.  Those prices leave out what is the
+  // same for all of their plans: measured, on such shapes, the windowed fold takes 1.18 times its price (5 to 95 %: 1.07 to
+  // 1.35), the few-tiles fold 1.7 (fp32) to 1.9 times (its longest calls less, hence 1.65), the atomics about 1.8 times.
   const double t_scatter = 0.9 * (double)K * N / 184e3 + 2.0 * M * (double)K * N / 800e6;
-  const double t_other = other.fold.use ? other.fold_us : t_scatter;
+  const double t_other = other.fold.use ? other.fold_us * (other.fold.small ? 1.65 : 1.18) : 1.8 * t_scatter;
   pl.use = t.window == 1 || t_window < t_other;
   return pl;
 }

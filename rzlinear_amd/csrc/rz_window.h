@@ -9,16 +9,18 @@
 // cut into strips of 32 rows, in ascending order — or, when the caller holds a layer plan, reads
 // that list from it (offsets and lists depend on the layer alone).  Then
 // every WAVEFRONT takes strips from the list on its own: it computes the whole X^T.dY product
-// of a strip — the operands are small and stay in L2; a wavefront fetches its own operand
-// pieces (16-bit types: 16-byte pieces through a small LDS area of its own and the LDS
-// transpose read; otherwise the MFMA fragments element by element in their register layout),
+// of a strip — the operands are small and stay in L2; a wavefront fetches its own operands
+// (the MFMA fragments that a kernel ahead of this one has made of them; without a workspace for those 16-byte pieces through a
+// small LDS area of its own, or the fragments element by element in their register layout),
 // so no wavefront waits for another — and adds the part inside the window with plain LDS
 // read-add-write.  Slices of different
 // tiles may overlap: a tile is added only after every earlier tile of the list whose slice
 // meets its own has been added (the wavefronts' progress, polled in LDS), so the summation order
 // of every element is the list order whatever the timing.  Finally the window is stored: every
 // element of dHW is written exactly once, with no atomics and no clearing pass.  A tile that
-// straddles a window boundary is computed by both neighbours.
+// straddles a window boundary is computed by both neighbours.  A window that leaves room for it has several images in LDS,
+// which are added up when it is stored: wavefront w adds into image w mod images, and only units of one image wait for each
+// other (see window_images in rz_launch.h).
 #pragma once
 
 #include <type_traits>
@@ -45,6 +47,7 @@ struct WindowParams {
   float scale;
   HashParams h;
   int window;        // elements of dHW per workgroup (a multiple of 4)
+  int images;        // images of the window in LDS (a power of two, at most the wavefronts of a workgroup), see window_images
   int tiles_k, tiles_n;
   int accumulate;    // dHW += gradient instead of dHW = gradient
   int out_f32;       // dHW is fp32 whatever T is
@@ -52,12 +55,17 @@ struct WindowParams {
   int dbias_f32;     // ... as fp32 whatever T is
   int windows;       // workgroups that own a window
   int poll_limit;    // looks at the flags of earlier strips before a wavefront gives up (kWindowPollLimit)
+  // Non-null: X and dY as MFMA fragments (see window_pack_kernel), which the packed form of the kernel reads
+  void* packed_x;
+  void* packed_y;
 };
 
 // How often a wavefront looks at the flags of the earlier strips it must wait for before it gives
 // up.  A look takes at least 64 clocks (the sleep between two), so the limit is some seconds —
 // far beyond any real wait (a strip's product takes microseconds) and still an end.
 static constexpr int kWindowPollLimit = 1 << 24;
+
+static constexpr int kFragBytes = 1024;   // a fragment of a wavefront: 16 bytes per lane
 
 // The hashed tile is BK x TBN: TBN (32, 64 or 128) at compile time — it is the row pitch of a tile's
 // slice of hashed_weight — BK (a multiple of 32) at run time.  The unit of work is 32 rows by UC =
@@ -69,8 +77,17 @@ static constexpr int kWindowPollLimit = 1 << 24;
 // STAGED (K and N multiples of the 16-byte piece): operands travel as 16-byte pieces through the
 // wavefront's staging area (a quarter of the load instructions per byte for fp32, an eighth for the
 // 16-bit types); otherwise fragments are loaded element by element.
-template <typename T, int TBN, bool STAGED>
+// PACKED (the caller's workspace has room): a kernel ahead of this one has laid X and dY out as fragments, zeros where
+// they end, so that an item is BJ + 1 loads of 1 KB in a row straight into the registers the MFMAs read.  What the staged form
+// loses is around its MFMAs: per item 6 KB through LDS next to the window's adds, which alone keep it busy for 14 us at
+// K = N = 10240, and loads in row pieces of 64 and 128 bytes (that shape, H = 6.5 M, bf16, with the kernel ahead: M = 32 59 -> 53,
+// 128 99 -> 77, 256 180 -> 144 us; of the 77 loads take most: 67 without the adds).  Not faster: four or five
+// items in flight (spills), eight wavefronts with up to eight (87 us), units in the order of their offsets (fewer waits,
+// but units of one window then share no rows or columns in the L2: 120 us against 92 staged).
+enum WindowOperands { kByElement = 0, kStaged = 1, kPacked = 2 };
+template <typename T, int TBN, int OPERANDS>
 struct WindowKernel {
+  static constexpr bool STAGED = OPERANDS == kStaged, PACKED = OPERANDS == kPacked;
   static_assert(TBN == 32 || TBN == 64 || TBN == 128, "tiles of 32, 64 or 128 columns");
   typedef ElemTraits<T> Tr;
   typedef typename Mfma<T>::Frag Frag;
@@ -85,18 +102,18 @@ struct WindowKernel {
   // rows of M loaded ahead as one group (16 wavefronts per compute unit leave 128 registers each)
   static constexpr int kGroupRows = sizeof(T) == 4 ? 8 : 16;
   static constexpr int GS = kGroupRows / KS;             // MFMA steps per group
-  static constexpr int kBatch = STAGED ? 8 : 4;           // tile offsets a lane loads at a time
+  static constexpr int kBatch = OPERANDS != kByElement ? 8 : 4;           // tile offsets a lane loads at a time
   // Items (one group of rows of one strip) whose operand loads are in flight while one is being
   // multiplied, plus that one: a ring of register sets.  An item is a few loads and a few MFMAs,
   // so a wavefront's rate is (items in flight) / (memory latency).
-  static constexpr int kDepth = (STAGED || sizeof(T) == 4) ? 3 : 2;
+  static constexpr int kDepth = (OPERANDS != kByElement || sizeof(T) == 4) ? 3 : 2;
   static constexpr bool k16 = sizeof(T) == 2;
   // staged: a wavefront's own staging area, one group of rows of X (32 columns) and of dY (TBN
   // columns), 3 KB; the list is kept shorter to make room for it next to the window
   static constexpr int VEC = Tr::kVec;                   // elements of a 16-byte piece
   static constexpr int kStageX = kGroupRows * 32, kStageElems = STAGED ? kStageX + kGroupRows * UC : 8;
   static constexpr int kList = 960;   // capacity of the list of units found
-  static_assert(!STAGED || (64 * VEC == kGroupRows * 32), "one piece of X and BJ of dY per lane and group");
+  static_assert(OPERANDS == kByElement || (64 * VEC == kGroupRows * 32), "one piece of X and BJ of dY per lane and group");
 
   struct Smem {
     int list[kList];              // units found in this pass (tile id * units per tile + unit), ascending
@@ -105,10 +122,13 @@ struct WindowKernel {
     int count[2][kWaves];
     int spoilt;                   // a wavefront gave up waiting for an earlier strip: the window is stored as NaN
     alignas(16) T stage[kWaves][kStageElems];
-    alignas(16) float window[4];  // the image of dHW[w0, w0 + window) starts here, then 64
+    alignas(16) float window[4];  // the images of dHW[w0, w0 + window) start here, then 64
                                   // dump slots
   };
   static constexpr size_t kFixedBytes = offsetof(Smem, window) + sizeof(float) * 64;   // + dump slots
+  // Floats for images of the window (see window_images in rz_launch.h)
+  static constexpr int kImageFloats = window_image_floats(PACKED);
+  static_assert(kFixedBytes + sizeof(float) * kImageFloats <= 160 * 1024, "the images do not fit the LDS");
 
   // MFMA fragment of a 32-wide block of a row-major matrix (rows = the contracted dimension M).
   //   16-bit: lane l holds rows m0 + r0 + (l >> 5) * 8 + j, j = 0..7, of column (l & 31)
@@ -152,12 +172,13 @@ struct WindowKernel {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     float* __restrict__ win = sm.window;
+    const int image = (wave & (p.images - 1)) * p.window;   // where this wavefront's image begins
     const long long w0 = (long long)blockIdx.x * p.window;
     const int wlen = (p.H - w0) < p.window ? (int)(p.H - w0) : p.window;
     const T* __restrict__ gX = static_cast<const T*>(p.X);
     const T* __restrict__ gdY = static_cast<const T*>(p.dY);
 
-    for (int i = tid * 4; i < p.window; i += kThreads * 4) {
+    for (int i = tid * 4; i < p.images * p.window; i += kThreads * 4) {
       const float4 z = {0.f, 0.f, 0.f, 0.f};
       *reinterpret_cast<float4*>(win + i) = z;
     }
@@ -232,7 +253,7 @@ struct WindowKernel {
     const int plan_lo = planned ? min(max(p.plan_start[blockIdx.x], 0), plan_entries) : 0;
     const int plan_n = planned ? min(max(p.plan_start[blockIdx.x + 1], plan_lo), plan_entries) - plan_lo : 0;
     const int list_total = planned ? plan_n : total;   // what the rounds below work through: entries, or tile ids
-    int lo = 0;
+    int lo = 0, done = 0;   // (done: units of the rounds before)
     while (lo < list_total) {
       int hi = total, found = 0, chunk = 0;
       if (planned) {
@@ -314,10 +335,14 @@ struct WindowKernel {
       if (tid < kWaves) sm.progress[tid] = 0;
       __syncthreads();   // list complete, progress cleared
 
-      // ---- every wavefront works through list entries wave, wave + kWaves, ... on its own ----
+      // ---- every wavefront works through its list entries on its own ----
+      // Unit number u of the window (over all rounds) belongs to wavefront u % kWaves, and so to an image, however the
+      // rounds cut the list: entries my_first, my_first + kWaves, ... of this round's.
+      const int shift = done % kWaves, my_first = (wave - shift) & (kWaves - 1);
+      done += found;
       // An item is one group of rows of M of one tile.  No barrier in here: a wavefront that
       // waits for an earlier tile's flag must never be waited for by the owner of that tile.
-      const int my_tiles = found > wave ? (found - wave + kWaves - 1) / kWaves : 0;
+      const int my_tiles = found > my_first ? (found - my_first + kWaves - 1) / kWaves : 0;
       const int items = my_tiles * ngroups;
       int ft = 0, fg = 0;      // tile ordinal and group of the next item to load
       // The loads of an item are issued unconditionally, in straight-line code: the compiler
@@ -336,6 +361,12 @@ struct WindowKernel {
       typedef const char __attribute__((address_space(1)))* global_ptr;
       auto load_piece = [&](const T* rows, uint32_t at) -> u32x4_t {
         return *reinterpret_cast<const u32x4_any_t __attribute__((address_space(1)))*>((global_ptr)rows + at);
+      };
+      // Packed form: the next group's fragments of the unit being fetched, and the bytes of a block of 32 columns.
+      const int64_t packed_block = (int64_t)ngroups * kFragBytes;
+      global_ptr packed_x = (global_ptr)p.packed_x, packed_y = (global_ptr)p.packed_y;
+      auto load_packed = [&](global_ptr at) -> u32x4_t {
+        return *reinterpret_cast<const u32x4_t __attribute__((address_space(1)))*>(at + (uint32_t)lane * 16u);
       };
       const T* rows_x = gX;
       const T* rows_y = gdY;
@@ -360,10 +391,30 @@ struct WindowKernel {
       bool mult_whole = all_whole;
       auto fetch_next = [&](auto set) {
         constexpr int S = decltype(set)::value;
+        if constexpr (PACKED) {
+          if (fg == 0) {   // (uniform) a new unit
+            const int ftc = ft < my_tiles ? ft : my_tiles - 1;
+            const int v = __builtin_amdgcn_readfirstlane(sm.list[my_first + ftc * kWaves]);
+            const int id = v >> ushift, un = v & (units - 1);
+            const int tk = id / p.tiles_n, tn = id - tk * p.tiles_n;
+            packed_x = (global_ptr)p.packed_x + (int64_t)(tk * (p.h.BK >> 5) + un / kParts) * packed_block;
+            packed_y = (global_ptr)p.packed_y + (int64_t)(tn * (TBN >> 5) + (un % kParts) * BJ) * packed_block;
+          }
+          px[S] = load_packed(packed_x);
+#pragma unroll
+          for (int q = 0; q < BJ; q++) py[S][q] = load_packed(packed_y + q * packed_block);
+          packed_x += kFragBytes;
+          packed_y += kFragBytes;
+          if (++fg == ngroups) {
+            fg = 0;
+            ft++;
+          }
+          return;
+        }
         if constexpr (STAGED) {
           if (fg == 0) {   // (uniform) a new strip
             const int ftc = ft < my_tiles ? ft : my_tiles - 1;
-            const int v = __builtin_amdgcn_readfirstlane(sm.list[wave + ftc * kWaves]);
+            const int v = __builtin_amdgcn_readfirstlane(sm.list[my_first + ftc * kWaves]);
             const int id = v >> ushift, un = v & (units - 1);
             const int tk = id / p.tiles_n, tn = id - tk * p.tiles_n;
             strip_k0 = tk * p.h.BK + (un / kParts) * 32;   // the unit's first row of W
@@ -406,7 +457,7 @@ struct WindowKernel {
         }
         {
           const int ftc = ft < my_tiles ? ft : my_tiles - 1;
-          const int v = __builtin_amdgcn_readfirstlane(sm.list[wave + ftc * kWaves]);
+          const int v = __builtin_amdgcn_readfirstlane(sm.list[my_first + ftc * kWaves]);
           const int id = v >> ushift, un = v & (units - 1);
           const int tk = id / p.tiles_n, tn = id - tk * p.tiles_n;
           const int k0 = tk * p.h.BK + (un / kParts) * 32;   // the unit's first row of W
@@ -438,15 +489,17 @@ struct WindowKernel {
           }
         }
       };
-      // The earlier entries whose spans meet that of entry e must be added before it.  Lane l looks at the entries l,
-      // l + 64, ..., all of wavefront l % kWaves, which adds its entries in order: what counts is the last of them that
-      // meets.  Worked out when a unit begins, while its loads are on their way; what is left for the end, where other
+      // The earlier entries of the same image whose spans meet that of entry e must be added before it.  Lane l looks at the
+      // entries l, l + 64, ..., all of one wavefront, which adds its entries in order: what counts is the last of them
+      // that meets.  Worked out when a unit begins, while its loads are on their way; what is left for the end, where other
       // wavefronts wait in turn, is one look at the wavefronts' progress.  (Looking at every earlier entry's offset and flag
       // there: K = N = 10240 bf16 with M = 32 / 128 62.1 / 95.6 us; so 56.4 / 91.3.)
+      const int other = (lane + shift) & (kWaves - 1);   // that wavefront
       int need_added = 0;
       auto must_be_added = [&](int e) -> int {
         const int off = __builtin_amdgcn_readfirstlane(sm.offs[e]);
         int need = 0;
+        const bool same_image = ((other ^ wave) & (p.images - 1)) == 0;
         for (int f0 = 0; f0 < e; f0 += 4 * 64) {   // (uniform; four reads at a time)
           int d[4];
 #pragma unroll
@@ -457,7 +510,7 @@ struct WindowKernel {
 #pragma unroll
           for (int q = 0; q < 4; q++) {
             const int f = f0 + q * 64 + lane;
-            if (f < e && d[q] < kUnitSpan && d[q] > -kUnitSpan) need = f / kWaves + 1;
+            if (same_image && f < e && d[q] < kUnitSpan && d[q] > -kUnitSpan) need = f / kWaves + 1;
           }
         }
         return need;
@@ -466,13 +519,13 @@ struct WindowKernel {
       // slices meet its own, and count it
       auto add_tile = [&](int e) {
         const int tile_off = __builtin_amdgcn_readfirstlane(sm.offs[e]);
-        // (need_added: how many units lane l's wavefront, l % kWaves, must have added, see must_be_added: one LDS read per look)
+        // (need_added: how many units lane l's wavefront, `other`, must have added, see must_be_added: one LDS read per look)
         // The wait is bounded: an entry only waits for earlier ones, whose owners wait for still
         // earlier ones, so it ends by itself; should one never be added all the same (a list that
         // is not what this kernel expects), the wavefront gives up after poll_limit looks, marks
         // the window as spoilt and goes on, so that every wavefront reaches the end of the kernel.
         for (int polls = 0;; polls++) {
-          const int added = __hip_atomic_load(&sm.progress[lane % kWaves], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          const int added = __hip_atomic_load(&sm.progress[other], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
           if (!__any(added < need_added)) break;
           if (polls >= p.poll_limit) {   // (uniform)
             if (lane == 0) __hip_atomic_store(&sm.spoilt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -486,7 +539,7 @@ struct WindowKernel {
           // the whole unit lies inside the window (the usual case): no checks, constant offsets
 #pragma unroll
           for (int b = 0; b < BJ; b++) {
-            float* at = win + rel + ((lane >> 5) * 4) * TBN + b * 32 + (lane & 31);
+            float* at = win + image + rel + ((lane >> 5) * 4) * TBN + b * 32 + (lane & 31);
             // (eight elements at a time: 16 wavefronts per compute unit leave few registers)
 #pragma unroll
             for (int half = 0; half < 2; half++) {
@@ -508,7 +561,7 @@ struct WindowKernel {
           // elements outside the window go to a dump slot behind it: no branches, so the reads
           // and the writes of a block go out back to back (the addresses of a lane are distinct;
           // the dump slots are shared between wavefronts, their contents are never used)
-          const int dump = p.window + lane;
+          const int dump = p.images * p.window + lane;
 #pragma unroll
           for (int b = 0; b < BJ; b++) {
             const int base = rel + ((lane >> 5) * 4) * TBN + b * 32 + (lane & 31);
@@ -521,7 +574,7 @@ struct WindowKernel {
               for (int q = 0; q < 8; q++) {
                 const int i = half * 8 + q;
                 const int x = base + ((i >> 2) * 8 + (i & 3)) * TBN;
-                at[q] = (x >= 0 && x < wlen) ? x : dump;
+                at[q] = (x >= 0 && x < wlen) ? image + x : dump;
                 cur[q] = win[at[q]];
               }
 #pragma unroll
@@ -540,7 +593,25 @@ struct WindowKernel {
         constexpr int S = decltype(set)::value;
         // the set freed by the previous item takes the loads of the item kDepth - 1 ahead
         fetch_next(std::integral_constant<int, (S + kDepth - 1) % kDepth>{});
-        if (pg == 0 && pt < my_tiles) need_added = must_be_added(wave + pt * kWaves);   // (uniform)
+        if (pg == 0 && pt < my_tiles) need_added = must_be_added(my_first + pt * kWaves);   // (uniform)
+        if constexpr (PACKED) {
+          if constexpr (k16) {
+#pragma unroll
+            for (int j = 0; j < BJ; j++) acc[0][j] = Mfma<T>::run(px[S], py[S][j], acc[0][j]);
+          } else {
+#pragma unroll
+            for (int g = 0; g < GS; g++)
+#pragma unroll
+              for (int j = 0; j < BJ; j++)
+                acc[0][j] = Mfma<T>::run(__builtin_bit_cast(f32x4_t, px[S])[g], __builtin_bit_cast(f32x4_t, py[S][j])[g], acc[0][j]);
+          }
+          if (pt < my_tiles && ++pg == ngroups) {
+            add_tile(my_first + pt * kWaves);
+            pg = 0;
+            pt++;
+          }
+          return;
+        }
         if constexpr (STAGED) {
           {
             // pieces -> this wavefront's staging area (LDS operations of one wavefront are carried
@@ -554,7 +625,7 @@ struct WindowKernel {
             for (int q = 0; q < BJ; q++) wy[q] = py[S][q];
             if (pg == 0 && !all_whole) {   // (uniform) a new unit
               const int ptc = pt < my_tiles ? pt : my_tiles - 1;
-              const int v = __builtin_amdgcn_readfirstlane(sm.list[wave + ptc * kWaves]);
+              const int v = __builtin_amdgcn_readfirstlane(sm.list[my_first + ptc * kWaves]);
               const int id = v >> ushift, un = v & (units - 1), tk = id / p.tiles_n;
               mult_k0 = tk * p.h.BK + (un / kParts) * 32;
               mult_n0 = (id - tk * p.tiles_n) * TBN + (un % kParts) * UC;
@@ -624,7 +695,7 @@ struct WindowKernel {
                 for (int j = 0; j < BJ; j++) acc[0][j] = Mfma<T>::run(a[g], b[g][j], acc[0][j]);
             }
             if (pt < my_tiles && ++pg == ngroups) {
-              add_tile(wave + pt * kWaves);
+              add_tile(my_first + pt * kWaves);
               pg = 0;
               pt++;
             }
@@ -638,7 +709,7 @@ struct WindowKernel {
 #pragma unroll
             for (int b = 0; b < BJ; b++) acc[a][b] = Mfma<T>::run(fa[S][s][a], fb[S][s][b], acc[a][b]);
         if (pt < my_tiles && ++pg == ngroups) {
-          add_tile(wave + pt * kWaves);
+          add_tile(my_first + pt * kWaves);
           pg = 0;
           pt++;
         }
@@ -677,16 +748,51 @@ struct WindowKernel {
       for (int i = tid; i < wlen; i += kThreads) win[i] = nan;
       __syncthreads();
     }
+    auto value = [&](int i) -> float {
+      float v = win[i];
+      for (int m = 1; m < p.images; m++) v += win[m * p.window + i];
+      return v;
+    };
     if (p.out_f32 || sizeof(T) == 4) {
       float* out = static_cast<float*>(p.dHW) + w0;
-      for (int i = tid; i < wlen; i += kThreads) out[i] = win[i] + (p.accumulate ? out[i] : 0.f);
+      for (int i = tid; i < wlen; i += kThreads) out[i] = value(i) + (p.accumulate ? out[i] : 0.f);
     } else {
       T* out = static_cast<T*>(p.dHW) + w0;
       for (int i = tid; i < wlen; i += kThreads)
-        out[i] = Tr::from_float(win[i] + (p.accumulate ? Tr::to_float(out[i]) : 0.f));
+        out[i] = Tr::from_float(value(i) + (p.accumulate ? Tr::to_float(out[i]) : 0.f));
     }
   }
 };
+
+// X and dY as the fragments of the MFMAs above, for the packed form of the kernel: block by block of 32 columns, group by
+// group of rows (kGroupRows), the 64 lanes' 16 bytes in a row; zeros for rows and columns beyond the matrix, up to
+// whole hashed tiles.  A wavefront makes one fragment; four neighbouring blocks of columns share a workgroup, so that a
+// line of X or dY is read by one compute unit.  Any element alignment, any row pitch.
+//   16-bit: lane l holds rows (l >> 5) * 8 + j, j = 0..7, of column l & 31; fp32: rows 2 j + (l >> 5), j = 0..3.
+template <typename T>
+__global__ __launch_bounds__(256) void window_pack_kernel(WindowParams p, int blocks_x, int blocks_y, int ngroups) {
+  constexpr int kRows = sizeof(T) == 4 ? 8 : 16, VEC = ElemTraits<T>::kVec;
+  typedef typename std::conditional<sizeof(T) == 4, uint32_t, uint16_t>::type Bits;
+  const int lane = threadIdx.x & 63;
+  const int id = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blocks = blocks_x + blocks_y;
+  const int g = id / blocks, b = id - g * blocks;
+  if (g >= ngroups) return;
+  const bool is_x = b < blocks_x;   // (uniform)
+  const int block = is_x ? b : b - blocks_x, cols = is_x ? p.K : p.N;
+  const int64_t ld = is_x ? p.ldx : p.lddy;
+  const Bits* from = static_cast<const Bits*>(is_x ? p.X : p.dY);
+  const int col = block * 32 + (lane & 31), row0 = g * kRows + (lane >> 5) * (sizeof(T) == 4 ? 1 : VEC);
+  u32x4_t v = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int j = 0; j < VEC; j++) {
+    const int row = row0 + (sizeof(T) == 4 ? 2 * j : j);
+    const uint32_t e = col < cols && row < p.M ? (uint32_t)from[(int64_t)row * ld + col] : 0u;
+    if constexpr (sizeof(T) == 4) v[j] = e;
+    else v[j >> 1] |= e << (16 * (j & 1));
+  }
+  *reinterpret_cast<u32x4_t*>(static_cast<char*>(is_x ? p.packed_x : p.packed_y) +
+                              ((int64_t)block * ngroups + g) * kFragBytes + lane * 16) = v;
+}
 
 // dbias[n] = sum over the rows m of dY[m][n].  A workgroup of 1024 threads owns 256 columns; four thread groups each add
 // up every fourth row, then the groups are combined through LDS in a fixed order.  (Two microseconds of work for a few
@@ -711,9 +817,9 @@ __device__ __forceinline__ void window_colsum(const WindowParams& p, int block, 
   }
 }
 
-template <typename T, int TBN, bool STAGED>
-__global__ __launch_bounds__((WindowKernel<T, TBN, STAGED>::kThreads)) void rz_window_kernel(WindowParams p) {
-  typedef WindowKernel<T, TBN, STAGED> K;
+template <typename T, int TBN, int OPERANDS>
+__global__ __launch_bounds__((WindowKernel<T, TBN, OPERANDS>::kThreads)) void rz_window_kernel(WindowParams p) {
+  typedef WindowKernel<T, TBN, OPERANDS> K;
   extern __shared__ __attribute__((aligned(16))) unsigned char rz_window_smem[];
   static_assert(K::kThreads == 4 * kWindowBiasCols && K::kFixedBytes >= sizeof(float) * K::kThreads, "four row groups, whose sums fit the LDS of any window");
   if ((int)blockIdx.x >= p.windows) {   // (uniform)
