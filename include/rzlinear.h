@@ -324,8 +324,9 @@ int rz_weight_grad_planned(const void* X, const void* dY, void* dHW, void* dbias
  * Fills out[8] = { C-tile edge, slices, contracted elements per slice, contracted elements per
  * kernel step, mode, workgroups, workgroups per window of the fold kernel (mode 5; mode 1: 1 if the kernel
  * finishes its own tiles, 0 if a second kernel adds the slices up; else 0), windows of dHW
- * (modes 4 and 5, else 0) } with mode 0 = plain store, 1 = split contraction with
- * fp32 partial planes, 2 = weight-grad through LDS images of dHW, 3 = weight-grad by global
+ * (modes 4 and 5; mode 1: steps of a run, 0 if cut into slices; else 0) } with mode 0 = plain store, 1 = split contraction with
+ * fp32 partial planes (16-bit: in slices, or dealt out to the workgroups in runs of equal length, where slices is
+ * the most parts that a tile has), 2 = weight-grad through LDS images of dHW, 3 = weight-grad by global
  * atomics, 4 = weight-grad by windows of dHW, 5 = weight-grad stored tile by tile and folded
  * into dHW by a second kernel.  RZ_PLAN_TILE_BYTES in flags: out[6] of a mode 5 answer is instead how many
  * bytes a stored element of X^T.dY takes: 4 (fp32), or 2 (the layer's dtype: one more rounding).  For tests of

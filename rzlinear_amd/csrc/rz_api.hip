@@ -317,6 +317,11 @@ static int run_plain_op(int op, int dtype, GemmParams p, const void* bias, void*
     if (sp.splits > 1) {
       if (workspace == nullptr || workspace_bytes < sp.workspace_bytes) return RZ_ERR_WORKSPACE;
       p.partial = (float*)workspace;
+      if (sp.run_steps > 0) {   // (without counters the launch adds a kernel that sums the parts: the same bits)
+        p.finish = tuning.finish != -1 ? finish_counters_for(sp.run_tiles, s) : nullptr;
+        p.bias = bias;
+        return launch_gemm(dtype, op, p, nullptr, &sp, tuning, s) == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;
+      }
       // the slice that arrives last at a tile finishes it (adds the slices in slice order, then the
       // bias: the bits of the second kernel's sum) — unless told otherwise, or out of counters
       p.finish = (tuning.finish != -1 && sp.splits <= finish_slices(sp.tile, p.I, p.J, p.R, dtype_bytes(dtype), tuning)) ? finish_counters_for(tile_count(p.I, p.J, sp.tile), s) : nullptr;
@@ -1037,6 +1042,10 @@ RZ_API int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int
   const int chunk = cut ? sp.r_chunk : R;
   const KernelForm f = kernel_form(op, I, J, R, chunk, sp.tile, tile_count(I, J, sp.tile) * sp.splits, eb, t);
   out[0] = sp.tile; out[1] = sp.splits; out[2] = chunk; out[3] = f.step; out[4] = cut ? 1 : 0;
+  if (sp.run_steps > 0) {
+    out[2] = ((R + 63) / 64 + sp.splits - 1) / sp.splits * 64; out[3] = 64; out[5] = sp.run_groups; out[6] = t.finish != -1 ? 1 : 0; out[7] = sp.run_steps;
+    return RZ_OK;
+  }
   const long long tiles = f.rows == sp.tile ? tile_count(I, J, sp.tile) : (long long)((I + f.rows - 1) / f.rows) * ((J + f.cols - 1) / f.cols);
   out[5] = (int32_t)(tiles * sp.splits);
   out[6] = (cut && t.finish != -1 && sp.splits <= finish_slices(sp.tile, I, J, R, eb, t) && tile_count(I, J, sp.tile) <= (long long)kFinishPerStream) ? 1 : 0;

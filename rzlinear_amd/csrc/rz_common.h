@@ -138,6 +138,9 @@ struct GemmParams {
   int64_t lda, ldb, ldc;
   int tiles_i, tiles_j;
   int r_chunk;        // rows of R handled by one blockIdx.y slice (multiple of the R step)
+  int run_steps;      // forward / input-grad in runs of this many R steps by run_groups workgroups, each of which has
+  int run_rounds;     // run_rounds whole tiles besides; partial then holds [parts][tiles cut][TI * TJ]
+  int run_groups;
   float scale;
   HashParams h;
 };

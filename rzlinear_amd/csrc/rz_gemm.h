@@ -379,23 +379,20 @@ struct GemmKernel {
     return v;
   }
 
-  static __device__ __forceinline__ void run(const GemmParams& p, Smem& sm) {
-    run_item(p, sm, threadIdx.x, blockIdx.x, blockIdx.y, gridDim.x, gridDim.y);
+  // What a workgroup works on: C tile `id` at (ti, tj), rows r_begin .. r_end of the contracted dimension, which are part `by` of
+  // the tile's `slices`; `run_tile` is the tile's number among those that are cut into runs (run_all).
+  struct Item { int id, ti, tj, by, slices, r_begin, r_end, run_tile; };
+
+  // into how many parts tile t of run_all's is cut: F whole runs of L steps, and its end of r steps, cut where a multiple of L lies
+  // inside t * r .. (t + 1) * r
+  static __device__ __forceinline__ int run_parts(int t, int F, int r, int L) {
+    return r == 0 ? F : F + 1 + (((t + 1) * r - 1) / L * L > t * r ? 1 : 0);
   }
 
-  // One C tile and slice of the contracted dimension, chosen by the workgroup id (bx, by) of a grid of gx x gy.
-  static __device__ __forceinline__ void run_item(const GemmParams& p, Smem& sm, const int tid, int bx, int by, int gx, int gy) {
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // (uniform: lives in a scalar register)
-    const int wave_k = wave / (WI * WJ);                 // which part of every R step
-    const int wave_i = (wave % (WI * WJ)) / WJ, wave_j = wave % WJ;
-    // Offset in the C tile of a wavefront's 32x32 block (a, b).  Forward and input-grad give a
-    // wavefront one contiguous WTI x WTJ sub-tile (whole cache lines per store).  Weight-grad
-    // deals the blocks round-robin instead, so that the blocks of one hashed tile belong to
-    // different wavefronts and its scatter round is shared between them.
-    auto blk_i = [&](int a) -> int { return (OP == kWeightGrad) ? (a * WI + wave_i) * 32 : wave_i * WTI + a * 32; };
-    auto blk_j = [&](int b) -> int { return (OP == kWeightGrad) ? (b * WJ + wave_j) * 32 : wave_j * WTJ + b * 32; };
-
+  // One C tile and slice of the contracted dimension, chosen by the workgroup id.
+  static __device__ __forceinline__ void run(const GemmParams& p, Smem& sm) {
+    const int bx = blockIdx.x, gx = gridDim.x, gy = gridDim.y;
+    int by = blockIdx.y;
     // Workgroup ids are dealt round-robin to the 8 XCDs; renumber so that each XCD (one L2)
     // gets a contiguous run of tiles, then walk tiles with J fastest (forward/input-grad
     // share the streamed A panel) or in square-ish groups (weight-grad streams both).
@@ -427,9 +424,95 @@ struct GemmKernel {
       ti = id / p.tiles_j;
       tj = id % p.tiles_j;
     }
-    const int i0 = ti * TI, j0 = tj * TJ;
     const int r_begin = by * p.r_chunk;
     const int r_end = (r_begin + p.r_chunk) < p.R ? (r_begin + p.r_chunk) : p.R;
+    run_item<0>(p, sm, threadIdx.x, gx, Item{id, ti, tj, by, gy, r_begin, r_end, 0});
+  }
+
+  // Forward / input-grad in runs of p.run_steps R steps: every workgroup takes p.run_rounds whole tiles, and the tiles that are left,
+  // too few for the compute units, are cut so that all workgroups get the same number of steps of them.  Of each such tile whole runs come off
+  // first (the workgroups of an XCD are then at the same place in R of neighbouring tiles); the ends, shorter than a run, are laid behind
+  // one another and cut again, so that a workgroup has pieces of one to a few tiles, and an end is cut at most once.  The parts of a
+  // tile are added up by the one that arrives last (see the epilogue).
+  static __device__ __forceinline__ void run_all(const GemmParams& p, Smem& sm) {
+    const int g = gridDim.x, per = g >> 3, rem = g & 7, x = blockIdx.x & 7;
+    const int id = x * per + (x < rem ? x : rem) + ((int)blockIdx.x >> 3);   // (as in run: a contiguous piece for every XCD)
+    const int first = p.run_rounds * g, tiles = p.tiles_i * p.tiles_j - first;
+    const int steps = (p.R + TR - 1) / TR, L = p.run_steps, F = steps / L, r = steps - F * L, full = tiles * F;
+    int round = 0, at = 0, end = 0;
+    if (id >= full) {
+      at = (id - full) * L;
+      end = at + L < tiles * r ? at + L : tiles * r;
+    }
+    bool whole_run = id < full, again = false;
+    for (;;) {
+      Item it;
+      int s0, n;
+      if (round < p.run_rounds) {
+        it.id = round++ * g + id;
+        it.by = 0; it.slices = 1; it.run_tile = 0;
+        s0 = 0; n = steps;
+      } else {
+        int t;
+        if (whole_run) {
+          whole_run = false;
+          it.by = id / tiles;
+          t = id - it.by * tiles;
+          s0 = it.by * L; n = L;
+        } else if (at < end) {
+          t = at / r;
+          const int o = at - t * r;
+          n = r - o < end - at ? r - o : end - at;
+          s0 = F * L + o;
+          it.by = F + (o > 0 ? 1 : 0);
+          at += n;
+        } else {
+          break;
+        }
+        it.id = first + t;
+        it.run_tile = t;
+        it.slices = run_parts(t, F, r, L);
+      }
+      it.ti = it.id / p.tiles_j;
+      it.tj = it.id - it.ti * p.tiles_j;
+      it.r_begin = s0 * TR;
+      it.r_end = (s0 + n) * TR < p.R ? (s0 + n) * TR : p.R;
+      if (again) __syncthreads();   // (every wavefront is done with the stages and the offset table)
+      again = true;
+      run_item<1>(p, sm, threadIdx.x, g, it);
+    }
+  }
+
+  // ... and where no counters are to be had: the parts of tile blockIdx.x of those that were cut, added up by a kernel of its own.
+  static __device__ __forceinline__ void finish_runs(const GemmParams& p, Smem& sm) {
+    const int t = blockIdx.x, steps = (p.R + TR - 1) / TR, L = p.run_steps, F = steps / L;
+    Item it;
+    it.run_tile = t;
+    it.id = p.run_rounds * p.run_groups + t;
+    it.ti = it.id / p.tiles_j;
+    it.tj = it.id - it.ti * p.tiles_j;
+    it.by = -1;
+    it.slices = run_parts(t, F, steps - F * L, L);
+    it.r_begin = it.r_end = 0;
+    run_item<2>(p, sm, threadIdx.x, p.run_groups, it);
+  }
+
+  // RUNS: 1 a part of run_all, 2 the parts' sum alone
+  template <int RUNS>
+  static __device__ __forceinline__ void run_item(const GemmParams& p, Smem& sm, const int tid, const int gx, const Item& it) {
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // (uniform: lives in a scalar register)
+    const int wave_k = wave / (WI * WJ);                 // which part of every R step
+    const int wave_i = (wave % (WI * WJ)) / WJ, wave_j = wave % WJ;
+    // Offset in the C tile of a wavefront's 32x32 block (a, b).  Forward and input-grad give a
+    // wavefront one contiguous WTI x WTJ sub-tile (whole cache lines per store).  Weight-grad
+    // deals the blocks round-robin instead, so that the blocks of one hashed tile belong to
+    // different wavefronts and its scatter round is shared between them.
+    auto blk_i = [&](int a) -> int { return (OP == kWeightGrad) ? (a * WI + wave_i) * 32 : wave_i * WTI + a * 32; };
+    auto blk_j = [&](int b) -> int { return (OP == kWeightGrad) ? (b * WJ + wave_j) * 32 : wave_j * WTJ + b * 32; };
+
+    const int id = it.id, ti = it.ti, tj = it.tj, by = it.by, r_begin = it.r_begin, r_end = it.r_end;
+    const int i0 = ti * TI, j0 = tj * TJ;
     const int steps = (r_end - r_begin + TR - 1) / TR;
 
     const T* __restrict__ gA = static_cast<const T*>(p.A);
@@ -1667,7 +1750,86 @@ struct GemmKernel {
         bias[b] = 0.f;
         if (gBias != nullptr && (FULL || col < p.J)) bias[b] = Tr::to_float(gBias[col]);
       }
-      if (p.partial != nullptr) {
+      if constexpr (RUNS != 0) {
+        // The parts of a tile that was cut go to planes of TI x TJ floats in the order of the registers, two to a lane and store;
+        // the last to arrive adds them up in the order of R, its own from its registers.  A part that finds all others there
+        // already stores no plane.  What bounds this is the planes' way through memory, 256 KB each for the 256 tile: sixteen bytes
+        // to a lane, or a block's loads ahead of the sums of the block before it, were no faster and cost spilled registers.
+        if (it.slices > 1) {   // (uniform)
+          constexpr int kPairs = MI * MJ * 8;
+          static_assert(WK == 1 && kElems == 16, "all sixteen elements of a block");
+          const size_t plane = (size_t)(TI * TJ / 2) * (size_t)(p.tiles_i * p.tiles_j - p.run_rounds * gx);
+          uint64_t* const at = reinterpret_cast<uint64_t*>(p.partial) + (size_t)it.run_tile * (TI * TJ / 2) + (size_t)wave * (kPairs * 64) + lane;
+          unsigned* counter = p.finish + it.run_tile;
+          int* arrived = sm.off;   // (the offsets are no longer read)
+          if constexpr (RUNS == 1) {
+            const bool finishing = p.finish != nullptr;   // (uniform)
+            bool last = false;
+            if (finishing) {
+              __syncthreads();   // (... by any wavefront)
+              if (tid == 0) *arrived = (int)__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              __syncthreads();
+              last = *arrived == it.slices - 1;
+            }
+            if (!last) {
+#pragma unroll
+              for (int a = 0; a < MI; a++)
+#pragma unroll
+                for (int b = 0; b < MJ; b++)
+#pragma unroll
+                  for (int e = 0; e < 16; e += 2) {
+                    const float v0 = acc[a][b][e] * p.scale, v1 = acc[a][b][e + 1] * p.scale;
+                    const uint64_t v = (uint64_t)__builtin_bit_cast(uint32_t, v1) << 32 | __builtin_bit_cast(uint32_t, v0);
+                    __hip_atomic_store(at + (size_t)by * plane + ((a * MJ + b) * 8 + e / 2) * 64, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                  }
+              if (!finishing) return;
+              asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part of the plane is where the others will look
+              __syncthreads();
+              if (tid == 0) *arrived = (int)__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              __syncthreads();
+              if (*arrived != it.slices - 1) return;   // (uniform) another part will finish this tile
+            }
+            if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // (as the next launch expects it)
+          }
+#pragma unroll
+          for (int a = 0; a < MI; a++) {
+#pragma unroll
+            for (int b = 0; b < MJ; b++) {
+              // (half a block at a time: see below)
+#pragma unroll
+              for (int h = 0; h < 2; h++) {
+                uint64_t v[kFinishSlices][4];
+#pragma unroll
+                for (int sl = 0; sl < kFinishSlices; sl++) {
+                  if (sl < it.slices && sl != by) {   // (uniform)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                      v[sl][e] = __hip_atomic_load(at + (size_t)sl * plane + ((a * MJ + b) * 8 + h * 4 + e) * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                  }
+                }
+                float sum[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) sum[e] = 0.f;
+#pragma unroll
+                for (int sl = 0; sl < kFinishSlices; sl++) {
+                  if (sl == by) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) sum[e] = add_product(sum[e], acc[a][b][h * 8 + e], p.scale);   // (the product as it was stored)
+                  } else if (sl < it.slices) {
+#pragma unroll
+                    for (int e = 0; e < 8; e++) sum[e] += __builtin_bit_cast(float, (uint32_t)(v[sl][e / 2] >> (e & 1 ? 32 : 0)));
+                  }
+                }
+#pragma unroll
+                for (int e = 0; e < 8; e++) acc[a][b][h * 8 + e] = sum[e] + bias[b];
+              }
+            }
+          }
+          out_scale = 1.f;
+#pragma unroll
+          for (int b = 0; b < MJ; b++) bias[b] = 0.f;
+        }
+      } else if (p.partial != nullptr) {
         // R is split over the slices `by` (few C tiles, long R): this slice's scaled fp32 partial
         // result goes to its own [I][J] plane.  The planes are added up by a second kernel — or,
         // with a counter per C tile (p.finish), by the slice that arrives at the tile last: it
@@ -1692,7 +1854,7 @@ struct GemmKernel {
           }
         }
         if (!finishing) return;
-        const int slices = (int)gridDim.y;
+        const int slices = it.slices;
         unsigned* counter = p.finish + (size_t)ti * (size_t)p.tiles_j + tj;
         int* arrived = sm.off;   // (the offsets are no longer read)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part of the plane is where the others will look
@@ -1807,6 +1969,16 @@ __global__ __launch_bounds__(64 * WI * WJ * WK, gemm_waves_per_simd(WI * WJ * WK
   typedef GemmKernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK, SHORT> K;
   extern __shared__ __attribute__((aligned(16))) unsigned char rz_smem_raw[];
   K::run(p, *reinterpret_cast<typename K::Smem*>(rz_smem_raw));
+}
+
+// Forward / input-grad in runs of equal length (GemmKernel::run_all), and the kernel that adds a tile's parts up where that one could not.
+template <typename T, int OP, int TI, int TJ, int WI, int WJ, int NSTAGE, bool FULL, bool CLAMP, bool FINISH>
+__global__ __launch_bounds__(64 * WI * WJ, gemm_waves_per_simd(WI * WJ, NSTAGE)) void rz_gemm_runs_kernel(GemmParams p) {
+  typedef GemmKernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, false, CLAMP> K;
+  extern __shared__ __attribute__((aligned(16))) unsigned char rz_smem_raw[];
+  typename K::Smem& sm = *reinterpret_cast<typename K::Smem*>(rz_smem_raw);
+  if constexpr (FINISH) K::finish_runs(p, sm);
+  else K::run_all(p, sm);
 }
 
 }  // namespace rz

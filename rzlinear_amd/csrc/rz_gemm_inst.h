@@ -144,9 +144,46 @@ static hipError_t launch_op(GemmParams p, const WeightGradPlan* plan, const Spli
 //        16-bit forward / input-grad of at most 32 rows: 32 x 128 (eight wavefronts of 32 x 32 in two groups
 //        that share every R step, three LDS stages)
 //    32:  32 x  64 (fp32 forward / input-grad whose rows would leave a 64-row tile at most half full): four wavefronts of 32 x 32 in two such groups
+// 16-bit forward / input-grad in runs (plan_runs), and without counters the kernel that adds the parts up.
+template <typename T, int OP, int TJ, int WI, int WJ, int NSTAGE, bool FULL>
+static hipError_t launch_runs_form(const GemmParams& p, const SplitPlan& plan, hipStream_t stream) {
+  typedef GemmKernel<T, OP, 256, TJ, WI, WJ, NSTAGE, FULL, false, !FULL> K;
+  static std::atomic<uint64_t> lds_limit_raised{0}, lds_limit_raised_finish{0};
+  auto kernel = rz_gemm_runs_kernel<T, OP, 256, TJ, WI, WJ, NSTAGE, FULL, !FULL, false>;
+  auto finish = rz_gemm_runs_kernel<T, OP, 256, TJ, WI, WJ, NSTAGE, FULL, !FULL, true>;
+  const size_t smem = sizeof(typename K::Smem);
+  hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds_limit_raised);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)plan.run_groups), dim3(K::kThreads), smem, stream, p);
+  e = hipGetLastError();
+  if (e != hipSuccess || p.finish != nullptr) return e;
+  e = raise_lds_limit(reinterpret_cast<const void*>(finish), lds_limit_raised_finish);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(finish, dim3((unsigned)plan.run_tiles), dim3(K::kThreads), smem, stream, p);
+  return hipGetLastError();
+}
+
+template <typename T, int OP, int TJ, int WI, int WJ, int NSTAGE>
+static hipError_t launch_runs(GemmParams p, const SplitPlan& plan, hipStream_t stream) {
+  p.tiles_i = (p.I + 255) / 256;
+  p.tiles_j = (p.J + TJ - 1) / TJ;
+  p.run_steps = plan.run_steps;
+  p.run_rounds = plan.run_rounds;
+  p.run_groups = plan.run_groups;
+  if (p.partial == nullptr || plan.splits > kFinishSlices || plan.run_tiles < 1 || plan.run_tiles > kComputeUnits ||
+      (long long)plan.run_rounds * plan.run_groups + plan.run_tiles != (long long)p.tiles_i * p.tiles_j)
+    return hipErrorInvalidValue;
+  if (p.I % 256 == 0 && p.J % TJ == 0 && p.R % 64 == 0) return launch_runs_form<T, OP, TJ, WI, WJ, NSTAGE, true>(p, plan, stream);
+  return launch_runs_form<T, OP, TJ, WI, WJ, NSTAGE, false>(p, plan, stream);
+}
+
 template <typename T, int OP>
 static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
                                 const rz_tuning& tuning, hipStream_t stream) {
+  if constexpr (sizeof(T) == 2 && OP != kWeightGrad) if (split != nullptr && split->run_steps > 0) {
+    if (split->tile == 256) return launch_runs<T, OP, 256, 2, 4, 2>(p, *split, stream);
+    return launch_runs<T, OP, 128, 4, 2, 3>(p, *split, stream);
+  }
   const bool wg = OP == kWeightGrad && plan != nullptr;
   const bool cut = !wg && split != nullptr && split->splits > 1;
   const int tile = wg ? plan->tile : (split != nullptr ? split->tile : pick_tile(p.I, p.J, (int)sizeof(T), tuning));

