@@ -373,6 +373,20 @@ int rz_adam_step(void* param, const void* grad, float* exp_avg, float* exp_avg_s
                  int param_dtype, int grad_dtype, float lr, float beta1, float beta2, float eps,
                  float weight_decay, int decoupled, int step, float grad_scale, void* stream);
 
+/* rz_adam_step of `count` tensors at the same step, in order, in as few launches as their memory allows (tensors that
+ * overlap one another go apart).  An invalid tensor ends the call with its status; those before it are updated. */
+typedef struct rz_adam_tensor {
+  void* param;
+  const void* grad;
+  float* exp_avg;
+  float* exp_avg_sq;
+  float* master;          /* or NULL */
+  int64_t n;
+  int64_t param_dtype, grad_dtype;
+} rz_adam_tensor;
+int rz_adam_step_many(const rz_adam_tensor* tensors, int count, float lr, float beta1, float beta2, float eps,
+                      float weight_decay, int decoupled, int step, float grad_scale, void* stream);
+
 /*
  * Measurement aid, no counterpart in the reference: the MFMA rate this GPU sustains on the
  * matrix work of the contraction kernels' inner loop when nothing else is in the way.  Launches

@@ -24,7 +24,7 @@ EXPORTS = (
     "rz_forward_hashed_workspace_bytes", "rz_input_grad_hashed_workspace_bytes",
     "rz_weight_grad_hashed_workspace_bytes", "rz_plan_query", "rz_weight_grad_static",
     "rz_layer_plan_bytes", "rz_layer_plan_build", "rz_weight_grad_planned",
-    "rz_sgd_step", "rz_adam_step", "rz_mfma_probe",
+    "rz_sgd_step", "rz_adam_step", "rz_adam_step_many", "rz_mfma_probe",
 )
 
 
@@ -172,6 +172,8 @@ def load():
     f32p = c_vp
     lib.rz_sgd_step.restype = c_int
     lib.rz_sgd_step.argtypes = [c_vp, c_vp, f32p, f32p, c_i64, c_int, c_int, c_f, c_f, c_f, c_f, c_int, c_int, c_f, c_vp]
+    lib.rz_adam_step_many.restype = c_int
+    lib.rz_adam_step_many.argtypes = [c_vp, c_int, c_f, c_f, c_f, c_f, c_f, c_int, c_int, c_f, c_vp]
     lib.rz_adam_step.restype = c_int
     lib.rz_adam_step.argtypes = [c_vp, c_vp, f32p, f32p, f32p, c_i64, c_int, c_int, c_f, c_f, c_f, c_f, c_f, c_int,
                                  c_int, c_f, c_vp]

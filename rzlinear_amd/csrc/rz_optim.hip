@@ -43,10 +43,10 @@ __global__ __launch_bounds__(256) void sgd_step_kernel(P* __restrict__ param, co
 }
 
 template <typename P, typename G>
-__global__ __launch_bounds__(256) void adam_step_kernel(P* __restrict__ param, const G* __restrict__ grad,
-                                                        float* __restrict__ exp_avg, float* __restrict__ exp_avg_sq,
-                                                        float* __restrict__ master, int64_t n, AdamArgs a) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+__device__ __forceinline__ void adam_step(P* __restrict__ param, const G* __restrict__ grad,
+                                          float* __restrict__ exp_avg, float* __restrict__ exp_avg_sq,
+                                          float* __restrict__ master, int64_t n, const AdamArgs& a, int block, int blocks) {
+  for (int64_t i = (int64_t)block * blockDim.x + threadIdx.x; i < n; i += (int64_t)blocks * blockDim.x) {
     float w = master != nullptr ? master[i] : ElemTraits<P>::to_float(param[i]);
     float g = ElemTraits<G>::to_float(grad[i]) * a.grad_scale;
     if (a.weight_decay != 0.f) {
@@ -62,6 +62,33 @@ __global__ __launch_bounds__(256) void adam_step_kernel(P* __restrict__ param, c
     if (master != nullptr) master[i] = w;
     param[i] = ElemTraits<P>::from_float(w);
   }
+}
+
+// The tensors of one launch: a parameter of a few hundred or thousand elements (a bias) beside a hashed_weight costs a launch of 2.4 to
+// 3 us by itself, of which the work is next to nothing; here it is a few more workgroups.
+static constexpr int kAdamTensors = 24;
+struct AdamTensors {
+  rz_adam_tensor t[kAdamTensors];
+  int first_block[kAdamTensors + 1];
+  int count;
+};
+
+template <typename P, typename G>
+__device__ __forceinline__ void adam_step_of(const rz_adam_tensor& t, const AdamArgs& a, int block, int blocks) {
+  adam_step((P*)t.param, (const G*)t.grad, t.exp_avg, t.exp_avg_sq, t.master, t.n, a, block, blocks);
+}
+
+__global__ __launch_bounds__(256) void adam_step_kernel(AdamTensors tensors, AdamArgs a) {
+  int i = 0;   // (uniform)
+  while (i + 1 < tensors.count && (int)blockIdx.x >= tensors.first_block[i + 1]) i++;
+  const rz_adam_tensor& t = tensors.t[i];
+  const int first = tensors.first_block[i], block = (int)blockIdx.x - first, blocks = tensors.first_block[i + 1] - first;
+  const bool own = t.grad_dtype == t.param_dtype;
+  if (t.param_dtype == RZ_F32) adam_step_of<float, float>(t, a, block, blocks);
+  else if (t.param_dtype == RZ_BF16 && own) adam_step_of<bf16_t, bf16_t>(t, a, block, blocks);
+  else if (t.param_dtype == RZ_BF16) adam_step_of<bf16_t, float>(t, a, block, blocks);
+  else if (own) adam_step_of<f16_t, f16_t>(t, a, block, blocks);
+  else adam_step_of<f16_t, float>(t, a, block, blocks);
 }
 
 static inline unsigned blocks_for(int64_t n) {
@@ -107,23 +134,62 @@ RZ_API int rz_sgd_step(void* param, const void* grad, float* momentum_buf, float
   });
 }
 
+RZ_API int rz_adam_step_many(const rz_adam_tensor* tensors, int count, float lr, float beta1, float beta2, float eps,
+                             float weight_decay, int decoupled, int step, float grad_scale, void* stream) {
+  if (count < 0) return RZ_ERR_BAD_ARGUMENT;
+  if (count > 0 && tensors == nullptr) return RZ_ERR_NULL_POINTER;
+  int refused = RZ_OK;   // (by the first invalid tensor, at which the call ends)
+  for (int i = 0; i < count && refused == RZ_OK; i++) {
+    const rz_adam_tensor& t = tensors[i];
+    if (t.param == nullptr || t.grad == nullptr || t.exp_avg == nullptr || t.exp_avg_sq == nullptr) refused = RZ_ERR_NULL_POINTER;
+    else if (t.n < 0) refused = RZ_ERR_BAD_SHAPE;
+    else if (t.n > 0) refused = with_types((int)t.param_dtype, (int)t.grad_dtype, [](auto*, auto*) -> int { return RZ_OK; });
+    if (refused != RZ_OK) count = i;
+  }
+  if (refused != RZ_OK && count == 0 && refused != RZ_ERR_BAD_DTYPE) return refused;
+  if (step < 1 || !(beta1 >= 0.f && beta1 < 1.f) || !(beta2 >= 0.f && beta2 < 1.f)) return RZ_ERR_BAD_ARGUMENT;
+  const AdamArgs a = {lr, beta1, beta2, eps, weight_decay, grad_scale,
+                      (float)(1.0 - pow((double)beta1, (double)step)), (float)sqrt(1.0 - pow((double)beta2, (double)step)),
+                      decoupled ? 1 : 0};
+  // whether a later tensor reads or writes what this one writes: they then keep their order, in launches of their own
+  auto meets = [](const rz_adam_tensor& x, const rz_adam_tensor& y) -> bool {
+    auto bytes = [](int64_t dtype) -> int64_t { return dtype == RZ_F32 ? 4 : 2; };
+    const struct { uintptr_t at; int64_t bytes; } wx[4] = {{(uintptr_t)x.param, x.n * bytes(x.param_dtype)}, {(uintptr_t)x.exp_avg, x.n * 4},
+                                                           {(uintptr_t)x.exp_avg_sq, x.n * 4}, {(uintptr_t)x.master, x.master ? x.n * 4 : 0}},
+                                                  wy[5] = {{(uintptr_t)y.param, y.n * bytes(y.param_dtype)}, {(uintptr_t)y.exp_avg, y.n * 4},
+                                                           {(uintptr_t)y.exp_avg_sq, y.n * 4}, {(uintptr_t)y.master, y.master ? y.n * 4 : 0},
+                                                           {(uintptr_t)y.grad, y.n * bytes(y.grad_dtype)}};
+    for (const auto& p : wx)
+      for (const auto& q : wy)
+        if (p.bytes > 0 && q.bytes > 0 && p.at < q.at + (uintptr_t)q.bytes && q.at < p.at + (uintptr_t)p.bytes) return true;
+    return false;
+  };
+  AdamTensors now;
+  now.count = 0;
+  now.first_block[0] = 0;
+  auto launch = [&]() -> bool {
+    if (now.count == 0) return true;
+    hipLaunchKernelGGL(adam_step_kernel, dim3((unsigned)now.first_block[now.count]), dim3(256), 0, (hipStream_t)stream, now, a);
+    now.count = 0;
+    return hipGetLastError() == hipSuccess;
+  };
+  for (int i = 0; i < count; i++) {
+    if (tensors[i].n == 0) continue;
+    bool apart = now.count == kAdamTensors;
+    for (int k = 0; k < now.count && !apart; k++) apart = meets(now.t[k], tensors[i]) || meets(tensors[i], now.t[k]);
+    if (apart && !launch()) return RZ_ERR_LAUNCH;
+    now.t[now.count] = tensors[i];
+    now.first_block[now.count + 1] = now.first_block[now.count] + (int)blocks_for(tensors[i].n);
+    now.count++;
+  }
+  return launch() ? refused : RZ_ERR_LAUNCH;
+}
+
 RZ_API int rz_adam_step(void* param, const void* grad, float* exp_avg, float* exp_avg_sq, float* master, int64_t n,
                         int param_dtype, int grad_dtype, float lr, float beta1, float beta2, float eps,
                         float weight_decay, int decoupled, int step, float grad_scale, void* stream) {
-  if (param == nullptr || grad == nullptr || exp_avg == nullptr || exp_avg_sq == nullptr) return RZ_ERR_NULL_POINTER;
-  if (n < 0) return RZ_ERR_BAD_SHAPE;
-  if (step < 1 || !(beta1 >= 0.f && beta1 < 1.f) || !(beta2 >= 0.f && beta2 < 1.f)) return RZ_ERR_BAD_ARGUMENT;
-  if (n == 0) return RZ_OK;
-  AdamArgs a = {lr, beta1, beta2, eps, weight_decay, grad_scale,
-                (float)(1.0 - pow((double)beta1, (double)step)), (float)sqrt(1.0 - pow((double)beta2, (double)step)),
-                decoupled ? 1 : 0};
-  return with_types(param_dtype, grad_dtype, [&](auto* p, auto* g) -> int {
-    typedef typename std::remove_pointer<decltype(p)>::type P;
-    typedef typename std::remove_pointer<decltype(g)>::type G;
-    hipLaunchKernelGGL((adam_step_kernel<P, G>), dim3(blocks_for(n)), dim3(256), 0, (hipStream_t)stream, (P*)param,
-                       (const G*)grad, exp_avg, exp_avg_sq, master, n, a);
-    return hipGetLastError() == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;
-  });
+  const rz_adam_tensor t = {param, grad, exp_avg, exp_avg_sq, master, n, param_dtype, grad_dtype};
+  return rz_adam_step_many(&t, 1, lr, beta1, beta2, eps, weight_decay, decoupled, step, grad_scale, stream);
 }
 
 }  // extern "C"

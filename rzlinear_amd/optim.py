@@ -1,12 +1,14 @@
 """Fused optimiser steps for RzLinear parameters (``rz_sgd_step`` / ``rz_adam_step``).
 
 The reference leaves the update to ``torch.optim``; these classes apply the same rules
-(``torch.optim.SGD``, ``torch.optim.Adam`` / ``AdamW``) with one kernel per parameter and step.
+(``torch.optim.SGD``, ``torch.optim.Adam`` / ``AdamW``) with one kernel per parameter and step (Adam: per parameter group).
 They read the gradient from ``param.main_grad`` when the parameter has one (the fp32 buffer
 that ``RzLinear(..., fuse_grad_accumulation=True)`` adds into) and from ``param.grad`` otherwise,
 and can keep an fp32 master copy of 16-bit parameters.  Parameters must live on the GPU: there
 is no CPU path.
 """
+import ctypes
+
 import torch
 
 from . import _lib
@@ -84,7 +86,7 @@ class FusedSGD(_Fused):
 
 
 class FusedAdam(_Fused):
-    """``torch.optim.Adam`` (``decoupled_weight_decay=True``: ``AdamW``), amsgrad off, in one kernel per parameter."""
+    """``torch.optim.Adam`` (``decoupled_weight_decay=True``: ``AdamW``), amsgrad off, in one kernel for a group's parameters."""
 
     def __init__(self, params, lr=1e-3, betas=(0.9, 0.999), eps=1e-8, weight_decay=0.0,
                  decoupled_weight_decay=False, master_weights=False, grad_scale=1.0):
@@ -98,24 +100,34 @@ class FusedAdam(_Fused):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
-        lib = _lib.load()
         for group in self.param_groups:
-            for p in group["params"]:
-                g = _gradient(p)
-                if g is None:
-                    continue
-                _check(p, g)
-                state = self.state[p]
-                if "step" not in state:
-                    state["step"] = 0
-                    state["exp_avg"] = torch.zeros(p.shape, dtype=torch.float32, device=p.device)
-                    state["exp_avg_sq"] = torch.zeros(p.shape, dtype=torch.float32, device=p.device)
-                state["step"] += 1
-                b1, b2 = group["betas"]
-                _lib.check(lib.rz_adam_step(p.data_ptr(), g.data_ptr(), state["exp_avg"].data_ptr(),
-                                            state["exp_avg_sq"].data_ptr(), self._master(p, state, group), p.numel(),
-                                            _lib.dtype_code(p), _lib.dtype_code(g), group["lr"], b1, b2, group["eps"],
-                                            group["weight_decay"], int(group["decoupled_weight_decay"]),
-                                            state["step"], group["grad_scale"],
-                                            torch.cuda.current_stream(p.device).cuda_stream))
+            b1, b2 = group["betas"]
+            batches = {}   # (device, step): the words of their struct rz_adam_tensor
+
+            def launch():
+                for (device, step), words in batches.items():
+                    _lib.check(_lib.load().rz_adam_step_many((ctypes.c_int64 * len(words))(*words), len(words) // 8, group["lr"], b1, b2,
+                                                             group["eps"], group["weight_decay"], int(group["decoupled_weight_decay"]),
+                                                             step, group["grad_scale"], torch.cuda.current_stream(device).cuda_stream))
+                batches.clear()
+
+            try:
+                for p in group["params"]:
+                    g = _gradient(p)
+                    if g is None:
+                        continue
+                    _check(p, g)
+                    state = self.state[p]
+                    if "step" not in state:
+                        state["step"] = 0
+                        state["exp_avg"] = torch.zeros(p.shape, dtype=torch.float32, device=p.device)
+                        state["exp_avg_sq"] = torch.zeros(p.shape, dtype=torch.float32, device=p.device)
+                    state["step"] += 1
+                    if group["master_weights"] and p.dtype != torch.float32 and "master" not in state:
+                        launch()   # (a master copy starts from the parameter as the updates before it leave it, which may share its memory)
+                    batches.setdefault((p.device, state["step"]), []).extend(
+                        (p.data_ptr(), g.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(),
+                         self._master(p, state, group) or 0, p.numel(), _lib.dtype_code(p), _lib.dtype_code(g)))
+            finally:   # (a parameter that is refused leaves those before it updated)
+                launch()
         return loss

@@ -124,3 +124,49 @@ def test_layers_sharing_a_parameter_train_with_the_fused_step(oracle):
         oracle.weight_grad(f64(x2), f64(dy2), H, 64, 64, R2, second._init_factor)
     want = before - 0.25 * g
     assert np.abs(f64(hw.detach()) - want).max() <= 1e-4 * np.abs(want).max()
+
+
+def test_one_launch_for_a_groups_parameters_gives_the_bits_of_one_each():
+    """Parameters of every dtype pair and of many sizes — one element, a workgroup's and one more, more tensors than a launch
+    holds — and a parameter that is a view of another, whose updates keep their order."""
+    from rzlinear_amd.optim import FusedAdam
+    gen = torch.Generator().manual_seed(12)
+    base = []
+    for i, n in enumerate([262144, 1024, 1, 255, 256, 257, 70001] + [64 + k for k in range(24)]):
+        dtype = [torch.bfloat16, torch.float32, torch.float16][i % 3]
+        base.append((torch.randn((n,), generator=gen).to(dtype), torch.randn((n,), generator=gen), i % 2 == 0))
+
+    def params():
+        out = []
+        for w, g, wide in base:
+            p = torch.nn.Parameter(w.clone().cuda())
+            if wide:
+                p.main_grad = g.clone().cuda()
+            else:
+                p.grad = g.to(p.dtype).cuda()
+            out.append(p)
+        view = torch.nn.Parameter(out[0].detach()[1000:5000])
+        view.grad = torch.ones_like(view)
+        return out + [view]
+
+    together, alone = params(), params()
+    kw = dict(lr=1e-2, weight_decay=0.1, decoupled_weight_decay=True, master_weights=True)
+    one, each = FusedAdam(together, **kw), [FusedAdam([p], **kw) for p in alone]
+    for _ in range(3):
+        one.step()
+        for o in each:
+            o.step()
+    torch.cuda.synchronize()
+    for a, b in zip(together, alone):
+        assert torch.equal(a.detach(), b.detach())
+
+
+def test_a_refused_parameter_leaves_those_before_it_updated():
+    from rzlinear_amd.optim import FusedAdam
+    a, b = (torch.nn.Parameter(torch.zeros((8, 8), device="cuda")) for _ in range(2))
+    a.grad, b.grad = torch.ones_like(a), torch.ones_like(b)
+    b.main_grad = torch.ones((8, 9), device="cuda")
+    with pytest.raises(RuntimeError):
+        FusedAdam([a, b], lr=0.5).step()
+    torch.cuda.synchronize()
+    assert float(a.detach().max()) < 0 and float(b.detach().abs().max()) == 0
