@@ -130,17 +130,25 @@ struct GemmParams {
                       // at ((s * tiles_k + tk) * tiles_n + tn) * BK*BN (only the part inside K x N is defined), and a
                       // second kernel folds the tiles into dHW
   int tiles_out_16;   // ... as elements of the layer's 16-bit dtype instead of floats (same element indices)
-  int out_tiles_k, out_tiles_n;   // ... its tile grid: ceil(K / BK) x ceil(N / BN)
+  // (unions: the struct keeps its size, which the smallest calls feel: fp32 M = 32, K = N = 1024 7.94 us, 8.08 with twelve bytes more)
+  union {
+    int out_tiles_k;   // ... its tile grid: ceil(K / BK) x ceil(N / BN)
+    int run_rounds;    // forward / input-grad in runs: whole tiles of every workgroup,
+  };
+  union {
+    int out_tiles_n;
+    int run_groups;    // workgroups,
+  };
   float* colsum;      // weight-grad that also yields the bias gradient: partial column sums of B
                       // (dY), one row per (slice, tile row): [slices * tiles_i][colsum_pitch]
-  int colsum_pitch;   // floats per row of colsum (J rounded up to the tile)
+  union {
+    int colsum_pitch;   // floats per row of colsum (J rounded up to the tile)
+    int run_steps;      // and R steps of a run; partial then holds [parts][tiles cut][TI * TJ]
+  };
   int I, J, R;
   int64_t lda, ldb, ldc;
   int tiles_i, tiles_j;
   int r_chunk;        // rows of R handled by one blockIdx.y slice (multiple of the R step)
-  int run_steps;      // forward / input-grad in runs of this many R steps by run_groups workgroups, each of which has
-  int run_rounds;     // run_rounds whole tiles besides; partial then holds [parts][tiles cut][TI * TJ]
-  int run_groups;
   float scale;
   HashParams h;
 };

@@ -1854,7 +1854,7 @@ struct GemmKernel {
           }
         }
         if (!finishing) return;
-        const int slices = it.slices;
+        const int slices = (int)gridDim.y;
         unsigned* counter = p.finish + (size_t)ti * (size_t)p.tiles_j + tj;
         int* arrived = sm.off;   // (the offsets are no longer read)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part of the plane is where the others will look
