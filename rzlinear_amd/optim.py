@@ -102,14 +102,15 @@ class FusedAdam(_Fused):
                 loss = closure()
         for group in self.param_groups:
             b1, b2 = group["betas"]
-            batches = {}   # (device, step): the words of their struct rz_adam_tensor
+            key, words = None, []   # the parameters to be launched next: their device and step, the words of their struct rz_adam_tensor
 
             def launch():
-                for (device, step), words in batches.items():
+                if words:
+                    device, step = key
                     _lib.check(_lib.load().rz_adam_step_many((ctypes.c_int64 * len(words))(*words), len(words) // 8, group["lr"], b1, b2,
                                                              group["eps"], group["weight_decay"], int(group["decoupled_weight_decay"]),
                                                              step, group["grad_scale"], torch.cuda.current_stream(device).cuda_stream))
-                batches.clear()
+                    words.clear()
 
             try:
                 for p in group["params"]:
@@ -123,11 +124,13 @@ class FusedAdam(_Fused):
                         state["exp_avg"] = torch.zeros(p.shape, dtype=torch.float32, device=p.device)
                         state["exp_avg_sq"] = torch.zeros(p.shape, dtype=torch.float32, device=p.device)
                     state["step"] += 1
-                    if group["master_weights"] and p.dtype != torch.float32 and "master" not in state:
-                        launch()   # (a master copy starts from the parameter as the updates before it leave it, which may share its memory)
-                    batches.setdefault((p.device, state["step"]), []).extend(
-                        (p.data_ptr(), g.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(),
-                         self._master(p, state, group) or 0, p.numel(), _lib.dtype_code(p), _lib.dtype_code(g)))
+                    # the group's order is kept (parameters may share memory): another device or step begins a new launch, and a
+                    # master copy starts from the parameter as the updates before it leave it
+                    if key != (p.device, state["step"]) or (group["master_weights"] and p.dtype != torch.float32 and "master" not in state):
+                        launch()
+                        key = (p.device, state["step"])
+                    words.extend((p.data_ptr(), g.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(),
+                                  self._master(p, state, group) or 0, p.numel(), _lib.dtype_code(p), _lib.dtype_code(g)))
             finally:   # (a parameter that is refused leaves those before it updated)
                 launch()
         return loss

@@ -170,3 +170,31 @@ def test_a_refused_parameter_leaves_those_before_it_updated():
         FusedAdam([a, b], lr=0.5).step()
     torch.cuda.synchronize()
     assert float(a.detach().max()) < 0 and float(b.detach().abs().max()) == 0
+
+
+def test_a_parameter_that_skipped_a_step_keeps_its_place():
+    """A, B and C, a view of B, each with an fp32 master copy, so that whoever writes the shared memory last decides it: the group's
+    order holds although B is a step behind."""
+    from rzlinear_amd.optim import FusedAdam
+
+    def params():
+        gen = torch.Generator().manual_seed(3)
+        a, b = (torch.nn.Parameter(torch.randn((512,), generator=gen).to(torch.bfloat16).cuda()) for _ in range(2))
+        c = torch.nn.Parameter(b.detach()[100:300])
+        for p in (a, b, c):
+            p.grad = torch.randn(p.shape, generator=gen).to(torch.bfloat16).cuda()
+        return [a, b, c]
+
+    together, alone = params(), params()
+    kw = dict(lr=1e-1, master_weights=True)
+    one, each = FusedAdam(together, **kw), [FusedAdam([p], **kw) for p in alone]
+    grads = [ps[1].grad for ps in (together, alone)]
+    for step in range(3):
+        for ps, g in zip((together, alone), grads):
+            ps[1].grad = None if step == 0 else g
+        one.step()
+        for o in each:
+            o.step()
+    torch.cuda.synchronize()
+    for a, b in zip(together, alone):
+        assert torch.equal(a.detach(), b.detach())
