@@ -102,7 +102,9 @@ class FusedAdam(_Fused):
                 loss = closure()
         for group in self.param_groups:
             b1, b2 = group["betas"]
-            key, words = None, []   # the parameters to be launched next: their device and step, the words of their struct rz_adam_tensor
+            # the parameters to be launched next: their device and step, the words of their struct rz_adam_tensor, and their gradients,
+            # held until the launch (a main_grad that is made when it is asked for has no other owner)
+            key, words, held = None, [], []
 
             def launch():
                 if words:
@@ -111,6 +113,7 @@ class FusedAdam(_Fused):
                                                              group["eps"], group["weight_decay"], int(group["decoupled_weight_decay"]),
                                                              step, group["grad_scale"], torch.cuda.current_stream(device).cuda_stream))
                     words.clear()
+                    held.clear()
 
             try:
                 for p in group["params"]:
@@ -129,6 +132,7 @@ class FusedAdam(_Fused):
                     if key != (p.device, state["step"]) or (group["master_weights"] and p.dtype != torch.float32 and "master" not in state):
                         launch()
                         key = (p.device, state["step"])
+                    held.append(g)
                     words.extend((p.data_ptr(), g.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(),
                                   self._master(p, state, group) or 0, p.numel(), _lib.dtype_code(p), _lib.dtype_code(g)))
             finally:   # (a parameter that is refused leaves those before it updated)

@@ -1,5 +1,5 @@
 """What FusedAdam hands to rz_adam_step_many, and when: a stand-in for the library records the launches (no GPU)."""
-import ctypes
+import weakref
 
 import pytest
 import torch
@@ -61,3 +61,29 @@ def test_parameters_of_unequal_steps_keep_the_groups_order(library):
     opt.step()
     assert [p for launch in library.order() for p in launch] == [a.data_ptr(), b.data_ptr(), c.data_ptr()]
     assert [step for step, words in library.launches for _ in words] == [2, 1, 2]
+
+
+class _MadeWhenAsked(torch.nn.Parameter):
+    """A parameter whose main_grad has no owner but who asked for it."""
+
+    @property
+    def main_grad(self):
+        g = torch.ones(self.shape)
+        self.freed = []
+        weakref.finalize(g, self.freed.append, True)
+        return g
+
+
+def test_a_gradient_is_held_until_its_launch(library):
+    params = [_MadeWhenAsked(torch.zeros(16)) for _ in range(3)]
+    launch = library.rz_adam_step_many
+    alive = []
+
+    def look(*args):
+        alive.extend(not p.freed for p in params)
+        return launch(*args)
+
+    library.rz_adam_step_many = look
+    optim.FusedAdam(params).step()
+    assert alive == [True] * 3
+    assert all(p.freed for p in params)   # (and no longer)
