@@ -109,10 +109,11 @@ class FusedAdam(_Fused):
             def launch():
                 if words:
                     device, step = key
-                    _lib.check(_lib.load().rz_adam_step_many((ctypes.c_int64 * len(words))(*words), len(words) // 8, group["lr"], b1, b2,
+                    tensors = (ctypes.c_int64 * len(words))(*words)
+                    words.clear()   # (whatever becomes of the launch, it is not made again)
+                    _lib.check(_lib.load().rz_adam_step_many(tensors, len(tensors) // 8, group["lr"], b1, b2,
                                                              group["eps"], group["weight_decay"], int(group["decoupled_weight_decay"]),
                                                              step, group["grad_scale"], torch.cuda.current_stream(device).cuda_stream))
-                    words.clear()
                     held.clear()
 
             try:

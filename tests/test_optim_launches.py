@@ -87,3 +87,13 @@ def test_a_gradient_is_held_until_its_launch(library):
     optim.FusedAdam(params).step()
     assert alive == [True] * 3
     assert all(p.freed for p in params)   # (and no longer)
+
+
+def test_a_launch_that_failed_is_not_made_again(library):
+    """The second parameter's master copy forces a launch of the first; it fails, and its error is the one that is seen."""
+    a, b = _params(2, torch.bfloat16)
+    opt = optim.FusedAdam([a, b], master_weights=True)
+    library.fail_at = 0
+    with pytest.raises(_lib.RzLinearError, match="refused by the stand-in") as e:
+        opt.step()
+    assert library.launches == [] and e.value.__context__ is None
