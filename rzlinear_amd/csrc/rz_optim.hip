@@ -143,6 +143,7 @@ RZ_API int rz_adam_step_many(const rz_adam_tensor* tensors, int count, float lr,
     const rz_adam_tensor& t = tensors[i];
     if (t.param == nullptr || t.grad == nullptr || t.exp_avg == nullptr || t.exp_avg_sq == nullptr) refused = RZ_ERR_NULL_POINTER;
     else if (t.n < 0) refused = RZ_ERR_BAD_SHAPE;
+    else if (t.n > 0 && (t.param_dtype != (int)t.param_dtype || t.grad_dtype != (int)t.grad_dtype)) refused = RZ_ERR_BAD_DTYPE;   // (the kernel looks at all 64 bits)
     else if (t.n > 0) refused = with_types((int)t.param_dtype, (int)t.grad_dtype, [](auto*, auto*) -> int { return RZ_OK; });
     if (refused != RZ_OK) count = i;
   }

@@ -295,3 +295,15 @@ def test_layer_plan_argument_checks(lib):
                                       _R(R1024), 2, 1.0, 1024, 1024, 0, 0, None, None) != 0
     assert lib.rz_weight_grad_planned(1, 1, 1, None, None, 0, None, n, 32, 1024, 1024, 65536, 64, 64,
                                       _R(R1024), 2, 1.0, 1024, 1024, 0, 0, None, None) != 0
+
+
+def test_adam_step_many_looks_at_the_whole_dtype_word():
+    """A word that is a valid code only when cut to 32 bits is refused, as the kernel would see all of it."""
+    import ctypes
+    from rzlinear_amd import _lib
+    lib = _lib.load()
+    buf = (ctypes.c_float * 64)()
+    at = ctypes.addressof(buf)
+    for dtypes in ((1 << 32, 0), (0, 1 << 32), (1 << 32, 1 << 32), ((1 << 33) | _lib.RZ_BF16, _lib.RZ_F32), (-(1 << 32), -(1 << 32))):
+        words = (ctypes.c_int64 * 8)(at, at, at, at, 0, 16, *dtypes)
+        assert lib.rz_adam_step_many(words, 1, 1e-3, 0.9, 0.999, 1e-8, 0.0, 0, 1, 1.0, None) == -5, dtypes   # RZ_ERR_BAD_DTYPE
