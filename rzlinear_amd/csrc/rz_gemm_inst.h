@@ -225,12 +225,12 @@ static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const 
 template <typename T, int TBN, int OPERANDS>
 static hipError_t launch_window_form(WindowParams p, int windows, hipStream_t stream) {
   typedef WindowKernel<T, TBN, OPERANDS> K;
-  static_assert(K::kImageFloats >= kWindowFloats, "window does not fit the LDS");
+  static_assert(K::kFixedBytes + sizeof(float) * kWindowFloats <= 160 * 1024, "the images of a window do not fit the LDS");
   if (p.window < 4 || p.window > kWindowFloats || (p.window & 3) || windows < 1) return hipErrorInvalidValue;
   if ((long long)windows * p.window < p.H) return hipErrorInvalidValue;
   if (p.h.BN != TBN || !window_tile_supported(p.h.BK, p.h.BN)) return hipErrorInvalidValue;
   auto kernel = rz_window_kernel<T, TBN, OPERANDS>;
-  p.images = window_images(p.window, OPERANDS == kPacked);
+  p.images = window_images(p.window);
   const size_t smem = K::kFixedBytes + sizeof(float) * (size_t)p.window * p.images;
   static std::atomic<uint64_t> lds_limit_raised{0};
   if (smem > 64 * 1024) {

@@ -610,11 +610,11 @@ static inline void window_geometry(int H, int* window, int* windows) {
 // Images of a window that a workgroup keeps in LDS, a power of two up to its sixteen wavefronts.  With a small window nearly every
 // unit meets the one before it in the list, and the chain of adds takes most of the time; with images a unit waits for those of
 // its own image only (bf16, windows of 4096: M = 16, K = 2048, N = 8192 35.6 -> 20 us, M = 64, K = N = 4096 39.4 -> 24.7;
-// windows of 1024: M = 32, K = N = 2048 37 -> 15.5).  The packed form has no staging area, so that half as much again fits.
-constexpr int window_image_floats(bool packed) { return packed ? kWindowFloats * 3 / 2 : kWindowFloats; }
-static inline int window_images(int window, bool packed) {
+// windows of 1024: M = 32, K = N = 2048 37 -> 15.5).  A function of the window alone: the packed form, which has no staging area, would have
+// room for half as many again, but the order of the sums, and with it the bits of dHW, would then depend on the workspace that the caller has.
+static inline int window_images(int window) {
   int n = 1;
-  while (n < 16 && 2 * n * window <= window_image_floats(packed)) n *= 2;
+  while (n < 16 && 2 * n * window <= kWindowFloats) n *= 2;
   return n;
 }
 
@@ -641,7 +641,7 @@ static inline double window_us(int M, int K, int N, int H, int BK, int BN, int e
   const double rounds = (double)((windows + kComputeUnits - 1) / kComputeUnits);
   const double chunks = M > 16 ? M / 32.0 : 0.5, mb = (double)M * ((double)K + N) * elem_bytes * 1e-6;
   const double work_us = rounds * units * (f.unit + chunks * (f.rows + (mb > 4.3 ? f.misses * (1.0 - 4.3 / mb) : 0.0)));
-  const double chain_us = f.link * (double)K * N / (double)H / window_images(window, packed);
+  const double chain_us = f.link * (double)K * N / (double)H / window_images(window);
   return f.fixed + f.per_mb * mb + (work_us > chain_us ? work_us + f.rest * chain_us : chain_us + f.rest * work_us);
 }
 

@@ -126,9 +126,6 @@ struct WindowKernel {
                                   // dump slots
   };
   static constexpr size_t kFixedBytes = offsetof(Smem, window) + sizeof(float) * 64;   // + dump slots
-  // Floats for images of the window (see window_images in rz_launch.h)
-  static constexpr int kImageFloats = window_image_floats(PACKED);
-  static_assert(kFixedBytes + sizeof(float) * kImageFloats <= 160 * 1024, "the images do not fit the LDS");
 
   // MFMA fragment of a 32-wide block of a row-major matrix (rows = the contracted dimension M).
   //   16-bit: lane l holds rows m0 + r0 + (l >> 5) * 8 + j, j = 0..7, of column (l & 31)

@@ -97,3 +97,31 @@ def test_workspace_query_has_room_for_the_fragments_of_a_planned_call():
                 need = lib.rz_weight_grad_hashed_workspace_bytes(M, K, N, H, 64, 64, code, 0, 0, None)
                 assert need >= (M + 15) // 16 * 16 * (K + N) * 2, (M, K, N)
     assert differ > 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("shape", [
+    (31, 4096, 4100, 3300000, 64, 64),   # windows of 12892: two images would fit beside the fragments, one beside the staging area
+    (20, 2100, 4096, 1664000, 32, 64),   # ... of 6500: four and two
+    (64, 1001, 3333, 1100000, 64, 128),  # ... of 4300: eight and four; element by element without the fragments
+    (40, 2048, 2048, 262144, 32, 32),    # ... of 1024: sixteen either way
+], ids=lambda s: "x".join(map(str, s)))
+def test_the_bits_do_not_depend_on_the_workspace(shape, dtype):
+    """The same order of the sums with the operands as fragments, and without room for them."""
+    from rzlinear_amd import _lib
+    M, K, N, H, BK, BN = shape
+    print("window bits", shape, dtype, flush=True)
+    (x, _, dy), _ = make_inputs(M, K, N, H, dtype, seed=6)
+    lib = _lib.load()
+    code = _lib.dtype_code(x)
+    t = _lib.Tuning(window=1)
+    tuning = ctypes.byref(t)
+    need = lib.rz_weight_grad_hashed_workspace_bytes(M, K, N, H, BK, BN, code, 0, 0, tuning)
+    ws = torch.empty((need,), dtype=torch.uint8, device=x.device)
+    plan = _lib.layer_plan(K, N, H, BK, BN, _lib.hash_constants(*rargs(R1024)), 2, x.device)
+    got = []
+    for at, nbytes, p in ((ws.data_ptr(), need, None), (ws.data_ptr(), need, plan), (None, 0, plan)):
+        out = torch.full((H,), float("nan"), dtype=dtype, device=x.device)
+        _call(lib, x, dy, out, at, nbytes, p, shape, code, tuning)
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
