@@ -745,18 +745,25 @@ struct WindowKernel {
       for (int i = tid; i < wlen; i += kThreads) win[i] = nan;
       __syncthreads();
     }
-    auto value = [&](int i) -> float {
-      float v = win[i];
-      for (int m = 1; m < p.images; m++) v += win[m * p.window + i];
-      return v;
+    // (one image: no loop over images in the loop over elements, which the compiler could then not unroll: 1 us per window)
+    auto store = [&](auto&& value) {
+      if (p.out_f32 || sizeof(T) == 4) {
+        float* out = static_cast<float*>(p.dHW) + w0;
+        for (int i = tid; i < wlen; i += kThreads) out[i] = value(i) + (p.accumulate ? out[i] : 0.f);
+      } else {
+        T* out = static_cast<T*>(p.dHW) + w0;
+        for (int i = tid; i < wlen; i += kThreads)
+          out[i] = Tr::from_float(value(i) + (p.accumulate ? Tr::to_float(out[i]) : 0.f));
+      }
     };
-    if (p.out_f32 || sizeof(T) == 4) {
-      float* out = static_cast<float*>(p.dHW) + w0;
-      for (int i = tid; i < wlen; i += kThreads) out[i] = value(i) + (p.accumulate ? out[i] : 0.f);
+    if (p.images == 1) {   // (uniform)
+      store([&](int i) -> float { return win[i]; });
     } else {
-      T* out = static_cast<T*>(p.dHW) + w0;
-      for (int i = tid; i < wlen; i += kThreads)
-        out[i] = Tr::from_float(value(i) + (p.accumulate ? Tr::to_float(out[i]) : 0.f));
+      store([&](int i) -> float {
+        float v = win[i];
+        for (int m = 1; m < p.images; m++) v += win[m * p.window + i];
+        return v;
+      });
     }
   }
 };
