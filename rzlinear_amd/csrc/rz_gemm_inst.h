@@ -222,14 +222,14 @@ static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const 
   }
 }
 
-template <typename T, int TBN, int OPERANDS>
-static hipError_t launch_window_form(WindowParams p, int windows, hipStream_t stream) {
-  typedef WindowKernel<T, TBN, OPERANDS> K;
+template <typename T, int TBN, int OPERANDS, bool WHOLE>
+static hipError_t launch_window_whole(WindowParams p, int windows, hipStream_t stream) {
+  typedef WindowKernel<T, TBN, OPERANDS, WHOLE> K;
   static_assert(K::kFixedBytes + sizeof(float) * kWindowFloats <= 160 * 1024, "the images of a window do not fit the LDS");
   if (p.window < 4 || p.window > kWindowFloats || (p.window & 3) || windows < 1) return hipErrorInvalidValue;
   if ((long long)windows * p.window < p.H) return hipErrorInvalidValue;
   if (p.h.BN != TBN || !window_tile_supported(p.h.BK, p.h.BN)) return hipErrorInvalidValue;
-  auto kernel = rz_window_kernel<T, TBN, OPERANDS>;
+  auto kernel = rz_window_kernel<T, TBN, OPERANDS, WHOLE>;
   p.images = window_images(p.window);
   const size_t smem = K::kFixedBytes + sizeof(float) * (size_t)p.window * p.images;
   static std::atomic<uint64_t> lds_limit_raised{0};
@@ -243,6 +243,13 @@ static hipError_t launch_window_form(WindowParams p, int windows, hipStream_t st
   return hipGetLastError();
 }
 
+template <typename T, int TBN, int OPERANDS>
+static hipError_t launch_window_form(const WindowParams& p, int windows, hipStream_t stream) {
+  if constexpr (OPERANDS == kPacked)
+    if (p.K % p.h.BK == 0 && p.N % TBN == 0) return launch_window_whole<T, TBN, OPERANDS, true>(p, windows, stream);
+  return launch_window_whole<T, TBN, OPERANDS, false>(p, windows, stream);
+}
+
 // With room for them the operands are laid out as fragments first; else, where their rows hold whole 16-byte pieces, they go
 // through the staged form.
 template <typename T, int TBN>
@@ -251,7 +258,7 @@ static hipError_t launch_window_one(const WindowParams& p, int windows, hipStrea
   if (p.packed_x != nullptr && p.packed_y != nullptr) {
     // (blocks of 32 columns up to whole hashed tiles: every unit of every tile has its fragments, see window_pack_bytes)
     const long long blocks_x = (long long)p.tiles_k * (p.h.BK / 32), blocks_y = (long long)p.tiles_n * (TBN / 32);
-    constexpr int kRows = WindowKernel<T, TBN, kPacked>::kGroupRows;
+    constexpr int kRows = WindowKernel<T, TBN, kPacked, true>::kGroupRows;
     const long long ngroups = (p.M + kRows - 1) / kRows, wgs = ((blocks_x + blocks_y) * ngroups + 3) / 4;
     if (wgs > 0x1fffffffLL) return hipErrorInvalidValue;
     hipLaunchKernelGGL(window_pack_kernel<T>, dim3((unsigned)wgs), dim3(256), 0, stream, p, (int)blocks_x, (int)blocks_y, (int)ngroups);

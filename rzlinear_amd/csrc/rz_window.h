@@ -85,7 +85,10 @@ static constexpr int kFragBytes = 1024;   // a fragment of a wavefront: 16 bytes
 // items in flight (spills), eight wavefronts with up to eight (87 us), units in the order of their offsets (fewer waits,
 // but units of one window then share no rows or columns in the L2: 120 us against 92 staged).
 enum WindowOperands { kByElement = 0, kStaged = 1, kPacked = 2 };
-template <typename T, int TBN, int OPERANDS>
+// WHOLE: K and N are multiples of the hashed tile's sides, so that every unit lies inside W and nothing looks where it ends.  Packed form alone:
+// looking there costs it 1 to 4 %, the staged one, which has to look before it multiplies, nothing (without, it spills more registers: 16-bit 1.5 %
+// slower).
+template <typename T, int TBN, int OPERANDS, bool WHOLE>
 struct WindowKernel {
   static constexpr bool STAGED = OPERANDS == kStaged, PACKED = OPERANDS == kPacked;
   static_assert(TBN == 32 || TBN == 64 || TBN == 128, "tiles of 32, 64 or 128 columns");
@@ -371,8 +374,6 @@ struct WindowKernel {
       uint32_t at_x = 0, at_y[BJ];
 #pragma unroll
       for (int q = 0; q < BJ; q++) at_y[q] = 0;
-      // every unit lies inside the matrices as a whole
-      const bool all_whole = (p.K & (p.h.BK - 1)) == 0 && (p.N & (TBN - 1)) == 0;
       int strip_k0 = 0, strip_n0 = 0;
       bool strip_whole = false;
       // which of a lane's pieces of the group at row m0 of the unit at (k0, n0) lie inside the matrices
@@ -383,9 +384,12 @@ struct WindowKernel {
 #pragma unroll
         for (int q = 0; q < BJ; q++) oky[q] = m0 + lane / PY + q * (64 / PY) < p.M && col_ok;
       };
-      // ... and the same for the strip being multiplied
+      // every unit lies inside the matrices as a whole
+      const bool all_whole = WHOLE || ((p.K & (p.h.BK - 1)) == 0 && (p.N & (TBN - 1)) == 0);
+      // ... and the same for the unit being multiplied (zero, which every K and N of whole tiles has room for, where the staged form finds all_whole)
       int mult_k0 = 0, mult_n0 = 0;
       bool mult_whole = all_whole;
+      int set_k0[kDepth], set_n0[kDepth];   // (not staged) ... and of every set
       auto fetch_next = [&](auto set) {
         constexpr int S = decltype(set)::value;
         if constexpr (PACKED) {
@@ -396,6 +400,12 @@ struct WindowKernel {
             const int tk = id / p.tiles_n, tn = id - tk * p.tiles_n;
             packed_x = (global_ptr)p.packed_x + (int64_t)(tk * (p.h.BK >> 5) + un / kParts) * packed_block;
             packed_y = (global_ptr)p.packed_y + (int64_t)(tn * (TBN >> 5) + (un % kParts) * BJ) * packed_block;
+            strip_k0 = tk * p.h.BK + (un / kParts) * 32;
+            strip_n0 = tn * TBN + (un % kParts) * UC;
+          }
+          if constexpr (!WHOLE) {
+            set_k0[S] = strip_k0;
+            set_n0[S] = strip_n0;
           }
           px[S] = load_packed(packed_x);
 #pragma unroll
@@ -459,6 +469,8 @@ struct WindowKernel {
           const int tk = id / p.tiles_n, tn = id - tk * p.tiles_n;
           const int k0 = tk * p.h.BK + (un / kParts) * 32;   // the unit's first row of W
           const int n0 = tn * TBN + (un % kParts) * UC;      // ... and first column
+          set_k0[S] = k0;
+          set_n0[S] = n0;
           const int m0 = fg * kGroupRows;
           const bool whole = m0 + kGroupRows <= p.M;
           // (a strip that begins beyond K contributes nothing; its base is kept inside the matrix)
@@ -532,7 +544,12 @@ struct WindowKernel {
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         const int rel = (int)((long long)tile_off - w0);   // (offsets and window starts are below 2^31)
-        if (rel >= 0 && rel + kUnitSpan <= wlen) {
+        // What a unit spans beyond K and N is not added: a product with zeros, but a NaN where the other factor is not finite, and its
+        // places in hashed_weight belong to other tiles, or to none.  (x below, the place in the window of row r and column c of
+        // the unit, is rel + r * TBN + c with c < TBN, so that a bound on x is one on r.)
+        const int rows = WHOLE ? 32 : p.K - mult_k0, cols = WHOLE ? UC : p.N - mult_n0;   // (of the unit and beyond, inside W)
+        const int limit = rows < 32 && rel + rows * TBN < wlen ? rel + rows * TBN : wlen;
+        if (rel >= 0 && rel + kUnitSpan <= limit && cols >= UC) {
           // the whole unit lies inside the window (the usual case): no checks, constant offsets
 #pragma unroll
           for (int b = 0; b < BJ; b++) {
@@ -555,13 +572,13 @@ struct WindowKernel {
             }
           }
         } else {
-          // elements outside the window go to a dump slot behind it: no branches, so the reads
+          // elements outside the window (or W) go to a dump slot behind it: no branches, so the reads
           // and the writes of a block go out back to back (the addresses of a lane are distinct;
           // the dump slots are shared between wavefronts, their contents are never used)
           const int dump = p.images * p.window + lane;
 #pragma unroll
           for (int b = 0; b < BJ; b++) {
-            const int base = rel + ((lane >> 5) * 4) * TBN + b * 32 + (lane & 31);
+            const int base = b * 32 + (lane & 31) < cols ? rel + ((lane >> 5) * 4) * TBN + b * 32 + (lane & 31) : -(1 << 30);
             // (eight elements at a time: 16 wavefronts per compute unit leave few registers)
 #pragma unroll
             for (int half = 0; half < 2; half++) {
@@ -571,7 +588,7 @@ struct WindowKernel {
               for (int q = 0; q < 8; q++) {
                 const int i = half * 8 + q;
                 const int x = base + ((i >> 2) * 8 + (i & 3)) * TBN;
-                at[q] = (x >= 0 && x < wlen) ? image + x : dump;
+                at[q] = (x >= 0 && x < limit) ? image + x : dump;
                 cur[q] = win[at[q]];
               }
 #pragma unroll
@@ -591,6 +608,17 @@ struct WindowKernel {
         // the set freed by the previous item takes the loads of the item kDepth - 1 ahead
         fetch_next(std::integral_constant<int, (S + kDepth - 1) % kDepth>{});
         if (pg == 0 && pt < my_tiles) need_added = must_be_added(my_first + pt * kWaves);   // (uniform)
+        if constexpr (!STAGED && !WHOLE) {   // where the item's unit lies
+          mult_k0 = set_k0[S];
+          mult_n0 = set_n0[S];
+        } else if (pg == 0 && !all_whole) {   // (uniform)
+          const int ptc = pt < my_tiles ? pt : my_tiles - 1;
+          const int v = __builtin_amdgcn_readfirstlane(sm.list[my_first + ptc * kWaves]);
+          const int id = v >> ushift, un = v & (units - 1), tk = id / p.tiles_n;
+          mult_k0 = tk * p.h.BK + (un / kParts) * 32;
+          mult_n0 = (id - tk * p.tiles_n) * TBN + (un % kParts) * UC;
+          mult_whole = mult_k0 + 32 <= p.K && mult_n0 + UC <= p.N;
+        }
         if constexpr (PACKED) {
           if constexpr (k16) {
 #pragma unroll
@@ -620,14 +648,6 @@ struct WindowKernel {
             u32x4_t wx = px[S], wy[BJ];
 #pragma unroll
             for (int q = 0; q < BJ; q++) wy[q] = py[S][q];
-            if (pg == 0 && !all_whole) {   // (uniform) a new unit
-              const int ptc = pt < my_tiles ? pt : my_tiles - 1;
-              const int v = __builtin_amdgcn_readfirstlane(sm.list[my_first + ptc * kWaves]);
-              const int id = v >> ushift, un = v & (units - 1), tk = id / p.tiles_n;
-              mult_k0 = tk * p.h.BK + (un / kParts) * 32;
-              mult_n0 = (id - tk * p.tiles_n) * TBN + (un % kParts) * UC;
-              mult_whole = mult_k0 + 32 <= p.K && mult_n0 + UC <= p.N;
-            }
             if (!(mult_whole && (pg + 1) * kGroupRows <= p.M)) {
               asm volatile("" ::: "memory");
               // (with all_whole the coordinates are zero: only the rows can lie outside)
@@ -821,9 +841,9 @@ __device__ __forceinline__ void window_colsum(const WindowParams& p, int block, 
   }
 }
 
-template <typename T, int TBN, int OPERANDS>
-__global__ __launch_bounds__((WindowKernel<T, TBN, OPERANDS>::kThreads)) void rz_window_kernel(WindowParams p) {
-  typedef WindowKernel<T, TBN, OPERANDS> K;
+template <typename T, int TBN, int OPERANDS, bool WHOLE>
+__global__ __launch_bounds__((WindowKernel<T, TBN, OPERANDS, WHOLE>::kThreads)) void rz_window_kernel(WindowParams p) {
+  typedef WindowKernel<T, TBN, OPERANDS, WHOLE> K;
   extern __shared__ __attribute__((aligned(16))) unsigned char rz_window_smem[];
   static_assert(K::kThreads == 4 * kWindowBiasCols && K::kFixedBytes >= sizeof(float) * K::kThreads, "four row groups, whose sums fit the LDS of any window");
   if ((int)blockIdx.x >= p.windows) {   // (uniform)

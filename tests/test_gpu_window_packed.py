@@ -125,3 +125,38 @@ def test_the_bits_do_not_depend_on_the_workspace(shape, dtype):
         _call(lib, x, dy, out, at, nbytes, p, shape, code, tuning)
         got.append(out)
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16], ids=lambda d: str(d).split(".")[-1])
+@pytest.mark.parametrize("shape", [
+    (20, 2047, 3003, 700001, 64, 64),
+    (33, 2080, 4104, 1000000, 64, 128),   # rows of whole pieces
+    (7, 1030, 1030, 200000, 128, 32),
+], ids=lambda s: "x".join(map(str, s)))
+def test_infinities_stay_where_w_has_elements(oracle, shape, dtype):
+    """One infinite gradient reaches the places of its column of W, one infinite input those of its row, and none of the places
+    that a tile at the edge of W spans beyond it."""
+    from rzlinear_amd import _lib
+    M, K, N, H, BK, BN = shape
+    print("window infinities", shape, dtype, flush=True)
+    (x, _, dy), _ = make_inputs(M, K, N, H, dtype, seed=7)
+    x[x == 0] = 1
+    dy[dy == 0] = 1
+    k_inf, n_inf = K - 3, N - 2
+    x[M - 1, k_inf] = float("inf")
+    dy[M // 2, n_inf] = float("-inf")
+    idx = oracle.index_map(K, N, H, BK, BN, R1024)
+    touched = np.zeros(H, dtype=bool)
+    touched[idx[k_inf]] = True
+    touched[idx[:, n_inf]] = True
+    lib = _lib.load()
+    code = _lib.dtype_code(x)
+    t = _lib.Tuning(window=1)
+    tuning = ctypes.byref(t)
+    need = lib.rz_weight_grad_hashed_workspace_bytes(M, K, N, H, BK, BN, code, 0, 0, tuning)
+    ws = torch.empty((need,), dtype=torch.uint8, device=x.device)
+    plan = _lib.layer_plan(K, N, H, BK, BN, _lib.hash_constants(*rargs(R1024)), 2, x.device)
+    for at, nbytes in ((ws.data_ptr(), need), (None, 0)):
+        out = torch.zeros((H,), dtype=dtype, device=x.device)
+        _call(lib, x, dy, out, at, nbytes, plan, shape, code, tuning)
+        assert ((~torch.isfinite(out)).cpu().numpy() == touched).all()
