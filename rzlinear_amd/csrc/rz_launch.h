@@ -645,6 +645,48 @@ static inline double window_us(int M, int K, int N, int H, int BK, int BN, int e
   return f.fixed + f.per_mb * mb + (work_us > chain_us ? work_us + f.rest * chain_us : chain_us + f.rest * work_us);
 }
 
+// A second fit of the same times, over what the first one leaves out: 3300 drawn calls of 1 to 4000 rows, 64 to 16384 columns, every hashed tile that
+// the kernel serves, K * N / H of 1 to 2000 (of 1500 other such calls nine tenths are within 0.69 to 1.2 of the measured time, half within
+// 8 %).  Beside what the first one knows: the busiest window has a few times the square root of the mean number of units more; a unit that
+// reaches beyond the window is added with checks; a handful of units leave wavefronts idle; 32-column units are about half the work,
+// those of 128-column tiles, which lie further apart, more.
+static inline double window_us_any_tile(int M, int K, int N, int H, int BK, int BN, int elem_bytes, int window, int windows, bool packed) {
+  struct Fit { double fixed, per_mb, unit, rows, misses, link, rest, beyond, narrow_unit, narrow_rows, per_m, wide, busiest, few; };
+  static const Fit fits[2][3] = {
+    {{9.27, 0.80, 0.0833, 0.0266, 0.0196, 0.726, 1.25, 0.0317, 0.567, 0.715, 1.04, 0.302, 4.18, 4.33},
+     {8.34, 0.0, 0.1107, 0.0454, 0.0332, 1.48, 0.418, 0.0489, 0.469, 0.774, 1.20, 0.150, 3.72, 5.43},
+     {8.66, 0.37, 0.1473, 0.1136, 0.0659, 1.17, 0.499, 0.0562, 0.356, 0.723, 1.09, 0.230, 4.29, 10.2}},
+    {{9.69, 1.0, 0.1080, 0.2395, 0.0122, 1.72, 0.433, 0.0286, 0.495, 0.528, 1.43, 0.200, 2.87, 2.47},
+     {8.75, 0.02, 0.1604, 0.2143, 0.0108, 2.45, 0.258, 0.0317, 0.423, 0.579, 1.52, 0.163, 3.48, 6.69},
+     {9.44, 0.0, 0.0768, 0.3956, 0.0370, 2.03, 0.405, 0.0662, 0.382, 0.627, 1.72, 0.147, 3.80, 7.03}}};
+  const bool whole = K % (16 / elem_bytes) == 0 && N % (16 / elem_bytes) == 0, narrow = BN == 32;
+  const Fit& f = fits[elem_bytes == 4][packed ? 0 : whole ? 1 : 2];
+  const double span = window_unit_span(BN), all = (double)((K + BK - 1) / BK) * (double)((N + BN - 1) / BN) * window_units(BK, BN);
+  const double meets = ((double)window + span) / (double)H, mean = all * (meets < 1.0 ? meets : 1.0), units = mean + f.busiest * sqrt(mean);
+  const double beyond = window > span ? 2.0 * span / (window + span) : 1.0;   // the share of the units that do not lie inside the window
+  const int group = elem_bytes == 4 ? 8 : 16;
+  const double rounds = (double)((windows + kComputeUnits - 1) / kComputeUnits), chunks = (double)((M + group - 1) / group * group) / 32.0;
+  const double mb = (double)M * ((double)K + N) * elem_bytes * 1e-6;
+  const double unit = (f.unit + f.beyond * beyond) * (narrow ? f.narrow_unit : 1.0);
+  const double rows = (f.rows + (mb > 4.3 ? f.misses * (1.0 - 4.3 / mb) : 0.0)) * (narrow ? f.narrow_rows : 1.0);
+  const double work_us = rounds * (units * unit + sqrt(units * units + f.few * f.few) * chunks * rows) * (BN == 128 ? 1.0 + f.wide : 1.0);
+  const double chain_us = f.link * (double)K * N / (double)H / window_images(window);
+  return f.fixed + f.per_mb * mb + f.per_m * H * 1e-6 + (work_us > chain_us ? work_us + f.rest * chain_us : chain_us + f.rest * work_us);
+}
+
+// ... and what the fold (priced by plan_weight_grad, whose prices leave out what all of its plans share) or the atomics take on such calls,
+// fitted to the same measurements: nine tenths are within 0.8 to 1.3 (fold) and 0.88 to 1.13 (atomics) of the measured time.
+static inline double scatter_us(int M, int K, int N, int H, int elem_bytes, const WeightGradPlan& other) {
+  const bool f32 = elem_bytes == 4;
+  const double kn = (double)K * N * 1e-6, h = H * 1e-6, mb = (double)M * ((double)K + N) * elem_bytes * 1e-6;
+  if (other.fold.use && other.fold.small)
+    return f32 ? 3.0 + 1.28 * other.fold_us + 9.8 * h + 0.34 * kn + 0.235 * mb : 8.3 + 0.557 * other.fold_us + 2.23 * h + 1.37 * kn + 0.47 * mb;
+  if (other.fold.use) return f32 ? 2.2 + 1.13 * other.fold_us + 1.2 * h + 0.13 * mb : 2.1 + 1.04 * other.fold_us + 0.9 * h + 0.08 * kn;
+  const double rounds = (double)((tile_count(K, N, 128) + kComputeUnits - 1) / kComputeUnits), steps = (double)((M + 63) / 64), gmac = kn * M * 1e-3;
+  return f32 ? 5.7 + 3.95 * kn + 16.5 * gmac + 1.5 * h + 0.0279 * (kn / h) + rounds * (0.55 + 0.17 * steps)
+             : 8.2 + 4.14 * kn + 2.37 * gmac + 2.26 * h + 0.0107 * (kn / h) + rounds * (0.64 + 0.142 * steps);
+}
+
 // limit: bytes of workspace that the call may have.  planned: the caller holds a layer plan, so the kernel neither hashes the tile offsets nor scans
 // them for its strips (some 25 us less, measured at K = N = 10240).
 static inline WindowPlan plan_window(int M, int K, int N, int H, int BK, int BN, int elem_bytes, const rz_tuning& t,
@@ -671,7 +713,13 @@ static inline WindowPlan plan_window(int M, int K, int N, int H, int BK, int BN,
   // 1.35), the few-tiles fold 1.7 (fp32) to 1.9 times (its longest calls less, hence 1.65), the atomics about 1.8 times.
   const double t_scatter = 0.9 * (double)K * N / 184e3 + 2.0 * M * (double)K * N / 800e6;
   const double t_other = other.fold.use ? other.fold_us * (other.fold.small ? 1.65 : 1.18) : 1.8 * t_scatter;
-  pl.use = t.window == 1 || t_window < t_other;
+  // The first fits are good on average but far off for some tiles: by them alone 16-bit 256 x 128 tiles with M = 2258, K = 14448, N = 12316 took 5548 us,
+  // by atomics 1069.  So the second ones must agree.  4800 drawn calls, against the window kernel without fragments and images by a rule on rates:
+  // by the first fits 84 take more than 10 % longer, the worst 3.6 times, the mean is 0.926; by both 23, 1.65, 0.919; by the second alone
+  // 68, 2.4, 0.914, and by it 118 take more than 10 % longer than by the first (by both: 3).
+  double t_second = window_us_any_tile(M, K, N, H, BK, BN, elem_bytes, pl.window, pl.windows, pl.pack_bytes > 0);
+  if (!planned) t_second += 23.0;
+  pl.use = t.window == 1 || (t_window < t_other && t_second < scatter_us(M, K, N, H, elem_bytes, other));
   return pl;
 }
 
