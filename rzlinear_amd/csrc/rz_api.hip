@@ -317,7 +317,9 @@ static int run_plain_op(int op, int dtype, GemmParams p, const void* bias, void*
     if (sp.splits > 1) {
       if (workspace == nullptr || workspace_bytes < sp.workspace_bytes) return RZ_ERR_WORKSPACE;
       p.partial = (float*)workspace;
-      if (sp.run_steps > 0) {   // (without counters the launch adds a kernel that sums the parts: the same bits)
+      if (sp.run_steps > 0) {
+        p.partial = (float*)(((uintptr_t)workspace + kRunAlign - 1) & ~(uintptr_t)(kRunAlign - 1));   // (the plan's bytes have room for it)
+        // (without counters the launch adds a kernel that sums the parts: the same bits)
         p.finish = tuning.finish != -1 ? finish_counters_for(sp.run_tiles, s) : nullptr;
         p.bias = bias;
         return launch_gemm(dtype, op, p, nullptr, &sp, tuning, s) == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;

@@ -1018,6 +1018,7 @@ static inline SplitPlan plan_split_by_slices(int I, int J, int R, int elem_bytes
 // at most as many parts as the kernel adds up.  Of the lengths of a run from an even share to a quarter more, the one with the least
 // time by what forward16_us was fitted to: steps, a fixed part for every tile and piece, planes written and read (a longer run may leave
 // the tiles' ends in fewer pieces).  The 256 tile's runs are 4 % faster than that says, those of 256 x 128 up to 8 % slower.
+static constexpr size_t kRunAlign = 16;   // (the planes are read and written two floats at a time, whatever address the workspace has)
 static inline SplitPlan plan_runs(int I, int J, int R, int cols) {
   SplitPlan best = {};
   const long long tiles = (long long)((I + 255) / 256) * ((J + cols - 1) / cols);
@@ -1052,7 +1053,7 @@ static inline SplitPlan plan_runs(int I, int J, int R, int cols) {
     best.run_tiles = (int)rest;
     best.est_us = us;
   }
-  best.workspace_bytes = (size_t)best.splits * (size_t)best.run_tiles * 256 * (size_t)cols * sizeof(float);
+  if (best.tile != 0) best.workspace_bytes = (size_t)best.splits * (size_t)best.run_tiles * 256 * (size_t)cols * sizeof(float) + kRunAlign;
   return best;
 }
 static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz_tuning& t) {

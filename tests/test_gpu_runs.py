@@ -100,3 +100,82 @@ def test_runs_on_several_streams_at_once():
                 got.append(run())
     torch.cuda.synchronize()
     assert all(torch.equal(g, want) for g in got)
+
+
+def _ws_call(op, x, hw, bias, out, ld_in, ld_out, ws, nbytes, shape, tuning=None):
+    """rz_forward_hashed / rz_input_grad_hashed over a workspace and pitches of the test's choice; returns the status."""
+    from rzlinear_amd import _lib
+    M, K, N, H, BK, BN = shape
+    lib = _lib.load()
+    R = _lib.hash_constants(*rargs(R1024))
+    stream = torch.cuda.current_stream().cuda_stream
+    code = _lib.dtype_code(x)
+    if op == 0:
+        st = lib.rz_forward_hashed(x.data_ptr(), hw.data_ptr(), bias.data_ptr(), out.data_ptr(), ws, nbytes, M, K, N, H, BK, BN, R, 2, 0.75,
+                                   ld_in, ld_out, code, tuning, stream)
+    else:
+        st = lib.rz_input_grad_hashed(x.data_ptr(), hw.data_ptr(), out.data_ptr(), ws, nbytes, M, K, N, H, BK, BN, R, 2, 0.75, ld_in, ld_out,
+                                      code, tuning, stream)
+    torch.cuda.synchronize()
+    return st
+
+
+def _need(op, shape, code, tuning=None):
+    from rzlinear_amd import _lib
+    lib = _lib.load()
+    return (lib.rz_forward_hashed_workspace_bytes if op == 0 else lib.rz_input_grad_hashed_workspace_bytes)(*shape, code, tuning)
+
+
+def _operands(op, shape, dtype, seed=4):
+    M, K, N, H, BK, BN = shape
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn((M, K if op == 0 else N), generator=g).to(dtype).cuda()
+    hw = ((torch.rand((H,), generator=g) * 2 - 1) / K ** 0.5).to(dtype).cuda()
+    bias = torch.randn((N,), generator=g).to(dtype).cuda()
+    return x, hw, bias, torch.empty((M, N if op == 0 else K), dtype=dtype, device="cuda")
+
+
+@pytest.mark.parametrize("op,shape,tile,slices,dtype", [CASES[0], CASES[3], CASES[5]], ids=str)
+def test_runs_over_any_workspace_address_and_pitch(op, shape, tile, slices, dtype):
+    """The planes are read and written two floats at a time: a workspace at any address has room to align them.  Rows of the operand and the
+    result at odd pitches, between NaN and values that must stay."""
+    from rzlinear_amd import _lib
+    print("runs at odd addresses", op, shape, dtype, flush=True)
+    x, hw, bias, out = _operands(op, shape, dtype)
+    M, cols, J = shape[0], x.shape[1], out.shape[1]
+    need = _need(op, shape, _lib.dtype_code(x))
+    ws = torch.full((need + 256,), 255, dtype=torch.uint8, device="cuda")
+    assert _ws_call(op, x, hw, bias, out, cols, J, ws.data_ptr(), need, shape) == 0
+    wide_x = torch.full((M + 1, cols + 3), float("nan"), dtype=dtype, device="cuda")
+    wide_x[:M, :cols] = x
+    wide_out = torch.full((M + 1, J + 5), 7.0, dtype=dtype, device="cuda")
+    for shift in (4, 1, 12):
+        ws.fill_(255)
+        out2 = wide_out[:M, :J]
+        out2.fill_(float("nan"))
+        assert _ws_call(op, wide_x, hw, bias, wide_out, cols + 3, J + 5, ws.data_ptr() + shift, need, shape) == 0
+        assert torch.equal(out2, out), shift
+        assert bool((wide_out[:, J:] == 7).all()) and bool((wide_out[M] == 7).all())
+        assert bool((ws[:shift] == 255).all()) and bool((ws[need + shift:] == 255).all())
+
+
+@pytest.mark.parametrize("op,shape,tile,slices,dtype", [CASES[0], CASES[3]], ids=str)
+def test_runs_keep_infinities_and_nan_where_they_belong(op, shape, tile, slices, dtype):
+    """A row with one infinite or NaN element gives a row without finite ones; the other rows have the bits they have without it."""
+    print("runs with infinities", op, shape, dtype, flush=True)
+    from rzlinear_amd import _lib
+    x, hw, bias, out = _operands(op, shape, dtype)
+    hw[hw == 0] = 1
+    M, cols, J = shape[0], x.shape[1], out.shape[1]
+    need = _need(op, shape, _lib.dtype_code(x))
+    ws = torch.empty((need,), dtype=torch.uint8, device="cuda")
+    assert _ws_call(op, x, hw, bias, out, cols, J, ws.data_ptr(), need, shape) == 0
+    rows = {0: float("inf"), 255: float("nan"), M // 2: float("-inf"), M - 1: float("inf")}
+    for i, (row, v) in enumerate(rows.items()):
+        x[row, (cols - 1) * i // 3] = v
+    got = torch.empty_like(out)
+    assert _ws_call(op, x, hw, bias, got, cols, J, ws.data_ptr(), need, shape) == 0
+    finite = torch.isfinite(got)
+    keep = torch.ones(M, dtype=torch.bool, device="cuda")
+    keep[list(rows)] = False
+    assert not bool(finite[~keep].any()) and torch.equal(got[keep], out[keep])
