@@ -156,7 +156,11 @@ int rz_input_grad(const void* dY, const void* HW, void* dX, int M, int K, int N,
  * contracted dimension (skinny batches such as M = 32 against K = N = 10240) the work is cut
  * into slices that write fp32 partial results to `workspace`, and a second kernel adds them
  * (plus bias) into the output.  *_workspace_bytes returns the size needed (0 = no split; then
- * these calls equal rz_forward_bias / rz_input_grad and workspace may be NULL).  No
+ * these calls equal rz_forward_bias / rz_input_grad and workspace may be NULL).  16-bit calls
+ * whose last round of workgroups would be far from full deal the R steps of its tiles out in runs of equal
+ * length, which takes a workspace of up to 154 MB; with less, down to none, these calls do what they would
+ * without runs (slices, if their planes fit, or whole tiles; then with the bits of that), and
+ * RZ_ERR_WORKSPACE is left to a workspace that slices need and do not get.  Any address will do.  No
  * counterpart in the reference, whose kernels never split (impl/RzLinearForward.py:37-40,
  * impl/RzLinearBackward.py:407-410).
  */

@@ -109,9 +109,11 @@ struct PlanMemo {
 
 #define RZ_TUNING_WORDS(t) (t).tile, (t).stages, (t).lds_image, (t).window, (t).split, (t).clamp, (t).fold, (t).fold_tiles, (t).finish, (t).poll_limit
 
-static SplitPlan split_plan(int I, int J, int R, int elem_bytes, const rz_tuning& t) {
-  static thread_local PlanMemo<SplitPlan, 14> memo;
-  return memo.get({I, J, R, elem_bytes, RZ_TUNING_WORDS(t)}, [&] { return plan_split(I, J, R, elem_bytes, t); });
+// (runs = false: without dealing tiles out in runs, which takes a workspace where slices may need none, or less)
+static SplitPlan split_plan(int I, int J, int R, int elem_bytes, const rz_tuning& t, bool runs = true) {
+  static thread_local PlanMemo<SplitPlan, 15> memo;
+  return memo.get({I, J, R, elem_bytes, runs ? 1 : 0, RZ_TUNING_WORDS(t)},
+                  [&] { return runs ? plan_split(I, J, R, elem_bytes, t) : plan_split_by_slices(I, J, R, elem_bytes, t); });
 }
 
 // How a weight gradient is carried out, for a caller with (`planned`) or without a layer plan.
@@ -312,8 +314,10 @@ static int run_plain_op(int op, int dtype, GemmParams p, const void* bias, void*
   // in cache when the next kernel reads it)
   p.stream_c = (size_t)p.I * (size_t)p.J * dtype_bytes(dtype) >= ((size_t)8 << 20) ? 1 : 0;
   if (may_split) {
-    // tile and slices are chosen together
-    const SplitPlan sp = split_plan(p.I, p.J, p.R, dtype_bytes(dtype), tuning);
+    // tile and slices are chosen together; a workspace that does not hold the planes of runs is enough where it holds those of slices
+    SplitPlan sp = split_plan(p.I, p.J, p.R, dtype_bytes(dtype), tuning);
+    if (sp.run_steps > 0 && (workspace == nullptr || workspace_bytes < sp.workspace_bytes))
+      sp = split_plan(p.I, p.J, p.R, dtype_bytes(dtype), tuning, false);
     if (sp.splits > 1) {
       if (workspace == nullptr || workspace_bytes < sp.workspace_bytes) return RZ_ERR_WORKSPACE;
       p.partial = (float*)workspace;

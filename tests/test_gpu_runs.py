@@ -179,3 +179,39 @@ def test_runs_keep_infinities_and_nan_where_they_belong(op, shape, tile, slices,
     keep = torch.ones(M, dtype=torch.bool, device="cuda")
     keep[list(rows)] = False
     assert not bool(finite[~keep].any()) and torch.equal(got[keep], out[keep])
+
+
+@pytest.mark.parametrize("op,shape,dtype,slices_bytes", [
+    (0, (3328, 7680, 10624, 81592, 64, 64), torch.bfloat16, 0),
+    (1, (1895, 5660, 15920, 100000, 32, 64), torch.float16, 0),
+    (0, (1024, 10240, 10240, 655360, 32, 64), torch.bfloat16, 3 * 1024 * 10240 * 4),   # (slices need planes too)
+], ids=str)
+def test_a_call_without_room_for_runs_does_what_it_would_without_them(op, shape, dtype, slices_bytes):
+    """No workspace, or too little for the planes of runs: whole tiles, or slices, as such calls have always been accepted; an error only
+    where slices need more."""
+    import ctypes
+    from rzlinear_amd import _lib
+    print("no room for runs", op, shape, dtype, flush=True)
+    x, hw, bias, out = _operands(op, shape, dtype)
+    M, cols, J = shape[0], x.shape[1], out.shape[1]
+    code = _lib.dtype_code(x)
+    assert _lib.plan_query(op, *shape, code)["windows"] > 0
+    need = _need(op, shape, code)
+    assert slices_bytes < need
+    ws = torch.empty((need,), dtype=torch.uint8, device="cuda")
+    runs, whole = torch.empty_like(out), torch.empty_like(out)
+    assert _ws_call(op, x, hw, bias, runs, cols, J, ws.data_ptr(), need, shape) == 0
+    assert _ws_call(op, x, hw, bias, whole, cols, J, None, 0, shape, ctypes.byref(_lib.Tuning(split=-1))) == 0
+
+    def close(a):
+        return float((a.float() - whole.float()).abs().max() / whole.float().abs().max()) <= 2e-2
+    assert close(runs)
+    assert _ws_call(op, x, hw, bias, out, cols, J, None, 0, shape) == (0 if slices_bytes == 0 else -7)
+    if slices_bytes > 0:
+        assert _ws_call(op, x, hw, bias, out, cols, J, ws.data_ptr(), slices_bytes - 1, shape) == -7
+    out.fill_(float("nan"))
+    ws.fill_(255)
+    assert _ws_call(op, x, hw, bias, out, cols, J, ws.data_ptr(), slices_bytes, shape) == 0 and close(out)
+    assert bool((ws[slices_bytes:] == 255).all())
+    again = torch.empty_like(out)
+    assert _ws_call(op, x, hw, bias, again, cols, J, ws.data_ptr(), need - 1, shape) == 0 and torch.equal(again, out)
