@@ -885,6 +885,8 @@ static inline double forward16_us(int rows, int cols, int I, int J, int R, int s
                         : c.second + c.second_mb * (2.0 * slices + 0.5) * mb + (slices > 8 ? c.second_slice * (slices - 8) : 0.0));
 }
 
+// (The plans take a cut as finished by its own kernel wherever finish_slices says so, whatever rz_tuning.finish: with a second kernel, by that
+// override or for want of counters, a call keeps its cut, and so its bits.)
 // Tile and number of slices together: the pair with the least estimated time.  A slice pays the
 // fill and drain of its pipeline (about three steps), the cut pays the fp32 partial planes
 // (written, read back) and the launch of the kernel that adds them.
@@ -940,7 +942,7 @@ static inline SplitPlan plan_split_by_rate(int I, int J, int R, int elem_bytes, 
       //  back by the finishing workgroups, and no second kernel is launched — worth a couple of microseconds
       //  and a plane; fp32, M = 16384, K = 512, N = 1024 input-grad, planes of 33 MB: the 256 tile in two
       //  slices 155 us against the whole 128 tile's 136)
-      const bool finished = slices > 1 && slices <= finish_slices(tile, I, J, R, elem_bytes, t) && t.finish != -1;
+      const bool finished = slices > 1 && slices <= finish_slices(tile, I, J, R, elem_bytes, t);
       if (slices > 1 && fitted) us += finished ? (2.0 * slices - 1.0) * (double)I * J * 4.0 / 8.0e6 + 3.5 : (2.0 * slices * (double)I * J * 4.0 + (double)I * J * elem_bytes) / 7.0e6 + 0.5;
       else if (finished) us += (2.0 * slices - 1.0) * (double)I * J * 4.0 / 4.0e6 + 2.0;
       else if (slices > 1) us += (2.0 * slices * (double)I * J * 4.0 + (double)I * J * elem_bytes) / 4.0e6 + (direct ? 3.0 : 4.0);
@@ -984,7 +986,7 @@ static inline SplitPlan plan_split_by_slices(int I, int J, int R, int elem_bytes
   if (elem_bytes != 2 || I <= 64 || R < 8 || t.tile != 0 || t.split != 0 || t.stages == 1 || t.clamp == -1) return by_rate;
   auto time_of = [&](int tile, int slices, int chunk) {
     const bool pair = pair_form(tile, I, J, R, slices > 1 ? chunk : R, elem_bytes, t);
-    const bool finished = slices > 1 && slices <= finish_slices(tile, I, J, R, elem_bytes, t) && t.finish != -1;
+    const bool finished = slices > 1 && slices <= finish_slices(tile, I, J, R, elem_bytes, t);
     return forward16_us(pair ? 256 : tile, tile, I, J, R, slices, chunk / 64, finished);
   };
   SplitPlan best = by_rate;
@@ -1064,7 +1066,7 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
   // 194 / 177, input-grad 191 / 178; M = 5031, 4002 <- 6371 296 / 230; M = 8864, 9146 -> 934 222 / 165; M = 3744, 9622 <- 9701 698 / 609;
   // M = 1286, 9678 -> 16359 432 / 369.  Taken for 1 to 2 of 100 drawn calls, those with a long R and a last round that is far from full: on 20 of them 0.91
   // times the time in the mean, at most 0.99.
-  const bool finished = best.splits > 1 && best.splits <= finish_slices(best.tile, I, J, R, elem_bytes, t) && t.finish != -1;
+  const bool finished = best.splits > 1 && best.splits <= finish_slices(best.tile, I, J, R, elem_bytes, t);
   const int unit = slice_unit(best.tile, elem_bytes), chunk = best.splits > 1 ? best.r_chunk : (R + unit - 1) / unit * unit;
   const bool pairs = pair_form(best.tile, I, J, R, best.splits > 1 ? chunk : R, elem_bytes, t);
   const double us = forward16_us(pairs ? 256 : best.tile, best.tile, I, J, R, best.splits, chunk / 64, finished);

@@ -87,3 +87,29 @@ def test_drawn_plans_in_runs_cover_every_step_once():
 def test_an_override_is_never_dealt_out_in_runs(tuning):
     with _lib.tuning(**tuning):
         assert _lib.plan_query(0, 1024, 10240, 10240, 6553600, 32, 64, _lib.RZ_BF16)["windows"] == 0
+
+
+def test_the_second_kernel_gets_the_plan_of_the_first():
+    """finish=-1 promises the same bits: the same tile, slices and runs, whoever adds them up."""
+    rng = random.Random(13)
+    cut = runs = 0
+    for _ in range(3000):
+        code = rng.choice([_lib.RZ_F32, _lib.RZ_BF16, _lib.RZ_F16])
+        call = (rng.randint(0, 1), int(2 ** rng.uniform(0, 13)), rng.randint(128, 12000), rng.randint(128, 12000), 1 << 20, 64, 64, code)
+        q = _lib.plan_query(*call)
+        with _lib.tuning(finish=-1):
+            q2 = _lib.plan_query(*call)
+        assert q2["shares"] == 0
+        assert {**q, "shares": 0} == q2, call
+        cut += q["mode"] == "split"
+        runs += q["mode"] == "split" and q["windows"] > 0
+    assert cut > 500 and runs > 10
+
+
+@pytest.mark.parametrize("slices", [dict(tile=256, split=3), dict(tile=128, split=2)], ids=str)
+def test_a_cut_that_is_asked_for_is_the_same_with_a_second_kernel(slices):
+    for code in (_lib.RZ_F32, _lib.RZ_BF16):
+        with _lib.tuning(**slices):
+            q = _lib.plan_query(0, 512, 8192, 1024, 1 << 20, 64, 64, code)
+        with _lib.tuning(finish=-1, **slices):
+            assert _lib.plan_query(0, 512, 8192, 1024, 1 << 20, 64, 64, code) == {**q, "shares": 0}
