@@ -1071,6 +1071,10 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
   const bool pairs = pair_form(best.tile, I, J, R, best.splits > 1 ? chunk : R, elem_bytes, t);
   const double us = forward16_us(pairs ? 256 : best.tile, best.tile, I, J, R, best.splits, chunk / 64, finished);
   const SplitPlan& runs = pair.tile == 0 || (wide.tile != 0 && wide.est_us <= pair.est_us) ? wide : pair;
+  // (nor for planes of more than twice what the call reads and writes, unless slices take as much: M = 653, K = 11012 <- 6869 would have 104 MB
+  //  beside 23 MB of dY and dX.  Of the plans in runs 7 % are left out by that, all of short batches.)
+  const size_t most = 2 * (size_t)elem_bytes * (size_t)I * ((size_t)J + (size_t)R);
+  if (runs.workspace_bytes > (best.workspace_bytes > most ? best.workspace_bytes : most) + kRunAlign) return best;
   return runs.tile != 0 && runs.est_us < 0.95 * us ? runs : best;
 }
 

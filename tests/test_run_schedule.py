@@ -113,3 +113,14 @@ def test_a_cut_that_is_asked_for_is_the_same_with_a_second_kernel(slices):
             q = _lib.plan_query(0, 512, 8192, 1024, 1 << 20, 64, 64, code)
         with _lib.tuning(finish=-1, **slices):
             assert _lib.plan_query(0, 512, 8192, 1024, 1 << 20, 64, 64, code) == {**q, "shares": 0}
+
+
+@pytest.mark.parametrize("op,shape", [(1, (653, 11012, 6869)), (0, (317, 16216, 10935)), (1, (420, 11279, 13216)), (1, (578, 11175, 9098))], ids=str)
+def test_planes_of_runs_stay_in_proportion_to_the_call(op, shape):
+    """Planes of more than twice what the call reads and writes are not asked for where slices do without (these would have 90 to 104 MB
+    beside 17 to 24 MB)."""
+    lib = _lib.load()
+    M, K, N = shape
+    assert _lib.plan_query(op, *shape, 200000, 64, 64, _lib.RZ_BF16)["windows"] == 0
+    need = lib.rz_forward_hashed_workspace_bytes if op == 0 else lib.rz_input_grad_hashed_workspace_bytes
+    assert need(*shape, 200000, 64, 64, _lib.RZ_BF16, None) <= 4 * M * (K + N)
