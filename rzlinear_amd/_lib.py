@@ -206,7 +206,7 @@ def native():
         from .RzLinearFunction import _function_output
         lib = load()
         module.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in EXPORTS},
-                    lambda K, N, H, BK, BN, R, levels, index: layer_plan(
+                    lambda K, N, H, BK, BN, R, levels, index: layer_plan_for_call(
                         K, N, H, BK, BN, (ctypes.c_int32 * 8)(*R), levels, torch.device("cuda", index)), check, _function_output)
         torch.autograd.graph.Node.register(module.RzLinearFunctionBackward)   # (isinstance, as for any other node)
         _native = module
@@ -317,6 +317,14 @@ def layer_plan(K, N, H, BK, BN, R, hash_levels, device):
         check(lib.rz_layer_plan_build(host.data_ptr(), nbytes, K, N, H, BK, BN, R, hash_levels))
         plan = _layer_plans[key] = host.to(device)
     return plan
+
+
+def layer_plan_for_call(K, N, H, BK, BN, R, hash_levels, device):
+    """layer_plan for a call that can do without: None where it would have to be built while the current stream is being captured."""
+    key = (K, N, H, BK, BN, tuple(int(v) for v in R), int(hash_levels), str(device))
+    if key not in _layer_plans and torch.cuda.is_current_stream_capturing():
+        return None
+    return layer_plan(K, N, H, BK, BN, R, hash_levels, device)
 
 
 PLAN_MODES = {0: "store", 1: "split", 2: "lds_image", 3: "atomics", 4: "window", 5: "fold"}

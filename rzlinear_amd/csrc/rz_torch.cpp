@@ -57,7 +57,7 @@ struct Library {
   decltype(&rz_plan_query) plan_query = nullptr;
 };
 Library lib;
-PyObject* plan_provider = nullptr;    // Python: (K, N, H, BK, BN, constants, levels, device index) -> plan tensor
+PyObject* plan_provider = nullptr;    // Python: (K, N, H, BK, BN, constants, levels, device index) -> plan tensor, or None
 PyObject* status_check = nullptr;     // Python: raises for a non-zero status
 PyObject* function_node = nullptr;    // Python: the Function's own node for given saved tensors and arguments
 // What the Python side's `tuning` context has set (tests, benchmarks): a copy, which a call that is under way
@@ -155,9 +155,11 @@ Tensor layer_plan(const Geometry& g, int device) {
   python_error err;
   if (r == nullptr) err.persist();
   else if (THPVariable_Check(r)) plan = THPVariable_Unpack(r);
+  const bool none = r == Py_None;
   Py_XDECREF(r);
   PyGILState_Release(gil);
   if (r == nullptr) throw err;
+  if (none) return plan;   // (this call has to do without one, see _lib.layer_plan_for_call)
   TORCH_CHECK(plan.defined(), "a layer plan must be a tensor");
   std::lock_guard<std::mutex> lock(plans_mutex);
   plans.emplace(key, plan);

@@ -34,7 +34,8 @@ def weight_grad_hashed(input, output_grad, init_factor, M, K, N, H, R, BLOCK_SIZ
 
     Where the library would work by windows of dHW or fold stored tiles into dHW (a hashed_weight
     too large for an image in LDS), the call goes through rz_weight_grad_planned with the layer's
-    plan, which _lib.layer_plan builds once per (K, N, H, tile, constants) and keeps on the device;
+    plan, which _lib.layer_plan builds once per (K, N, H, tile, constants) and keeps on the device (a
+    stream under capture cannot have one built: a layer that has none yet is then captured without);
     everything else, and use_layer_plan=False (default: _lib.use_layer_plans), goes through
     rz_weight_grad_hashed."""
     stream = _lib.require_gpu(input, output_grad)
@@ -73,7 +74,7 @@ def weight_grad_hashed(input, output_grad, init_factor, M, K, N, H, R, BLOCK_SIZ
         use_layer_plan = _lib.use_layer_plans
     if use_layer_plan and _lib.plan_query(2, M, K, N, H, BLOCK_SIZE_K, BLOCK_SIZE_N, code, flags,
                                           with_bias_grad, planned=True)["mode"] in ("window", "fold"):
-        plan = _lib.layer_plan(K, N, H, BLOCK_SIZE_K, BLOCK_SIZE_N, R, hash_levels, output_grad.device)
+        plan = _lib.layer_plan_for_call(K, N, H, BLOCK_SIZE_K, BLOCK_SIZE_N, R, hash_levels, output_grad.device)
     if plan is not None:
         _lib.check(lib.rz_weight_grad_planned(
             x.data_ptr(), dy.data_ptr(), out.data_ptr(), bias_grad.data_ptr() if with_bias_grad else None,

@@ -7,7 +7,7 @@ import sys
 import pytest
 import torch
 
-from helpers import SEED_CONSTANTS
+from helpers import SEED_CONSTANTS, rargs
 
 pytestmark = pytest.mark.gpu
 
@@ -91,3 +91,62 @@ def test_step_captured_in_a_graph_replays_correctly(cfg):
                 assert torch.allclose(a.float(), b.float(), rtol=1e-4, atol=1e-4 * float(b.float().abs().max())), (name, replay)
             else:
                 assert torch.equal(a, b), (name, replay)
+
+
+@pytest.mark.parametrize("shape", [
+    (16, 1024, 2048, 524288),     # by windows with a layer plan, by atomics without
+    (32, 4096, 4096, 1 << 20),    # by windows, or folded without
+    (520, 4096, 4096, 200000),    # folded
+], ids=str)
+@pytest.mark.parametrize("native", [True, False], ids=["module", "launcher"])
+def test_a_layer_without_a_plan_is_captured_without_one(oracle, shape, native):
+    """A layer plan is built with a copy that a capture does not take: a backward that is captured before the layer has one goes without, as
+    calls of paths that have none always have.  The kernels are warm: another layer of the same shape has run."""
+    import numpy as np
+    from helpers import TOL, rel_err
+    from rzlinear_amd import RzLinear, _lib
+    from rzlinear_amd.impl.RzLinearBackward import weight_grad_hashed
+    M, K, N, H = shape
+    dtype, BK, BN = torch.bfloat16, 64, 64
+    _say("capture without a plan", shape, native)
+    g = torch.Generator().manual_seed(2)
+    x = torch.randn((M, K), generator=g).to(dtype).cuda().requires_grad_(True)
+    dy = torch.randn((M, N), generator=g).to(dtype).cuda()
+    layers = [RzLinear(K, N, hashed_weight=torch.nn.Parameter(((torch.rand((H,), generator=g) * 2 - 1) / K ** 0.5).to(dtype)), seed=seed, dtype=dtype,
+                       block_size_k=BK, block_size_n=BN).cuda() for seed in (31, 32)]
+
+    def backward(layer, with_plans=None):
+        if native:
+            return torch.autograd.grad(layer(x), (layer._hashed_weight,), dy)[0]
+        R = _lib.hash_constants(*rargs([int(v) for v in layer._random_numbers]))
+        return weight_grad_hashed(x.detach(), dy, layer._init_factor, M, K, N, H, R, BK, BN, use_layer_plan=with_plans)[0]
+
+    _lib.clear_layer_plans()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        backward(layers[0])
+        _lib.use_layer_plans = False
+        try:
+            backward(layers[0])   # (the kernels of the way without a plan)
+        finally:
+            _lib.use_layer_plans = True
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    plans = len(_lib._layer_plans)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        dhw = backward(layers[1])
+    assert len(_lib._layer_plans) == plans
+    for replay in range(3):
+        with torch.no_grad():
+            x.copy_(torch.randn((M, K), generator=g).to(dtype))
+        dhw.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        ref = oracle.weight_grad(x.detach().double().cpu().numpy(), dy.double().cpu().numpy(), H, BK, BN,
+                                 [int(v) for v in layers[1]._random_numbers], layers[1]._init_factor)
+        assert rel_err(dhw.float().cpu().numpy(), ref) <= TOL[dtype], replay
+    eager = backward(layers[1])   # (which builds the plan: a capture from now on has it)
+    assert len(_lib._layer_plans) == plans + 1
+    assert rel_err(eager.float().cpu().numpy(), np.asarray(ref)) <= TOL[dtype]
