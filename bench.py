@@ -103,9 +103,9 @@ TRAFFIC = {
     },
     ("grid_1024_10240", "bf16"): {
         "profile": "profiles/rz_gemm_fold_bf16_grid_1024_10240.txt",
-        "bytes": {"forward": int((398007.3 * 2.0 + 143380.0) * 1024),     # (three slices: fp32 partial planes written, read back by the slice that finishes)
-                  "input_grad": int((377290.8 * 2.0 + 143380.0) * 1024),
-                  "weight_grad": int((172182.1 * 2.0 + 204800.0) * 1024)},      # (X^T.dY tile by tile in bf16: 200 MiB)
+        "bytes": {"forward": int((341673.5 * 2.0 + 84059.5) * 1024),      # (runs: fp32 planes of the parts written, read back by the part that finishes)
+                  "input_grad": int((371741.6 * 2.0 + 82897.5) * 1024),
+                  "weight_grad": int((172180.9 * 2.0 + 204800.3) * 1024)},      # (X^T.dY tile by tile in bf16: 200 MiB)
     },
 }
 
