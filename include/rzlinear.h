@@ -185,7 +185,7 @@ int rz_input_grad_ws(const void* dY, const void* HW, void* dX, void* workspace,
  * per W tile) — 16-bit: wherever that is the faster, though it can take several times the bytes of X and
  * dY where atomic adds would need 4 * H (rz_tuning.fold = -1 forgoes it); with M small against K*N, dHW is computed in windows and the workspace holds
  * the offsets and X and dY once more, as the fragments that the kernel multiplies (a workspace with room for the offsets
- * alone, or none where a layer plan has them, is enough: the call is then slower); with few tiles the 16-bit types need an fp32 image of dHW (H floats) for
+ * alone, or none where a layer plan has them, is enough: the call is then slower, its bits are the same); with few tiles the 16-bit types need an fp32 image of dHW (H floats) for
  * atomic adds and fp32 needs nothing.  The size depends on M: ask again when the batch size
  * changes.
  */
@@ -202,7 +202,7 @@ size_t rz_weight_grad_workspace_bytes(int M, int K, int N, int H, int BK, int BN
  * the reference rounds the running sum at every atomic add).  The LDS-image, fold and
  * window paths add in a fixed order (plain read-add-write in LDS, ordered by barriers, by list
  * order or by flags; partial images are added in index order): the same inputs give the same
- * bits on every call.  Two cases leave the summation order across tiles open, as the reference
+ * bits on every call, whatever workspace it has beyond what it needs.  Two cases leave the summation order across tiles open, as the reference
  * does everywhere: the global-atomic path (a hashed_weight too large for LDS with hashed tiles of more than
  * 16384 elements, or with few tiles per element of dHW where it is the faster: rz_plan_query says so, mode 3,
  * and rz_tuning.fold = 1 takes the fold in its place), and hashed tiles of 16 rows or
@@ -297,7 +297,9 @@ int rz_weight_grad_hashed(const void* X, const void* dY, void* dHW, void* dbias,
  * tile strips (of tiles) that land in it.  Without a plan every weight-grad call on a large
  * hashed_weight hashes the tile offsets again and every workgroup searches them for its strips or
  * tiles (some 25 us of an 85 us call at M = 32, K = N = 10240; 5 us of the fold kernel's 60 to 90);
- * with one it reads its list.  The result is the same bit for bit.
+ * with one it reads its list.  The result is the same bit for bit where both calls take the same path; windows are
+ * cheaper with a plan, so that some calls fold, or add by atomics, only without one (rz_plan_query with and
+ * without RZ_PLAN_WITH_LAYER_PLAN).
  *   rz_layer_plan_bytes   size of the plan (0: bad arguments)
  *   rz_layer_plan_build   fills plan_host[plan_bytes] on the HOST (no device is touched); the
  *                         caller copies it to device memory once and keeps it with the layer
@@ -378,7 +380,8 @@ int rz_adam_step(void* param, const void* grad, float* exp_avg, float* exp_avg_s
                  float weight_decay, int decoupled, int step, float grad_scale, void* stream);
 
 /* rz_adam_step of `count` tensors at the same step, in order, in as few launches as their memory allows (tensors that
- * overlap one another go apart).  An invalid tensor ends the call with its status; those before it are updated. */
+ * overlap one another go apart).  An invalid tensor ends the call with its status; those before it are updated.  (Tensors at
+ * different steps take a call each; in order, if they may overlap.) */
 typedef struct rz_adam_tensor {
   void* param;
   const void* grad;

@@ -1064,7 +1064,7 @@ static inline SplitPlan plan_split(int I, int J, int R, int elem_bytes, const rz
   const SplitPlan wide = plan_runs(I, J, R, 256), pair = plan_runs(I, J, R, 128);
   // the plan by slices, by the same times; runs have to promise 5 %.  bf16 / fp16, by slices or whole / in runs, us: M = 1024, K = N = 10240 forward
   // 194 / 177, input-grad 191 / 178; M = 5031, 4002 <- 6371 296 / 230; M = 8864, 9146 -> 934 222 / 165; M = 3744, 9622 <- 9701 698 / 609;
-  // M = 1286, 9678 -> 16359 432 / 369.  Taken for 1 to 2 of 100 drawn calls, those with a long R and a last round that is far from full: on 20 of them 0.91
+  // M = 1286, 9678 -> 16359 432 / 369.  Taken for 3 of 100 drawn calls of more than 64 rows, those with a long R and a last round that is far from full: on 20 of them 0.91
   // times the time in the mean, at most 0.99.
   const bool finished = best.splits > 1 && best.splits <= finish_slices(best.tile, I, J, R, elem_bytes, t);
   const int unit = slice_unit(best.tile, elem_bytes), chunk = best.splits > 1 ? best.r_chunk : (R + unit - 1) / unit * unit;

@@ -86,7 +86,8 @@ class FusedSGD(_Fused):
 
 
 class FusedAdam(_Fused):
-    """``torch.optim.Adam`` (``decoupled_weight_decay=True``: ``AdamW``), amsgrad off, in one kernel for a group's parameters."""
+    """``torch.optim.Adam`` (``decoupled_weight_decay=True``: ``AdamW``), amsgrad off, in one kernel for a group's parameters
+    (in the group's order: one at another step, or on another device, begins a kernel of its own)."""
 
     def __init__(self, params, lr=1e-3, betas=(0.9, 0.999), eps=1e-8, weight_decay=0.0,
                  decoupled_weight_decay=False, master_weights=False, grad_scale=1.0):
