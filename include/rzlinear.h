@@ -343,6 +343,20 @@ int rz_weight_grad_planned(const void* X, const void* dY, void* dHW, void* dbias
 int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int dtype, unsigned flags,
                   int with_dbias, const rz_tuning* tuning, int32_t out[8]);
 
+/* ---- input-grad and weight-grad of one backward pass -----------------------------------
+ * Replaces rz_linear_backward_tl                                      impl/RzLinearBackward.py:7-20
+ * rz_input_grad_hashed followed by rz_weight_grad_hashed (layer_plan NULL) or rz_weight_grad_planned, with the same
+ * results to the bit, but for an input-grad that would be dealt out in runs (rz_plan_query): beside a weight-grad it may
+ * go in whole tiles, whose sums over N are in one piece.  Where the two contractions' kernels go together they are
+ * enqueued as ONE launch: a launch less, and workgroups of the one fill what those of the other leave idle.  The two workspaces
+ * (rz_input_grad_hashed_workspace_bytes, rz_weight_grad_hashed_workspace_bytes) and the outputs must not overlap. */
+int rz_linear_backward_hashed(const void* X, const void* dY, const void* HW, void* dX, void* dHW, void* dbias,
+                              void* workspace_dx, size_t workspace_dx_bytes, void* workspace_dhw,
+                              size_t workspace_dhw_bytes, const void* layer_plan, size_t layer_plan_bytes,
+                              int M, int K, int N, int H, int BK, int BN, const int32_t R[8], int hash_levels,
+                              float init_factor, int64_t ldx, int64_t lddy, int64_t lddx, int dtype,
+                              unsigned flags, const rz_tuning* tuning, void* stream);
+
 /*
  * Materialise W[K,N] (row pitch ldw) from hashed_weight; edge tiles are clipped.
  * Replaces rz_linear_idx_tl                                           impl/RzLinearIdx.py:6-45

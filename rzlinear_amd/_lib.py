@@ -23,7 +23,7 @@ EXPORTS = (
     "rz_weight_grad_ex", "rz_forward_hashed", "rz_input_grad_hashed", "rz_weight_grad_hashed", "rz_materialize",
     "rz_forward_hashed_workspace_bytes", "rz_input_grad_hashed_workspace_bytes",
     "rz_weight_grad_hashed_workspace_bytes", "rz_plan_query", "rz_weight_grad_static",
-    "rz_layer_plan_bytes", "rz_layer_plan_build", "rz_weight_grad_planned",
+    "rz_layer_plan_bytes", "rz_layer_plan_build", "rz_weight_grad_planned", "rz_linear_backward_hashed",
     "rz_sgd_step", "rz_adam_step", "rz_adam_step_many", "rz_mfma_probe",
 )
 
@@ -167,6 +167,10 @@ def load():
     lib.rz_weight_grad_planned.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_sz, c_vp, c_sz, c_int, c_int, c_int,
                                            c_int, c_int, c_int, i32p, c_int, c_f, c_i64, c_i64, c_int,
                                            ctypes.c_uint, tun, c_vp]
+    lib.rz_linear_backward_hashed.restype = c_int
+    lib.rz_linear_backward_hashed.argtypes = [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_sz, c_vp, c_sz, c_vp, c_sz, c_int, c_int,
+                                              c_int, c_int, c_int, c_int, i32p, c_int, c_f, c_i64, c_i64, c_i64, c_int,
+                                              ctypes.c_uint, tun, c_vp]
     lib.rz_plan_query.restype = c_int
     lib.rz_plan_query.argtypes = [c_int] * 8 + [ctypes.c_uint, c_int, tun, i32p]
     f32p = c_vp

@@ -306,42 +306,73 @@ static unsigned* finish_counters_for(long long tiles, hipStream_t s) {
   return nullptr;
 }
 
+// What a forward or input-grad that may split its contraction needs of its workspace: p's fields for the plan *sp.
+static int prepare_plain_op(int dtype, GemmParams& p, const void* bias, void* workspace, size_t workspace_bytes,
+                            const rz_tuning& tuning, hipStream_t s, SplitPlan* sp) {
+  // an output of more than twice an L2 goes out with streaming stores (a smaller one may still be
+  // in cache when the next kernel reads it)
+  p.stream_c = (size_t)p.I * (size_t)p.J * dtype_bytes(dtype) >= ((size_t)8 << 20) ? 1 : 0;
+  // tile and slices are chosen together; a workspace that does not hold the planes of runs is enough where it holds those of slices
+  *sp = split_plan(p.I, p.J, p.R, dtype_bytes(dtype), tuning);
+  if (sp->run_steps > 0 && (workspace == nullptr || workspace_bytes < sp->workspace_bytes))
+    *sp = split_plan(p.I, p.J, p.R, dtype_bytes(dtype), tuning, false);
+  p.bias = bias;
+  if (sp->splits <= 1) return RZ_OK;
+  if (workspace == nullptr || workspace_bytes < sp->workspace_bytes) return RZ_ERR_WORKSPACE;
+  p.partial = (float*)workspace;
+  if (sp->run_steps > 0) {
+    p.partial = (float*)(((uintptr_t)workspace + kRunAlign - 1) & ~(uintptr_t)(kRunAlign - 1));   // (the plan's bytes have room for it)
+    // (without counters the launch adds a kernel that sums the parts: the same bits)
+    p.finish = tuning.finish != -1 ? finish_counters_for(sp->run_tiles, s) : nullptr;
+    return RZ_OK;
+  }
+  // the slice that arrives last at a tile finishes it (adds the slices in slice order, then the
+  // bias: the bits of the second kernel's sum) — unless told otherwise, or out of counters
+  p.finish = (tuning.finish != -1 && sp->splits <= finish_slices(sp->tile, p.I, p.J, p.R, dtype_bytes(dtype), tuning)) ? finish_counters_for(tile_count(p.I, p.J, sp->tile), s) : nullptr;
+  if (p.finish == nullptr) p.bias = nullptr;   // (added by the second kernel)
+  return RZ_OK;
+}
+
+// ... and, once its contraction has been launched, the second kernel where there is one.
+static int finish_plain_op(int dtype, const GemmParams& p, const void* bias, const SplitPlan& sp, hipStream_t s) {
+  if (sp.splits <= 1 || sp.run_steps > 0 || p.finish != nullptr) return RZ_OK;
+  return reduce_slices_dtype(dtype, p.partial, p.C, bias, p.I, p.J, p.ldc, sp.splits, s) == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;
+}
+
 // Forward (op kForward) or input-grad through one code path: p holds the operands; with a
 // workspace the contraction may be split over R (skinny problems).
 static int run_plain_op(int op, int dtype, GemmParams p, const void* bias, void* workspace,
                         size_t workspace_bytes, bool may_split, const rz_tuning& tuning, hipStream_t s) {
-  // an output of more than twice an L2 goes out with streaming stores (a smaller one may still be
-  // in cache when the next kernel reads it)
-  p.stream_c = (size_t)p.I * (size_t)p.J * dtype_bytes(dtype) >= ((size_t)8 << 20) ? 1 : 0;
   if (may_split) {
-    // tile and slices are chosen together; a workspace that does not hold the planes of runs is enough where it holds those of slices
-    SplitPlan sp = split_plan(p.I, p.J, p.R, dtype_bytes(dtype), tuning);
-    if (sp.run_steps > 0 && (workspace == nullptr || workspace_bytes < sp.workspace_bytes))
-      sp = split_plan(p.I, p.J, p.R, dtype_bytes(dtype), tuning, false);
-    if (sp.splits > 1) {
-      if (workspace == nullptr || workspace_bytes < sp.workspace_bytes) return RZ_ERR_WORKSPACE;
-      p.partial = (float*)workspace;
-      if (sp.run_steps > 0) {
-        p.partial = (float*)(((uintptr_t)workspace + kRunAlign - 1) & ~(uintptr_t)(kRunAlign - 1));   // (the plan's bytes have room for it)
-        // (without counters the launch adds a kernel that sums the parts: the same bits)
-        p.finish = tuning.finish != -1 ? finish_counters_for(sp.run_tiles, s) : nullptr;
-        p.bias = bias;
-        return launch_gemm(dtype, op, p, nullptr, &sp, tuning, s) == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;
-      }
-      // the slice that arrives last at a tile finishes it (adds the slices in slice order, then the
-      // bias: the bits of the second kernel's sum) — unless told otherwise, or out of counters
-      p.finish = (tuning.finish != -1 && sp.splits <= finish_slices(sp.tile, p.I, p.J, p.R, dtype_bytes(dtype), tuning)) ? finish_counters_for(tile_count(p.I, p.J, sp.tile), s) : nullptr;
-      p.bias = p.finish != nullptr ? bias : nullptr;
-      if (launch_gemm(dtype, op, p, nullptr, &sp, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
-      if (p.finish != nullptr) return RZ_OK;
-      return reduce_slices_dtype(dtype, p.partial, p.C, bias, p.I, p.J, p.ldc, sp.splits, s) == hipSuccess
-                 ? RZ_OK : RZ_ERR_LAUNCH;
-    }
-    p.bias = bias;
-    return launch_gemm(dtype, op, p, nullptr, &sp, tuning, s) == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;
+    SplitPlan sp;
+    const int st = prepare_plain_op(dtype, p, bias, workspace, workspace_bytes, tuning, s, &sp);
+    if (st != RZ_OK) return st;
+    if (launch_gemm(dtype, op, p, nullptr, &sp, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
+    return finish_plain_op(dtype, p, bias, sp, s);
   }
+  p.stream_c = (size_t)p.I * (size_t)p.J * dtype_bytes(dtype) >= ((size_t)8 << 20) ? 1 : 0;
   p.bias = bias;
   return launch_gemm(dtype, op, p, nullptr, nullptr, tuning, s) == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;
+}
+
+// The input-grad that goes with a weight-grad call: its operands, and once prepared how it is carried out.
+struct InputGradCall {
+  GemmParams p;
+  void* workspace;
+  size_t workspace_bytes;
+  SplitPlan split;
+};
+
+// The contraction of a weight-grad, with the input-grad's in the same launch where `form` says so.
+static hipError_t launch_weight_contraction(int dtype, const GemmParams& p, const WeightGradPlan& plan, const InputGradCall* with,
+                                            const BackwardForm& form, const rz_tuning& tuning, hipStream_t s) {
+  if (with == nullptr || form.pair == kApart) return launch_gemm(dtype, kWeightGrad, p, &plan, nullptr, tuning, s);
+  switch (dtype) {
+    case RZ_F32: return launch_backward_f32(with->p, &with->split, p, &plan, form, s);
+    case RZ_BF16: return launch_backward_bf16(with->p, &with->split, p, &plan, form, s);
+    case RZ_F16: return launch_backward_f16(with->p, &with->split, p, &plan, form, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 static hipError_t zero_words(void* p, size_t bytes, hipStream_t s) {
@@ -448,7 +479,7 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
                             const int32_t R[8], float init_factor, int64_t ldx, int64_t lddy, int dtype,
                             unsigned flags, void* stream, int hash_levels = RZ_HASH_TWO_LEVEL,
                             const rz_tuning* tuning_arg = nullptr, const int32_t* layer_plan = nullptr,
-                            size_t layer_plan_bytes = 0, size_t limit = (size_t)-1) {
+                            size_t layer_plan_bytes = 0, size_t limit = (size_t)-1, InputGradCall* with = nullptr) {
   if (X == nullptr || dY == nullptr || dHW == nullptr) return RZ_ERR_NULL_POINTER;
   if (dtype_bytes(dtype) == 0) return RZ_ERR_BAD_DTYPE;
   if (M < 1 || ldx < K || lddy < N) return RZ_ERR_BAD_SHAPE;
@@ -478,6 +509,26 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
   const WeightGradWorkspace ws = weight_grad_workspace(plan, wp, H, dhw_dtype == RZ_F32, dbias != nullptr, planned);
   if (ws.total_bytes > 0 && (workspace == nullptr || workspace_bytes < ws.total_bytes)) return RZ_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
+  // (an input-grad that shares no launch with this call's contraction is enqueued first, like the reference's)
+  BackwardForm form = {};
+  if (with != nullptr) {
+    st = prepare_plain_op(dtype, with->p, nullptr, with->workspace, with->workspace_bytes, tuning, s, &with->split);
+    if (st != RZ_OK) return st;
+    if (!wp.use) {
+      const SplitPlan whole = backward_whole_tiles(M, K, N, with->split, plan);
+      if (whole.tile != 0) {
+        with->split = whole;
+        with->p.partial = nullptr;
+        with->p.finish = nullptr;
+      }
+      form = backward_form(M, K, N, H, with->split, plan, dbias != nullptr, dtype_bytes(dtype), tuning);
+    }
+    if (form.pair == kApart) {
+      if (launch_gemm(dtype, kInputGrad, with->p, nullptr, &with->split, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
+      st = finish_plain_op(dtype, with->p, nullptr, with->split, s);
+      if (st != RZ_OK) return st;
+    }
+  }
   p.A = X;
   p.B = dY;
   p.I = K;
@@ -547,7 +598,7 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
     const int tile_dtype = p.tiles_out_16 ? dtype : RZ_F32;
     p.out_tiles_k = (K + BK - 1) / BK;
     p.out_tiles_n = (N + BN - 1) / BN;
-    if (launch_gemm(dtype, kWeightGrad, p, &plan, nullptr, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
+    if (launch_weight_contraction(dtype, p, plan, with, form, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
     FoldParams fp;
     fp.bias = f.shares > 1 ? ColsumTail{} : bias;   // (carried by the last kernel)
     fp.tiles = p.tiles_out;
@@ -596,7 +647,7 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
     // every workgroup sums its tiles into an LDS image of dHW and stores it as a partial image;
     // the partial images are then added up (no global atomics, fixed summation order)
     p.scatter = (float*)workspace;
-    if (launch_gemm(dtype, kWeightGrad, p, &plan, nullptr, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
+    if (launch_weight_contraction(dtype, p, plan, with, form, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
     if (accumulate) launch_reduce_partials<true>(dhw_dtype, p.scatter, dHW, H, plan.image_pitch, (int)plan.workgroups, bias, s);
     else launch_reduce_partials<false>(dhw_dtype, p.scatter, dHW, H, plan.image_pitch, (int)plan.workgroups, bias, s);
   } else {
@@ -607,14 +658,15 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
         zero_words(image, (size_t)H * sizeof(float), s) != hipSuccess)
       return RZ_ERR_LAUNCH;
     p.scatter = image;
-    if (launch_gemm(dtype, kWeightGrad, p, &plan, nullptr, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
+    if (launch_weight_contraction(dtype, p, plan, with, form, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
     if (dhw_dtype != RZ_F32) {
       if (accumulate) launch_convert<true>(dhw_dtype, image, dHW, H, s);
       else launch_convert<false>(dhw_dtype, image, dHW, H, s);
     }
     if (bias.part != nullptr) hipLaunchKernelGGL(colsum_kernel, dim3(colsum_blocks(bias, 256)), dim3(256), 0, s, bias);
   }
-  return hipGetLastError() == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;
+  if (hipGetLastError() != hipSuccess) return RZ_ERR_LAUNCH;
+  return with != nullptr && form.pair != kApart ? finish_plain_op(dtype, with->p, nullptr, with->split, s) : RZ_OK;
 }
 
 // Workspace of a weight-grad call without a layer plan (0: bad arguments).
@@ -748,16 +800,14 @@ static int forward_impl(const void* X, const void* HW, const void* bias, void* Y
   return run_plain_op(kForward, dtype, p, bias, workspace, workspace_bytes, may_split, tuning, (hipStream_t)stream);
 }
 
-static int input_grad_impl(const void* dY, const void* HW, void* dX, void* workspace, size_t workspace_bytes,
-                           bool may_split, int M, int K, int N, int H, int BK, int BN, const int32_t R[8],
-                           float init_factor, int64_t lddy, int64_t lddx, int dtype, void* stream,
-                           int hash_levels = RZ_HASH_TWO_LEVEL, const rz_tuning* tuning_arg = nullptr) {
+static int input_grad_operands(GemmParams& p, const void* dY, const void* HW, void* dX, int M, int K, int N, int H, int BK, int BN,
+                               const int32_t R[8], float init_factor, int64_t lddy, int64_t lddx, int dtype, int hash_levels,
+                               const rz_tuning& tuning) {
   if (dY == nullptr || HW == nullptr || dX == nullptr) return RZ_ERR_NULL_POINTER;
   if (dtype_bytes(dtype) == 0) return RZ_ERR_BAD_DTYPE;
   if (M < 1 || lddy < N || lddx < K || !pitch_ok(lddy, dtype_bytes(dtype)) || !pitch_ok(lddx, dtype_bytes(dtype))) return RZ_ERR_BAD_SHAPE;
-  const rz_tuning tuning = tuning_or_default(tuning_arg);
   if (!tuning_valid(tuning)) return RZ_ERR_BAD_ARGUMENT;
-  GemmParams p = {};
+  p = {};
   int st = make_hash(&p.h, K, N, H, BK, BN, R, hash_levels);
   if (st != RZ_OK) return st;
   p.A = dY;
@@ -769,6 +819,17 @@ static int input_grad_impl(const void* dY, const void* HW, void* dX, void* works
   p.lda = lddy;
   p.ldc = lddx;
   p.scale = init_factor;
+  return RZ_OK;
+}
+
+static int input_grad_impl(const void* dY, const void* HW, void* dX, void* workspace, size_t workspace_bytes,
+                           bool may_split, int M, int K, int N, int H, int BK, int BN, const int32_t R[8],
+                           float init_factor, int64_t lddy, int64_t lddx, int dtype, void* stream,
+                           int hash_levels = RZ_HASH_TWO_LEVEL, const rz_tuning* tuning_arg = nullptr) {
+  const rz_tuning tuning = tuning_or_default(tuning_arg);
+  GemmParams p;
+  const int st = input_grad_operands(p, dY, HW, dX, M, K, N, H, BK, BN, R, init_factor, lddy, lddx, dtype, hash_levels, tuning);
+  if (st != RZ_OK) return st;
   return run_plain_op(kInputGrad, dtype, p, nullptr, workspace, workspace_bytes, may_split, tuning,
                       (hipStream_t)stream);
 }
@@ -1006,6 +1067,21 @@ RZ_API int rz_weight_grad_planned(const void* X, const void* dY, void* dHW, void
   return weight_grad_impl(X, dY, dHW, dbias, workspace, workspace_bytes, M, K, N, H, BK, BN, R, init_factor, ldx,
                           lddy, dtype, flags, stream, hash_levels, tuning, static_cast<const int32_t*>(layer_plan),
                           layer_plan_bytes);
+}
+
+RZ_API int rz_linear_backward_hashed(const void* X, const void* dY, const void* HW, void* dX, void* dHW, void* dbias, void* workspace_dx,
+                                     size_t workspace_dx_bytes, void* workspace_dhw, size_t workspace_dhw_bytes,
+                                     const void* layer_plan, size_t layer_plan_bytes, int M, int K, int N, int H, int BK, int BN,
+                                     const int32_t R[8], int hash_levels, float init_factor, int64_t ldx, int64_t lddy, int64_t lddx,
+                                     int dtype, unsigned flags, const rz_tuning* tuning, void* stream) {
+  InputGradCall with = {};
+  with.workspace = workspace_dx;
+  with.workspace_bytes = workspace_dx_bytes;
+  const int st = input_grad_operands(with.p, dY, HW, dX, M, K, N, H, BK, BN, R, init_factor, lddy, lddx, dtype, hash_levels,
+                                     tuning_or_default(tuning));
+  if (st != RZ_OK) return st;
+  return weight_grad_impl(X, dY, dHW, dbias, workspace_dhw, workspace_dhw_bytes, M, K, N, H, BK, BN, R, init_factor, ldx, lddy, dtype,
+                          flags, stream, hash_levels, tuning, static_cast<const int32_t*>(layer_plan), layer_plan_bytes, (size_t)-1, &with);
 }
 
 RZ_API int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int dtype, unsigned flags,

@@ -1,0 +1,9 @@
+// Instantiation of the backward pass in one launch for element type bf16_t.
+#include "rz_gemm_inst.h"
+
+namespace rz {
+hipError_t launch_backward_bf16(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, const BackwardForm& form,
+                        hipStream_t stream) {
+  return launch_backward_t<bf16_t>(ig, split, wg, plan, form, stream);
+}
+}  // namespace rz

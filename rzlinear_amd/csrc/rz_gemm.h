@@ -156,6 +156,10 @@ __device__ __forceinline__ u32x4_t shift_down_16(u32x4_t v, int sh) {
   return r;
 }
 
+// Wavefronts per SIMD that the register allocation has to leave room for: the workgroup's own — and two
+// workgroups' for the sixteen-wavefront form with two stages, which shares its compute unit.
+constexpr int gemm_waves_per_simd(int waves, int stages) { return waves == 16 && stages == 2 ? 8 : (waves + 3) / 4; }
+
 // COLSUM (weight-grad only): also sum the columns of B (dY) for the bias gradient.
 // CLAMP (with FULL = false): ragged shapes.  The last R step may be partial (its excess is
 // cleared in LDS) and the C tile grid may have ragged edges.  Tiles are then still staged directly: a piece that
@@ -182,6 +186,7 @@ struct GemmKernel {
   static_assert(!COLSUM || OP == kWeightGrad, "column sums belong to the weight-grad contraction");
   typedef ElemTraits<T> Tr;
   static constexpr int kThreads = 64 * WI * WJ * WK;
+  static constexpr int kWavesPerSimd = gemm_waves_per_simd(WI * WJ * WK, NSTAGE);
   static constexpr int VEC = Tr::kVec;
   static constexpr bool k16 = (Tr::kBytes == 2);
   // R step: 128 bytes of R — except the directly staged 16-bit 64 and 32 x 128 tiles, whose groups of wavefronts
@@ -389,10 +394,8 @@ struct GemmKernel {
     return r == 0 ? F : F + 1 + (((t + 1) * r - 1) / L * L > t * r ? 1 : 0);
   }
 
-  // One C tile and slice of the contracted dimension, chosen by the workgroup id.
-  static __device__ __forceinline__ void run(const GemmParams& p, Smem& sm) {
-    const int bx = blockIdx.x, gx = gridDim.x, gy = gridDim.y;
-    int by = blockIdx.y;
+  // One C tile and slice of the contracted dimension, chosen by the workgroup id (bx, by) of gx x gy.
+  static __device__ __forceinline__ void run(const GemmParams& p, Smem& sm, int bx, int by, int gx, int gy) {
     // Workgroup ids are dealt round-robin to the 8 XCDs; renumber so that each XCD (one L2)
     // gets a contiguous run of tiles, then walk tiles with J fastest (forward/input-grad
     // share the streamed A panel) or in square-ish groups (weight-grad streams both).
@@ -1854,7 +1857,7 @@ struct GemmKernel {
           }
         }
         if (!finishing) return;
-        const int slices = (int)gridDim.y;
+        const int slices = it.slices;
         unsigned* counter = p.finish + (size_t)ti * (size_t)p.tiles_j + tj;
         int* arrived = sm.off;   // (the offsets are no longer read)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wavefront's part of the plane is where the others will look
@@ -1960,15 +1963,29 @@ struct GemmKernel {
   }
 };
 
-// Wavefronts per SIMD that the register allocation has to leave room for: the workgroup's own — and two
-// workgroups' for the sixteen-wavefront form with two stages, which shares its compute unit.
-constexpr int gemm_waves_per_simd(int waves, int stages) { return waves == 16 && stages == 2 ? 8 : (waves + 3) / 4; }
-
 template <typename T, int OP, int TI, int TJ, int WI, int WJ, int NSTAGE, bool FULL, bool COLSUM, bool CLAMP, int WK = 1, bool SHORT = false>
 __global__ __launch_bounds__(64 * WI * WJ * WK, gemm_waves_per_simd(WI * WJ * WK, NSTAGE)) void rz_gemm_kernel(GemmParams p) {
   typedef GemmKernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK, SHORT> K;
   extern __shared__ __attribute__((aligned(16))) unsigned char rz_smem_raw[];
-  K::run(p, *reinterpret_cast<typename K::Smem*>(rz_smem_raw));
+  K::run(p, *reinterpret_cast<typename K::Smem*>(rz_smem_raw), blockIdx.x, blockIdx.y, gridDim.x, gridDim.y);
+}
+
+// Input-grad and weight-grad of one backward pass in one launch: the workgroups of the one, then those of the other (`wg_first`: which),
+// each as in its own kernel, with the same bits.  Neither reads what the other writes.
+struct BackwardGrid { int ig_x, ig_y, wg_x, wg_y, wg_first; };
+template <typename IG, typename WG>
+__global__ __launch_bounds__(IG::kThreads, IG::kWavesPerSimd > WG::kWavesPerSimd ? IG::kWavesPerSimd : WG::kWavesPerSimd) void rz_backward_kernel(GemmParams ig, GemmParams wg, BackwardGrid g) {
+  static_assert(IG::kThreads == WG::kThreads, "one workgroup size");
+  extern __shared__ __attribute__((aligned(16))) unsigned char rz_smem_raw[];
+  const int n_ig = g.ig_x * g.ig_y, n_wg = g.wg_x * g.wg_y, b = blockIdx.x;
+  const bool is_wg = g.wg_first ? b < n_wg : b >= n_ig;   // (uniform)
+  if (is_wg) {
+    const int id = g.wg_first ? b : b - n_ig, by = id / g.wg_x;
+    WG::run(wg, *reinterpret_cast<typename WG::Smem*>(rz_smem_raw), id - by * g.wg_x, by, g.wg_x, g.wg_y);
+  } else {
+    const int id = g.wg_first ? b - n_wg : b, by = id / g.ig_x;
+    IG::run(ig, *reinterpret_cast<typename IG::Smem*>(rz_smem_raw), id - by * g.ig_x, by, g.ig_x, g.ig_y);
+  }
 }
 
 // Forward / input-grad in runs of equal length (GemmKernel::run_all), and the kernel that adds a tile's parts up where that one could not.

@@ -9,12 +9,9 @@
 
 namespace rz {
 
-template <typename T, int OP, int TI, int TJ, int WI, int WJ, int NSTAGE, bool FULL, bool COLSUM, bool CLAMP = false,
-          int WK = 1, bool SHORT = false>
-static hipError_t launch_one(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
-                             hipStream_t stream) {
-  static std::atomic<uint64_t> lds_limit_raised{0};
-  typedef GemmKernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK, SHORT> K;
+// The fields of p that the launch of kernel K fills in, its grid and its LDS bytes.
+template <typename K, typename T, int OP, int TI, int TJ, bool COLSUM>
+static hipError_t prepare_one(GemmParams& p, const WeightGradPlan* plan, const SplitPlan* split, dim3* grid, size_t* smem) {
   p.tiles_i = (p.I + TI - 1) / TI;
   p.tiles_j = (p.J + TJ - 1) / TJ;
   const long long tiles = (long long)p.tiles_i * p.tiles_j;
@@ -52,20 +49,33 @@ static hipError_t launch_one(GemmParams p, const WeightGradPlan* plan, const Spl
     p.partial = nullptr;
     p.finish = nullptr;
   }
-  auto kernel = rz_gemm_kernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK, SHORT>;
-  size_t smem = sizeof(typename K::Smem);
+  *smem = sizeof(typename K::Smem);
   static_assert(sizeof(typename K::Smem) <= 160 * 1024, "tile does not fit the 160 KB LDS of a compute unit");
   if (OP == kWeightGrad && p.image_pitch > 0) {
     // the dHW image and the scatter's offset table behind it may need more than the stages
     const size_t need = (size_t)p.image_pitch * sizeof(float) + (K::kOffEntries + K::kTurnEntries) * sizeof(int);
-    if (need > smem) smem = need;
+    if (need > *smem) *smem = need;
   }
+  *grid = dim3((unsigned)tiles, (unsigned)splits, 1);
+  return hipSuccess;
+}
+
+template <typename T, int OP, int TI, int TJ, int WI, int WJ, int NSTAGE, bool FULL, bool COLSUM, bool CLAMP = false,
+          int WK = 1, bool SHORT = false>
+static hipError_t launch_one(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
+                             hipStream_t stream) {
+  static std::atomic<uint64_t> lds_limit_raised{0};
+  typedef GemmKernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK, SHORT> K;
+  dim3 grid;
+  size_t smem;
+  hipError_t e = prepare_one<K, T, OP, TI, TJ, COLSUM>(p, plan, split, &grid, &smem);
+  if (e != hipSuccess) return e;
+  auto kernel = rz_gemm_kernel<T, OP, TI, TJ, WI, WJ, NSTAGE, FULL, COLSUM, CLAMP, WK, SHORT>;
   if (smem > 64 * 1024) {
-    hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds_limit_raised);
+    e = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds_limit_raised);
     if (e != hipSuccess) return e;
   }
-  dim3 grid((unsigned)tiles, (unsigned)splits, 1), block(K::kThreads, 1, 1);
-  hipLaunchKernelGGL(kernel, grid, block, smem, stream, p);
+  hipLaunchKernelGGL(kernel, grid, dim3(K::kThreads), smem, stream, p);
   return hipGetLastError();
 }
 
@@ -87,7 +97,7 @@ static hipError_t launch_tile(GemmParams p, const WeightGradPlan* plan, const Sp
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false>::TR) return hipErrorInvalidValue;
     return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, false, WK>(p, plan, split, stream);
   }
-  // (the 16-bit 64 tile of four wavefronts, and the 128 tile of eight with two stages, serve rows shorter than a 16-byte piece only)
+  // (the 64 tile of four wavefronts, and the 16-bit 128 tile of eight with two stages, serve rows shorter than a 16-byte piece only)
   // (16-bit 256 tile, a few R steps)
   if constexpr (sizeof(T) == 2 && TILE == 256 && TILE_J == 256) if (form.short_loop) {
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true, false, false, WK, true>::TR) return hipErrorInvalidValue;
@@ -95,7 +105,7 @@ static hipError_t launch_tile(GemmParams p, const WeightGradPlan* plan, const Sp
     if (form.clamp) return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, true, WK, true>(p, plan, split, stream);
     return hipErrorInvalidValue;
   }
-  constexpr bool kCheckedOnly = sizeof(T) == 2 && WK == 1 && (TILE == 64 || (TILE == 128 && WI * WJ == 8 && NSTAGE == 2));
+  constexpr bool kCheckedOnly = WK == 1 && (TILE == 64 || (sizeof(T) == 2 && TILE == 128 && WI * WJ == 8 && NSTAGE == 2));
   if constexpr (!kCheckedOnly) if (form.full) {
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true>::TR) return hipErrorInvalidValue;
     return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true, COLSUM, false, WK>(p, plan, split, stream);
@@ -119,13 +129,9 @@ template <typename T, int OP, int TILE, int WI, int WJ, int NSTAGE, int WK = 1>
 static hipError_t launch_op(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split,
                             const KernelForm& form, hipStream_t stream) {
   if constexpr (OP == kWeightGrad) {
-    if constexpr (WK > 1 && sizeof(T) == 4) {
-      return hipErrorInvalidValue;   // (groups of wavefronts share an R step in the fp32 store kernels only)
-    } else {
-      // with a column-sum target the kernel also produces the bias gradient's partial sums
-      if (p.colsum != nullptr) return launch_tile<T, OP, TILE, WI, WJ, NSTAGE, true, WK>(p, plan, split, form, stream);
-      return launch_tile<T, OP, TILE, WI, WJ, NSTAGE, false, WK>(p, plan, split, form, stream);
-    }
+    // with a column-sum target the kernel also produces the bias gradient's partial sums
+    if (p.colsum != nullptr) return launch_tile<T, OP, TILE, WI, WJ, NSTAGE, true, WK>(p, plan, split, form, stream);
+    return launch_tile<T, OP, TILE, WI, WJ, NSTAGE, false, WK>(p, plan, split, form, stream);
   } else {
     return launch_tile<T, OP, TILE, WI, WJ, NSTAGE, false, WK>(p, plan, split, form, stream);
   }
@@ -139,8 +145,7 @@ static hipError_t launch_op(GemmParams p, const WeightGradPlan* plan, const Spli
 //        instead of a pipeline (tuning aid)
 //        16-bit forward / input-grad: 256 x 128, eight wavefronts of 64 x 64, three LDS stages, where pairs are faster
 //    64:  64 x  64, for problems with few tiles: 16-bit sixteen wavefronts of 32 x 32 in four groups that
-//        share every R step between them; fp32 forward / input-grad eight, in two such groups; fp32
-//        weight-grad, and 16-bit rows shorter than a 16-byte piece, four
+//        share every R step between them; fp32 eight, in two such groups; rows shorter than a 16-byte piece (fp32: weight-grad), four
 //        16-bit forward / input-grad of at most 32 rows: 32 x 128 (eight wavefronts of 32 x 32 in two groups
 //        that share every R step, three LDS stages)
 //    32:  32 x  64 (fp32 forward / input-grad whose rows would leave a 64-row tile at most half full): four wavefronts of 32 x 32 in two such groups
@@ -199,14 +204,16 @@ static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const 
   if (form.rows != form.tile || form.cols != tile_cols(form.tile)) return hipErrorInvalidValue;
   switch (form.tile * 1000 + form.waves * 10 + form.stages) {
     case 256082: return launch_op<T, OP, 256, 2, 4, 2>(p, plan, split, form, stream);
-    case 64042: return launch_op<T, OP, 64, 2, 2, 2>(p, plan, split, form, stream);
+    case 64042:
+      if constexpr (sizeof(T) == 2 || OP == kWeightGrad) return launch_op<T, OP, 64, 2, 2, 2>(p, plan, split, form, stream);
+      return hipErrorInvalidValue;
     case 64164:   // 16-bit, at most one workgroup per compute unit: four groups of four wavefronts share every R step
       if constexpr (sizeof(T) == 2) return launch_op<T, OP, 64, 2, 2, 4, 4>(p, plan, split, form, stream);
       return hipErrorInvalidValue;
     case 64162:   // ... more of them: two LDS stages
       if constexpr (sizeof(T) == 2) return launch_op<T, OP, 64, 2, 2, 2, 4>(p, plan, split, form, stream);
       return hipErrorInvalidValue;
-    case 64082:   // fp32 forward / input-grad: two groups of four wavefronts share every R step
+    case 64082:   // fp32: two groups of four wavefronts share every R step
       if constexpr (sizeof(T) == 4) return launch_op<T, OP, 64, 2, 2, 2, 2>(p, plan, split, form, stream);
       return hipErrorInvalidValue;
     case 32042:   // fp32 forward / input-grad, rows in 32s: 32 x 64, two groups of two wavefronts
@@ -220,6 +227,62 @@ static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const 
     case 128042: return launch_op<T, OP, 128, 2, 2, 2>(p, plan, split, form, stream);
     default: return hipErrorInvalidValue;
   }
+}
+
+// The two kernels of a backward pass in one launch.  What a boundary between two launches costs a GPU that is waiting for it is 5 to 6 us, and
+// the host a launch; where neither op fills the chip their workgroups run side by side as well.  GPU-bound, with what finishes dHW (apart / in
+// one launch, us): bf16 M = 78, K = 752, N = 133 17.2 / 11.4; M = 160, K = 448, N = 1216 22.6 / 15.0; M = 6016, K = 3200, N = 1600 156 / 135;
+// fp16 M = 3663, K = 13603, N = 1370 360 / 294; fp32 M = 2025, K = 848, N = 1941 148 / 131; 1024^3 through the module, forward included, 68.9 / 63.6.  Over 90
+// drawn shapes none slower by more than runs differ.  Not with the 256 x 128 and 128 tiles: M = 2048, K = 4096, N = 1024 4 us slower (two kernels of full rounds).
+template <typename T, int TI, int TJ, int WI, int WJ, int IG_STAGES, int WK, int TILE, int WG_WI, int WG_WJ, int WG_STAGES, int WG_WK, bool FULL>
+static hipError_t launch_backward_form(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, bool wg_first,
+                                       hipStream_t stream) {
+  static std::atomic<uint64_t> lds_limit_raised{0};
+  typedef GemmKernel<T, kInputGrad, TI, TJ, WI, WJ, IG_STAGES, FULL, false, !FULL, WK> IG;
+  typedef GemmKernel<T, kWeightGrad, TILE, TILE, WG_WI, WG_WJ, WG_STAGES, FULL, true, !FULL, WG_WK> WG;
+  dim3 ig_grid, wg_grid;
+  size_t ig_smem, smem;
+  hipError_t e = prepare_one<IG, T, kInputGrad, TI, TJ, false>(ig, nullptr, split, &ig_grid, &ig_smem);
+  if (e == hipSuccess) e = prepare_one<WG, T, kWeightGrad, TILE, TILE, true>(wg, plan, nullptr, &wg_grid, &smem);
+  if (e != hipSuccess) return e;
+  if (ig_smem > smem) smem = ig_smem;
+  const long long groups = (long long)ig_grid.x * ig_grid.y + (long long)wg_grid.x * wg_grid.y;
+  if (groups > 0x7fffffffLL) return hipErrorInvalidValue;
+  auto kernel = rz_backward_kernel<IG, WG>;
+  if (smem > 64 * 1024) {
+    e = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds_limit_raised);
+    if (e != hipSuccess) return e;
+  }
+  const BackwardGrid g = {(int)ig_grid.x, (int)ig_grid.y, (int)wg_grid.x, (int)wg_grid.y, wg_first ? 1 : 0};
+  hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(IG::kThreads), smem, stream, ig, wg, g);
+  return hipGetLastError();
+}
+
+template <typename T, int TI, int TJ, int WI, int WJ, int IG_STAGES, int WK, int TILE, int WG_WI, int WG_WJ, int WG_STAGES, int WG_WK>
+static hipError_t launch_backward_pair(const GemmParams& ig, const SplitPlan* split, const GemmParams& wg, const WeightGradPlan* plan,
+                                       const BackwardForm& form, hipStream_t stream) {
+  if (form.full) return launch_backward_form<T, TI, TJ, WI, WJ, IG_STAGES, WK, TILE, WG_WI, WG_WJ, WG_STAGES, WG_WK, true>(ig, split, wg, plan, form.wg_first, stream);
+  return launch_backward_form<T, TI, TJ, WI, WJ, IG_STAGES, WK, TILE, WG_WI, WG_WJ, WG_STAGES, WG_WK, false>(ig, split, wg, plan, form.wg_first, stream);
+}
+
+template <typename T>
+static hipError_t launch_backward_t(const GemmParams& ig, const SplitPlan* split, const GemmParams& wg, const WeightGradPlan* plan,
+                                    const BackwardForm& form, hipStream_t stream) {
+  if constexpr (sizeof(T) == 4) {
+    if (form.pair == k64With64) return launch_backward_pair<T, 64, 64, 2, 2, 2, 2, 64, 2, 2, 2, 2>(ig, split, wg, plan, form, stream);
+  } else {
+    switch (form.pair) {
+      case k64With64:
+        if (form.stages == 4) return launch_backward_pair<T, 64, 64, 2, 2, 4, 4, 64, 2, 2, 4, 4>(ig, split, wg, plan, form, stream);
+        return launch_backward_pair<T, 64, 64, 2, 2, 2, 4, 64, 2, 2, 2, 4>(ig, split, wg, plan, form, stream);
+      case k64With128: return launch_backward_pair<T, 64, 64, 2, 2, 4, 4, 128, 4, 4, 4, 1>(ig, split, wg, plan, form, stream);
+      case kPairWith256: return launch_backward_pair<T, 256, 128, 4, 2, 3, 1, 256, 2, 4, 2, 1>(ig, split, wg, plan, form, stream);
+      case k256With256: return launch_backward_pair<T, 256, 256, 2, 4, 2, 1, 256, 2, 4, 2, 1>(ig, split, wg, plan, form, stream);
+      case k128With128: return launch_backward_pair<T, 128, 128, 2, 4, 4, 1, 128, 2, 4, 4, 1>(ig, split, wg, plan, form, stream);
+      default: break;
+    }
+  }
+  return hipErrorInvalidValue;
 }
 
 template <typename T, int TBN, int OPERANDS, bool WHOLE>

@@ -1125,7 +1125,7 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
   f.step = (f.full || f.clamp) ? step_direct : step_plain;
   f.waves = tile == 256 ? 8
             : tile == 32 ? 4
-            : tile == 64 ? ((many64 && (f.full || f.clamp)) ? 16 : (elem_bytes == 4 && op != kWeightGrad) ? 8 : 4)
+            : tile == 64 ? ((many64 && (f.full || f.clamp)) ? 16 : (elem_bytes == 4 && (op != kWeightGrad || f.full || f.clamp)) ? 8 : 4)
                          : waves128;
   if (tile == 128 && f.waves == 8 && elem_bytes == 2 && (f.full || f.clamp)) f.stages = 4;
   if (f.waves == 16) f.stages = workgroups <= kComputeUnits ? 4 : 2;
@@ -1153,6 +1153,69 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
   f.short_loop = elem_bytes == 2 && tile == 256 && (f.full || f.clamp) && short_loop(op, f.full, ((chunk < R ? chunk : R) + 63) / 64);
   return f;
 }
+
+// An input-grad planned in runs, beside a weight-grad on the same tile in one launch: its tiles whole, since what they leave idle the
+// weight-grad's workgroups fill and no planes are needed.  tile = 0: in runs, as by itself.  By the times that forward16_us was fitted to:
+// the launch takes the sum of what its workgroups take, spread over the compute units, and half a workgroup of the op whose
+// workgroups come last, but no less than the longest.  (M = 1024, K = N = 10240 bf16: 181 + 199 us in runs and apart, 347 in one launch.)
+static inline SplitPlan backward_whole_tiles(int M, int K, int N, const SplitPlan& sp, const WeightGradPlan& plan) {
+  SplitPlan whole = {};
+  if (sp.run_steps == 0 || sp.tile != 256 || plan.tile != 256) return whole;
+  const Forward16Times& c = kForward16Times[6];
+  const double step = c.step + c.step_fill, fixed = c.round + c.round_fill;
+  const double ig_us = (double)((N + 63) / 64) * step + fixed, wg_us = (double)((plan.r_chunk + 63) / 64) * step + fixed;
+  const double ig_wgs = (double)tile_count(M, K, 256), wg_wgs = (double)plan.workgroups;
+  const double spread = (ig_wgs * ig_us + wg_wgs * wg_us) / kComputeUnits + 0.5 * (ig_us < wg_us ? ig_us : wg_us);
+  const double longest = ig_us > wg_us ? ig_us : wg_us, together = c.launch + (spread > longest ? spread : longest);
+  const double apart = sp.est_us + c.launch + (double)(((long long)plan.workgroups + kComputeUnits - 1) / kComputeUnits) * wg_us;
+  if (together >= 0.97 * apart) return whole;
+  whole.tile = 256;
+  whole.splits = 1;
+  whole.r_chunk = N;
+  whole.est_us = together;
+  return whole;
+}
+
+// Input-grad and weight-grad of one backward pass in one launch (rz_backward_kernel): which pair of kernels, kApart where the two
+// have no launch in common.
+enum BackwardPair { kApart = 0, k64With64, k64With128, kPairWith256, k256With256, k128With128 };
+struct BackwardForm {
+  int pair;
+  bool full;      // both without bounds checks (else both with)
+  int stages;     // of the 16-bit 64 tiles
+  bool wg_first;  // whose workgroups come first in the grid: those that take longer
+};
+static inline BackwardForm backward_form(int M, int K, int N, int H, const SplitPlan& sp, const WeightGradPlan& plan, bool with_dbias,
+                                         int elem_bytes, const rz_tuning& t) {
+  BackwardForm b = {kApart, false, 2, false};
+  if (!with_dbias || sp.run_steps > 0 || t.tile != 0 || t.stages == 1 || t.clamp == -1 || (long long)H * 4 > 0x7fffffffLL) return b;
+  const long long ig_wgs = tile_count(M, K, sp.tile) * sp.splits;
+  const KernelForm i = kernel_form(kInputGrad, M, K, N, sp.splits > 1 ? sp.r_chunk : N, sp.tile, ig_wgs, elem_bytes, t);
+  const KernelForm w = kernel_form(kWeightGrad, K, N, M, plan.r_chunk, plan.tile, plan.workgroups, elem_bytes, t);
+  if (!(i.full || i.clamp) || !(w.full || w.clamp) || i.short_loop || w.short_loop) return b;
+  const bool pair = i.rows == 256 && i.cols == 128;
+  if (i.rows != i.cols && !pair) return b;
+  b.full = i.full && w.full;
+  if (i.rows == 64 && w.tile == 64) {
+    b.pair = k64With64;
+    b.stages = elem_bytes == 2 && ig_wgs + plan.workgroups <= kComputeUnits ? 4 : 2;
+  } else if (elem_bytes == 2 && i.rows == 64 && w.tile == 128 && w.waves == 8) {
+    // (the 128 tile by sixteen wavefronts of 32 x 32 here: a third more LDS traffic, for a few steps)
+    if (ig_wgs <= kComputeUnits && plan.r_chunk <= 2048) b.pair = k64With128;
+  } else if (elem_bytes == 2 && pair && w.tile == 256) {
+    b.pair = kPairWith256;
+  } else if (elem_bytes == 2 && i.rows == 256 && w.tile == 256) {
+    b.pair = k256With256;
+  } else if (elem_bytes == 2 && i.rows == 128 && i.waves == 8 && w.tile == 128 && w.waves == 8) {
+    b.pair = k128With128;
+  }
+  const double ig_work = (double)i.rows * i.cols * (sp.splits > 1 ? sp.r_chunk : N), wg_work = (double)w.tile * w.tile * plan.r_chunk;
+  b.wg_first = wg_work > ig_work;
+  return b;
+}
+hipError_t launch_backward_f32(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, const BackwardForm& form, hipStream_t stream);
+hipError_t launch_backward_bf16(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, const BackwardForm& form, hipStream_t stream);
+hipError_t launch_backward_f16(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, const BackwardForm& form, hipStream_t stream);
 
 // Fill in the tiling fields of `p` and enqueue the kernel of one op and element type on `stream`; weight-grad
 // takes its plan (tile, split of M, scatter mode) from `plan`, the others ignore it.

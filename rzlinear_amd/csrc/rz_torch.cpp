@@ -54,6 +54,7 @@ struct Library {
   decltype(&rz_weight_grad_hashed) weight_grad = nullptr;
   decltype(&rz_weight_grad_planned) weight_grad_planned = nullptr;
   decltype(&rz_weight_grad_hashed_workspace_bytes) weight_grad_workspace = nullptr;
+  decltype(&rz_linear_backward_hashed) backward = nullptr;
   decltype(&rz_plan_query) plan_query = nullptr;
 };
 Library lib;
@@ -194,8 +195,9 @@ Tensor input_grad(const Geometry& g, const Tensor& dy, int64_t lddy, const Tenso
   return dx;
 }
 
+// (hw defined: the input gradient too, into *dx)
 void weight_grad(const Geometry& g, const Tensor& input, const Tensor& dy, int64_t lddy, const Tensor& out, bool accumulate,
-                 const Tensor& dbias, bool with_plans) {
+                 const Tensor& dbias, bool with_plans, const Tensor& hw, Tensor* dx) {
   int64_t ldx;
   const Tensor x = rows(input, &ldx);
   const int M = (int)x.size(0), code = dtype_code(dy.scalar_type());
@@ -214,7 +216,14 @@ void weight_grad(const Geometry& g, const Tensor& input, const Tensor& dy, int64
   const size_t need = lib.weight_grad_workspace(M, g.K, g.N, g.H, g.BK, g.BN, code, flags, with_dbias, t);
   const at::DataPtr ws = scratch(need);
   void* db = dbias.defined() ? dbias.data_ptr() : nullptr;
-  if (plan.defined())
+  if (hw.defined()) {
+    *dx = empty({M, g.K}, dy);
+    const size_t need_dx = lib.input_grad_workspace(M, g.K, g.N, g.H, g.BK, g.BN, code, t);
+    const at::DataPtr ws_dx = scratch(need_dx);
+    check(lib.backward(x.data_ptr(), dy.data_ptr(), hw.data_ptr(), dx->data_ptr(), out.data_ptr(), db, ws_dx.get(), need_dx, ws.get(), need,
+                       plan.defined() ? plan.data_ptr<int32_t>() : nullptr, plan.defined() ? (size_t)plan.numel() * 4 : 0, M, g.K, g.N, g.H,
+                       g.BK, g.BN, g.R, RZ_HASH_TWO_LEVEL, g.scale, ldx, lddy, g.K, code, flags, t, stream_of(dy)));
+  } else if (plan.defined())
     check(lib.weight_grad_planned(x.data_ptr(), dy.data_ptr(), out.data_ptr(), db, ws.get(), need, plan.data_ptr<int32_t>(),
                                   (size_t)plan.numel() * 4, M, g.K, g.N, g.H, g.BK, g.BN, g.R, RZ_HASH_TWO_LEVEL, g.scale, ldx, lddy,
                                   code, flags, t, stream_of(dy)));
@@ -337,7 +346,7 @@ struct RzLinearNode : public Node {
     at::DeviceGuard guard(grad.device());
     int64_t lddy;
     const Tensor dy = rows(grad, &lddy);
-    if (need_input) result[kInput] = input_grad(g, dy, lddy, hw.contiguous());   // (enqueued first, like the reference)
+    if (need_input && !need_weight) result[kInput] = input_grad(g, dy, lddy, hw.contiguous());
     if (need_weight) {   // (with a bias: one pass over dy yields both gradients)
       if (need_bias) bias_grad = empty({g.N}, dy);
       bool accumulate = false;
@@ -347,7 +356,7 @@ struct RzLinearNode : public Node {
       } else {
         out = result[kWeight] = empty({g.H}, dy);
       }
-      weight_grad(g, x, dy, lddy, out, accumulate, bias_grad, with_plans);
+      weight_grad(g, x, dy, lddy, out, accumulate, bias_grad, with_plans, need_input ? hw.contiguous() : Tensor(), &result[kInput]);
     } else if (need_bias) {
       bias_grad = grad.sum(0);
     }
@@ -479,6 +488,7 @@ PyObject* bind(PyObject*, PyObject* args) {
   RZ_BIND(weight_grad, rz_weight_grad_hashed);
   RZ_BIND(weight_grad_planned, rz_weight_grad_planned);
   RZ_BIND(weight_grad_workspace, rz_weight_grad_hashed_workspace_bytes);
+  RZ_BIND(backward, rz_linear_backward_hashed);
   RZ_BIND(plan_query, rz_plan_query);
 #undef RZ_BIND
   Py_INCREF(provider);

@@ -14,23 +14,27 @@ def rz_linear_backward_tl(input: torch.Tensor, hashed_weight: torch.Tensor, outp
                           allow_tf32: bool = True, allow_autotune: bool = False,
                           BLOCK_SIZE_M: int = 64, BLOCK_SIZE_N: int = 64, BLOCK_SIZE_K: int = 32,
                           GROUP_SIZE: int = 4) -> Tuple[torch.Tensor, torch.Tensor]:
-    """(input_grad, weight_grad), input-grad enqueued first as in the reference
-    (python/rz_linear/impl/RzLinearBackward.py:7-20)."""
-    input_grad = rz_linear_backward_input_grad_tl(
-        output_grad, hashed_weight, init_factor, M, K, N, H, R7, R6, R5, R4, R3, R2, R1, R0,
-        allow_tf32=allow_tf32, allow_autotune=allow_autotune, BLOCK_SIZE_M=BLOCK_SIZE_M,
-        BLOCK_SIZE_N=BLOCK_SIZE_N, BLOCK_SIZE_K=BLOCK_SIZE_K, GROUP_SIZE=GROUP_SIZE)
-    weight_grad = rz_linear_backward_weight_grad_tl(
-        input, output_grad, init_factor, M, K, N, H, R7, R6, R5, R4, R3, R2, R1, R0,
-        allow_tf32=allow_tf32, allow_autotune=allow_autotune, BLOCK_SIZE_M=BLOCK_SIZE_M,
-        BLOCK_SIZE_N=BLOCK_SIZE_N, BLOCK_SIZE_K=BLOCK_SIZE_K, GROUP_SIZE=GROUP_SIZE)
-    return input_grad, weight_grad
+    """(input_grad, weight_grad), as in the reference (python/rz_linear/impl/RzLinearBackward.py:7-20)."""
+    assert (H > (BLOCK_SIZE_K * BLOCK_SIZE_N))
+    R = _lib.hash_constants(R7, R6, R5, R4, R3, R2, R1, R0)
+    return backward_hashed(input, hashed_weight, output_grad, init_factor, M, K, N, H, R, BLOCK_SIZE_K, BLOCK_SIZE_N)[:2]
+
+
+def backward_hashed(input, hashed_weight, output_grad, init_factor, M, K, N, H, R, BLOCK_SIZE_K, BLOCK_SIZE_N, out=None,
+                    accumulate=False, with_bias_grad=False, hash_levels=_lib.HASH_TWO_LEVEL):
+    """(input_grad, hashed_weight_grad, bias_grad or None) by one call of rz_linear_backward_hashed, which enqueues the two
+    contractions as one launch where their kernels go together; arguments as weight_grad_hashed."""
+    weight_grad, bias_grad, input_grad = weight_grad_hashed(input, output_grad, init_factor, M, K, N, H, R, BLOCK_SIZE_K, BLOCK_SIZE_N,
+                                                            out=out, accumulate=accumulate, with_bias_grad=with_bias_grad,
+                                                            hash_levels=hash_levels, hashed_weight=hashed_weight)
+    return input_grad, weight_grad, bias_grad
 
 
 def weight_grad_hashed(input, output_grad, init_factor, M, K, N, H, R, BLOCK_SIZE_K, BLOCK_SIZE_N,
                        out=None, accumulate=False, with_bias_grad=False, hash_levels=_lib.HASH_TWO_LEVEL,
-                       use_layer_plan=None):
-    """One weight-grad call; returns (hashed_weight_grad, bias_grad or None).
+                       use_layer_plan=None, hashed_weight=None):
+    """One weight-grad call; returns (hashed_weight_grad, bias_grad or None) — with hashed_weight the whole backward
+    pass, and the input gradient as a third value.
 
     Where the library would work by windows of dHW or fold stored tiles into dHW (a hashed_weight
     too large for an image in LDS), the call goes through rz_weight_grad_planned with the layer's
@@ -41,6 +45,11 @@ def weight_grad_hashed(input, output_grad, init_factor, M, K, N, H, R, BLOCK_SIZ
     stream = _lib.require_gpu(input, output_grad)
     if input.dtype != output_grad.dtype:
         raise TypeError("input is %s but output_grad is %s" % (input.dtype, output_grad.dtype))
+    both = hashed_weight is not None
+    if both:
+        _lib.require_gpu(output_grad, hashed_weight)
+        if hashed_weight.dtype != output_grad.dtype:
+            raise TypeError("output_grad is %s but hashed_weight is %s" % (output_grad.dtype, hashed_weight.dtype))
     lib = _lib.load()
     code = _lib.dtype_code(output_grad)
     flags = 0
@@ -61,7 +70,10 @@ def weight_grad_hashed(input, output_grad, init_factor, M, K, N, H, R, BLOCK_SIZ
     if M == 0:   # an empty batch contributes a zero gradient (the reference returns its zeros(H))
         if not accumulate:
             out.zero_()
-        return out, (torch.zeros((N,), device=output_grad.device, dtype=output_grad.dtype) if with_bias_grad else None)
+        bias_grad = torch.zeros((N,), device=output_grad.device, dtype=output_grad.dtype) if with_bias_grad else None
+        if both:
+            return out, bias_grad, torch.empty((0, K), device=output_grad.device, dtype=output_grad.dtype)
+        return out, bias_grad
     x, ldx = _lib.rows(input)
     dy, lddy = _lib.rows(output_grad)
     bias_grad = torch.empty((N,), device=output_grad.device, dtype=output_grad.dtype) if with_bias_grad else None
@@ -75,6 +87,18 @@ def weight_grad_hashed(input, output_grad, init_factor, M, K, N, H, R, BLOCK_SIZ
     if use_layer_plan and _lib.plan_query(2, M, K, N, H, BLOCK_SIZE_K, BLOCK_SIZE_N, code, flags,
                                           with_bias_grad, planned=True)["mode"] in ("window", "fold"):
         plan = _lib.layer_plan_for_call(K, N, H, BLOCK_SIZE_K, BLOCK_SIZE_N, R, hash_levels, output_grad.device)
+    if both:
+        hw = hashed_weight.contiguous()
+        input_grad = torch.empty((M, K), device=output_grad.device, dtype=output_grad.dtype)
+        need_dx = _lib.host_query("rz_input_grad_hashed_workspace_bytes", M, K, N, H, BLOCK_SIZE_K, BLOCK_SIZE_N, code)
+        ws_dx = _lib.workspace(need_dx, output_grad.device)
+        _lib.check(lib.rz_linear_backward_hashed(
+            x.data_ptr(), dy.data_ptr(), hw.data_ptr(), input_grad.data_ptr(), out.data_ptr(),
+            bias_grad.data_ptr() if with_bias_grad else None, ws_dx.data_ptr() if need_dx else None, need_dx,
+            ws.data_ptr() if need else None, need, plan.data_ptr() if plan is not None else None,
+            plan.numel() * 4 if plan is not None else 0, M, K, N, H, BLOCK_SIZE_K, BLOCK_SIZE_N, R, hash_levels,
+            float(init_factor), ldx, lddy, K, code, flags, tuning, stream))
+        return out, bias_grad, input_grad
     if plan is not None:
         _lib.check(lib.rz_weight_grad_planned(
             x.data_ptr(), dy.data_ptr(), out.data_ptr(), bias_grad.data_ptr() if with_bias_grad else None,
