@@ -233,7 +233,7 @@ static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const 
 // the host a launch; where neither op fills the chip their workgroups run side by side as well.  GPU-bound, with what finishes dHW (apart / in
 // one launch, us): bf16 M = 78, K = 752, N = 133 17.2 / 11.4; M = 160, K = 448, N = 1216 22.6 / 15.0; M = 6016, K = 3200, N = 1600 156 / 135;
 // fp16 M = 3663, K = 13603, N = 1370 360 / 294; fp32 M = 2025, K = 848, N = 1941 148 / 131; 1024^3 through the module, forward included, 68.9 / 63.6.  Over 90
-// drawn shapes none slower by more than runs differ.  Not with the 256 x 128 and 128 tiles: M = 2048, K = 4096, N = 1024 4 us slower (two kernels of full rounds).
+// drawn shapes none slower by more than runs differ.
 template <typename T, int TI, int TJ, int WI, int WJ, int IG_STAGES, int WK, int TILE, int WG_WI, int WG_WJ, int WG_STAGES, int WG_WK, bool FULL>
 static hipError_t launch_backward_form(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, bool wg_first,
                                        hipStream_t stream) {
@@ -276,6 +276,7 @@ static hipError_t launch_backward_t(const GemmParams& ig, const SplitPlan* split
         if (form.stages == 4) return launch_backward_pair<T, 64, 64, 2, 2, 4, 4, 64, 2, 2, 4, 4>(ig, split, wg, plan, form, stream);
         return launch_backward_pair<T, 64, 64, 2, 2, 2, 4, 64, 2, 2, 2, 4>(ig, split, wg, plan, form, stream);
       case k64With128: return launch_backward_pair<T, 64, 64, 2, 2, 4, 4, 128, 4, 4, 4, 1>(ig, split, wg, plan, form, stream);
+      case kPairWith128: return launch_backward_pair<T, 256, 128, 4, 2, 3, 1, 128, 2, 4, 4, 1>(ig, split, wg, plan, form, stream);
       case kPairWith256: return launch_backward_pair<T, 256, 128, 4, 2, 3, 1, 256, 2, 4, 2, 1>(ig, split, wg, plan, form, stream);
       case k256With256: return launch_backward_pair<T, 256, 256, 2, 4, 2, 1, 256, 2, 4, 2, 1>(ig, split, wg, plan, form, stream);
       case k128With128: return launch_backward_pair<T, 128, 128, 2, 4, 4, 1, 128, 2, 4, 4, 1>(ig, split, wg, plan, form, stream);

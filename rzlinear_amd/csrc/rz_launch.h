@@ -1178,7 +1178,7 @@ static inline SplitPlan backward_whole_tiles(int M, int K, int N, const SplitPla
 
 // Input-grad and weight-grad of one backward pass in one launch (rz_backward_kernel): which pair of kernels, kApart where the two
 // have no launch in common.
-enum BackwardPair { kApart = 0, k64With64, k64With128, kPairWith256, k256With256, k128With128 };
+enum BackwardPair { kApart = 0, k64With64, k64With128, kPairWith128, kPairWith256, k256With256, k128With128 };
 struct BackwardForm {
   int pair;
   bool full;      // both without bounds checks (else both with)
@@ -1202,6 +1202,8 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
   } else if (elem_bytes == 2 && i.rows == 64 && w.tile == 128 && w.waves == 8) {
     // (the 128 tile by sixteen wavefronts of 32 x 32 here: a third more LDS traffic, for a few steps)
     if (ig_wgs <= kComputeUnits && plan.r_chunk <= 2048) b.pair = k64With128;
+  } else if (elem_bytes == 2 && pair && w.tile == 128 && w.waves == 8) {
+    b.pair = kPairWith128;
   } else if (elem_bytes == 2 && pair && w.tile == 256) {
     b.pair = kPairWith256;
   } else if (elem_bytes == 2 && i.rows == 256 && w.tile == 256) {
@@ -1210,7 +1212,9 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
     b.pair = k128With128;
   }
   const double ig_work = (double)i.rows * i.cols * (sp.splits > 1 ? sp.r_chunk : N), wg_work = (double)w.tile * w.tile * plan.r_chunk;
-  b.wg_first = wg_work > ig_work;
+  // (the 128 tile takes longer for its work than a pair of them: M = 2048, K = 4096, N = 1024, a round of compute units each, apart 51.4 us, the input-grad's first
+  //  50.7, the weight-grad's 48.3)
+  b.wg_first = b.pair == kPairWith128 ? 4 * wg_work > 3 * ig_work : wg_work > ig_work;
   return b;
 }
 hipError_t launch_backward_f32(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, const BackwardForm& form, hipStream_t stream);
