@@ -279,6 +279,7 @@ static hipError_t launch_backward_t(const GemmParams& ig, const SplitPlan* split
       case kPairWith128: return launch_backward_pair<T, 256, 128, 4, 2, 3, 1, 128, 2, 4, 4, 1>(ig, split, wg, plan, form, stream);
       case kPairWith256: return launch_backward_pair<T, 256, 128, 4, 2, 3, 1, 256, 2, 4, 2, 1>(ig, split, wg, plan, form, stream);
       case k256With256: return launch_backward_pair<T, 256, 256, 2, 4, 2, 1, 256, 2, 4, 2, 1>(ig, split, wg, plan, form, stream);
+      case k256With128: return launch_backward_pair<T, 256, 256, 2, 4, 2, 1, 128, 2, 4, 4, 1>(ig, split, wg, plan, form, stream);
       case k128With128: return launch_backward_pair<T, 128, 128, 2, 4, 4, 1, 128, 2, 4, 4, 1>(ig, split, wg, plan, form, stream);
       default: break;
     }

@@ -1178,13 +1178,16 @@ static inline SplitPlan backward_whole_tiles(int M, int K, int N, const SplitPla
 
 // Input-grad and weight-grad of one backward pass in one launch (rz_backward_kernel): which pair of kernels, kApart where the two
 // have no launch in common.
-enum BackwardPair { kApart = 0, k64With64, k64With128, kPairWith128, kPairWith256, k256With256, k128With128 };
+enum BackwardPair { kApart = 0, k64With64, k64With128, kPairWith128, kPairWith256, k256With256, k256With128, k128With128 };
 struct BackwardForm {
   int pair;
   bool full;      // both without bounds checks (else both with)
   int stages;     // of the 16-bit 64 tiles
   bool wg_first;  // whose workgroups come first in the grid: those that take longer
 };
+static inline long long f_tiles(const KernelForm& f, int I, int J) {
+  return (long long)((I + f.rows - 1) / f.rows) * ((J + f.cols - 1) / f.cols);
+}
 static inline BackwardForm backward_form(int M, int K, int N, int H, const SplitPlan& sp, const WeightGradPlan& plan, bool with_dbias,
                                          int elem_bytes, const rz_tuning& t) {
   BackwardForm b = {kApart, false, 2, false};
@@ -1208,13 +1211,51 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
     b.pair = kPairWith256;
   } else if (elem_bytes == 2 && i.rows == 256 && w.tile == 256) {
     b.pair = k256With256;
+  } else if (elem_bytes == 2 && i.rows == 256 && w.tile == 128 && w.waves == 8) {
+    b.pair = k256With128;
   } else if (elem_bytes == 2 && i.rows == 128 && i.waves == 8 && w.tile == 128 && w.waves == 8) {
     b.pair = k128With128;
   }
-  const double ig_work = (double)i.rows * i.cols * (sp.splits > 1 ? sp.r_chunk : N), wg_work = (double)w.tile * w.tile * plan.r_chunk;
-  // (the 128 tile takes longer for its work than a pair of them: M = 2048, K = 4096, N = 1024, a round of compute units each, apart 51.4 us, the input-grad's first
-  //  50.7, the weight-grad's 48.3)
-  b.wg_first = b.pair == kPairWith128 ? 4 * wg_work > 3 * ig_work : wg_work > ig_work;
+  if (b.pair == kApart) return b;
+  if (b.pair == k64With64) {
+    // (several workgroups of each on a compute unit: those of the longer loop first.  16-bit: an input-grad of at most one workgroup a unit has four
+    //  stages by itself; beside a weight-grad that fills the units twice over anyway it would only lose them — M = 3968, K = 256, N = 2688 35.1 apart, 36.2 us)
+    if (elem_bytes == 2 && ig_wgs <= kComputeUnits && ig_wgs + plan.workgroups > 2 * kComputeUnits && N >= 1024) b.pair = kApart;
+    b.wg_first = plan.r_chunk > (sp.splits > 1 ? sp.r_chunk : N);
+    return b;
+  }
+  // One workgroup on a compute unit: by what the two kernels and the common one take.  A workgroup takes its steps of 64 and a fixed part
+  // (forward16_us), the steps longer the fuller the chip; in the common launch the compute units that one op leaves idle
+  // take workgroups of the other, and all of them run at a full chip's pace.  (Two ops of 153 and 162 workgroups, bf16 M = 4288, K = 2304, N = 4544, are 315
+  // for 256 units: 211 us, apart 197.)
+  auto times = [&](const KernelForm& f, bool wg, int chunk, int R, double fill) {
+    const Forward16Times& c = kForward16Times[f.rows == 256 ? (f.cols == 256 ? 6 : 4) : f.rows == 128 ? 2 : 0];
+    return ((chunk < R ? chunk : R) + 63) / 64 * (c.step + c.step_fill * fill) * (wg && f.rows == 128 ? 1.15 : 1.0) + c.round + c.round_fill * fill;
+  };
+  const long long n_i = f_tiles(i, M, K) * sp.splits, n_w = plan.workgroups;
+  auto alone = [&](const KernelForm& f, bool wg, int chunk, int R, long long n) {
+    const double rounds = (double)((n + kComputeUnits - 1) / kComputeUnits);
+    return rounds * times(f, wg, chunk, R, (double)n / (rounds * kComputeUnits));
+  };
+  const int ig_chunk = sp.splits > 1 ? sp.r_chunk : N;
+  const double full = n_i + n_w >= kComputeUnits ? 1.0 : (double)(n_i + n_w) / kComputeUnits;
+  const double d_i = times(i, false, ig_chunk, N, full), d_w = times(w, true, plan.r_chunk, M, full);
+  b.wg_first = d_w > d_i;
+  const double d1 = b.wg_first ? d_w : d_i, d2 = b.wg_first ? d_i : d_w;
+  const long long n1 = b.wg_first ? n_w : n_i, n2 = b.wg_first ? n_i : n_w;
+  // the first op's last round leaves `late` units a workgroup longer; the second op's go to whichever unit is free
+  const long long rounds1 = n1 / kComputeUnits, late = n1 - rounds1 * kComputeUnits;
+  const double from_a = (double)rounds1 * d1, from_b = from_a + d1;
+  double end = late > 0 ? from_b : from_a;
+  for (long long done_a = 0, done_b = 0; done_a * (kComputeUnits - late) + done_b * late < n2;) {
+    const double next_a = from_a + (double)(done_a + 1) * d2, next_b = from_b + (double)(done_b + 1) * d2;
+    if (late == 0 || next_a <= next_b) done_a++;
+    else done_b++;
+    const double last = late == 0 || next_a <= next_b ? next_a : next_b;
+    end = last > end ? last : end;
+  }
+  const double boundary_us = 4.0;
+  if (end > (alone(i, false, ig_chunk, N, n_i) + alone(w, true, plan.r_chunk, M, n_w)) + boundary_us) b.pair = kApart;
   return b;
 }
 hipError_t launch_backward_f32(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, const BackwardForm& form, hipStream_t stream);

@@ -28,9 +28,14 @@ PAIRS = [
     ((3001, 2047, 1531, 31340, 64, 64), FP16),     # ... nothing a multiple of anything
     ((6144, 2048, 1536, 31340, 64, 64), BF16),     # 256 with 256
     ((6011, 2050, 1530, 31340, 64, 64), BF16),
+    ((14456, 556, 802, 27869, 64, 64), BF16),      # 256 with 128, seven slices
+    ((5056, 2304, 256, 36864, 64, 64), FP16),
+    ((4288, 2304, 4544, 654336, 64, 64), BF16),    # 256 with 256, apart: no compute unit would be done sooner
     ((513, 6143, 6145, 300000, 64, 64), BF16),     # 256 x 128 with 256, stored tiles, ragged
     ((128, 2048, 4096, 400000, 32, 64), BF16),     # windows of dHW: no launch in common
-    ((2048, 1024, 4096, 16384, 64, 64), BF16),     # 256 x 128 with 128: none either
+    ((16384, 512, 1024, 5243, 64, 64), BF16),      # 256 x 128 with 128
+    ((5001, 1030, 1021, 20000, 64, 64), FP16),
+    ((2048, 4096, 1024, 262144, 32, 64), BF16),    # ... stored tiles
 ]
 
 
@@ -56,7 +61,7 @@ def test_same_bits_as_apart(shape, dtype):
         assert torch.isfinite(b.float()).all() and torch.equal(a, b), name
 
 
-@pytest.mark.parametrize("shape,dtype", [PAIRS[3], PAIRS[5], PAIRS[14]], ids=str)
+@pytest.mark.parametrize("shape,dtype", [PAIRS[3], PAIRS[5], PAIRS[14], PAIRS[17]], ids=str)
 def test_accumulating_into_an_fp32_gradient(shape, dtype):
     both, apart = _both_and_apart(shape, dtype, dhw_dtype=FP32, accumulate=True)
     for a, b in zip(both, apart):
