@@ -703,7 +703,7 @@ static inline WindowPlan plan_window(int M, int K, int N, int H, int BK, int BN,
   double t_window = window_us(M, K, N, H, BK, BN, elem_bytes, pl.window, pl.windows, false);
   const size_t pack_bytes = window_pack_bytes(M, K, N, BK, BN, elem_bytes);
   const double packed_us = window_us(M, K, N, H, BK, BN, elem_bytes, pl.window, pl.windows, true);
-  if (packed_us + 3.0 < t_window && pack_bytes <= limit && (size_t)tiles * sizeof(int32_t) + 512 <= limit - pack_bytes) {
+  if (packed_us + 3.0 < t_window && pack_bytes <= limit && (unsigned long long)pack_bytes <= 0xffffffffULL && (size_t)tiles * sizeof(int32_t) + 512 <= limit - pack_bytes) {
     t_window = packed_us;
     pl.pack_bytes = pack_bytes;
   }

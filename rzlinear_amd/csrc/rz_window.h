@@ -362,12 +362,6 @@ struct WindowKernel {
       auto load_piece = [&](const T* rows, uint32_t at) -> u32x4_t {
         return *reinterpret_cast<const u32x4_any_t __attribute__((address_space(1)))*>((global_ptr)rows + at);
       };
-      // Packed form: the next group's fragments of the unit being fetched, and the bytes of a block of 32 columns.
-      const int64_t packed_block = (int64_t)ngroups * kFragBytes;
-      global_ptr packed_x = (global_ptr)p.packed_x, packed_y = (global_ptr)p.packed_y;
-      auto load_packed = [&](global_ptr at) -> u32x4_t {
-        return *reinterpret_cast<const u32x4_t __attribute__((address_space(1)))*>(at + (uint32_t)lane * 16u);
-      };
       const T* rows_x = gX;
       const T* rows_y = gdY;
       const int64_t next_x = kGroupRows * p.ldx, next_y = kGroupRows * p.lddy;
@@ -392,32 +386,6 @@ struct WindowKernel {
       int set_k0[kDepth], set_n0[kDepth];   // (not staged) ... and of every set
       auto fetch_next = [&](auto set) {
         constexpr int S = decltype(set)::value;
-        if constexpr (PACKED) {
-          if (fg == 0) {   // (uniform) a new unit
-            const int ftc = ft < my_tiles ? ft : my_tiles - 1;
-            const int v = __builtin_amdgcn_readfirstlane(sm.list[my_first + ftc * kWaves]);
-            const int id = v >> ushift, un = v & (units - 1);
-            const int tk = id / p.tiles_n, tn = id - tk * p.tiles_n;
-            packed_x = (global_ptr)p.packed_x + (int64_t)(tk * (p.h.BK >> 5) + un / kParts) * packed_block;
-            packed_y = (global_ptr)p.packed_y + (int64_t)(tn * (TBN >> 5) + (un % kParts) * BJ) * packed_block;
-            strip_k0 = tk * p.h.BK + (un / kParts) * 32;
-            strip_n0 = tn * TBN + (un % kParts) * UC;
-          }
-          if constexpr (!WHOLE) {
-            set_k0[S] = strip_k0;
-            set_n0[S] = strip_n0;
-          }
-          px[S] = load_packed(packed_x);
-#pragma unroll
-          for (int q = 0; q < BJ; q++) py[S][q] = load_packed(packed_y + q * packed_block);
-          packed_x += kFragBytes;
-          packed_y += kFragBytes;
-          if (++fg == ngroups) {
-            fg = 0;
-            ft++;
-          }
-          return;
-        }
         if constexpr (STAGED) {
           if (fg == 0) {   // (uniform) a new strip
             const int ftc = ft < my_tiles ? ft : my_tiles - 1;
@@ -528,6 +496,12 @@ struct WindowKernel {
       // slices meet its own, and count it
       auto add_tile = [&](int e) {
         const int tile_off = __builtin_amdgcn_readfirstlane(sm.offs[e]);
+        const int rel = (int)((long long)tile_off - w0);   // (offsets and window starts are below 2^31)
+        // What a unit spans beyond K and N is not added: a product with zeros, but a NaN where the other factor is not finite, and its
+        // places in hashed_weight belong to other tiles, or to none.  (x below, the place in the window of row r and column c of
+        // the unit, is rel + r * TBN + c with c < TBN, so that a bound on x is one on r.)
+        const int rows = WHOLE ? 32 : p.K - mult_k0, cols = WHOLE ? UC : p.N - mult_n0;   // (of the unit and beyond, inside W)
+        const int limit = rows < 32 && rel + rows * TBN < wlen ? rel + rows * TBN : wlen;
         // (need_added: how many units lane l's wavefront, `other`, must have added, see must_be_added: one LDS read per look)
         // The wait is bounded: an entry only waits for earlier ones, whose owners wait for still
         // earlier ones, so it ends by itself; should one never be added all the same (a list that
@@ -543,29 +517,28 @@ struct WindowKernel {
           __builtin_amdgcn_s_sleep(1);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        const int rel = (int)((long long)tile_off - w0);   // (offsets and window starts are below 2^31)
-        // What a unit spans beyond K and N is not added: a product with zeros, but a NaN where the other factor is not finite, and its
-        // places in hashed_weight belong to other tiles, or to none.  (x below, the place in the window of row r and column c of
-        // the unit, is rel + r * TBN + c with c < TBN, so that a bound on x is one on r.)
-        const int rows = WHOLE ? 32 : p.K - mult_k0, cols = WHOLE ? UC : p.N - mult_n0;   // (of the unit and beyond, inside W)
-        const int limit = rows < 32 && rel + rows * TBN < wlen ? rel + rows * TBN : wlen;
+        // (others wait for this unit now, link by link of their chains: ahead of the other wavefronts of the SIMD until it is added.  bf16, planned, with
+        //  addresses worked out before the wait: M = 17, K = 2048, N = 15552 39.3 -> 37.2 us, M = 32, K = N = 10240 49.9 -> 48.2, M = 130, K = N = 4096, 128 x 128
+        //  tiles 35.7 -> 34.4)
+        __builtin_amdgcn_s_setprio(3);
         if (rel >= 0 && rel + kUnitSpan <= limit && cols >= UC) {
           // the whole unit lies inside the window (the usual case): no checks, constant offsets
 #pragma unroll
           for (int b = 0; b < BJ; b++) {
             float* at = win + image + rel + ((lane >> 5) * 4) * TBN + b * 32 + (lane & 31);
-            // (eight elements at a time: 16 wavefronts per compute unit leave few registers)
+            // (eight elements at a time: 16 wavefronts per compute unit leave few registers; packed, sixteen)
+            constexpr int kAt = PACKED ? 16 : 8;
 #pragma unroll
-            for (int half = 0; half < 2; half++) {
-              float cur[8];
+            for (int half = 0; half < 16 / kAt; half++) {
+              float cur[kAt];
 #pragma unroll
-              for (int q = 0; q < 8; q++) {
-                const int i = half * 8 + q;
+              for (int q = 0; q < kAt; q++) {
+                const int i = half * kAt + q;
                 cur[q] = at[((i >> 2) * 8 + (i & 3)) * TBN];
               }
 #pragma unroll
-              for (int q = 0; q < 8; q++) {
-                const int i = half * 8 + q;
+              for (int q = 0; q < kAt; q++) {
+                const int i = half * kAt + q;
                 at[((i >> 2) * 8 + (i & 3)) * TBN] = cur[q] + acc[0][b][i] * p.scale;
                 acc[0][b][i] = 0.f;
               }
@@ -601,6 +574,7 @@ struct WindowKernel {
           }
         }
         if (lane == 0) __hip_atomic_store(&sm.progress[wave], e / kWaves + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __builtin_amdgcn_s_setprio(0);
       };
       int pt = 0, pg = 0;      // tile ordinal and group of the item being multiplied
       auto item = [&](auto set) {
@@ -608,7 +582,7 @@ struct WindowKernel {
         // the set freed by the previous item takes the loads of the item kDepth - 1 ahead
         fetch_next(std::integral_constant<int, (S + kDepth - 1) % kDepth>{});
         if (pg == 0 && pt < my_tiles) need_added = must_be_added(my_first + pt * kWaves);   // (uniform)
-        if constexpr (!STAGED && !WHOLE) {   // where the item's unit lies
+        if constexpr (!STAGED) {   // where the item's unit lies
           mult_k0 = set_k0[S];
           mult_n0 = set_n0[S];
         } else if (pg == 0 && !all_whole) {   // (uniform)
@@ -618,24 +592,6 @@ struct WindowKernel {
           mult_k0 = tk * p.h.BK + (un / kParts) * 32;
           mult_n0 = (id - tk * p.tiles_n) * TBN + (un % kParts) * UC;
           mult_whole = mult_k0 + 32 <= p.K && mult_n0 + UC <= p.N;
-        }
-        if constexpr (PACKED) {
-          if constexpr (k16) {
-#pragma unroll
-            for (int j = 0; j < BJ; j++) acc[0][j] = Mfma<T>::run(px[S], py[S][j], acc[0][j]);
-          } else {
-#pragma unroll
-            for (int g = 0; g < GS; g++)
-#pragma unroll
-              for (int j = 0; j < BJ; j++)
-                acc[0][j] = Mfma<T>::run(__builtin_bit_cast(f32x4_t, px[S])[g], __builtin_bit_cast(f32x4_t, py[S][j])[g], acc[0][j]);
-          }
-          if (pt < my_tiles && ++pg == ngroups) {
-            add_tile(my_first + pt * kWaves);
-            pg = 0;
-            pt++;
-          }
-          return;
         }
         if constexpr (STAGED) {
           {
@@ -731,7 +687,96 @@ struct WindowKernel {
           pt++;
         }
       };
-      if (my_tiles > 0) {
+      if constexpr (PACKED) {
+        // What bounds the packed form is what its wavefronts issue beside loads and MFMAs, four of them on a SIMD: with a state of the fetches as
+        // general as the other forms' an item took 40 scalar and 30 vector instructions, a good part of them spilled scalars.  So an item's
+        // loads are three bases in scalar registers, the same for the whole kernel, and two 32-bit offsets of a lane that move on by a fragment,
+        // and where a unit lies is worked out once per unit, without a division.
+        // (Planned, with the kernel ahead, bf16: K = N = 10240, H = 6.5 M, M = 128 76.4 -> 72.0 us, M = 32 52.1 -> 49.7, fp32 103.5 -> 97.0; M = 64, K = N = 4096, 64 x 32 tiles 21.5 -> 19.7.
+        //  From M = 256 on at that K = N, X and dY are more than an L2 holds, and nothing changes.  A fourth set: 74.2, M = 130 of 128 x 128 tiles 36.2 -> 43.4, spills.)
+        if (my_tiles > 0) {
+          const uint32_t block = (uint32_t)ngroups * (uint32_t)kFragBytes;   // bytes of a block of 32 columns
+          global_ptr from_x = (global_ptr)p.packed_x, from_y[BJ];
+#pragma unroll
+          for (int q = 0; q < BJ; q++) from_y[q] = (global_ptr)p.packed_y + q * (int64_t)block;
+          const int last = my_first + (my_tiles - 1) * kWaves;
+          const uint32_t tiles_n = (uint32_t)p.tiles_n, inverse = 0xffffffffu / tiles_n;
+          // tile row, tile column and unit of list entry e (the quotient by the inverse is at most one too small)
+          auto unit_at = [&](int e, int& tk, int& tn, int& un) {
+            const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane(sm.list[e]), id = v >> ushift;
+            uint32_t quotient = (uint32_t)(((uint64_t)id * inverse) >> 32), rest = id - quotient * tiles_n;
+            while (rest >= tiles_n) {   // (uniform)
+              quotient++;
+              rest -= tiles_n;
+            }
+            tk = (int)quotient;
+            tn = (int)rest;
+            un = (int)(v & (uint32_t)(units - 1));
+          };
+          uint32_t at_fx = 0, at_fy = 0;
+          int ahead = my_first - kWaves, left = 0;   // the entry whose fragments are being fetched, and how many of its groups are to come
+          auto fetch = [&](auto set) {
+            constexpr int S = decltype(set)::value;
+            if (left == 0) {   // (uniform; beyond the wavefront's last unit that one again: see the ring below)
+              ahead = ahead + kWaves < last ? ahead + kWaves : last;
+              int tk, tn, un;
+              unit_at(ahead, tk, tn, un);
+              at_fx = (uint32_t)(tk * (p.h.BK >> 5) + un / kParts) * block + (uint32_t)lane * 16u;
+              at_fy = (uint32_t)(tn * (TBN >> 5) + (un % kParts) * BJ) * block + (uint32_t)lane * 16u;
+              left = ngroups;
+            }
+            px[S] = *reinterpret_cast<const u32x4_t __attribute__((address_space(1)))*>(from_x + at_fx);
+#pragma unroll
+            for (int q = 0; q < BJ; q++) py[S][q] = *reinterpret_cast<const u32x4_t __attribute__((address_space(1)))*>(from_y[q] + at_fy);
+            at_fx += (uint32_t)kFragBytes;
+            at_fy += (uint32_t)kFragBytes;
+            left--;
+          };
+          int e = my_first, group = 0;
+          auto item = [&](auto set) {
+            constexpr int S = decltype(set)::value;
+            // the set freed by the previous item takes the loads of the item kDepth - 1 ahead
+            fetch(std::integral_constant<int, (S + kDepth - 1) % kDepth>{});
+            if (group == 0 && e <= last) need_added = must_be_added(e);   // (uniform)
+            if constexpr (k16) {
+#pragma unroll
+              for (int j = 0; j < BJ; j++) acc[0][j] = Mfma<T>::run(px[S], py[S][j], acc[0][j]);
+            } else {
+#pragma unroll
+              for (int g = 0; g < GS; g++)
+#pragma unroll
+                for (int j = 0; j < BJ; j++)
+                  acc[0][j] = Mfma<T>::run(__builtin_bit_cast(f32x4_t, px[S])[g], __builtin_bit_cast(f32x4_t, py[S][j])[g], acc[0][j]);
+            }
+            if (++group == ngroups && e <= last) {   // (uniform)
+              if constexpr (!WHOLE) {
+                int tk, tn, un;
+                unit_at(e, tk, tn, un);
+                mult_k0 = tk * p.h.BK + (un / kParts) * 32;
+                mult_n0 = tn * TBN + (un % kParts) * UC;
+              }
+              add_tile(e);
+              group = 0;
+              e += kWaves;
+            }
+          };
+          // whole turns of the ring: the up to kDepth - 1 items past the end are padding, multiplied and not added
+          static_assert(kDepth == 3 || kDepth == 4, "the turn below");
+          fetch(std::integral_constant<int, 0>{});
+          fetch(std::integral_constant<int, 1>{});
+          if constexpr (kDepth == 4) fetch(std::integral_constant<int, 2>{});
+          for (int i = 0; i < items; i += kDepth) {
+            item(std::integral_constant<int, 0>{});
+            item(std::integral_constant<int, 1>{});
+            item(std::integral_constant<int, 2>{});
+            if constexpr (kDepth == 4) item(std::integral_constant<int, kDepth - 1>{});
+          }
+#pragma unroll
+          for (int b = 0; b < BJ; b++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[0][b][i] = 0.f;
+        }
+      } else if (my_tiles > 0) {
         // whole turns of the ring: the up to kDepth - 1 items past the end are padding (see fetch_next)
         static_assert(kDepth >= 2 && kDepth <= 8, "the ring below is written out for up to eight sets");
         auto each_set = [&](auto&& f, auto count) {   // f(0), ..., f(count - 1) with compile-time arguments
