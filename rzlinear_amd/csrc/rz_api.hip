@@ -509,6 +509,24 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
   const WeightGradWorkspace ws = weight_grad_workspace(plan, wp, H, dhw_dtype == RZ_F32, dbias != nullptr, planned);
   if (ws.total_bytes > 0 && (workspace == nullptr || workspace_bytes < ws.total_bytes)) return RZ_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
+  WindowParams w = {};
+  if (wp.use) {
+    if (planned && (lay.windows != wp.windows || lay.window != wp.window)) return RZ_ERR_BAD_ARGUMENT;
+    w.X = X; w.dY = dY;
+    w.M = M; w.K = K; w.N = N;
+    w.ldx = ldx; w.lddy = lddy;
+    w.h = p.h;
+    w.tiles_k = (K + BK - 1) / BK;
+    w.tiles_n = (N + BN - 1) / BN;
+    // where the workspace has room behind the offsets: X and dY as fragments (the same bits, faster)
+    const uintptr_t pack_at = ((uintptr_t)workspace + ws.main_bytes + 15) & ~(uintptr_t)15;
+    if (wp.pack_bytes > 0 && workspace != nullptr && pack_at - (uintptr_t)workspace <= workspace_bytes &&
+        workspace_bytes - (pack_at - (uintptr_t)workspace) >= wp.pack_bytes) {
+      const size_t group = dtype == RZ_F32 ? 8 : 16, rows = ((size_t)M + group - 1) / group * group;
+      w.packed_x = (void*)pack_at;
+      w.packed_y = (void*)(pack_at + rows * dtype_bytes(dtype) * (size_t)w.tiles_k * BK);
+    }
+  }
   // (an input-grad that shares no launch with this call's contraction is enqueued first, like the reference's)
   BackwardForm form = {};
   if (with != nullptr) {
@@ -523,8 +541,18 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
       }
       form = backward_form(M, K, N, H, with->split, plan, dbias != nullptr, dtype_bytes(dtype), tuning);
     }
+    if (w.packed_x != nullptr) {
+      const bool pieces = ((uintptr_t)X | (uintptr_t)dY) % 16 == 0 && (ldx | lddy) % 8 == 0;
+      const PackForm pack = pack_form(M, K, N, BK, BN, pieces, with->split, dtype_bytes(dtype), tuning);
+      if (pack.groups > 0) {
+        const hipError_t e = dtype == RZ_BF16 ? launch_input_grad_pack_bf16(with->p, &with->split, w, pack, s)
+                                              : launch_input_grad_pack_f16(with->p, &with->split, w, pack, s);
+        if (e != hipSuccess) return RZ_ERR_LAUNCH;
+        w.packed = 1;
+      }
+    }
     if (form.pair == kApart) {
-      if (launch_gemm(dtype, kInputGrad, with->p, nullptr, &with->split, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
+      if (!w.packed && launch_gemm(dtype, kInputGrad, with->p, nullptr, &with->split, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
       st = finish_plain_op(dtype, with->p, nullptr, with->split, s);
       if (st != RZ_OK) return st;
     }
@@ -542,9 +570,7 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
     // large hashed_weight, short contraction: windows of dHW instead of K*N atomics.  The
     // tile offsets are hashed once into the workspace; every workgroup scans them.
     {
-      WindowParams w = {};
       if (planned) {
-        if (lay.windows != wp.windows || lay.window != wp.window) return RZ_ERR_BAD_ARGUMENT;
         w.offsets = layer_plan + lay.offsets_at;
         w.plan_start = layer_plan + lay.start_at;
         w.plan_list = layer_plan + lay.list_at;
@@ -557,27 +583,15 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
         if (hipGetLastError() != hipSuccess) return RZ_ERR_LAUNCH;
         w.offsets = (const int32_t*)workspace;
       }
-      w.X = X; w.dY = dY; w.dHW = dHW;
-      w.M = M; w.K = K; w.N = N; w.H = H;
-      w.ldx = ldx; w.lddy = lddy;
+      w.dHW = dHW;
+      w.H = H;
       w.scale = init_factor;
-      w.h = p.h;
       w.window = wp.window;
-      w.tiles_k = (K + BK - 1) / BK;
-      w.tiles_n = (N + BN - 1) / BN;
       w.accumulate = accumulate ? 1 : 0;
       w.out_f32 = dhw_dtype == RZ_F32 ? 1 : 0;
       w.dbias = dbias;
       w.dbias_f32 = dbias_dtype == RZ_F32 ? 1 : 0;
       w.windows = wp.windows;
-      // where the workspace has room behind the offsets: X and dY as fragments (the same bits, faster)
-      const uintptr_t pack_at = ((uintptr_t)workspace + ws.main_bytes + 15) & ~(uintptr_t)15;
-      if (wp.pack_bytes > 0 && workspace != nullptr && pack_at - (uintptr_t)workspace <= workspace_bytes &&
-          workspace_bytes - (pack_at - (uintptr_t)workspace) >= wp.pack_bytes) {
-        const size_t group = dtype == RZ_F32 ? 8 : 16, rows = ((size_t)M + group - 1) / group * group;
-        w.packed_x = (void*)pack_at;
-        w.packed_y = (void*)(pack_at + rows * dtype_bytes(dtype) * (size_t)w.tiles_k * BK);
-      }
       w.poll_limit = tuning.poll_limit > 0 ? tuning.poll_limit : kWindowPollLimit;
       hipError_t e = dtype == RZ_F32 ? launch_window_f32(w, wp.windows, s)
                      : dtype == RZ_BF16 ? launch_window_bf16(w, wp.windows, s)

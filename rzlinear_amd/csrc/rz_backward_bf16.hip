@@ -6,4 +6,8 @@ hipError_t launch_backward_bf16(GemmParams ig, const SplitPlan* split, GemmParam
                         hipStream_t stream) {
   return launch_backward_t<bf16_t>(ig, split, wg, plan, form, stream);
 }
+hipError_t launch_input_grad_pack_bf16(const GemmParams& ig, const SplitPlan* split, const WindowParams& w, const PackForm& form,
+                                       hipStream_t stream) {
+  return launch_input_grad_pack_t<bf16_t>(ig, split, w, form, stream);
+}
 }  // namespace rz

@@ -6,4 +6,8 @@ hipError_t launch_backward_f16(GemmParams ig, const SplitPlan* split, GemmParams
                         hipStream_t stream) {
   return launch_backward_t<f16_t>(ig, split, wg, plan, form, stream);
 }
+hipError_t launch_input_grad_pack_f16(const GemmParams& ig, const SplitPlan* split, const WindowParams& w, const PackForm& form,
+                                       hipStream_t stream) {
+  return launch_input_grad_pack_t<f16_t>(ig, split, w, form, stream);
+}
 }  // namespace rz

@@ -287,6 +287,55 @@ static hipError_t launch_backward_t(const GemmParams& ig, const SplitPlan* split
   return hipErrorInvalidValue;
 }
 
+// What the kernels that make the fragments take; returns how many there are.  (Blocks of 32 columns up to whole hashed tiles: every unit of
+// every tile has its fragments, see window_pack_bytes.)
+template <typename T>
+static long long pack_params(const WindowParams& w, PackParams* pk) {
+  constexpr int kRows = sizeof(T) == 4 ? 8 : 16;
+  const long long blocks_x = (long long)w.tiles_k * (w.h.BK / 32), blocks_y = (long long)w.tiles_n * (w.h.BN / 32);
+  const long long ngroups = ((long long)w.M + kRows - 1) / kRows;
+  *pk = {w.X, w.dY, w.packed_x, w.packed_y, w.M, w.K, w.N, (int)blocks_x, (int)blocks_y, (int)ngroups, w.ldx, w.lddy};
+  return (blocks_x + blocks_y) * ngroups;
+}
+
+// An input-grad and, in the same launch, the fragments of the weight-grad behind it (pack_groups).
+template <typename T, int TI, int TJ, int WI, int WJ, int STAGES, int WK, bool FULL>
+static hipError_t launch_pack_form(GemmParams ig, const SplitPlan* split, const PackParams& pk, int groups, hipStream_t stream) {
+  static std::atomic<uint64_t> lds_limit_raised{0};
+  typedef GemmKernel<T, kInputGrad, TI, TJ, WI, WJ, STAGES, FULL, false, !FULL, WK> IG;
+  dim3 grid;
+  size_t smem;
+  hipError_t e = prepare_one<IG, T, kInputGrad, TI, TJ, false>(ig, nullptr, split, &grid, &smem);
+  if (e != hipSuccess) return e;
+  auto kernel = rz_input_grad_pack_kernel<T, IG>;
+  if (smem > 64 * 1024) {
+    e = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds_limit_raised);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(kernel, dim3(grid.x * grid.y + (unsigned)groups), dim3(IG::kThreads), smem, stream, ig, pk, (int)grid.x, (int)grid.y);
+  return hipGetLastError();
+}
+
+template <typename T, int TI, int TJ, int WI, int WJ, int STAGES, int WK>
+static hipError_t launch_pack_tile(const GemmParams& ig, const SplitPlan* split, const PackParams& pk, const PackForm& form, hipStream_t stream) {
+  if (form.full) return launch_pack_form<T, TI, TJ, WI, WJ, STAGES, WK, true>(ig, split, pk, form.groups, stream);
+  return launch_pack_form<T, TI, TJ, WI, WJ, STAGES, WK, false>(ig, split, pk, form.groups, stream);
+}
+
+template <typename T>
+static hipError_t launch_input_grad_pack_t(const GemmParams& ig, const SplitPlan* split, const WindowParams& w, const PackForm& form,
+                                           hipStream_t stream) {
+  PackParams pk;
+  if (w.packed_x == nullptr || w.packed_y == nullptr || pack_params<T>(w, &pk) != form.fragments) return hipErrorInvalidValue;
+  switch (form.rows) {
+    case 32: return launch_pack_tile<T, 32, 128, 1, 4, 3, 2>(ig, split, pk, form, stream);
+    case 64: return launch_pack_tile<T, 64, 64, 2, 2, 4, 4>(ig, split, pk, form, stream);
+    case 128: return launch_pack_tile<T, 128, 128, 2, 4, 4, 1>(ig, split, pk, form, stream);
+    case 256: return launch_pack_tile<T, 256, 128, 4, 2, 3, 1>(ig, split, pk, form, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 template <typename T, int TBN, int OPERANDS, bool WHOLE>
 static hipError_t launch_window_whole(WindowParams p, int windows, hipStream_t stream) {
   typedef WindowKernel<T, TBN, OPERANDS, WHOLE> K;
@@ -321,12 +370,12 @@ template <typename T, int TBN>
 static hipError_t launch_window_one(const WindowParams& p, int windows, hipStream_t stream) {
   constexpr int kVec = 16 / (int)sizeof(T);
   if (p.packed_x != nullptr && p.packed_y != nullptr) {
-    // (blocks of 32 columns up to whole hashed tiles: every unit of every tile has its fragments, see window_pack_bytes)
-    const long long blocks_x = (long long)p.tiles_k * (p.h.BK / 32), blocks_y = (long long)p.tiles_n * (TBN / 32);
-    constexpr int kRows = WindowKernel<T, TBN, kPacked, true>::kGroupRows;
-    const long long ngroups = (p.M + kRows - 1) / kRows, wgs = ((blocks_x + blocks_y) * ngroups + 3) / 4;
-    if (wgs > 0x1fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(window_pack_kernel<T>, dim3((unsigned)wgs), dim3(256), 0, stream, p, (int)blocks_x, (int)blocks_y, (int)ngroups);
+    if (!p.packed) {
+      PackParams pk;
+      const long long wgs = (pack_params<T>(p, &pk) + 3) / 4;
+      if (wgs > 0x1fffffffLL) return hipErrorInvalidValue;
+      hipLaunchKernelGGL(window_pack_kernel<T>, dim3((unsigned)wgs), dim3(256), 0, stream, pk);
+    }
     hipError_t e = hipGetLastError();
     return e != hipSuccess ? e : launch_window_form<T, TBN, kPacked>(p, windows, stream);
   }

@@ -1260,6 +1260,39 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
   if (end * mixing > (alone(i, false, ig_chunk, N, n_i) + alone(w, true, plan.r_chunk, M, n_w)) + boundary_us) b.pair = kApart;
   return b;
 }
+
+// An input-grad beside which the fragments of a windowed weight-grad are made (rz_input_grad_pack_kernel); groups = 0: by a kernel of their own, which takes
+// 4 to 5 us of which 1 to 2 are work.  16-bit; fp32's tiles share compute units, so that none is idle.
+struct PackForm {
+  int groups;           // workgroups that make them, behind those of the input-grad
+  long long fragments;
+  int rows;             // of the input-grad's C tile, which tells its kernel
+  bool full;
+};
+// whole_pieces: X and dY lie at, and their rows are multiples of, 16 bytes.
+static inline PackForm pack_form(int M, int K, int N, int BK, int BN, bool whole_pieces, const SplitPlan& sp, int elem_bytes, const rz_tuning& t) {
+  PackForm f = {};
+  if (elem_bytes != 2 || !whole_pieces || K % 8 != 0 || N % 8 != 0 || sp.run_steps > 0 || t.tile != 0 || t.stages == 1 || t.clamp == -1) return f;
+  const int chunk = sp.splits > 1 ? sp.r_chunk : N;
+  const KernelForm i = kernel_form(kInputGrad, M, K, N, chunk, sp.tile, tile_count(M, K, sp.tile) * sp.splits, elem_bytes, t);
+  const bool served = (i.rows == 32 && i.cols == 128) || (i.rows == 64 && i.stages == 4) || (i.rows == 128 && i.waves == 8 && i.stages == 4) ||
+                      (i.rows == 256 && i.cols == 128);
+  if (!served || !(i.full || i.clamp)) return f;
+  const long long idle = kComputeUnits - f_tiles(i, M, K) * sp.splits;
+  const long long blocks = (long long)((K + BK - 1) / BK) * (BK / 32) + (long long)((N + BN - 1) / BN) * (BN / 32);
+  f.fragments = blocks * ((M + 15) / 16);
+  if (idle < 1) return f;
+  // The workgroups that make them, one on each idle compute unit, must be done before the input-grad is: 0.06 us a fragment and unit.  Passes, GPU-bound, apart /
+  // beside, us: bf16 K = N = 10240, H = 6.5 M, 16 idle units: M = 32 107.2 / 104.6, 128 152.0 / 150.2, 200 228.0 / 225.3; M = 96 5008 x 7008, 56 of them,
+  // 91.7 / 88.1; M = 152 3008 x 5008 65.2 / 62.4; M = 128 3072 x 6144, 64 of them, 57.2 / 54.3.  (Element by element in these workgroups, 0.19 us a fragment, M = 128 took 181.)
+  const double pack_us = 3.0 + 0.06 * (double)f.fragments / (double)idle;
+  if (pack_us > sp.est_us) return f;
+  const long long most = (f.fragments + i.waves - 1) / i.waves;
+  f.groups = (int)(idle < most ? idle : most);
+  f.rows = i.rows;
+  f.full = i.full;
+  return f;
+}
 hipError_t launch_backward_f32(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, const BackwardForm& form, hipStream_t stream);
 hipError_t launch_backward_bf16(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, const BackwardForm& form, hipStream_t stream);
 hipError_t launch_backward_f16(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, const BackwardForm& form, hipStream_t stream);
@@ -1278,6 +1311,8 @@ hipError_t launch_input_grad_f16(GemmParams p, const WeightGradPlan* plan, const
 hipError_t launch_weight_grad_f16(GemmParams p, const WeightGradPlan* plan, const SplitPlan* split, const rz_tuning& tuning, hipStream_t stream);
 
 struct WindowParams;
+hipError_t launch_input_grad_pack_bf16(const GemmParams& ig, const SplitPlan* split, const WindowParams& w, const PackForm& form, hipStream_t stream);
+hipError_t launch_input_grad_pack_f16(const GemmParams& ig, const SplitPlan* split, const WindowParams& w, const PackForm& form, hipStream_t stream);
 // Enqueues the windowed weight-grad kernel; p.window and the tile grid must come from plan_window.
 hipError_t launch_window_f32(const WindowParams& p, int windows, hipStream_t stream);
 hipError_t launch_window_bf16(const WindowParams& p, int windows, hipStream_t stream);

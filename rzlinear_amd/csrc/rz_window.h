@@ -58,6 +58,7 @@ struct WindowParams {
   // Non-null: X and dY as MFMA fragments (see window_pack_kernel), which the packed form of the kernel reads
   void* packed_x;
   void* packed_y;
+  int packed;        // the input-grad's launch makes them (rz_input_grad_pack_kernel)
 };
 
 // How often a wavefront looks at the flags of the earlier strips it must wait for before it gives
@@ -838,16 +839,25 @@ struct WindowKernel {
 // whole hashed tiles.  A wavefront makes one fragment; four neighbouring blocks of columns share a workgroup, so that a
 // line of X or dY is read by one compute unit.  Any element alignment, any row pitch.
 //   16-bit: lane l holds rows (l >> 5) * 8 + j, j = 0..7, of column l & 31; fp32: rows 2 j + (l >> 5), j = 0..3.
+struct PackParams {
+  const void* X;
+  const void* dY;
+  void* packed_x;
+  void* packed_y;
+  int M, K, N, blocks_x, blocks_y, ngroups;
+  int64_t ldx, lddy;
+};
+
 template <typename T>
-__global__ __launch_bounds__(256) void window_pack_kernel(WindowParams p, int blocks_x, int blocks_y, int ngroups) {
+__global__ __launch_bounds__(256) void window_pack_kernel(PackParams p) {
   constexpr int kRows = sizeof(T) == 4 ? 8 : 16, VEC = ElemTraits<T>::kVec;
   typedef typename std::conditional<sizeof(T) == 4, uint32_t, uint16_t>::type Bits;
   const int lane = threadIdx.x & 63;
-  const int id = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blocks = blocks_x + blocks_y;
+  const int id = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), blocks = p.blocks_x + p.blocks_y;
   const int g = id / blocks, b = id - g * blocks;
-  if (g >= ngroups) return;
-  const bool is_x = b < blocks_x;   // (uniform)
-  const int block = is_x ? b : b - blocks_x, cols = is_x ? p.K : p.N;
+  if (g >= p.ngroups) return;
+  const bool is_x = b < p.blocks_x;   // (uniform)
+  const int block = is_x ? b : b - p.blocks_x, cols = is_x ? p.K : p.N;
   const int64_t ld = is_x ? p.ldx : p.lddy;
   const Bits* from = static_cast<const Bits*>(is_x ? p.X : p.dY);
   const int col = block * 32 + (lane & 31), row0 = g * kRows + (lane >> 5) * (sizeof(T) == 4 ? 1 : VEC);
@@ -860,7 +870,66 @@ __global__ __launch_bounds__(256) void window_pack_kernel(WindowParams p, int bl
     else v[j >> 1] |= e << (16 * (j & 1));
   }
   *reinterpret_cast<u32x4_t*>(static_cast<char*>(is_x ? p.packed_x : p.packed_y) +
-                              ((int64_t)block * ngroups + g) * kFragBytes + lane * 16) = v;
+                              ((int64_t)block * p.ngroups + g) * kFragBytes + lane * 16) = v;
+}
+
+// 16-bit fragments id, id + stride, ... by one wavefront.  The rows of X and dY are whole 16-byte pieces (PackForm): a fragment is one load, whose piece
+// lane l has of row l >> 2, and turns round in LDS, where the wavefront has FRAGS places of its own; as many loads are in flight.
+// (Element by element, as above, a compute unit makes one in 0.19 us, since it takes a load of two bytes a lane in about 50 clocks.)
+static constexpr int kTurnPitch = 40;                                 // 16-bit elements; rows of 80 bytes: both halves of a wavefront read other banks
+static constexpr int kTurnElems = 16 * kTurnPitch;
+template <int FRAGS>
+__device__ __forceinline__ void window_pack_pieces(const PackParams& p, int id, int stride, int lane, uint16_t* turn) {
+  const int blocks = p.blocks_x + p.blocks_y, total = blocks * p.ngroups;
+  for (; id < total; id += FRAGS * stride) {
+    u32x4_t v[FRAGS];
+#pragma unroll
+    for (int q = 0; q < FRAGS; q++) {
+      const int at = id + q * stride, g = at / blocks, b = at - g * blocks;
+      const bool is_x = b < p.blocks_x;   // (uniform)
+      const int row = g * 16 + (lane >> 2), col = (is_x ? b : b - p.blocks_x) * 32 + (lane & 3) * 8;
+      v[q] = u32x4_t{0u, 0u, 0u, 0u};
+      if (at < total && row < p.M && col < (is_x ? p.K : p.N))
+        v[q] = *reinterpret_cast<const u32x4_t*>(static_cast<const uint16_t*>(is_x ? p.X : p.dY) + (int64_t)row * (is_x ? p.ldx : p.lddy) + col);
+    }
+#pragma unroll
+    for (int q = 0; q < FRAGS; q++) *reinterpret_cast<u32x4_t*>(turn + q * kTurnElems + (lane >> 2) * kTurnPitch + (lane & 3) * 8) = v[q];
+    // (a wavefront's LDS instructions are carried out in order: the compiler has to keep it)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < FRAGS; q++) {
+      const int at = id + q * stride, g = at / blocks, b = at - g * blocks;
+      if (at >= total) break;   // (uniform)
+      const bool is_x = b < p.blocks_x;
+      const uint16_t* e = turn + q * kTurnElems + (lane >> 5) * 8 * kTurnPitch + (lane & 31);
+      u32x4_t f;
+#pragma unroll
+      for (int j = 0; j < 4; j++) f[j] = (uint32_t)e[2 * j * kTurnPitch] | (uint32_t)e[(2 * j + 1) * kTurnPitch] << 16;
+      *reinterpret_cast<u32x4_t*>(static_cast<char*>(is_x ? p.packed_x : p.packed_y) +
+                                  ((int64_t)(is_x ? b : b - p.blocks_x) * p.ngroups + g) * kFragBytes + lane * 16) = f;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// The fragments beside the input-grad of the same backward pass: its grid leaves some compute units idle, and the workgroups behind it
+// make the fragments there (pack_form: where).
+template <typename T, typename IG>
+__global__ __launch_bounds__(IG::kThreads, IG::kWavesPerSimd) void rz_input_grad_pack_kernel(GemmParams ig, PackParams pk, int ig_x, int ig_y) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char rz_smem_raw[];
+  constexpr int kWaves = IG::kThreads / 64, kFrags = 64 / kWaves;
+  static_assert(sizeof(typename IG::Smem) >= 64 * kTurnElems * 2, "64 fragments turn round in the input-grad's LDS");
+  const int n_ig = ig_x * ig_y, b = blockIdx.x;
+  if (b >= n_ig) {   // (uniform)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    window_pack_pieces<kFrags>(pk, (b - n_ig) * kWaves + wave, ((int)gridDim.x - n_ig) * kWaves, threadIdx.x & 63,
+                               reinterpret_cast<uint16_t*>(rz_smem_raw) + wave * kFrags * kTurnElems);
+    return;
+  }
+  const int by = b / ig_x;
+  IG::run(ig, *reinterpret_cast<typename IG::Smem*>(rz_smem_raw), b - by * ig_x, by, ig_x, ig_y);
 }
 
 // dbias[n] = sum over the rows m of dY[m][n].  A workgroup of 1024 threads owns 256 columns; four thread groups each add

@@ -68,6 +68,28 @@ def test_accumulating_into_an_fp32_gradient(shape, dtype):
         assert torch.equal(a, b)
 
 
+# Windows of dHW whose operands' fragments are made beside the input-grad: its 32 x 128, 64, 128 and 256 x 128 tiles, complete and ragged
+FRAGMENTS = [
+    ((32, 10240, 10240, 6553600, 32, 64), BF16),
+    ((19, 10232, 10240, 6553600, 32, 64), FP16),
+    ((61, 3000, 4008, 750000, 32, 64), FP16),
+    ((128, 4096, 4096, 700000, 32, 64), BF16),
+    ((128, 10240, 10240, 6553600, 32, 64), BF16),
+    ((96, 5000, 7000, 2200000, 32, 64), BF16),
+    ((150, 3000, 5000, 937500, 32, 64), FP16),
+    ((224, 10240, 10240, 6553600, 32, 64), BF16),
+    ((61, 3001, 4008, 750000, 32, 64), FP16),      # rows that are not whole pieces: by a kernel of their own
+]
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("shape,dtype", FRAGMENTS, ids=str)
+def test_fragments_beside_the_input_grad(shape, dtype, accumulate):
+    both, apart = _both_and_apart(shape, dtype, accumulate=accumulate)
+    for name, a, b in zip(("dx", "dhw", "dbias"), both, apart):
+        assert torch.isfinite(b.float()).all() and torch.equal(a, b), name
+
+
 def test_an_input_grad_in_runs_goes_in_whole_tiles():
     # M = 1024, K = N = 10240: by itself in runs, whose parts are added up in fp32; the whole tiles' sums are in one piece.  Two
     # correctly accumulated results, each rounded once: they differ by an fp32 sum's error (10240 terms, < 1e-5 of the largest value)
