@@ -1255,8 +1255,11 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
     end = last > end ? last : end;
   }
   // (Workgroups of the two side by side miss the L2s more often than those of one, which costs about 2 % of a launch that shares nothing else: M = 8192,
-  //  K = 4096, N = 16384, whose ops fill whole rounds, a pass 2316 us apart, 2349 in one launch; where M = K = N = 4096 it and the boundary are even.)
+  // K = 4096, N = 16384, whose ops fill whole rounds, a pass 2316 us apart, 2349 in one launch.
+  // And where both ops fill whole rounds there is the boundary alone to gain, nothing if X and dY, which both ops read, are more than the L2s hold (32 MB in all): M = 4096,
+  // K = 512, N = 1024 61.8 us a pass apart, 59.0 in one launch, M = 8192 60.8 and 59.1; M = 16384 70.2 and 69.9, and 1 us slower where the host is as slow.)
   const double boundary_us = 4.0, mixing = 1.02;
+  if (n_i % kComputeUnits == 0 && n_w % kComputeUnits == 0 && (double)M * ((double)K + N) * elem_bytes > 32.0e6) b.pair = kApart;
   if (end * mixing > (alone(i, false, ig_chunk, N, n_i) + alone(w, true, plan.r_chunk, M, n_w)) + boundary_us) b.pair = kApart;
   return b;
 }
