@@ -101,7 +101,7 @@ def test_an_input_grad_in_runs_goes_in_whole_tiles():
     assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-5 * b.abs().max()).all()
 
 
-@pytest.mark.parametrize("shape,dtype", [PAIRS[0], PAIRS[3], PAIRS[5], PAIRS[11]], ids=str)
+@pytest.mark.parametrize("shape,dtype", [PAIRS[0], PAIRS[3], PAIRS[5], PAIRS[11], FRAGMENTS[0], FRAGMENTS[5]], ids=str)
 def test_captured_backward(shape, dtype):
     # (a cut input-grad has no counters under capture: a second kernel behind the common launch, the same bits)
     from rzlinear_amd import RzLinear
