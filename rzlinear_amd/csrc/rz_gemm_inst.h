@@ -97,7 +97,7 @@ static hipError_t launch_tile(GemmParams p, const WeightGradPlan* plan, const Sp
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false>::TR) return hipErrorInvalidValue;
     return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, false, WK>(p, plan, split, stream);
   }
-  // (the 64 tile of four wavefronts, and the 16-bit 128 tile of eight with two stages, serve rows shorter than a 16-byte piece only)
+  // (the 64 tile of four wavefronts but for fp32 weight-grad, and the 16-bit 128 tile of eight with two stages, serve rows shorter than a 16-byte piece only)
   // (16-bit 256 tile, a few R steps)
   if constexpr (sizeof(T) == 2 && TILE == 256 && TILE_J == 256) if (form.short_loop) {
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true, false, false, WK, true>::TR) return hipErrorInvalidValue;
@@ -105,7 +105,7 @@ static hipError_t launch_tile(GemmParams p, const WeightGradPlan* plan, const Sp
     if (form.clamp) return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, false, COLSUM, true, WK, true>(p, plan, split, stream);
     return hipErrorInvalidValue;
   }
-  constexpr bool kCheckedOnly = WK == 1 && (TILE == 64 || (sizeof(T) == 2 && TILE == 128 && WI * WJ == 8 && NSTAGE == 2));
+  constexpr bool kCheckedOnly = WK == 1 && ((TILE == 64 && !(sizeof(T) == 4 && OP == kWeightGrad)) || (sizeof(T) == 2 && TILE == 128 && WI * WJ == 8 && NSTAGE == 2));
   if constexpr (!kCheckedOnly) if (form.full) {
     if (form.step != GemmKernel<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true>::TR) return hipErrorInvalidValue;
     return launch_one<T, OP, TILE, TILE_J, WI, WJ, NSTAGE, true, COLSUM, false, WK>(p, plan, split, stream);
@@ -145,7 +145,7 @@ static hipError_t launch_op(GemmParams p, const WeightGradPlan* plan, const Spli
 //        instead of a pipeline (tuning aid)
 //        16-bit forward / input-grad: 256 x 128, eight wavefronts of 64 x 64, three LDS stages, where pairs are faster
 //    64:  64 x  64, for problems with few tiles: 16-bit sixteen wavefronts of 32 x 32 in four groups that
-//        share every R step between them; fp32 eight, in two such groups; rows shorter than a 16-byte piece (fp32: weight-grad), four
+//        share every R step between them; fp32 eight, in two such groups; weight-grad of many short loops, and rows shorter than a 16-byte piece, four
 //        16-bit forward / input-grad of at most 32 rows: 32 x 128 (eight wavefronts of 32 x 32 in two groups
 //        that share every R step, three LDS stages)
 //    32:  32 x  64 (fp32 forward / input-grad whose rows would leave a 64-row tile at most half full): four wavefronts of 32 x 32 in two such groups

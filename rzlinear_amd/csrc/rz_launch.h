@@ -1123,9 +1123,13 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
   const bool pieces_ok = (op == kWeightGrad ? (I >= vec && J >= vec) : R >= vec) && (chunk >= R || chunk % step_direct == 0);
   f.clamp = !f.full && direct_capable && pieces_ok && t.clamp != -1;
   f.step = (f.full || f.clamp) ? step_direct : step_plain;
+  // (fp32 weight-grad on the 64 tile: in two groups, as forward and input-grad, but for many workgroups of a short loop, where adding the groups up costs
+  //  more than they hide.  Four wavefronts / eight, us: M = 160, 3008 x 6400, 4700 workgroups 67.2 / 76.3; M = 160, 3008 x 1024, 752 of them 15.5 / 16.5; 1024^3 and the
+  //  fold behind it 31.1 / 30.1.)
+  const bool two_groups = workgroups <= 2 * kComputeUnits || (chunk < R ? chunk : R) >= 384;
   f.waves = tile == 256 ? 8
             : tile == 32 ? 4
-            : tile == 64 ? ((many64 && (f.full || f.clamp)) ? 16 : (elem_bytes == 4 && (op != kWeightGrad || f.full || f.clamp)) ? 8 : 4)
+            : tile == 64 ? ((many64 && (f.full || f.clamp)) ? 16 : (elem_bytes == 4 && (op != kWeightGrad || (two_groups && (f.full || f.clamp)))) ? 8 : 4)
                          : waves128;
   if (tile == 128 && f.waves == 8 && elem_bytes == 2 && (f.full || f.clamp)) f.stages = 4;
   if (f.waves == 16) f.stages = workgroups <= kComputeUnits ? 4 : 2;
@@ -1200,6 +1204,7 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
   if (i.rows != i.cols && !pair) return b;
   b.full = i.full && w.full;
   if (i.rows == 64 && w.tile == 64) {
+    if (w.waves != i.waves) return b;
     b.pair = k64With64;
     b.stages = elem_bytes == 2 && ig_wgs + plan.workgroups <= kComputeUnits ? 4 : 2;
   } else if (elem_bytes == 2 && i.rows == 64 && w.tile == 128 && w.waves == 8) {

@@ -21,7 +21,7 @@ PAIRS = [
     ((62, 1001, 1203, 65536, 32, 64), BF16),       # ... stored tiles
     ((1024, 1024, 1024, 65536, 64, 64), FP32),     # fp32 64 with 64
     ((300, 135, 961, 16384, 64, 64), FP32),        # ... both cut, ragged
-    ((61, 8384, 448, 234752, 64, 64), FP32),       # ... many more workgroups than compute units
+    ((61, 8384, 448, 234752, 64, 64), FP32),       # ... many more workgroups than compute units, of a short loop: apart
     ((2048, 1024, 1024, 20000, 64, 64), BF16),     # 128 with 128
     ((3738, 679, 525, 8192, 64, 64), FP16),        # ... ragged, eight slices (whole ones to an XCD)
     ((3072, 2048, 2048, 31340, 64, 64), BF16),     # 256 x 128 with 256
