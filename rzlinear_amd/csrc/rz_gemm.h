@@ -283,6 +283,9 @@ struct GemmKernel {
   // spills instead comes back through the vector-memory counter, where waiting for it means waiting for the operand
   // loads just issued as well.
   static constexpr bool kColsumInLds = COLSUM && TI == 256 && kDirect;
+  // The threads that add column sums: all of them, but for the 16-bit 128 tile of sixteen wavefronts (the common launch's, beside a 64 tile),
+  // where the first half adds what all threads of the tile's own kernel of eight wavefronts do, so that dbias has the same bits.
+  static constexpr int kColsumThreads = kDirect16 && TI == 128 && kThreads == 1024 ? 512 : kThreads;
   struct Smem {
     alignas(16) T a[NSTAGE][LA::kElems];
     alignas(16) T b[NSTAGE][LB::kElems];
@@ -713,9 +716,9 @@ struct GemmKernel {
     // (tid / kCpr, tid % kCpr) adds rows g, g + groups, ... of the 16-byte column position c
     // (16-bit: the rows are a multiple of four apart, so they share one swizzle).
     auto colsum_from_stage = [&](int st) {
-      constexpr int kGroups = kThreads / LB::kCpr;
+      constexpr int kGroups = kColsumThreads / LB::kCpr;
       static_assert(!(COLSUM && kDirect) || (TR % kGroups == 0 && (!k16 || kGroups % 4 == 0)), "rows must share a swizzle");
-      if (colsum_turn == ti) {
+      if (colsum_turn == ti && (kColsumThreads == kThreads || tid < kColsumThreads)) {   // (uniform in a wavefront)
         const int g = tid / LB::kCpr, c = tid % LB::kCpr;
         colsum_fetch();
 #pragma unroll
@@ -1512,11 +1515,13 @@ struct GemmKernel {
       __syncthreads();                                 // every wavefront is done reading them
       if constexpr (COLSUM) {
         // combine the threads that share columns (fixed order), one row of partial sums out
-        constexpr int kGroups = kThreads / LB::kCpr;
+        constexpr int kGroups = kColsumThreads / LB::kCpr;
         static_assert(sizeof(float) * kGroups * TJ <= sizeof(Smem), "column sums must fit the stages");
-        colsum_fetch();
+        if (kColsumThreads == kThreads || tid < kColsumThreads) {
+          colsum_fetch();
 #pragma unroll
-        for (int e = 0; e < VEC; e++) image[(tid / LB::kCpr) * TJ + (tid % LB::kCpr) * VEC + e] = colsum[e];
+          for (int e = 0; e < VEC; e++) image[(tid / LB::kCpr) * TJ + (tid % LB::kCpr) * VEC + e] = colsum[e];
+        }
         __syncthreads();
         for (int c = tid; c < TJ; c += kThreads) {
           float s = 0.f;

@@ -61,6 +61,29 @@ def test_same_bits_as_apart(shape, dtype):
         assert torch.isfinite(b.float()).all() and torch.equal(a, b), name
 
 
+@pytest.mark.parametrize("shape,dtype", PAIRS, ids=str)
+def test_same_fp32_bits_of_the_bias_gradient(shape, dtype):
+    # (in fp32: rounded to 16 bits, sums in another order hardly ever differ)
+    from rzlinear_amd import _lib
+    M, K, N, H, BK, BN = shape
+    print(shape, dtype, flush=True)
+    (x, hw, dy), _ = make_inputs(M, K, N, H, dtype, seed=M + N)
+    R = _lib.hash_constants(*[R1024[7 - i] for i in range(8)])
+    lib, code, flags, stream = _lib.load(), _lib.dtype_code(x), _lib.WG_DHW_F32 | _lib.WG_DBIAS_F32, _lib.require_gpu(x, hw, dy)
+    sizes = (M, K, N, H, BK, BN)
+    ws = [_lib.workspace(n + 256, x.device) for n in (lib.rz_input_grad_hashed_workspace_bytes(*sizes, code, None),
+                                                      lib.rz_weight_grad_hashed_workspace_bytes(*sizes, code, flags, 1, None))]
+    dx, dhw = torch.empty_like(x), torch.empty((H,), device=x.device)
+    together, apart = (torch.full((N,), float("nan"), device=x.device) for _ in range(2))
+    _lib.check(lib.rz_linear_backward_hashed(
+        x.data_ptr(), dy.data_ptr(), hw.data_ptr(), dx.data_ptr(), dhw.data_ptr(), together.data_ptr(), ws[0].data_ptr(), ws[0].numel(),
+        ws[1].data_ptr(), ws[1].numel(), None, 0, *sizes, R, _lib.HASH_TWO_LEVEL, 0.75, K, N, K, code, flags, None, stream))
+    _lib.check(lib.rz_weight_grad_hashed(
+        x.data_ptr(), dy.data_ptr(), dhw.data_ptr(), apart.data_ptr(), ws[1].data_ptr(), ws[1].numel(), *sizes, R, _lib.HASH_TWO_LEVEL, 0.75,
+        K, N, code, flags, None, stream))
+    assert torch.isfinite(apart).all() and torch.equal(together, apart)
+
+
 @pytest.mark.parametrize("shape,dtype", [PAIRS[3], PAIRS[5], PAIRS[14], PAIRS[17]], ids=str)
 def test_accumulating_into_an_fp32_gradient(shape, dtype):
     both, apart = _both_and_apart(shape, dtype, dhw_dtype=FP32, accumulate=True)
