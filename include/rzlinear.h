@@ -357,6 +357,15 @@ int rz_linear_backward_hashed(const void* X, const void* dY, const void* HW, voi
                               float init_factor, int64_t ldx, int64_t lddy, int64_t lddx, int dtype,
                               unsigned flags, const rz_tuning* tuning, void* stream);
 
+/* How that call would be carried out (host-side, touches no device; flags as for rz_plan_query).  Fills out[8] = { which two kernels share a launch:
+ * 0 none, 1 the 64 tile with 64, 2 64 with 128, 3 256 x 128 with 128, 4 256 x 128 with 256, 5 256 with 256, 6 256 with 128, 7 128 with 128 (input-grad's
+ * with weight-grad's); 1: without bounds checks; LDS stages of the 64 tiles; 1: the weight-grad's workgroups come first; input-grad: 0 as planned without
+ * runs, 1 in whole tiles in place of runs, 2 in runs; for windows of dHW, with X and dY of whole 16-byte pieces in every row and a workspace with room for
+ * the fragments: workgroups beside the input-grad that make them (-1: a kernel of their own, 0: none are made), rows of the input-grad's C tile there,
+ * 1: without bounds checks }.  For tests; no counterpart in the reference. */
+int rz_backward_query(int M, int K, int N, int H, int BK, int BN, int dtype, unsigned flags, int with_dbias,
+                      const rz_tuning* tuning, int32_t out[8]);
+
 /*
  * Materialise W[K,N] (row pitch ldw) from hashed_weight; edge tiles are clipped.
  * Replaces rz_linear_idx_tl                                           impl/RzLinearIdx.py:6-45

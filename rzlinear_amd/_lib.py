@@ -24,6 +24,7 @@ EXPORTS = (
     "rz_forward_hashed_workspace_bytes", "rz_input_grad_hashed_workspace_bytes",
     "rz_weight_grad_hashed_workspace_bytes", "rz_plan_query", "rz_weight_grad_static",
     "rz_layer_plan_bytes", "rz_layer_plan_build", "rz_weight_grad_planned", "rz_linear_backward_hashed",
+    "rz_backward_query",
     "rz_sgd_step", "rz_adam_step", "rz_adam_step_many", "rz_mfma_probe",
 )
 
@@ -173,6 +174,8 @@ def load():
                                               ctypes.c_uint, tun, c_vp]
     lib.rz_plan_query.restype = c_int
     lib.rz_plan_query.argtypes = [c_int] * 8 + [ctypes.c_uint, c_int, tun, i32p]
+    lib.rz_backward_query.restype = c_int
+    lib.rz_backward_query.argtypes = [c_int] * 7 + [ctypes.c_uint, c_int, tun, i32p]
     f32p = c_vp
     lib.rz_sgd_step.restype = c_int
     lib.rz_sgd_step.argtypes = [c_vp, c_vp, f32p, f32p, c_i64, c_int, c_int, c_f, c_f, c_f, c_f, c_int, c_int, c_f, c_vp]
@@ -355,3 +358,16 @@ def plan_query(op, M, K, N, H, BK, BN, dtype_code_, flags=0, with_dbias=False, p
         ans = _host_answers[key] = dict(tile=out[0], slices=out[1], slice_len=out[2], step=out[3],
                                         mode=PLAN_MODES[out[4]], workgroups=out[5], shares=out[6], windows=out[7])
     return dict(ans)
+
+
+BACKWARD_PAIRS = {0: None, 1: "64+64", 2: "64+128", 3: "256x128+128", 4: "256x128+256", 5: "256+256", 6: "256+128", 7: "128+128"}
+
+
+def backward_query(M, K, N, H, BK, BN, dtype_code_, flags=0, with_dbias=True, planned=True):
+    """How rz_linear_backward_hashed would carry out a call (rz_backward_query), under the current tuning: dict(pair (None: two
+    launches), full, stages, weight_grad_first, input_grad ("plain", "whole", "runs"), fragments (workgroups or -1, rows of the C tile, full))."""
+    out = (ctypes.c_int32 * 8)()
+    check(load().rz_backward_query(M, K, N, H, BK, BN, dtype_code_, flags | (PLAN_WITH_LAYER_PLAN if planned else 0), int(with_dbias),
+                                   current_tuning(), out))
+    return dict(pair=BACKWARD_PAIRS[out[0]], full=bool(out[1]), stages=out[2], weight_grad_first=bool(out[3]),
+                input_grad=("plain", "whole", "runs")[out[4]], fragments=(out[5], out[6], bool(out[7])))

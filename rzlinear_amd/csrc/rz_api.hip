@@ -363,6 +363,17 @@ struct InputGradCall {
   SplitPlan split;
 };
 
+// Which launch the two contractions of a backward pass have in common, if any; *split, the input-grad's plan, becomes one in whole tiles where
+// those go beside the weight-grad in place of runs.
+static BackwardForm backward_choice(int M, int K, int N, int H, int elem_bytes, bool with_dbias, const WeightGradChoice& choice,
+                                    const rz_tuning& tuning, SplitPlan* split) {
+  BackwardForm form = {};
+  if (choice.window.use) return form;
+  const SplitPlan whole = backward_whole_tiles(M, K, N, *split, choice.plan);
+  if (whole.tile != 0) *split = whole;
+  return backward_form(M, K, N, H, *split, choice.plan, with_dbias, elem_bytes, tuning);
+}
+
 // The contraction of a weight-grad, with the input-grad's in the same launch where `form` says so.
 static hipError_t launch_weight_contraction(int dtype, const GemmParams& p, const WeightGradPlan& plan, const InputGradCall* with,
                                             const BackwardForm& form, const rz_tuning& tuning, hipStream_t s) {
@@ -532,14 +543,11 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
   if (with != nullptr) {
     st = prepare_plain_op(dtype, with->p, nullptr, with->workspace, with->workspace_bytes, tuning, s, &with->split);
     if (st != RZ_OK) return st;
-    if (!wp.use) {
-      const SplitPlan whole = backward_whole_tiles(M, K, N, with->split, plan);
-      if (whole.tile != 0) {
-        with->split = whole;
-        with->p.partial = nullptr;
-        with->p.finish = nullptr;
-      }
-      form = backward_form(M, K, N, H, with->split, plan, dbias != nullptr, dtype_bytes(dtype), tuning);
+    const bool runs = with->split.run_steps > 0;
+    form = backward_choice(M, K, N, H, dtype_bytes(dtype), dbias != nullptr, choice, tuning, &with->split);
+    if (runs && with->split.run_steps == 0) {
+      with->p.partial = nullptr;
+      with->p.finish = nullptr;
     }
     if (w.packed_x != nullptr) {
       const bool pieces = ((uintptr_t)X | (uintptr_t)dY) % 16 == 0 && (ldx | lddy) % 8 == 0;
@@ -1145,6 +1153,34 @@ RZ_API int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int
   const long long tiles = f.rows == sp.tile ? tile_count(I, J, sp.tile) : (long long)((I + f.rows - 1) / f.rows) * ((J + f.cols - 1) / f.cols);
   out[5] = (int32_t)(tiles * sp.splits);
   out[6] = (cut && t.finish != -1 && sp.splits <= finish_slices(sp.tile, I, J, R, eb, t) && tile_count(I, J, sp.tile) <= (long long)kFinishPerStream) ? 1 : 0;
+  return RZ_OK;
+}
+
+RZ_API int rz_backward_query(int M, int K, int N, int H, int BK, int BN, int dtype, unsigned flags, int with_dbias,
+                             const rz_tuning* tuning, int32_t out[8]) {
+  if (out == nullptr) return RZ_ERR_NULL_POINTER;
+  const int eb = dtype_bytes(dtype);
+  if (eb == 0) return RZ_ERR_BAD_DTYPE;
+  if (M < 1 || K < 1 || N < 1 || H < 1) return RZ_ERR_BAD_SHAPE;
+  const rz_tuning t = tuning_or_default(tuning);
+  if (!tuning_valid(t)) return RZ_ERR_BAD_ARGUMENT;
+  const int st = check_tile(BK, BN);
+  if (st != RZ_OK) return st;
+  const bool dhw_f32 = (flags & RZ_WG_DHW_F32) != 0 || dtype == RZ_F32, planned = (flags & RZ_PLAN_WITH_LAYER_PLAN) != 0;
+  const WeightGradChoice c = weight_grad_choice(M, K, N, H, BK, BN, eb, fold_tile_bytes(eb, dhw_f32, t), t,
+                                                planned && layer_plan_layout(K, N, H, BK, BN).windows > 0);
+  SplitPlan split = split_plan(M, K, N, eb, t);
+  const bool runs = split.run_steps > 0;
+  const BackwardForm f = backward_choice(M, K, N, H, eb, with_dbias != 0, c, t, &split);
+  for (int i = 0; i < 8; i++) out[i] = 0;
+  out[4] = split.run_steps > 0 ? 2 : runs ? 1 : 0;
+  if (f.pair != kApart) {
+    out[0] = f.pair; out[1] = f.full; out[2] = f.stages; out[3] = f.wg_first;
+  }
+  if (c.window.use && c.window.pack_bytes > 0) {
+    const PackForm pack = pack_form(M, K, N, BK, BN, true, split, eb, t);
+    out[5] = pack.groups > 0 ? pack.groups : -1; out[6] = pack.rows; out[7] = pack.full;
+  }
   return RZ_OK;
 }
 

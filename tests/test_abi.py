@@ -307,3 +307,40 @@ def test_adam_step_many_looks_at_the_whole_dtype_word():
     for dtypes in ((1 << 32, 0), (0, 1 << 32), (1 << 32, 1 << 32), ((1 << 33) | _lib.RZ_BF16, _lib.RZ_F32), (-(1 << 32), -(1 << 32))):
         words = (ctypes.c_int64 * 8)(at, at, at, at, 0, 16, *dtypes)
         assert lib.rz_adam_step_many(words, 1, 1e-3, 0.9, 0.999, 1e-8, 0.0, 0, 1, 1.0, None) == -5, dtypes   # RZ_ERR_BAD_DTYPE
+
+
+def test_linear_backward_argument_checks(lib):
+    """rz_linear_backward_hashed refuses what the two calls refuse, before anything is enqueued."""
+    from rzlinear_amd import _lib
+    one = ctypes.c_void_p(256)
+
+    def call(M=96, K=320, N=192, H=8192, BK=32, BN=64, x=one, dy=one, hw=one, dx=one, dhw=one, db=one, ws_dx=(None, 0), ws_dhw=(one, 1 << 30),
+             plan=(None, 0), R=R1024, levels=2, ldx=None, lddy=None, lddx=None, dtype=1, flags=0, tuning=None):
+        return lib.rz_linear_backward_hashed(x, dy, hw, dx, dhw, db, *ws_dx, *ws_dhw, *plan, M, K, N, H, BK, BN, _R(R), levels, 1.0,
+                                             K if ldx is None else ldx, N if lddy is None else lddy, K if lddx is None else lddx, dtype,
+                                             flags, tuning, None)
+    for name in ("x", "dy", "hw", "dx", "dhw"):
+        assert call(**{name: None}) == -1, name
+    assert call(dtype=3) == -5
+    assert call(M=0) == -2 and call(K=0, ldx=8, lddx=8) == -2
+    for pitch in (dict(ldx=319), dict(lddy=191), dict(lddx=319), dict(ldx=1 << 40), dict(lddx=1 << 40)):
+        assert call(**pitch) == -2, pitch
+    assert call(BK=48) == -3
+    assert call(H=2048) == -4
+    assert call(R=[2**31 - 1] + R1024[1:]) == -6
+    assert call(levels=4) == -9 and call(flags=0x100) == -9 and call(tuning=ctypes.byref(_lib.Tuning(tile=77))) == -9
+    assert call(plan=(one, 4)) == -9   # not the size of this layer's plan
+    # each of the two workspaces is asked for: column sums and images of dHW ...
+    need = lib.rz_weight_grad_hashed_workspace_bytes(96, 320, 192, 8192, 32, 64, 1, 0, 1, None)
+    assert need > 0 and call(ws_dhw=(one, need - 1)) == -7 and call(ws_dhw=(None, need)) == -7
+    # ... and the planes of an input-grad that is cut
+    cut = dict(M=160, K=320, N=1536, H=8192, BK=64, BN=64)
+    need = lib.rz_input_grad_hashed_workspace_bytes(*cut.values(), 1, None)
+    assert need > 0 and call(**cut, ws_dx=(one, need - 1)) == -7 and call(**cut, ws_dx=(None, need)) == -7
+
+
+def test_backward_query_argument_checks(lib):
+    out = (ctypes.c_int32 * 8)()
+    call = lambda M=96, K=320, N=192, H=8192, BK=32, BN=64, dtype=1, o=out: lib.rz_backward_query(M, K, N, H, BK, BN, dtype, 0, 1, None, o)
+    assert call() == 0 and list(out[:5]) == [1, 0, 4, 0, 0]
+    assert call(o=None) == -1 and call(M=0) == -2 and call(BK=48) == -3 and call(dtype=3) == -5

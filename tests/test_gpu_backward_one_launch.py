@@ -9,34 +9,50 @@ pytestmark = pytest.mark.gpu
 R1024 = SEED_CONSTANTS[1024]
 BF16, FP16, FP32 = torch.bfloat16, torch.float16, torch.float32
 
-# (M, K, N, H, BK, BN), dtype: every pair of kernels, complete and ragged, at its smallest and around a round of workgroups
+# (M, K, N, H, BK, BN), dtype, the form that it takes (_lib.backward_query): every pair of kernels, complete and ragged, at its smallest and around a
+# round of workgroups
+APART = (None, False, 0)
 PAIRS = [
-    ((96, 320, 192, 8192, 32, 64), BF16),          # 64 with 64, four stages, a ragged M
-    ((1, 8, 9, 4096, 32, 64), BF16),               # ... one tile each, rows that are not whole pieces
-    ((263, 286, 163, 8192, 64, 64), FP16),         # ... three slices of M
-    ((128, 1024, 1024, 65536, 32, 64), BF16),      # ... more workgroups than compute units: two stages; stored tiles
-    ((128, 256, 256, 16384, 32, 64), FP16),        # 64 with 128, complete
-    ((160, 320, 1536, 8192, 64, 64), BF16),        # ... the input-grad cut
-    ((337, 885, 1501, 13268, 32, 64), FP16),       # ... ragged, three slices of M
-    ((62, 1001, 1203, 65536, 32, 64), BF16),       # ... stored tiles
-    ((1024, 1024, 1024, 65536, 64, 64), FP32),     # fp32 64 with 64
-    ((300, 135, 961, 16384, 64, 64), FP32),        # ... both cut, ragged
-    ((61, 8384, 448, 234752, 64, 64), FP32),       # ... many more workgroups than compute units, of a short loop: apart
-    ((2048, 1024, 1024, 20000, 64, 64), BF16),     # 128 with 128
-    ((3738, 679, 525, 8192, 64, 64), FP16),        # ... ragged, eight slices (whole ones to an XCD)
-    ((3072, 2048, 2048, 31340, 64, 64), BF16),     # 256 x 128 with 256
-    ((3001, 2047, 1531, 31340, 64, 64), FP16),     # ... nothing a multiple of anything
-    ((6144, 2048, 1536, 31340, 64, 64), BF16),     # 256 with 256
-    ((6011, 2050, 1530, 31340, 64, 64), BF16),
-    ((14456, 556, 802, 27869, 64, 64), BF16),      # 256 with 128, seven slices
-    ((5056, 2304, 256, 36864, 64, 64), FP16),
-    ((4288, 2304, 4544, 654336, 64, 64), BF16),    # 256 with 256, apart: no compute unit would be done sooner
-    ((513, 6143, 6145, 300000, 64, 64), BF16),     # 256 x 128 with 256, stored tiles, ragged
-    ((128, 2048, 4096, 400000, 32, 64), BF16),     # windows of dHW: no launch in common
-    ((16384, 512, 1024, 5243, 64, 64), BF16),      # 256 x 128 with 128
-    ((5001, 1030, 1021, 20000, 64, 64), FP16),
-    ((2048, 4096, 1024, 262144, 32, 64), BF16),    # ... stored tiles
+    ((96, 320, 192, 8192, 32, 64), BF16, ("64+64", False, 4)),        # a ragged M
+    ((1, 8, 9, 4096, 32, 64), BF16, APART),                           # rows that are not whole pieces
+    ((263, 286, 163, 8192, 64, 64), FP16, ("64+64", False, 4)),       # three slices of M
+    ((128, 1024, 1024, 65536, 32, 64), BF16, ("64+64", True, 2)),     # more workgroups than compute units; stored tiles
+    ((128, 256, 256, 16384, 32, 64), FP16, ("64+128", True)),
+    ((160, 320, 1536, 8192, 64, 64), BF16, ("64+128", False)),        # the input-grad cut
+    ((337, 885, 1501, 13268, 32, 64), FP16, ("64+128", False)),       # three slices of M
+    ((62, 1001, 1203, 65536, 32, 64), BF16, ("64+128", False)),       # stored tiles
+    ((1024, 1024, 1024, 65536, 64, 64), FP32, ("64+64", True, 2)),
+    ((300, 135, 961, 16384, 64, 64), FP32, ("64+64", False, 2)),      # both cut
+    ((61, 8384, 448, 234752, 64, 64), FP32, APART),                   # many more workgroups than compute units, of a short loop
+    ((2048, 1024, 1024, 20000, 64, 64), BF16, ("128+128", True)),
+    ((3738, 679, 525, 8192, 64, 64), FP16, ("128+128", False)),       # eight slices (whole ones to an XCD)
+    ((3072, 2048, 2048, 31340, 64, 64), BF16, ("256x128+256", True)),
+    ((3001, 2047, 1531, 31340, 64, 64), FP16, ("256x128+256", False)),   # nothing a multiple of anything
+    ((6144, 2048, 1536, 31340, 64, 64), BF16, APART),
+    ((6011, 2050, 1530, 31340, 64, 64), BF16, APART),
+    ((14456, 556, 802, 27869, 64, 64), BF16, ("256+128", False)),     # seven slices
+    ((5056, 2304, 256, 36864, 64, 64), FP16, APART),
+    ((4288, 2304, 4544, 654336, 64, 64), BF16, APART),                # no compute unit would be done sooner
+    ((513, 6143, 6145, 300000, 64, 64), BF16, APART),
+    ((128, 2048, 4096, 400000, 32, 64), BF16, APART),                 # windows of dHW
+    ((16384, 512, 1024, 5243, 64, 64), BF16, APART),                  # whole rounds of both
+    ((5001, 1030, 1021, 20000, 64, 64), FP16, ("256x128+128", False)),
+    ((2048, 4096, 1024, 262144, 32, 64), BF16, ("256x128+128", True)),   # stored tiles
+    ((128, 192, 128, 8192, 32, 64), BF16, ("64+64", True, 4)),
+    ((7, 4387, 161, 8192, 32, 64), FP16, ("64+64", False, 2)),
+    ((320, 14336, 768, 110100, 32, 64), BF16, ("256x128+256", False)),
+    ((768, 11008, 512, 8192, 32, 64), FP16, ("256+256", True)),
+    ((1056, 7616, 704, 8192, 32, 64), BF16, ("256+256", False)),
+    ((3584, 2816, 384, 16384, 64, 64), BF16, ("256+128", True)),
+    ((3328, 1280, 256, 20480, 64, 64), FP16, ("256x128+128", True)),
 ]
+CODES = {FP32: 0, BF16: 1, FP16: 2}
+
+
+def assert_form(shape, dtype, form):
+    from rzlinear_amd import _lib
+    q = _lib.backward_query(*shape, CODES[dtype])
+    assert (q["pair"], q["full"], q["stages"])[:len(form)] == form, q
 
 
 def _both_and_apart(shape, dtype, dhw_dtype=None, accumulate=False):
@@ -54,14 +70,15 @@ def _both_and_apart(shape, dtype, dhw_dtype=None, accumulate=False):
     return both, (dx, dhw, db)
 
 
-@pytest.mark.parametrize("shape,dtype", PAIRS, ids=str)
-def test_same_bits_as_apart(shape, dtype):
+@pytest.mark.parametrize("shape,dtype,form", PAIRS, ids=str)
+def test_same_bits_as_apart(shape, dtype, form):
+    assert_form(shape, dtype, form)
     both, apart = _both_and_apart(shape, dtype)
     for name, a, b in zip(("dx", "dhw", "dbias"), both, apart):
         assert torch.isfinite(b.float()).all() and torch.equal(a, b), name
 
 
-@pytest.mark.parametrize("shape,dtype", PAIRS, ids=str)
+@pytest.mark.parametrize("shape,dtype", [p[:2] for p in PAIRS], ids=str)
 def test_same_fp32_bits_of_the_bias_gradient(shape, dtype):
     # (in fp32: rounded to 16 bits, sums in another order hardly ever differ)
     from rzlinear_amd import _lib
@@ -84,30 +101,37 @@ def test_same_fp32_bits_of_the_bias_gradient(shape, dtype):
     assert torch.isfinite(apart).all() and torch.equal(together, apart)
 
 
-@pytest.mark.parametrize("shape,dtype", [PAIRS[3], PAIRS[5], PAIRS[14], PAIRS[17]], ids=str)
+@pytest.mark.parametrize("shape,dtype", [PAIRS[i][:2] for i in (3, 5, 14, 17)], ids=str)
 def test_accumulating_into_an_fp32_gradient(shape, dtype):
     both, apart = _both_and_apart(shape, dtype, dhw_dtype=FP32, accumulate=True)
     for a, b in zip(both, apart):
         assert torch.equal(a, b)
 
 
-# Windows of dHW whose operands' fragments are made beside the input-grad: its 32 x 128, 64, 128 and 256 x 128 tiles, complete and ragged
+# Windows of dHW whose operands' fragments are made beside the input-grad: by rows of its C tile (32, 64, 128, 256 x 128), complete and ragged
 FRAGMENTS = [
-    ((32, 10240, 10240, 6553600, 32, 64), BF16),
-    ((19, 10232, 10240, 6553600, 32, 64), FP16),
-    ((61, 3000, 4008, 750000, 32, 64), FP16),
-    ((128, 4096, 4096, 700000, 32, 64), BF16),
-    ((128, 10240, 10240, 6553600, 32, 64), BF16),
-    ((96, 5000, 7000, 2200000, 32, 64), BF16),
-    ((150, 3000, 5000, 937500, 32, 64), FP16),
-    ((224, 10240, 10240, 6553600, 32, 64), BF16),
-    ((61, 3001, 4008, 750000, 32, 64), FP16),      # rows that are not whole pieces: by a kernel of their own
+    ((32, 10240, 10240, 6553600, 32, 64), BF16, (32, True)),
+    ((19, 10232, 10240, 6553600, 32, 64), FP16, (32, False)),
+    ((61, 3000, 4008, 750000, 32, 64), FP16, None),               # none are made
+    ((128, 4096, 4096, 700000, 32, 64), BF16, "own"),             # no compute unit is idle: by a kernel of their own
+    ((128, 10240, 10240, 6553600, 32, 64), BF16, (128, True)),
+    ((96, 5000, 7000, 2200000, 32, 64), BF16, (128, False)),
+    ((150, 3000, 5000, 937500, 32, 64), FP16, (128, False)),
+    ((224, 10240, 10240, 6553600, 32, 64), BF16, (256, False)),
+    ((61, 3001, 4008, 750000, 32, 64), FP16, "own"),              # rows that are not whole pieces
+    ((256, 3328, 2048, 425984, 32, 64), BF16, (64, True)),
+    ((5, 1344, 12736, 171171, 64, 64), FP16, (64, False)),
+    ((256, 5888, 5120, 1884160, 64, 64), BF16, (256, True)),
+    ((32, 10240, 10240, 6553600, 32, 64), FP32, "own"),
 ]
 
 
 @pytest.mark.parametrize("accumulate", [False, True])
-@pytest.mark.parametrize("shape,dtype", FRAGMENTS, ids=str)
-def test_fragments_beside_the_input_grad(shape, dtype, accumulate):
+@pytest.mark.parametrize("shape,dtype,beside", FRAGMENTS, ids=str)
+def test_fragments_beside_the_input_grad(shape, dtype, beside, accumulate):
+    from rzlinear_amd import _lib
+    groups, *form = _lib.backward_query(*shape, CODES[dtype])["fragments"]
+    assert (None if groups == 0 else "own" if groups < 0 else tuple(form)) == beside
     both, apart = _both_and_apart(shape, dtype, accumulate=accumulate)
     for name, a, b in zip(("dx", "dhw", "dbias"), both, apart):
         assert torch.isfinite(b.float()).all() and torch.equal(a, b), name
@@ -124,7 +148,7 @@ def test_an_input_grad_in_runs_goes_in_whole_tiles():
     assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-5 * b.abs().max()).all()
 
 
-@pytest.mark.parametrize("shape,dtype", [PAIRS[0], PAIRS[3], PAIRS[5], PAIRS[11], FRAGMENTS[0], FRAGMENTS[5]], ids=str)
+@pytest.mark.parametrize("shape,dtype", [p[:2] for p in (PAIRS[0], PAIRS[3], PAIRS[5], PAIRS[11], FRAGMENTS[0], FRAGMENTS[5])], ids=str)
 def test_captured_backward(shape, dtype):
     # (a cut input-grad has no counters under capture: a second kernel behind the common launch, the same bits)
     from rzlinear_amd import RzLinear
