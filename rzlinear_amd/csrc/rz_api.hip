@@ -68,7 +68,7 @@ static int make_hash(HashParams* h, int K, int N, int H, int BK, int BN, const i
 
 // Row pitches are limited so that a tile's rows stay within the 32-bit byte offsets of the kernels'
 // load addresses (256 rows of 2^23 four-byte elements are 2^33 bytes: the limit is per element type below).
-static bool pitch_ok(int64_t ld, int elem_bytes) { return ld > 0 && ld * elem_bytes * 256 < (1LL << 32); }
+static bool pitch_ok(int64_t ld, int elem_bytes) { return ld > 0 && ld < (1LL << 32) / (elem_bytes * 256); }
 
 static int dtype_bytes(int dtype) {
   switch (dtype) {

@@ -323,7 +323,7 @@ def test_linear_backward_argument_checks(lib):
         assert call(**{name: None}) == -1, name
     assert call(dtype=3) == -5
     assert call(M=0) == -2 and call(K=0, ldx=8, lddx=8) == -2
-    for pitch in (dict(ldx=319), dict(lddy=191), dict(lddx=319), dict(ldx=1 << 40), dict(lddx=1 << 40)):
+    for pitch in (dict(ldx=319), dict(lddy=191), dict(lddx=319), dict(ldx=1 << 23), dict(ldx=1 << 62), dict(lddy=1 << 62), dict(lddx=1 << 62)):
         assert call(**pitch) == -2, pitch
     assert call(BK=48) == -3
     assert call(H=2048) == -4
@@ -344,3 +344,14 @@ def test_backward_query_argument_checks(lib):
     call = lambda M=96, K=320, N=192, H=8192, BK=32, BN=64, dtype=1, o=out: lib.rz_backward_query(M, K, N, H, BK, BN, dtype, 0, 1, None, o)
     assert call() == 0 and list(out[:5]) == [1, 0, 4, 0, 0]
     assert call(o=None) == -1 and call(M=0) == -2 and call(BK=48) == -3 and call(dtype=3) == -5
+
+
+def test_row_pitches_beyond_the_kernels_offsets_are_refused(lib):
+    """256 rows have to stay within 32-bit byte offsets: also a pitch whose product with that wraps round in 64 bits (2^62 elements) is refused."""
+    one = ctypes.c_void_p(256)
+    for dtype, first in ((0, 1 << 22), (1, 1 << 23), (2, 1 << 23)):
+        for ld in (first, 1 << 40, 1 << 54, 1 << 55, 1 << 62, (1 << 62) + 320, (1 << 63) - 1):
+            for ldx, ldy in ((ld, 192), (320, ld)):
+                assert lib.rz_forward(one, one, one, 96, 320, 192, 8192, 32, 64, _R(R1024), 1.0, ldx, ldy, dtype, None) == -2
+                assert lib.rz_input_grad(one, one, one, 96, 320, 192, 8192, 32, 64, _R(R1024), 1.0, ldy, ldx, dtype, None) == -2
+                assert lib.rz_weight_grad(one, one, one, one, 1 << 30, 96, 320, 192, 8192, 32, 64, _R(R1024), 1.0, ldx, ldy, dtype, None) == -2
