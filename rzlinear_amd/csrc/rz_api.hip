@@ -306,12 +306,16 @@ static unsigned* finish_counters_for(long long tiles, hipStream_t s) {
   return nullptr;
 }
 
+// An output of more than twice an L2 goes out with streaming stores (a smaller one may still be
+// in cache when the next kernel reads it).
+static int streams_output(int dtype, const GemmParams& p) {
+  return (size_t)p.I * (size_t)p.J * dtype_bytes(dtype) >= ((size_t)8 << 20) ? 1 : 0;
+}
+
 // What a forward or input-grad that may split its contraction needs of its workspace: p's fields for the plan *sp.
 static int prepare_plain_op(int dtype, GemmParams& p, const void* bias, void* workspace, size_t workspace_bytes,
                             const rz_tuning& tuning, hipStream_t s, SplitPlan* sp) {
-  // an output of more than twice an L2 goes out with streaming stores (a smaller one may still be
-  // in cache when the next kernel reads it)
-  p.stream_c = (size_t)p.I * (size_t)p.J * dtype_bytes(dtype) >= ((size_t)8 << 20) ? 1 : 0;
+  p.stream_c = streams_output(dtype, p);
   // tile and slices are chosen together; a workspace that does not hold the planes of runs is enough where it holds those of slices
   *sp = split_plan(p.I, p.J, p.R, dtype_bytes(dtype), tuning);
   if (sp->run_steps > 0 && (workspace == nullptr || workspace_bytes < sp->workspace_bytes))
@@ -350,7 +354,7 @@ static int run_plain_op(int op, int dtype, GemmParams p, const void* bias, void*
     if (launch_gemm(dtype, op, p, nullptr, &sp, tuning, s) != hipSuccess) return RZ_ERR_LAUNCH;
     return finish_plain_op(dtype, p, bias, sp, s);
   }
-  p.stream_c = (size_t)p.I * (size_t)p.J * dtype_bytes(dtype) >= ((size_t)8 << 20) ? 1 : 0;
+  p.stream_c = streams_output(dtype, p);
   p.bias = bias;
   return launch_gemm(dtype, op, p, nullptr, nullptr, tuning, s) == hipSuccess ? RZ_OK : RZ_ERR_LAUNCH;
 }
@@ -363,15 +367,18 @@ struct InputGradCall {
   SplitPlan split;
 };
 
-// Which launch the two contractions of a backward pass have in common, if any; *split, the input-grad's plan, becomes one in whole tiles where
-// those go beside the weight-grad in place of runs.
+// Which launch the two contractions of a backward pass have in common, if any.  *split, the input-grad's plan: where it is in runs, the
+// common launch takes whole tiles in their place; apart, it is left as it is.
 static BackwardForm backward_choice(int M, int K, int N, int H, int elem_bytes, bool with_dbias, const WeightGradChoice& choice,
                                     const rz_tuning& tuning, SplitPlan* split) {
   BackwardForm form = {};
   if (choice.window.use) return form;
+  if (split->run_steps == 0) return backward_form(M, K, N, H, *split, choice.plan, with_dbias, elem_bytes, tuning);
   const SplitPlan whole = backward_whole_tiles(M, K, N, *split, choice.plan);
-  if (whole.tile != 0) *split = whole;
-  return backward_form(M, K, N, H, *split, choice.plan, with_dbias, elem_bytes, tuning);
+  if (whole.tile == 0) return form;
+  form = backward_form(M, K, N, H, whole, choice.plan, with_dbias, elem_bytes, tuning, split->est_us);
+  if (form.pair != kApart) *split = whole;
+  return form;
 }
 
 // The contraction of a weight-grad, with the input-grad's in the same launch where `form` says so.
@@ -541,13 +548,15 @@ static int weight_grad_impl(const void* X, const void* dY, void* dHW, void* dbia
   // (an input-grad that shares no launch with this call's contraction is enqueued first, like the reference's)
   BackwardForm form = {};
   if (with != nullptr) {
-    st = prepare_plain_op(dtype, with->p, nullptr, with->workspace, with->workspace_bytes, tuning, s, &with->split);
-    if (st != RZ_OK) return st;
-    const bool runs = with->split.run_steps > 0;
-    form = backward_choice(M, K, N, H, dtype_bytes(dtype), dbias != nullptr, choice, tuning, &with->split);
-    if (runs && with->split.run_steps == 0) {
-      with->p.partial = nullptr;
-      with->p.finish = nullptr;
+    const int eb = dtype_bytes(dtype);
+    with->split = split_plan(M, K, N, eb, tuning);
+    if (with->split.run_steps > 0) form = backward_choice(M, K, N, H, eb, dbias != nullptr, choice, tuning, &with->split);
+    if (form.pair != kApart) {   // (whole tiles in place of runs: no planes)
+      with->p.stream_c = streams_output(dtype, with->p);
+    } else {
+      st = prepare_plain_op(dtype, with->p, nullptr, with->workspace, with->workspace_bytes, tuning, s, &with->split);
+      if (st != RZ_OK) return st;
+      form = backward_choice(M, K, N, H, eb, dbias != nullptr, choice, tuning, &with->split);
     }
     if (w.packed_x != nullptr) {
       const bool pieces = ((uintptr_t)X | (uintptr_t)dY) % 16 == 0 && (ldx | lddy) % 8 == 0;

@@ -1192,8 +1192,9 @@ struct BackwardForm {
 static inline long long f_tiles(const KernelForm& f, int I, int J) {
   return (long long)((I + f.rows - 1) / f.rows) * ((J + f.cols - 1) / f.cols);
 }
+// runs_us: sp are whole tiles in place of runs, which take so long by themselves (0: sp is how the input-grad goes by itself).
 static inline BackwardForm backward_form(int M, int K, int N, int H, const SplitPlan& sp, const WeightGradPlan& plan, bool with_dbias,
-                                         int elem_bytes, const rz_tuning& t) {
+                                         int elem_bytes, const rz_tuning& t, double runs_us = 0.0) {
   BackwardForm b = {kApart, false, 2, false};
   if (!with_dbias || sp.run_steps > 0 || t.tile != 0 || t.stages == 1 || t.clamp == -1 || (long long)H * 4 > 0x7fffffffLL) return b;
   const long long ig_wgs = tile_count(M, K, sp.tile) * sp.splits;
@@ -1265,7 +1266,8 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
   // K = 512, N = 1024 61.8 us a pass apart, 59.0 in one launch, M = 8192 60.8 and 59.1; M = 16384 70.2 and 69.9, and 1 us slower where the host is as slow.)
   const double boundary_us = 4.0, mixing = 1.02;
   if (n_i % kComputeUnits == 0 && n_w % kComputeUnits == 0 && (double)M * ((double)K + N) * elem_bytes > 32.0e6) b.pair = kApart;
-  if (end * mixing > (alone(i, false, ig_chunk, N, n_i) + alone(w, true, plan.r_chunk, M, n_w)) + boundary_us) b.pair = kApart;
+  const double ig_alone = runs_us > 0.0 ? runs_us - kForward16Times[6].launch : alone(i, false, ig_chunk, N, n_i);
+  if (end * mixing > (ig_alone + alone(w, true, plan.r_chunk, M, n_w)) + boundary_us) b.pair = kApart;
   return b;
 }
 

@@ -137,15 +137,39 @@ def test_fragments_beside_the_input_grad(shape, dtype, beside, accumulate):
         assert torch.isfinite(b.float()).all() and torch.equal(a, b), name
 
 
-def test_an_input_grad_in_runs_goes_in_whole_tiles():
-    # M = 1024, K = N = 10240: by itself in runs, whose parts are added up in fp32; the whole tiles' sums are in one piece.  Two
-    # correctly accumulated results, each rounded once: they differ by an fp32 sum's error (10240 terms, < 1e-5 of the largest value)
-    # and one unit in the last place of a bf16 value.
-    shape = (1024, 10240, 10240, 6553600, 32, 64)
-    both, apart = _both_and_apart(shape, BF16)
+@pytest.mark.parametrize("shape,dtype,full", [
+    ((1024, 10240, 10240, 6553600, 32, 64), BF16, True), ((2560, 3328, 7168, 23855, 32, 64), FP16, True), ((1044, 16012, 2555, 40910, 64, 64), FP16, False),
+], ids=str)
+def test_an_input_grad_in_runs_goes_in_whole_tiles(shape, dtype, full):
+    # By itself in runs, whose parts are added up in fp32; the whole tiles' sums are in one piece.  Two correctly accumulated results,
+    # each rounded once: they differ by an fp32 sum's error (at most 10240 terms, < 1e-5 of the largest value) and one unit in the last
+    # place of the 16-bit value.
+    from rzlinear_amd import _lib
+    assert_form(shape, dtype, ("256+256", full))
+    assert _lib.backward_query(*shape, CODES[dtype])["input_grad"] == "whole"
+    both, apart = _both_and_apart(shape, dtype)
     assert torch.equal(both[1], apart[1]) and torch.equal(both[2], apart[2])
     a, b = both[0].double(), apart[0].double()
-    assert ((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-5 * b.abs().max()).all()
+    assert ((a - b).abs() <= (2.0 ** -7 if dtype == BF16 else 2.0 ** -10) * b.abs() + 1e-5 * b.abs().max()).all()
+
+
+@pytest.mark.parametrize("shape,dtype,with_bias", [
+    ((1024, 10240, 10240, 6553600, 32, 64), BF16, False), ((3469, 5867, 14924, 5472443, 32, 64), FP16, False),
+    ((5031, 4002, 6371, 1593546, 32, 64), BF16, False),
+    ((15870, 1471, 4555, 418776, 64, 64), BF16, True), ((27152, 604, 3009, 113589, 64, 64), FP16, True),
+], ids=str)
+def test_an_input_grad_apart_stays_in_runs(shape, dtype, with_bias):
+    # where the two ops share no launch (none does without a bias gradient) dX is the separate call's, by the same plan
+    from rzlinear_amd import _lib
+    from rzlinear_amd.impl.RzLinearBackward import backward_hashed, input_grad_hashed
+    q = _lib.backward_query(*shape, CODES[dtype], with_dbias=with_bias)
+    assert (q["pair"], q["input_grad"]) == (None, "runs")
+    M, K, N, H, BK, BN = shape
+    print(shape, dtype, flush=True)
+    (x, hw, dy), _ = make_inputs(M, K, N, H, dtype, seed=5)
+    R = _lib.hash_constants(*[R1024[7 - i] for i in range(8)])
+    dx = backward_hashed(x, hw, dy, 0.75, M, K, N, H, R, BK, BN, with_bias_grad=with_bias)[0]
+    assert torch.equal(dx, input_grad_hashed(dy, hw, 0.75, M, K, N, H, R, BK, BN, _lib.HASH_TWO_LEVEL))
 
 
 @pytest.mark.parametrize("shape,dtype", [p[:2] for p in (PAIRS[0], PAIRS[3], PAIRS[5], PAIRS[11], FRAGMENTS[0], FRAGMENTS[5])], ids=str)

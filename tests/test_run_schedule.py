@@ -124,3 +124,21 @@ def test_planes_of_runs_stay_in_proportion_to_the_call(op, shape):
     assert _lib.plan_query(op, *shape, 200000, 64, 64, _lib.RZ_BF16)["windows"] == 0
     need = lib.rz_forward_hashed_workspace_bytes if op == 0 else lib.rz_input_grad_hashed_workspace_bytes
     assert need(*shape, 200000, 64, 64, _lib.RZ_BF16, None) <= 4 * M * (K + N)
+
+
+def test_a_backward_pass_takes_an_input_grad_out_of_its_runs_only_for_a_common_launch():
+    rng = random.Random(17)
+    runs = whole = 0
+    for _ in range(6000):
+        code = rng.choice([_lib.RZ_BF16, _lib.RZ_F16])
+        call = (rng.randint(65, 16000), rng.randint(512, 16000), rng.randint(512, 16000), 300000, 64, 64, code)
+        alone = _lib.plan_query(1, *call)
+        in_runs = alone["mode"] == "split" and alone["windows"] > 0
+        for with_dbias in (False, True):
+            q = _lib.backward_query(*call, with_dbias=with_dbias)
+            assert (q["input_grad"] == "plain") == (not in_runs), call
+            assert (q["input_grad"] == "whole") == (in_runs and q["pair"] is not None), call
+            assert with_dbias or q["pair"] is None
+            runs += q["input_grad"] == "runs"
+            whole += q["input_grad"] == "whole"
+    assert runs > 50 and whole > 20
