@@ -349,7 +349,10 @@ int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int dtype,
  * results to the bit, but for an input-grad that would be dealt out in runs (rz_plan_query): beside a weight-grad it may
  * go in whole tiles, whose sums over N are in one piece.  Where the two contractions' kernels go together they are
  * enqueued as ONE launch: a launch less, and workgroups of the one fill what those of the other leave idle.  The two workspaces
- * (rz_input_grad_hashed_workspace_bytes, rz_weight_grad_hashed_workspace_bytes) and the outputs must not overlap. */
+ * (rz_linear_backward_hashed_dx_workspace_bytes, which is never more than rz_input_grad_hashed_workspace_bytes, with
+ * RZ_PLAN_WITH_LAYER_PLAN in its flags where the call carries a plan; rz_weight_grad_hashed_workspace_bytes) and the outputs must not overlap. */
+size_t rz_linear_backward_hashed_dx_workspace_bytes(int M, int K, int N, int H, int BK, int BN, int dtype, unsigned flags,
+                                                    int with_dbias, const rz_tuning* tuning);
 int rz_linear_backward_hashed(const void* X, const void* dY, const void* HW, void* dX, void* dHW, void* dbias,
                               void* workspace_dx, size_t workspace_dx_bytes, void* workspace_dhw,
                               size_t workspace_dhw_bytes, const void* layer_plan, size_t layer_plan_bytes,

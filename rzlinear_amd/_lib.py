@@ -24,7 +24,7 @@ EXPORTS = (
     "rz_forward_hashed_workspace_bytes", "rz_input_grad_hashed_workspace_bytes",
     "rz_weight_grad_hashed_workspace_bytes", "rz_plan_query", "rz_weight_grad_static",
     "rz_layer_plan_bytes", "rz_layer_plan_build", "rz_weight_grad_planned", "rz_linear_backward_hashed",
-    "rz_backward_query",
+    "rz_linear_backward_hashed_dx_workspace_bytes", "rz_backward_query",
     "rz_sgd_step", "rz_adam_step", "rz_adam_step_many", "rz_mfma_probe",
 )
 
@@ -174,6 +174,8 @@ def load():
                                               ctypes.c_uint, tun, c_vp]
     lib.rz_plan_query.restype = c_int
     lib.rz_plan_query.argtypes = [c_int] * 8 + [ctypes.c_uint, c_int, tun, i32p]
+    lib.rz_linear_backward_hashed_dx_workspace_bytes.restype = c_sz
+    lib.rz_linear_backward_hashed_dx_workspace_bytes.argtypes = [c_int] * 7 + [ctypes.c_uint, c_int, tun]
     lib.rz_backward_query.restype = c_int
     lib.rz_backward_query.argtypes = [c_int] * 7 + [ctypes.c_uint, c_int, tun, i32p]
     f32p = c_vp

@@ -1165,6 +1165,21 @@ RZ_API int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int
   return RZ_OK;
 }
 
+RZ_API size_t rz_linear_backward_hashed_dx_workspace_bytes(int M, int K, int N, int H, int BK, int BN, int dtype, unsigned flags,
+                                                           int with_dbias, const rz_tuning* tuning) {
+  const rz_tuning t = tuning_or_default(tuning);
+  const int eb = dtype_bytes(dtype);
+  if (eb == 0 || M < 1 || K < 1 || N < 1 || H < 1 || !tuning_valid(t) || check_tile(BK, BN) != RZ_OK) return 0;
+  SplitPlan split = split_plan(M, K, N, eb, t);
+  if (split.run_steps > 0) {   // (no planes for whole tiles in their place)
+    const bool dhw_f32 = (flags & RZ_WG_DHW_F32) != 0 || dtype == RZ_F32, planned = (flags & RZ_PLAN_WITH_LAYER_PLAN) != 0;
+    const WeightGradChoice c = weight_grad_choice(M, K, N, H, BK, BN, eb, fold_tile_bytes(eb, dhw_f32, t), t,
+                                                  planned && layer_plan_layout(K, N, H, BK, BN).windows > 0);
+    backward_choice(M, K, N, H, eb, with_dbias != 0, c, t, &split);
+  }
+  return split.workspace_bytes;
+}
+
 RZ_API int rz_backward_query(int M, int K, int N, int H, int BK, int BN, int dtype, unsigned flags, int with_dbias,
                              const rz_tuning* tuning, int32_t out[8]) {
   if (out == nullptr) return RZ_ERR_NULL_POINTER;

@@ -55,6 +55,7 @@ struct Library {
   decltype(&rz_weight_grad_planned) weight_grad_planned = nullptr;
   decltype(&rz_weight_grad_hashed_workspace_bytes) weight_grad_workspace = nullptr;
   decltype(&rz_linear_backward_hashed) backward = nullptr;
+  decltype(&rz_linear_backward_hashed_dx_workspace_bytes) backward_dx_workspace = nullptr;
   decltype(&rz_plan_query) plan_query = nullptr;
 };
 Library lib;
@@ -218,7 +219,8 @@ void weight_grad(const Geometry& g, const Tensor& input, const Tensor& dy, int64
   void* db = dbias.defined() ? dbias.data_ptr() : nullptr;
   if (hw.defined()) {
     *dx = empty({M, g.K}, dy);
-    const size_t need_dx = lib.input_grad_workspace(M, g.K, g.N, g.H, g.BK, g.BN, code, t);
+    const size_t need_dx = lib.backward_dx_workspace(M, g.K, g.N, g.H, g.BK, g.BN, code, flags | (plan.defined() ? RZ_PLAN_WITH_LAYER_PLAN : 0u),
+                                                     with_dbias, t);
     const at::DataPtr ws_dx = scratch(need_dx);
     check(lib.backward(x.data_ptr(), dy.data_ptr(), hw.data_ptr(), dx->data_ptr(), out.data_ptr(), db, ws_dx.get(), need_dx, ws.get(), need,
                        plan.defined() ? plan.data_ptr<int32_t>() : nullptr, plan.defined() ? (size_t)plan.numel() * 4 : 0, M, g.K, g.N, g.H,
@@ -489,6 +491,7 @@ PyObject* bind(PyObject*, PyObject* args) {
   RZ_BIND(weight_grad_planned, rz_weight_grad_planned);
   RZ_BIND(weight_grad_workspace, rz_weight_grad_hashed_workspace_bytes);
   RZ_BIND(backward, rz_linear_backward_hashed);
+  RZ_BIND(backward_dx_workspace, rz_linear_backward_hashed_dx_workspace_bytes);
   RZ_BIND(plan_query, rz_plan_query);
 #undef RZ_BIND
   Py_INCREF(provider);

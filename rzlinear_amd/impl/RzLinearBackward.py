@@ -90,7 +90,8 @@ def weight_grad_hashed(input, output_grad, init_factor, M, K, N, H, R, BLOCK_SIZ
     if both:
         hw = hashed_weight.contiguous()
         input_grad = torch.empty((M, K), device=output_grad.device, dtype=output_grad.dtype)
-        need_dx = _lib.host_query("rz_input_grad_hashed_workspace_bytes", M, K, N, H, BLOCK_SIZE_K, BLOCK_SIZE_N, code)
+        need_dx = _lib.host_query("rz_linear_backward_hashed_dx_workspace_bytes", M, K, N, H, BLOCK_SIZE_K, BLOCK_SIZE_N, code,
+                                  flags | (_lib.PLAN_WITH_LAYER_PLAN if plan is not None else 0), int(with_bias_grad))
         ws_dx = _lib.workspace(need_dx, output_grad.device)
         _lib.check(lib.rz_linear_backward_hashed(
             x.data_ptr(), dy.data_ptr(), hw.data_ptr(), input_grad.data_ptr(), out.data_ptr(),

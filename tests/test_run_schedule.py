@@ -127,7 +127,7 @@ def test_planes_of_runs_stay_in_proportion_to_the_call(op, shape):
 
 
 def test_a_backward_pass_takes_an_input_grad_out_of_its_runs_only_for_a_common_launch():
-    rng = random.Random(17)
+    lib, rng = _lib.load(), random.Random(17)
     runs = whole = 0
     for _ in range(6000):
         code = rng.choice([_lib.RZ_BF16, _lib.RZ_F16])
@@ -139,6 +139,10 @@ def test_a_backward_pass_takes_an_input_grad_out_of_its_runs_only_for_a_common_l
             assert (q["input_grad"] == "plain") == (not in_runs), call
             assert (q["input_grad"] == "whole") == (in_runs and q["pair"] is not None), call
             assert with_dbias or q["pair"] is None
+            # (planes are asked for where they are used: whole tiles need none)
+            need = lib.rz_input_grad_hashed_workspace_bytes(*call, None)
+            assert lib.rz_linear_backward_hashed_dx_workspace_bytes(*call, _lib.PLAN_WITH_LAYER_PLAN, int(with_dbias), None) == (
+                0 if q["input_grad"] == "whole" else need), call
             runs += q["input_grad"] == "runs"
             whole += q["input_grad"] == "whole"
     assert runs > 50 and whole > 20
