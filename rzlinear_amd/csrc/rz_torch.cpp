@@ -358,7 +358,12 @@ struct RzLinearNode : public Node {
       } else {
         out = result[kWeight] = empty({g.H}, dy);
       }
-      weight_grad(g, x, dy, lddy, out, accumulate, bias_grad, with_plans, need_input ? hw.contiguous() : Tensor(), &result[kInput]);
+      try {
+        weight_grad(g, x, dy, lddy, out, accumulate, bias_grad, with_plans, need_input ? hw.contiguous() : Tensor(), &result[kInput]);
+      } catch (...) {   // (nothing has been written to a fresh buffer: the next backward must not add to it)
+        if (fuse_grad_accumulation && !accumulate) hw.mutable_grad() = Tensor();
+        throw;
+      }
     } else if (need_bias) {
       bias_grad = grad.sum(0);
     }

@@ -124,6 +124,26 @@ def test_a_fused_weight_gradient_is_added_whichever_gradients_the_backward_retur
     assert buffers[0].abs().sum() > 0 and torch.equal(*buffers)
 
 
+@pytest.mark.parametrize("with_input", [False, True], ids=["weight", "weight and input"])
+def test_a_backward_that_fails_leaves_no_fresh_gradient_buffer(with_input):
+    """The buffer that a fused weight gradient makes for a parameter without one holds nothing until the kernels have filled it: after
+    an error (here a refused override) the next backward must not add to it."""
+    from rzlinear_amd import _lib
+    for function in _functions():
+        x, hw, bias, dy = _inputs()
+        y = _call(function, x.requires_grad_(with_input), hw.requires_grad_(), bias, fuse=True)
+        with _lib.tuning(tile=77), pytest.raises(_lib.RzLinearError):
+            y.backward(dy, retain_graph=True)
+        assert hw.grad is None
+        y.backward(dy, retain_graph=True)
+        once = hw.grad.clone()
+        with _lib.tuning(tile=77), pytest.raises(_lib.RzLinearError):   # (one that was there before stays as it is)
+            y.backward(dy, retain_graph=True)
+        assert torch.equal(hw.grad, once)
+        y.backward(dy)
+        assert torch.allclose(hw.grad, 2 * once)
+
+
 def test_no_fused_gradient_for_a_weight_that_needs_none():
     for function in _functions():
         x, hw, bias, dy = _inputs()
