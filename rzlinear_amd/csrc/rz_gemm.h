@@ -283,9 +283,13 @@ struct GemmKernel {
   // spills instead comes back through the vector-memory counter, where waiting for it means waiting for the operand
   // loads just issued as well.
   static constexpr bool kColsumInLds = COLSUM && TI == 256 && kDirect;
-  // The threads that add column sums: all of them, but for the 16-bit 128 tile of sixteen wavefronts (the common launch's, beside a 64 tile),
-  // where the first half adds what all threads of the tile's own kernel of eight wavefronts do, so that dbias has the same bits.
-  static constexpr int kColsumThreads = kDirect16 && TI == 128 && kThreads == 1024 ? 512 : kThreads;
+  // The threads that add column sums: all of them, but for the 16-bit 128 tile of sixteen wavefronts and the fp32 64 tile of eight,
+  // where the first half adds what all threads of the same tile's kernel of half as many wavefronts do, so that dbias has the same bits.
+  static constexpr int kColsumThreads = (kDirect16 && TI == 128 && kThreads == 1024) || (kDirect32 && TI == 64 && kThreads == 512) ? kThreads / 2 : kThreads;
+  // The fp32 64 tile of weight-grad is run by four wavefronts or by two groups of four that share every step (kernel_form; in the common launch with an
+  // input-grad always the latter).  The four add up the halves of a step as the groups do, so that dHW has the same bits whichever runs: 16 registers more, of
+  // which a SIMD has enough for as many workgroups as before.
+  static constexpr bool kTwoHalves = kDirect32 && OP == kWeightGrad && TI == 64 && TJ == 64 && WK == 1;
   struct Smem {
     alignas(16) T a[NSTAGE][LA::kElems];
     alignas(16) T b[NSTAGE][LB::kElems];
@@ -1353,11 +1357,24 @@ struct GemmKernel {
         for (int b = 0; b < MJ; b++)
           fb[buf][b] = lds_frag<B_LAYOUT, LB>(sm.b[st], blk_j(b), ks0 + ks, lane);
       };
-      auto mfmas = [&](int buf) {
+      // (kTwoHalves: the second half of every step into accumulators of its own, as the second group of two does)
+      f32x16_t second[kTwoHalves ? MI : 1][kTwoHalves ? MJ : 1];
+      if constexpr (kTwoHalves) {
 #pragma unroll
         for (int a = 0; a < MI; a++)
 #pragma unroll
-          for (int b = 0; b < MJ; b++) acc[a][b] = mma(fa[buf][a], fb[buf][b], acc[a][b]);
+          for (int b = 0; b < MJ; b++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) second[a][b][e] = 0.f;
+      }
+      auto mfmas = [&](int buf, int ks) {
+#pragma unroll
+        for (int a = 0; a < MI; a++)
+#pragma unroll
+          for (int b = 0; b < MJ; b++) {
+            if (kTwoHalves && ks >= NKS / 2) second[kTwoHalves ? a : 0][kTwoHalves ? b : 0] = mma(fa[buf][a], fb[buf][b], second[kTwoHalves ? a : 0][kTwoHalves ? b : 0]);
+            else acc[a][b] = mma(fa[buf][a], fb[buf][b], acc[a][b]);
+          }
       };
       // one R step; the flags say which of the side jobs still exist near the end of the loop
       // `late` staggers the side jobs of the two wavefronts that share a SIMD: one does them
@@ -1405,7 +1422,7 @@ struct GemmKernel {
               if constexpr (decltype(do_fetch)::value) fetch(s + 2);
             }
           }
-          mfmas(ks & 1);
+          mfmas(ks & 1, ks);
         }
       };
       auto loop = [&](auto late) {
@@ -1444,6 +1461,14 @@ struct GemmKernel {
         // wavefronts w and w + 4 of a workgroup share a SIMD
         if (kThreads == 512 && wave >= 4) loop(std::true_type{});
         else loop(std::false_type{});
+      }
+      if constexpr (kTwoHalves) {
+#pragma unroll
+        for (int a = 0; a < MI; a++)
+#pragma unroll
+          for (int b = 0; b < MJ; b++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[a][b][e] += second[a][b][e];
       }
     }
 

@@ -1123,10 +1123,11 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
   const bool pieces_ok = (op == kWeightGrad ? (I >= vec && J >= vec) : R >= vec) && (chunk >= R || chunk % step_direct == 0);
   f.clamp = !f.full && direct_capable && pieces_ok && t.clamp != -1;
   f.step = (f.full || f.clamp) ? step_direct : step_plain;
-  // (fp32 weight-grad on the 64 tile: in two groups, as forward and input-grad, but for many workgroups of a short loop, where adding the groups up costs
-  //  more than they hide.  Four wavefronts / eight, us: M = 160, 3008 x 6400, 4700 workgroups 67.2 / 76.3; M = 160, 3008 x 1024, 752 of them 15.5 / 16.5; 1024^3 and the
-  //  fold behind it 31.1 / 30.1.)
-  const bool two_groups = workgroups <= 2 * kComputeUnits || (chunk < R ? chunk : R) >= 384;
+  // (fp32 weight-grad on the 64 tile: in two groups, as forward and input-grad, for at most one workgroup per compute unit and a long loop.  With
+  //  more of them, the four-wavefront workgroups that share a unit hide as much, and adding the groups up costs.  124 drawn calls, eight wavefronts
+  //  in place of four, times the time: at most 256 workgroups of 512 rows and more 0.95 to 0.99, of fewer 1.01 to 1.04; up to 512 workgroups 1.02 to 1.09, up to
+  //  1024 1.02 to 1.04, beyond 1.00 to 1.02.)
+  const bool two_groups = workgroups <= kComputeUnits && (chunk < R ? chunk : R) >= 512;
   f.waves = tile == 256 ? 8
             : tile == 32 ? 4
             : tile == 64 ? ((many64 && (f.full || f.clamp)) ? 16 : (elem_bytes == 4 && (op != kWeightGrad || (two_groups && (f.full || f.clamp)))) ? 8 : 4)
@@ -1192,6 +1193,22 @@ struct BackwardForm {
 static inline long long f_tiles(const KernelForm& f, int I, int J) {
   return (long long)((I + f.rows - 1) / f.rows) * ((J + f.cols - 1) / f.cols);
 }
+// When the last of n1 workgroups of d1 each, then n2 of d2, is done, each on the compute unit that is free first: the first op's last round leaves
+// `late` units a workgroup longer.
+static inline double list_schedule(long long n1, double d1, long long n2, double d2) {
+  const long long rounds1 = n1 / kComputeUnits, late = n1 - rounds1 * kComputeUnits;
+  const double from_a = (double)rounds1 * d1, from_b = from_a + d1;
+  double end = late > 0 ? from_b : from_a;
+  for (long long done_a = 0, done_b = 0; done_a * (kComputeUnits - late) + done_b * late < n2;) {
+    const double next_a = from_a + (double)(done_a + 1) * d2, next_b = from_b + (double)(done_b + 1) * d2;
+    if (late == 0 || next_a <= next_b) done_a++;
+    else done_b++;
+    const double last = late == 0 || next_a <= next_b ? next_a : next_b;
+    end = last > end ? last : end;
+  }
+  return end;
+}
+
 // runs_us: sp are whole tiles in place of runs, which take so long by themselves (0: sp is how the input-grad goes by itself).
 static inline BackwardForm backward_form(int M, int K, int N, int H, const SplitPlan& sp, const WeightGradPlan& plan, bool with_dbias,
                                          int elem_bytes, const rz_tuning& t, double runs_us = 0.0) {
@@ -1205,7 +1222,8 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
   if (i.rows != i.cols && !pair) return b;
   b.full = i.full && w.full;
   if (i.rows == 64 && w.tile == 64) {
-    if (w.waves != i.waves) return b;
+    // (fp32: by eight wavefronts here, see kernel_form; many workgroups of a short loop lose more by that than a boundary)
+    if (elem_bytes == 4 && plan.workgroups > 2 * kComputeUnits && (plan.r_chunk < M ? plan.r_chunk : M) < 384) return b;
     b.pair = k64With64;
     b.stages = elem_bytes == 2 && ig_wgs + plan.workgroups <= kComputeUnits ? 4 : 2;
   } else if (elem_bytes == 2 && i.rows == 64 && w.tile == 128 && w.waves == 8) {
@@ -1223,11 +1241,37 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
     b.pair = k128With128;
   }
   if (b.pair == kApart) return b;
-  if (b.pair == k64With64) {
-    // (several workgroups of each on a compute unit: those of the longer loop first.  16-bit: an input-grad of at most one workgroup a unit has four
-    //  stages by itself; beside a weight-grad that fills the units twice over anyway it would only lose them — M = 3968, K = 256, N = 2688 35.1 apart, 36.2 us)
-    if (elem_bytes == 2 && ig_wgs <= kComputeUnits && ig_wgs + plan.workgroups > 2 * kComputeUnits && N >= 1024) b.pair = kApart;
-    b.wg_first = plan.r_chunk > (sp.splits > 1 ? sp.r_chunk : N);
+  if (b.pair == k64With64) {   // (several workgroups of each on a compute unit: those of the longer loop first)
+    const int ig_loop = sp.splits > 1 ? sp.r_chunk : N, wg_loop = plan.r_chunk < M ? plan.r_chunk : M;
+    b.wg_first = plan.r_chunk > ig_loop;
+    // (an image of dHW that leaves a compute unit room for one workgroup, the input-grad's as well)
+    const size_t image_bytes = plan.image_pitch > 0 ? (size_t)plan.image_pitch * sizeof(float) + (16 + 65) * sizeof(int) : 0;
+    const bool one_each = image_bytes > 80 * 1024, two_each = !one_each && 3 * image_bytes > 160 * 1024;
+    if (elem_bytes == 2) {
+      // An input-grad of at most one workgroup a unit has four stages by itself; beside a weight-grad that fills the units twice over anyway it
+      // would only lose them (M = 3968, K = 256, N = 2688 35.1 apart, 36.2 us).  One of more than three to two units, of a long loop, would lose its
+      // neighbour to an image (bf16 M = 9856, K = 192, N = 2688, 129 KB, 462 of them: 117 / 122; fp16 M = 5664, N = 2560, 267: 99 / 91).
+      if (ig_wgs <= kComputeUnits && ig_wgs + plan.workgroups > 2 * kComputeUnits && N >= 1024) b.pair = kApart;
+      if (one_each && ig_wgs > 3 * kComputeUnits / 2 && N >= 1024) b.pair = kApart;
+      return b;
+    }
+    // fp32, in rows of the contracted dimension at 0.02 us on a compute unit, with a fixed part: the two ops one after the other, each in rounds (of
+    // four-wavefront workgroups with an image more than two may share a unit, so that their last round counts by its share), against a list schedule.
+    // Apart there is a boundary more.  Together the weight-grad's workgroups have eight wavefronts, which costs 3 % (6.5 % if an image also takes an
+    // input-grad's neighbour), but gains 3 % where an image leaves room for two workgroups, and beyond two workgroups a unit the second op's come to lie as
+    // they fall, which costs a quarter of one.
+    // Fitted to 503 drawn calls: of those that it joins 15 are slower than apart by more than 1 % (at most 9 %), the others up to 33 % faster; 18 that it does
+    // not join would be 3 to 9 % faster.  Joined wherever the kernels match, 97 were slower by 1 to 11 %.  Apart / together, us: M = 50, 1920 -> 192
+    // 25.6 / 19.3; M = 384, 3008 -> 832 (282 and 611 workgroups) 66.2 / 51.3; but M = 1984, 320 -> 3008 (465 and 235 workgroups) 88.5 / 97.6,
+    // M = 6688, 192 -> 12672 with an image of 97 KB 665 / 742.
+    const double di = ig_loop + 100.0, dw = wg_loop + 130.0, n_w = (double)plan.workgroups;
+    double rounds_w = (double)((plan.workgroups + kComputeUnits - 1) / kComputeUnits);
+    if (plan.image_pitch > 0 && !two_each && plan.workgroups > 2 * kComputeUnits && n_w / kComputeUnits + 0.25 < rounds_w) rounds_w = n_w / kComputeUnits + 0.25;
+    const double apart = (double)((ig_wgs + kComputeUnits - 1) / kComputeUnits) * di + rounds_w * dw;
+    const double together = b.wg_first ? list_schedule(plan.workgroups, dw, ig_wgs, di) : list_schedule(ig_wgs, di, plan.workgroups, dw);
+    const double loose = ig_wgs + plan.workgroups > 2 * kComputeUnits ? 0.25 * (b.wg_first ? di : dw) : 0.0;
+    const double larger = (one_each && ig_wgs > kComputeUnits ? 0.065 : two_each ? -0.03 : 0.03) * apart;
+    if ((apart - together - loose - larger) * 0.02 + 5.0 <= 0.0) b.pair = kApart;
     return b;
   }
   // One workgroup on a compute unit: by what the two kernels and the common one take.  A workgroup takes its steps of 64 and a fixed part
@@ -1249,17 +1293,7 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
   b.wg_first = d_w > d_i;
   const double d1 = b.wg_first ? d_w : d_i, d2 = b.wg_first ? d_i : d_w;
   const long long n1 = b.wg_first ? n_w : n_i, n2 = b.wg_first ? n_i : n_w;
-  // the first op's last round leaves `late` units a workgroup longer; the second op's go to whichever unit is free
-  const long long rounds1 = n1 / kComputeUnits, late = n1 - rounds1 * kComputeUnits;
-  const double from_a = (double)rounds1 * d1, from_b = from_a + d1;
-  double end = late > 0 ? from_b : from_a;
-  for (long long done_a = 0, done_b = 0; done_a * (kComputeUnits - late) + done_b * late < n2;) {
-    const double next_a = from_a + (double)(done_a + 1) * d2, next_b = from_b + (double)(done_b + 1) * d2;
-    if (late == 0 || next_a <= next_b) done_a++;
-    else done_b++;
-    const double last = late == 0 || next_a <= next_b ? next_a : next_b;
-    end = last > end ? last : end;
-  }
+  const double end = list_schedule(n1, d1, n2, d2);
   // (Workgroups of the two side by side miss the L2s more often than those of one, which costs about 2 % of a launch that shares nothing else: M = 8192,
   // K = 4096, N = 16384, whose ops fill whole rounds, a pass 2316 us apart, 2349 in one launch.
   // And where both ops fill whole rounds there is the boundary alone to gain, nothing if X and dY, which both ops read, are more than the L2s hold (32 MB in all): M = 4096,

@@ -45,6 +45,11 @@ PAIRS = [
     ((1056, 7616, 704, 8192, 32, 64), BF16, ("256+256", False)),
     ((3584, 2816, 384, 16384, 64, 64), BF16, ("256+128", True)),
     ((3328, 1280, 256, 20480, 64, 64), FP16, ("256x128+128", True)),
+    ((50, 1920, 192, 23040, 64, 64), FP32, ("64+64", False, 2)),      # fp32 images of dHW; weight-grad by four wavefronts apart
+    ((512, 512, 512, 65536, 64, 64), FP32, ("64+64", True, 2)),
+    ((1984, 320, 3008, 60160, 64, 64), FP32, APART),                  # as many rounds together as apart
+    ((6688, 192, 12672, 24330, 64, 64), FP32, APART),                 # an image that takes the input-grad's neighbour
+    ((9856, 192, 2688, 32256, 64, 64), BF16, APART),                  # ... the same in 16 bits
 ]
 CODES = {FP32: 0, BF16: 1, FP16: 2}
 
