@@ -1294,11 +1294,16 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
   const double d1 = b.wg_first ? d_w : d_i, d2 = b.wg_first ? d_i : d_w;
   const long long n1 = b.wg_first ? n_w : n_i, n2 = b.wg_first ? n_i : n_w;
   const double end = list_schedule(n1, d1, n2, d2);
-  // (Workgroups of the two side by side miss the L2s more often than those of one, which costs about 2 % of a launch that shares nothing else: M = 8192,
-  // K = 4096, N = 16384, whose ops fill whole rounds, a pass 2316 us apart, 2349 in one launch.
-  // And where both ops fill whole rounds there is the boundary alone to gain, nothing if X and dY, which both ops read, are more than the L2s hold (32 MB in all): M = 4096,
-  // K = 512, N = 1024 61.8 us a pass apart, 59.0 in one launch, M = 8192 60.8 and 59.1; M = 16384 70.2 and 69.9, and 1 us slower where the host is as slow.)
-  const double boundary_us = 4.0, mixing = 1.02;
+  // What the two lose side by side: about 2 % of a launch that shares nothing else (M = 8192, K = 4096, N = 16384, whose ops fill whole rounds, a pass
+  // 2316 us apart, 2349 in one launch), and 15 % of one of complete 128 tiles: bf16 M = 14336, K = 128, N = 6912 110 / 124, fp16 M = 16128, K = 256,
+  // N = 2816 82 / 95; of 108 drawn passes 56 of the 61 that this leaves apart are slower in one launch, by up to 15 %, and 42 of the 47 that it joins
+  // faster, by up to 26 % (bf16 M = 1408, K = 1920, N = 2816, 165 and 330 workgroups, 84 / 69), the others slower by at most 6 %.  (Why is not known: the
+  // L2s miss as often, 2.2 and 2.3 million requests a pass of the second.)
+  // And where both ops fill whole rounds there is the boundary alone to gain, nothing if X and dY, which both ops read, are more than the L2s hold (32 MB
+  // in all): M = 4096, K = 512, N = 1024 61.8 us a pass apart, 59.0 in one launch, M = 8192 60.8 and 59.1; M = 16384 70.2 and 69.9, and 1 us slower where
+  // the host is as slow; of 24 drawn ones none gains more than 2.3 %.  (Nearly whole rounds gain: 96 drawn passes on other tiles 0.97 in the mean.)
+  // (A complete op beside a ragged one takes the checks too, which is not priced: 150 such drawn passes 0.94 in the mean, the slowest 1.03.)
+  const double boundary_us = 4.0, mixing = b.pair == k128With128 && b.full ? 1.15 : 1.02;
   if (n_i % kComputeUnits == 0 && n_w % kComputeUnits == 0 && (double)M * ((double)K + N) * elem_bytes > 32.0e6) b.pair = kApart;
   const double ig_alone = runs_us > 0.0 ? runs_us - kForward16Times[6].launch : alone(i, false, ig_chunk, N, n_i);
   if (end * mixing > (ig_alone + alone(w, true, plan.r_chunk, M, n_w)) + boundary_us) b.pair = kApart;
