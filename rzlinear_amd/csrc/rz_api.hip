@@ -1138,7 +1138,7 @@ RZ_API int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int
       out[0] = 0; out[1] = 1; out[2] = M; out[3] = 32; out[4] = 4; out[5] = wp.windows; out[7] = wp.windows;
       return RZ_OK;
     }
-    const KernelForm f = kernel_form(op, K, N, M, plan.r_chunk, plan.tile, plan.workgroups, eb, t);
+    const KernelForm f = kernel_form(op, K, N, M, plan.r_chunk, plan.tile, plan.workgroups, eb, t, plan.image_pitch > 0);
     out[0] = plan.tile; out[1] = plan.splits; out[2] = plan.r_chunk; out[3] = f.step;
     out[4] = plan.fold.use ? 5 : plan.image_pitch > 0 ? 2 : 3;
     out[5] = (int32_t)plan.workgroups;

@@ -194,7 +194,7 @@ static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const 
   const int tile = wg ? plan->tile : (split != nullptr ? split->tile : pick_tile(p.I, p.J, (int)sizeof(T), tuning));
   const int chunk = wg ? plan->r_chunk : (cut ? split->r_chunk : p.R);
   const long long workgroups = wg ? plan->workgroups : tile_count(p.I, p.J, tile) * (cut ? split->splits : 1);
-  const KernelForm form = kernel_form(OP, p.I, p.J, p.R, chunk, tile, workgroups, (int)sizeof(T), tuning);
+  const KernelForm form = kernel_form(OP, p.I, p.J, p.R, chunk, tile, workgroups, (int)sizeof(T), tuning, wg && plan->image_pitch > 0);
   if constexpr (sizeof(T) == 2 && OP != kWeightGrad) {
     if (form.rows == 32 && form.cols == 128) return launch_tile<T, OP, 32, 1, 4, 3, false, 2, 128>(p, plan, split, form, stream);
   }
@@ -229,11 +229,11 @@ static hipError_t launch_gemm_t(GemmParams p, const WeightGradPlan* plan, const 
   }
 }
 
-// The two kernels of a backward pass in one launch.  What a boundary between two launches costs a GPU that is waiting for it is 5 to 6 us, and
-// the host a launch; where neither op fills the chip their workgroups run side by side as well.  GPU-bound, with what finishes dHW (apart / in
-// one launch, us): bf16 M = 78, K = 752, N = 133 17.2 / 11.4; M = 160, K = 448, N = 1216 22.6 / 15.0; M = 6016, K = 3200, N = 1600 156 / 135;
-// fp16 M = 3663, K = 13603, N = 1370 360 / 294; fp32 M = 2025, K = 848, N = 1941 148 / 131; 1024^3 through the module, forward included, 68.9 / 63.6.  Over 90
-// drawn shapes none slower by more than runs differ.
+// The two kernels of a backward pass in one launch (with column sums: there is none without a bias gradient).  What a boundary between two launches costs a GPU
+// that is waiting for it is 4 to 6 us, and the host a launch; where neither op fills the chip their workgroups run side by side as well.  GPU-bound, with what
+// finishes dHW (apart / in one launch, us): bf16 M = 78, K = 752, N = 133 17.2 / 11.4; M = 160, K = 448, N = 1216 22.6 / 15.0; M = 6016, K = 3200, N = 1600
+// 156 / 135; fp16 M = 3663, K = 13603, N = 1370 360 / 294; fp32 M = 50, K = 1920, N = 192 25.6 / 19.3; fp32 1024^3 through the module, forward included,
+// 68.8 / 63.6.  Where it is not faster: backward_form.
 template <typename T, int TI, int TJ, int WI, int WJ, int IG_STAGES, int WK, int TILE, int WG_WI, int WG_WJ, int WG_STAGES, int WG_WK, bool FULL>
 static hipError_t launch_backward_form(GemmParams ig, const SplitPlan* split, GemmParams wg, const WeightGradPlan* plan, bool wg_first,
                                        hipStream_t stream) {

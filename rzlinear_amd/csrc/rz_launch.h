@@ -1090,8 +1090,9 @@ struct KernelForm {
   int step;
 };
 
+// (image: a weight-grad whose workgroups hold an image of dHW in LDS)
 static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int tile, long long workgroups,
-                                     int elem_bytes, const rz_tuning& t) {
+                                     int elem_bytes, const rz_tuning& t, bool image = false) {
   KernelForm f;
   f.tile = tile;
   f.rows = tile;
@@ -1123,11 +1124,11 @@ static inline KernelForm kernel_form(int op, int I, int J, int R, int chunk, int
   const bool pieces_ok = (op == kWeightGrad ? (I >= vec && J >= vec) : R >= vec) && (chunk >= R || chunk % step_direct == 0);
   f.clamp = !f.full && direct_capable && pieces_ok && t.clamp != -1;
   f.step = (f.full || f.clamp) ? step_direct : step_plain;
-  // (fp32 weight-grad on the 64 tile: in two groups, as forward and input-grad, for at most one workgroup per compute unit and a long loop.  With
-  //  more of them, the four-wavefront workgroups that share a unit hide as much, and adding the groups up costs.  124 drawn calls, eight wavefronts
-  //  in place of four, times the time: at most 256 workgroups of 512 rows and more 0.95 to 0.99, of fewer 1.01 to 1.04; up to 512 workgroups 1.02 to 1.09, up to
-  //  1024 1.02 to 1.04, beyond 1.00 to 1.02.)
-  const bool two_groups = workgroups <= kComputeUnits && (chunk < R ? chunk : R) >= 512;
+  // (fp32 weight-grad on the 64 tile: in two groups, as forward and input-grad, for at most one workgroup per compute unit and a long loop, or an image, which
+  //  more wavefronts clear and store.  With more workgroups, the four-wavefront ones that share a unit hide as much, and adding the groups up costs.  124 drawn
+  //  calls, eight wavefronts in place of four, times the time: at most 256 workgroups of 512 rows and more 0.95 to 0.99, of fewer 1.01 to 1.04, of a few rows
+  //  and an image 0.98 to 0.99 (M = 3, K = N = 192, a pass 18.2 / 17.8 us); up to 512 workgroups 1.02 to 1.09, up to 1024 1.02 to 1.04, beyond 1.00 to 1.02.)
+  const bool two_groups = workgroups <= kComputeUnits && (image || (chunk < R ? chunk : R) >= 512);
   f.waves = tile == 256 ? 8
             : tile == 32 ? 4
             : tile == 64 ? ((many64 && (f.full || f.clamp)) ? 16 : (elem_bytes == 4 && (op != kWeightGrad || (two_groups && (f.full || f.clamp)))) ? 8 : 4)
@@ -1216,7 +1217,7 @@ static inline BackwardForm backward_form(int M, int K, int N, int H, const Split
   if (!with_dbias || sp.run_steps > 0 || t.tile != 0 || t.stages == 1 || t.clamp == -1 || (long long)H * 4 > 0x7fffffffLL) return b;
   const long long ig_wgs = tile_count(M, K, sp.tile) * sp.splits;
   const KernelForm i = kernel_form(kInputGrad, M, K, N, sp.splits > 1 ? sp.r_chunk : N, sp.tile, ig_wgs, elem_bytes, t);
-  const KernelForm w = kernel_form(kWeightGrad, K, N, M, plan.r_chunk, plan.tile, plan.workgroups, elem_bytes, t);
+  const KernelForm w = kernel_form(kWeightGrad, K, N, M, plan.r_chunk, plan.tile, plan.workgroups, elem_bytes, t, plan.image_pitch > 0);
   if (!(i.full || i.clamp) || !(w.full || w.clamp) || i.short_loop || w.short_loop) return b;
   const bool pair = i.rows == 256 && i.cols == 128;
   if (i.rows != i.cols && !pair) return b;
