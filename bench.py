@@ -91,8 +91,8 @@ TRAFFIC = {
     },
     ("cpu_ref_1024", "fp32"): {
         "profile": "profiles/rz_gemm_fp32_cpu_ref_1024.txt",
-        "bytes": {"forward": int((3162.0 * 2.0 + 4096.0) * 1024), "input_grad": int((3157.0 * 2.0 + 4096.0) * 1024),
-                  "weight_grad": int((12338.5 * 2.0 + 4096.0) * 1024)},   # X^T.dY written tile by tile: 4 MiB
+        "bytes": {"forward": int((3152.3 * 2.0 + 4096.0) * 1024), "input_grad": int((3151.8 * 2.0 + 4096.0) * 1024),
+                  "weight_grad": int((12351.3 * 2.0 + 4096.0) * 1024)},   # X^T.dY written tile by tile: 4 MiB
     },
     ("ffn", "bf16"): {
         "profile": "profiles/rz_gemm_fold_bf16_ffn.txt",

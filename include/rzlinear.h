@@ -346,11 +346,14 @@ int rz_plan_query(int op, int M, int K, int N, int H, int BK, int BN, int dtype,
 /* ---- input-grad and weight-grad of one backward pass -----------------------------------
  * Replaces rz_linear_backward_tl                                      impl/RzLinearBackward.py:7-20
  * rz_input_grad_hashed followed by rz_weight_grad_hashed (layer_plan NULL) or rz_weight_grad_planned, with the same
- * results to the bit, but for an input-grad that would be dealt out in runs (rz_plan_query): beside a weight-grad it may
- * go in whole tiles, whose sums over N are in one piece.  Where the two contractions' kernels go together they are
- * enqueued as ONE launch: a launch less, and workgroups of the one fill what those of the other leave idle.  The two workspaces
- * (rz_linear_backward_hashed_dx_workspace_bytes, which is never more than rz_input_grad_hashed_workspace_bytes, with
- * RZ_PLAN_WITH_LAYER_PLAN in its flags where the call carries a plan; rz_weight_grad_hashed_workspace_bytes) and the outputs must not overlap. */
+ * results to the bit (a dHW by global atomics is never the same to the bit), but for an input-grad that by itself would
+ * be dealt out in runs (rz_plan_query): where it shares a launch with the weight-grad (rz_backward_query) it goes in
+ * whole tiles, whose sums over N are in one piece.  Where the two contractions' kernels go together, and that is faster,
+ * they are enqueued as ONE launch: a launch less, and workgroups of the one fill what those of the other leave idle.
+ * That asks for a bias gradient (dbias): without one the two are enqueued one after the other, the input-grad first.
+ * The two workspaces (rz_linear_backward_hashed_dx_workspace_bytes, which is never more than
+ * rz_input_grad_hashed_workspace_bytes, with RZ_PLAN_WITH_LAYER_PLAN in its flags where the call carries a plan;
+ * rz_weight_grad_hashed_workspace_bytes) and the outputs must not overlap. */
 size_t rz_linear_backward_hashed_dx_workspace_bytes(int M, int K, int N, int H, int BK, int BN, int dtype, unsigned flags,
                                                     int with_dbias, const rz_tuning* tuning);
 int rz_linear_backward_hashed(const void* X, const void* dY, const void* HW, void* dX, void* dHW, void* dbias,
